@@ -2,6 +2,7 @@
 // declared in include/cascade_hip.h. gfx950 only.
 #include "../../include/cascade_hip.h"
 
+#include "coded_keys.hpp"
 #include "device_pool.hpp"
 #include "device_utils.hpp"
 #include "doubling.hpp"
@@ -177,6 +178,7 @@ constexpr int SMALL_MAXG_HI = CSA_SMALL_MAXG_HI;
 constexpr u32 SMALL_AVG_LIMIT = CSA_SMALL_AVG_LIMIT;
 static_assert(SMALL_MAXG_HI >= SMALL_MAXG, "the higher group limit is the higher one");
 constexpr u32 TICKET_POOL = 4096;
+constexpr u64 CODE_TABLE_WORDS = SYMBOLS + RESOLVE_MARK_WORDS + SYMBOLS + 4; // symbol counts, marks, shares (and entry [SYMBOLS])
 constexpr u32 PINNED_HIST = 32;        // host mirror: words [0, 16) mirror the device counters, [16, 32) single values, then the histograms
 constexpr u32 MSG_OFF_WORDS = 32769;   // p + 1 outbox counters, p <= 32768
 constexpr int EVENT_POOL = 2 * CSA_MAX_GENERATIONS * MAX_PASSES * 2;
@@ -292,6 +294,7 @@ struct csa_handle {
     u64* lookback = nullptr;
     u64 lookback_words = 0;
     u64 lookback_tile_words = 0;
+    u32* code_tables = nullptr; // resident sort: symbol counts, marks of codes, shares of the symbols (sort_by_codes)
     u32* tile_tables = nullptr; // rerank: [rank_tiles_cap][4] tile aggregates, the same of prefixes, [rank_tiles_cap] splits,
                                 // [RERANK_SLABS][5] slab totals
     u64 rank_tiles_cap = 0;
@@ -400,35 +403,36 @@ void launch_onesweep(const csa_handle* h, OnesweepArgs& a, hipStream_t s)
         launch_onesweep_shape<SRC, SORT_BLOCK, VALS>(tile_order_of(h), a, s);
 }
 
+template <int SRC>
 void launch_onesweep32(const csa_handle* hh, OnesweepArgs& a, hipStream_t s)
 {
     const TileOrder h = tile_order_of(hh);
     if (wide_workgroups(a)) {
         set_tile_order(h, a, SORT_WIDE_BLOCK * SORT32_ITEMS);
-        hipLaunchKernelGGL((onesweep_kernel<u32, SORT_WIDE_BLOCK, SORT32_ITEMS, SRC_PAIRS, 0>), dim3(a.tiles), dim3(SORT_WIDE_BLOCK), 0, s, a);
+        hipLaunchKernelGGL((onesweep_kernel<u32, SORT_WIDE_BLOCK, SORT32_ITEMS, SRC, 0>), dim3(a.tiles), dim3(SORT_WIDE_BLOCK), 0, s, a);
     } else {
         set_tile_order(h, a, SORT_BLOCK * SORT32_ITEMS);
-        hipLaunchKernelGGL((onesweep_kernel<u32, SORT_BLOCK, SORT32_ITEMS, SRC_PAIRS, 0>), dim3(a.tiles), dim3(SORT_BLOCK), 0, s, a);
+        hipLaunchKernelGGL((onesweep_kernel<u32, SORT_BLOCK, SORT32_ITEMS, SRC, 0>), dim3(a.tiles), dim3(SORT_BLOCK), 0, s, a);
     }
 }
 
 // Sorts n pairs by the digits of `plan`. The first pass that runs takes its input as `src` says
-// (pairs kin/vin, or the text); passes alternate between the (kin, vin) and (kout, vout) sets, the
+// (pairs kin/vin, or keys built on the way in); passes alternate between the (kin, vin) and (kout, vout) sets, the
 // very first one writing to (kout, vout). *result_in_out = 1 if the sorted pairs ended in (kout, vout).
 // Passes whose digit is the same for every pair are skipped (they would be the identity).
 // src = SRC_RANKS: pair i is ((rank_src[i], rank_src[i + hop]), i), i < n, built by the first pass that runs; the two
 // ranks are combined as rank_pair_key says for `radix`.
 // src = SRC_PACKED: the first pass cuts its keys from the code stream `packed` describes; the caller has filled
-// ghist already (hist_ready = 2). hist_ready = 1 (SRC_TEXT): the byte histograms of the text are in place.
+// ghist already.
 struct PackedSource {
     const u32* stream;
     u64 words;
     u32 sym_bits, key_bits;
 };
 
-int radix_sort(Launch& L, int src, const u16* text, u32 text_n, u32 tail, u32 word, u64* kin, u32* vin, u64* kout,
+int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64* kout,
                u32* vout, u32 n, const PassPlan& plan, int* result_in_out, int* passes_run, const u32* rank_src = nullptr,
-               u32 hop = 0, u32 radix = 0, const PackedSource* packed = nullptr, int hist_ready = 0)
+               u32 hop = 0, u32 radix = 0, const PackedSource* packed = nullptr)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -436,20 +440,14 @@ int radix_sort(Launch& L, int src, const u16* text, u32 text_n, u32 tail, u32 wo
     *passes_run = 0;
     if (n == 0)
         return CSA_OK;
-    // ghist[MAX_PASSES][256] followed by the two byte histograms of the text
-    if (hist_ready == 0)
-        HIP_TRY(hipMemsetAsync(h->ghist, 0, (MAX_PASSES + 2) * RADIX_BINS * sizeof(u32), s));
     if (src == SRC_PACKED) {
-        if (!packed || hist_ready != 2)
-            return fail(CSA_ERR_INTERNAL, "radix_sort: packed keys come with their histograms");
-    } else if (src == SRC_PAIRS || src == SRC_RANKS) {
+        if (!packed)
+            return fail(CSA_ERR_INTERNAL, "radix_sort: packed keys come with their stream");
+    } else {
+        HIP_TRY(hipMemsetAsync(h->ghist, 0, MAX_PASSES * RADIX_BINS * sizeof(u32), s));
         HistArgs ha;
         ha.keys = kin;
-        ha.vals = vin;
-        ha.text = text;
         ha.n = n;
-        ha.text_n = text_n;
-        ha.word = word;
         ha.plan = plan;
         ha.ghist = h->ghist;
         if (src == SRC_RANKS) {
@@ -485,14 +483,6 @@ int radix_sort(Launch& L, int src, const u16* text, u32 text_n, u32 tail, u32 wo
         } else {
             hipLaunchKernelGGL(radix_hist_kernel, dim3(hist_blocks(256 * 16, n)), dim3(256), 0, s, ha);
         }
-    } else {
-        // every suffix of the text takes part and the plan is the eight bytes of one key word: the digit
-        // histograms follow from the byte histogram of the text, whatever order the pairs are in
-        u32* bytehist = h->ghist + MAX_PASSES * RADIX_BINS;
-        if (hist_ready == 0)
-            hipLaunchKernelGGL(text_byte_hist_kernel, dim3(hist_blocks(256 * 8 * 16, text_n)), dim3(256), 0, s, text, text_n,
-                               bytehist);
-        hipLaunchKernelGGL(text_hist_expand_kernel, dim3(1), dim3(256), 0, s, text, text_n, word, bytehist, h->ghist);
     }
     hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, plan.num_passes);
     HIP_TRY(hipGetLastError());
@@ -523,11 +513,9 @@ int radix_sort(Launch& L, int src, const u16* text, u32 text_n, u32 tail, u32 wo
         a.vals_in = where == 0 ? vin : vout;
         a.keys_out = where == 0 ? kout : kin;
         a.vals_out = where == 0 ? vout : vin;
-        a.text = text;
         a.n = n;
         a.text_n = text_n;
         a.tail = tail;
-        a.word = word;
         a.shift = plan.shift[p];
         a.bits = plan.bits[p];
         a.digit_base = h->digit_base + p * RADIX_BINS;
@@ -555,10 +543,8 @@ int radix_sort(Launch& L, int src, const u16* text, u32 text_n, u32 tail, u32 wo
             launch_onesweep<SRC_PAIRS>(h, a, s);
         else if (use_src == SRC_RANKS)
             launch_onesweep<SRC_RANKS>(h, a, s);
-        else if (use_src == SRC_PACKED)
-            launch_onesweep<SRC_PACKED>(h, a, s);
         else
-            launch_onesweep<SRC_TEXT>(h, a, s);
+            launch_onesweep<SRC_PACKED>(h, a, s);
         if (timed) {
             HIP_TRY(hipEventRecord(h->events[L.events_used + 1], s));
             L.timed.push_back({L.events_used, (u64)n});
@@ -689,11 +675,9 @@ int deferred_rank_update(Launch& L, const DeferBuffers& buf, u32 n)
             a.vals_in = nullptr; // the records travel alone
             a.keys_out = buf.recs[(p + 1) & 1];
             a.vals_out = nullptr;
-            a.text = nullptr;
             a.n = n;
             a.text_n = n;
             a.tail = 0;
-            a.word = 0;
             a.shift = 32 + xshift[p]; // the position is the high half of a record
             a.bits = xbits[p];
             a.digit_base = h->digit_base + p * RADIX_BINS;
@@ -740,11 +724,9 @@ int windowed_rank_update(Launch& L, const u32* pos, const DeferBuffers& buf, u32
         a.vals_in = buf.vals;
         a.keys_out = buf.t1_pos;
         a.vals_out = buf.t1_val;
-        a.text = nullptr;
         a.n = m;
         a.text_n = n;
         a.tail = 0;
-        a.word = 0;
         a.shift = shift;
         a.bits = top;
         a.digit_base = h->digit_base;
@@ -755,7 +737,7 @@ int windowed_rank_update(Launch& L, const u32* pos, const DeferBuffers& buf, u32
         int rc = next_ticket(L, &a.ticket);
         if (rc)
             return rc;
-        launch_onesweep32(h, a, s);
+        launch_onesweep32<SRC_PAIRS>(h, a, s);
         in_pos = buf.t1_pos;
         in_val = buf.t1_val;
     }
@@ -873,10 +855,112 @@ PackedPlan plan_packed_text(const u32* bytehist, u32 n, int key_words, u64 room_
     return pp;
 }
 
+// Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their four symbols, with the ties marked,
+// in ra.sufs' array. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into idx[1]; the codes
+// live in the halves of key[0], their text order in key[1]. `marked` is left ready for sort_marked_runs.
+int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, ResolveArgs& marked)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    u32* const counts = h->code_tables; // [SYMBOLS], then the marks, then cum[SYMBOLS + 1]
+    u32* const marks = counts + SYMBOLS;
+    u32* const cum = marks + RESOLVE_MARK_WORDS;
+    HIP_TRY(hipMemsetAsync(counts, 0, (SYMBOLS + RESOLVE_MARK_WORDS) * sizeof(u32), s));
+    const u32 chunks = (n + SAMPLE_CHUNK - 1) / SAMPLE_CHUNK;
+    const u32 taken = chunks < SAMPLE_CHUNKS_MAX ? chunks : SAMPLE_CHUNKS_MAX;
+    const u64 sampled = (u64)taken * SAMPLE_CHUNK < n ? (u64)taken * SAMPLE_CHUNK : (u64)n;
+    hipLaunchKernelGGL(sample_symbols_kernel, dim3((taken + SAMPLE_CHUNKS_PER_BLOCK - 1) / SAMPLE_CHUNKS_PER_BLOCK), dim3(SAMPLE_BLOCK), 0, s,
+                       d_text, n, chunks, taken, counts);
+    hipLaunchKernelGGL(symbol_shares_kernel, dim3(1), dim3(1024), 0, s, (const u32*)counts, SAMPLE_LOG2 - bit_length(sampled - 1), cum);
+    u32* const codes = reinterpret_cast<u32*>(h->key[1]); // by virtual position
+    hipLaunchKernelGGL(code_suffixes_kernel, dim3(hist_blocks(CODE_BLOCK * CODE_ITEMS, n)), dim3(CODE_BLOCK), 0, s, d_text, n, tail,
+                       (const u32*)cum, codes, h->ghist);
+    hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, CODE_PASSES);
+    u32* const sorted[2] = {reinterpret_cast<u32*>(h->key[0]), reinterpret_cast<u32*>(h->key[0]) + h->cap};
+    static_assert(CODE_PASSES % 2 == 0, "the sorted codes end in the first half of key[0], their suffixes in idx[0]");
+    for (int p = 0; p < CODE_PASSES; ++p) {
+        OnesweepArgs a;
+        a.keys_in = p == 0 ? codes : sorted[p & 1];
+        a.vals_in = h->idx[p & 1];
+        a.keys_out = sorted[(p + 1) & 1];
+        a.vals_out = h->idx[(p + 1) & 1];
+        a.n = n;
+        a.text_n = n;
+        a.tail = tail;
+        a.shift = 8 * p;
+        a.bits = 8;
+        a.digit_base = h->digit_base + p * RADIX_BINS;
+        a.lookback = h->lookback;
+        a.lookback_groups = h->lookback + h->lookback_tile_words;
+        a.epoch = next_epoch(h);
+        a.err = h->counts + 2;
+        int rc = next_ticket(L, &a.ticket);
+        if (rc)
+            return rc;
+        if (p == 0)
+            launch_onesweep32<SRC_CODED>(h, a, s);
+        else
+            launch_onesweep32<SRC_PAIRS>(h, a, s);
+    }
+    memset(&marked, 0, sizeof(marked));
+    marked.codes = sorted[0];
+    marked.sufs = h->idx[0];
+    marked.text = d_text;
+    marked.n = n;
+    marked.ell = ell;
+    marked.sufs_out = h->idx[1];
+    marked.marks = marks;
+    marked.unordered = h->counts + 4;
+    hipLaunchKernelGGL(resolve_runs_kernel, dim3((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, marked);
+    HIP_TRY(hipGetLastError());
+    return CSA_OK;
+}
+
+// The runs whose codes are marked (long and out of order): their members are collected in list order, radix sorted by their four
+// symbols and put back. Works in key[1], key[2] and idx[2..4], which hold nothing before the list is ranked.
+int sort_marked_runs(Launch& L, ResolveArgs a, int* passes)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    const RankTables r = rank_tables(h, a.n, COLLECT_TILE);
+    a.keys = h->key[1];
+    a.members = h->idx[3];
+    a.places = h->idx[2];
+    a.tile_agg = r.tile_agg;
+    a.tile_splits = r.tile_splits;
+    a.tile_prefix = r.tile_prefix;
+    a.slab_total = r.slab_total;
+    a.slab = r.slab;
+    hipLaunchKernelGGL((collect_marked_kernel<false>), dim3(r.tiles), dim3(COLLECT_BLOCK), 0, s, a);
+    hipLaunchKernelGGL(rerank_scan_kernel, dim3(r.slabs), dim3(1024), 0, s, r.tile_agg, r.tile_prefix, r.tiles, r.slab, r.slab_total,
+                       r.tile_splits);
+    hipLaunchKernelGGL((collect_marked_kernel<true>), dim3(r.tiles), dim3(COLLECT_BLOCK), 0, s, a);
+    HIP_TRY(hipGetLastError());
+    u32* h_slabs = h->h_pinned + PINNED_HIST;
+    HIP_TRY(hipMemcpyAsync(h_slabs, r.slab_total, r.slabs * 5 * sizeof(u32), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    u64 count = 0;
+    for (u32 sl = 0; sl < r.slabs; ++sl)
+        count += h_slabs[sl * 5 + 2];
+    int in_out = 0, run = 0;
+    int rc = radix_sort(L, SRC_PAIRS, 0, 0, h->key[1], h->idx[3], h->key[2], h->idx[4], (u32)count, make_plan(0, 64), &in_out, &run);
+    if (rc)
+        return rc;
+    *passes += run;
+    if (in_out) {
+        a.keys = h->key[2];
+        a.members = h->idx[4];
+    }
+    hipLaunchKernelGGL(place_marked_kernel, dim3((u32)((count + 255) / 256)), dim3(256), 0, s, a, (u32)count);
+    HIP_TRY(hipGetLastError());
+    return CSA_OK;
+}
+
 // Generation 0: ranks the sorted list described by `ra`: counts per tile, scans the counts, reads the totals back, then
 // applies them and brings rank[] up to date, directly from the kernel or through the two-pass bucketed update.
+// coded: the list comes from sort_by_codes and carries its ties.
 int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivors, u32* groups, int* rank_update,
-                u32* level_counts = nullptr)
+                u32* level_counts = nullptr, const ResolveArgs* coded = nullptr, int* passes = nullptr)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -894,12 +978,24 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
         ra.level_totals = reinterpret_cast<unsigned long long*>(h->ghist);
         HIP_TRY(hipMemsetAsync(ra.level_totals, 0, LEVEL_SLOTS * 8 * sizeof(unsigned long long), s));
     }
-    hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
+    if (coded)
+        hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS, true>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
+    else
+        hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS, false>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
     if (ra.levels)
         HIP_TRY(hipMemcpyAsync(h_levels, ra.level_totals, LEVEL_SLOTS * 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     int rc = rank_totals(L, r, true, ra.m, ra.n, false, survivors, groups, rank_update);
     if (rc)
         return rc;
+    if (coded && h->h_pinned[4] != 0) { // long runs of one code are out of order: they are sorted now, and the list is counted again
+        rc = sort_marked_runs(L, *coded, passes);
+        if (rc)
+            return rc;
+        hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS, true>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
+        rc = rank_totals(L, r, true, ra.m, ra.n, false, survivors, groups, rank_update);
+        if (rc)
+            return rc;
+    }
     for (u32 i = 0; i < ra.levels && level_counts; ++i) {
         u64 sv = 0, hd = 0;
         for (u32 slot = 0; slot < LEVEL_SLOTS; ++slot) {
@@ -913,7 +1009,10 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
     ra.ordinals = dense_generation(*survivors, *groups, ra.n) ? 1u : 0u;
     if (*rank_update != 0)
         ra.rank_recs = buf.recs[0];
-    hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
+    if (coded)
+        hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS, true>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
+    else
+        hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS, false>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
     HIP_TRY(hipGetLastError());
     if (*rank_update == 1)
         return deferred_rank_update(L, buf, ra.n);
@@ -936,19 +1035,19 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     const u64 wide_ell = 4ull * (u64)h->key_words;
 
     RangeScope range_sort("sort_partition n=%u", n);
-    HIP_TRY(hipMemsetAsync(h->counts, 0, 4 * sizeof(u32), s));
+    HIP_TRY(hipMemsetAsync(h->counts, 0, 5 * sizeof(u32), s));
     HIP_TRY(hipEventRecord(h->ev_gen[0], s));
 
     // ---- generation 0: sort every suffix by its K-gram key, ties of tail suffixes broken by length ----
     RangeScope range_gen0("generation 0 m=%u", n);
-    // The byte histograms of the text come first: they give the digit counts of the passes and tell whether the alphabet
-    // is small enough for keys of more than four symbols.
+    // The byte histograms of the text come first: they tell whether the alphabet is small enough for keys of more than four
+    // symbols. (The digit counts are zeroed with them.)
     HIP_TRY(hipMemsetAsync(h->ghist, 0, (MAX_PASSES + 2) * RADIX_BINS * sizeof(u32), s));
     u32* const bytehist = h->ghist + MAX_PASSES * RADIX_BINS;
-    hipLaunchKernelGGL(text_byte_hist_kernel, dim3(hist_blocks(256 * 8 * 16, n)), dim3(256), 0, s, d_text, n, bytehist);
     PackedPlan pp;
     memset(&pp, 0, sizeof(pp));
     if (h->pack_symbols) {
+        hipLaunchKernelGGL(text_byte_hist_kernel, dim3(hist_blocks(256 * 8 * 16, n)), dim3(256), 0, s, d_text, n, bytehist);
         u32* h_bytes = h->h_pinned + PINNED_HIST;
         HIP_TRY(hipMemcpyAsync(h_bytes, bytehist, 2 * RADIX_BINS * sizeof(u32), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
@@ -962,9 +1061,9 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     int passes = 0, p1 = 0, in_out = 0;
     u64* K[2] = {h->key[0], h->key[1]};
     u32* V[2] = {h->idx[0], h->idx[1]};
-    int cur; // the (K, V) set that holds the sorted pairs
+    int cur = 0; // the (K, V) set that holds the sorted pairs
     int rc;
-    cur = 0;
+    ResolveArgs marked;
     if (pp.enabled) {
         // the code stream lives in rank[], which nothing uses before the sorted list is ranked
         PackedSource ps;
@@ -982,10 +1081,11 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         hipLaunchKernelGGL(packed_hist_expand_kernel, dim3(1), dim3(256), 0, s, ps.stream, n, ps.sym_bits, pp.codes.key_syms,
                            plan.num_passes, gramhist, h->ghist);
         HIP_TRY(hipGetLastError());
-        rc = radix_sort(L, SRC_PACKED, d_text, n, tail, 0, K[0], V[0], K[1], V[1], n, plan, &in_out, &p1, nullptr, 0, 0, &ps, 2);
+        rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, plan, &in_out, &p1, nullptr, 0, 0, &ps);
     } else {
-        rc = radix_sort(L, SRC_TEXT, d_text, n, tail, 0, K[0], V[0], K[1], V[1], n, make_plan(0, 64), &in_out, &p1, nullptr, 0, 0,
-                        nullptr, 1);
+        rc = sort_by_codes(L, d_text, n, tail, ell, marked);
+        p1 = CODE_PASSES;
+        in_out = 1; // idx[1] holds the list, key[0] and key[1] what the sort has left behind
     }
     if (rc)
         return rc;
@@ -1007,10 +1107,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     ra.keys = k_sorted;
     ra.sufs = sa32;
     ra.m = n;
-    ra.key_words = 1;
     ra.n = n;
     ra.ell = ell;
-    ra.text = d_text;
     ra.rank = h->rank;
     ra.sufs_out = ax;
     ra.gids_out = agid;
@@ -1033,7 +1131,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         ra.level_ell[i] = (u32)wide_ell << i;
         ra.level_drop[i] = (ell - ra.level_ell[i]) * pp.codes.bits;
     }
-    rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], level_counts);
+    rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], level_counts, pp.enabled ? nullptr : &marked, &passes);
     range_gen0.close();
     if (rc)
         return rc;
@@ -1078,7 +1176,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                 const u64 runs = (u64)groups + ((u64)n - m_in);
                 const u32 radix = (u32)runs;
                 const PassPlan plan = make_plan(0, runs > 1 ? bit_length(runs * runs - 1) : 1);
-                rc = radix_sort(L, SRC_RANKS, nullptr, n, 0, 0, bkey[0], bx[0], bkey[1], bx[1], n, plan, &in_out, &passes, h->rank,
+                rc = radix_sort(L, SRC_RANKS, n, 0, bkey[0], bx[0], bkey[1], bx[1], n, plan, &in_out, &passes, h->rank,
                                 (u32)hop, radix);
             } else {
                 PassPlan plan; // the digits of the two ranks of a key: bits [0, sec_bits) and [32, 32 + sec_bits)
@@ -1089,7 +1187,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                         plan.bits[plan.num_passes] = sec_bits - b < RADIX_BITS ? sec_bits - b : RADIX_BITS;
                         plan.num_passes++;
                     }
-                rc = radix_sort(L, SRC_RANKS, nullptr, n, 0, 0, bkey[0], bx[0], bkey[1], bx[1], n, plan, &in_out, &passes, h->rank,
+                rc = radix_sort(L, SRC_RANKS, n, 0, bkey[0], bx[0], bkey[1], bx[1], n, plan, &in_out, &passes, h->rank,
                                 (u32)hop, 0u);
             }
             if (rc)
@@ -1099,10 +1197,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             rd.keys = bkey[in_out];
             rd.sufs = bx[in_out];
             rd.m = n;
-            rd.key_words = 1;
             rd.n = n;
             rd.ell = 0; // no suffix is set apart for running off the text: the tied ones never do, the others are alone anyway
-            rd.text = d_text;
             rd.rank = h->rank;
             rd.sufs_out = ax;
             rd.gids_out = agid;
@@ -1261,7 +1357,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             if (big > 0 && unordered != 0) {
                 const int gid_bits = bit_length(groups > 1 ? groups - 1 : 0);
                 const PassPlan plan = make_plan(0, sec_bits + gid_bits);
-                rc = radix_sort(L, SRC_PAIRS, nullptr, n, 0, 0, bkey[0], bx[0], bkey[1], bx[1], big, plan, &in_out, &passes);
+                rc = radix_sort(L, SRC_PAIRS, n, 0, bkey[0], bx[0], bkey[1], bx[1], big, plan, &in_out, &passes);
                 if (rc)
                     return rc;
                 PlaceArgs pa;
@@ -1639,7 +1735,7 @@ int csa_join_messages_sorted_dev(csa_handle* h, const uint8_t* d_msg_target, con
     HIP_TRY(hipMemcpyAsync(V[0], d_msg_rank, (u64)msg_c * sizeof(u32), hipMemcpyDeviceToDevice, s));
     int in_out = 0, passes = 0;
     const PassPlan plan = make_plan(0, 40);
-    int rc = radix_sort(L, SRC_PAIRS, nullptr, 0, 0, 0, K[0], V[0], K[1], V[1], msg_c, plan, &in_out, &passes);
+    int rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], V[0], K[1], V[1], msg_c, plan, &in_out, &passes);
     if (rc)
         return rc;
     u32 dir_log2 = 0;
@@ -1724,7 +1820,7 @@ int scatter_to_rank_order(csa_handle* h, const char* who, const u8* d_suf, const
                            K[0], V[0], h->counts + 3);
         const int window_bits = bit_length((part_sz - 1) >> SCATTER_WINDOW_LOG2);
         int in_out = 0, passes = 0;
-        const int rc = radix_sort(L, SRC_PAIRS, nullptr, 0, 0, 0, K[0], V[0], K[1], V[1], (u32)part_sz,
+        const int rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], V[0], K[1], V[1], (u32)part_sz,
                                   make_plan(40, 40 + window_bits), &in_out, &passes);
         if (rc)
             return rc;
@@ -1824,7 +1920,8 @@ WorkspaceSizes workspace_sizes(u64 cap)
     w.rank_tiles_cap = rank_tiles + 1;
     w.bytes = w.lookback_words * 8 + (w.rank_tiles_cap * 9 + RERANK_SLABS * 5) * sizeof(u32) + (MAX_PASSES + 2) * RADIX_BINS * 4 +
               MAX_PASSES * RADIX_BINS * 4 + TICKET_POOL * 4 + 16 * 4 + MSG_OFF_WORDS * 4;
-    w.bytes += 9 * 4096; // nine allocations, each rounded up by the runtime
+    w.bytes += CODE_TABLE_WORDS * sizeof(u32);
+    w.bytes += 10 * 4096; // ten allocations, each rounded up by the runtime
     return w;
 }
 
@@ -1892,6 +1989,8 @@ int create_handle(const char* who, u64 max_part_sz, int key_words, u32 kinds, cs
     h->rank_tiles_cap = ws.rank_tiles_cap;
     alloc((void**)&h->tile_tables, (h->rank_tiles_cap * 9 + RERANK_SLABS * 5) * sizeof(u32));
     alloc((void**)&h->ghist, (MAX_PASSES + 2) * RADIX_BINS * 4);
+    if (kinds & KIND_RESIDENT)
+        alloc((void**)&h->code_tables, CODE_TABLE_WORDS * sizeof(u32));
     alloc((void**)&h->digit_base, MAX_PASSES * RADIX_BINS * 4);
     alloc((void**)&h->tickets, TICKET_POOL * 4);
     alloc((void**)&h->counts, 16 * 4);
@@ -1972,6 +2071,7 @@ void csa_destroy(csa_handle* h)
     (void)hipFree(h->lookback);
     (void)hipFree(h->tile_tables);
     (void)hipFree(h->ghist);
+    (void)hipFree(h->code_tables);
     (void)hipFree(h->digit_base);
     (void)hipFree(h->tickets);
     (void)hipFree(h->counts);
@@ -2070,7 +2170,7 @@ int csa_radix_sort_pairs_dev(csa_handle* h, uint64_t* d_keys, uint32_t* d_vals, 
                     (unsigned long long)h->pool.bytes());
     int in_out = 0, passes = 0;
     const PassPlan plan = make_plan(begin_bit, end_bit);
-    int rc = radix_sort(L, SRC_PAIRS, nullptr, 0, 0, 0, d_keys, d_vals, tmp_keys, tmp_vals, (u32)n, plan, &in_out, &passes);
+    int rc = radix_sort(L, SRC_PAIRS, 0, 0, d_keys, d_vals, tmp_keys, tmp_vals, (u32)n, plan, &in_out, &passes);
     if (rc)
         return rc;
     if (in_out) {
@@ -2140,11 +2240,7 @@ int csa_radix_sort_pairs_static_dev(uint64_t* d_keys, uint32_t* d_vals, uint64_t
     const PassPlan plan = make_plan(begin_bit, end_bit);
     HistArgs ha;
     ha.keys = d_keys;
-    ha.vals = d_vals;
-    ha.text = nullptr;
     ha.n = (u32)n;
-    ha.text_n = 0;
-    ha.word = 0;
     ha.plan = plan;
     ha.ghist = ghist;
     hipLaunchKernelGGL(radix_hist_kernel, dim3(hist_blocks(256 * 16, n)), dim3(256), 0, s, ha);
@@ -2158,11 +2254,9 @@ int csa_radix_sort_pairs_static_dev(uint64_t* d_keys, uint32_t* d_vals, uint64_t
         a.vals_in = where == 0 ? d_vals : tmp_vals;
         a.keys_out = where == 0 ? tmp_keys : d_keys;
         a.vals_out = where == 0 ? tmp_vals : d_vals;
-        a.text = nullptr;
         a.n = (u32)n;
         a.text_n = 0;
         a.tail = 0;
-        a.word = 0;
         a.shift = plan.shift[p];
         a.bits = plan.bits[p];
         a.digit_base = digit_base + p * RADIX_BINS;

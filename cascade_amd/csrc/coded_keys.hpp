@@ -1,0 +1,400 @@
+// Generation 0 of a text over a large alphabet: the first sort on 32-bit codes instead of 64-bit K-gram keys.
+//
+// The code of a suffix is the place of its four symbols among all four-symbol strings, weighted by how often the symbols
+// occur: with cum[s] the share of symbols below s (as a 32-bit fraction) and w[s] = cum[s + 1] - cum[s],
+//   code(s0 s1 s2 s3) = cum[s0] + w[s0] (cum[s1] + w[s1] (cum[s2] + w[s2] cum[s3])),
+// an arithmetic code cut to 32 bits (every product is a 32 x 32 multiplication whose upper half is kept). A larger string never
+// has a smaller code, whatever the shares are, so they may come from a sample of the text; frequent symbols take wide
+// intervals, so that the codes spread evenly over the 32 bits where the raw symbols of a token text crowd into few values.
+// Four passes over 8-byte (code, suffix) pairs put the suffixes into the order of their codes, where K-gram keys take
+// eight passes over 12-byte pairs: 66 instead of 185 bytes moved per suffix (2^28 Zipf tokens: generation 0's passes 11.5 ->
+// 4.9 ms).
+//
+// What the sort leaves open are the suffixes that share a code: those whose strings are equal, and a few whose strings are not
+// (n / 2^32 of them by chance). resolve_runs_kernel reads the strings of such suffixes from the text (and of no others),
+// sorts every run of up to RESOLVE_MAX suffixes inside its tile and sets bit 31 of every suffix that ties with its left
+// neighbour, which is all the rank step needs to know. Longer runs are nearly always one string repeated (a string that is this
+// frequent has codes of its own) and in order as they stand; the rare ones that are not are collected and radix sorted by the
+// string itself.
+#pragma once
+
+#include "device_utils.hpp"
+#include "doubling.hpp"
+#include "radix_sort.hpp"
+
+namespace csa {
+
+// ---- shares of the symbols, from a sample ----
+
+constexpr int SYMBOLS = 1 << 16;
+constexpr int SAMPLE_BLOCK = 1024;
+constexpr u32 SAMPLE_CHUNK = 64;              // consecutive symbols, one wave's worth
+constexpr u32 SAMPLE_CHUNKS_PER_BLOCK = 256;  // 16384 symbols: a 16-bit counter holds them all
+constexpr u32 SAMPLE_CHUNKS_MAX = 1u << 14;   // 2^20 symbols are looked at, at most
+constexpr int SAMPLE_LOG2 = 20;
+
+// counts[s] += occurrences of symbol s in the sample: `taken` chunks spread evenly over the text (all of them when the text is short).
+__global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16* __restrict__ text, u32 n, u32 chunks, u32 taken,
+                                                                      u32* __restrict__ counts)
+{
+    __shared__ u32 s_cnt[SYMBOLS / 2]; // two 16-bit counters per word
+    const u32 t = threadIdx.x;
+    for (u32 i = t; i < (u32)SYMBOLS / 2; i += SAMPLE_BLOCK)
+        s_cnt[i] = 0;
+    __syncthreads();
+    const u32 first = blockIdx.x * SAMPLE_CHUNKS_PER_BLOCK;
+#pragma unroll 4
+    for (u32 r = t / SAMPLE_CHUNK; r < SAMPLE_CHUNKS_PER_BLOCK; r += SAMPLE_BLOCK / SAMPLE_CHUNK) {
+        const u32 c = first + r;
+        if (c < taken) {
+            const u64 p = (u64)c * chunks / taken * SAMPLE_CHUNK + (t & (SAMPLE_CHUNK - 1));
+            if (p < n) {
+                const u32 s = text[p];
+                atomicAdd(&s_cnt[s >> 1], (s & 1u) ? 0x10000u : 1u);
+            }
+        }
+    }
+    __syncthreads();
+    for (u32 i = t; i < (u32)SYMBOLS / 2; i += SAMPLE_BLOCK) {
+        const u32 v = s_cnt[i];
+        if (v & 0xFFFFu)
+            atomicAdd(&counts[2 * i], v & 0xFFFFu);
+        if (v >> 16)
+            atomicAdd(&counts[2 * i + 1], v >> 16);
+    }
+}
+
+// cum[s], s <= SYMBOLS: the share of symbols below s as a 32-bit fraction, every symbol counted once more than the sample
+// (scaled by 2^weight_log2) has it, so that one the sample missed has a place too.
+__global__ __launch_bounds__(1024) void symbol_shares_kernel(const u32* __restrict__ counts, int weight_log2, u32* __restrict__ cum)
+{
+    constexpr int PER = SYMBOLS / 1024;
+    __shared__ u32 s_w[16];
+    const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    u32 weight[PER], mine = 0;
+    const uint4* c4 = reinterpret_cast<const uint4*>(counts + t * PER);
+#pragma unroll
+    for (int k = 0; k < PER; k += 4) {
+        const uint4 v = c4[k / 4];
+        weight[k] = (v.x << weight_log2) + 1u;
+        weight[k + 1] = (v.y << weight_log2) + 1u;
+        weight[k + 2] = (v.z << weight_log2) + 1u;
+        weight[k + 3] = (v.w << weight_log2) + 1u;
+        mine += weight[k] + weight[k + 1] + weight[k + 2] + weight[k + 3];
+    }
+    const u32 incl = wave_incl_sum(mine);
+    if (lane == 63u)
+        s_w[w] = incl;
+    __syncthreads();
+    u32 before = incl - mine, total = 0;
+    for (u32 ww = 0; ww < 16; ++ww) {
+        if (ww < w)
+            before += s_w[ww];
+        total += s_w[ww];
+    }
+    const u64 scale = (1ull << 53) / total; // before <= total: before * scale <= 2^53
+    uint4* o4 = reinterpret_cast<uint4*>(cum + t * PER);
+#pragma unroll
+    for (int k = 0; k < PER; k += 4) {
+        u32 v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            v[q] = (u32)((u64)before * scale >> 21); // (below 2^32: every symbol's weight is at least 1)
+            before += weight[k + q];
+        }
+        o4[k / 4] = make_uint4(v[0], v[1], v[2], v[3]);
+    }
+    if (t == 1023u)
+        cum[SYMBOLS] = 0xFFFFFFFFu;
+}
+
+// ---- the codes of all suffixes, and the digit counts of the four passes ----
+
+constexpr int CODE_BLOCK = 256;
+constexpr int CODE_ITEMS = 8;
+constexpr int CODE_PASSES = 4;
+constexpr int CODE_COPIES = 8;
+
+// codes[v] = code of the suffix at virtual position v (virtual_to_suffix with `tail` = min(n, 4)). Bounded by the lookups
+// of cum[]: one 8-byte gather per symbol (the table is 256 KB: it lives in the L2s), shared by the four suffixes it appears in.
+__global__ __launch_bounds__(CODE_BLOCK) void code_suffixes_kernel(const u16* __restrict__ text, u32 n, u32 tail, const u32* __restrict__ cum,
+                                                                   u32* __restrict__ codes, u32* __restrict__ ghist)
+{
+    constexpr u32 TILE = CODE_BLOCK * CODE_ITEMS;
+    __shared__ u64 s_text[(TILE + 3 + 6) / 4 + 2];
+    __shared__ u32 s_hist[CODE_PASSES * RADIX_BINS * CODE_COPIES];
+    const u32 t = threadIdx.x;
+    for (u32 i = t; i < CODE_PASSES * RADIX_BINS * CODE_COPIES; i += CODE_BLOCK)
+        s_hist[i] = 0;
+    const u32 copy = t & (CODE_COPIES - 1);
+    const u64 tiles = ((u64)n + TILE - 1) / TILE;
+    for (u64 tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const u64 p0 = tile * TILE;
+        __syncthreads(); // the counters are cleared; the stretch of the round before has been read
+        const u32 sym_off = stage_text(text, n, p0, TILE + 3u, s_text, t, CODE_BLOCK);
+        __syncthreads();
+        const u16* s16 = reinterpret_cast<const u16*>(s_text) + sym_off + t * CODE_ITEMS;
+        u32 lo[CODE_ITEMS + 3], width[CODE_ITEMS + 3];
+#pragma unroll
+        for (int k = 0; k < CODE_ITEMS + 3; ++k) {
+            const u32 s = s16[k];
+            u32 pair[2];
+            __builtin_memcpy(pair, cum + s, 8); // entries s and s + 1 (4-byte aligned)
+            lo[k] = pair[0];
+            width[k] = pair[1] - pair[0];
+        }
+        u32 code[CODE_ITEMS];
+#pragma unroll
+        for (int k = 0; k < CODE_ITEMS; ++k) {
+            u32 f = lo[k + 3];
+#pragma unroll
+            for (int q = 2; q >= 0; --q)
+                f = lo[k + q] + (u32)(((u64)width[k + q] * f) >> 32);
+            code[k] = f;
+        }
+        const u64 x0 = p0 + (u64)t * CODE_ITEMS;
+        if (tail == 4 && x0 + CODE_ITEMS + tail <= n) { // no suffix of the text's end among them: places x0 + 4 on, 16-byte aligned
+            uint4* out = reinterpret_cast<uint4*>(codes + x0 + 4);
+#pragma unroll
+            for (int k = 0; k < CODE_ITEMS; k += 4)
+                out[k / 4] = make_uint4(code[k], code[k + 1], code[k + 2], code[k + 3]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < CODE_ITEMS; ++k) {
+                const u64 x = x0 + k;
+                if (x < n)
+                    codes[x + tail >= n ? n - 1 - x : x + tail] = code[k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < CODE_ITEMS; ++k)
+            if (x0 + k < n) {
+#pragma unroll
+                for (int p = 0; p < CODE_PASSES; ++p)
+                    atomicAdd(&s_hist[(p * RADIX_BINS + ((code[k] >> (8 * p)) & 0xFFu)) * CODE_COPIES + copy], 1u);
+            }
+    }
+    __syncthreads();
+    for (u32 i = t; i < CODE_PASSES * RADIX_BINS; i += CODE_BLOCK) {
+        u32 v = 0;
+#pragma unroll
+        for (int c = 0; c < CODE_COPIES; ++c)
+            v += s_hist[i * CODE_COPIES + c];
+        if (v)
+            atomicAdd(&ghist[i], v);
+    }
+}
+
+// ---- runs of equal codes ----
+
+constexpr int RESOLVE_BLOCK = 512;
+constexpr int RESOLVE_ITEMS = 4;
+constexpr int RESOLVE_TILE = RESOLVE_BLOCK * RESOLVE_ITEMS;
+#ifndef CSA_RESOLVE_MAX
+#define CSA_RESOLVE_MAX 256
+#endif
+constexpr int RESOLVE_MAX = CSA_RESOLVE_MAX; // longest run that is sorted inside its tile
+static_assert(RESOLVE_MAX % 64 == 0 && RESOLVE_MAX <= RESOLVE_BLOCK, "the halo is read in whole waves, one element per thread");
+constexpr u32 RESOLVE_MARK_BITS = 20;
+constexpr u32 RESOLVE_MARK_WORDS = 1u << (RESOLVE_MARK_BITS - 5);
+
+// The mark of a code: codes that share one only cost time (their runs are sorted again although they are in order).
+__device__ __forceinline__ u32 resolve_mark(u32 code) { return (code * 0x9E3779B1u) >> (32 - RESOLVE_MARK_BITS); }
+
+struct ResolveArgs {
+    const u32* codes; // sorted
+    const u32* sufs;
+    const u16* text;
+    u32 n;
+    u32 ell; // symbols of a string; a suffix that runs off the text inside them ties with nobody
+    u32* sufs_out; // the list in order, TIED_LEFT where a suffix's string is its left neighbour's
+    u32* marks;    // [RESOLVE_MARK_WORDS], zeroed: codes of long runs that are not in order
+    u32* unordered; // zeroed: set if there are any
+    // the collected members of marked runs (collect_marked_kernel, place_marked_kernel)
+    u64* keys;
+    u32* members;
+    u32* places;
+    u32* tile_agg;
+    u32* tile_splits;
+    const u32* tile_prefix;
+    const u32* slab_total;
+    u32 slab;
+};
+
+__global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs a)
+{
+    constexpr int H = RESOLVE_MAX, SPAN = RESOLVE_TILE + 2 * H;
+    __shared__ u64 s_head[SPAN / 64]; // bit j: the element at span place j starts a run (places outside the list count as starts)
+    __shared__ u64 s_key[SPAN];
+    __shared__ u32 s_suf[SPAN];
+    const u32 t = threadIdx.x;
+    const long long t0 = (long long)blockIdx.x * RESOLVE_TILE, lo = t0 - H, n = a.n;
+    // whole waves take consecutive places: one ballot per wave and round gives 64 bits of s_head
+    for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (the same rounds for every lane of a wave: SPAN is a multiple of 64)
+        const long long e = lo + j;
+        const bool head = e <= 0 || e >= n || a.codes[e] != a.codes[e - 1];
+        const u64 b = __ballot(head);
+        if ((t & 63u) == 0)
+            s_head[j / 64] = b;
+    }
+    __syncthreads();
+    // the run around place j: first place and first place behind it; false if it has more than H members
+    auto run_of = [&](int j, int& first, int& last) -> bool {
+        int wd = j / 64;
+        u64 b = s_head[wd] & (~0ull >> (63 - (j & 63))); // starts at or before j
+        while (b == 0 && wd > 0 && wd * 64 > j - H)
+            b = s_head[--wd];
+        first = b ? wd * 64 + 63 - __builtin_clzll(b) : -1;
+        if (first < 0 || j - first > H)
+            return false;
+        wd = j / 64;
+        b = (j & 63) == 63 ? 0ull : s_head[wd] & (~0ull << ((j & 63) + 1)); // starts behind j
+        while (b == 0 && wd + 1 < SPAN / 64 && (wd + 1) * 64 <= j + H)
+            b = s_head[++wd];
+        last = b ? wd * 64 + __builtin_ctzll(b) : SPAN + H;
+        return last - first <= H;
+    };
+    // own elements: suffix, run, and the string where there is company
+    u32 x[RESOLVE_ITEMS];
+    int first[RESOLVE_ITEMS], last[RESOLVE_ITEMS]; // last = 0: a long run; last - first = 1: alone
+#pragma unroll
+    for (int k = 0; k < RESOLVE_ITEMS; ++k) {
+        const int j = H + k * RESOLVE_BLOCK + (int)t;
+        const long long e = lo + j;
+        x[k] = 0;
+        first[k] = j;
+        last[k] = j + 1;
+        if (e < n) {
+            x[k] = a.sufs[e];
+            if (!run_of(j, first[k], last[k])) {
+                first[k] = j;
+                last[k] = 0;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < RESOLVE_ITEMS; ++k) {
+        const int j = H + k * RESOLVE_BLOCK + (int)t;
+        if (last[k] - first[k] != 1) {
+            s_key[j] = load_kgram(a.text, a.n, x[k], 0);
+            s_suf[j] = x[k];
+        }
+    }
+    // of the halo: the members of short runs that reach into the tile, and the left neighbour of the tile's first element
+    {
+        int f0, l0, f1, l1;
+        const int j_last = (int)((t0 + RESOLVE_TILE < n ? t0 + RESOLVE_TILE : n) - 1 - lo);
+        const bool short0 = run_of(H, f0, l0), short1 = run_of(j_last, f1, l1);
+        for (int i = t; i < 2 * H; i += RESOLVE_BLOCK) {
+            const int j = i < H ? i : RESOLVE_TILE + i;
+            const long long e = lo + j;
+            const bool wanted = i < H ? (short0 ? j >= f0 : j == H - 1) : (short1 && j < l1);
+            if (wanted && e >= 0 && e < n) {
+                s_suf[j] = a.sufs[e];
+                s_key[j] = load_kgram(a.text, a.n, s_suf[j], 0);
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RESOLVE_ITEMS; ++k) {
+        const int j = H + k * RESOLVE_BLOCK + (int)t;
+        const long long e = lo + j;
+        if (e >= n)
+            continue;
+        const bool whole = (u64)x[k] + a.ell < a.n;
+        int place = j;
+        bool tied = false;
+        if (last[k] == 0) {
+            if (!((s_head[j / 64] >> (j & 63)) & 1ull)) {
+                const u64 mine = s_key[j], before = s_key[j - 1];
+                tied = mine == before && whole && (u64)s_suf[j - 1] + a.ell < a.n;
+                if (mine < before) {
+                    const u32 mark = resolve_mark(a.codes[e]), bit = 1u << (mark & 31u);
+                    if (!(a.marks[mark >> 5] & bit)) // (soon set for all to see: few of a run's members get to the atomic)
+                        atomicOr(&a.marks[mark >> 5], bit);
+                    *a.unordered = 1u;
+                }
+            }
+        } else if (last[k] - first[k] > 1) {
+            const u64 mine = s_key[j];
+            place = first[k];
+            for (int i = first[k]; i < last[k]; ++i) {
+                const u64 v = s_key[i];
+                if (v < mine || (v == mine && i < j))
+                    ++place;
+                if (v == mine && i < j && whole && (u64)s_suf[i] + a.ell < a.n)
+                    tied = true; // (the suffixes that run off the text come first among equal strings)
+            }
+        }
+        a.sufs_out[lo + place] = x[k] | (tied ? TIED_LEFT : 0u);
+    }
+}
+
+// Members of marked runs, in list order: APPLY = false counts them per tile, APPLY = true (after rerank_scan_kernel) writes
+// their strings, suffixes and list places. A run is marked as a whole, so the list of them sorted by string, which
+// is also the order of the codes, goes back to the same places.
+constexpr int COLLECT_BLOCK = 256;
+constexpr int COLLECT_ITEMS = 4;
+constexpr int COLLECT_TILE = COLLECT_BLOCK * COLLECT_ITEMS;
+
+template <bool APPLY>
+__global__ __launch_bounds__(COLLECT_BLOCK) void collect_marked_kernel(ResolveArgs a)
+{
+    __shared__ u32 s_w[COLLECT_BLOCK / WAVE];
+    const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    const u32 tile = blockIdx.x;
+    const u64 base = (u64)tile * COLLECT_TILE + (u64)t * COLLECT_ITEMS;
+    u32 flags = 0, mine = 0;
+#pragma unroll
+    for (int k = 0; k < COLLECT_ITEMS; ++k)
+        if (base + k < a.n) {
+            const u32 mark = resolve_mark(a.codes[base + k]);
+            const u32 in = (a.marks[mark >> 5] >> (mark & 31u)) & 1u;
+            flags |= in << k;
+            mine += in;
+        }
+    const u32 incl = wave_incl_sum(mine);
+    if (lane == 63u)
+        s_w[w] = incl;
+    __syncthreads();
+    u32 slot = incl - mine, total = 0;
+    for (u32 ww = 0; ww < COLLECT_BLOCK / WAVE; ++ww) {
+        if (ww < w)
+            slot += s_w[ww];
+        total += s_w[ww];
+    }
+    if (!APPLY) {
+        if (t == 0) {
+            a.tile_agg[(u64)tile * 4 + 0] = 0;
+            a.tile_agg[(u64)tile * 4 + 1] = 0;
+            a.tile_agg[(u64)tile * 4 + 2] = total;
+            a.tile_agg[(u64)tile * 4 + 3] = 0;
+            a.tile_splits[tile] = 0;
+        }
+        return;
+    }
+    slot += a.tile_prefix[(u64)tile * 4 + 2] + slabs_before(a.slab_total, tile / a.slab).sum2;
+#pragma unroll
+    for (int k = 0; k < COLLECT_ITEMS; ++k)
+        if ((flags >> k) & 1u) {
+            const u32 x = a.sufs_out[base + k] & ~TIED_LEFT;
+            a.keys[slot] = load_kgram(a.text, a.n, x, 0);
+            a.members[slot] = x;
+            a.places[slot] = (u32)(base + k);
+            ++slot;
+        }
+}
+
+// The collected members, sorted by string, back to their places.
+__global__ __launch_bounds__(256) void place_marked_kernel(ResolveArgs a, u32 count)
+{
+    const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count)
+        return;
+    const u32 x = a.members[i];
+    const bool tied = i > 0 && a.keys[i] == a.keys[i - 1] && (u64)x + a.ell < a.n && (u64)a.members[i - 1] + a.ell < a.n;
+    a.sufs_out[a.places[i]] = x | (tied ? TIED_LEFT : 0u);
+}
+
+} // namespace csa

@@ -21,6 +21,8 @@ namespace csa {
 // ---------------------------------------------------------------------------------------------
 
 constexpr u32 NO_RANK = 0xFFFFFFFFu; // ranks are below 2^31
+// Bit 31 of a suffix in a list whose ties have been resolved already (coded_keys.hpp): its key is that of the suffix before it.
+constexpr u32 TIED_LEFT = 0x80000000u; // suffixes are below 2^31
 
 // The tiles of a rank step are scanned in RERANK_SLABS slabs (rerank_scan_kernel): a tile's prefix is its prefix inside
 // its slab combined with the totals (max, max, sum, sum, -) of the slabs before. One slab per lane: a wave fetches the
@@ -57,10 +59,9 @@ __device__ __forceinline__ SlabPrefix slabs_before(const u32* __restrict__ slab_
 constexpr u32 MAX_LEVELS = 4, LEVEL_SLOTS = 64;
 
 struct RerankArgs {
-    const u64* keys;
+    const u64* keys; // unused where the list carries its ties (TIED)
     const u32* sufs;
     u32 m;         // = n: generation 0 ranks every suffix
-    int key_words; // 1..4 (the words after the first are re-read from the text where the first words tie)
     u32 n;         // partition size
     u32 ell;       // symbols in the generation-0 key
     // Packed keys of many symbols (packed_text.hpp): the counting pass also counts what the list would leave at shorter
@@ -71,8 +72,7 @@ struct RerankArgs {
     u32 level_drop[4];
     u32 level_ell[4];
     unsigned long long* level_totals;
-    const u16* text;
-    u32* rank;     // [n] by text position
+    u32* rank; // [n] by text position
     // Deferred rank update: instead of the scattered write rank[x] = r, the suffix at sorted index c leaves the record
     // (x << 32) | r at rank_recs[c] (a coalesced stream). The records then go through radix passes on the high bits of
     // x before they are written to rank[], so that those writes fall into one window of rank[] at a time.
@@ -97,19 +97,23 @@ struct RerankArgs {
 
 // Elements base - 1 .. base + ITEMS of the sorted (key, suffix) list, m elements long, for the thread that owns
 // elements base .. base + ITEMS - 1 (base a multiple of ITEMS): its own in whole 16-byte loads where they all exist,
-// zeros outside the list.
-template <int ITEMS>
+// zeros outside the list. KEYS = false: the suffixes alone (the keys are left as they are).
+template <int ITEMS, bool KEYS>
 __device__ __forceinline__ void load_with_neighbours(const u64* __restrict__ keys, const u32* __restrict__ sufs, u64 base, u32 m,
                                                      u64 (&key)[ITEMS + 2], u32 (&suf)[ITEMS + 2])
 {
     if (ITEMS % 4 == 0 && base + ITEMS <= m) {
-        const uint4* k4 = reinterpret_cast<const uint4*>(keys + base);
         const uint4* s4 = reinterpret_cast<const uint4*>(sufs + base);
+        if constexpr (KEYS) {
+            const uint4* k4 = reinterpret_cast<const uint4*>(keys + base);
 #pragma unroll
-        for (int k = 0; k < ITEMS; k += 2) {
-            const uint4 v = k4[k / 2];
-            key[k + 1] = (u64)v.x | ((u64)v.y << 32);
-            key[k + 2] = (u64)v.z | ((u64)v.w << 32);
+            for (int k = 0; k < ITEMS; k += 2) {
+                const uint4 v = k4[k / 2];
+                key[k + 1] = (u64)v.x | ((u64)v.y << 32);
+                key[k + 2] = (u64)v.z | ((u64)v.w << 32);
+            }
+            key[0] = base >= 1 ? keys[base - 1] : 0;
+            key[ITEMS + 1] = base + ITEMS < m ? keys[base + ITEMS] : 0;
         }
 #pragma unroll
         for (int k = 0; k < ITEMS; k += 4) {
@@ -119,26 +123,36 @@ __device__ __forceinline__ void load_with_neighbours(const u64* __restrict__ key
             suf[k + 3] = v.z;
             suf[k + 4] = v.w;
         }
-        key[0] = base >= 1 ? keys[base - 1] : 0;
         suf[0] = base >= 1 ? sufs[base - 1] : 0;
-        const bool last_in = base + ITEMS < m;
-        key[ITEMS + 1] = last_in ? keys[base + ITEMS] : 0;
-        suf[ITEMS + 1] = last_in ? sufs[base + ITEMS] : 0;
+        suf[ITEMS + 1] = base + ITEMS < m ? sufs[base + ITEMS] : 0;
     } else {
 #pragma unroll
         for (int k = 0; k < ITEMS + 2; ++k) {
             const u64 c = base + k; // element c - 1
             const bool in = c >= 1 && c - 1 < m;
-            key[k] = in ? keys[c - 1] : 0;
+            if constexpr (KEYS)
+                key[k] = in ? keys[c - 1] : 0;
             suf[k] = in ? sufs[c - 1] : 0;
         }
     }
 }
 
+// Whether sorted element c (key_c, suf_c) belongs to the run of element c - 1 (key_b, suf_b); both exist. TIED: the
+// list says so itself, and carries no keys.
+template <bool TIED>
+__device__ __forceinline__ bool same_run(const RerankArgs& a, u64 key_b, u32 suf_b, u64 key_c, u32 suf_c)
+{
+    if constexpr (TIED)
+        return (suf_c & TIED_LEFT) != 0;
+    // a suffix that runs off the text inside its key ties with nobody (include/bit-layout.hpp:99-100)
+    return key_b == key_c && (u64)suf_b + a.ell < a.n && (u64)suf_c + a.ell < a.n;
+}
+
 // The counting pass of generation 0 on its own: the per-tile aggregates need no ordering inside the tile, so every
 // thread reads its ITEMS elements and their two neighbours straight from the arrays (no exchange through LDS, one
 // barrier) and the tile reduces instead of scanning. Same run and tail rules as rerank_kernel below.
-template <int BLOCK, int ITEMS>
+// TIED: the list carries its ties (RerankArgs::sufs with TIED_LEFT) instead of keys: 4 bytes read per suffix, not 12.
+template <int BLOCK, int ITEMS, bool TIED>
 __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
 {
     constexpr int TILE = BLOCK * ITEMS;
@@ -150,20 +164,15 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
     const u32 tile = blockIdx.x;
     const u64 base = (u64)tile * TILE + (u64)t * ITEMS;
     const u32 m = a.m;
-    u64 key[ITEMS + 2]; // elements base - 1 .. base + ITEMS
+    u64 key[ITEMS + 2] = {}; // elements base - 1 .. base + ITEMS
     u32 suf[ITEMS + 2];
-    load_with_neighbours<ITEMS>(a.keys, a.sufs, base, m, key, suf);
+    load_with_neighbours<ITEMS, !TIED>(a.keys, a.sufs, base, m, key, suf);
     u32 la = 0, lcnt = 0, lheads = 0;
     bool prev_eq = false;
 #pragma unroll
     for (int k = 0; k < ITEMS + 1; ++k) {
         const u64 c = base + k; // right element of the pair (c - 1, c)
-        bool e = c >= 1 && c < m && key[k] == key[k + 1];
-        for (int word = 1; e && word < a.key_words; ++word)
-            e = load_kgram(a.text, a.n, suf[k], (u32)word) == load_kgram(a.text, a.n, suf[k + 1], (u32)word);
-        // a suffix that runs off the text inside its key ties with nobody (include/bit-layout.hpp:99-100)
-        if (e && ((u64)suf[k] + a.ell >= a.n || (u64)suf[k + 1] + a.ell >= a.n))
-            e = false;
+        const bool e = c >= 1 && c < m && same_run<TIED>(a, key[k], suf[k], key[k + 1], suf[k + 1]);
         if (k >= 1 && c - 1 < m) { // element c - 1 = base + k - 1: prev_eq ties it to its left, e to its right
             const bool ka = !prev_eq;
             const bool single = ka && !e;
@@ -176,7 +185,7 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
     }
     // the same counts at the shorter contexts of packed keys (one-word keys: nothing is read from the text)
     __shared__ u32 s_level[WAVES][MAX_LEVELS];
-    for (u32 i = 0; i < a.levels; ++i) {
+    for (u32 i = 0; !TIED && i < a.levels; ++i) {
         const u32 drop = a.level_drop[i];
         const u64 lell = a.level_ell[i];
         u32 cs = 0, ch = 0;
@@ -241,7 +250,7 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
 // The applying pass: reads the tile's exclusive prefix from tile_prefix (rerank_count_kernel and rerank_scan_kernel
 // before it) and does the work. What the tile produces is collected in LDS and leaves in striped order (consecutive
 // lanes, consecutive elements).
-template <int BLOCK, int ITEMS>
+template <int BLOCK, int ITEMS, bool TIED>
 __global__ __launch_bounds__(BLOCK) void rerank_kernel(RerankArgs a)
 {
     constexpr int TILE = BLOCK * ITEMS;
@@ -262,20 +271,15 @@ __global__ __launch_bounds__(BLOCK) void rerank_kernel(RerankArgs a)
 
     // every thread reads its ITEMS elements (whole 16-byte loads where the tile is full) and their two neighbours
     // straight from the arrays: elements base - 1 .. base + ITEMS
-    u64 key[ITEMS + 2];
+    u64 key[ITEMS + 2] = {};
     u32 suf[ITEMS + 2];
-    load_with_neighbours<ITEMS>(a.keys, a.sufs, base, m, key, suf);
+    load_with_neighbours<ITEMS, !TIED>(a.keys, a.sufs, base, m, key, suf);
     // eq[k]: elements (base+k-1) and (base+k) exist and belong to one run of equal keys
     bool eq[ITEMS + 1];
 #pragma unroll
     for (int k = 0; k < ITEMS + 1; ++k) {
         const u64 c = base + k; // right element of the pair
-        bool e = c >= 1 && c < m && key[k] == key[k + 1];
-        for (int word = 1; e && word < a.key_words; ++word)
-            e = load_kgram(a.text, a.n, suf[k], (u32)word) == load_kgram(a.text, a.n, suf[k + 1], (u32)word);
-        // a suffix that runs off the text inside its key ties with nobody (include/bit-layout.hpp:99-100)
-        if (e && ((u64)suf[k] + a.ell >= a.n || (u64)suf[k + 1] + a.ell >= a.n))
-            e = false;
+        const bool e = c >= 1 && c < m && same_run<TIED>(a, key[k], suf[k], key[k + 1], suf[k + 1]);
         eq[k] = e;
     }
 
@@ -337,7 +341,7 @@ __global__ __launch_bounds__(BLOCK) void rerank_kernel(RerankArgs a)
             const bool single = ka && !eq[k + 1];
             if (ka)
                 ra = (u32)c + 1u;
-            const u32 x = suf[k + 1];
+            const u32 x = TIED ? suf[k + 1] & ~TIED_LEFT : suf[k + 1];
             const u32 nr = ra - 1u; // element 0 is always a head, so ra >= 1 here
             if (ra == 0 || nr >= a.n || x >= a.n) { // a corrupt sorted list: report it instead of writing out of bounds
                 atomicExch(a.err, DEV_ERR_RERANK_RANGE);

@@ -27,7 +27,7 @@ struct PassPlan {
 // How a pass obtains its input pairs.
 enum : int {
     SRC_PAIRS = 0, // keys_in[i], vals_in[i]
-    SRC_TEXT = 1,  // generation 0, first pass: the pair of virtual position i is built from the text
+    SRC_CODED = 1, // generation 0, first pass: keys_in holds the codes of virtual positions (coded_keys.hpp), the suffixes follow from them
     SRC_RANKS = 2, // a dense later generation, first pass: pair i = ((rank[i], rank[i + hop]), i), built from rank[]
     SRC_PACKED = 3 // generation 0 over a small alphabet, first pass: the key of virtual position i is cut from the code stream
 };
@@ -56,11 +56,7 @@ __device__ __forceinline__ u32 virtual_to_suffix(u32 i, u32 n, u32 tail)
 
 struct HistArgs {
     const u64* keys;
-    const u32* vals;
-    const u16* text;
-    u32 n;      // pairs
-    u32 text_n; // symbols in the text
-    u32 word;   // key word to build from the text
+    u32 n; // pairs
     PassPlan plan;
     u32* ghist; // [MAX_PASSES][256], zeroed by the caller
     const u32* rank = nullptr; // non-null: the keys are rank_pair_key(rank, n, hop, i, radix) instead of keys[i]
@@ -187,7 +183,7 @@ __global__ __launch_bounds__(256) void rank_hist_combine_kernel(u32* ghist, int 
 }
 
 // Histogram of the low and of the high byte of every symbol of the text: bytehist[0][d], bytehist[1][d].
-// The eight digit histograms of a K-gram key word follow from these two (text_hist_expand_kernel).
+// They tell whether the alphabet is small enough for keys of packed symbols.
 constexpr int TEXT_HIST_COPIES = 16;
 
 __global__ __launch_bounds__(256) void text_byte_hist_kernel(const u16* __restrict__ text, u32 n, u32* bytehist)
@@ -230,29 +226,6 @@ __global__ __launch_bounds__(256) void text_byte_hist_kernel(const u16* __restri
     }
 }
 
-// ghist[p][d] for the 8 byte-wide passes of key word `word` over all n suffixes. Pass p looks at byte (p & 1) of
-// the symbol at offset pos = 4 * word + 3 - p / 2 of each suffix, i.e. at T[pos .. n) followed by min(pos, n) padding
-// zeros: the whole-text byte histogram minus the first min(pos, n) symbols, plus that many zeros.
-__global__ __launch_bounds__(256) void text_hist_expand_kernel(const u16* __restrict__ text, u32 n, u32 word,
-                                                               const u32* __restrict__ bytehist, u32* ghist)
-{
-    const u32 d = threadIdx.x;
-    for (int p = 0; p < 8; ++p) {
-        const u32 byte = p & 1;
-        const u32 pos = 4 * word + 3 - p / 2;
-        const u32 cut = pos < n ? pos : n;
-        u32 v = bytehist[byte * RADIX_BINS + d];
-        for (u32 i = 0; i < cut; ++i) {
-            const u32 b = byte ? (text[i] >> 8) : (text[i] & 0xFFu);
-            if (b == d)
-                --v;
-        }
-        if (d == 0)
-            v += cut;
-        ghist[p * RADIX_BINS + d] = v;
-    }
-}
-
 // digit_base[p][d] = number of pairs whose pass-p digit is < d.
 __global__ __launch_bounds__(256) void radix_scan_hist_kernel(const u32* ghist, u32* digit_base, int num_passes)
 {
@@ -277,11 +250,9 @@ struct OnesweepArgs {
     const u32* vals_in;  // unused by the instantiations without values, like vals_out
     void* keys_out;
     u32* vals_out;
-    const u16* text;
     u32 n;      // pairs
-    u32 text_n; // symbols in the text (SRC_TEXT)
-    u32 tail;   // suffixes that run off the text inside their key (SRC_TEXT)
-    u32 word;   // key word to build (SRC_TEXT)
+    u32 text_n; // symbols in the text (SRC_CODED, SRC_PACKED)
+    u32 tail;   // suffixes that run off the text inside their key (SRC_CODED, SRC_PACKED)
     int shift;
     int bits;
     const u32* digit_base; // [256] for this pass
@@ -358,7 +329,8 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
     constexpr int TILE = BLOCK * ITEMS;
     constexpr int WAVES = BLOCK / WAVE;
     static_assert(BLOCK >= RADIX_BINS, "one thread per digit is assumed");
-    static_assert(sizeof(KeyT) == 8 || (SRC == SRC_PAIRS && HI == 0), "narrow keys are plain pairs");
+    static_assert(sizeof(KeyT) == 8 || ((SRC == SRC_PAIRS || SRC == SRC_CODED) && HI == 0), "narrow keys are read from an array");
+    constexpr bool KEYS_IN = SRC == SRC_PAIRS || SRC == SRC_CODED;
     auto rank_key = [&](u32 i) -> u64 { return rank_pair_key(a.rank, a.n, a.hop, i, a.radix); }; // SRC_RANKS: pair i is text position i
     const KeyT* __restrict__ keys_in = static_cast<const KeyT*>(a.keys_in);
     KeyT* __restrict__ keys_out = static_cast<KeyT*>(a.keys_out);
@@ -395,20 +367,10 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
 #define CSA_LDS_ORDER() __builtin_amdgcn_wave_barrier() /* CPU emulation: lanes are threads, order them for real */
 #define CSA_OPAQUE(x) ((void)0)
 #endif
-    // ---- first pass of generation 0: stage the tile's stretch of the text in LDS ----
+    // ---- first pass of generation 0 over a small alphabet ----
     // The tile covers consecutive virtual positions, i.e. (after the few tail suffixes of tile 0) consecutive text
-    // positions j0, j0 + 1, ...; the (still unused) reorder buffer holds the stretch, and each key is assembled
-    // from three LDS words instead of four narrow global loads.
-    u32 j0 = 0, sym_off = 0;
-    if constexpr (SRC == SRC_TEXT) {
-        const u32 first_virtual = (u32)base > a.tail ? (u32)base : a.tail;
-        j0 = first_virtual - a.tail;
-        const u32 count = (u32)TILE - (first_virtual - (u32)base) + 3u; // the last key reaches 3 symbols further
-        static_assert(sizeof(KeyT) * TILE >= 8 * ((TILE + 3 + 6) / 4 + 2), "the staged text must fit the reorder buffer");
-        sym_off = stage_text(a.text, a.text_n, (u64)j0 + 4ull * a.word, count, reinterpret_cast<u64*>(s_keys), t, BLOCK);
-        __syncthreads();
-    }
-    // the same over a small alphabet: the tile's stretch of the code stream (TILE * sym_bits bits and a key's worth more)
+    // positions; the (still unused) reorder buffer holds their stretch of the code stream (TILE * sym_bits bits and a key's
+    // worth more), and each key is cut from it.
     u64 stream_bit0 = 0;
     if constexpr (SRC == SRC_PACKED) {
         const u32 first_virtual = (u32)base > a.tail ? (u32)base : a.tail;
@@ -421,15 +383,10 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
             s_codes[i] = first_word + i < a.stream_words ? a.stream[first_word + i] : 0u;
         __syncthreads();
     }
-    auto text_key = [&](u32 i) -> u64 { // key of virtual position i of this tile (SRC_TEXT, SRC_PACKED)
-        if constexpr (SRC == SRC_PACKED) {
-            if (i < a.tail)
-                return packed_window(a.stream, (u64)(a.text_n - 1u - i) * a.sym_bits, a.key_bits);
-            return packed_window(reinterpret_cast<const u32*>(s_keys), (u64)(i - a.tail) * a.sym_bits - stream_bit0, a.key_bits);
-        }
+    auto text_key = [&](u32 i) -> u64 { // key of virtual position i of this tile (SRC_PACKED)
         if (i < a.tail)
-            return load_kgram(a.text, a.text_n, a.text_n - 1u - i, a.word);
-        return staged_kgram(reinterpret_cast<const u32*>(s_keys), (i - a.tail) - j0 + sym_off);
+            return packed_window(a.stream, (u64)(a.text_n - 1u - i) * a.sym_bits, a.key_bits);
+        return packed_window(reinterpret_cast<const u32*>(s_keys), (u64)(i - a.tail) * a.sym_bits - stream_bit0, a.key_bits);
     };
 
     // ---- load: wave-striped, so that consecutive lanes read consecutive pairs ----
@@ -441,7 +398,7 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k) {
             const u64 i = base + first_local + k * WAVE;
-            if (SRC == SRC_PAIRS)
+            if (KEYS_IN)
                 key[k] = keys_in[i];
             else if (SRC == SRC_RANKS)
                 key[k] = (KeyT)rank_key((u32)i);
@@ -455,7 +412,7 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
             const u64 i = base + local;
             key[k] = ~(KeyT)0; // padding: largest digit, and behind every real pair of the tile
             if (local < valid) {
-                if (SRC == SRC_PAIRS)
+                if (KEYS_IN)
                     key[k] = keys_in[i];
                 else if (SRC == SRC_RANKS)
                     key[k] = (KeyT)rank_key((u32)i);
@@ -548,7 +505,7 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
         const u32 local = first_local + k * WAVE;
         val[k] = 0;
         if (VALS && local < valid)
-            val[k] = (SRC == SRC_TEXT || SRC == SRC_PACKED) ? virtual_to_suffix((u32)(base + local), a.text_n, a.tail)
+            val[k] = (SRC == SRC_CODED || SRC == SRC_PACKED) ? virtual_to_suffix((u32)(base + local), a.text_n, a.tail)
                      : SRC == SRC_RANKS                     ? (u32)(base + local)
                                                             : a.vals_in[base + local];
     }

@@ -249,12 +249,12 @@ int step_init(Launch& L, const char* who, StepColumns& c, const StepPlan& pl, in
         // (64-bit key, permutation) pairs
         hipLaunchKernelGGL(iota_kernel, dim3(blocks), dim3(256), 0, s, P[pc], m);
         hipLaunchKernelGGL(carried_tag_keys_kernel, dim3(blocks), dim3(256), 0, s, (const uint4*)carried, m, K[kc]);
-        rc = radix_sort(L, SRC_PAIRS, nullptr, 0, 0, 0, K[kc], P[pc], K[kc ^ 1], P[pc ^ 1], (u32)m, make_plan(0, 16), &in_out, &passes);
+        rc = radix_sort(L, SRC_PAIRS, 0, 0, K[kc], P[pc], K[kc ^ 1], P[pc ^ 1], (u32)m, make_plan(0, 16), &in_out, &passes);
         if (rc)
             return rc;
         pc ^= in_out;
         hipLaunchKernelGGL(gather_u64_kernel, dim3(blocks), dim3(256), 0, s, c.keys, (const u32*)P[pc], m, 1u, 0u, K[0]);
-        rc = radix_sort(L, SRC_PAIRS, nullptr, 0, 0, 0, K[0], P[pc], K[1], P[pc ^ 1], (u32)m, make_plan(0, 64), &in_out, &passes);
+        rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], P[pc], K[1], P[pc ^ 1], (u32)m, make_plan(0, 64), &in_out, &passes);
         if (rc)
             return rc;
         kc = in_out;
@@ -270,7 +270,7 @@ int step_init(Launch& L, const char* who, StepColumns& c, const StepPlan& pl, in
         // partition; this costs 8, plus 2 + 8 W over the tied ones.
         hipLaunchKernelGGL(iota_kernel, dim3(blocks), dim3(256), 0, s, P[pc], m);
         hipLaunchKernelGGL(gather_u64_kernel, dim3(blocks), dim3(256), 0, s, c.keys, (const u32*)P[pc], m, (u32)key_words, 0u, K[0]);
-        rc = radix_sort(L, SRC_PAIRS, nullptr, 0, 0, 0, K[0], P[pc], K[1], P[pc ^ 1], (u32)m, make_plan(0, 64), &in_out, &passes);
+        rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], P[pc], K[1], P[pc ^ 1], (u32)m, make_plan(0, 64), &in_out, &passes);
         if (rc)
             return rc;
         kc = in_out;
@@ -307,14 +307,14 @@ int step_init(Launch& L, const char* who, StepColumns& c, const StepPlan& pl, in
             u32* SV[2] = {P[pc ^ 1], pl.at<u32>(36)};
             int sv = 0;
             hipLaunchKernelGGL(gather_tag_keys_kernel, dim3(tblocks), dim3(256), 0, s, c.beta, (const u32*)SV[sv], tied, SK[0]);
-            rc = radix_sort(L, SRC_PAIRS, nullptr, 0, 0, 0, SK[0], SV[sv], SK[1], SV[sv ^ 1], (u32)tied, make_plan(0, 16), &in_out, &passes);
+            rc = radix_sort(L, SRC_PAIRS, 0, 0, SK[0], SV[sv], SK[1], SV[sv ^ 1], (u32)tied, make_plan(0, 16), &in_out, &passes);
             if (rc)
                 return rc;
             sv ^= in_out;
             for (int w = key_words - 1; w >= 0; --w) {
                 hipLaunchKernelGGL(gather_u64_kernel, dim3(tblocks), dim3(256), 0, s, c.keys, (const u32*)SV[sv], tied, (u32)key_words,
                                    (u32)w, SK[0]);
-                rc = radix_sort(L, SRC_PAIRS, nullptr, 0, 0, 0, SK[0], SV[sv], SK[1], SV[sv ^ 1], (u32)tied, make_plan(0, 64), &in_out, &passes);
+                rc = radix_sort(L, SRC_PAIRS, 0, 0, SK[0], SV[sv], SK[1], SV[sv ^ 1], (u32)tied, make_plan(0, 64), &in_out, &passes);
                 if (rc)
                     return rc;
                 sv ^= in_out;
@@ -375,7 +375,7 @@ int step_rerank(Launch& L, const char* who, StepColumns& c, const StepPlan& pl, 
     u64* keys_partner = pl.at<u64>(32);
     hipLaunchKernelGGL(iota_kernel, dim3(blocks), dim3(256), 0, s, P[0], m);
     int in_out = 0, passes = 0;
-    rc = radix_sort(L, SRC_PAIRS, nullptr, 0, 0, 0, keys, P[0], keys_partner, P[1], (u32)m, make_plan(0, 62), &in_out, &passes);
+    rc = radix_sort(L, SRC_PAIRS, 0, 0, keys, P[0], keys_partner, P[1], (u32)m, make_plan(0, 62), &in_out, &passes);
     if (rc)
         return rc;
     const u64* sorted_keys = in_out ? keys_partner : keys;

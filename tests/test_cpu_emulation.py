@@ -647,3 +647,27 @@ def test_chunked_tile_order_without_resident_workgroups_ends_in_an_error_not_a_h
         assert np.array_equal(out[:5 * small.size], oracle_lib.build_sa40(small))
     finally:
         emu.csa_destroy(h)
+
+
+def test_first_sort_on_codes_with_runs_that_share_a_code(emu):
+    """Runs of one code around the limit of the in-tile sort (64 members in this build) and past it, of one string and of two
+    out of order: the long mixed ones are collected and radix sorted. Suffix array and generation sizes against the oracle."""
+    T = texts.text_with_shared_codes(130000, [2, 5, 63, 64, 65, 70, 90], 3)
+    got, active, _ = emu_sort(emu, T, 1)
+    assert emu_sort.passes[0] > 4  # four passes over all suffixes, and those over the collected runs
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8, 11, 12, 13, 17, 511, 1023, 1025])
+def test_first_sort_on_codes_at_small_and_ragged_sizes(emu, n):
+    """The places of the last four suffixes, the 8-suffix groups of the coding kernel and the sample of a short text, at sizes
+    around their borders; the text ends in a repeat and in zeros."""
+    rng = np.random.default_rng(n)
+    T = rng.choice(np.array([0, 1, 255, 256, 511, 4000, 65535, 65534] + list(range(300, 40000, 97))), n).astype(np.uint16)
+    if n > 30:
+        T[n - 20:n - 3] = T[2:19]
+        T[-3:] = 0
+    got, active, _ = emu_sort(emu, T, 1, pack=False)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts

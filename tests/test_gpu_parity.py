@@ -658,3 +658,19 @@ def test_command_line_builder_writes_the_oracles_suffix_array(tmp_path):
     r = subprocess.run([exe, str(tmp_path / "missing.u16"), str(tmp_path / "x.sa40")], capture_output=True, text=True, timeout=100)
     assert r.returncode == 1 and "cannot open" in r.stderr
 
+
+
+@pytest.mark.parametrize("repeats", [[2, 3, 255, 256], [257, 258, 300, 700, 700]])
+def test_first_sort_on_codes_with_runs_that_share_a_code(torch_mod, repeats):
+    """The first sort of a token text goes by 32-bit codes of four symbols; runs of suffixes that share a code are put in order
+    inside a tile up to 256 members and radix sorted past that. Planted runs on both sides of the limit, of one string and of
+    two strings out of order, against the oracle: suffix array and generation sizes."""
+    from cascade_amd import PartitionSorter
+    T = texts.text_with_shared_codes(1 << 20, repeats, len(repeats))
+    with PartitionSorter(T.size, key_words=1) as s:
+        print(f"  shared codes {repeats}", flush=True)
+        got = gpu_sa40(torch_mod, s, T)
+        stats = s.last_stats
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
+    assert (stats["passes"][0] > 4) == (max(repeats) > 256)

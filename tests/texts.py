@@ -65,3 +65,23 @@ def fixture_suite():
     for k, c in enumerate(hand_cases()):
         out.append((f"hand_{k}", c))
     return out
+
+
+def text_with_shared_codes(n, repeats, seed):
+    """n random token ids into which strings of rare symbols are planted: for every r in `repeats`, r times the same three
+    symbols of their own followed by one of two neighbouring symbols, the larger one first more often than not. Sorted by arithmetic
+    codes of 32 bits, all r of them share one code as long as (r / n)^3 is far below 2^-32 times the symbols of the alphabet:
+    runs of that length, out of order as they stand; each next to one planted the same way with a single string."""
+    rng = np.random.default_rng(seed)
+    T = rng.integers(1, 40000, n).astype(np.uint16)
+    slots = rng.permutation(n // 5 - 2)
+    at = 0
+    for i, r in enumerate(repeats):
+        for mixed in (0, 1):
+            base = 50000 + 16 * (2 * i + mixed)
+            for k in range(r):
+                p = 5 * int(slots[at])
+                at += 1
+                T[p:p + 4] = [base, base + 1, base + 2, base + 4 - (mixed and int(rng.integers(0, 2)))]
+    T[-2:] = 0
+    return T
