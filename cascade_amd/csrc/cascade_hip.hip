@@ -857,7 +857,7 @@ PackedPlan plan_packed_text(const u32* bytehist, u32 n, int key_words, u64 room_
 
 // Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their four symbols, with the ties marked,
 // in ra.sufs' array. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into idx[1]; the codes
-// live in the halves of key[0], their text order in key[1]. `marked` is left ready for sort_marked_runs.
+// live in the halves of key[0], their text order and the flags in key[1]. `marked` is left ready for sort_marked_runs.
 int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, ResolveArgs& marked)
 {
     csa_handle* h = L.h;
@@ -867,14 +867,20 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, Resolv
     u32* const cum = marks + RESOLVE_MARK_WORDS;
     HIP_TRY(hipMemsetAsync(counts, 0, (SYMBOLS + RESOLVE_MARK_WORDS) * sizeof(u32), s));
     const u32 chunks = (n + SAMPLE_CHUNK - 1) / SAMPLE_CHUNK;
-    const u32 taken = chunks < SAMPLE_CHUNKS_MAX ? chunks : SAMPLE_CHUNKS_MAX;
+    // one chunk in 16, at least SAMPLE_CHUNKS_PER_BLOCK of them (or all there are) and at most SAMPLE_CHUNKS_MAX
+    u32 taken = chunks / 16 < SAMPLE_CHUNKS_PER_BLOCK ? SAMPLE_CHUNKS_PER_BLOCK : chunks / 16;
+    taken = taken < SAMPLE_CHUNKS_MAX ? taken : SAMPLE_CHUNKS_MAX;
+    taken = taken < chunks ? taken : chunks;
     const u64 sampled = (u64)taken * SAMPLE_CHUNK < n ? (u64)taken * SAMPLE_CHUNK : (u64)n;
     hipLaunchKernelGGL(sample_symbols_kernel, dim3((taken + SAMPLE_CHUNKS_PER_BLOCK - 1) / SAMPLE_CHUNKS_PER_BLOCK), dim3(SAMPLE_BLOCK), 0, s,
                        d_text, n, chunks, taken, counts);
-    hipLaunchKernelGGL(symbol_shares_kernel, dim3(1), dim3(1024), 0, s, (const u32*)counts, SAMPLE_LOG2 - bit_length(sampled - 1), cum);
-    u32* const codes = reinterpret_cast<u32*>(h->key[1]); // by virtual position
+    const int weight_log2 = SAMPLE_LOG2 - bit_length(sampled - 1);
+    hipLaunchKernelGGL(symbol_shares_kernel, dim3(SYMBOLS / SHARES_TILE), dim3(SHARES_TILE), 0, s, (const u32*)counts, weight_log2,
+                       (u32)((sampled << weight_log2) + SYMBOLS), cum);
+    u32* const codes = reinterpret_cast<u32*>(h->key[1]);          // by virtual position
+    u8* const own = reinterpret_cast<u8*>(h->key[1]) + 4 * h->cap; // flags by text position
     hipLaunchKernelGGL(code_suffixes_kernel, dim3(hist_blocks(CODE_BLOCK * CODE_ITEMS, n)), dim3(CODE_BLOCK), 0, s, d_text, n, tail,
-                       (const u32*)cum, codes, h->ghist);
+                       (const u32*)cum, codes, own, h->ghist);
     hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, CODE_PASSES);
     u32* const sorted[2] = {reinterpret_cast<u32*>(h->key[0]), reinterpret_cast<u32*>(h->key[0]) + h->cap};
     static_assert(CODE_PASSES % 2 == 0, "the sorted codes end in the first half of key[0], their suffixes in idx[0]");
@@ -887,6 +893,7 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, Resolv
         a.n = n;
         a.text_n = n;
         a.tail = tail;
+        a.own = own;
         a.shift = 8 * p;
         a.bits = 8;
         a.digit_base = h->digit_base + p * RADIX_BINS;

@@ -8,14 +8,18 @@
 // intervals, so that the codes spread evenly over the 32 bits where the raw symbols of a token text crowd into few values.
 // Four passes over 8-byte (code, suffix) pairs put the suffixes into the order of their codes, where K-gram keys take
 // eight passes over 12-byte pairs: 66 instead of 185 bytes moved per suffix (2^28 Zipf tokens: generation 0's passes 11.5 ->
-// 4.9 ms).
+// 4.1 ms).
 //
-// What the sort leaves open are the suffixes that share a code: those whose strings are equal, and a few whose strings are not
-// (n / 2^32 of them by chance). resolve_runs_kernel reads the strings of such suffixes from the text (and of no others),
-// sorts every run of up to RESOLVE_MAX suffixes inside its tile and sets bit 31 of every suffix that ties with its left
-// neighbour, which is all the rank step needs to know. Longer runs are nearly always one string repeated (a string that is this
-// frequent has codes of its own) and in order as they stand; the rare ones that are not are collected and radix sorted by the
-// string itself.
+// A string whose interval of codes holds at least two 32-bit values takes the second of them, which no other string can
+// have: its suffixes carry a flag (OWN_CODE) through the sort and are known to be equal where their codes are.
+//
+// What the sort leaves open are the other suffixes that share a code: those whose strings are equal though rare by the shares of
+// their symbols (copied passages), and those whose strings are not (n / 2^32 of the rare ones by chance). resolve_runs_kernel
+// reads the strings of such suffixes from the text (and of no others: a random 128-byte line each, which is what bounds it;
+// 8.0 ms on 1e9 tokens; 14.8 when it read those of the flagged ones too), sorts every run of up to RESOLVE_MAX suffixes inside its
+// tile and sets bit 31 of every suffix that ties with its left neighbour, which is all the rank step needs to know. Longer runs
+// are nearly always one string repeated and in order as they stand; the rare ones that are not are collected and radix
+// sorted by the string itself.
 #pragma once
 
 #include "device_utils.hpp"
@@ -65,46 +69,38 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16*
 }
 
 // cum[s], s <= SYMBOLS: the share of symbols below s as a 32-bit fraction, every symbol counted once more than the sample
-// (scaled by 2^weight_log2) has it, so that one the sample missed has a place too.
-__global__ __launch_bounds__(1024) void symbol_shares_kernel(const u32* __restrict__ counts, int weight_log2, u32* __restrict__ cum)
+// (scaled by 2^weight_log2) has it, so that one the sample missed has a place too. total = the sum of all weights.
+// Workgroup b writes the entries of SHARES_TILE symbols; it sums the counts of the symbols before them by itself (at most 64
+// coalesced rounds over a table in the L2), which takes a third of the time of one workgroup that scans them all (18 us).
+constexpr int SHARES_TILE = 1024;
+
+__global__ __launch_bounds__(SHARES_TILE) void symbol_shares_kernel(const u32* __restrict__ counts, int weight_log2, u32 total, u32* __restrict__ cum)
 {
-    constexpr int PER = SYMBOLS / 1024;
-    __shared__ u32 s_w[16];
+    __shared__ u32 s_sum[16], s_own[16];
     const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6;
-    u32 weight[PER], mine = 0;
-    const uint4* c4 = reinterpret_cast<const uint4*>(counts + t * PER);
-#pragma unroll
-    for (int k = 0; k < PER; k += 4) {
-        const uint4 v = c4[k / 4];
-        weight[k] = (v.x << weight_log2) + 1u;
-        weight[k + 1] = (v.y << weight_log2) + 1u;
-        weight[k + 2] = (v.z << weight_log2) + 1u;
-        weight[k + 3] = (v.w << weight_log2) + 1u;
-        mine += weight[k] + weight[k + 1] + weight[k + 2] + weight[k + 3];
+    const u32 first = blockIdx.x * SHARES_TILE;
+    u32 earlier = 0;
+#pragma unroll 4
+    for (u32 i = t * 4; i < first; i += SHARES_TILE * 4) {
+        const uint4 v = *reinterpret_cast<const uint4*>(counts + i);
+        earlier += v.x + v.y + v.z + v.w;
     }
-    const u32 incl = wave_incl_sum(mine);
+    const u32 weight = (counts[first + t] << weight_log2) + 1u;
+    const u32 sum = wave_reduce_sum(earlier), incl = wave_incl_sum(weight);
+    if (lane == 0)
+        s_sum[w] = sum;
     if (lane == 63u)
-        s_w[w] = incl;
+        s_own[w] = incl;
     __syncthreads();
-    u32 before = incl - mine, total = 0;
+    u32 counted = 0, before = incl - weight;
     for (u32 ww = 0; ww < 16; ++ww) {
-        if (ww < w)
-            before += s_w[ww];
-        total += s_w[ww];
+        counted += s_sum[ww];
+        before += ww < w ? s_own[ww] : 0u;
     }
-    const u64 scale = (1ull << 53) / total; // before <= total: before * scale <= 2^53
-    uint4* o4 = reinterpret_cast<uint4*>(cum + t * PER);
-#pragma unroll
-    for (int k = 0; k < PER; k += 4) {
-        u32 v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            v[q] = (u32)((u64)before * scale >> 21); // (below 2^32: every symbol's weight is at least 1)
-            before += weight[k + q];
-        }
-        o4[k / 4] = make_uint4(v[0], v[1], v[2], v[3]);
-    }
-    if (t == 1023u)
+    before += (counted << weight_log2) + first;
+    const u64 scale = (1ull << 53) / total; // before < total: every symbol weighs at least 1
+    cum[first + t] = (u32)((u64)before * scale >> 21);
+    if (first + t == (u32)SYMBOLS - 1)
         cum[SYMBOLS] = 0xFFFFFFFFu;
 }
 
@@ -115,10 +111,13 @@ constexpr int CODE_ITEMS = 8;
 constexpr int CODE_PASSES = 4;
 constexpr int CODE_COPIES = 8;
 
-// codes[v] = code of the suffix at virtual position v (virtual_to_suffix with `tail` = min(n, 4)). Bounded by the lookups
+// codes[v] = code of the suffix at virtual position v (virtual_to_suffix with `tail` = min(n, 4)); bit x & 7 of own[x >> 3]: the
+// suffix at text position x has a code that only its string can have. [low, high) below is the string's interval: the map from
+// the last symbol's entries to both ends is monotone, so the next string starts at `high` or later, and low + 1, where it
+// is below `high`, is above every code of a smaller string and below every code of a larger one. Bounded by the lookups
 // of cum[]: one 8-byte gather per symbol (the table is 256 KB: it lives in the L2s), shared by the four suffixes it appears in.
 __global__ __launch_bounds__(CODE_BLOCK) void code_suffixes_kernel(const u16* __restrict__ text, u32 n, u32 tail, const u32* __restrict__ cum,
-                                                                   u32* __restrict__ codes, u32* __restrict__ ghist)
+                                                                   u32* __restrict__ codes, u8* __restrict__ own, u32* __restrict__ ghist)
 {
     constexpr u32 TILE = CODE_BLOCK * CODE_ITEMS;
     __shared__ u64 s_text[(TILE + 3 + 6) / 4 + 2];
@@ -143,16 +142,22 @@ __global__ __launch_bounds__(CODE_BLOCK) void code_suffixes_kernel(const u16* __
             lo[k] = pair[0];
             width[k] = pair[1] - pair[0];
         }
-        u32 code[CODE_ITEMS];
+        u32 code[CODE_ITEMS], owners = 0;
 #pragma unroll
         for (int k = 0; k < CODE_ITEMS; ++k) {
-            u32 f = lo[k + 3];
+            u32 low = lo[k + 3], high = lo[k + 3] + width[k + 3];
 #pragma unroll
-            for (int q = 2; q >= 0; --q)
-                f = lo[k + q] + (u32)(((u64)width[k + q] * f) >> 32);
-            code[k] = f;
+            for (int q = 2; q >= 0; --q) {
+                low = lo[k + q] + (u32)(((u64)width[k + q] * low) >> 32);
+                high = lo[k + q] + (u32)(((u64)width[k + q] * high) >> 32);
+            }
+            const u32 alone = high - low >= 2u ? 1u : 0u;
+            code[k] = low + alone;
+            owners |= alone << k;
         }
         const u64 x0 = p0 + (u64)t * CODE_ITEMS;
+        if (x0 < n)
+            own[x0 / 8] = (u8)owners;
         if (tail == 4 && x0 + CODE_ITEMS + tail <= n) { // no suffix of the text's end among them: places x0 + 4 on, 16-byte aligned
             uint4* out = reinterpret_cast<uint4*>(codes + x0 + 4);
 #pragma unroll
@@ -194,6 +199,7 @@ constexpr int RESOLVE_TILE = RESOLVE_BLOCK * RESOLVE_ITEMS;
 #define CSA_RESOLVE_MAX 256
 #endif
 constexpr int RESOLVE_MAX = CSA_RESOLVE_MAX; // longest run that is sorted inside its tile
+static_assert(CODE_ITEMS == 8, "a thread of the coding kernel writes one byte of flags");
 static_assert(RESOLVE_MAX % 64 == 0 && RESOLVE_MAX <= RESOLVE_BLOCK, "the halo is read in whole waves, one element per thread");
 constexpr u32 RESOLVE_MARK_BITS = 20;
 constexpr u32 RESOLVE_MARK_WORDS = 1u << (RESOLVE_MARK_BITS - 5);
@@ -203,7 +209,7 @@ __device__ __forceinline__ u32 resolve_mark(u32 code) { return (code * 0x9E3779B
 
 struct ResolveArgs {
     const u32* codes; // sorted
-    const u32* sufs;
+    const u32* sufs;  // OWN_CODE: no other string has this suffix's code
     const u16* text;
     u32 n;
     u32 ell; // symbols of a string; a suffix that runs off the text inside them ties with nobody
@@ -255,7 +261,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         return last - first <= H;
     };
     // own elements: suffix, run, and the string where there is company
-    u32 x[RESOLVE_ITEMS];
+    u32 x[RESOLVE_ITEMS], owners = 0; // bit k of owners: element k has OWN_CODE
     int first[RESOLVE_ITEMS], last[RESOLVE_ITEMS]; // last = 0: a long run; last - first = 1: alone
 #pragma unroll
     for (int k = 0; k < RESOLVE_ITEMS; ++k) {
@@ -266,6 +272,8 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         last[k] = j + 1;
         if (e < n) {
             x[k] = a.sufs[e];
+            owners |= (x[k] & OWN_CODE ? 1u : 0u) << k;
+            x[k] &= ~OWN_CODE;
             if (!run_of(j, first[k], last[k])) {
                 first[k] = j;
                 last[k] = 0;
@@ -276,8 +284,9 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     for (int k = 0; k < RESOLVE_ITEMS; ++k) {
         const int j = H + k * RESOLVE_BLOCK + (int)t;
         if (last[k] - first[k] != 1) {
-            s_key[j] = load_kgram(a.text, a.n, x[k], 0);
             s_suf[j] = x[k];
+            if (!((owners >> k) & 1u))
+                s_key[j] = load_kgram(a.text, a.n, x[k], 0);
         }
     }
     // of the halo: the members of short runs that reach into the tile, and the left neighbour of the tile's first element
@@ -290,8 +299,10 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
             const long long e = lo + j;
             const bool wanted = i < H ? (short0 ? j >= f0 : j == H - 1) : (short1 && j < l1);
             if (wanted && e >= 0 && e < n) {
-                s_suf[j] = a.sufs[e];
-                s_key[j] = load_kgram(a.text, a.n, s_suf[j], 0);
+                const u32 y = a.sufs[e];
+                s_suf[j] = y & ~OWN_CODE;
+                if (!(y & OWN_CODE))
+                    s_key[j] = load_kgram(a.text, a.n, y, 0);
             }
         }
     }
@@ -305,7 +316,10 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         const bool whole = (u64)x[k] + a.ell < a.n;
         int place = j;
         bool tied = false;
-        if (last[k] == 0) {
+        if ((owners >> k) & 1u) { // one string, in order as it stands
+            if (!((s_head[j / 64] >> (j & 63)) & 1ull))
+                tied = whole && (u64)s_suf[j - 1] + a.ell < a.n;
+        } else if (last[k] == 0) {
             if (!((s_head[j / 64] >> (j & 63)) & 1ull)) {
                 const u64 mine = s_key[j], before = s_key[j - 1];
                 tied = mine == before && whole && (u64)s_suf[j - 1] + a.ell < a.n;

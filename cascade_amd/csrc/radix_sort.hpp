@@ -44,6 +44,9 @@ __device__ __forceinline__ u64 rank_pair_key(const u32* __restrict__ rank, u32 n
     return radix ? (u64)rank[i] * radix + second : ((u64)rank[i] << 32) | second;
 }
 
+// Bit 31 of a suffix in a sort by codes (coded_keys.hpp): no other string has this suffix's code. Suffixes are below 2^31.
+constexpr u32 OWN_CODE = 0x80000000u;
+
 // Generation 0 feeds the suffixes in the order (n-1, n-2, ..., n-tail, 0, 1, ..., n-tail-1): the last
 // `tail` suffixes run off the text inside their key, must each stay a group of one and sort
 // shorter-first before any real suffix with the same (zero-padded) key. Putting them first, shortest
@@ -264,6 +267,7 @@ struct OnesweepArgs {
     u32 tiles;             // tiles of the pass = workgroups of the launch
     u32 epoch;
     u32* err;
+    const u8* own = nullptr;   // SRC_CODED: flags by text position, 8 to a byte
     const u32* rank = nullptr; // SRC_RANKS: rank[] by text position ...
     u32 hop = 0;               // ... the distance to the second rank of a key ...
     u32 radix = 0;             // ... and how the two make the key (rank_pair_key)
@@ -504,8 +508,13 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
     for (int k = 0; k < ITEMS; ++k) {
         const u32 local = first_local + k * WAVE;
         val[k] = 0;
-        if (VALS && local < valid)
-            val[k] = (SRC == SRC_CODED || SRC == SRC_PACKED) ? virtual_to_suffix((u32)(base + local), a.text_n, a.tail)
+        if (SRC == SRC_CODED) {
+            if (local < valid) {
+                const u32 x = virtual_to_suffix((u32)(base + local), a.text_n, a.tail);
+                val[k] = x | ((a.own[x >> 3] >> (x & 7u)) & 1u ? OWN_CODE : 0u);
+            }
+        } else if (VALS && local < valid)
+            val[k] = SRC == SRC_PACKED ? virtual_to_suffix((u32)(base + local), a.text_n, a.tail)
                      : SRC == SRC_RANKS                     ? (u32)(base + local)
                                                             : a.vals_in[base + local];
     }
