@@ -1393,8 +1393,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                 hipLaunchKernelGGL((place_big_kernel<RANK_BLOCK, RANK_ITEMS, true>), dim3(pr.tiles), dim3(RANK_BLOCK), 0, s, pa);
                 HIP_TRY(hipGetLastError());
             }
-            // 3. per-tile counts of the sorted list (4 bytes read per member)
-            hipLaunchKernelGGL((count_ranks_kernel<SMALL_BLOCK, SMALL_ITEMS>), dim3(r.tiles), dim3(SMALL_BLOCK), 0, s, nr_list, m_in,
+            // 3. per-tile counts of the sorted list (8 bytes read per member)
+            hipLaunchKernelGGL((count_ranks_kernel<SMALL_BLOCK, SMALL_ITEMS>), dim3(r.tiles), dim3(SMALL_BLOCK), 0, s, nr_list, x_out, m_in,
                                r.tile_agg, r.tile_splits);
             HIP_TRY(hipGetLastError());
         }

@@ -785,9 +785,14 @@ __global__ __launch_bounds__(BLOCK) void smallsort_kernel(SmallSortArgs a)
 }
 
 // Counts of the sorted list (suffix, refined rank) per tile, for generations in which large groups came back through
-// the radix sort: survivors (members whose rank is shared), new groups, changed ranks. Reads 4 bytes per member.
+// the radix sort: survivors (members whose rank is shared), new groups, changed ranks. Reads 8 bytes per member.
+// A changed rank counts only if its suffix is not next to the one before it in the list (in the same 64 bytes of rank[]): the
+// count decides whether the rank writes are bucketed first, and the members of a run or a period, whose suffixes follow one
+// another in the list, write whole lines of rank[] as they stand. 2^26 symbols of runs, periods and tokens, 20
+// generations of 10 M such members: 15.9 ms with the bucketed update (histogram, pass, scatter: 0.24 ms each), 12.8 without.
 template <int BLOCK, int ITEMS>
-__global__ __launch_bounds__(BLOCK) void count_ranks_kernel(const u32* __restrict__ nr, u32 m, u32* __restrict__ tile_agg,
+__global__ __launch_bounds__(BLOCK) void count_ranks_kernel(const u32* __restrict__ nr, const u32* __restrict__ sufs, u32 m,
+                                                            u32* __restrict__ tile_agg,
                                                             u32* __restrict__ tile_splits)
 {
     constexpr int TILE = BLOCK * ITEMS;
@@ -798,11 +803,17 @@ __global__ __launch_bounds__(BLOCK) void count_ranks_kernel(const u32* __restric
     // from the list (whole 16-byte loads where they all exist)
     const u64 base = (u64)blockIdx.x * TILE + (u64)t * ITEMS;
     u32 nrw[ITEMS + 2]; // places base - 1 .. base + ITEMS
+    u32 x[ITEMS + 1];   // places base - 1 .. base + ITEMS - 1
     if (ITEMS % 4 == 0 && base + ITEMS <= m) {
         const uint4* n4 = reinterpret_cast<const uint4*>(nr + base); // base is a multiple of ITEMS
+        const uint4* x4 = reinterpret_cast<const uint4*>(sufs + base);
 #pragma unroll
         for (int k = 0; k < ITEMS; k += 4) {
-            const uint4 v = n4[k / 4];
+            const uint4 v = n4[k / 4], xv = x4[k / 4];
+            x[k + 1] = xv.x;
+            x[k + 2] = xv.y;
+            x[k + 3] = xv.z;
+            x[k + 4] = xv.w;
             nrw[k + 1] = v.x;
             nrw[k + 2] = v.y;
             nrw[k + 3] = v.z;
@@ -810,11 +821,14 @@ __global__ __launch_bounds__(BLOCK) void count_ranks_kernel(const u32* __restric
         }
         nrw[0] = base >= 1 ? nr[base - 1] : 0u;
         nrw[ITEMS + 1] = base + ITEMS < m ? nr[base + ITEMS] : 0u;
+        x[0] = base >= 1 ? sufs[base - 1] : 0u;
     } else {
 #pragma unroll
         for (int k = 0; k < ITEMS + 2; ++k) {
             const u64 c = base + k; // place c - 1
             nrw[k] = (c >= 1 && c - 1 < m) ? nr[c - 1] : 0u;
+            if (k <= ITEMS)
+                x[k] = (c >= 1 && c - 1 < m) ? sufs[c - 1] : 0u;
         }
     }
     u32 c_surv = 0, c_head = 0, c_chg = 0;
@@ -828,7 +842,8 @@ __global__ __launch_bounds__(BLOCK) void count_ranks_kernel(const u32* __restric
             const bool surv = !(head && last);
             c_surv += surv ? 1u : 0u;
             c_head += (head && surv) ? 1u : 0u;
-            c_chg += word >> 31;
+            const bool next_to = c > 0 && x[k + 1] - x[k] + 15u <= 30u; // at most 15 places apart, either way
+            c_chg += next_to ? 0u : word >> 31;
         }
     }
     static_assert(64 * ITEMS < 1024, "three counts are packed into one 32-bit word");

@@ -671,3 +671,18 @@ def test_first_sort_on_codes_at_small_and_ragged_sizes(emu, n):
     got, active, _ = emu_sort(emu, T, 1, pack=False)
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
+@pytest.mark.parametrize("period", [1, 7, 15, 16, 40])
+def test_ranks_of_neighbouring_suffixes_are_written_in_place(emu, period):
+    """A periodic stretch among random tokens: the members of its groups stand in the list in the order of the text, `period`
+    symbols apart. Up to 15 apart (one line of rank[]) their rank writes are not bucketed, past that they are; suffix array
+    and generation sizes are the oracle's either way."""
+    rng = np.random.default_rng(period)
+    T = rng.integers(300, 60000, 6000).astype(np.uint16)
+    T[1000:4600] = np.tile(rng.integers(300, 60000, period).astype(np.uint16), 3600 // period + 1)[:3600]
+    got, active, big = emu_sort(emu, T, 1, pack=False)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    late = [u for u, b, d in zip(emu_sort.rank_update, big, emu_sort.dense) if b and not d][1:-1]
+    assert late and (all(u == 0 for u in late) if period <= 15 else any(u == 2 for u in late))
