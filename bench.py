@@ -21,6 +21,9 @@ sys.path.insert(0, os.path.join(ROOT, "tests"))
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, published
 # algorithmic bytes of one radix pass per (key, index) pair: read + write of an 8-byte key and a 5-byte index
 RADIX_PASS_BYTES_PER_PAIR = 2 * (8 + 5)
+# the same of a pass of the first sort over (32-bit code, index) pairs, which texts over large alphabets take: a 4-byte key
+CODED_PASS_BYTES_PER_PAIR = 2 * (4 + 5)
+CODED_PASSES = 4
 
 
 def algorithmic_bytes(n, active):
@@ -623,7 +626,9 @@ def main():
 
     # dominant kernel: the one-sweep radix pass, timed per launch with HIP events on the sort's stream
     avg_launch_ms = radix_ms / radix_launches if radix_launches else 0.0
-    achieved = (RADIX_PASS_BYTES_PER_PAIR * radix_pairs / (radix_ms * 1e-3) / 1e9) if radix_ms > 0 else 0.0
+    coded_pairs = CODED_PASSES * n * args.steps if st["key_symbols"] == 4 else 0  # a first sort on packed symbols resolves 8 or more
+    radix_bytes = RADIX_PASS_BYTES_PER_PAIR * (radix_pairs - coded_pairs) + CODED_PASS_BYTES_PER_PAIR * coded_pairs
+    achieved = radix_bytes / (radix_ms * 1e-3) / 1e9 if radix_ms > 0 else 0.0
     pairs_per_launch = radix_pairs / radix_launches if radix_launches else 0
     roofline = {
         "bound": "hbm", "kernel": "onesweep_kernel (one radix pass over (key, index) pairs)",
@@ -632,7 +637,7 @@ def main():
         "traffic": round(per_pair * pairs_per_launch) if per_pair is not None else None,
         "traffic_source": traffic_source,
         "frac_moved": round(per_pair * radix_pairs / (radix_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if per_pair is not None and radix_ms > 0 else None,
-        "algorithmic_bytes_per_launch": round(RADIX_PASS_BYTES_PER_PAIR * pairs_per_launch),
+        "algorithmic_bytes_per_launch": round(radix_bytes / radix_launches) if radix_launches else 0,
         "launches_per_step": radix_launches / args.steps, "avg_launch_ms": round(avg_launch_ms, 4),
         "pairs_per_launch": pairs_per_launch,
         "share_of_step": round(radix_ms / args.steps / ms_per_step, 3),

@@ -416,6 +416,23 @@ void launch_onesweep32(const csa_handle* hh, OnesweepArgs& a, hipStream_t s)
     }
 }
 
+// One radix pass over n pairs, between two events where the caller asked for its time.
+template <typename LaunchPass>
+int launch_pass(Launch& L, u32 n, LaunchPass launch)
+{
+    csa_handle* h = L.h;
+    const bool timed = (L.flags & CSA_FLAG_KERNEL_TIMING) && L.events_used + 2 <= (int)h->events.size();
+    if (timed)
+        HIP_TRY(hipEventRecord(h->events[L.events_used], L.stream));
+    launch();
+    if (timed) {
+        HIP_TRY(hipEventRecord(h->events[L.events_used + 1], L.stream));
+        L.timed.push_back({L.events_used, (u64)n});
+        L.events_used += 2;
+    }
+    return CSA_OK;
+}
+
 // Sorts n pairs by the digits of `plan`. The first pass that runs takes its input as `src` says
 // (pairs kin/vin, or keys built on the way in); passes alternate between the (kin, vin) and (kout, vout) sets, the
 // very first one writing to (kout, vout). *result_in_out = 1 if the sorted pairs ended in (kout, vout).
@@ -535,21 +552,17 @@ int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64
         int rc = next_ticket(L, &a.ticket);
         if (rc)
             return rc;
-        const bool timed = (L.flags & CSA_FLAG_KERNEL_TIMING) && L.events_used + 2 <= (int)h->events.size();
-        if (timed)
-            HIP_TRY(hipEventRecord(h->events[L.events_used], s));
         const int use_src = first ? src : SRC_PAIRS;
-        if (use_src == SRC_PAIRS)
-            launch_onesweep<SRC_PAIRS>(h, a, s);
-        else if (use_src == SRC_RANKS)
-            launch_onesweep<SRC_RANKS>(h, a, s);
-        else
-            launch_onesweep<SRC_PACKED>(h, a, s);
-        if (timed) {
-            HIP_TRY(hipEventRecord(h->events[L.events_used + 1], s));
-            L.timed.push_back({L.events_used, (u64)n});
-            L.events_used += 2;
-        }
+        rc = launch_pass(L, n, [&] {
+            if (use_src == SRC_PAIRS)
+                launch_onesweep<SRC_PAIRS>(h, a, s);
+            else if (use_src == SRC_RANKS)
+                launch_onesweep<SRC_RANKS>(h, a, s);
+            else
+                launch_onesweep<SRC_PACKED>(h, a, s);
+        });
+        if (rc)
+            return rc;
         first = false;
         where ^= 1;
         (*passes_run)++;
@@ -904,10 +917,14 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, Resolv
         int rc = next_ticket(L, &a.ticket);
         if (rc)
             return rc;
-        if (p == 0)
-            launch_onesweep32<SRC_CODED>(h, a, s);
-        else
-            launch_onesweep32<SRC_PAIRS>(h, a, s);
+        rc = launch_pass(L, n, [&] {
+            if (p == 0)
+                launch_onesweep32<SRC_CODED>(h, a, s);
+            else
+                launch_onesweep32<SRC_PAIRS>(h, a, s);
+        });
+        if (rc)
+            return rc;
     }
     memset(&marked, 0, sizeof(marked));
     marked.codes = sorted[0];

@@ -674,3 +674,21 @@ def test_first_sort_on_codes_with_runs_that_share_a_code(torch_mod, repeats):
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
     assert (stats["passes"][0] > 4) == (max(repeats) > 256)
+
+
+@pytest.mark.parametrize("letters", [40000, 4])
+def test_kernel_timing_counts_every_radix_pass(torch_mod, letters):
+    """CSA_FLAG_KERNEL_TIMING brackets every launch of the radix pass: those of the first sort on codes or on packed symbols
+    and those of later generations."""
+    from cascade_amd import PartitionSorter, _native
+    rng = np.random.default_rng(letters)
+    T = rng.integers(1, letters + 1, 1 << 18).astype(np.uint16)
+    T[1000:3000] = 7  # a group that is too long for the in-tile sort
+    d = torch_mod.from_numpy(T.view(np.int16)).to("cuda:0")
+    with PartitionSorter(T.size, key_words=1) as s:
+        print(f"  timed passes, {letters} letters", flush=True)
+        s.sort(d, flags=_native.CSA_FLAG_KERNEL_TIMING)
+        torch_mod.cuda.synchronize()
+        stats = s.last_stats
+    assert stats["radix_launches"] == sum(stats["passes"]) >= 4
+    assert stats["radix_pairs"] >= T.size * stats["passes"][0] and stats["radix_ms"] > 0
