@@ -892,8 +892,12 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, Resolv
                        (u32)((sampled << weight_log2) + SYMBOLS), cum);
     u32* const codes = reinterpret_cast<u32*>(h->key[1]);          // by virtual position
     u8* const own = reinterpret_cast<u8*>(h->key[1]) + 4 * h->cap; // flags by text position
-    hipLaunchKernelGGL(code_suffixes_kernel, dim3(hist_blocks(CODE_BLOCK * CODE_ITEMS, n)), dim3(CODE_BLOCK), 0, s, d_text, n, tail,
-                       (const u32*)cum, codes, own, h->ghist);
+    if (n >= SORT_WIDE_MIN) // 2048 tiles of the wide workgroups: four for each of those a device holds at a time
+        hipLaunchKernelGGL(code_suffixes_kernel<CODE_WIDE_BLOCK>, dim3(hist_blocks(CODE_WIDE_BLOCK * CODE_ITEMS, n)), dim3(CODE_WIDE_BLOCK), 0,
+                           s, d_text, n, tail, (const u32*)cum, codes, own, h->ghist);
+    else
+        hipLaunchKernelGGL(code_suffixes_kernel<CODE_BLOCK>, dim3(hist_blocks(CODE_BLOCK * CODE_ITEMS, n)), dim3(CODE_BLOCK), 0, s, d_text, n,
+                           tail, (const u32*)cum, codes, own, h->ghist);
     hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, CODE_PASSES);
     u32* const sorted[2] = {reinterpret_cast<u32*>(h->key[0]), reinterpret_cast<u32*>(h->key[0]) + h->cap};
     static_assert(CODE_PASSES % 2 == 0, "the sorted codes end in the first half of key[0], their suffixes in idx[0]");

@@ -107,6 +107,7 @@ __global__ __launch_bounds__(SHARES_TILE) void symbol_shares_kernel(const u32* _
 // ---- the codes of all suffixes, and the digit counts of the four passes ----
 
 constexpr int CODE_BLOCK = 256;
+constexpr int CODE_WIDE_BLOCK = 1024;
 constexpr int CODE_ITEMS = 8;
 constexpr int CODE_PASSES = 4;
 constexpr int CODE_COPIES = 8;
@@ -116,21 +117,25 @@ constexpr int CODE_COPIES = 8;
 // the last symbol's entries to both ends is monotone, so the next string starts at `high` or later, and low + 1, where it
 // is below `high`, is above every code of a smaller string and below every code of a larger one. Bounded by the lookups
 // of cum[]: one 8-byte gather per symbol (the table is 256 KB: it lives in the L2s), shared by the four suffixes it appears in.
-__global__ __launch_bounds__(CODE_BLOCK) void code_suffixes_kernel(const u16* __restrict__ text, u32 n, u32 tail, const u32* __restrict__ cum,
+// BLOCK: the 32 KB of digit counters decide how many waves a CU holds, 16 in workgroups of 256 and 32 in workgroups of 1024,
+// which code 1e9 tokens in 2.27 instead of 3.06 ms and 2^28 in 0.58 instead of 0.78 (512: 2.69, 0.66; 256 with half the
+// counters: 2.92, 0.75). Short texts take 256, so that there are workgroups for every CU.
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void code_suffixes_kernel(const u16* __restrict__ text, u32 n, u32 tail, const u32* __restrict__ cum,
                                                                    u32* __restrict__ codes, u8* __restrict__ own, u32* __restrict__ ghist)
 {
-    constexpr u32 TILE = CODE_BLOCK * CODE_ITEMS;
+    constexpr u32 TILE = BLOCK * CODE_ITEMS;
     __shared__ u64 s_text[(TILE + 3 + 6) / 4 + 2];
     __shared__ u32 s_hist[CODE_PASSES * RADIX_BINS * CODE_COPIES];
     const u32 t = threadIdx.x;
-    for (u32 i = t; i < CODE_PASSES * RADIX_BINS * CODE_COPIES; i += CODE_BLOCK)
+    for (u32 i = t; i < CODE_PASSES * RADIX_BINS * CODE_COPIES; i += BLOCK)
         s_hist[i] = 0;
     const u32 copy = t & (CODE_COPIES - 1);
     const u64 tiles = ((u64)n + TILE - 1) / TILE;
     for (u64 tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const u64 p0 = tile * TILE;
         __syncthreads(); // the counters are cleared; the stretch of the round before has been read
-        const u32 sym_off = stage_text(text, n, p0, TILE + 3u, s_text, t, CODE_BLOCK);
+        const u32 sym_off = stage_text(text, n, p0, TILE + 3u, s_text, t, BLOCK);
         __syncthreads();
         const u16* s16 = reinterpret_cast<const u16*>(s_text) + sym_off + t * CODE_ITEMS;
         u32 lo[CODE_ITEMS + 3], width[CODE_ITEMS + 3];
@@ -180,7 +185,7 @@ __global__ __launch_bounds__(CODE_BLOCK) void code_suffixes_kernel(const u16* __
             }
     }
     __syncthreads();
-    for (u32 i = t; i < CODE_PASSES * RADIX_BINS; i += CODE_BLOCK) {
+    for (u32 i = t; i < CODE_PASSES * RADIX_BINS; i += BLOCK) {
         u32 v = 0;
 #pragma unroll
         for (int c = 0; c < CODE_COPIES; ++c)

@@ -659,7 +659,7 @@ def test_first_sort_on_codes_with_runs_that_share_a_code(emu):
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
 
 
-@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8, 11, 12, 13, 17, 511, 1023, 1025])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8, 11, 12, 13, 17, 511, 1023, 1025, 1599, 1600, 8191, 8193])
 def test_first_sort_on_codes_at_small_and_ragged_sizes(emu, n):
     """The places of the last four suffixes, the 8-suffix groups of the coding kernel and the sample of a short text, at sizes
     around their borders; the text ends in a repeat and in zeros."""
