@@ -37,7 +37,18 @@ constexpr u32 SAMPLE_CHUNKS_PER_BLOCK = 256;  // 16384 symbols: a 16-bit counter
 constexpr u32 SAMPLE_CHUNKS_MAX = 1u << 14;   // 2^20 symbols are looked at, at most
 constexpr int SAMPLE_LOG2 = 20;
 
-// counts[s] += occurrences of symbol s in the sample: `taken` chunks spread evenly over the text (all of them when the text is short).
+// Chunk c of a sample of `taken` out of `chunks`: one of the c-th of `taken` equal stretches of the text, at the place in it that the
+// multiples of the golden ratio, cut to their fractions, give. At equal distances the chunks would see only a few columns of a text
+// in rows of a fixed length (2^28 symbols in rows of 1024, the first 64 of each over values of their own: at a stride of
+// 16384 symbols only those columns were sampled, most suffixes shared their code with thousands of others, and generation 0
+// took 37.0 ms).
+__device__ __forceinline__ u32 sampled_chunk(u32 c, u32 chunks, u32 taken)
+{
+    const u32 lo = (u32)((u64)c * chunks / taken), hi = (u32)((u64)(c + 1) * chunks / taken);
+    return lo + (u32)(((u64)(c * 0x9E3779B1u) * (hi - lo)) >> 32);
+}
+
+// counts[s] += occurrences of symbol s in the sample: `taken` chunks (all of them when the text is short).
 __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16* __restrict__ text, u32 n, u32 chunks, u32 taken,
                                                                       u32* __restrict__ counts)
 {
@@ -51,7 +62,7 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16*
     for (u32 r = t / SAMPLE_CHUNK; r < SAMPLE_CHUNKS_PER_BLOCK; r += SAMPLE_BLOCK / SAMPLE_CHUNK) {
         const u32 c = first + r;
         if (c < taken) {
-            const u64 p = (u64)c * chunks / taken * SAMPLE_CHUNK + (t & (SAMPLE_CHUNK - 1));
+            const u64 p = (u64)sampled_chunk(c, chunks, taken) * SAMPLE_CHUNK + (t & (SAMPLE_CHUNK - 1));
             if (p < n) {
                 const u32 s = text[p];
                 atomicAdd(&s_cnt[s >> 1], (s & 1u) ? 0x10000u : 1u);
@@ -69,8 +80,9 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16*
 }
 
 // cum[s], s <= SYMBOLS: the share of symbols below s as a 32-bit fraction, every symbol counted once more than the sample
-// (scaled by 2^weight_log2) has it, so that one the sample missed has a place too. total = the sum of all weights.
-// Workgroup b writes the entries of SHARES_TILE symbols; it sums the counts of the symbols before them by itself (at most 64
+// (scaled by 2^weight_log2) has it, so that one the sample missed has a place too. total >= the sum of all weights (the
+// sample holds the text's last chunk or not, which may be a short one).
+// Workgroup b writes the entries of SHARES_TILE symbols; it sums the counts of the symbols before them by itself (at most 16
 // coalesced rounds over a table in the L2), which takes a third of the time of one workgroup that scans them all (18 us).
 constexpr int SHARES_TILE = 1024;
 

@@ -686,3 +686,17 @@ def test_ranks_of_neighbouring_suffixes_are_written_in_place(emu, period):
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
     late = [u for u, b, d in zip(emu_sort.rank_update, big, emu_sort.dense) if b and not d][1:-1]
     assert late and (all(u == 0 for u in late) if period <= 15 else any(u == 2 for u in late))
+
+
+@pytest.mark.parametrize("row", [512, 500])
+def test_first_sort_on_codes_of_a_text_in_rows_of_a_fixed_length(emu, row):
+    """Rows whose first 64 columns hold values of their own, as long as the stretches the sample of the symbols takes one chunk from
+    (512 symbols at 2^17) or not: the sample sees all columns either way, so no long run of suffixes shares a code and the first sort
+    makes its four passes alone."""
+    n = 1 << 17
+    rng = np.random.default_rng(row)
+    T = np.where(np.arange(n) % row < 64, rng.integers(0, 300, n), rng.integers(10000, 10500, n)).astype(np.uint16)
+    got, active, _ = emu_sort(emu, T, 1)
+    assert emu_sort.passes[0] == 4
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
