@@ -11,6 +11,7 @@
 #include "pipeline_steps.hpp"
 #include "radix_sort.hpp"
 
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -178,7 +179,23 @@ constexpr int SMALL_MAXG_HI = CSA_SMALL_MAXG_HI;
 constexpr u32 SMALL_AVG_LIMIT = CSA_SMALL_AVG_LIMIT;
 static_assert(SMALL_MAXG_HI >= SMALL_MAXG, "the higher group limit is the higher one");
 constexpr u32 TICKET_POOL = 4096;
-constexpr u64 CODE_TABLE_WORDS = SYMBOLS + RESOLVE_MARK_WORDS + SYMBOLS + 4; // symbol counts, marks, shares (and entry [SYMBOLS])
+constexpr u32 PROBE_FEW_CHUNKS = 512;                             // 2^15 suffixes, whose table ...
+constexpr u64 PROBE_TABLE = 2ull * PROBE_FEW_CHUNKS * SAMPLE_CHUNK; // ... is one of the handle's own
+constexpr u64 CODE_TABLE_WORDS = SYMBOLS + RESOLVE_MARK_WORDS + 8 + 2 * PROBE_TABLE + SYMBOLS + 4; // symbol counts, marks, ProbeCounts, its table, shares (and entry [SYMBOLS])
+// Texts of at least this many symbols are probed before they are sorted by codes (probe_codes_kernel, 15 us with its round trip). Shorter
+// ones have few runs of a code that are too long for a tile: generation 0 of 2^18 symbols of phrases takes 205 us on codes
+// and 185 on K-gram keys, of 2^19 symbols 381 and 207; of independent symbols 153 and 185, 168 and 207.
+#ifndef CSA_PROBE_MIN
+#define CSA_PROBE_MIN (1u << 19)
+#endif
+constexpr u32 PROBE_MIN = CSA_PROBE_MIN;
+// Shorter texts are coded while the host waits for the probe, which takes about as long, longer ones when it has advised that: 2^22
+// independent symbols 353 us coded ahead, 364 else, and 2^22 symbols of phrases, which go by K-grams then, 499 and 463.
+#ifndef CSA_CODE_AHEAD_MAX
+#define CSA_CODE_AHEAD_MAX (1u << 22)
+#endif
+constexpr u32 CODE_AHEAD_MAX = CSA_CODE_AHEAD_MAX;
+static_assert(PROBE_MIN >= 16 * SAMPLE_CHUNK, "the probe looks at one chunk at least");
 constexpr u32 PINNED_HIST = 32;        // host mirror: words [0, 16) mirror the device counters, [16, 32) single values, then the histograms
 constexpr u32 MSG_OFF_WORDS = 32769;   // p + 1 outbox counters, p <= 32768
 constexpr int EVENT_POOL = 2 * CSA_MAX_GENERATIONS * MAX_PASSES * 2;
@@ -439,17 +456,19 @@ int launch_pass(Launch& L, u32 n, LaunchPass launch)
 // Passes whose digit is the same for every pair are skipped (they would be the identity).
 // src = SRC_RANKS: pair i is ((rank_src[i], rank_src[i + hop]), i), i < n, built by the first pass that runs; the two
 // ranks are combined as rank_pair_key says for `radix`.
-// src = SRC_PACKED: the first pass cuts its keys from the code stream `packed` describes; the caller has filled
-// ghist already.
-struct PackedSource {
-    const u32* stream;
+// src = SRC_PACKED, SRC_TEXT: the first pass cuts its keys from the code stream, or builds them from the text, that `source`
+// describes; the caller has filled ghist already.
+struct TextSource {
+    const u16* text;   // SRC_TEXT ...
+    bool byte_wide;    // ... whose symbols may differ in one of their bytes only
+    const u32* stream; // SRC_PACKED
     u64 words;
     u32 sym_bits, key_bits;
 };
 
 int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64* kout,
                u32* vout, u32 n, const PassPlan& plan, int* result_in_out, int* passes_run, const u32* rank_src = nullptr,
-               u32 hop = 0, u32 radix = 0, const PackedSource* packed = nullptr)
+               u32 hop = 0, u32 radix = 0, const TextSource* source = nullptr)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -457,9 +476,9 @@ int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64
     *passes_run = 0;
     if (n == 0)
         return CSA_OK;
-    if (src == SRC_PACKED) {
-        if (!packed)
-            return fail(CSA_ERR_INTERNAL, "radix_sort: packed keys come with their stream");
+    if (src == SRC_PACKED || src == SRC_TEXT) {
+        if (!source)
+            return fail(CSA_ERR_INTERNAL, "radix_sort: keys of the text come with their source");
     } else {
         HIP_TRY(hipMemsetAsync(h->ghist, 0, MAX_PASSES * RADIX_BINS * sizeof(u32), s));
         HistArgs ha;
@@ -503,14 +522,18 @@ int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64
     }
     hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, plan.num_passes);
     HIP_TRY(hipGetLastError());
+    // (the digits of K-gram keys are the two bytes of a symbol, four times: where both take several values no pass is skipped)
+    const bool all_run = src == SRC_TEXT && !source->byte_wide;
     u32* h_hist = h->h_pinned + PINNED_HIST;
-    HIP_TRY(hipMemcpyAsync(h_hist, h->ghist, plan.num_passes * RADIX_BINS * sizeof(u32), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    if (!all_run) {
+        HIP_TRY(hipMemcpyAsync(h_hist, h->ghist, plan.num_passes * RADIX_BINS * sizeof(u32), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+    }
     bool run[MAX_PASSES];
     int n_run = 0;
     for (int p = 0; p < plan.num_passes; ++p) {
         bool trivial = false;
-        for (int d = 0; d < RADIX_BINS; ++d)
+        for (int d = 0; d < RADIX_BINS && !all_run; ++d)
             if (h_hist[p * RADIX_BINS + d] == n)
                 trivial = true;
         run[p] = !trivial;
@@ -543,11 +566,12 @@ int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64
         a.rank = rank_src;
         a.hop = hop;
         a.radix = radix;
-        if (packed) {
-            a.stream = packed->stream;
-            a.stream_words = packed->words;
-            a.sym_bits = packed->sym_bits;
-            a.key_bits = packed->key_bits;
+        if (source) {
+            a.text = source->text;
+            a.stream = source->stream;
+            a.stream_words = source->words;
+            a.sym_bits = source->sym_bits;
+            a.key_bits = source->key_bits;
         }
         int rc = next_ticket(L, &a.ticket);
         if (rc)
@@ -558,6 +582,8 @@ int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64
                 launch_onesweep<SRC_PAIRS>(h, a, s);
             else if (use_src == SRC_RANKS)
                 launch_onesweep<SRC_RANKS>(h, a, s);
+            else if (use_src == SRC_TEXT)
+                launch_onesweep<SRC_TEXT>(h, a, s);
             else
                 launch_onesweep<SRC_PACKED>(h, a, s);
         });
@@ -830,6 +856,7 @@ bool dense_generation(u32 m, u32 groups, u32 n)
 // of the caller's key width reaches inside 64 bits: S = 4 W 2^j symbols, which covers j generations after the first.
 struct PackedPlan {
     bool enabled;
+    bool byte_wide; // the symbols differ in one of their bytes only: half the passes over K-gram keys have nothing to do
     SymbolCodes codes;
     u32 skipped; // j
 };
@@ -846,6 +873,7 @@ PackedPlan plan_packed_text(const u32* bytehist, u32 n, int key_words, u64 room_
             pp.codes.hi[d] = (u8)nhi++;
     }
     const u32 codes = nlo * nhi;
+    pp.byte_wide = nlo == 1 || nhi == 1;
     if (codes > 256)
         return pp;
     const u32 b = codes <= 2 ? 1u : codes <= 4 ? 2u : codes <= 16 ? 4u : 8u;
@@ -868,49 +896,149 @@ PackedPlan plan_packed_text(const u32* bytehist, u32 n, int key_words, u64 room_
     return pp;
 }
 
-// Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their four symbols, with the ties marked,
-// in ra.sufs' array. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into idx[1]; the codes
-// live in the halves of key[0], their text order and the flags in key[1]. `marked` is left ready for sort_marked_runs.
-int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, ResolveArgs& marked)
+// Chunks of the text that the probe looks at: one in 16 while they are few, then one in 512, at most 2^20 suffixes.
+u32 probe_chunks(u32 n)
+{
+    const u32 few = n / (16 * SAMPLE_CHUNK) < PROBE_FEW_CHUNKS ? n / (16 * SAMPLE_CHUNK) : PROBE_FEW_CHUNKS;
+    const u32 k = n / (512 * SAMPLE_CHUNK) > few ? n / (512 * SAMPLE_CHUNK) : few;
+    return k < SAMPLE_CHUNKS_MAX ? k : SAMPLE_CHUNKS_MAX;
+}
+
+struct CodeTables {
+    u32 *counts, *marks; // zeroed together, with the counters of the probe and its table of up to PROBE_FEW_CHUNKS chunks
+    ProbeCounts* probe;
+    unsigned long long* table;
+    u32* cum;
+};
+
+CodeTables code_tables(const csa_handle* h)
+{
+    CodeTables c;
+    c.counts = h->code_tables;
+    c.marks = c.counts + SYMBOLS;
+    c.probe = reinterpret_cast<ProbeCounts*>(c.marks + RESOLVE_MARK_WORDS);
+    c.table = reinterpret_cast<unsigned long long*>(c.probe + 1);
+    c.cum = reinterpret_cast<u32*>(c.table + PROBE_TABLE);
+    return c;
+}
+
+// What a sort by codes starts from: the shares of the symbols, and for texts of PROBE_MIN symbols or more what a sample of the suffixes
+// (probe_chunks) shows about shared codes, on its way to *seen; ev_gen[1] tells that it is there. A large sample's table is
+// key[0], which holds nothing yet.
+int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
-    u32* const counts = h->code_tables; // [SYMBOLS], then the marks, then cum[SYMBOLS + 1]
-    u32* const marks = counts + SYMBOLS;
-    u32* const cum = marks + RESOLVE_MARK_WORDS;
-    HIP_TRY(hipMemsetAsync(counts, 0, (SYMBOLS + RESOLVE_MARK_WORDS) * sizeof(u32), s));
+    const CodeTables c = code_tables(h);
     const u32 chunks = (n + SAMPLE_CHUNK - 1) / SAMPLE_CHUNK;
-    // one chunk in 16, at least SAMPLE_CHUNKS_PER_BLOCK of them (or all there are) and at most SAMPLE_CHUNKS_MAX
-    u32 taken = chunks / 16 < SAMPLE_CHUNKS_PER_BLOCK ? SAMPLE_CHUNKS_PER_BLOCK : chunks / 16;
+    u64 zeros = (SYMBOLS + RESOLVE_MARK_WORDS) * sizeof(u32);
+    ProbeArgs a;
+    memset(&a, 0, sizeof(a));
+    if (n >= PROBE_MIN) {
+        a.text = d_text;
+        a.n = n;
+        a.chunks = chunks;
+        a.taken = probe_chunks(n);
+        a.cum = c.cum;
+        a.table_log2 = (u32)bit_length((u64)a.taken * SAMPLE_CHUNK - 1) + 1;
+        const u32 per_suffix = n / (a.taken * SAMPLE_CHUNK);
+        a.long_from = RESOLVE_MAX / per_suffix > 2 ? RESOLVE_MAX / per_suffix : 2;
+        a.counts = c.probe;
+        const bool few = a.taken <= PROBE_FEW_CHUNKS;
+        a.table = few ? c.table : reinterpret_cast<unsigned long long*>(h->key[0]);
+        zeros += sizeof(ProbeCounts);
+        if (few)
+            zeros += sizeof(u64) << a.table_log2;
+        else
+            HIP_TRY(hipMemsetAsync(a.table, 0, sizeof(u64) << a.table_log2, s));
+    }
+    HIP_TRY(hipMemsetAsync(c.counts, 0, zeros, s));
+    // one chunk in 16, at least SAMPLE_CHUNKS_MIN of them (or all there are) and at most SAMPLE_CHUNKS_MAX
+    u32 taken = chunks / 16 < SAMPLE_CHUNKS_MIN ? SAMPLE_CHUNKS_MIN : chunks / 16;
     taken = taken < SAMPLE_CHUNKS_MAX ? taken : SAMPLE_CHUNKS_MAX;
     taken = taken < chunks ? taken : chunks;
     const u64 sampled = (u64)taken * SAMPLE_CHUNK < n ? (u64)taken * SAMPLE_CHUNK : (u64)n;
     hipLaunchKernelGGL(sample_symbols_kernel, dim3((taken + SAMPLE_CHUNKS_PER_BLOCK - 1) / SAMPLE_CHUNKS_PER_BLOCK), dim3(SAMPLE_BLOCK), 0, s,
-                       d_text, n, chunks, taken, counts);
+                       d_text, n, chunks, taken, c.counts);
     const int weight_log2 = SAMPLE_LOG2 - bit_length(sampled - 1);
-    hipLaunchKernelGGL(symbol_shares_kernel, dim3(SYMBOLS / SHARES_TILE), dim3(SHARES_TILE), 0, s, (const u32*)counts, weight_log2,
-                       (u32)((sampled << weight_log2) + SYMBOLS), cum);
-    u32* const codes = reinterpret_cast<u32*>(h->key[1]);          // by virtual position
-    u8* const own = reinterpret_cast<u8*>(h->key[1]) + 4 * h->cap; // flags by text position
+    hipLaunchKernelGGL(symbol_shares_kernel, dim3(SYMBOLS / SHARES_TILE), dim3(SHARES_TILE), 0, s, (const u32*)c.counts, weight_log2,
+                       (u32)((sampled << weight_log2) + SYMBOLS), c.cum);
+    if (n >= PROBE_MIN) {
+        hipLaunchKernelGGL(probe_codes_kernel, dim3((a.taken * SAMPLE_CHUNK + PROBE_BLOCK - 1) / PROBE_BLOCK), dim3(PROBE_BLOCK), 0, s, a);
+        HIP_TRY(hipMemcpyAsync(seen, a.counts, sizeof(ProbeCounts), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipEventRecord(h->ev_gen[1], s)); // (recorded again when the generation ends)
+    }
+    HIP_TRY(hipGetLastError());
+    return CSA_OK;
+}
+
+// Whether a text is sorted by codes or by K-gram keys. Codes save passes, and lose time to suffixes that share one with others and
+// have to be told apart by the text. Both per suffix in picoseconds, from generation 0 of texts of 2^19 to 2^28 symbols on either kind of key:
+// independent symbols are 15 to 23 faster on codes, short texts by 25 us for the launches and a round trip alone; a line of the
+// text for every suffix costs about 20; a suffix is compared with the others of its run, at 0.2 to 0.5 each; collecting and
+// sorting the members of long runs that are out of order costs 60 each and 200 us in all.
+// Measured (ms; K-grams, codes, chosen, with the probe): 2^28 Zipf tokens 16.0, 11.0, 11.0; 2^28 symbols of a chain in which a symbol
+// has 3 successors 15.7, 38.8, 15.8; 20 successors 16.3, 34.4, 16.5; 2^28 symbols of 100000 phrases 16.4, 25.7, 16.5; 2^22 of them
+// 0.40, 0.72, 0.45; 2^20 of them 0.23, 0.44, 0.28.
+bool codes_pay(const ProbeCounts& c, u32 n)
+{
+    const double seen = (double)probe_chunks(n) * SAMPLE_CHUNK, per_seen = n / seen;
+    const double second = 2.0 * (c.second - c.third) / seen, third = 3.0 * (c.third - c.fourth) / seen; // in codes seen twice, thrice
+    const double more = ((double)c.again + c.second) / seen - second;                                    // ... thrice and more often
+    // The suffixes whose company the sample missed: a code of m suffixes shows x = m / per_seen of them on average, and e^x / x
+    // times as many suffixes belong to such codes as belong to codes seen twice; x follows from how many are seen thrice.
+    double x = second > 0 ? 2.0 * third / second : 0.0;
+    x = x < 1.0 / per_seen ? 1.0 / per_seen : x > 3.0 ? 3.0 : x;
+    double company = more + second * std::exp(x) / x;
+    company = company < 1.0 ? company : 1.0;
+    const double others = company > 0 ? 2.0 * (double)c.pairs / seen * per_seen / company : 0.0; // with the code of one with company
+    const double mixed = c.again ? (double)c.other / c.again : 0.0;
+    // read from the text, and compared with its run: at most RESOLVE_MAX others
+    double cost = company * (20.0 + 0.5 * mixed * (others < RESOLVE_MAX ? others : RESOLVE_MAX));
+    if (c.crowded > 4) // collected and sorted once more
+        cost += 60.0 * c.crowded / seen + 2e8 / n;
+    return cost < 18.0 + 2.5e7 / n;
+}
+
+// Where the codes live until the first pass has read them: by virtual position, with the flags by text position behind them.
+u32* codes_of(const csa_handle* h) { return reinterpret_cast<u32*>(h->key[1]); }
+u8* own_of(const csa_handle* h) { return reinterpret_cast<u8*>(h->key[1]) + 4 * h->cap; }
+
+int code_suffixes(Launch& L, const u16* d_text, u32 n, u32 tail)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    const u32* const cum = code_tables(h).cum;
     if (n >= SORT_WIDE_MIN) // 2048 tiles of the wide workgroups: four for each of those a device holds at a time
         hipLaunchKernelGGL(code_suffixes_kernel<CODE_WIDE_BLOCK>, dim3(hist_blocks(CODE_WIDE_BLOCK * CODE_ITEMS, n)), dim3(CODE_WIDE_BLOCK), 0,
-                           s, d_text, n, tail, (const u32*)cum, codes, own, h->ghist);
+                           s, d_text, n, tail, cum, codes_of(h), own_of(h), h->ghist);
     else
         hipLaunchKernelGGL(code_suffixes_kernel<CODE_BLOCK>, dim3(hist_blocks(CODE_BLOCK * CODE_ITEMS, n)), dim3(CODE_BLOCK), 0, s, d_text, n,
-                           tail, (const u32*)cum, codes, own, h->ghist);
+                           tail, cum, codes_of(h), own_of(h), h->ghist);
+    HIP_TRY(hipGetLastError());
+    return CSA_OK;
+}
+
+// Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their four symbols, with the ties marked,
+// in ra.sufs' array; code_suffixes ran before. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into
+// idx[1]; the codes live in the halves of key[0]. `marked` is left ready for sort_marked_runs.
+int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, ResolveArgs& marked)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
     hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, CODE_PASSES);
     u32* const sorted[2] = {reinterpret_cast<u32*>(h->key[0]), reinterpret_cast<u32*>(h->key[0]) + h->cap};
     static_assert(CODE_PASSES % 2 == 0, "the sorted codes end in the first half of key[0], their suffixes in idx[0]");
     for (int p = 0; p < CODE_PASSES; ++p) {
         OnesweepArgs a;
-        a.keys_in = p == 0 ? codes : sorted[p & 1];
+        a.keys_in = p == 0 ? codes_of(h) : sorted[p & 1];
         a.vals_in = h->idx[p & 1];
         a.keys_out = sorted[(p + 1) & 1];
         a.vals_out = h->idx[(p + 1) & 1];
         a.n = n;
         a.text_n = n;
         a.tail = tail;
-        a.own = own;
+        a.own = own_of(h);
         a.shift = 8 * p;
         a.bits = 8;
         a.digit_base = h->digit_base + p * RADIX_BINS;
@@ -937,7 +1065,7 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, Resolv
     marked.n = n;
     marked.ell = ell;
     marked.sufs_out = h->idx[1];
-    marked.marks = marks;
+    marked.marks = code_tables(h).marks;
     marked.unordered = h->counts + 4;
     hipLaunchKernelGGL(resolve_runs_kernel, dim3((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, marked);
     HIP_TRY(hipGetLastError());
@@ -1074,8 +1202,11 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     u32* const bytehist = h->ghist + MAX_PASSES * RADIX_BINS;
     PackedPlan pp;
     memset(&pp, 0, sizeof(pp));
-    if (h->pack_symbols) {
+    auto count_bytes = [&] {
         hipLaunchKernelGGL(text_byte_hist_kernel, dim3(hist_blocks(256 * 8 * 16, n)), dim3(256), 0, s, d_text, n, bytehist);
+    };
+    if (h->pack_symbols) {
+        count_bytes();
         u32* h_bytes = h->h_pinned + PINNED_HIST;
         HIP_TRY(hipMemcpyAsync(h_bytes, bytehist, 2 * RADIX_BINS * sizeof(u32), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
@@ -1086,15 +1217,29 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     for (u64 c = ell; c < wide_ell; c += (c < wide_ell - c ? c : wide_ell - c))
         ++folded;
     const u32 tail = n < ell ? n : ell;
+    int rc;
+    bool coded = !pp.enabled && !pp.byte_wide;
+    if (coded) {
+        const bool probed = n >= PROBE_MIN, ahead = !probed || n < CODE_AHEAD_MAX;
+        ProbeCounts* const seen = reinterpret_cast<ProbeCounts*>(h->h_pinned + PINNED_HIST);
+        if ((rc = share_symbols(L, d_text, n, seen)) != CSA_OK || (ahead && (rc = code_suffixes(L, d_text, n, tail)) != CSA_OK))
+            return rc;
+        if (probed) {
+            HIP_TRY(hipEventSynchronize(h->ev_gen[1]));
+            coded = codes_pay(*seen, n);
+        }
+        if (coded && !ahead && (rc = code_suffixes(L, d_text, n, tail)) != CSA_OK)
+            return rc;
+    }
     int passes = 0, p1 = 0, in_out = 0;
     u64* K[2] = {h->key[0], h->key[1]};
     u32* V[2] = {h->idx[0], h->idx[1]};
     int cur = 0; // the (K, V) set that holds the sorted pairs
-    int rc;
     ResolveArgs marked;
+    TextSource ps;
+    memset(&ps, 0, sizeof(ps));
     if (pp.enabled) {
         // the code stream lives in rank[], which nothing uses before the sorted list is ranked
-        PackedSource ps;
         u32* const stream = h->rank;
         ps.stream = stream;
         ps.sym_bits = pp.codes.bits;
@@ -1110,10 +1255,18 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                            plan.num_passes, gramhist, h->ghist);
         HIP_TRY(hipGetLastError());
         rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, plan, &in_out, &p1, nullptr, 0, 0, &ps);
-    } else {
+    } else if (coded) {
         rc = sort_by_codes(L, d_text, n, tail, ell, marked);
         p1 = CODE_PASSES;
         in_out = 1; // idx[1] holds the list, key[0] and key[1] what the sort has left behind
+    } else {
+        if (!h->pack_symbols)
+            count_bytes();
+        ps.text = d_text;
+        ps.byte_wide = pp.byte_wide || !h->pack_symbols;
+        hipLaunchKernelGGL(text_hist_expand_kernel, dim3(1), dim3(256), 0, s, d_text, n, (const u32*)bytehist, h->ghist);
+        HIP_TRY(hipGetLastError());
+        rc = radix_sort(L, SRC_TEXT, n, tail, K[0], V[0], K[1], V[1], n, make_plan(0, 64), &in_out, &p1, nullptr, 0, 0, &ps);
     }
     if (rc)
         return rc;
@@ -1159,7 +1312,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         ra.level_ell[i] = (u32)wide_ell << i;
         ra.level_drop[i] = (ell - ra.level_ell[i]) * pp.codes.bits;
     }
-    rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], level_counts, pp.enabled ? nullptr : &marked, &passes);
+    rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], level_counts, coded ? &marked : nullptr, &passes);
     range_gen0.close();
     if (rc)
         return rc;

@@ -18,8 +18,13 @@
 // reads the strings of such suffixes from the text (and of no others: a random 128-byte line each, which is what bounds it;
 // 8.0 ms on 1e9 tokens; 14.8 when it read those of the flagged ones too), sorts every run of up to RESOLVE_MAX suffixes inside its
 // tile and sets bit 31 of every suffix that ties with its left neighbour, which is all the rank step needs to know. Longer runs
-// are nearly always one string repeated and in order as they stand; the rare ones that are not are collected and radix
-// sorted by the string itself.
+// that are one string repeated are in order as they stand; those that are not are collected and radix sorted by the string itself.
+//
+// The shares are those of single symbols, so the codes are only as even as neighbouring symbols are independent. Where a symbol has few
+// successors (phrases, records), strings that are rare by the shares of their symbols are common, and most suffixes end up in long
+// runs of one code: such texts lose more than they win (2^28 symbols of a chain with 3 successors each: generation 0 38.8 ms,
+// 15.7 on K-gram keys). probe_codes_kernel looks for that in a sample of the suffixes, and the first sort of such a text takes
+// K-gram keys. Short texts are not probed.
 #pragma once
 
 #include "device_utils.hpp"
@@ -33,8 +38,9 @@ namespace csa {
 constexpr int SYMBOLS = 1 << 16;
 constexpr int SAMPLE_BLOCK = 1024;
 constexpr u32 SAMPLE_CHUNK = 64;              // consecutive symbols, one wave's worth
-constexpr u32 SAMPLE_CHUNKS_PER_BLOCK = 256;  // 16384 symbols: a 16-bit counter holds them all
-constexpr u32 SAMPLE_CHUNKS_MAX = 1u << 14;   // 2^20 symbols are looked at, at most
+constexpr u32 SAMPLE_CHUNKS_PER_BLOCK = 64;   // 4096 symbols: a 16-bit counter holds them all (16384: 9 us more at 2^20 symbols)
+constexpr u32 SAMPLE_CHUNKS_MIN = 256;        // 2^14 symbols are looked at, at least ...
+constexpr u32 SAMPLE_CHUNKS_MAX = 1u << 14;   // ... and 2^20 at most
 constexpr int SAMPLE_LOG2 = 20;
 
 // Chunk c of a sample of `taken` out of `chunks`: one of the c-th of `taken` equal stretches of the text, at the place in it that the
@@ -42,10 +48,11 @@ constexpr int SAMPLE_LOG2 = 20;
 // in rows of a fixed length (2^28 symbols in rows of 1024, the first 64 of each over values of their own: at a stride of
 // 16384 symbols only those columns were sampled, most suffixes shared their code with thousands of others, and generation 0
 // took 37.0 ms).
-__device__ __forceinline__ u32 sampled_chunk(u32 c, u32 chunks, u32 taken)
+// `start` shifts the places.
+__device__ __forceinline__ u32 sampled_chunk(u32 c, u32 chunks, u32 taken, u32 start)
 {
     const u32 lo = (u32)((u64)c * chunks / taken), hi = (u32)((u64)(c + 1) * chunks / taken);
-    return lo + (u32)(((u64)(c * 0x9E3779B1u) * (hi - lo)) >> 32);
+    return lo + (u32)(((u64)(c * 0x9E3779B1u + start) * (hi - lo)) >> 32);
 }
 
 // counts[s] += occurrences of symbol s in the sample: `taken` chunks (all of them when the text is short).
@@ -62,7 +69,7 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16*
     for (u32 r = t / SAMPLE_CHUNK; r < SAMPLE_CHUNKS_PER_BLOCK; r += SAMPLE_BLOCK / SAMPLE_CHUNK) {
         const u32 c = first + r;
         if (c < taken) {
-            const u64 p = (u64)sampled_chunk(c, chunks, taken) * SAMPLE_CHUNK + (t & (SAMPLE_CHUNK - 1));
+            const u64 p = (u64)sampled_chunk(c, chunks, taken, 0) * SAMPLE_CHUNK + (t & (SAMPLE_CHUNK - 1));
             if (p < n) {
                 const u32 s = text[p];
                 atomicAdd(&s_cnt[s >> 1], (s & 1u) ? 0x10000u : 1u);
@@ -116,6 +123,117 @@ __global__ __launch_bounds__(SHARES_TILE) void symbol_shares_kernel(const u32* _
         cum[SYMBOLS] = 0xFFFFFFFFu;
 }
 
+// ---- do the codes tell this text's suffixes apart? ----
+
+// The interval of codes [low, high) of the string of four symbols with shares lo[k], width[k]: the map from the last symbol's entries
+// to both ends is monotone, so the next string starts at `high` or later, and low + 1, where it is below `high`, is above every
+// code of a smaller string and below every code of a larger one: true if the string takes that code, which is its own then.
+__device__ __forceinline__ bool string_code(const u32 (&lo)[4], const u32 (&width)[4], u32& code)
+{
+    u32 low = lo[3], high = lo[3] + width[3];
+#pragma unroll
+    for (int q = 2; q >= 0; --q) {
+        low = lo[q] + (u32)(((u64)width[q] * low) >> 32);
+        high = lo[q] + (u32)(((u64)width[q] * high) >> 32);
+    }
+    const bool alone = high - low >= 2u;
+    code = low + (alone ? 1u : 0u);
+    return alone;
+}
+
+constexpr int PROBE_BLOCK = 256;
+constexpr u32 PROBE_START = 0x55555555u; // (the sample of the symbols is taken elsewhere: what its own places show is too good)
+
+// What a sample of suffixes shows about codes that are not one string's alone: how often a suffix finds its code taken by one, two,
+// three others and so on, by another string, by so many that a run of it is longer than RESOLVE_MAX in the whole text.
+struct ProbeCounts {
+    u32 again;  // suffixes that find their code taken ...
+    u32 second, third, fourth; // ... by one, by two, by three others
+    u32 other;  // of `again`: whose string is not that of the first one there
+    u32 crowded; // of `other`: by `long_from` others or more
+    unsigned long long pairs; // pairs of suffixes with one code
+};
+static_assert(sizeof(ProbeCounts) == 8 * sizeof(u32), "the counters take eight words of the tables");
+
+struct ProbeArgs {
+    const u16* text;
+    u32 n;
+    u32 chunks, taken; // of SAMPLE_CHUNK suffixes (sampled_chunk)
+    const u32* cum;
+    unsigned long long* table; // [1 << table_log2], zeroed, at least twice as many as suffixes are looked at
+    u32 table_log2;
+    u32 long_from;
+    ProbeCounts* counts; // zeroed
+};
+
+// An entry of the table is a code (high half), eight bits of the first string's hash and the number of suffixes that came.
+// At most 2^20 suffixes come, so a count never reaches the hash. Bounded by the latency of the table's atomics (a random line each).
+__global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
+{
+    __shared__ unsigned long long s_pairs[PROBE_BLOCK / WAVE];
+    __shared__ u32 s_cnt[6];
+    const u32 t = threadIdx.x;
+    if (t < 6)
+        s_cnt[t] = 0;
+    __syncthreads();
+    u32 pairs = 0, flags = 0;
+    const u64 i = (u64)blockIdx.x * PROBE_BLOCK + t;
+    const u32 c = (u32)(i / SAMPLE_CHUNK);
+    if (c < a.taken) {
+        const u64 x = (u64)sampled_chunk(c, a.chunks, a.taken, PROBE_START) * SAMPLE_CHUNK + (i & (SAMPLE_CHUNK - 1));
+        if (x < a.n) {
+            u32 lo[4], width[4], hash = 0, code;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const u32 s = x + k < a.n ? a.text[x + k] : 0u;
+                u32 pair[2];
+                __builtin_memcpy(pair, a.cum + s, 8); // entries s and s + 1 (4-byte aligned)
+                lo[k] = pair[0];
+                width[k] = pair[1] - pair[0];
+                hash = (hash + s + 1u) * 0x9E3779B1u;
+            }
+            if (!string_code(lo, width, code)) {
+                const unsigned long long entry = ((unsigned long long)code << 32) | (hash >> 24 << 24) | 1u;
+                const u32 mask = (1u << a.table_log2) - 1u;
+                u32 slot = (code * 0x9E3779B1u) >> (32 - a.table_log2);
+                for (u32 tries = 0; tries <= mask; ++tries, slot = (slot + 1u) & mask) { // (half of the table stays empty)
+                    unsigned long long seen = atomicCAS(&a.table[slot], 0ull, entry);
+                    if (seen == 0)
+                        break;
+                    if ((u32)(seen >> 32) != code)
+                        continue;
+                    seen = atomicAdd(&a.table[slot], 1ull);
+                    const u32 before = (u32)seen & 0xFFFFFFu;
+                    const bool other = (((u32)seen ^ (u32)entry) >> 24) != 0;
+                    pairs = before;
+                    flags = 1u | (before == 1u ? 2u : 0u) | (before == 2u ? 4u : 0u) | (before == 3u ? 8u : 0u) | (other ? 16u : 0u) |
+                            (other && before >= a.long_from ? 32u : 0u);
+                    break;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const u64 b = __ballot((flags >> k) & 1u);
+        if ((t & 63u) == 0 && b)
+            atomicAdd(&s_cnt[k], (u32)__popcll(b));
+    }
+    const u32 sum = wave_reduce_sum(pairs); // at most 64 * 2^20
+    if ((t & 63u) == 0)
+        s_pairs[t / WAVE] = sum;
+    __syncthreads();
+    if (t < 6 && s_cnt[t])
+        atomicAdd(reinterpret_cast<u32*>(a.counts) + t, s_cnt[t]);
+    if (t == 0) {
+        unsigned long long all = 0;
+        for (int w = 0; w < PROBE_BLOCK / WAVE; ++w)
+            all += s_pairs[w];
+        if (all)
+            atomicAdd(&a.counts->pairs, all);
+    }
+}
+
 // ---- the codes of all suffixes, and the digit counts of the four passes ----
 
 constexpr int CODE_BLOCK = 256;
@@ -125,16 +243,14 @@ constexpr int CODE_PASSES = 4;
 constexpr int CODE_COPIES = 8;
 
 // codes[v] = code of the suffix at virtual position v (virtual_to_suffix with `tail` = min(n, 4)); bit x & 7 of own[x >> 3]: the
-// suffix at text position x has a code that only its string can have. [low, high) below is the string's interval: the map from
-// the last symbol's entries to both ends is monotone, so the next string starts at `high` or later, and low + 1, where it
-// is below `high`, is above every code of a smaller string and below every code of a larger one. Bounded by the lookups
+// suffix at text position x has a code that only its string can have (string_code). Bounded by the lookups
 // of cum[]: one 8-byte gather per symbol (the table is 256 KB: it lives in the L2s), shared by the four suffixes it appears in.
 // BLOCK: the 32 KB of digit counters decide how many waves a CU holds, 16 in workgroups of 256 and 32 in workgroups of 1024,
 // which code 1e9 tokens in 2.27 instead of 3.06 ms and 2^28 in 0.58 instead of 0.78 (512: 2.69, 0.66; 256 with half the
 // counters: 2.92, 0.75). Short texts take 256, so that there are workgroups for every CU.
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void code_suffixes_kernel(const u16* __restrict__ text, u32 n, u32 tail, const u32* __restrict__ cum,
-                                                                   u32* __restrict__ codes, u8* __restrict__ own, u32* __restrict__ ghist)
+                                                              u32* __restrict__ codes, u8* __restrict__ own, u32* __restrict__ ghist)
 {
     constexpr u32 TILE = BLOCK * CODE_ITEMS;
     __shared__ u64 s_text[(TILE + 3 + 6) / 4 + 2];
@@ -162,15 +278,9 @@ __global__ __launch_bounds__(BLOCK) void code_suffixes_kernel(const u16* __restr
         u32 code[CODE_ITEMS], owners = 0;
 #pragma unroll
         for (int k = 0; k < CODE_ITEMS; ++k) {
-            u32 low = lo[k + 3], high = lo[k + 3] + width[k + 3];
-#pragma unroll
-            for (int q = 2; q >= 0; --q) {
-                low = lo[k + q] + (u32)(((u64)width[k + q] * low) >> 32);
-                high = lo[k + q] + (u32)(((u64)width[k + q] * high) >> 32);
-            }
-            const u32 alone = high - low >= 2u ? 1u : 0u;
-            code[k] = low + alone;
-            owners |= alone << k;
+            const u32 lo4[4] = {lo[k], lo[k + 1], lo[k + 2], lo[k + 3]};
+            const u32 width4[4] = {width[k], width[k + 1], width[k + 2], width[k + 3]};
+            owners |= (string_code(lo4, width4, code[k]) ? 1u : 0u) << k;
         }
         const u64 x0 = p0 + (u64)t * CODE_ITEMS;
         if (x0 < n)

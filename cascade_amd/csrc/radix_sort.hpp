@@ -29,7 +29,8 @@ enum : int {
     SRC_PAIRS = 0, // keys_in[i], vals_in[i]
     SRC_CODED = 1, // generation 0, first pass: keys_in holds the codes of virtual positions (coded_keys.hpp), the suffixes follow from them
     SRC_RANKS = 2, // a dense later generation, first pass: pair i = ((rank[i], rank[i + hop]), i), built from rank[]
-    SRC_PACKED = 3 // generation 0 over a small alphabet, first pass: the key of virtual position i is cut from the code stream
+    SRC_PACKED = 3, // generation 0 over a small alphabet, first pass: the key of virtual position i is cut from the code stream
+    SRC_TEXT = 4   // generation 0 on K-gram keys, first pass: the pair of virtual position i is built from the text
 };
 
 // Key of text position i in a dense generation: its rank, then the rank of the suffix `hop` symbols on (0 past the
@@ -186,7 +187,8 @@ __global__ __launch_bounds__(256) void rank_hist_combine_kernel(u32* ghist, int 
 }
 
 // Histogram of the low and of the high byte of every symbol of the text: bytehist[0][d], bytehist[1][d].
-// They tell whether the alphabet is small enough for keys of packed symbols.
+// They tell whether the alphabet is small enough for keys of packed symbols, and the eight digit histograms of the K-gram keys
+// follow from them (text_hist_expand_kernel).
 constexpr int TEXT_HIST_COPIES = 16;
 
 __global__ __launch_bounds__(256) void text_byte_hist_kernel(const u16* __restrict__ text, u32 n, u32* bytehist)
@@ -229,6 +231,28 @@ __global__ __launch_bounds__(256) void text_byte_hist_kernel(const u16* __restri
     }
 }
 
+// ghist[p][d] for the 8 byte-wide passes over the K-gram keys of all n suffixes. Pass p looks at byte (p & 1) of the symbol at offset
+// pos = 3 - p / 2 of each suffix, i.e. at T[pos .. n) followed by min(pos, n) padding zeros: the whole-text byte
+// histogram minus the first min(pos, n) symbols, plus that many zeros.
+__global__ __launch_bounds__(256) void text_hist_expand_kernel(const u16* __restrict__ text, u32 n, const u32* __restrict__ bytehist, u32* ghist)
+{
+    const u32 d = threadIdx.x;
+    for (int p = 0; p < 8; ++p) {
+        const u32 byte = p & 1;
+        const u32 pos = 3 - p / 2;
+        const u32 cut = pos < n ? pos : n;
+        u32 v = bytehist[byte * RADIX_BINS + d];
+        for (u32 i = 0; i < cut; ++i) {
+            const u32 b = byte ? (text[i] >> 8) : (text[i] & 0xFFu);
+            if (b == d)
+                --v;
+        }
+        if (d == 0)
+            v += cut;
+        ghist[p * RADIX_BINS + d] = v;
+    }
+}
+
 // digit_base[p][d] = number of pairs whose pass-p digit is < d.
 __global__ __launch_bounds__(256) void radix_scan_hist_kernel(const u32* ghist, u32* digit_base, int num_passes)
 {
@@ -254,8 +278,8 @@ struct OnesweepArgs {
     void* keys_out;
     u32* vals_out;
     u32 n;      // pairs
-    u32 text_n; // symbols in the text (SRC_CODED, SRC_PACKED)
-    u32 tail;   // suffixes that run off the text inside their key (SRC_CODED, SRC_PACKED)
+    u32 text_n; // symbols in the text (SRC_CODED, SRC_PACKED, SRC_TEXT)
+    u32 tail;   // suffixes that run off the text inside their key (SRC_CODED, SRC_PACKED, SRC_TEXT)
     int shift;
     int bits;
     const u32* digit_base; // [256] for this pass
@@ -267,6 +291,7 @@ struct OnesweepArgs {
     u32 tiles;             // tiles of the pass = workgroups of the launch
     u32 epoch;
     u32* err;
+    const u16* text = nullptr; // SRC_TEXT
     const u8* own = nullptr;   // SRC_CODED: flags by text position, 8 to a byte
     const u32* rank = nullptr; // SRC_RANKS: rank[] by text position ...
     u32 hop = 0;               // ... the distance to the second rank of a key ...
@@ -371,10 +396,20 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
 #define CSA_LDS_ORDER() __builtin_amdgcn_wave_barrier() /* CPU emulation: lanes are threads, order them for real */
 #define CSA_OPAQUE(x) ((void)0)
 #endif
-    // ---- first pass of generation 0 over a small alphabet ----
+    // ---- first pass of generation 0 on K-gram keys: stage the tile's stretch of the text in LDS ----
     // The tile covers consecutive virtual positions, i.e. (after the few tail suffixes of tile 0) consecutive text
-    // positions; the (still unused) reorder buffer holds their stretch of the code stream (TILE * sym_bits bits and a key's
-    // worth more), and each key is cut from it.
+    // positions j0, j0 + 1, ...; the (still unused) reorder buffer holds the stretch, and each key is assembled
+    // from three LDS words instead of four narrow global loads.
+    u32 j0 = 0, sym_off = 0;
+    if constexpr (SRC == SRC_TEXT) {
+        const u32 first_virtual = (u32)base > a.tail ? (u32)base : a.tail;
+        j0 = first_virtual - a.tail;
+        const u32 count = (u32)TILE - (first_virtual - (u32)base) + 3u; // the last key reaches 3 symbols further
+        static_assert(sizeof(KeyT) * TILE >= 8 * ((TILE + 3 + 6) / 4 + 2), "the staged text must fit the reorder buffer");
+        sym_off = stage_text(a.text, a.text_n, j0, count, reinterpret_cast<u64*>(s_keys), t, BLOCK);
+        __syncthreads();
+    }
+    // the same over a small alphabet: the tile's stretch of the code stream (TILE * sym_bits bits and a key's worth more)
     u64 stream_bit0 = 0;
     if constexpr (SRC == SRC_PACKED) {
         const u32 first_virtual = (u32)base > a.tail ? (u32)base : a.tail;
@@ -387,10 +422,15 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
             s_codes[i] = first_word + i < a.stream_words ? a.stream[first_word + i] : 0u;
         __syncthreads();
     }
-    auto text_key = [&](u32 i) -> u64 { // key of virtual position i of this tile (SRC_PACKED)
+    auto text_key = [&](u32 i) -> u64 { // key of virtual position i of this tile (SRC_TEXT, SRC_PACKED)
+        if constexpr (SRC == SRC_PACKED) {
+            if (i < a.tail)
+                return packed_window(a.stream, (u64)(a.text_n - 1u - i) * a.sym_bits, a.key_bits);
+            return packed_window(reinterpret_cast<const u32*>(s_keys), (u64)(i - a.tail) * a.sym_bits - stream_bit0, a.key_bits);
+        }
         if (i < a.tail)
-            return packed_window(a.stream, (u64)(a.text_n - 1u - i) * a.sym_bits, a.key_bits);
-        return packed_window(reinterpret_cast<const u32*>(s_keys), (u64)(i - a.tail) * a.sym_bits - stream_bit0, a.key_bits);
+            return load_kgram(a.text, a.text_n, a.text_n - 1u - i, 0);
+        return staged_kgram(reinterpret_cast<const u32*>(s_keys), (i - a.tail) - j0 + sym_off);
     };
 
     // ---- load: wave-striped, so that consecutive lanes read consecutive pairs ----
@@ -514,7 +554,7 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
                 val[k] = x | ((a.own[x >> 3] >> (x & 7u)) & 1u ? OWN_CODE : 0u);
             }
         } else if (VALS && local < valid)
-            val[k] = SRC == SRC_PACKED ? virtual_to_suffix((u32)(base + local), a.text_n, a.tail)
+            val[k] = (SRC == SRC_TEXT || SRC == SRC_PACKED) ? virtual_to_suffix((u32)(base + local), a.text_n, a.tail)
                      : SRC == SRC_RANKS                     ? (u32)(base + local)
                                                             : a.vals_in[base + local];
     }

@@ -654,7 +654,7 @@ def test_first_sort_on_codes_with_runs_that_share_a_code(emu):
     out of order: the long mixed ones are collected and radix sorted. Suffix array and generation sizes against the oracle."""
     T = texts.text_with_shared_codes(130000, [2, 5, 63, 64, 65, 70, 90], 3)
     got, active, _ = emu_sort(emu, T, 1)
-    assert emu_sort.passes[0] > 4  # four passes over all suffixes, and those over the collected runs
+    assert emu_sort.passes[0] > 8  # four passes over all suffixes, and eight over the collected runs
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
 
@@ -699,4 +699,31 @@ def test_first_sort_on_codes_of_a_text_in_rows_of_a_fixed_length(emu, row):
     got, active, _ = emu_sort(emu, T, 1)
     assert emu_sort.passes[0] == 4
     sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
+@pytest.mark.parametrize("n,repeats,pack", [(90000, 70, True), (90000, 70, False), (130000, 90, True), (130000, 90, False)])
+def test_texts_whose_suffixes_share_codes_are_sorted_by_kgrams(emu, n, repeats, pack):
+    """A sample of the suffixes shows that many codes belong to long runs of several strings: the first sort takes K-gram keys, all
+    eight passes of them, with and without the byte counts of the text at hand, and with the codes made before the sample was
+    looked at (90000 symbols in this build) or not made at all. Suffix array and generation sizes against the oracle; the same
+    text without the plants is sorted by codes."""
+    T = texts.text_with_shared_codes(n, [repeats] * 60, n)
+    got, active, _ = emu_sort(emu, T, 1, pack=pack)
+    assert emu_sort.passes[0] == 8
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    T = texts.text_with_shared_codes(n, [], n)
+    emu_sort(emu, T, 1, pack=pack)
+    assert emu_sort.passes[0] == 4
+
+
+@pytest.mark.parametrize("symbols", [np.arange(97, 123), np.arange(256) * 256, np.array([0, 7])])
+def test_first_sort_of_byte_wide_symbols_takes_half_the_passes(emu, symbols):
+    """Symbols that differ in one byte only and a key too wide for packed symbols: K-gram keys, whose other bytes need no pass."""
+    rng = np.random.default_rng(symbols.size)
+    T = rng.choice(symbols, 3001).astype(np.uint16)
+    T[2000:2600] = T[100:700]
+    got, active, _ = emu_sort(emu, T, 4)
+    sa, counts = oracle_lib.prefix_doubling(T, 4)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts

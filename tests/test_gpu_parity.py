@@ -692,3 +692,18 @@ def test_kernel_timing_counts_every_radix_pass(torch_mod, letters):
         stats = s.last_stats
     assert stats["radix_launches"] == sum(stats["passes"]) >= 4
     assert stats["radix_pairs"] >= T.size * stats["passes"][0] and stats["radix_ms"] > 0
+
+
+@pytest.mark.parametrize("n,phrases,passes", [(1 << 20, 5000, 8), ((1 << 22) + 5, 5000, 8), (1 << 19, 0, 4)])
+def test_first_sort_chooses_between_codes_and_kgrams(torch_mod, n, phrases, passes):
+    """Texts of 2^19 symbols or more are probed for codes that many suffixes share. A text of phrases goes by K-gram keys (2^20: coded
+    before the host knows; past 2^22: not coded at all), one of independent symbols by codes; all against the oracle."""
+    from cascade_amd import PartitionSorter
+    T = texts.text_of_phrases(n, phrases, 10, 60, 1) if phrases else np.random.default_rng(n).integers(1, 50000, n).astype(np.uint16)
+    with PartitionSorter(T.size, key_words=1) as s:
+        print(f"  {n} symbols of {phrases} phrases", flush=True)
+        got = gpu_sa40(torch_mod, s, T)
+        stats = s.last_stats
+    assert stats["passes"][0] == passes
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts

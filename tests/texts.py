@@ -85,3 +85,16 @@ def text_with_shared_codes(n, repeats, seed):
                 T[p:p + 4] = [base, base + 1, base + 2, base + 4 - (mixed and int(rng.integers(0, 2)))]
     T[-2:] = 0
     return T
+
+
+def text_of_phrases(n, phrases, lo, hi, seed):
+    """n token ids made of `phrases` different sequences of lo to hi random ids each, drawn with Zipf(0.8) shares: symbols are rare and
+    their successors few, so that the shares of single symbols say little about the strings that occur."""
+    rng = np.random.default_rng(seed)
+    ln = rng.integers(lo, hi + 1, phrases)
+    start = np.cumsum(ln) - ln
+    ids = rng.integers(1, 50000, int(ln.sum())).astype(np.uint16)
+    share = np.arange(1, phrases + 1) ** -0.8
+    draws = rng.choice(phrases, n // lo + 1, p=share / share.sum())
+    at = np.repeat(start[draws] - (np.cumsum(ln[draws]) - ln[draws]), ln[draws]) + np.arange(int(ln[draws].sum()))
+    return ids[at[:n]]
