@@ -786,16 +786,22 @@ int windowed_rank_update(Launch& L, const u32* pos, const DeferBuffers& buf, u32
     return CSA_OK;
 }
 
-// Sizes of the rank step's tables for a list of m suffixes cut into tiles of `tile` elements.
+// The smallest tile of the kernels that share the rank step's tables: the tables are sized for it.
+constexpr int smaller(int a, int b) { return a < b ? a : b; }
+constexpr int TABLE_TILE = smaller(smaller(RANK_TILE, SMALL_TILE), smaller(COLLECT_TILE, STEP_TILE));
+
+// Sizes of the rank step's tables for a list of m suffixes cut into tiles of TILE elements.
 struct RankTables {
     u32 tiles, slab, slabs;
     u32 *tile_agg, *tile_prefix, *tile_splits, *slab_total;
 };
 
-RankTables rank_tables(csa_handle* h, u32 m, u32 tile)
+template <int TILE>
+RankTables rank_tables(csa_handle* h, u32 m)
 {
+    static_assert(TILE >= TABLE_TILE, "the tables hold fewer tiles than this list has");
     RankTables r;
-    r.tiles = (u32)(((u64)m + tile - 1) / tile);
+    r.tiles = (u32)(((u64)m + TILE - 1) / TILE);
     r.slab = (r.tiles + RERANK_SLABS - 1) / RERANK_SLABS;
     r.slabs = (r.tiles + r.slab - 1) / r.slab;
     r.tile_agg = h->tile_tables;
@@ -1078,7 +1084,7 @@ int sort_marked_runs(Launch& L, ResolveArgs a, int* passes)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
-    const RankTables r = rank_tables(h, a.n, COLLECT_TILE);
+    const RankTables r = rank_tables<COLLECT_TILE>(h, a.n);
     a.keys = h->key[1];
     a.members = h->idx[3];
     a.places = h->idx[2];
@@ -1120,7 +1126,7 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
-    const RankTables r = rank_tables(h, ra.m, RANK_TILE);
+    const RankTables r = rank_tables<RANK_TILE>(h, ra.m);
     ra.tile_agg = r.tile_agg;
     ra.tile_prefix = r.tile_prefix;
     ra.tile_splits = r.tile_splits;
@@ -1410,7 +1416,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         }
         if (ordinals_in_rank)
             return fail(CSA_ERR_INTERNAL, "generation %d reads ranks but the one before it left ordinals", gen);
-        const RankTables r = rank_tables(h, m_in, SMALL_TILE);
+        const RankTables r = rank_tables<SMALL_TILE>(h, m_in);
         u32* nr_list = reinterpret_cast<u32*>(key_out); // refined rank at every place of the sorted list
         // 1. gather rank[x + h]; small groups are sorted and ranked inside their tile, members of large groups set aside
         SmallSortArgs sa;
@@ -1463,7 +1469,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                 // where every large group's members start in the list of large-group members, and how many there are
                 // (counts[4]): a prefix sum over the group table
                 u32* big_first = reinterpret_cast<u32*>(bkey[1]);
-                const RankTables gr = rank_tables(h, groups, 1024);
+                const RankTables gr = rank_tables<1024>(h, groups);
                 hipLaunchKernelGGL((big_prefix_kernel<false>), dim3(gr.tiles), dim3(256), 0, s, (const u32*)h->gstart[gp], groups, maxg, big_first,
                                    gr.tile_agg, gr.tile_splits, (const u32*)gr.tile_prefix, (const u32*)gr.slab_total, gr.slab, gr.slabs,
                                    h->counts + 4);
@@ -1521,7 +1527,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                 pa.err = h->counts + 2;
                 // (512 x 4 tiles: 0.8 ms per sort of the adversarial workload ahead of 256 x 4; 8 elements per thread: 8 ms behind)
                 constexpr int PRESORTED_BLOCK = 512, PRESORTED_ITEMS = 4;
-                const RankTables pr = rank_tables(h, m_in, PRESORTED_BLOCK * PRESORTED_ITEMS);
+                const RankTables pr = rank_tables<PRESORTED_BLOCK * PRESORTED_ITEMS>(h, m_in);
                 pa.tile_agg = pr.tile_agg;
                 pa.tile_splits = pr.tile_splits;
                 pa.tile_prefix = pr.tile_prefix;
@@ -1555,7 +1561,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                 pa.nr_out = nr_list;
                 pa.err = h->counts + 2;
                 // (the tile tables are free between the small-group kernel and the counting pass below)
-                const RankTables pr = rank_tables(h, big, RANK_TILE);
+                const RankTables pr = rank_tables<RANK_TILE>(h, big);
                 pa.tile_agg = pr.tile_agg;
                 pa.tile_splits = pr.tile_splits;
                 pa.tile_prefix = pr.tile_prefix;
@@ -2093,7 +2099,7 @@ WorkspaceSizes workspace_sizes(u64 cap)
 {
     WorkspaceSizes w;
     const u64 sort_tiles = (cap + SORT_TILE - 1) / SORT_TILE;
-    const u64 rank_tiles = (cap + RANK_TILE - 1) / RANK_TILE;
+    const u64 rank_tiles = (cap + TABLE_TILE - 1) / TABLE_TILE;
     w.lookback_tile_words = sort_tiles * RADIX_BINS; // the group words of the radix pass follow the tile words
     w.lookback_words = w.lookback_tile_words + (sort_tiles / LB_GROUP + 1) * RADIX_BINS;
     if (rank_tiles * 4 > w.lookback_words)

@@ -125,7 +125,7 @@ int finish_partition_step(Launch& L, const char* who, StepColumns& c, const Tail
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
-    const RankTables r = rank_tables(h, (u32)m, STEP_TILE);
+    const RankTables r = rank_tables<STEP_TILE>(h, (u32)m);
     unsigned long long* d_active = reinterpret_cast<unsigned long long*>(h->counts + 8);
     StepRankArgs ra;
     ra.key0 = sorted_key0;
@@ -275,7 +275,7 @@ int step_init(Launch& L, const char* who, StepColumns& c, const StepPlan& pl, in
             return rc;
         kc = in_out;
         pc ^= in_out;
-        const RankTables r = rank_tables(h, (u32)m, STEP_TILE);
+        const RankTables r = rank_tables<STEP_TILE>(h, (u32)m);
         u32* tied_pos = pl.at<u32>(24);
         TieArgs ta;
         ta.keys = K[kc];

@@ -727,3 +727,14 @@ def test_first_sort_of_byte_wide_symbols_takes_half_the_passes(emu, symbols):
     got, active, _ = emu_sort(emu, T, 4)
     sa, counts = oracle_lib.prefix_doubling(T, 4)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
+def test_tables_of_the_rank_step_hold_the_smallest_tiles():
+    """A build with larger rank tiles (CSA_RANK_BLOCK, for tuning runs): the kernel that collects long mixed runs cuts the list into
+    smaller tiles than the rank step and shares its tables."""
+    lib = load_emulation("libcascade_emu_rank.so")
+    T = texts.text_with_shared_codes(130000, [2, 5, 63, 64, 65, 70, 90], 3)
+    got, active, _ = emu_sort(lib, T, 1)
+    assert emu_sort.passes[0] > 8  # the long runs were collected
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
