@@ -786,6 +786,15 @@ int windowed_rank_update(Launch& L, const u32* pos, const DeferBuffers& buf, u32
     return CSA_OK;
 }
 
+// How far apart in rank[] two writes in a row may lie to count as one (count_ranks_kernel). Half a text of one period, ms per sort
+// written in place and bucketed: 2^27 symbols, period 8 68 and 76, 10 67 and 81, 15 73 and 84; 2^29 symbols, period 7 280 and 303, 8 311
+// and 310, 12 370 and 340, 15 420 and 358; 2^28 symbols, period 8 153 and 151, 12 175 and 170, 15 190 and 177. Past 2^27
+// symbols rank[] is larger than the last-level cache, and a line leaves it before the next residue of the period comes by.
+#ifndef CSA_FAR_REACH_MAX
+#define CSA_FAR_REACH_MAX (1u << 27)
+#endif
+u32 run_reach(u32 n) { return n <= CSA_FAR_REACH_MAX ? 15u : 8u; }
+
 // The smallest tile of the kernels that share the rank step's tables: the tables are sized for it.
 constexpr int smaller(int a, int b) { return a < b ? a : b; }
 constexpr int TABLE_TILE = smaller(smaller(RANK_TILE, SMALL_TILE), smaller(COLLECT_TILE, STEP_TILE));
@@ -1575,7 +1584,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             }
             // 3. per-tile counts of the sorted list (8 bytes read per member)
             hipLaunchKernelGGL((count_ranks_kernel<SMALL_BLOCK, SMALL_ITEMS>), dim3(r.tiles), dim3(SMALL_BLOCK), 0, s, nr_list, x_out, m_in,
-                               r.tile_agg, r.tile_splits);
+                               run_reach(n), r.tile_agg, r.tile_splits);
             HIP_TRY(hipGetLastError());
         }
         st->big[gen] = big;

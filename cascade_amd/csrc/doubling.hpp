@@ -786,14 +786,14 @@ __global__ __launch_bounds__(BLOCK) void smallsort_kernel(SmallSortArgs a)
 
 // Counts of the sorted list (suffix, refined rank) per tile, for generations in which large groups came back through
 // the radix sort: survivors (members whose rank is shared), new groups, changed ranks. Reads 8 bytes per member.
-// A changed rank counts only if its suffix is not next to the one before it in the list (in the same 64 bytes of rank[]): the
-// count decides whether the rank writes are bucketed first, and the members of a run or a period, whose suffixes follow one
-// another in the list, write whole lines of rank[] as they stand. 2^26 symbols of runs, periods and tokens, 20
-// generations of 10 M such members: 15.9 ms with the bucketed update (histogram, pass, scatter: 0.24 ms each), 12.8 without.
+// A changed rank counts only if the rank written just before it, that of the member before it in the list, lies more than `reach`
+// places away in rank[]: the count decides whether the rank writes are bucketed first, and the members of a run or a period follow one
+// another in the list at the distance of the period, so that a line of rank[] they stand on is written several times in a row
+// (reach: run_reach). The kernel of the small groups (smallsort_kernel) counts every changed rank: what stands next to each other there
+// are the members of one group, which come from all over the text.
 template <int BLOCK, int ITEMS>
-__global__ __launch_bounds__(BLOCK) void count_ranks_kernel(const u32* __restrict__ nr, const u32* __restrict__ sufs, u32 m,
-                                                            u32* __restrict__ tile_agg,
-                                                            u32* __restrict__ tile_splits)
+__global__ __launch_bounds__(BLOCK) void count_ranks_kernel(const u32* __restrict__ nr, const u32* __restrict__ sufs, u32 m, u32 reach,
+                                                            u32* __restrict__ tile_agg, u32* __restrict__ tile_splits)
 {
     constexpr int TILE = BLOCK * ITEMS;
     constexpr int WAVES = BLOCK / WAVE;
@@ -842,8 +842,8 @@ __global__ __launch_bounds__(BLOCK) void count_ranks_kernel(const u32* __restric
             const bool surv = !(head && last);
             c_surv += surv ? 1u : 0u;
             c_head += (head && surv) ? 1u : 0u;
-            const bool next_to = c > 0 && x[k + 1] - x[k] + 15u <= 30u; // at most 15 places apart, either way
-            c_chg += next_to ? 0u : word >> 31;
+            const bool follows = (nrw[k] >> 31) && x[k + 1] - x[k] + reach <= 2u * reach; // either way (the place before the list: unchanged)
+            c_chg += follows ? 0u : word >> 31;
         }
     }
     static_assert(64 * ITEMS < 1024, "three counts are packed into one 32-bit word");

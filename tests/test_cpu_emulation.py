@@ -673,19 +673,31 @@ def test_first_sort_on_codes_at_small_and_ragged_sizes(emu, n):
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
 
 
-@pytest.mark.parametrize("period", [1, 7, 15, 16, 40])
-def test_ranks_of_neighbouring_suffixes_are_written_in_place(emu, period):
+@pytest.mark.parametrize("n,period,in_place", [(6000, 1, True), (6000, 7, True), (6000, 15, True), (6000, 16, False), (6000, 40, False),
+                                               (9000, 1, True), (9000, 8, True), (9000, 9, False), (9000, 15, False)])
+def test_ranks_of_neighbouring_suffixes_are_written_in_place(emu, n, period, in_place):
     """A periodic stretch among random tokens: the members of its groups stand in the list in the order of the text, `period`
-    symbols apart. Up to 15 apart (one line of rank[]) their rank writes are not bucketed, past that they are; suffix array
-    and generation sizes are the oracle's either way."""
+    symbols apart. Up to 15 apart (8 in partitions past 7000 symbols in this build) their rank writes are not bucketed, past that they
+    are; suffix array and generation sizes are the oracle's either way."""
     rng = np.random.default_rng(period)
-    T = rng.integers(300, 60000, 6000).astype(np.uint16)
+    T = rng.integers(300, 60000, n).astype(np.uint16)
     T[1000:4600] = np.tile(rng.integers(300, 60000, period).astype(np.uint16), 3600 // period + 1)[:3600]
+    T[4600] = 7  # what runs off the stretch comes first, and the ranks of all that is left change in every generation
     got, active, big = emu_sort(emu, T, 1, pack=False)
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
     late = [u for u, b, d in zip(emu_sort.rank_update, big, emu_sort.dense) if b and not d][1:-1]
-    assert late and (all(u == 0 for u in late) if period <= 15 else any(u == 2 for u in late))
+    assert late and (all(u == 0 for u in late) if in_place else any(u == 2 for u in late))
+
+
+def test_a_changed_rank_beside_an_unchanged_one_counts_as_a_write_of_its_own(emu):
+    """Runs of five equal symbols, another symbol each: generation 1 splits groups of two neighbours, and one rank of every two
+    changes. No two writes fall on neighbouring places, so they are bucketed."""
+    T = np.append(np.repeat(np.random.default_rng(5).permutation(np.arange(300, 1500)), 5), [7] * 4).astype(np.uint16)
+    got, active, _ = emu_sort(emu, T, 1, pack=False)
+    assert active[1] == 2400 and emu_sort.rank_update[1] == 2
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
 
 
 @pytest.mark.parametrize("row", [512, 500])
