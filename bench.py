@@ -670,6 +670,9 @@ def main():
         # peak says by how much that list is undercut, not how busy HBM was (that is job_frac_moved)
         result["job_alg_note"] = (f"the first sort (keys of {st['key_symbols']} packed symbols) stands for generations 0-"
                                   f"{st['first_sort_generations'] - 1} of the reference's list, whose bytes the yardstick still counts")
+    elif coded_pairs:
+        result["job_alg_note"] = ("the yardstick counts generation 0 as eight passes over (64-bit key, index) pairs; the sort makes four over "
+                                  "(32-bit code, index) pairs")
     if moved_gen_dropped:
         result["generation_traffic_dropped"] = moved_gen_dropped
     if args.cpu_sample > 0:

@@ -1209,7 +1209,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     HIP_TRY(hipMemsetAsync(h->counts, 0, 5 * sizeof(u32), s));
     HIP_TRY(hipEventRecord(h->ev_gen[0], s));
 
-    // ---- generation 0: sort every suffix by its K-gram key, ties of tail suffixes broken by length ----
+    // ---- generation 0: every suffix sorted by its first symbols (four of them, by codes or K-gram keys, or as many as a packed
+    // key holds), ties of tail suffixes broken by length ----
     RangeScope range_gen0("generation 0 m=%u", n);
     // The byte histograms of the text come first: they tell whether the alphabet is small enough for keys of more than four
     // symbols. (The digit counts are zeroed with them.)

@@ -8,12 +8,12 @@
 namespace csa {
 
 // ---------------------------------------------------------------------------------------------
-// Generation 0: rank assignment + compaction of the sorted K-gram keys in three launches: per-tile aggregates, a scan
+// Generation 0: rank assignment + compaction of the sorted list in three launches: per-tile aggregates, a scan
 // of the aggregates over the tiles, and the pass that applies them. (A single launch with a decoupled look-back
 // was measured at 2.5 to 4 times the duration of these three on this part: with 8 XCDs the look-back words travel
 // over the fabric, and the few resident workgroups per CU spent most of their life waiting for their predecessors.)
 //
-// Input: all suffixes sorted by key, keys[c] / sufs[c] for c in [0, n). The rank of a suffix is the index of the
+// Input: all suffixes sorted by key, keys[c] / sufs[c] for c in [0, n), or a list that carries its ties (TIED_LEFT). The rank of a suffix is the index of the
 // head of its run of equal keys (reference: include/GPU_SACA.cuh:191-208; the max-scan of src/GPU_SACA.cu:1241-1247
 // is the max chain here). A suffix whose run has length 1 retires: its rank is final, and the sorted index array
 // already holds it at its place of the suffix array. The others are compacted, in order, into the first active list

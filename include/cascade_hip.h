@@ -50,7 +50,8 @@ typedef struct csa_stats {
     uint64_t active[CSA_MAX_GENERATIONS]; /* suffixes active entering generation g; active[0] = n */
     uint64_t groups[CSA_MAX_GENERATIONS]; /* unresolved groups entering generation g (0 for g = 0) */
     uint64_t big[CSA_MAX_GENERATIONS];    /* of active[g], members of groups too large for the in-tile sort */
-    int32_t passes[CSA_MAX_GENERATIONS];  /* radix passes run in generation g (over the large groups for g > 0) */
+    int32_t passes[CSA_MAX_GENERATIONS];  /* radix passes run in generation g (over the large groups for g > 0; for g = 0 four
+                                             on codes or up to eight on keys, and those over runs that had to be sorted again) */
     int32_t rank_update[CSA_MAX_GENERATIONS]; /* how generation g wrote its ranks: 0 scattered from the rank pass,
                                                  1 bucketed by two passes into LDS-sized windows (generation 0),
                                                  2 bucketed by one pass into cache-sized windows */
@@ -68,8 +69,9 @@ typedef struct csa_stats {
     uint64_t presorted[CSA_MAX_GENERATIONS]; /* of big[g], members that skipped the radix sort: every large group of the
                                                 list was in order of rank[x + h] already (rising or falling along the
                                                 list, as in runs of one token and periodic stretches) */
-    uint32_t key_symbols;            /* symbols the first sort resolved: 4 (one K-gram word), or up to 64 when the text's
-                                        alphabet is small enough for packed codes of 1, 2, 4 or 8 bits */
+    uint32_t key_symbols;            /* symbols the first sort resolved: 4 (by 32-bit codes of them, or by K-gram words where
+                                        too many suffixes would share a code), or up to 64 when the text's alphabet is small
+                                        enough for packed codes of 1, 2, 4 or 8 bits */
     uint32_t first_sort_generations; /* generations of the reference that sort stands for: 1, or 1 + j when its keys held
                                         4 * key_words * 2^j symbols. Generations 1 .. j are then reported with the lists
                                         they would have had (active[], groups[]) and with no time or passes of their own */
@@ -144,7 +146,7 @@ int csa_set_device_exclusive(csa_handle* h, int exclusive);
  *   CSA_TUNE_PACK_SYMBOLS        1 (default): a text whose symbols take at most 256 values (by the values its low and its
  *                                high bytes take) is sorted first on keys of as many packed symbols as 64 bits hold, which
  *                                covers the first generations of the doubling (csa_stats.first_sort_generations); 0: the
- *                                first sort always takes one K-gram word
+ *                                first sort always resolves four symbols
  *   CSA_TUNE_EXPECT_PRESORTED    0 (default): a generation leaves out the (key, suffix) pairs of its large groups' radix sort
  *                                when every large group of the generation before was in order as it stood (csa_stats.presorted),
  *                                and gathers again with them if this one's are not; 1: every generation starts that way
