@@ -179,14 +179,16 @@ constexpr int SMALL_MAXG_HI = CSA_SMALL_MAXG_HI;
 constexpr u32 SMALL_AVG_LIMIT = CSA_SMALL_AVG_LIMIT;
 static_assert(SMALL_MAXG_HI >= SMALL_MAXG, "the higher group limit is the higher one");
 constexpr u32 TICKET_POOL = 4096;
-constexpr u32 PROBE_FEW_CHUNKS = 512;                             // 2^15 suffixes, whose table ...
-constexpr u64 PROBE_TABLE = 2ull * PROBE_FEW_CHUNKS * SAMPLE_CHUNK; // ... is one of the handle's own
+constexpr u32 PROBE_FEW = 1u << 15;           // suffixes that are probed, whose table ...
+constexpr u64 PROBE_TABLE = 2ull * PROBE_FEW; // ... is one of the handle's own
 constexpr u64 CODE_TABLE_WORDS = SYMBOLS + RESOLVE_MARK_WORDS + 8 + 2 * PROBE_TABLE + SYMBOLS + 4; // symbol counts, marks, ProbeCounts, its table, shares (and entry [SYMBOLS])
-// Texts of at least this many symbols are probed before they are sorted by codes (probe_codes_kernel, 15 us with its round trip). Shorter
-// ones have few runs of a code that are too long for a tile: generation 0 of 2^18 symbols of phrases takes 205 us on codes
-// and 185 on K-gram keys, of 2^19 symbols 381 and 207; of independent symbols 153 and 185, 168 and 207.
+// Texts of at least this many symbols are probed before they are sorted by codes (probe_codes_kernel, 12 us with its round trip). Shorter
+// ones have no runs of one code that are too long for a tile, out of order and not planted: strings of four symbols that are
+// rare enough to share a code with others can come up 256 times from there on. Generation 0 of records of four symbols, one of
+// them of many values, in us on K-gram keys, on codes and with the choice: 2^16.9 symbols 173, 189, -; 2^18 185, 419, 211;
+// 2^18.9 202, 423, 232; of independent symbols 172, 142, -; 184, 151, 165; 203, 165, 180.
 #ifndef CSA_PROBE_MIN
-#define CSA_PROBE_MIN (1u << 19)
+#define CSA_PROBE_MIN (1u << 17)
 #endif
 constexpr u32 PROBE_MIN = CSA_PROBE_MIN;
 // Shorter texts are coded while the host waits for the probe, which takes about as long, longer ones when it has advised that: 2^22
@@ -195,7 +197,7 @@ constexpr u32 PROBE_MIN = CSA_PROBE_MIN;
 #define CSA_CODE_AHEAD_MAX (1u << 22)
 #endif
 constexpr u32 CODE_AHEAD_MAX = CSA_CODE_AHEAD_MAX;
-static_assert(PROBE_MIN >= 16 * SAMPLE_CHUNK, "the probe looks at one chunk at least");
+static_assert(PROBE_MIN >= 32, "two suffixes are the fewest that can share a code");
 constexpr u32 PINNED_HIST = 32;        // host mirror: words [0, 16) mirror the device counters, [16, 32) single values, then the histograms
 constexpr u32 MSG_OFF_WORDS = 32769;   // p + 1 outbox counters, p <= 32768
 constexpr int EVENT_POOL = 2 * CSA_MAX_GENERATIONS * MAX_PASSES * 2;
@@ -911,16 +913,15 @@ PackedPlan plan_packed_text(const u32* bytehist, u32 n, int key_words, u64 room_
     return pp;
 }
 
-// Chunks of the text that the probe looks at: one in 16 while they are few, then one in 512, at most 2^20 suffixes.
-u32 probe_chunks(u32 n)
+// Suffixes that the probe looks at: one in 16 while they are few, then one in 512, at most 2^PROBE_MOST_LOG2.
+u32 probed_suffixes(u32 n)
 {
-    const u32 few = n / (16 * SAMPLE_CHUNK) < PROBE_FEW_CHUNKS ? n / (16 * SAMPLE_CHUNK) : PROBE_FEW_CHUNKS;
-    const u32 k = n / (512 * SAMPLE_CHUNK) > few ? n / (512 * SAMPLE_CHUNK) : few;
-    return k < SAMPLE_CHUNKS_MAX ? k : SAMPLE_CHUNKS_MAX;
+    const u32 few = n / 16 < PROBE_FEW ? n / 16 : PROBE_FEW, many = n / 512 > few ? n / 512 : few;
+    return many < 1u << PROBE_MOST_LOG2 ? many : 1u << PROBE_MOST_LOG2;
 }
 
 struct CodeTables {
-    u32 *counts, *marks; // zeroed together, with the counters of the probe and its table of up to PROBE_FEW_CHUNKS chunks
+    u32 *counts, *marks; // zeroed together, with the counters of the probe and its table of up to PROBE_FEW suffixes
     ProbeCounts* probe;
     unsigned long long* table;
     u32* cum;
@@ -938,7 +939,7 @@ CodeTables code_tables(const csa_handle* h)
 }
 
 // What a sort by codes starts from: the shares of the symbols, and for texts of PROBE_MIN symbols or more what a sample of the suffixes
-// (probe_chunks) shows about shared codes, on its way to *seen; ev_gen[1] tells that it is there. A large sample's table is
+// (probed_suffixes) shows about shared codes, on its way to *seen; ev_gen[1] tells that it is there. A large sample's table is
 // key[0], which holds nothing yet.
 int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
 {
@@ -952,14 +953,14 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
     if (n >= PROBE_MIN) {
         a.text = d_text;
         a.n = n;
-        a.chunks = chunks;
-        a.taken = probe_chunks(n);
+        a.taken = probed_suffixes(n);
         a.cum = c.cum;
-        a.table_log2 = (u32)bit_length((u64)a.taken * SAMPLE_CHUNK - 1) + 1;
-        const u32 per_suffix = n / (a.taken * SAMPLE_CHUNK);
-        a.long_from = RESOLVE_MAX / per_suffix > 2 ? RESOLVE_MAX / per_suffix : 2;
+        a.table_log2 = (u32)bit_length((u64)a.taken - 1) + 1;
+        // (an eighth more than a tile sorts: a run of just that many would be taken for a longer one as often as not)
+        const u32 long_run = RESOLVE_MAX * 9 / 8 / (n / a.taken);
+        a.long_from = long_run > 2 ? long_run : 2;
         a.counts = c.probe;
-        const bool few = a.taken <= PROBE_FEW_CHUNKS;
+        const bool few = a.taken <= PROBE_FEW;
         a.table = few ? c.table : reinterpret_cast<unsigned long long*>(h->key[0]);
         zeros += sizeof(ProbeCounts);
         if (few)
@@ -979,7 +980,7 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
     hipLaunchKernelGGL(symbol_shares_kernel, dim3(SYMBOLS / SHARES_TILE), dim3(SHARES_TILE), 0, s, (const u32*)c.counts, weight_log2,
                        (u32)((sampled << weight_log2) + SYMBOLS), c.cum);
     if (n >= PROBE_MIN) {
-        hipLaunchKernelGGL(probe_codes_kernel, dim3((a.taken * SAMPLE_CHUNK + PROBE_BLOCK - 1) / PROBE_BLOCK), dim3(PROBE_BLOCK), 0, s, a);
+        hipLaunchKernelGGL(probe_codes_kernel, dim3((a.taken + PROBE_BLOCK - 1) / PROBE_BLOCK), dim3(PROBE_BLOCK), 0, s, a);
         HIP_TRY(hipMemcpyAsync(seen, a.counts, sizeof(ProbeCounts), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipEventRecord(h->ev_gen[1], s)); // (recorded again when the generation ends)
     }
@@ -997,7 +998,7 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
 // 0.40, 0.72, 0.45; 2^20 of them 0.23, 0.44, 0.28.
 bool codes_pay(const ProbeCounts& c, u32 n)
 {
-    const double seen = (double)probe_chunks(n) * SAMPLE_CHUNK, per_seen = n / seen;
+    const double seen = probed_suffixes(n), per_seen = n / seen;
     const double second = 2.0 * (c.second - c.third) / seen, third = 3.0 * (c.third - c.fourth) / seen; // in codes seen twice, thrice
     const double more = ((double)c.again + c.second) / seen - second;                                    // ... thrice and more often
     // The suffixes whose company the sample missed: a code of m suffixes shows x = m / per_seen of them on average, and e^x / x
@@ -1010,7 +1011,9 @@ bool codes_pay(const ProbeCounts& c, u32 n)
     const double mixed = c.again ? (double)c.other / c.again : 0.0;
     // read from the text, and compared with its run: at most RESOLVE_MAX others
     double cost = company * (20.0 + 0.5 * mixed * (others < RESOLVE_MAX ? others : RESOLVE_MAX));
-    if (c.crowded > 4) // collected and sorted once more
+    // Collected and sorted once more. Where a long run would show two or three suffixes only, short ones do so by chance: then a
+    // few of them count only if runs are long on average.
+    if (c.crowded > (per_seen <= 64 || x * per_seen >= RESOLVE_MAX / 2 ? 2.0 : seen / 1000))
         cost += 60.0 * c.crowded / seen + 2e8 / n;
     return cost < 18.0 + 2.5e7 / n;
 }

@@ -43,7 +43,7 @@ constexpr u32 SAMPLE_CHUNKS_MIN = 256;        // 2^14 symbols are looked at, at 
 constexpr u32 SAMPLE_CHUNKS_MAX = 1u << 14;   // ... and 2^20 at most
 constexpr int SAMPLE_LOG2 = 20;
 
-// Chunk c of a sample of `taken` out of `chunks`: one of the c-th of `taken` equal stretches of the text, at the place in it that the
+// Chunk (or place) c of a sample of `taken` out of `chunks`: one of the c-th of `taken` equal stretches of the text, at the place in it that the
 // multiples of the golden ratio, cut to their fractions, give. At equal distances the chunks would see only a few columns of a text
 // in rows of a fixed length (2^28 symbols in rows of 1024, the first 64 of each over values of their own: at a stride of
 // 16384 symbols only those columns were sampled, most suffixes shared their code with thousands of others, and generation 0
@@ -143,6 +143,7 @@ __device__ __forceinline__ bool string_code(const u32 (&lo)[4], const u32 (&widt
 
 constexpr int PROBE_BLOCK = 256;
 constexpr u32 PROBE_START = 0x55555555u; // (the sample of the symbols is taken elsewhere: what its own places show is too good)
+constexpr u32 PROBE_MOST_LOG2 = 20;      // suffixes that are looked at
 
 // What a sample of suffixes shows about codes that are not one string's alone: how often a suffix finds its code taken by one, two,
 // three others and so on, by another string, by so many that a run of it is longer than RESOLVE_MAX in the whole text.
@@ -158,7 +159,7 @@ static_assert(sizeof(ProbeCounts) == 8 * sizeof(u32), "the counters take eight w
 struct ProbeArgs {
     const u16* text;
     u32 n;
-    u32 chunks, taken; // of SAMPLE_CHUNK suffixes (sampled_chunk)
+    u32 taken; // suffixes, one out of each of as many stretches (sampled_chunk; not in runs, which would meet their copies in runs)
     const u32* cum;
     unsigned long long* table; // [1 << table_log2], zeroed, at least twice as many as suffixes are looked at
     u32 table_log2;
@@ -177,39 +178,36 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
         s_cnt[t] = 0;
     __syncthreads();
     u32 pairs = 0, flags = 0;
-    const u64 i = (u64)blockIdx.x * PROBE_BLOCK + t;
-    const u32 c = (u32)(i / SAMPLE_CHUNK);
-    if (c < a.taken) {
-        const u64 x = (u64)sampled_chunk(c, a.chunks, a.taken, PROBE_START) * SAMPLE_CHUNK + (i & (SAMPLE_CHUNK - 1));
-        if (x < a.n) {
-            u32 lo[4], width[4], hash = 0, code;
+    const u32 i = blockIdx.x * PROBE_BLOCK + t;
+    if (i < a.taken) {
+        const u64 x = sampled_chunk(i, a.n, a.taken, PROBE_START);
+        u32 lo[4], width[4], hash = 0, code;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const u32 s = x + k < a.n ? a.text[x + k] : 0u;
-                u32 pair[2];
-                __builtin_memcpy(pair, a.cum + s, 8); // entries s and s + 1 (4-byte aligned)
-                lo[k] = pair[0];
-                width[k] = pair[1] - pair[0];
-                hash = (hash + s + 1u) * 0x9E3779B1u;
-            }
-            if (!string_code(lo, width, code)) {
-                const unsigned long long entry = ((unsigned long long)code << 32) | (hash >> 24 << 24) | 1u;
-                const u32 mask = (1u << a.table_log2) - 1u;
-                u32 slot = (code * 0x9E3779B1u) >> (32 - a.table_log2);
-                for (u32 tries = 0; tries <= mask; ++tries, slot = (slot + 1u) & mask) { // (half of the table stays empty)
-                    unsigned long long seen = atomicCAS(&a.table[slot], 0ull, entry);
-                    if (seen == 0)
-                        break;
-                    if ((u32)(seen >> 32) != code)
-                        continue;
-                    seen = atomicAdd(&a.table[slot], 1ull);
-                    const u32 before = (u32)seen & 0xFFFFFFu;
-                    const bool other = (((u32)seen ^ (u32)entry) >> 24) != 0;
-                    pairs = before;
-                    flags = 1u | (before == 1u ? 2u : 0u) | (before == 2u ? 4u : 0u) | (before == 3u ? 8u : 0u) | (other ? 16u : 0u) |
-                            (other && before >= a.long_from ? 32u : 0u);
+        for (int k = 0; k < 4; ++k) {
+            const u32 s = x + k < a.n ? a.text[x + k] : 0u;
+            u32 pair[2];
+            __builtin_memcpy(pair, a.cum + s, 8); // entries s and s + 1 (4-byte aligned)
+            lo[k] = pair[0];
+            width[k] = pair[1] - pair[0];
+            hash = (hash + s + 1u) * 0x9E3779B1u;
+        }
+        if (!string_code(lo, width, code)) {
+            const unsigned long long entry = ((unsigned long long)code << 32) | (hash >> 24 << 24) | 1u;
+            const u32 mask = (1u << a.table_log2) - 1u;
+            u32 slot = (code * 0x9E3779B1u) >> (32 - a.table_log2);
+            for (u32 tries = 0; tries <= mask; ++tries, slot = (slot + 1u) & mask) { // (half of the table stays empty)
+                unsigned long long seen = atomicCAS(&a.table[slot], 0ull, entry);
+                if (seen == 0)
                     break;
-                }
+                if ((u32)(seen >> 32) != code)
+                    continue;
+                seen = atomicAdd(&a.table[slot], 1ull);
+                const u32 before = (u32)seen & 0xFFFFFFu;
+                const bool other = (((u32)seen ^ (u32)entry) >> 24) != 0;
+                pairs = before;
+                flags = 1u | (before == 1u ? 2u : 0u) | (before == 2u ? 4u : 0u) | (before == 3u ? 8u : 0u) | (other ? 16u : 0u) |
+                        (other && before >= a.long_from ? 32u : 0u);
+                break;
             }
         }
     }

@@ -663,8 +663,9 @@ def test_command_line_builder_writes_the_oracles_suffix_array(tmp_path):
 @pytest.mark.parametrize("repeats", [[2, 3, 255, 256], [257, 258, 300, 700, 700]])
 def test_first_sort_on_codes_with_runs_that_share_a_code(torch_mod, repeats):
     """The first sort of a token text goes by 32-bit codes of four symbols; runs of suffixes that share a code are put in order
-    inside a tile up to 256 members and radix sorted past that. Planted runs on both sides of the limit, of one string and of
-    two strings out of order, against the oracle: suffix array and generation sizes."""
+    inside a tile up to 256 members and radix sorted past that (or the whole text is, by K-grams, where the probe sees the long
+    ones). Planted runs on both sides of the limit, of one string and of two strings out of order, against the oracle:
+    suffix array and generation sizes."""
     from cascade_amd import PartitionSorter
     T = texts.text_with_shared_codes(1 << 20, repeats, len(repeats))
     with PartitionSorter(T.size, key_words=1) as s:
@@ -674,6 +675,20 @@ def test_first_sort_on_codes_with_runs_that_share_a_code(torch_mod, repeats):
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
     assert (stats["passes"][0] > 4) == (max(repeats) > 256)
+
+
+def test_first_sort_on_codes_collects_long_runs_that_are_out_of_order(torch_mod):
+    """In a text of 2^24 symbols a few long runs of one code are no reason to leave the codes: their members are collected, radix
+    sorted and put back."""
+    from cascade_amd import PartitionSorter
+    T = texts.text_with_shared_codes(1 << 24, [257, 258, 300, 700, 700], 5)
+    with PartitionSorter(T.size, key_words=1) as s:
+        print("  collected runs", flush=True)
+        got = gpu_sa40(torch_mod, s, T)
+        stats = s.last_stats
+    assert stats["passes"][0] > 8  # four passes over all suffixes, and those over the collected ones
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
 
 
 @pytest.mark.parametrize("letters", [40000, 4])
@@ -694,12 +709,18 @@ def test_kernel_timing_counts_every_radix_pass(torch_mod, letters):
     assert stats["radix_pairs"] >= T.size * stats["passes"][0] and stats["radix_ms"] > 0
 
 
-@pytest.mark.parametrize("n,phrases,passes", [(1 << 20, 5000, 8), ((1 << 22) + 5, 5000, 8), (1 << 19, 0, 4)])
+@pytest.mark.parametrize("n,phrases,passes", [(1 << 20, 5000, 8), ((1 << 22) + 5, 5000, 8), (1 << 17, 0, 4), (1 << 18, -256, 8)])
 def test_first_sort_chooses_between_codes_and_kgrams(torch_mod, n, phrases, passes):
-    """Texts of 2^19 symbols or more are probed for codes that many suffixes share. A text of phrases goes by K-gram keys (2^20: coded
-    before the host knows; past 2^22: not coded at all), one of independent symbols by codes; all against the oracle."""
+    """Texts of 2^17 symbols or more are probed for codes that many suffixes share. Texts of phrases and of records (phrases < 0: that
+    many kinds) go by K-gram keys (2^18 and 2^20: coded before the host knows; past 2^22: not coded at all), one of
+    independent symbols by codes; all against the oracle."""
     from cascade_amd import PartitionSorter
-    T = texts.text_of_phrases(n, phrases, 10, 60, 1) if phrases else np.random.default_rng(n).integers(1, 50000, n).astype(np.uint16)
+    if phrases > 0:
+        T = texts.text_of_phrases(n, phrases, 10, 60, 1)
+    elif phrases < 0:
+        T = texts.text_of_shared_records(n, -phrases, 1)
+    else:
+        T = np.random.default_rng(n).integers(1, 50000, n).astype(np.uint16)
     with PartitionSorter(T.size, key_words=1) as s:
         print(f"  {n} symbols of {phrases} phrases", flush=True)
         got = gpu_sa40(torch_mod, s, T)

@@ -98,3 +98,12 @@ def text_of_phrases(n, phrases, lo, hi, seed):
     draws = rng.choice(phrases, n // lo + 1, p=share / share.sum())
     at = np.repeat(start[draws] - (np.cumsum(ln[draws]) - ln[draws]), ln[draws]) + np.arange(int(ln[draws].sum()))
     return ids[at[:n]]
+
+
+def text_of_shared_records(n, records, seed):
+    """Records of four symbols: three that belong to the record's kind (`records` kinds) and one of 5000 values. All suffixes
+    that start a record of one kind share an arithmetic code of 32 bits once (4 * records)^3 is near 2^32 / 4."""
+    rng = np.random.default_rng(seed)
+    kind = rng.integers(0, records, n // 4 + 1)
+    T = np.stack([kind + 300, kind + 3000, kind + 6000, rng.integers(30000, 35000, kind.size)], axis=1)
+    return T.reshape(-1)[:n].astype(np.uint16)
