@@ -355,10 +355,15 @@ struct ResolveArgs {
 __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs a)
 {
     constexpr int H = RESOLVE_MAX, SPAN = RESOLVE_TILE + 2 * H;
+    constexpr int FEW = 16; // runs of up to this many members are sorted without a look whether they are in order
     __shared__ u64 s_head[SPAN / 64]; // bit j: the element at span place j starts a run (places outside the list count as starts)
+    __shared__ u64 s_down[SPAN / 64]; // bit j: its string is smaller than that of the element before it in its run
+    __shared__ u32 s_many;            // some run of the tile has more members
     __shared__ u64 s_key[SPAN];
     __shared__ u32 s_suf[SPAN];
     const u32 t = threadIdx.x;
+    if (t == 0)
+        s_many = 0;
     const long long t0 = (long long)blockIdx.x * RESOLVE_TILE, lo = t0 - H, n = a.n;
     // whole waves take consecutive places: one ballot per wave and round gives 64 bits of s_head
     for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (the same rounds for every lane of a wave: SPAN is a multiple of 64)
@@ -410,8 +415,11 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         const int j = H + k * RESOLVE_BLOCK + (int)t;
         if (last[k] - first[k] != 1) {
             s_suf[j] = x[k];
-            if (!((owners >> k) & 1u))
+            if (!((owners >> k) & 1u)) {
                 s_key[j] = load_kgram(a.text, a.n, x[k], 0);
+                if (last[k] - first[k] > FEW)
+                    s_many = 1;
+            }
         }
     }
     // of the halo: the members of short runs that reach into the tile, and the left neighbour of the tile's first element
@@ -432,6 +440,31 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         }
     }
     __syncthreads();
+    // A run that is one string repeated, or several in order, stays as it is: its members need not be compared with each other. (In a
+    // short text the kernel takes as long as the longest run of a tile: generation 0 of 2^18 symbols of phrases 221 us with
+    // all comparisons, 191 without these; texts without such runs are as fast as before.)
+    const bool many = s_many != 0;
+    if (many) {
+        for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (places whose strings were not wanted hold anything: no run looked at below has any)
+            const bool down = j > 0 && !((s_head[j / 64] >> (j & 63)) & 1ull) && s_key[j] < s_key[j - 1];
+            const u64 b = __ballot(down);
+            if ((t & 63u) == 0)
+                s_down[j / 64] = b;
+        }
+        __syncthreads();
+    }
+    auto in_order = [&](int from, int to) -> bool { // places from + 1 .. to - 1: at most RESOLVE_MAX of them
+        u64 seen = 0;
+        for (int wd = from / 64; wd <= (to - 1) / 64; ++wd) {
+            u64 b = s_down[wd];
+            if (wd == from / 64)
+                b &= (from & 63) == 63 ? 0ull : ~0ull << ((from & 63) + 1);
+            if (wd == (to - 1) / 64)
+                b &= ~0ull >> (63 - ((to - 1) & 63));
+            seen |= b;
+        }
+        return seen == 0;
+    };
 #pragma unroll
     for (int k = 0; k < RESOLVE_ITEMS; ++k) {
         const int j = H + k * RESOLVE_BLOCK + (int)t;
@@ -455,6 +488,9 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
                     *a.unordered = 1u;
                 }
             }
+        } else if (last[k] - first[k] > FEW && in_order(first[k], last[k])) {
+            if (j != first[k])
+                tied = s_key[j] == s_key[j - 1] && whole && (u64)s_suf[j - 1] + a.ell < a.n;
         } else if (last[k] - first[k] > 1) {
             const u64 mine = s_key[j];
             place = first[k];

@@ -752,3 +752,19 @@ def test_tables_of_the_rank_step_hold_the_smallest_tiles(records):
     assert emu_sort.passes[0] > 8  # the long runs were collected
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
+@pytest.mark.parametrize("zeros,tail", [(15, 2), (16, 3), (30, 1), (30, 7), (62, 5)])
+def test_runs_of_one_code_that_are_in_order_and_end_with_the_text(emu, zeros, tail):
+    """Strings of four zeros, rare enough to share a code with nobody's flag: their run is one string repeated and stays as it is, the
+    suffixes that run off the text (whose padding is the same string) first and tied with none. Below and above the number
+    of members that are compared with each other."""
+    rng = np.random.default_rng(zeros)
+    T = rng.integers(1, 40000, 60000).astype(np.uint16)
+    for at in rng.permutation(59000 // 6)[:zeros]:
+        T[6 * at:6 * at + 4] = 0
+    T[-tail:] = 0
+    got, active, _ = emu_sort(emu, T, 1)
+    assert emu_sort.passes[0] == 4
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
