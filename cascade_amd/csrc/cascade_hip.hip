@@ -974,8 +974,9 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
     taken = taken < SAMPLE_CHUNKS_MAX ? taken : SAMPLE_CHUNKS_MAX;
     taken = taken < chunks ? taken : chunks;
     const u64 sampled = (u64)taken * SAMPLE_CHUNK < n ? (u64)taken * SAMPLE_CHUNK : (u64)n;
-    hipLaunchKernelGGL(sample_symbols_kernel, dim3((taken + SAMPLE_CHUNKS_PER_BLOCK - 1) / SAMPLE_CHUNKS_PER_BLOCK), dim3(SAMPLE_BLOCK), 0, s,
-                       d_text, n, chunks, taken, c.counts);
+    const u32 per_block = sample_chunks_per_block(taken);
+    hipLaunchKernelGGL(sample_symbols_kernel, dim3((taken + per_block - 1) / per_block), dim3(SAMPLE_BLOCK), 0, s, d_text, n, chunks, taken,
+                       c.counts);
     const int weight_log2 = SAMPLE_LOG2 - bit_length(sampled - 1);
     hipLaunchKernelGGL(symbol_shares_kernel, dim3(SYMBOLS / SHARES_TILE), dim3(SHARES_TILE), 0, s, (const u32*)c.counts, weight_log2,
                        (u32)((sampled << weight_log2) + SYMBOLS), c.cum);

@@ -38,9 +38,9 @@ namespace csa {
 constexpr int SYMBOLS = 1 << 16;
 constexpr int SAMPLE_BLOCK = 1024;
 constexpr u32 SAMPLE_CHUNK = 64;              // consecutive symbols, one wave's worth
-constexpr u32 SAMPLE_CHUNKS_PER_BLOCK = 64;   // 4096 symbols: a 16-bit counter holds them all (16384: 9 us more at 2^20 symbols)
 constexpr u32 SAMPLE_CHUNKS_MIN = 256;        // 2^14 symbols are looked at, at least ...
 constexpr u32 SAMPLE_CHUNKS_MAX = 1u << 14;   // ... and 2^20 at most
+constexpr u32 SAMPLE_CHUNKS_WIDE = 1u << 13;  // (samples of this many chunks or more take workgroups of twice as many)
 constexpr int SAMPLE_LOG2 = 20;
 
 // Chunk (or place) c of a sample of `taken` out of `chunks`: one of the c-th of `taken` equal stretches of the text, at the place in it that the
@@ -55,6 +55,11 @@ __device__ __forceinline__ u32 sampled_chunk(u32 c, u32 chunks, u32 taken, u32 s
     return lo + (u32)(((u64)(c * 0x9E3779B1u + start) * (hi - lo)) >> 32);
 }
 
+// Chunks of a workgroup (a 16-bit counter holds all their symbols). What bounds the kernel is clearing the counters and adding them to the
+// table: more workgroups work at it side by side, and add the same symbol more often. us for 64, 128 and 256 chunks: 2^20 Zipf tokens
+// 11, 14, 18, 2^23 17, 17, 20, 2^25 24, 23, 32; independent ids 2^20 12, 15, 18, 2^23 36, 31, 29, 2^25 54, 44, 40.
+__host__ __device__ __forceinline__ u32 sample_chunks_per_block(u32 taken) { return taken < SAMPLE_CHUNKS_WIDE ? 64u : 128u; }
+
 // counts[s] += occurrences of symbol s in the sample: `taken` chunks (all of them when the text is short).
 __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16* __restrict__ text, u32 n, u32 chunks, u32 taken,
                                                                       u32* __restrict__ counts)
@@ -64,9 +69,9 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16*
     for (u32 i = t; i < (u32)SYMBOLS / 2; i += SAMPLE_BLOCK)
         s_cnt[i] = 0;
     __syncthreads();
-    const u32 first = blockIdx.x * SAMPLE_CHUNKS_PER_BLOCK;
+    const u32 per_block = sample_chunks_per_block(taken), first = blockIdx.x * per_block;
 #pragma unroll 4
-    for (u32 r = t / SAMPLE_CHUNK; r < SAMPLE_CHUNKS_PER_BLOCK; r += SAMPLE_BLOCK / SAMPLE_CHUNK) {
+    for (u32 r = t / SAMPLE_CHUNK; r < per_block; r += SAMPLE_BLOCK / SAMPLE_CHUNK) {
         const u32 c = first + r;
         if (c < taken) {
             const u64 p = (u64)sampled_chunk(c, chunks, taken, 0) * SAMPLE_CHUNK + (t & (SAMPLE_CHUNK - 1));
