@@ -447,7 +447,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     __syncthreads();
     // A run that is one string repeated, or several in order, stays as it is: its members need not be compared with each other. (In a
     // short text the kernel takes as long as the longest run of a tile: generation 0 of 2^18 symbols of phrases 221 us with
-    // all comparisons, 191 without these; texts without such runs are as fast as before.)
+    // all comparisons, 191 without these; the kernel takes 8.55 instead of 8.45 ms on 1e9 tokens for it.)
     const bool many = s_many != 0;
     if (many) {
         for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (places whose strings were not wanted hold anything: no run looked at below has any)
