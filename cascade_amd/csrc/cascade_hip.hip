@@ -1013,8 +1013,9 @@ bool codes_pay(const ProbeCounts& c, u32 n)
     // read from the text, and compared with its run: at most RESOLVE_MAX others
     double cost = company * (20.0 + 0.5 * mixed * (others < RESOLVE_MAX ? others : RESOLVE_MAX));
     // Collected and sorted once more. Where a long run would show two or three suffixes only, short ones do so by chance: then a
-    // few of them count only if runs are long on average.
-    if (c.crowded > (per_seen <= 64 || x * per_seen >= RESOLVE_MAX / 2 ? 2.0 : seen / 1000))
+    // few of them count only if runs are long on average. (Three of them are a run of RESOLVE_MAX that shows 12 of its members at one in 32,
+    // the last three of which differ from the first to arrive or do not: such a text would go one way or the other from call to call.)
+    if (c.crowded > (per_seen <= 64 || x * per_seen >= RESOLVE_MAX / 2 ? 3.0 : seen / 1000))
         cost += 60.0 * c.crowded / seen + 2e8 / n;
     return cost < 18.0 + 2.5e7 / n;
 }
