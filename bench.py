@@ -594,7 +594,7 @@ def main():
     # generations; a share of the peak above 1 is no measurement either. In both cases the per-generation figures of
     # the profile are dropped (not printed), and the line says why.
     moved_gen_dropped = None
-    ran = [g for g in range(st["generations"]) if not 1 <= g < st["first_sort_generations"]]  # (the others have no launches)
+    ran = [g for g in range(st["generations"]) if st["ms"][g] > 0]  # (the others have no launches of their own)
     if moved_gen and sorted(moved_gen) != ran:
         moved_gen_dropped = f"the profile holds generations {sorted(moved_gen)}, the run had {ran}"
     elif any(st["ms"][g] > 0 and moved_gen[g] / (st["ms"][g] * 1e-3) / 1e9 > HBM_PEAK_GBS for g in moved_gen):
@@ -612,8 +612,8 @@ def main():
         row = {"g": g, "active": st["active"][g], "groups": st["groups"][g], "big": st["big"][g], "presorted": st["presorted"][g], "passes": st["passes"][g],
                "rank_update": st["rank_update"][g], "small_only": st["small_only"][g], "dense": st["dense"][g], "ms": round(st["ms"][g], 3),
                "alg_GBps": round(gbs, 1), "alg_over_peak": round(gbs / HBM_PEAK_GBS, 4)}
-        if 1 <= g < st["first_sort_generations"]:
-            row["covered_by_first_sort"] = True  # its list is counted on the sorted keys; no time or passes of its own
+        if st["ms"][g] == 0:
+            row["covered_by_first_sort"] = True  # its list is counted on the sorted keys or their text; no time of its own
         if g in moved_gen and st["ms"][g] > 0:
             mv = moved_gen[g] / (st["ms"][g] * 1e-3) / 1e9
             row["moved_GBps"] = round(mv, 1)

@@ -1023,6 +1023,8 @@ bool codes_pay(const ProbeCounts& c, u32 n)
 // Where the codes live until the first pass has read them: by virtual position, with the flags by text position behind them.
 u32* codes_of(const csa_handle* h) { return reinterpret_cast<u32*>(h->key[1]); }
 u8* own_of(const csa_handle* h) { return reinterpret_cast<u8*>(h->key[1]) + 4 * h->cap; }
+// The ties of the sorted list live behind them, until it is ranked (cap is a multiple of 256).
+u8* ties_of(const csa_handle* h) { return own_of(h) + (h->cap / 8 + 255) / 256 * 256; }
 
 int code_suffixes(Launch& L, const u16* d_text, u32 n, u32 tail)
 {
@@ -1039,10 +1041,18 @@ int code_suffixes(Launch& L, const u16* d_text, u32 n, u32 tail)
     return CSA_OK;
 }
 
-// Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their four symbols, with the ties marked,
-// in ra.sufs' array; code_suffixes ran before. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into
-// idx[1]; the codes live in the halves of key[0]. `marked` is left ready for sort_marked_runs.
-int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, ResolveArgs& marked)
+// A list sorted by codes on its way to being ranked.
+struct CodedList {
+    ResolveArgs args;
+    u32 words;        // words of four symbols that its order and its ties stand for, at most 2
+    u64 long_members; // suffixes in runs that were too long for their tile, sorted by their second word in ...
+    int long_passes;  // ... so many radix passes
+};
+
+// Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their first `words` words of four symbols, with
+// their ties beside them; code_suffixes ran before. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into
+// idx[1]; the codes live in the halves of key[0]. What long runs leave open is finished by sort_marked_runs and sort_long_runs.
+int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, CodedList& list)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -1078,57 +1088,123 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 ell, Resolv
         if (rc)
             return rc;
     }
-    memset(&marked, 0, sizeof(marked));
-    marked.codes = sorted[0];
-    marked.sufs = h->idx[0];
-    marked.text = d_text;
-    marked.n = n;
-    marked.ell = ell;
-    marked.sufs_out = h->idx[1];
-    marked.marks = code_tables(h).marks;
-    marked.unordered = h->counts + 4;
-    hipLaunchKernelGGL(resolve_runs_kernel, dim3((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, marked);
+    memset(&list, 0, sizeof(list));
+    list.words = words;
+    ResolveArgs& r = list.args;
+    r.codes = sorted[0];
+    r.sufs = h->idx[0];
+    r.m = n;
+    r.text = d_text;
+    r.n = n;
+    r.words = words;
+    r.sufs_out = h->idx[1];
+    r.ties = ties_of(h);
+    r.marks = code_tables(h).marks;
+    r.unordered = h->counts + 4;
+    r.any_long = h->counts + 5;
+    r.text_codes = codes_of(h);
+    r.tail = tail;
+    hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false>), dim3((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, r);
     HIP_TRY(hipGetLastError());
     return CSA_OK;
 }
 
-// The runs whose codes are marked (long and out of order): their members are collected in list order, radix sorted by their four
-// symbols and put back. Works in key[1], key[2] and idx[2..4], which hold nothing before the list is ranked.
-int sort_marked_runs(Launch& L, ResolveArgs a, int* passes)
+// Counts the members of long runs (of those that are marked: MARKED) per tile, scans the counts and reads the totals back.
+template <bool MARKED>
+int count_long_runs(Launch& L, ResolveArgs& a, u64* members, u64* strings)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
-    const RankTables r = rank_tables<COLLECT_TILE>(h, a.n);
-    a.keys = h->key[1];
-    a.members = h->idx[3];
-    a.places = h->idx[2];
+    const RankTables r = rank_tables<COLLECT_TILE>(h, a.m);
     a.tile_agg = r.tile_agg;
     a.tile_splits = r.tile_splits;
     a.tile_prefix = r.tile_prefix;
     a.slab_total = r.slab_total;
     a.slab = r.slab;
-    hipLaunchKernelGGL((collect_marked_kernel<false>), dim3(r.tiles), dim3(COLLECT_BLOCK), 0, s, a);
+    hipLaunchKernelGGL((collect_runs_kernel<MARKED, false>), dim3(r.tiles), dim3(COLLECT_BLOCK), 0, s, a);
     hipLaunchKernelGGL(rerank_scan_kernel, dim3(r.slabs), dim3(1024), 0, s, r.tile_agg, r.tile_prefix, r.tiles, r.slab, r.slab_total,
                        r.tile_splits);
-    hipLaunchKernelGGL((collect_marked_kernel<true>), dim3(r.tiles), dim3(COLLECT_BLOCK), 0, s, a);
     HIP_TRY(hipGetLastError());
     u32* h_slabs = h->h_pinned + PINNED_HIST;
     HIP_TRY(hipMemcpyAsync(h_slabs, r.slab_total, r.slabs * 5 * sizeof(u32), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    u64 count = 0;
-    for (u32 sl = 0; sl < r.slabs; ++sl)
-        count += h_slabs[sl * 5 + 2];
+    *members = *strings = 0;
+    for (u32 sl = 0; sl < r.slabs; ++sl) {
+        *members += h_slabs[sl * 5 + 2];
+        *strings += h_slabs[sl * 5 + 3];
+    }
+    return CSA_OK;
+}
+
+// The runs whose codes are marked (long and out of order): their members are collected in list order, radix sorted by their four
+// symbols and put back. Works in key[0], key[2] and idx[2..4]: the sorted codes are not needed any more once the members are collected.
+int sort_marked_runs(Launch& L, ResolveArgs a, int* passes)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    u64 count = 0, strings = 0;
+    int rc = count_long_runs<true>(L, a, &count, &strings);
+    if (rc)
+        return rc;
+    u64* const K[2] = {h->key[2], h->key[0]};
+    u32* const V[2] = {h->idx[3], h->idx[4]};
+    a.run_keys = K[0];
+    a.members = V[0];
+    a.places = h->idx[2];
+    hipLaunchKernelGGL((collect_runs_kernel<true, true>), dim3((u32)(((u64)a.m + COLLECT_TILE - 1) / COLLECT_TILE)), dim3(COLLECT_BLOCK), 0, s, a);
+    HIP_TRY(hipGetLastError());
     int in_out = 0, run = 0;
-    int rc = radix_sort(L, SRC_PAIRS, 0, 0, h->key[1], h->idx[3], h->key[2], h->idx[4], (u32)count, make_plan(0, 64), &in_out, &run);
+    rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], V[0], K[1], V[1], (u32)count, make_plan(0, 64), &in_out, &run);
     if (rc)
         return rc;
     *passes += run;
-    if (in_out) {
-        a.keys = h->key[2];
-        a.members = h->idx[4];
-    }
+    a.run_keys = K[in_out];
+    a.members = V[in_out];
     hipLaunchKernelGGL(place_marked_kernel, dim3((u32)((count + 255) / 256)), dim3(256), 0, s, a, (u32)count);
     HIP_TRY(hipGetLastError());
+    return CSA_OK;
+}
+
+// The members of long runs, in the order of their first word by now, by their second one: collected in list order, radix sorted by the
+// ordinal of their string and the code of the next four symbols, resolved like the whole list was and put back. Leaves the
+// words that the list is resolved on: 1 if a run of that sort is too long again and out of order (or more than half
+// of the list would have to be sorted a second time), 2 otherwise. Works in key[2] and idx[2..4].
+int sort_long_runs(Launch& L, CodedList& list)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    ResolveArgs a = list.args;
+    u64 count = 0, strings = 0;
+    int rc = count_long_runs<false>(L, a, &count, &strings);
+    if (rc)
+        return rc;
+    if (count > h->cap / 2 || count > a.m / 2) {
+        list.words = 1;
+        return CSA_OK;
+    }
+    u64* const K[2] = {h->key[2], h->key[2] + h->cap / 2};
+    u32* const V[2] = {h->idx[3], h->idx[4]};
+    a.run_keys = K[0];
+    a.members = V[0];
+    a.places = h->idx[2];
+    hipLaunchKernelGGL((collect_runs_kernel<false, true>), dim3((u32)(((u64)a.m + COLLECT_TILE - 1) / COLLECT_TILE)), dim3(COLLECT_BLOCK), 0, s, a);
+    HIP_TRY(hipMemsetAsync(h->counts + 4, 0, 2 * sizeof(u32), s));
+    int in_out = 0;
+    rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], V[0], K[1], V[1], (u32)count, make_plan(0, 32 + bit_length(strings - 1)), &in_out,
+                    &list.long_passes);
+    if (rc)
+        return rc;
+    list.long_members = count;
+    a.codes = nullptr;
+    a.keys = K[in_out];
+    a.sufs = V[in_out];
+    a.m = (u32)count;
+    hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true>), dim3((u32)((count + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, a);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(h->h_pinned + 4, h->counts + 4, sizeof(u32), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    if (h->h_pinned[4] != 0)
+        list.words = 1;
     return CSA_OK;
 }
 
@@ -1136,7 +1212,7 @@ int sort_marked_runs(Launch& L, ResolveArgs a, int* passes)
 // applies them and brings rank[] up to date, directly from the kernel or through the two-pass bucketed update.
 // coded: the list comes from sort_by_codes and carries its ties.
 int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivors, u32* groups, int* rank_update,
-                u32* level_counts = nullptr, const ResolveArgs* coded = nullptr, int* passes = nullptr)
+                u32* level_counts = nullptr, CodedList* coded = nullptr, int* passes = nullptr)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -1150,29 +1226,37 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
     ra.rank_recs = nullptr;
     // the level counts of packed keys ride along: accumulated in the (idle) digit histograms, read back with the totals
     unsigned long long* const h_levels = reinterpret_cast<unsigned long long*>(h->h_pinned + PINNED_HIST + 512);
-    if (ra.levels) {
-        ra.level_totals = reinterpret_cast<unsigned long long*>(h->ghist);
-        HIP_TRY(hipMemsetAsync(ra.level_totals, 0, LEVEL_SLOTS * 8 * sizeof(unsigned long long), s));
-    }
-    if (coded)
-        hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS, true>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
-    else
-        hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS, false>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
-    if (ra.levels)
-        HIP_TRY(hipMemcpyAsync(h_levels, ra.level_totals, LEVEL_SLOTS * 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    int rc = rank_totals(L, r, true, ra.m, ra.n, false, survivors, groups, rank_update);
+    ra.level_totals = reinterpret_cast<unsigned long long*>(h->ghist);
+    auto count_and_read = [&]() -> int {
+        const bool levels = ra.levels > 0 || coded;
+        if (levels)
+            HIP_TRY(hipMemsetAsync(ra.level_totals, 0, LEVEL_SLOTS * 8 * sizeof(unsigned long long), s));
+        if (coded) {
+            ra.words = coded->words;
+            // (several tiles a wave on long lists: fewer additions to the level totals)
+            const u32 per_wave = r.tiles >= (1u << 15) ? 8u : 1u, waves = (r.tiles + per_wave - 1) / per_wave;
+            hipLaunchKernelGGL((count_ties_kernel<RANK_TILE>), dim3((waves + 3) / 4), dim3(256), 0, s, ra, r.tiles, per_wave);
+        } else {
+            hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
+        }
+        if (levels)
+            HIP_TRY(hipMemcpyAsync(h_levels, ra.level_totals, LEVEL_SLOTS * 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+        return rank_totals(L, r, true, ra.m, ra.n, false, survivors, groups, rank_update);
+    };
+    int rc = count_and_read();
     if (rc)
         return rc;
-    if (coded && h->h_pinned[4] != 0) { // long runs of one code are out of order: they are sorted now, and the list is counted again
-        rc = sort_marked_runs(L, *coded, passes);
-        if (rc)
+    if (coded) {
+        const bool unordered = h->h_pinned[4] != 0, second = h->h_pinned[5] != 0 && coded->words == 2;
+        if (unordered && (rc = sort_marked_runs(L, coded->args, passes)) != CSA_OK) // long runs of one code are out of order: they are sorted now
             return rc;
-        hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS, true>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
-        rc = rank_totals(L, r, true, ra.m, ra.n, false, survivors, groups, rank_update);
-        if (rc)
+        if (second && (rc = sort_long_runs(L, *coded)) != CSA_OK)
+            return rc;
+        if ((unordered || second) && (rc = count_and_read()) != CSA_OK)
             return rc;
     }
-    for (u32 i = 0; i < ra.levels && level_counts; ++i) {
+    const u32 levels = coded ? coded->words - 1 : ra.levels;
+    for (u32 i = 0; i < levels && level_counts; ++i) {
         u64 sv = 0, hd = 0;
         for (u32 slot = 0; slot < LEVEL_SLOTS; ++slot) {
             sv += h_levels[slot * 8 + 2 * i];
@@ -1211,7 +1295,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     const u64 wide_ell = 4ull * (u64)h->key_words;
 
     RangeScope range_sort("sort_partition n=%u", n);
-    HIP_TRY(hipMemsetAsync(h->counts, 0, 5 * sizeof(u32), s));
+    HIP_TRY(hipMemsetAsync(h->counts, 0, 6 * sizeof(u32), s));
     HIP_TRY(hipEventRecord(h->ev_gen[0], s));
 
     // ---- generation 0: every suffix sorted by its first symbols (four of them, by codes or K-gram keys, or as many as a packed
@@ -1256,7 +1340,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     u64* K[2] = {h->key[0], h->key[1]};
     u32* V[2] = {h->idx[0], h->idx[1]};
     int cur = 0; // the (K, V) set that holds the sorted pairs
-    ResolveArgs marked;
+    CodedList list;
     TextSource ps;
     memset(&ps, 0, sizeof(ps));
     if (pp.enabled) {
@@ -1277,7 +1361,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         HIP_TRY(hipGetLastError());
         rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, plan, &in_out, &p1, nullptr, 0, 0, &ps);
     } else if (coded) {
-        rc = sort_by_codes(L, d_text, n, tail, ell, marked);
+        rc = sort_by_codes(L, d_text, n, tail, h->pack_symbols ? 2u : 1u, list);
         p1 = CODE_PASSES;
         in_out = 1; // idx[1] holds the list, key[0] and key[1] what the sort has left behind
     } else {
@@ -1333,7 +1417,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         ra.level_ell[i] = (u32)wide_ell << i;
         ra.level_drop[i] = (ell - ra.level_ell[i]) * pp.codes.bits;
     }
-    rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], level_counts, coded ? &marked : nullptr, &passes);
+    ra.ties = ties_of(h);
+    rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], level_counts, coded ? &list : nullptr, &passes);
     range_gen0.close();
     if (rc)
         return rc;
@@ -1341,16 +1426,32 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     st->passes[0] = passes;
     st->active[0] = n;
     st->groups[0] = 0;
-    HIP_TRY(hipEventRecord(h->ev_gen[1], s));
 
     // ---- generations t >= 1 (reference loop: src/GPU_SACA.cu:1999-2103) ----
     int gen = 1;
+    u64 ctx = ell; // symbols resolved so far; the next generation looks hop symbols ahead
+    // A list that was resolved on two words leaves what generation 1 would: that one is reported with the lists it would have had, what
+    // the members of its large groups took, and no time of its own.
+    int resolved = 0;
+    if (coded && list.words == 2) {
+        if (level_counts[0] > 0) {
+            st->active[1] = level_counts[0];
+            st->groups[1] = level_counts[1];
+            st->big[1] = list.long_members;
+            st->passes[1] = list.long_passes;
+            resolved = 1;
+            gen = 2;
+        }
+        ctx = 2 * ell;
+    } else if (coded) {
+        st->passes[0] += list.long_passes;
+    }
+    HIP_TRY(hipEventRecord(h->ev_gen[gen], s));
     int gp = 0; // gprim[gp] / gstart[gp] describe the current groups
     bool all_small = false; // no group of the current list exceeds the limit of the generation that found it so
     bool presorted_before = false; // every large group of the generation before was in order as it stood
     bool high_limit = false; // that generation's limit was SMALL_MAXG_HI (groups only split: the limit stays from there on)
     const int sec_bits = bit_length(n > 1 ? n - 1 : 1);
-    u64 ctx = ell; // symbols resolved so far; the next generation looks hop symbols ahead
     while (m > 0) {
         if (gen >= CSA_MAX_GENERATIONS)
             return fail(CSA_ERR_INTERNAL, "generation cap reached with %u suffixes still active", m);
@@ -1641,8 +1742,11 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     if (rc)
         return rc;
 
-    for (int g = 0; g < gen; ++g)
-        HIP_TRY(hipEventElapsedTime(&st->ms[g], h->ev_gen[g], h->ev_gen[g + 1]));
+    for (int g = 0; g < gen; ++g) {
+        if (g >= 1 && g <= resolved)
+            continue;
+        HIP_TRY(hipEventElapsedTime(&st->ms[g], h->ev_gen[g], h->ev_gen[g == 0 ? resolved + 1 : g + 1]));
+    }
     HIP_TRY(hipEventElapsedTime(&st->ms_output, h->ev_gen[gen], h->ev_gen[gen + 1]));
     HIP_TRY(hipEventElapsedTime(&st->ms_total, h->ev_gen[0], h->ev_gen[gen + 1]));
     for (auto& tl : L.timed) {

@@ -13,12 +13,15 @@
 // A string whose interval of codes holds at least two 32-bit values takes the second of them, which no other string can
 // have: its suffixes carry a flag (OWN_CODE) through the sort and are known to be equal where their codes are.
 //
-// What the sort leaves open are the other suffixes that share a code: those whose strings are equal though rare by the shares of
-// their symbols (copied passages), and those whose strings are not (n / 2^32 of the rare ones by chance). resolve_runs_kernel
-// reads the strings of such suffixes from the text (and of no others: a random 128-byte line each, which is what bounds it;
-// 8.0 ms on 1e9 tokens; 14.8 when it read those of the flagged ones too), sorts every run of up to RESOLVE_MAX suffixes inside its
-// tile and sets bit 31 of every suffix that ties with its left neighbour, which is all the rank step needs to know. Longer runs
-// that are one string repeated are in order as they stand; those that are not are collected and radix sorted by the string itself.
+// What the sort leaves open are the suffixes that share a code. resolve_runs_kernel reads the strings of those whose code is not their own
+// and, of all of them, the four symbols after the string from the text (a random 128-byte line each, which is what bounds it), puts every
+// run of up to RESOLVE_MAX suffixes in order inside its tile, and notes beside every suffix on how many words of four symbols it
+// ties with its left neighbour, which is all the rank step needs to know: the list is that of generation 1, and what that generation
+// cost (a gathered line for every suffix that is tied on four symbols, a sort of its large groups, an update of the ranks) is not
+// paid. Longer runs that are one string repeated are in order as they stand; those that are not are collected and radix sorted by the
+// string itself. Then all members of long runs are sorted by the code of the next four symbols and resolved like the rest.
+// Time of whole sorts when the first sort resolves four symbols and eight: 1e9 Zipf tokens 73.2 and 65.4 ms, 2^28 18.6 and 16.9, 4096
+// 0.37 and 0.31; the kernel itself 8.1 and 13.8 ms on 1e9.
 //
 // The shares are those of single symbols, so the codes are only as even as neighbouring symbols are independent. Where a symbol has few
 // successors (phrases, records), strings that are rare by the shares of their symbols are common, and most suffixes end up in long
@@ -330,7 +333,7 @@ constexpr int RESOLVE_TILE = RESOLVE_BLOCK * RESOLVE_ITEMS;
 #endif
 constexpr int RESOLVE_MAX = CSA_RESOLVE_MAX; // longest run that is sorted inside its tile
 static_assert(CODE_ITEMS == 8, "a thread of the coding kernel writes one byte of flags");
-static_assert(RESOLVE_MAX % 64 == 0 && RESOLVE_MAX <= RESOLVE_BLOCK, "the halo is read in whole waves, one element per thread");
+static_assert(RESOLVE_MAX % 64 == 0 && 2 * RESOLVE_MAX <= RESOLVE_BLOCK, "the halo is read in whole waves, one element per thread");
 constexpr u32 RESOLVE_MARK_BITS = 20;
 constexpr u32 RESOLVE_MARK_WORDS = 1u << (RESOLVE_MARK_BITS - 5);
 
@@ -338,16 +341,22 @@ constexpr u32 RESOLVE_MARK_WORDS = 1u << (RESOLVE_MARK_BITS - 5);
 __device__ __forceinline__ u32 resolve_mark(u32 code) { return (code * 0x9E3779B1u) >> (32 - RESOLVE_MARK_BITS); }
 
 struct ResolveArgs {
-    const u32* codes; // sorted
-    const u32* sufs;  // OWN_CODE: no other string has this suffix's code
+    const u32* codes; // sorted by code: the codes ...
+    const u64* keys;  // ... or, of the members of long runs, (ordinal of the run's string << 32 | code of the four symbols after it)
+    const u32* sufs;  // OWN_CODE (with codes): no other string has this suffix's code
+    u32 m;            // entries of the list
     const u16* text;
     u32 n;
-    u32 ell; // symbols of a string; a suffix that runs off the text inside them ties with nobody
-    u32* sufs_out; // the list in order, TIED_LEFT where a suffix's string is its left neighbour's
+    u32 words; // 1: the list is resolved on the four symbols of the codes; 2: on the four after them, too
+    u32* sufs_out; // the list in order (the whole one: members of long runs go back to their places in it)
+    u8* ties;      // of every entry, TIE_LONG and on how many words it ties with its left neighbour (doubling.hpp)
     u32* marks;    // [RESOLVE_MARK_WORDS], zeroed: codes of long runs that are not in order
-    u32* unordered; // zeroed: set if there are any
-    // the collected members of marked runs (collect_marked_kernel, place_marked_kernel)
-    u64* keys;
+    u32* unordered; // zeroed: set if there are any; with keys: if the order of a long run is not that of its strings
+    u32* any_long;  // zeroed: set if there are long runs
+    // the collected members of long runs (collect_runs_kernel, place_marked_kernel)
+    const u32* text_codes; // the codes of all suffixes, by virtual position with `tail` suffixes at the front
+    u32 tail;
+    u64* run_keys;
     u32* members;
     u32* places;
     u32* tile_agg;
@@ -357,23 +366,51 @@ struct ResolveArgs {
     u32 slab;
 };
 
+// The runs of equal codes (KEYS = false: the list of all suffixes) or of equal keys (KEYS = true: the members of the long runs, sorted
+// once more by the code of the next four symbols) of one tile and the halo its first and last run reach into, refined word by word:
+// every member of a run of at most H counts those with a smaller word, which gives its place and
+// the sub-run it belongs to, and the next word is compared among the members of a sub-run only. A string and its follower lie in
+// one line of the text as a rule, so the second word costs one more line for one suffix in nine and saves a generation: its gather
+// of a line each, its list, its rank update (1e9 Zipf tokens: 13.8 ms instead of 8.1 here, 5.5 for the long runs, and 20.0 less in
+// generation 1).
+// The halo's members are refined too (by both tiles their run lies in, with the same result), so that a tile knows
+// all of its own places and writes them in order.
+template <int H, bool KEYS> // H: the longest run that is sorted inside its tile
 __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs a)
 {
-    constexpr int H = RESOLVE_MAX, SPAN = RESOLVE_TILE + 2 * H;
-    constexpr int FEW = 16; // runs of up to this many members are sorted without a look whether they are in order
+    constexpr int SPAN = RESOLVE_TILE + 2 * H;
+    constexpr int ITEMS = RESOLVE_ITEMS + 1; // the last one is the thread's element of the halo
+    constexpr int FEW = 16; // (sub-)runs of up to this many members are sorted without a look whether they are in order
     __shared__ u64 s_head[SPAN / 64]; // bit j: the element at span place j starts a run (places outside the list count as starts)
-    __shared__ u64 s_down[SPAN / 64]; // bit j: its string is smaller than that of the element before it in its run
-    __shared__ u32 s_many;            // some run of the tile has more members
-    __shared__ u64 s_key[SPAN];
-    __shared__ u32 s_suf[SPAN];
+    __shared__ u64 s_down[SPAN / 64]; // bit j: its word is smaller than that of the element before it ...
+    __shared__ u64 s_diff[SPAN / 64]; // ... or another one
+    __shared__ u32 s_many[2];         // some run of the tile has more members, by word
+    __shared__ u32 s_ends;            // some member of a run runs off the text inside its words
+    __shared__ __align__(16) u64 s_key[SPAN];
+    __shared__ __align__(16) u32 s_suf[SPAN];
+    __shared__ __align__(16) u8 s_tie[SPAN];
     const u32 t = threadIdx.x;
-    if (t == 0)
-        s_many = 0;
-    const long long t0 = (long long)blockIdx.x * RESOLVE_TILE, lo = t0 - H, n = a.n;
+    if (t < 2)
+        s_many[t] = 0;
+    if (t == 2)
+        s_ends = 0;
+    const long long t0 = (long long)blockIdx.x * RESOLVE_TILE, lo = t0 - H, m = a.m;
+    const u64 n = a.n;
     // whole waves take consecutive places: one ballot per wave and round gives 64 bits of s_head
     for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (the same rounds for every lane of a wave: SPAN is a multiple of 64)
         const long long e = lo + j;
-        const bool head = e <= 0 || e >= n || a.codes[e] != a.codes[e - 1];
+        bool head = e <= 0 || e >= m;
+        u8 tie = 0;
+        if (!head) {
+            if constexpr (KEYS) {
+                const u64 mine = a.keys[e], before = a.keys[e - 1];
+                head = mine != before;
+                tie = (mine >> 32) == (before >> 32) ? 1 : 0; // (members of one string that do not run off the text inside it)
+            } else {
+                head = a.codes[e] != a.codes[e - 1];
+            }
+        }
+        s_tie[j] = head ? tie : (u8)a.words;
         const u64 b = __ballot(head);
         if ((t & 63u) == 0)
             s_head[j / 64] = b;
@@ -395,186 +432,314 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         last = b ? wd * 64 + __builtin_ctzll(b) : SPAN + H;
         return last - first <= H;
     };
-    // own elements: suffix, run, and the string where there is company
-    u32 x[RESOLVE_ITEMS], owners = 0; // bit k of owners: element k has OWN_CODE
-    int first[RESOLVE_ITEMS], last[RESOLVE_ITEMS]; // last = 0: a long run; last - first = 1: alone
+    // the elements: suffix, place, run, and the words where there is company
+    u32 x[ITEMS], owners = 0, longs = 0; // bit k: element k has OWN_CODE; is one of a long run
+    int at[ITEMS], first[ITEMS], last[ITEMS]; // last - first = 1: alone
+    u64 w0[ITEMS], w1[ITEMS];
+    const bool two = KEYS || a.words == 2; // (keys come with two words)
 #pragma unroll
-    for (int k = 0; k < RESOLVE_ITEMS; ++k) {
-        const int j = H + k * RESOLVE_BLOCK + (int)t;
+    for (int k = 0; k < ITEMS; ++k) {
+        const bool halo = k == RESOLVE_ITEMS;
+        const int j = !halo ? H + k * RESOLVE_BLOCK + (int)t : (int)t < H ? (int)t : RESOLVE_TILE + (int)t;
         const long long e = lo + j;
         x[k] = 0;
-        first[k] = j;
+        at[k] = first[k] = j;
         last[k] = j + 1;
-        if (e < n) {
-            x[k] = a.sufs[e];
-            owners |= (x[k] & OWN_CODE ? 1u : 0u) << k;
-            x[k] &= ~OWN_CODE;
-            if (!run_of(j, first[k], last[k])) {
-                first[k] = j;
-                last[k] = 0;
-            }
+        w0[k] = w1[k] = 0;
+        if (e < 0 || e >= m || (halo && (int)t >= 2 * H))
+            continue;
+        int f, l;
+        const bool is_short = run_of(j, f, l);
+        if (halo) { // members of runs that reach into the tile; of a long run the left neighbour of the tile's first element alone
+            const bool left = (int)t < H;
+            if (is_short ? (left ? l <= H : f >= H + RESOLVE_TILE) : j != H - 1)
+                continue;
         }
-    }
-#pragma unroll
-    for (int k = 0; k < RESOLVE_ITEMS; ++k) {
-        const int j = H + k * RESOLVE_BLOCK + (int)t;
-        if (last[k] - first[k] != 1) {
-            s_suf[j] = x[k];
-            if (!((owners >> k) & 1u)) {
-                s_key[j] = load_kgram(a.text, a.n, x[k], 0);
-                if (last[k] - first[k] > FEW)
-                    s_many = 1;
-            }
+        x[k] = a.sufs[e];
+        if (!KEYS && (x[k] & OWN_CODE))
+            owners |= 1u << k;
+        x[k] &= ~OWN_CODE;
+        if (is_short) {
+            first[k] = f;
+            last[k] = l;
+            if (l - f == 1)
+                continue;
+        } else {
+            longs |= 1u << k;
         }
-    }
-    // of the halo: the members of short runs that reach into the tile, and the left neighbour of the tile's first element
-    {
-        int f0, l0, f1, l1;
-        const int j_last = (int)((t0 + RESOLVE_TILE < n ? t0 + RESOLVE_TILE : n) - 1 - lo);
-        const bool short0 = run_of(H, f0, l0), short1 = run_of(j_last, f1, l1);
-        for (int i = t; i < 2 * H; i += RESOLVE_BLOCK) {
-            const int j = i < H ? i : RESOLVE_TILE + i;
-            const long long e = lo + j;
-            const bool wanted = i < H ? (short0 ? j >= f0 : j == H - 1) : (short1 && j < l1);
-            if (wanted && e >= 0 && e < n) {
-                const u32 y = a.sufs[e];
-                s_suf[j] = y & ~OWN_CODE;
-                if (!(y & OWN_CODE))
-                    s_key[j] = load_kgram(a.text, a.n, y, 0);
-            }
+        const bool own = (owners >> k) & 1u;
+        if (!KEYS && !own)
+            w0[k] = load_kgram(a.text, a.n, x[k], 0);
+        if (two && (KEYS || is_short)) // (the members of long runs of codes get their second word when they are sorted by it)
+            w1[k] = load_kgram(a.text, a.n, x[k], 1);
+        if ((u64)x[k] + 4u * a.words >= n)
+            s_ends = 1;
+        if (is_short && l - f > FEW) {
+            s_many[0] = 1;
+            s_many[1] = 1;
         }
     }
     __syncthreads();
-    // A run that is one string repeated, or several in order, stays as it is: its members need not be compared with each other. (In a
-    // short text the kernel takes as long as the longest run of a tile: generation 0 of 2^18 symbols of phrases 221 us with
-    // all comparisons, 191 without these; the kernel takes 8.55 instead of 8.45 ms on 1e9 tokens for it.)
-    const bool many = s_many != 0;
-    if (many) {
-        for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (places whose strings were not wanted hold anything: no run looked at below has any)
-            const bool down = j > 0 && !((s_head[j / 64] >> (j & 63)) & 1ull) && s_key[j] < s_key[j - 1];
-            const u64 b = __ballot(down);
-            if ((t & 63u) == 0)
-                s_down[j / 64] = b;
-        }
-        __syncthreads();
-    }
-    auto in_order = [&](int from, int to) -> bool { // places from + 1 .. to - 1: at most RESOLVE_MAX of them
-        u64 seen = 0;
-        for (int wd = from / 64; wd <= (to - 1) / 64; ++wd) {
-            u64 b = s_down[wd];
-            if (wd == from / 64)
-                b &= (from & 63) == 63 ? 0ull : ~0ull << ((from & 63) + 1);
-            if (wd == (to - 1) / 64)
-                b &= ~0ull >> (63 - ((to - 1) & 63));
-            seen |= b;
-        }
-        return seen == 0;
-    };
+    const bool ends = s_ends != 0;
+    // One word of all elements that still have company: refines their runs. Whoever runs off the text inside the word ties with
+    // nobody and comes before those with the same padded word, shortest first.
+    auto refine = [&](int w) {
 #pragma unroll
-    for (int k = 0; k < RESOLVE_ITEMS; ++k) {
-        const int j = H + k * RESOLVE_BLOCK + (int)t;
-        const long long e = lo + j;
-        if (e >= n)
-            continue;
-        const bool whole = (u64)x[k] + a.ell < a.n;
-        int place = j;
-        bool tied = false;
-        if ((owners >> k) & 1u) { // one string, in order as it stands
-            if (!((s_head[j / 64] >> (j & 63)) & 1ull))
-                tied = whole && (u64)s_suf[j - 1] + a.ell < a.n;
-        } else if (last[k] == 0) {
-            if (!((s_head[j / 64] >> (j & 63)) & 1ull)) {
-                const u64 mine = s_key[j], before = s_key[j - 1];
-                tied = mine == before && whole && (u64)s_suf[j - 1] + a.ell < a.n;
-                if (mine < before) {
-                    const u32 mark = resolve_mark(a.codes[e]), bit = 1u << (mark & 31u);
-                    if (!(a.marks[mark >> 5] & bit)) // (soon set for all to see: few of a run's members get to the atomic)
-                        atomicOr(&a.marks[mark >> 5], bit);
-                    *a.unordered = 1u;
+        for (int k = 0; k < ITEMS; ++k)
+            if (last[k] - first[k] > 1 || ((longs >> k) & 1u)) {
+                s_suf[at[k]] = x[k];
+                if (w == 1 || !((owners >> k) & 1u))
+                    s_key[at[k]] = w == 0 ? w0[k] : w1[k];
+            }
+        __syncthreads();
+        const bool many = s_many[w] != 0 && !ends;
+        if (many) {
+            for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (places whose words were not wanted hold anything: no run looked at below has any)
+                const u64 down = __ballot(j > 0 && s_key[j] < s_key[j - 1]), diff = __ballot(j > 0 && s_key[j] != s_key[j - 1]);
+                if ((t & 63u) == 0) {
+                    s_down[j / 64] = down;
+                    s_diff[j / 64] = diff;
                 }
             }
-        } else if (last[k] - first[k] > FEW && in_order(first[k], last[k])) {
-            if (j != first[k])
-                tied = s_key[j] == s_key[j - 1] && whole && (u64)s_suf[j - 1] + a.ell < a.n;
-        } else if (last[k] - first[k] > 1) {
-            const u64 mine = s_key[j];
-            place = first[k];
-            for (int i = first[k]; i < last[k]; ++i) {
-                const u64 v = s_key[i];
-                if (v < mine || (v == mine && i < j))
-                    ++place;
-                if (v == mine && i < j && whole && (u64)s_suf[i] + a.ell < a.n)
-                    tied = true; // (the suffixes that run off the text come first among equal strings)
-            }
+            __syncthreads();
         }
-        a.sufs_out[lo + place] = x[k] | (tied ? TIED_LEFT : 0u);
+        const u64 ctx = 4u * (u32)(w + 1);
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const int f = first[k], l = last[k], j = at[k];
+            if ((longs >> k) & 1u || l - f <= 1)
+                continue;
+            const bool own = w == 0 && ((owners >> k) & 1u);
+            int nf = f, nl = l, place = j;
+            if (own) { // one string: those that run off the text come first as they stand
+                if (ends) {
+                    while (nf < l && (u64)s_suf[nf] + ctx >= n)
+                        ++nf;
+                    if (j < nf) {
+                        nf = j;
+                        nl = j + 1;
+                    }
+                }
+            } else {
+                bool counted = true;
+                if (many && l - f > FEW) {
+                    // A run that is one string repeated, or several in order, stays as it is: its members need not be compared with
+                    // each other. (In a short text the kernel takes as long as the longest run of a tile: generation 0 of 2^18
+                    // symbols of phrases 221 us with all comparisons, 191 without these.)
+                    u64 seen = 0;
+                    for (int wd = (f + 1) / 64; wd <= (l - 1) / 64; ++wd) { // places f + 1 .. l - 1
+                        u64 b = s_down[wd];
+                        if (wd == (f + 1) / 64)
+                            b &= ~0ull << ((f + 1) & 63);
+                        if (wd == (l - 1) / 64)
+                            b &= ~0ull >> (63 - ((l - 1) & 63));
+                        seen |= b;
+                    }
+                    if (seen == 0) {
+                        counted = false;
+                        int wd = j / 64; // the last other word at or before j, the first behind it
+                        u64 b = s_diff[wd] & (~0ull >> (63 - (j & 63)));
+                        while (b == 0 && wd > f / 64)
+                            b = s_diff[--wd];
+                        const int start = b ? wd * 64 + 63 - __builtin_clzll(b) : f;
+                        nf = start > f ? start : f;
+                        wd = j / 64;
+                        b = (j & 63) == 63 ? 0ull : s_diff[wd] & (~0ull << ((j & 63) + 1));
+                        while (b == 0 && wd < (l - 1) / 64)
+                            b = s_diff[++wd];
+                        const int stop = b ? wd * 64 + __builtin_ctzll(b) : l;
+                        nl = stop < l ? stop : l;
+                    }
+                }
+                if (counted) {
+                    const u64 mine = s_key[j];
+                    int less = 0, equal = 0, before = 0; // equal: itself included
+                    if (!ends) {
+                        for (int i = f; i < l; ++i) {
+                            const u64 v = s_key[i];
+                            less += v < mine ? 1 : 0;
+                            equal += v == mine ? 1 : 0;
+                            before += v == mine && i < j ? 1 : 0;
+                        }
+                    } else {
+                        const bool whole = (u64)x[k] + ctx < n;
+                        for (int i = f; i < l; ++i) {
+                            const u64 v = s_key[i];
+                            if (v < mine) {
+                                ++less;
+                            } else if (v == mine) {
+                                const u32 y = s_suf[i];
+                                const bool y_whole = (u64)y + ctx < n;
+                                if (whole != y_whole)
+                                    less += whole ? 1 : 0;
+                                else if (!whole)
+                                    less += y > x[k] ? 1 : 0;
+                                else
+                                    ++equal, before += i < j ? 1 : 0;
+                            }
+                        }
+                        equal = whole ? equal : 1;
+                    }
+                    nf = f + less;
+                    nl = nf + equal;
+                    place = nf + before;
+                }
+            }
+            if (place == nf && nf != f)
+                s_tie[nf] = (u8)w;
+            first[k] = nf;
+            last[k] = nl;
+            at[k] = place;
+        }
+        // the members of long runs stay where they are: do they tie with their left neighbours, are they in order?
+#pragma unroll
+        for (int k = 0; k < RESOLVE_ITEMS; ++k)
+            if ((longs >> k) & 1u && w == (KEYS ? 1 : 0)) {
+                const int j = at[k];
+                u8 tie = s_tie[j];
+                if (!((s_head[j / 64] >> (j & 63)) & 1ull)) {
+                    const bool whole = (u64)x[k] + ctx < n && (u64)s_suf[j - 1] + ctx < n;
+                    const bool own = w == 0 && ((owners >> k) & 1u);
+                    const u64 mine = own ? 0 : s_key[j], left = own ? 0 : s_key[j - 1];
+                    tie = (u8)(w + (mine == left && whole ? 1 : 0));
+                    if constexpr (KEYS) {
+                        if (mine < left || !whole)
+                            *a.unordered = 1u;
+                    } else if (mine < left) {
+                        const u32 mark = resolve_mark(a.codes[lo + j]), bit = 1u << (mark & 31u);
+                        if (!(a.marks[mark >> 5] & bit)) // (soon set for all to see: few of a run's members get to the atomic)
+                            atomicOr(&a.marks[mark >> 5], bit);
+                        *a.unordered = 1u;
+                    }
+                } else {
+                    *a.any_long = 1u;
+                }
+                s_tie[j] = tie | TIE_LONG;
+            }
+        __syncthreads();
+    };
+    if constexpr (!KEYS)
+        refine(0);
+    if (two)
+        refine(1);
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+        if (k < RESOLVE_ITEMS || (int)t < 2 * H)
+            s_suf[at[k]] = x[k];
+    __syncthreads();
+    const int j = H + (int)t * RESOLVE_ITEMS;
+    const long long e = lo + j;
+    if constexpr (!KEYS) {
+        if (e + RESOLVE_ITEMS <= m) { // (e is a multiple of RESOLVE_ITEMS, and the arrays are 16-byte aligned)
+            static_assert(RESOLVE_ITEMS == 4 && H % 4 == 0, "four suffixes leave in one 16-byte store");
+            *reinterpret_cast<uint4*>(a.sufs_out + e) = *reinterpret_cast<const uint4*>(s_suf + j);
+            *reinterpret_cast<u32*>(a.ties + e) = *reinterpret_cast<const u32*>(s_tie + j);
+            return;
+        }
     }
+#pragma unroll
+    for (int k = 0; k < RESOLVE_ITEMS; ++k)
+        if (e + k < m) {
+            const u64 to = KEYS ? (u64)a.places[e + k] : (u64)(e + k);
+            a.sufs_out[to] = s_suf[j + k];
+            a.ties[to] = s_tie[j + k];
+        }
 }
 
-// Members of marked runs, in list order: APPLY = false counts them per tile, APPLY = true (after rerank_scan_kernel) writes
-// their strings, suffixes and list places. A run is marked as a whole, so the list of them sorted by string, which
-// is also the order of the codes, goes back to the same places.
+// Members of long runs, in list order: APPLY = false counts them and the strings they begin per tile, APPLY = true (after
+// rerank_scan_kernel) writes what they are to be sorted by, their suffixes and their list places. MARKED: those of runs that are out of
+// order alone, by their strings; a run is marked as a whole, so the list of them sorted by string, which is also the order
+// of the codes, goes back to the same places. Otherwise all of them, by the ordinal of their string (they are in order by
+// now) and the code of the next four symbols.
 constexpr int COLLECT_BLOCK = 256;
 constexpr int COLLECT_ITEMS = 4;
 constexpr int COLLECT_TILE = COLLECT_BLOCK * COLLECT_ITEMS;
 
-template <bool APPLY>
-__global__ __launch_bounds__(COLLECT_BLOCK) void collect_marked_kernel(ResolveArgs a)
+template <bool MARKED, bool APPLY>
+__global__ __launch_bounds__(COLLECT_BLOCK) void collect_runs_kernel(ResolveArgs a)
 {
-    __shared__ u32 s_w[COLLECT_BLOCK / WAVE];
+    __shared__ u32 s_w[COLLECT_BLOCK / WAVE][2];
     const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6;
     const u32 tile = blockIdx.x;
     const u64 base = (u64)tile * COLLECT_TILE + (u64)t * COLLECT_ITEMS;
-    u32 flags = 0, mine = 0;
+    static_assert(COLLECT_ITEMS == 4, "the ties of a thread's entries come in one word");
+    u32 ties = 0;
+    if (base + COLLECT_ITEMS <= a.m) {
+        ties = *reinterpret_cast<const u32*>(a.ties + base);
+    } else {
+#pragma unroll
+        for (int k = 0; k < COLLECT_ITEMS; ++k)
+            ties |= base + k < a.m ? (u32)a.ties[base + k] << (8 * k) : 0u;
+    }
+    u32 flags = 0, mine = 0, heads = 0;
 #pragma unroll
     for (int k = 0; k < COLLECT_ITEMS; ++k)
-        if (base + k < a.n) {
-            const u32 mark = resolve_mark(a.codes[base + k]);
-            const u32 in = (a.marks[mark >> 5] >> (mark & 31u)) & 1u;
+        if ((ties >> (8 * k)) & TIE_LONG) {
+            u32 in = 1u;
+            if constexpr (MARKED) {
+                const u32 mark = resolve_mark(a.codes[base + k]);
+                in = (a.marks[mark >> 5] >> (mark & 31u)) & 1u;
+            }
             flags |= in << k;
             mine += in;
+            heads += in && ((ties >> (8 * k)) & TIE_WORDS) == 0 ? 1u : 0u;
         }
-    const u32 incl = wave_incl_sum(mine);
-    if (lane == 63u)
-        s_w[w] = incl;
+    const u32 incl = wave_incl_sum(mine), incl_heads = wave_incl_sum(heads);
+    if (lane == 63u) {
+        s_w[w][0] = incl;
+        s_w[w][1] = incl_heads;
+    }
     __syncthreads();
-    u32 slot = incl - mine, total = 0;
+    u32 slot = incl - mine, total = 0, ordinal = incl_heads - heads, total_heads = 0;
     for (u32 ww = 0; ww < COLLECT_BLOCK / WAVE; ++ww) {
-        if (ww < w)
-            slot += s_w[ww];
-        total += s_w[ww];
+        if (ww < w) {
+            slot += s_w[ww][0];
+            ordinal += s_w[ww][1];
+        }
+        total += s_w[ww][0];
+        total_heads += s_w[ww][1];
     }
     if (!APPLY) {
         if (t == 0) {
             a.tile_agg[(u64)tile * 4 + 0] = 0;
             a.tile_agg[(u64)tile * 4 + 1] = 0;
             a.tile_agg[(u64)tile * 4 + 2] = total;
-            a.tile_agg[(u64)tile * 4 + 3] = 0;
+            a.tile_agg[(u64)tile * 4 + 3] = total_heads;
             a.tile_splits[tile] = 0;
         }
         return;
     }
-    slot += a.tile_prefix[(u64)tile * 4 + 2] + slabs_before(a.slab_total, tile / a.slab).sum2;
+    const SlabPrefix sp = slabs_before(a.slab_total, tile / a.slab);
+    slot += a.tile_prefix[(u64)tile * 4 + 2] + sp.sum2;
+    ordinal += a.tile_prefix[(u64)tile * 4 + 3] + sp.sum3; // strings begun before this thread's entries
 #pragma unroll
     for (int k = 0; k < COLLECT_ITEMS; ++k)
         if ((flags >> k) & 1u) {
-            const u32 x = a.sufs_out[base + k] & ~TIED_LEFT;
-            a.keys[slot] = load_kgram(a.text, a.n, x, 0);
+            const u32 x = a.sufs_out[base + k];
+            if constexpr (MARKED) {
+                a.run_keys[slot] = load_kgram(a.text, a.n, x, 0);
+            } else {
+                ordinal += ((ties >> (8 * k)) & TIE_WORDS) == 0 ? 1u : 0u;
+                const u64 y = (u64)x + 4u; // (a suffix that has none there is a string of its own)
+                const u32 next = y >= a.n ? 0u : a.text_codes[y + a.tail >= a.n ? a.n - 1 - y : y + a.tail];
+                a.run_keys[slot] = ((u64)(ordinal - 1u) << 32) | next;
+            }
             a.members[slot] = x;
             a.places[slot] = (u32)(base + k);
             ++slot;
         }
 }
 
-// The collected members, sorted by string, back to their places.
+// The collected members of marked runs, sorted by string, back to their places.
 __global__ __launch_bounds__(256) void place_marked_kernel(ResolveArgs a, u32 count)
 {
     const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
     if (i >= count)
         return;
     const u32 x = a.members[i];
-    const bool tied = i > 0 && a.keys[i] == a.keys[i - 1] && (u64)x + a.ell < a.n && (u64)a.members[i - 1] + a.ell < a.n;
-    a.sufs_out[a.places[i]] = x | (tied ? TIED_LEFT : 0u);
+    const bool tied = i > 0 && a.run_keys[i] == a.run_keys[i - 1] && (u64)x + 4 < a.n && (u64)a.members[i - 1] + 4 < a.n;
+    a.sufs_out[a.places[i]] = x;
+    a.ties[a.places[i]] = (u8)(TIE_LONG | (tied ? 1u : 0u));
 }
 
 } // namespace csa

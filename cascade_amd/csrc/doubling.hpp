@@ -13,7 +13,7 @@ namespace csa {
 // was measured at 2.5 to 4 times the duration of these three on this part: with 8 XCDs the look-back words travel
 // over the fabric, and the few resident workgroups per CU spent most of their life waiting for their predecessors.)
 //
-// Input: all suffixes sorted by key, keys[c] / sufs[c] for c in [0, n), or a list that carries its ties (TIED_LEFT). The rank of a suffix is the index of the
+// Input: all suffixes sorted by key, keys[c] / sufs[c] for c in [0, n), or a list that carries its ties. The rank of a suffix is the index of the
 // head of its run of equal keys (reference: include/GPU_SACA.cuh:191-208; the max-scan of src/GPU_SACA.cu:1241-1247
 // is the max chain here). A suffix whose run has length 1 retires: its rank is final, and the sorted index array
 // already holds it at its place of the suffix array. The others are compacted, in order, into the first active list
@@ -21,8 +21,11 @@ namespace csa {
 // ---------------------------------------------------------------------------------------------
 
 constexpr u32 NO_RANK = 0xFFFFFFFFu; // ranks are below 2^31
-// Bit 31 of a suffix in a list whose ties have been resolved already (coded_keys.hpp): its key is that of the suffix before it.
-constexpr u32 TIED_LEFT = 0x80000000u; // suffixes are below 2^31
+// A list whose ties have been resolved already (coded_keys.hpp) carries a byte for every entry: how many words of four symbols it
+// shares with its left neighbour (as far as they were looked at), neither of them running off the text, and whether it is one of a
+// run that was too long to be resolved in its tile.
+constexpr u32 TIE_LONG = 0x80u, TIE_WORDS = 0x7Fu;
+constexpr u32 TIE_MOST_WORDS = 2;
 
 // The tiles of a rank step are scanned in RERANK_SLABS slabs (rerank_scan_kernel): a tile's prefix is its prefix inside
 // its slab combined with the totals (max, max, sum, sum, -) of the slabs before. One slab per lane: a wave fetches the
@@ -61,6 +64,8 @@ constexpr u32 MAX_LEVELS = 4, LEVEL_SLOTS = 64;
 struct RerankArgs {
     const u64* keys; // unused where the list carries its ties (TIED)
     const u32* sufs;
+    const u8* ties;  // TIED: the bytes of the list's entries, and the words that the list is ranked on: neighbours belong to one
+    u32 words;       // run if they share as many
     u32 m;         // = n: generation 0 ranks every suffix
     u32 n;         // partition size
     u32 ell;       // symbols in the generation-0 key
@@ -137,13 +142,9 @@ __device__ __forceinline__ void load_with_neighbours(const u64* __restrict__ key
     }
 }
 
-// Whether sorted element c (key_c, suf_c) belongs to the run of element c - 1 (key_b, suf_b); both exist. TIED: the
-// list says so itself, and carries no keys.
-template <bool TIED>
+// Whether sorted element c (key_c, suf_c) belongs to the run of element c - 1 (key_b, suf_b); both exist.
 __device__ __forceinline__ bool same_run(const RerankArgs& a, u64 key_b, u32 suf_b, u64 key_c, u32 suf_c)
 {
-    if constexpr (TIED)
-        return (suf_c & TIED_LEFT) != 0;
     // a suffix that runs off the text inside its key ties with nobody (include/bit-layout.hpp:99-100)
     return key_b == key_c && (u64)suf_b + a.ell < a.n && (u64)suf_c + a.ell < a.n;
 }
@@ -151,8 +152,7 @@ __device__ __forceinline__ bool same_run(const RerankArgs& a, u64 key_b, u32 suf
 // The counting pass of generation 0 on its own: the per-tile aggregates need no ordering inside the tile, so every
 // thread reads its ITEMS elements and their two neighbours straight from the arrays (no exchange through LDS, one
 // barrier) and the tile reduces instead of scanning. Same run and tail rules as rerank_kernel below.
-// TIED: the list carries its ties (RerankArgs::sufs with TIED_LEFT) instead of keys: 4 bytes read per suffix, not 12.
-template <int BLOCK, int ITEMS, bool TIED>
+template <int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
 {
     constexpr int TILE = BLOCK * ITEMS;
@@ -166,13 +166,13 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
     const u32 m = a.m;
     u64 key[ITEMS + 2] = {}; // elements base - 1 .. base + ITEMS
     u32 suf[ITEMS + 2];
-    load_with_neighbours<ITEMS, !TIED>(a.keys, a.sufs, base, m, key, suf);
+    load_with_neighbours<ITEMS, true>(a.keys, a.sufs, base, m, key, suf);
     u32 la = 0, lcnt = 0, lheads = 0;
     bool prev_eq = false;
 #pragma unroll
     for (int k = 0; k < ITEMS + 1; ++k) {
         const u64 c = base + k; // right element of the pair (c - 1, c)
-        const bool e = c >= 1 && c < m && same_run<TIED>(a, key[k], suf[k], key[k + 1], suf[k + 1]);
+        const bool e = c >= 1 && c < m && same_run(a, key[k], suf[k], key[k + 1], suf[k + 1]);
         if (k >= 1 && c - 1 < m) { // element c - 1 = base + k - 1: prev_eq ties it to its left, e to its right
             const bool ka = !prev_eq;
             const bool single = ka && !e;
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
     }
     // the same counts at the shorter contexts of packed keys (one-word keys: nothing is read from the text)
     __shared__ u32 s_level[WAVES][MAX_LEVELS];
-    for (u32 i = 0; !TIED && i < a.levels; ++i) {
+    for (u32 i = 0; i < a.levels; ++i) {
         const u32 drop = a.level_drop[i];
         const u64 lell = a.level_ell[i];
         u32 cs = 0, ch = 0;
@@ -247,6 +247,80 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
     }
 }
 
+// The same for a list that carries its ties, at every number of words up to TIE_MOST_WORDS at once: one byte read per suffix. A wave takes
+// whole tiles, PER bytes a lane, and `per_wave` of them one after the other; the tile aggregates are those at a.words, the
+// survivors and groups at i + 1 words are added to level_totals[.. + 2 i] and [.. + 2 i + 1].
+template <int TILE>
+__global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles, u32 per_wave)
+{
+    constexpr int PER = TILE / WAVE;
+    static_assert(PER % 16 == 0 && PER <= 32, "a lane's bytes come in 16-byte loads, their ties fit a word");
+    const u32 lane = threadIdx.x & 63u;
+    const u32 wave = blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
+    u32 sum_surv[TIE_MOST_WORDS] = {}, sum_heads[TIE_MOST_WORDS] = {};
+    for (u32 r = 0; r < per_wave; ++r) {
+        const u64 tile = (u64)wave * per_wave + r;
+        if (tile >= tiles)
+            break;
+        const u64 base = tile * TILE + (u64)lane * PER;
+        u32 tie[TIE_MOST_WORDS] = {}; // bit k: element base + k shares that many words with its left neighbour
+        if (base + PER <= a.m) {
+#pragma unroll
+            for (int q = 0; q < PER; q += 16) {
+                const uint4 v = *reinterpret_cast<const uint4*>(a.ties + base + q);
+                const u32 word[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int k = 0; k < 16; ++k)
+#pragma unroll
+                    for (u32 i = 0; i < TIE_MOST_WORDS; ++i)
+                        tie[i] |= (((word[k / 4] >> (8 * (k % 4))) & TIE_WORDS) > i ? 1u : 0u) << (q + k);
+            }
+        } else {
+            for (int k = 0; k < PER; ++k)
+                if (base + k < a.m)
+                    for (u32 i = 0; i < TIE_MOST_WORDS; ++i)
+                        tie[i] |= ((a.ties[base + k] & TIE_WORDS) > i ? 1u : 0u) << k;
+        }
+        const u64 behind = (tile + 1) * TILE;
+        const u32 after = behind < a.m ? a.ties[behind] & TIE_WORDS : 0u;
+        const u32 have = base >= a.m ? 0u : a.m - base >= PER ? PER : (u32)(a.m - base);
+        const u32 valid = have == 32u ? 0xFFFFFFFFu : (1u << have) - 1u;
+#pragma unroll
+        for (u32 i = 0; i < TIE_MOST_WORDS; ++i) {
+            const u64 firsts = __ballot(tie[i] & 1u);
+            const u32 next = lane == 63u ? (after > i ? 1u : 0u) : (u32)(firsts >> (lane + 1)) & 1u;
+            const u32 right = (tie[i] >> 1) | (next << (PER - 1)); // bit k: element base + k + 1 ties with it
+            const u32 surv = (u32)__popc((tie[i] | right) & valid), heads = (u32)__popc(~tie[i] & right & valid);
+            sum_surv[i] += surv;
+            sum_heads[i] += heads;
+            if (i + 1 == a.words) {
+                const u32 begin = ~tie[i] & valid; // (1-based: 0 means no head in the tile)
+                const u32 last = begin ? (u32)base + 32u - (u32)__builtin_clz(begin) : 0u;
+                u32 most = last, packed = surv | (heads << 16);
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) {
+                    const u32 other = __shfl_xor(most, o);
+                    most = most > other ? most : other;
+                    packed += __shfl_xor(packed, o);
+                }
+                if (lane == 0) {
+                    *reinterpret_cast<uint4*>(a.tile_agg + tile * 4) = make_uint4(most, 0u, packed & 0xFFFFu, packed >> 16);
+                    a.tile_splits[tile] = 0;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (u32 i = 0; i < TIE_MOST_WORDS; ++i) {
+        const u32 sv = wave_reduce_sum(sum_surv[i]), hd = wave_reduce_sum(sum_heads[i]);
+        unsigned long long* const slot = a.level_totals + (u64)(wave % LEVEL_SLOTS) * 8 + 2 * i;
+        if (lane == 0 && sv) {
+            atomicAdd(slot, (unsigned long long)sv);
+            atomicAdd(slot + 1, (unsigned long long)hd);
+        }
+    }
+}
+
 // The applying pass: reads the tile's exclusive prefix from tile_prefix (rerank_count_kernel and rerank_scan_kernel
 // before it) and does the work. What the tile produces is collected in LDS and leaves in striped order (consecutive
 // lanes, consecutive elements).
@@ -276,11 +350,26 @@ __global__ __launch_bounds__(BLOCK) void rerank_kernel(RerankArgs a)
     load_with_neighbours<ITEMS, !TIED>(a.keys, a.sufs, base, m, key, suf);
     // eq[k]: elements (base+k-1) and (base+k) exist and belong to one run of equal keys
     bool eq[ITEMS + 1];
+    if constexpr (TIED) {
+        static_assert(ITEMS == 4, "the ties of a thread's elements come in one word");
+        u32 ties = 0;
+        if (base + ITEMS <= m) {
+            ties = *reinterpret_cast<const u32*>(a.ties + base);
+        } else {
 #pragma unroll
-    for (int k = 0; k < ITEMS + 1; ++k) {
-        const u64 c = base + k; // right element of the pair
-        const bool e = c >= 1 && c < m && same_run<TIED>(a, key[k], suf[k], key[k + 1], suf[k + 1]);
-        eq[k] = e;
+            for (int k = 0; k < ITEMS; ++k)
+                ties |= base + k < m ? (u32)a.ties[base + k] << (8 * k) : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k)
+            eq[k] = ((ties >> (8 * k)) & TIE_WORDS) >= a.words;
+        eq[ITEMS] = base + ITEMS < m && (a.ties[base + ITEMS] & TIE_WORDS) >= a.words;
+    } else {
+#pragma unroll
+        for (int k = 0; k < ITEMS + 1; ++k) {
+            const u64 c = base + k; // right element of the pair
+            eq[k] = c >= 1 && c < m && same_run(a, key[k], suf[k], key[k + 1], suf[k + 1]);
+        }
     }
 
     // thread-local aggregates; head positions are kept 1-based (c + 1), so that 0 means "no head so far"
@@ -341,7 +430,7 @@ __global__ __launch_bounds__(BLOCK) void rerank_kernel(RerankArgs a)
             const bool single = ka && !eq[k + 1];
             if (ka)
                 ra = (u32)c + 1u;
-            const u32 x = TIED ? suf[k + 1] & ~TIED_LEFT : suf[k + 1];
+            const u32 x = suf[k + 1];
             const u32 nr = ra - 1u; // element 0 is always a head, so ra >= 1 here
             if (ra == 0 || nr >= a.n || x >= a.n) { // a corrupt sorted list: report it instead of writing out of bounds
                 atomicExch(a.err, DEV_ERR_RERANK_RANGE);

@@ -69,9 +69,11 @@ typedef struct csa_stats {
     uint64_t presorted[CSA_MAX_GENERATIONS]; /* of big[g], members that skipped the radix sort: every large group of the
                                                 list was in order of rank[x + h] already (rising or falling along the
                                                 list, as in runs of one token and periodic stretches) */
-    uint32_t key_symbols;            /* symbols the first sort resolved: 4 (by 32-bit codes of them, or by K-gram words where
+    uint32_t key_symbols;            /* symbols in the keys of the first sort: 4 (by 32-bit codes of them, or by K-gram words where
                                         too many suffixes would share a code), or up to 64 when the text's alphabet is small
-                                        enough for packed codes of 1, 2, 4 or 8 bits */
+                                        enough for packed codes of 1, 2, 4 or 8 bits. A sort by codes goes on to resolve the
+                                        next four symbols from the text: generation 1 is then reported with the list it would
+                                        have had, the members of long runs in big[1], their passes in passes[1], and no time */
     uint32_t first_sort_generations; /* generations of the reference that sort stands for: 1, or 1 + j when its keys held
                                         4 * key_words * 2^j symbols. Generations 1 .. j are then reported with the lists
                                         they would have had (active[], groups[]) and with no time or passes of their own */
@@ -145,8 +147,8 @@ int csa_set_device_exclusive(csa_handle* h, int exclusive);
  *                                together with room to spare: values above compute units / 16 fail with CSA_ERR_ARG
  *   CSA_TUNE_PACK_SYMBOLS        1 (default): a text whose symbols take at most 256 values (by the values its low and its
  *                                high bytes take) is sorted first on keys of as many packed symbols as 64 bits hold, which
- *                                covers the first generations of the doubling (csa_stats.first_sort_generations); 0: the
- *                                first sort always resolves four symbols
+ *                                covers the first generations of the doubling (csa_stats.first_sort_generations), and a sort
+ *                                by codes resolves eight symbols; 0: the first sort always resolves four symbols
  *   CSA_TUNE_EXPECT_PRESORTED    0 (default): a generation leaves out the (key, suffix) pairs of its large groups' radix sort
  *                                when every large group of the generation before was in order as it stood (csa_stats.presorted),
  *                                and gathers again with them if this one's are not; 1: every generation starts that way

@@ -768,3 +768,19 @@ def test_runs_of_one_code_that_are_in_order_and_end_with_the_text(emu, zeros, ta
     assert emu_sort.passes[0] == 4
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
+@pytest.mark.parametrize("key_words", [1, 3])
+@pytest.mark.parametrize("repeats,followers,end", [([64, 65, 300], 40, 0), ([200, 200, 65], 3, 0), ([200, 129], 2, 6), ([130, 2, 3], 50, 3),
+                                                   ([400], 1, 0), ([63, 64], 7, 4)])
+def test_runs_of_one_string_are_resolved_on_their_next_four_symbols(emu, repeats, followers, end, key_words):
+    """Runs of one code up to the limit of the in-tile sort (64 members in this build) take the next four symbols there, longer ones are
+    sorted by the code of them and resolved again, whether what they come apart into is short, long and in order or (at the end of the
+    text) long and not. Suffix array and generation sizes are the oracle's, with and without the second word."""
+    T = texts.text_with_repeated_strings(9000, repeats, followers, end, followers + end)
+    sa, counts = oracle_lib.prefix_doubling(T, key_words)
+    for pack in (True, False):
+        got, active, big = emu_sort(emu, T, key_words, pack=pack)
+        assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+        if pack and key_words == 1 and emu_sort.passes[0] == 4:  # (the probe may have sent the text to the K-grams)
+            assert (big[1] > 0) == (max(repeats) > 64)

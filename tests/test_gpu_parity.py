@@ -728,3 +728,19 @@ def test_first_sort_chooses_between_codes_and_kgrams(torch_mod, n, phrases, pass
     assert stats["passes"][0] == passes
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
+
+
+@pytest.mark.parametrize("repeats,followers,end", [([256, 257, 3000], 40, 0), ([900, 600], 3, 0), ([600, 515], 2, 6), ([255, 256], 7, 4)])
+def test_runs_of_one_string_are_resolved_on_their_next_four_symbols(torch_mod, repeats, followers, end):
+    """The first sort on codes resolves eight symbols: runs of one code of up to 256 suffixes take the second four in their tile, longer
+    ones are sorted by the code of them, and what they come apart into is resolved or, where it is long again, left to the doubling.
+    Against the oracle, generation sizes included."""
+    from cascade_amd import PartitionSorter
+    T = texts.text_with_repeated_strings(100000, repeats, followers, end, followers + end)
+    with PartitionSorter(T.size, key_words=1) as s:
+        print(f"  repeated strings {repeats} {followers} {end}", flush=True)
+        got = gpu_sa40(torch_mod, s, T)
+        stats = s.last_stats
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
+    assert (stats["big"][1] > 0) == (max(repeats) > 256)

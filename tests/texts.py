@@ -107,3 +107,24 @@ def text_of_shared_records(n, records, seed):
     kind = rng.integers(0, records, n // 4 + 1)
     T = np.stack([kind + 300, kind + 3000, kind + 6000, rng.integers(30000, 35000, kind.size)], axis=1)
     return T.reshape(-1)[:n].astype(np.uint16)
+
+
+def text_with_repeated_strings(n, repeats, followers, end, seed):
+    """n random token ids with four symbols planted r times for every r in `repeats`, each time followed by one of `followers` strings of
+    four symbols (two of which differ in their last one only): runs of one string that are told apart by the next four symbols, into
+    runs that are long again where r / followers is. `end`: the text ends in the planted string and as many zeros, which tie
+    with the padding of a string that runs off the text."""
+    rng = np.random.default_rng(seed)
+    T = rng.integers(300, 60000, n).astype(np.uint16)
+    slots = rng.permutation(n // 9 - 2)
+    at = 0
+    for i, r in enumerate(repeats):
+        for k in range(r):
+            p = 9 * int(slots[at])
+            at += 1
+            f = int(rng.integers(0, followers))
+            T[p:p + 8] = [i, i, i + 1, i, 7, 5, f // 2, f % 2]
+    if end:
+        T[-4 - end:] = 0
+        T[-4 - end:-end] = [0, 0, 1, 0]
+    return T
