@@ -3,6 +3,7 @@
 #include "../../include/cascade_hip.h"
 
 #include "coded_keys.hpp"
+#include "copies.hpp"
 #include "device_pool.hpp"
 #include "device_utils.hpp"
 #include "doubling.hpp"
@@ -333,6 +334,7 @@ struct csa_handle {
     u32 defer_min = DEFER_MIN; // lists at least this long use the bucketed rank update (csa_set_tuning)
     u32 window_min_changed = WINDOW_MIN_CHANGED; // csa_set_tuning (0xFFFFFFFF: never)
     u32 expect_presorted = 0; // csa_set_tuning: 1 = every generation first runs as if its large groups were in order already
+    u32 settle = 1;       // csa_set_tuning: 0 once a threshold of the rank updates has been set
     u32 pack_symbols = 1; // csa_set_tuning: texts over small alphabets start from keys of many symbols (packed_text.hpp)
     csa_step_result last_step = {};              // counters of the last partition step (csa_last_step_result)
     std::vector<hipEvent_t> events;
@@ -1047,6 +1049,7 @@ struct CodedList {
     u32 words;        // words of four symbols that its order and its ties stand for, at most 2
     u64 long_members; // suffixes in runs that were too long for their tile, sorted by their second word in ...
     int long_passes;  // ... so many radix passes
+    bool long_left;   // there are runs that are too long for a tile on both words
 };
 
 // Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their first `words` words of four symbols, with
@@ -1201,18 +1204,113 @@ int sort_long_runs(Launch& L, CodedList& list)
     a.m = (u32)count;
     hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true>), dim3((u32)((count + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, a);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(h->h_pinned + 4, h->counts + 4, sizeof(u32), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(h->h_pinned + 4, h->counts + 4, 2 * sizeof(u32), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     if (h->h_pinned[4] != 0)
         list.words = 1;
+    list.long_left = h->h_pinned[5] != 0;
+    return CSA_OK;
+}
+
+// Settles the ties of a list of short groups by where the copies they come from end (copies.hpp).
+struct Settle {
+    const u16* text;
+    u32* sa32;      // the sorted list, whose groups are put in order
+    u32 ctx, wide_ell; // symbols the groups are tied on; of the caller's key
+    bool settled;   // the list is in order, and the doubling would have gone through num generations more, of these sizes
+    u32 num;
+    u64 active[SETTLE_CONTEXTS], groups[SETTLE_CONTEXTS];
+};
+
+// Whether it is tried: a failed attempt costs the comparison of every member with its group's root, which is what a generation of the doubling
+// costs too. A list of copies has two or three members to a group; long groups are runs and periods, whose members agree with
+// their neighbours and not with their group's root, or short strings that are in the text a hundred times.
+constexpr u32 SETTLE_AVG_LIMIT = 4;
+
+// Works in key[2] (the anchors' records and bits: two bytes per suffix at most) and the symbol counts of the first sort.
+int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    SettleArgs a;
+    memset(&a, 0, sizeof(a));
+    a.text = st.text;
+    a.n = ra.n;
+    a.ctx = st.ctx;
+    a.log2_gap = (u32)bit_length(st.ctx) - 1u;
+    a.anchors = (a.n >> a.log2_gap) + 1u;
+    a.sufs = ra.sufs_out;
+    a.gids = ra.gids_out;
+    a.gstart = ra.gstart_out;
+    a.gprim = ra.gprim_out;
+    a.m = m;
+    a.groups = groups;
+    a.words[0] = (a.anchors + 63u) / 64u;
+    a.words[1] = (a.words[0] + 63u) / 64u;
+    a.words[2] = (a.words[1] + 63u) / 64u;
+    unsigned char* at = reinterpret_cast<unsigned char*>(h->key[2]);
+    unsigned char* const end = at + h->cap * sizeof(u64);
+    auto take = [&](u64 bytes) {
+        unsigned char* const p = at;
+        at += align256(bytes);
+        return p;
+    };
+    a.records = reinterpret_cast<u64*>(take(((u64)a.anchors + 1) * sizeof(u64)));
+    for (int i = 0; i < 3; ++i)
+        a.links[i] = reinterpret_cast<unsigned long long*>(take((u64)a.words[i] * sizeof(u64)));
+    if (at > end)
+        return CSA_OK; // (a handle of a few hundred suffixes)
+    a.sa32 = st.sa32;
+    u64 c = st.ctx;
+    do {
+        a.contexts[a.num_contexts++] = (u32)c;
+        c += c < st.wide_ell ? (c < st.wide_ell - c ? c : st.wide_ell - c) : c;
+    } while (c < a.n && a.num_contexts < SETTLE_CONTEXTS);
+    constexpr u32 TALLIES = 2 * (SETTLE_CONTEXTS + 1);
+    static_assert(SETTLE_SLOTS * TALLIES <= SYMBOLS && SETTLE_SLOTS * TALLIES <= MAX_PASSES * RADIX_BINS, "the tallies take the symbol counts' place, and the histograms' on the host");
+    a.tallies = code_tables(h).counts;
+    a.failed = h->counts + 4;
+    a.err = h->counts + 2;
+    HIP_TRY(hipMemsetAsync(a.failed, 0, sizeof(u32), s));
+    HIP_TRY(hipMemsetAsync(a.tallies, 0, SETTLE_SLOTS * TALLIES * sizeof(u32), s));
+    HIP_TRY(hipMemsetAsync(a.records, 0xFF, ((u64)a.anchors + 1) * sizeof(u64), s));
+    hipLaunchKernelGGL(copy_roots_kernel, dim3((u32)(((u64)m + 255) / 256)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(copy_links_kernel, dim3(a.words[1]), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL(copy_links_top_kernel, dim3((a.words[1] + 255u) / 256u), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(copy_spread_kernel, dim3((u32)(((u64)a.anchors + 255) / 256)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX>), dim3((u32)(((u64)m + SETTLE_TILE - 1) / SETTLE_TILE)), dim3(SETTLE_BLOCK), 0, s, a);
+    HIP_TRY(hipGetLastError());
+    u32* const h_tallies = h->h_pinned + PINNED_HIST;
+    HIP_TRY(hipMemcpyAsync(h_tallies, a.tallies, SETTLE_SLOTS * TALLIES * sizeof(u32), hipMemcpyDeviceToHost, s));
+    int rc = read_counts(L, nullptr);
+    if (rc || h->h_pinned[4] != 0)
+        return rc;
+    u64 members[SETTLE_CONTEXTS + 1] = {}, starts[SETTLE_CONTEXTS + 1] = {};
+    for (u32 slot = 0; slot < SETTLE_SLOTS; ++slot)
+        for (u32 i = 0; i <= SETTLE_CONTEXTS; ++i) {
+            members[i] += h_tallies[slot * TALLIES + i];
+            starts[i] += (u64)(int64_t)(int32_t)h_tallies[slot * TALLIES + SETTLE_CONTEXTS + 1 + i];
+        }
+    // a list on context i holds the members tied on more than i contexts, and the groups that start at or before it and have not ended
+    u64 above = 0;
+    for (int i = (int)a.num_contexts - 1; i >= 0; --i)
+        st.active[i] = above += members[i + 1];
+    u64 open = 0;
+    for (u32 i = 0; i < a.num_contexts; ++i)
+        st.groups[i] = open += starts[i];
+    st.num = 0;
+    while (st.num < a.num_contexts && st.active[st.num] > 0)
+        ++st.num;
+    st.settled = true;
     return CSA_OK;
 }
 
 // Generation 0: ranks the sorted list described by `ra`: counts per tile, scans the counts, reads the totals back, then
 // applies them and brings rank[] up to date, directly from the kernel or through the two-pass bucketed update.
-// coded: the list comes from sort_by_codes and carries its ties.
+// coded: the list comes from sort_by_codes and carries its ties. settle: the ties of a list of short groups are settled at once if possible; the
+// ranks are not needed then, nor are they when nothing is tied.
 int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivors, u32* groups, int* rank_update,
-                u32* level_counts = nullptr, CodedList* coded = nullptr, int* passes = nullptr)
+                u32* level_counts = nullptr, CodedList* coded = nullptr, int* passes = nullptr, Settle* settle = nullptr)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -1264,6 +1362,28 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
         }
         level_counts[2 * i] = (u32)sv;
         level_counts[2 * i + 1] = (u32)hd;
+    }
+    if (settle && *survivors == 0) {
+        *rank_update = 0;
+        return CSA_OK;
+    }
+    if (settle && (u64)*survivors <= (u64)*groups * SETTLE_AVG_LIMIT && !(coded && coded->long_left)) {
+        RerankArgs list = ra;
+        list.rank = nullptr;
+        if (coded)
+            hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS, true>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, list);
+        else
+            hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS, false>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, list);
+        HIP_TRY(hipGetLastError());
+        if (coded)
+            settle->ctx *= coded->words;
+        rc = settle_copies(L, *settle, ra, *survivors, *groups);
+        if (rc)
+            return rc;
+        if (settle->settled) {
+            *rank_update = 0;
+            return CSA_OK;
+        }
     }
     // what the list becomes decides what rank[] is to hold: ordinals for a dense generation, ranks otherwise
     ra.ordinals = dense_generation(*survivors, *groups, ra.n) ? 1u : 0u;
@@ -1418,7 +1538,14 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         ra.level_drop[i] = (ell - ra.level_ell[i]) * pp.codes.bits;
     }
     ra.ties = ties_of(h);
-    rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], level_counts, coded ? &list : nullptr, &passes);
+    Settle settle;
+    memset(&settle, 0, sizeof(settle));
+    settle.text = d_text;
+    settle.sa32 = sa32;
+    settle.ctx = ell;
+    settle.wide_ell = (u32)wide_ell;
+    rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], level_counts, coded ? &list : nullptr, &passes,
+                     h->pack_symbols && h->settle ? &settle : nullptr);
     range_gen0.close();
     if (rc)
         return rc;
@@ -1432,20 +1559,29 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     u64 ctx = ell; // symbols resolved so far; the next generation looks hop symbols ahead
     // A list that was resolved on two words leaves what generation 1 would: that one is reported with the lists it would have had, what
     // the members of its large groups took, and no time of its own.
-    int resolved = 0;
     if (coded && list.words == 2) {
         if (level_counts[0] > 0) {
             st->active[1] = level_counts[0];
             st->groups[1] = level_counts[1];
             st->big[1] = list.long_members;
             st->passes[1] = list.long_passes;
-            resolved = 1;
             gen = 2;
         }
         ctx = 2 * ell;
     } else if (coded) {
         st->passes[0] += list.long_passes;
     }
+    // Nor do the generations of a list whose ties have been settled.
+    if (settle.settled) {
+        if (gen + settle.num > CSA_MAX_GENERATIONS)
+            return fail(CSA_ERR_INTERNAL, "%u generations do not fit the statistics", gen + settle.num);
+        for (u32 i = 0; i < settle.num; ++i, ++gen) {
+            st->active[gen] = settle.active[i];
+            st->groups[gen] = settle.groups[i];
+        }
+        m = 0;
+    }
+    const int untimed = gen - 1; // generations 1 .. untimed
     HIP_TRY(hipEventRecord(h->ev_gen[gen], s));
     int gp = 0; // gprim[gp] / gstart[gp] describe the current groups
     bool all_small = false; // no group of the current list exceeds the limit of the generation that found it so
@@ -1743,9 +1879,9 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         return rc;
 
     for (int g = 0; g < gen; ++g) {
-        if (g >= 1 && g <= resolved)
+        if (g >= 1 && g <= untimed)
             continue;
-        HIP_TRY(hipEventElapsedTime(&st->ms[g], h->ev_gen[g], h->ev_gen[g == 0 ? resolved + 1 : g + 1]));
+        HIP_TRY(hipEventElapsedTime(&st->ms[g], h->ev_gen[g], h->ev_gen[g == 0 ? untimed + 1 : g + 1]));
     }
     HIP_TRY(hipEventElapsedTime(&st->ms_output, h->ev_gen[gen], h->ev_gen[gen + 1]));
     HIP_TRY(hipEventElapsedTime(&st->ms_total, h->ev_gen[0], h->ev_gen[gen + 1]));
@@ -2340,8 +2476,8 @@ int csa_set_tuning(csa_handle* h, int knob, uint32_t value)
     if (!h)
         return fail(CSA_ERR_ARG, "csa_set_tuning: null handle");
     switch (knob) {
-    case CSA_TUNE_DEFER_MIN: h->defer_min = value; break;
-    case CSA_TUNE_WINDOW_MIN_CHANGED: h->window_min_changed = value; break;
+    case CSA_TUNE_DEFER_MIN: h->defer_min = value, h->settle = 0; break;
+    case CSA_TUNE_WINDOW_MIN_CHANGED: h->window_min_changed = value, h->settle = 0; break;
     case CSA_TUNE_PACK_SYMBOLS: h->pack_symbols = value ? 1u : 0u; break;
     case CSA_TUNE_EXPECT_PRESORTED: h->expect_presorted = value ? 1u : 0u; break;
     case CSA_TUNE_XCD_CHUNK:

@@ -77,7 +77,7 @@ struct RerankArgs {
     u32 level_drop[4];
     u32 level_ell[4];
     unsigned long long* level_totals;
-    u32* rank; // [n] by text position
+    u32* rank; // [n] by text position; null (and no rank_recs): the list is compacted and nothing is ranked
     // Deferred rank update: instead of the scattered write rank[x] = r, the suffix at sorted index c leaves the record
     // (x << 32) | r at rank_recs[c] (a coalesced stream). The records then go through radix passes on the high bits of
     // x before they are written to rank[], so that those writes fall into one window of rank[] at a time.
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(BLOCK) void rerank_kernel(RerankArgs a)
             const u32 value = a.ordinals ? ordinal : nr;
             if (a.rank_recs)
                 rec[k] = ((u64)x << 32) | value;
-            else
+            else if (a.rank)
                 a.rank[x] = value;
             if (!single) {
                 if (ka) {

@@ -784,3 +784,30 @@ def test_runs_of_one_string_are_resolved_on_their_next_four_symbols(emu, repeats
         assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
         if pack and key_words == 1 and emu_sort.passes[0] == 4:  # (the probe may have sent the text to the K-grams)
             assert (big[1] > 0) == (max(repeats) > 64)
+
+
+@pytest.mark.parametrize("symbols,key_words", [(60000, 1), (60000, 3), (60000, 4), (256, 1), (4, 1), (4, 3), (2, 2)])
+def test_ties_of_copied_passages_are_settled_by_where_the_copies_end(emu, symbols, key_words):
+    """A list of short groups is put in order without ranks: every member is compared with its group's first one in the text, once for a whole
+    passage. Copies of copies, copies with changed symbols, copies over copies and up to the end of the text, from keys of codes (8
+    symbols apart at least) and of packed symbols (8 to 64). Suffix array and generation sizes are the oracle's; so they are
+    when the sort is told to double (a threshold of the rank updates set) and when every comparison runs into its limit."""
+    settled = 0
+    for seed in range(9):
+        T = texts.text_of_copies(1600 + 700 * seed, symbols, 10 * seed + symbols + key_words)
+        got, active, _ = emu_sort(emu, T, key_words)
+        sa, counts = oracle_lib.prefix_doubling(T, key_words)
+        assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts, seed
+        settled += len(active) > 1 and emu_sort.rank_update[0] == 0
+    assert settled >= 4
+
+
+@pytest.mark.parametrize("symbols,key_words", [(60000, 1), (4, 1), (60000, 4)])
+def test_copies_that_cannot_be_settled_are_left_to_the_doubling(symbols, key_words):
+    """A build in which every comparison of copies runs into its limit: the sort ranks its list and doubles from where it was."""
+    lib = load_emulation("libcascade_emu_rank.so")
+    T = texts.text_of_copies(5000, symbols, symbols + key_words)
+    got, active, _ = emu_sort(lib, T, key_words)
+    assert emu_sort.rank_update[0] == 1 and len(active) > 3
+    sa, counts = oracle_lib.prefix_doubling(T, key_words)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts

@@ -744,3 +744,31 @@ def test_runs_of_one_string_are_resolved_on_their_next_four_symbols(torch_mod, r
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
     assert (stats["big"][1] > 0) == (max(repeats) > 256)
+
+
+@pytest.mark.parametrize("symbols,key_words", [(60000, 1), (60000, 4), (256, 1), (4, 1), (4, 3)])
+def test_ties_of_copied_passages_are_settled_by_where_the_copies_end(torch_mod, symbols, key_words):
+    """Copies of copies, copies with changed symbols, copies over copies and up to the end of the text: ties are settled without ranks where
+    the list's groups are short, and by doubling where a threshold of the rank updates is set. Suffix array and generation sizes are
+    the oracle's either way; 2^22 symbols with copies of up to a million, where chains of anchors need both summaries, pass the
+    device verifier."""
+    from cascade_amd import PartitionSorter, _native
+    for seed in range(4):
+        T = texts.text_of_copies(20001 + 50000 * seed, symbols, 10 * seed + symbols + key_words)
+        sa, counts = oracle_lib.prefix_doubling(T, key_words)
+        for doubling in (False, True):
+            with PartitionSorter(T.size, key_words=key_words) as s:
+                if doubling:
+                    s.set_tuning(_native.CSA_TUNE_WINDOW_MIN_CHANGED, 1 << 22)
+                print(f"  copies {symbols} {key_words} {T.size} {doubling}", flush=True)
+                got = gpu_sa40(torch_mod, s, T)
+                assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and s.last_stats["active"] == counts, (seed, doubling)
+    T = texts.text_of_copies(1 << 22, symbols, symbols + key_words)
+    d = to_dev(torch_mod, T)
+    with PartitionSorter(T.size, key_words=key_words) as s:
+        out = s.sort(d)
+        settled = s.last_stats
+        assert s.verify(d, out)
+        s.set_tuning(_native.CSA_TUNE_WINDOW_MIN_CHANGED, 1 << 22)
+        assert torch_mod.equal(s.sort(d), out)
+        assert settled["active"] == s.last_stats["active"] and settled["groups"] == s.last_stats["groups"]

@@ -128,3 +128,25 @@ def text_with_repeated_strings(n, repeats, followers, end, seed):
         T[-4 - end:] = 0
         T[-4 - end:-end] = [0, 0, 1, 0]
     return T
+
+
+def text_of_copies(n, symbols, seed):
+    """n symbols below `symbols` into which passages are copied, several times over and over each other, some with a few symbols changed;
+    every third text ends in zeros, every third in a copy of its start."""
+    rng = np.random.default_rng(seed)
+    T = rng.integers(0, symbols, n).astype(np.uint16)
+    for _ in range(int(rng.integers(2, 12))):
+        length = int(rng.integers(4, n // 3))
+        src = int(rng.integers(0, n - length))
+        passage = T[src:src + length].copy()
+        for _ in range(int(rng.integers(1, 5))):
+            dst = int(rng.integers(0, n - length))
+            T[dst:dst + length] = passage
+            if rng.random() < 0.5:
+                at = dst + rng.integers(0, length, 3)
+                T[at] = rng.integers(0, symbols, 3)
+    if seed % 3 == 0:
+        T[-int(rng.integers(1, 20)):] = 0
+    elif seed % 3 == 1:
+        T[n - n // 5:] = T[:n // 5]
+    return T
