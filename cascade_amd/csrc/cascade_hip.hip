@@ -1371,7 +1371,7 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
         RerankArgs list = ra;
         list.rank = nullptr;
         if (coded)
-            hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS, true>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, list);
+            hipLaunchKernelGGL((compact_ties_kernel<RANK_TILE>), dim3((r.tiles + 3) / 4), dim3(256), 0, s, list, r.tiles);
         else
             hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS, false>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, list);
         HIP_TRY(hipGetLastError());

@@ -455,7 +455,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
             if (is_short ? (left ? l <= H : f >= H + RESOLVE_TILE) : j != H - 1)
                 continue;
         }
-        x[k] = a.sufs[e];
+        x[k] = a.sufs[e]; // (asked for before the runs are known, for all elements: no faster, 14.4 and 15.0 ms on 1e9 tokens)
         if (!KEYS && (x[k] & OWN_CODE))
             owners |= 1u << k;
         x[k] &= ~OWN_CODE;
@@ -671,7 +671,12 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_runs_kernel(ResolveArgs
         for (int k = 0; k < COLLECT_ITEMS; ++k)
             ties |= base + k < a.m ? (u32)a.ties[base + k] << (8 * k) : 0u;
     }
-    u32 flags = 0, mine = 0, heads = 0;
+    u32 flags = 0, mine = 0, heads = 0, x[COLLECT_ITEMS] = {};
+    if constexpr (APPLY) // (all loads of a thread before its first store: one after the other they took 2.7 ms for 57.7 M of 1e9 suffixes, 2.0 now)
+#pragma unroll
+        for (int k = 0; k < COLLECT_ITEMS; ++k)
+            if ((ties >> (8 * k)) & TIE_LONG)
+                x[k] = a.sufs_out[base + k];
 #pragma unroll
     for (int k = 0; k < COLLECT_ITEMS; ++k)
         if ((ties >> (8 * k)) & TIE_LONG) {
@@ -709,22 +714,33 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_runs_kernel(ResolveArgs
         }
         return;
     }
+    if (total == 0)
+        return;
+    u64 key[COLLECT_ITEMS];
+#pragma unroll
+    for (int k = 0; k < COLLECT_ITEMS; ++k) {
+        key[k] = 0;
+        if ((flags >> k) & 1u) {
+            if constexpr (MARKED) {
+                key[k] = load_kgram(a.text, a.n, x[k], 0);
+            } else {
+                const u64 y = (u64)x[k] + 4u; // (a suffix that has none there is a string of its own)
+                key[k] = y >= a.n ? 0u : a.text_codes[y + a.tail >= a.n ? a.n - 1 - y : y + a.tail];
+            }
+        }
+    }
     const SlabPrefix sp = slabs_before(a.slab_total, tile / a.slab);
     slot += a.tile_prefix[(u64)tile * 4 + 2] + sp.sum2;
     ordinal += a.tile_prefix[(u64)tile * 4 + 3] + sp.sum3; // strings begun before this thread's entries
 #pragma unroll
     for (int k = 0; k < COLLECT_ITEMS; ++k)
         if ((flags >> k) & 1u) {
-            const u32 x = a.sufs_out[base + k];
-            if constexpr (MARKED) {
-                a.run_keys[slot] = load_kgram(a.text, a.n, x, 0);
-            } else {
+            if constexpr (!MARKED) {
                 ordinal += ((ties >> (8 * k)) & TIE_WORDS) == 0 ? 1u : 0u;
-                const u64 y = (u64)x + 4u; // (a suffix that has none there is a string of its own)
-                const u32 next = y >= a.n ? 0u : a.text_codes[y + a.tail >= a.n ? a.n - 1 - y : y + a.tail];
-                a.run_keys[slot] = ((u64)(ordinal - 1u) << 32) | next;
+                key[k] |= (u64)(ordinal - 1u) << 32;
             }
-            a.members[slot] = x;
+            a.run_keys[slot] = key[k];
+            a.members[slot] = x[k];
             a.places[slot] = (u32)(base + k);
             ++slot;
         }

@@ -247,27 +247,24 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
     }
 }
 
-// The same for a list that carries its ties, at every number of words up to TIE_MOST_WORDS at once: one byte read per suffix. A wave takes
-// whole tiles, PER bytes a lane, and `per_wave` of them one after the other; the tile aggregates are those at a.words, the
-// survivors and groups at i + 1 words are added to level_totals[.. + 2 i] and [.. + 2 i + 1].
+// The ties of a tile of a list that carries them, for the wave that takes it: PER entries a lane. tie[i], bit k: element base + k shares
+// more than i words with its left neighbour; right[i], bit k: its right neighbour does with it; valid: the entries there are.
 template <int TILE>
-__global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles, u32 per_wave)
-{
-    constexpr int PER = TILE / WAVE;
+struct TileTies {
+    static constexpr int PER = TILE / WAVE;
     static_assert(PER % 16 == 0 && PER <= 32, "a lane's bytes come in 16-byte loads, their ties fit a word");
-    const u32 lane = threadIdx.x & 63u;
-    const u32 wave = blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
-    u32 sum_surv[TIE_MOST_WORDS] = {}, sum_heads[TIE_MOST_WORDS] = {};
-    for (u32 r = 0; r < per_wave; ++r) {
-        const u64 tile = (u64)wave * per_wave + r;
-        if (tile >= tiles)
-            break;
-        const u64 base = tile * TILE + (u64)lane * PER;
-        u32 tie[TIE_MOST_WORDS] = {}; // bit k: element base + k shares that many words with its left neighbour
-        if (base + PER <= a.m) {
+    u32 tie[TIE_MOST_WORDS], right[TIE_MOST_WORDS], valid;
+    __device__ __forceinline__ TileTies(const u8* __restrict__ ties, u32 m, u64 tile)
+    {
+        const u32 lane = threadIdx.x & 63u;
+        const u64 base = tile * TILE + (u64)lane * PER, behind = (tile + 1) * TILE;
+#pragma unroll
+        for (u32 i = 0; i < TIE_MOST_WORDS; ++i)
+            tie[i] = 0;
+        if (base + PER <= m) {
 #pragma unroll
             for (int q = 0; q < PER; q += 16) {
-                const uint4 v = *reinterpret_cast<const uint4*>(a.ties + base + q);
+                const uint4 v = *reinterpret_cast<const uint4*>(ties + base + q);
                 const u32 word[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
                 for (int k = 0; k < 16; ++k)
@@ -277,24 +274,44 @@ __global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles
             }
         } else {
             for (int k = 0; k < PER; ++k)
-                if (base + k < a.m)
+                if (base + k < m)
                     for (u32 i = 0; i < TIE_MOST_WORDS; ++i)
-                        tie[i] |= ((a.ties[base + k] & TIE_WORDS) > i ? 1u : 0u) << k;
+                        tie[i] |= ((ties[base + k] & TIE_WORDS) > i ? 1u : 0u) << k;
         }
-        const u64 behind = (tile + 1) * TILE;
-        const u32 after = behind < a.m ? a.ties[behind] & TIE_WORDS : 0u;
-        const u32 have = base >= a.m ? 0u : a.m - base >= PER ? PER : (u32)(a.m - base);
-        const u32 valid = have == 32u ? 0xFFFFFFFFu : (1u << have) - 1u;
+        const u32 after = behind < m ? ties[behind] & TIE_WORDS : 0u;
+        const u32 have = base >= m ? 0u : m - base >= PER ? PER : (u32)(m - base);
+        valid = have == 32u ? 0xFFFFFFFFu : (1u << have) - 1u;
 #pragma unroll
         for (u32 i = 0; i < TIE_MOST_WORDS; ++i) {
             const u64 firsts = __ballot(tie[i] & 1u);
             const u32 next = lane == 63u ? (after > i ? 1u : 0u) : (u32)(firsts >> (lane + 1)) & 1u;
-            const u32 right = (tie[i] >> 1) | (next << (PER - 1)); // bit k: element base + k + 1 ties with it
-            const u32 surv = (u32)__popc((tie[i] | right) & valid), heads = (u32)__popc(~tie[i] & right & valid);
+            right[i] = (tie[i] >> 1) | (next << (PER - 1));
+        }
+    }
+};
+
+// The same for a list that carries its ties, at every number of words up to TIE_MOST_WORDS at once: one byte read per suffix. A wave takes
+// whole tiles, `per_wave` of them one after the other; the tile aggregates are those at a.words, the
+// survivors and groups at i + 1 words are added to level_totals[.. + 2 i] and [.. + 2 i + 1].
+template <int TILE>
+__global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles, u32 per_wave)
+{
+    const u32 lane = threadIdx.x & 63u;
+    const u32 wave = blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
+    u32 sum_surv[TIE_MOST_WORDS] = {}, sum_heads[TIE_MOST_WORDS] = {};
+    for (u32 r = 0; r < per_wave; ++r) {
+        const u64 tile = (u64)wave * per_wave + r;
+        if (tile >= tiles)
+            break;
+        const TileTies<TILE> v(a.ties, a.m, tile);
+        const u64 base = tile * TILE + (u64)lane * TileTies<TILE>::PER;
+#pragma unroll
+        for (u32 i = 0; i < TIE_MOST_WORDS; ++i) {
+            const u32 surv = (u32)__popc((v.tie[i] | v.right[i]) & v.valid), heads = (u32)__popc(~v.tie[i] & v.right[i] & v.valid);
             sum_surv[i] += surv;
             sum_heads[i] += heads;
             if (i + 1 == a.words) {
-                const u32 begin = ~tie[i] & valid; // (1-based: 0 means no head in the tile)
+                const u32 begin = ~v.tie[i] & v.valid; // (1-based: 0 means no head in the tile)
                 const u32 last = begin ? (u32)base + 32u - (u32)__builtin_clz(begin) : 0u;
                 u32 most = last, packed = surv | (heads << 16);
 #pragma unroll
@@ -318,6 +335,48 @@ __global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles
             atomicAdd(slot, (unsigned long long)sv);
             atomicAdd(slot + 1, (unsigned long long)hd);
         }
+    }
+}
+
+// The active list alone, of a list that carries its ties and is not ranked (RerankArgs::rank null): its suffixes, groups and their
+// tables. A wave takes a tile and reads the suffixes of survivors only (1e9 tokens, 55.7 M of them tied: 2.2 ms when rerank_kernel did
+// it, 0.9 here).
+template <int TILE>
+__global__ __launch_bounds__(256) void compact_ties_kernel(RerankArgs a, u32 tiles)
+{
+    const u32 lane = threadIdx.x & 63u;
+    const u64 tile = (u64)blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
+    if (tile >= tiles)
+        return;
+    const TileTies<TILE> v(a.ties, a.m, tile);
+    const bool two = a.words == 2;
+    const u32 tie = two ? v.tie[1] : v.tie[0], right = two ? v.right[1] : v.right[0];
+    static_assert(TIE_MOST_WORDS == 2, "one word or two");
+    u32 surv = (tie | right) & v.valid;
+    const u32 heads = ~tie & right & v.valid;
+    const u32 mine = (u32)__popc(surv) | ((u32)__popc(heads) << 16); // at most TILE of each in all
+    const u32 incl = wave_incl_sum(mine), total = __shfl(incl, 63);
+    const bool last = (tile + 1) * TILE >= a.m;
+    if (total == 0 && !last)
+        return;
+    const SlabPrefix sp = slabs_before(a.slab_total, (u32)(tile / a.slab));
+    u32 at = a.tile_prefix[tile * 4 + 2] + sp.sum2, group = a.tile_prefix[tile * 4 + 3] + sp.sum3; // (group: groups begun so far)
+    if (last && lane == 0)
+        a.gstart_out[group + (total >> 16)] = at + (total & 0xFFFFu); // gstart[groups] = survivors
+    at += (incl - mine) & 0xFFFFu;
+    group += (incl - mine) >> 16;
+    const u64 base = tile * TILE + (u64)lane * TileTies<TILE>::PER;
+    while (surv) {
+        const u32 k = (u32)__builtin_ctz(surv);
+        surv &= surv - 1u;
+        if ((heads >> k) & 1u) {
+            a.gprim_out[group] = (u32)(base + k);
+            a.gstart_out[group] = at;
+            ++group;
+        }
+        a.sufs_out[at] = a.sufs[base + k];
+        a.gids_out[at] = group - 1u;
+        ++at;
     }
 }
 
