@@ -353,6 +353,31 @@ struct Launch {
     int events_used = 0;
 };
 
+void add_table(TableGroup& g, void* to, const void* from, u64 bytes)
+{
+    g.to[g.count] = static_cast<u32*>(to);
+    g.from[g.count] = static_cast<const u32*>(from);
+    g.words[g.count++] = (u32)(bytes / sizeof(u32));
+}
+
+// One launch for all of them: a workgroup for every 1024 words of the largest.
+int move_tables(const TableGroup& g, hipStream_t s)
+{
+    u32 most = 1;
+    for (u32 k = 0; k < g.count; ++k)
+        most = g.words[k] > most ? g.words[k] : most;
+    hipLaunchKernelGGL(move_tables_kernel, dim3((most + 1023u) / 1024u), dim3(256), 0, s, g);
+    HIP_TRY(hipGetLastError());
+    return CSA_OK;
+}
+
+int move_table(void* to, const void* from, u64 bytes, hipStream_t s)
+{
+    TableGroup g = {};
+    add_table(g, to, from, bytes);
+    return move_tables(g, s);
+}
+
 int next_ticket(Launch& L, u32** out)
 {
     csa_handle* h = L.h;
@@ -530,7 +555,9 @@ int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64
     const bool all_run = src == SRC_TEXT && !source->byte_wide;
     u32* h_hist = h->h_pinned + PINNED_HIST;
     if (!all_run) {
-        HIP_TRY(hipMemcpyAsync(h_hist, h->ghist, plan.num_passes * RADIX_BINS * sizeof(u32), hipMemcpyDeviceToHost, s));
+        const int rc = move_table(h_hist, h->ghist, plan.num_passes * RADIX_BINS * sizeof(u32), s);
+        if (rc)
+            return rc;
         HIP_TRY(hipStreamSynchronize(s));
     }
     bool run[MAX_PASSES];
@@ -635,11 +662,15 @@ int ensure_events(csa_handle* h, bool kernel_timing)
     return CSA_OK;
 }
 
-// counts: [2] device error flag, [3] verifier flag, [4] members of large groups. Waits for the stream.
-int read_counts(Launch& L, u32* big)
+// counts: [2] device error flag, [3] verifier flag, [4] members of large groups. Waits for the stream. `beside`: what else the host
+// wants to see by then.
+int read_counts(Launch& L, u32* big, TableGroup beside = {})
 {
     csa_handle* h = L.h;
-    HIP_TRY(hipMemcpyAsync(h->h_pinned, h->counts, 8 * sizeof(u32), hipMemcpyDeviceToHost, L.stream));
+    add_table(beside, h->h_pinned, h->counts, 8 * sizeof(u32));
+    const int rc = move_tables(beside, L.stream);
+    if (rc)
+        return rc;
     HIP_TRY(hipStreamSynchronize(L.stream));
     if (h->h_pinned[2]) {
         static const char* const what[] = {"", "a look-back wait ran into its spin limit",
@@ -828,7 +859,7 @@ RankTables rank_tables(csa_handle* h, u32 m)
 // decides the launches that follow) and chooses how the ranks are written: 0 scattered by the applying kernel,
 // 1 two-pass bucketed (generation 0 of large partitions), 2 one-pass bucketed (most of a later list changed).
 int rank_totals(Launch& L, const RankTables& r, bool gen0, u32 m, u32 n, bool expect_no_big, u32* survivors, u32* groups,
-                int* rank_update)
+                int* rank_update, TableGroup beside = {})
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -836,9 +867,9 @@ int rank_totals(Launch& L, const RankTables& r, bool gen0, u32 m, u32 n, bool ex
                        r.slab_total, r.tile_splits);
     HIP_TRY(hipGetLastError());
     u32* h_slabs = h->h_pinned + PINNED_HIST;
-    HIP_TRY(hipMemcpyAsync(h_slabs, r.slab_total, r.slabs * 5 * sizeof(u32), hipMemcpyDeviceToHost, s));
+    add_table(beside, h_slabs, r.slab_total, r.slabs * 5 * sizeof(u32));
     u32 big_seen = 0;
-    int rc = read_counts(L, &big_seen);
+    int rc = read_counts(L, &big_seen, beside);
     if (rc)
         return rc;
     if (expect_no_big && big_seen != 0) // groups only split; a large group after an all-small generation is a corrupt list
@@ -984,7 +1015,9 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
                        (u32)((sampled << weight_log2) + SYMBOLS), c.cum);
     if (n >= PROBE_MIN) {
         hipLaunchKernelGGL(probe_codes_kernel, dim3((a.taken + PROBE_BLOCK - 1) / PROBE_BLOCK), dim3(PROBE_BLOCK), 0, s, a);
-        HIP_TRY(hipMemcpyAsync(seen, a.counts, sizeof(ProbeCounts), hipMemcpyDeviceToHost, s));
+        const int rc = move_table(seen, a.counts, sizeof(ProbeCounts), s);
+        if (rc)
+            return rc;
         HIP_TRY(hipEventRecord(h->ev_gen[1], s)); // (recorded again when the generation ends)
     }
     HIP_TRY(hipGetLastError());
@@ -1129,7 +1162,9 @@ int count_long_runs(Launch& L, ResolveArgs& a, u64* members, u64* strings)
                        r.tile_splits);
     HIP_TRY(hipGetLastError());
     u32* h_slabs = h->h_pinned + PINNED_HIST;
-    HIP_TRY(hipMemcpyAsync(h_slabs, r.slab_total, r.slabs * 5 * sizeof(u32), hipMemcpyDeviceToHost, s));
+    const int rc = move_table(h_slabs, r.slab_total, r.slabs * 5 * sizeof(u32), s);
+    if (rc)
+        return rc;
     HIP_TRY(hipStreamSynchronize(s));
     *members = *strings = 0;
     for (u32 sl = 0; sl < r.slabs; ++sl) {
@@ -1204,7 +1239,9 @@ int sort_long_runs(Launch& L, CodedList& list)
     a.m = (u32)count;
     hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true>), dim3((u32)((count + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, a);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(h->h_pinned + 4, h->counts + 4, 2 * sizeof(u32), hipMemcpyDeviceToHost, s));
+    rc = move_table(h->h_pinned + 4, h->counts + 4, 2 * sizeof(u32), s);
+    if (rc)
+        return rc;
     HIP_TRY(hipStreamSynchronize(s));
     if (h->h_pinned[4] != 0)
         list.words = 1;
@@ -1271,8 +1308,12 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     a.tallies = code_tables(h).counts;
     a.failed = h->counts + 4;
     a.err = h->counts + 2;
-    HIP_TRY(hipMemsetAsync(a.failed, 0, sizeof(u32), s));
-    HIP_TRY(hipMemsetAsync(a.tallies, 0, SETTLE_SLOTS * TALLIES * sizeof(u32), s));
+    TableGroup zeros = {}, seen = {};
+    add_table(zeros, a.failed, nullptr, sizeof(u32));
+    add_table(zeros, a.tallies, nullptr, SETTLE_SLOTS * TALLIES * sizeof(u32));
+    int rc = move_tables(zeros, s);
+    if (rc)
+        return rc;
     HIP_TRY(hipMemsetAsync(a.records, 0xFF, ((u64)a.anchors + 1) * sizeof(u64), s));
     hipLaunchKernelGGL(copy_roots_kernel, dim3((u32)(((u64)m + 255) / 256)), dim3(256), 0, s, a);
     hipLaunchKernelGGL(copy_links_kernel, dim3(a.words[1]), dim3(1024), 0, s, a);
@@ -1281,8 +1322,8 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     hipLaunchKernelGGL((settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX>), dim3((u32)(((u64)m + SETTLE_TILE - 1) / SETTLE_TILE)), dim3(SETTLE_BLOCK), 0, s, a);
     HIP_TRY(hipGetLastError());
     u32* const h_tallies = h->h_pinned + PINNED_HIST;
-    HIP_TRY(hipMemcpyAsync(h_tallies, a.tallies, SETTLE_SLOTS * TALLIES * sizeof(u32), hipMemcpyDeviceToHost, s));
-    int rc = read_counts(L, nullptr);
+    add_table(seen, h_tallies, a.tallies, SETTLE_SLOTS * TALLIES * sizeof(u32));
+    rc = read_counts(L, nullptr, seen);
     if (rc || h->h_pinned[4] != 0)
         return rc;
     u64 members[SETTLE_CONTEXTS + 1] = {}, starts[SETTLE_CONTEXTS + 1] = {};
@@ -1329,6 +1370,7 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
         const bool levels = ra.levels > 0 || coded;
         if (levels)
             HIP_TRY(hipMemsetAsync(ra.level_totals, 0, LEVEL_SLOTS * 8 * sizeof(unsigned long long), s));
+        TableGroup beside = {};
         if (coded) {
             ra.words = coded->words;
             // (several tiles a wave on long lists: fewer additions to the level totals)
@@ -1338,8 +1380,8 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
             hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
         }
         if (levels)
-            HIP_TRY(hipMemcpyAsync(h_levels, ra.level_totals, LEVEL_SLOTS * 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-        return rank_totals(L, r, true, ra.m, ra.n, false, survivors, groups, rank_update);
+            add_table(beside, h_levels, ra.level_totals, LEVEL_SLOTS * 8 * sizeof(unsigned long long));
+        return rank_totals(L, r, true, ra.m, ra.n, false, survivors, groups, rank_update, beside);
     };
     int rc = count_and_read();
     if (rc)
@@ -1415,7 +1457,6 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     const u64 wide_ell = 4ull * (u64)h->key_words;
 
     RangeScope range_sort("sort_partition n=%u", n);
-    HIP_TRY(hipMemsetAsync(h->counts, 0, 6 * sizeof(u32), s));
     HIP_TRY(hipEventRecord(h->ev_gen[0], s));
 
     // ---- generation 0: every suffix sorted by its first symbols (four of them, by codes or K-gram keys, or as many as a packed
@@ -1423,7 +1464,12 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     RangeScope range_gen0("generation 0 m=%u", n);
     // The byte histograms of the text come first: they tell whether the alphabet is small enough for keys of more than four
     // symbols. (The digit counts are zeroed with them.)
-    HIP_TRY(hipMemsetAsync(h->ghist, 0, (MAX_PASSES + 2) * RADIX_BINS * sizeof(u32), s));
+    TableGroup zeros = {};
+    add_table(zeros, h->counts, nullptr, 6 * sizeof(u32));
+    add_table(zeros, h->ghist, nullptr, (MAX_PASSES + 2) * RADIX_BINS * sizeof(u32));
+    int rc = move_tables(zeros, s);
+    if (rc)
+        return rc;
     u32* const bytehist = h->ghist + MAX_PASSES * RADIX_BINS;
     PackedPlan pp;
     memset(&pp, 0, sizeof(pp));
@@ -1433,7 +1479,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     if (h->pack_symbols) {
         count_bytes();
         u32* h_bytes = h->h_pinned + PINNED_HIST;
-        HIP_TRY(hipMemcpyAsync(h_bytes, bytehist, 2 * RADIX_BINS * sizeof(u32), hipMemcpyDeviceToHost, s));
+        if ((rc = move_table(h_bytes, bytehist, 2 * RADIX_BINS * sizeof(u32), s)) != CSA_OK)
+            return rc;
         HIP_TRY(hipStreamSynchronize(s));
         pp = plan_packed_text(h_bytes, n, h->key_words, (u64)h->cap * sizeof(u32));
     }
@@ -1442,7 +1489,6 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     for (u64 c = ell; c < wide_ell; c += (c < wide_ell - c ? c : wide_ell - c))
         ++folded;
     const u32 tail = n < ell ? n : ell;
-    int rc;
     bool coded = !pp.enabled && !pp.byte_wide;
     if (coded) {
         const bool probed = n >= PROBE_MIN, ahead = !probed || n < CODE_AHEAD_MAX;
@@ -1695,8 +1741,11 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         if (all_small) {
             // Groups only ever split: once a generation had no large group, none can appear again. The small-group
             // kernel then also counts for the apply step, and nothing else runs before it.
-            HIP_TRY(hipMemsetAsync(r.tile_agg, 0, (u64)r.tiles * 4 * sizeof(u32), s));
-            HIP_TRY(hipMemsetAsync(r.tile_splits, 0, (u64)r.tiles * sizeof(u32), s));
+            TableGroup cleared = {};
+            add_table(cleared, r.tile_agg, nullptr, (u64)r.tiles * 4 * sizeof(u32));
+            add_table(cleared, r.tile_splits, nullptr, (u64)r.tiles * sizeof(u32));
+            if ((rc = move_tables(cleared, s)) != CSA_OK)
+                return rc;
             if (high_limit)
                 hipLaunchKernelGGL((smallsort_kernel<SMALL_BLOCK, SMALL_ITEMS, SMALL_MAXG_HI, true>), dim3(r.tiles), dim3(SMALL_BLOCK), 0,
                                    s, sa);
@@ -1706,7 +1755,6 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             HIP_TRY(hipGetLastError());
             st->small_only[gen] = 1;
         } else {
-            HIP_TRY(hipMemsetAsync(h->counts + 4, 0, 2 * sizeof(u32), s));
             // marks of the large groups whose gathered ranks are out of order, in the tables the next generation's groups
             // will be written to (free until the apply step)
             sa.big_sec = bx[1];
@@ -1715,8 +1763,12 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             high_limit = (u64)m_in <= (u64)groups * SMALL_AVG_LIMIT;
             const u32 maxg = high_limit ? (u32)SMALL_MAXG_HI : (u32)SMALL_MAXG;
             const u32 marks = m_in / maxg + 2u; // one mark index per large group at most
-            HIP_TRY(hipMemsetAsync(sa.not_asc, 0, (u64)marks * sizeof(u32), s));
-            HIP_TRY(hipMemsetAsync(sa.not_desc, 0, (u64)marks * sizeof(u32), s));
+            TableGroup cleared = {};
+            add_table(cleared, h->counts + 4, nullptr, 2 * sizeof(u32));
+            add_table(cleared, sa.not_asc, nullptr, (u64)marks * sizeof(u32));
+            add_table(cleared, sa.not_desc, nullptr, (u64)marks * sizeof(u32));
+            if ((rc = move_tables(cleared, s)) != CSA_OK)
+                return rc;
             {
                 // where every large group's members start in the list of large-group members, and how many there are
                 // (counts[4]): a prefix sum over the group table

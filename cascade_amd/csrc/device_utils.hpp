@@ -188,6 +188,29 @@ __device__ __forceinline__ u32 lb2_wait_exclusive(u64* tile_chain, u64* group_ch
     return gexcl + within;
 }
 
+// ---- small tables to host memory, and to zero ----
+
+// A few device tables and where each goes. The host mirror is pinned memory that the device writes: one launch and its
+// 4 us take the place of a copy per table, which costs 10 us of the stream each however few bytes it has.
+constexpr int TABLE_GROUP = 4;
+struct TableGroup {
+    u32 count;
+    u32* to[TABLE_GROUP];
+    const u32* from[TABLE_GROUP]; // null: the table is set to zero
+    u32 words[TABLE_GROUP];
+};
+
+__global__ __launch_bounds__(256) void move_tables_kernel(TableGroup g)
+{
+    const u32 first = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
+    for (u32 k = 0; k < g.count; ++k) {
+        u32* const to = g.to[k];
+        const u32* const from = g.from[k];
+        for (u32 i = first; i < g.words[k]; i += stride)
+            to[i] = from ? from[i] : 0u;
+    }
+}
+
 // ---- wave-wide reduction ----
 
 __device__ __forceinline__ u32 wave_reduce_sum(u32 v)

@@ -149,7 +149,12 @@ int finish_partition_step(Launch& L, const char* who, StepColumns& c, const Tail
     ra.unserved_out = reinterpret_cast<unsigned long long*>(h->counts + 10);
     ra.pills_out = reinterpret_cast<unsigned long long*>(h->counts + 12);
     ra.incoherent_out = h->counts + 14;
-    HIP_TRY(hipMemsetAsync(h->counts + 8, 0, 8 * sizeof(u32), s));
+    TableGroup zeros = {};
+    add_table(zeros, h->counts + 8, nullptr, 8 * sizeof(u32));
+    add_table(zeros, c.msg_off, nullptr, ((u64)p + 1) * sizeof(u32));
+    int rc = move_tables(zeros, s);
+    if (rc)
+        return rc;
     hipLaunchKernelGGL((step_rank_kernel<GEN0, false>), dim3(r.tiles), dim3(STEP_BLOCK), 0, s, ra);
     hipLaunchKernelGGL(rerank_scan_kernel, dim3(r.slabs), dim3(1024), 0, s, r.tile_agg, r.tile_prefix, r.tiles, r.slab, r.slab_total,
                        r.tile_splits);
@@ -162,10 +167,9 @@ int finish_partition_step(Launch& L, const char* who, StepColumns& c, const Tail
     if (!c.msg_rank)
         c.msg_rank = tp.msg_rank;
     MessageArgs ma;
-    int rc = fill_message_args(ma, who, tp.words_r, tp.key_r, tp.beta_r, m, ctx, GEN0 ? 0 : 1, p);
+    rc = fill_message_args(ma, who, tp.words_r, tp.key_r, tp.beta_r, m, ctx, GEN0 ? 0 : 1, p);
     if (rc)
         return rc;
-    HIP_TRY(hipMemsetAsync(c.msg_off, 0, ((u64)p + 1) * sizeof(u32), s));
     ma.msg_off = c.msg_off;
     const u32 grid = ma.tiles < 4096u ? ma.tiles : 4096u;
     hipLaunchKernelGGL(count_messages_kernel, dim3(grid), dim3(MSG_BLOCK), 0, s, ma);
@@ -187,9 +191,10 @@ int finish_partition_step(Launch& L, const char* who, StepColumns& c, const Tail
     hipLaunchKernelGGL(narrow_and_pack_kernel, dim3((u32)((m + 255) / 256)), dim3(256), 0, s, (const u64*)tp.key_r, (const u64*)tp.words_r, m,
                        GEN0 ? 0 : 1, c.rank_out, c.suf40_out);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(h->h_pinned + 8, h->counts + 8, 8 * sizeof(u32), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(h->h_pinned + 16, c.msg_off + (p - 1), sizeof(u32), hipMemcpyDeviceToHost, s));
-    rc = read_counts(L, nullptr);
+    TableGroup seen = {};
+    add_table(seen, h->h_pinned + 8, h->counts + 8, 8 * sizeof(u32));
+    add_table(seen, h->h_pinned + 16, c.msg_off + (p - 1), sizeof(u32));
+    rc = read_counts(L, nullptr, seen);
     if (rc)
         return rc;
     const u32* hp = h->h_pinned;
