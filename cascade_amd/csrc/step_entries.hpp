@@ -20,8 +20,9 @@
 //   [ 0, 5) outbox targets, [ 5, 9) outbox ranks, [ 9,13) ranks out, [40,45) lanes out
 // Generation 0, keys of W = 2..4 words (65 bytes per suffix for W = 2, 8 W + 52 = 76 / 84 for W = 3 / 4):
 //   [ 0,24) K0 K1 P0 P1 as above (the sort on word 0)
-//   [24,28) places of the tied, [28,36) [36,40) second key array and permutation of the tied suffixes' sort
-//           (their first ones are the spare K and the spare P)
+//   [28,29) bits of the members of long runs
+//   [24,28) their places, [28,36) [36,40) second key array and permutation of their sort
+//           (the first ones are the spare K and the spare P)
 //   [40,45) lanes in, [45,49) routing tags in, [ik, ik + 8 W) keys in, ik = 49 (W = 2) or 52
 //   sorted word 1 -> the spare K; [24,40) carried records; [40,48) sorted suffix words; sorted tags -> the spare P
 //   [24,32) ranked keys, [32,40) ranked suffix words; ranked tags -> the permutation's place (W = 2: the ranking reads
@@ -269,10 +270,11 @@ int step_init(Launch& L, const char* who, StepColumns& c, const StepPlan& pl, in
     } else {
         // Wider keys: the same order, (key words, forward tag), reached from the most significant word. All suffixes are
         // sorted by word 0 alone. Only those that tie with a neighbour on it can still change places, and only inside their
-        // run: they are taken out in order, sorted among themselves by (word 0, ..., word W - 1, tag) with the stable LSD
-        // passes of the reference (tag, then the words from the last, src/GPU_SACA.cu:1165-1227) and put back, in that
-        // order, at the places the tied entries held. Sorting every suffix on every word costs 2 + 8 W passes over the
-        // partition; this costs 8, plus 2 + 8 W over the tied ones.
+        // run: order_runs_kernel puts runs of up to ORDER_MAX of them in order where they stand. The members of longer runs are
+        // taken out in order, sorted among themselves by (word 0, ..., word W - 1, tag) with the stable LSD passes of the
+        // reference (tag, then the words from the last, src/GPU_SACA.cu:1165-1227) and put back, in that order, at the
+        // places they held. Sorting every suffix on every word costs 2 + 8 W passes over the partition; this costs 8, plus
+        // 2 + 8 W over the members of long runs.
         hipLaunchKernelGGL(iota_kernel, dim3(blocks), dim3(256), 0, s, P[pc], m);
         hipLaunchKernelGGL(gather_u64_kernel, dim3(blocks), dim3(256), 0, s, c.keys, (const u32*)P[pc], m, (u32)key_words, 0u, K[0]);
         rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], P[pc], K[1], P[pc ^ 1], (u32)m, make_plan(0, 64), &in_out, &passes);
@@ -280,32 +282,56 @@ int step_init(Launch& L, const char* who, StepColumns& c, const StepPlan& pl, in
             return rc;
         kc = in_out;
         pc ^= in_out;
-        const RankTables r = rank_tables<STEP_TILE>(h, (u32)m);
-        u32* tied_pos = pl.at<u32>(24);
-        TieArgs ta;
-        ta.keys = K[kc];
-        ta.perm = P[pc];
-        ta.m = m;
-        ta.pos_out = tied_pos;
-        ta.perm_out = P[pc ^ 1]; // the spare permutation array takes the tied suffixes
-        ta.tile_agg = r.tile_agg;
-        ta.tile_splits = r.tile_splits;
-        ta.tile_prefix = r.tile_prefix;
-        ta.slab_total = r.slab_total;
-        ta.slab = r.slab;
-        ta.slabs = r.slabs;
-        ta.total_out = reinterpret_cast<unsigned long long*>(h->counts + 6);
-        hipLaunchKernelGGL((tie_kernel<false>), dim3(r.tiles), dim3(STEP_BLOCK), 0, s, ta);
-        hipLaunchKernelGGL(rerank_scan_kernel, dim3(r.slabs), dim3(1024), 0, s, r.tile_agg, r.tile_prefix, r.tiles, r.slab, r.slab_total,
-                           r.tile_splits);
-        hipLaunchKernelGGL((tie_kernel<true>), dim3(r.tiles), dim3(STEP_BLOCK), 0, s, ta);
+        OrderRunsArgs oa;
+        oa.first_words = K[kc];
+        oa.m = m;
+        oa.perm = P[pc];
+        oa.keys = c.keys;
+        oa.beta = c.beta;
+        oa.long_bits = pl.at<unsigned long long>(28); // (free until the long runs are sorted, which starts after the last read of them)
+        oa.any_long = h->counts + 4;
+        const u32 order_tiles = (u32)((m + ORDER_TILE - 1) / ORDER_TILE);
+        if (key_words == 2)
+            hipLaunchKernelGGL((order_runs_kernel<2>), dim3(order_tiles), dim3(ORDER_BLOCK), 0, s, oa);
+        else if (key_words == 3)
+            hipLaunchKernelGGL((order_runs_kernel<3>), dim3(order_tiles), dim3(ORDER_BLOCK), 0, s, oa);
+        else
+            hipLaunchKernelGGL((order_runs_kernel<4>), dim3(order_tiles), dim3(ORDER_BLOCK), 0, s, oa);
         HIP_TRY(hipGetLastError());
-        rc = read_counts(L, nullptr);
+        u32 any_long = 0;
+        rc = read_counts(L, &any_long);
         if (rc)
             return rc;
-        const u64 tied = h->h_pinned[6];
-        if (tied > m)
-            return fail(CSA_ERR_INTERNAL, "%s: %llu of %llu suffixes counted as tied", who, (unsigned long long)tied, (unsigned long long)m);
+        u64 tied = 0;
+        u32* tied_pos = pl.at<u32>(24);
+        if (any_long) {
+            const RankTables r = rank_tables<STEP_TILE>(h, (u32)m);
+            TieArgs ta;
+            ta.bits = oa.long_bits;
+            ta.perm = P[pc];
+            ta.m = m;
+            ta.pos_out = tied_pos;
+            ta.perm_out = P[pc ^ 1]; // the spare permutation array takes the members
+            ta.tile_agg = r.tile_agg;
+            ta.tile_splits = r.tile_splits;
+            ta.tile_prefix = r.tile_prefix;
+            ta.slab_total = r.slab_total;
+            ta.slab = r.slab;
+            ta.slabs = r.slabs;
+            ta.total_out = reinterpret_cast<unsigned long long*>(h->counts + 6);
+            hipLaunchKernelGGL((tie_kernel<false>), dim3(r.tiles), dim3(STEP_BLOCK), 0, s, ta);
+            hipLaunchKernelGGL(rerank_scan_kernel, dim3(r.slabs), dim3(1024), 0, s, r.tile_agg, r.tile_prefix, r.tiles, r.slab, r.slab_total,
+                               r.tile_splits);
+            hipLaunchKernelGGL((tie_kernel<true>), dim3(r.tiles), dim3(STEP_BLOCK), 0, s, ta);
+            HIP_TRY(hipGetLastError());
+            rc = read_counts(L, nullptr);
+            if (rc)
+                return rc;
+            tied = h->h_pinned[6];
+            if (tied > m)
+                return fail(CSA_ERR_INTERNAL, "%s: %llu of %llu suffixes counted as members of long runs", who, (unsigned long long)tied,
+                            (unsigned long long)m);
+        }
         if (tied > 0) {
             const u32 tblocks = (u32)((tied + 255) / 256);
             u64* SK[2] = {K[kc ^ 1], pl.at<u64>(28)}; // the sorted word 0 stays in K[kc]

@@ -425,6 +425,14 @@ class HostArray:
         self.ptr = a.ctypes.data
 
 
+@pytest.mark.parametrize("key_words,long_runs", [(1, True), (2, False), (2, True), (3, True), (4, False), (4, True)])
+def test_emulated_runs_of_one_first_word_in_order(emu, key_words, long_runs):
+    """The first partition step with wide keys: runs of one first word, short ones sorted where they stand and long ones taken out."""
+    import message_cases
+    message_cases.check_runs_of_first_words(emu, lambda a: HostArray(np.array(a, copy=True)), lambda d: d.a.copy(),
+                                            steps_handle(emu, key_words), key_words, long_runs)
+
+
 @pytest.mark.parametrize("packed,ctx,n,p", [(False, 4, 3000, 5), (True, 8, 3000, 300), (True, 64, 1500, 2049)])
 def test_emulated_message_kernels_match_the_oracle(emu, packed, ctx, n, p):
     import test_gpu_messages

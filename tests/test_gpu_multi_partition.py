@@ -207,6 +207,15 @@ def test_the_references_own_predictor_gives_the_cohorts_and_pill_receipts_of_the
     assert len(ours["cohorts"]) >= 10 and sum(ours["pill_receipts"]) > 0
 
 
+@pytest.mark.parametrize("key_words,long_runs", [(1, True), (2, False), (2, True), (3, True), (4, False), (4, True)])
+def test_runs_of_one_first_word_in_order(gpu, key_words, long_runs):
+    """csa_sort_init_dev with runs of one first word at the edges of what is sorted in place, against a sort of whole keys."""
+    import message_cases
+    lib, to_dev, to_host = gpu
+    print(f"  runs of one first word: key_words={key_words} long_runs={long_runs}", flush=True)
+    message_cases.check_runs_of_first_words(lib, to_dev, to_host, steps_handle(lib, key_words), key_words, long_runs)
+
+
 def test_random_pipelines_through_the_step_entries(gpu):
     """Random texts (tiny alphabets, long repeats, zero tails), 1 to 200 partitions, all four key widths: every step
     passes the reference's validators inside the harness and the suffix array is the oracle's."""
