@@ -626,8 +626,10 @@ def main():
 
     # dominant kernel: the one-sweep radix pass, timed per launch with HIP events on the sort's stream
     avg_launch_ms = radix_ms / radix_launches if radix_launches else 0.0
-    # a first sort on packed symbols resolves 8 or more; one on K-gram keys, which none of these workloads takes, makes 8 passes
-    coded_pairs = CODED_PASSES * n * args.steps if st["key_symbols"] == 4 and st["passes"][0] != 8 else 0
+    # a first sort on packed symbols resolves 8 or more; one on K-gram keys, which none of these workloads takes, makes 8 passes, and so
+    # does one on 64-bit packed keys (32 letters on narrow keys: four, as codes, unless long runs were sorted again)
+    coded = st["passes"][0] != 8 if st["key_symbols"] == 4 else st["key_symbols"] == 32 and st["passes"][0] == 4
+    coded_pairs = CODED_PASSES * n * args.steps if coded else 0
     radix_bytes = RADIX_PASS_BYTES_PER_PAIR * (radix_pairs - coded_pairs) + CODED_PASS_BYTES_PER_PAIR * coded_pairs
     achieved = radix_bytes / (radix_ms * 1e-3) / 1e9 if radix_ms > 0 else 0.0
     pairs_per_launch = radix_pairs / radix_launches if radix_launches else 0

@@ -1024,6 +1024,45 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
     return CSA_OK;
 }
 
+// Texts of two-bit symbols from this length on may start from narrow keys. (They gain at every length measured: 2^25 + 5 independent letters
+// 2.0 -> 1.2 ms, 4 * 10^8, a fifth of them copies, 28.4 -> 21.4. Up to 2^24 the first sort keeps the eight passes that its statistics
+// have always shown.)
+#ifndef CSA_NARROW_MIN
+#define CSA_NARROW_MIN ((1u << 24) + 1)
+#endif
+
+// Whether the first sort of a packed text takes narrow keys, 32 bits of the code stream, and reads the next 32 for the suffixes that tie
+// on them (sort_by_codes): four passes over 8-byte pairs instead of eight over 12-byte ones save 27 ps a suffix, less 8 for the second half; a member of a
+// run that is too long for a tile costs 100 (it is collected and sorted again), and a sample of the suffixes shows how many there are.
+int narrow_keys_pay(Launch& L, const TextSource& ps, u32 n, bool* pay)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    const CodeTables c = code_tables(h);
+    ProbeCounts* const seen = reinterpret_cast<ProbeCounts*>(h->h_pinned + PINNED_HIST);
+    ProbeArgs a;
+    memset(&a, 0, sizeof(a));
+    a.n = n;
+    a.taken = probed_suffixes(n);
+    a.table = reinterpret_cast<unsigned long long*>(h->key[0]); // (nothing there yet)
+    a.table_log2 = (u32)bit_length((u64)a.taken - 1) + 1;
+    const u32 long_run = RESOLVE_MAX / (n / a.taken);
+    a.long_from = long_run > 2 ? long_run : 2;
+    a.counts = c.probe;
+    a.stream = ps.stream;
+    a.sym_bits = ps.sym_bits;
+    HIP_TRY(hipMemsetAsync(a.table, 0, sizeof(u64) << a.table_log2, s));
+    int rc = move_table(c.probe, nullptr, sizeof(ProbeCounts), s);
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(probe_codes_kernel, dim3((a.taken + PROBE_BLOCK - 1) / PROBE_BLOCK), dim3(PROBE_BLOCK), 0, s, a);
+    if ((rc = move_table(seen, c.probe, sizeof(ProbeCounts), s)) != CSA_OK)
+        return rc;
+    HIP_TRY(hipStreamSynchronize(s));
+    *pay = (u64)seen->crowded * 6 <= a.taken;
+    return CSA_OK;
+}
+
 // Whether a text is sorted by codes or by K-gram keys. Codes save passes, and lose time to suffixes that share one with others and
 // have to be told apart by the text. Both per suffix in picoseconds, from generation 0 of texts of 2^19 to 2^28 symbols on either kind of key:
 // independent symbols are 15 to 23 faster on codes, short texts by 25 us for the launches and a round trip alone; a line of the
@@ -1088,7 +1127,8 @@ struct CodedList {
 // Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their first `words` words of four symbols, with
 // their ties beside them; code_suffixes ran before. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into
 // idx[1]; the codes live in the halves of key[0]. What long runs leave open is finished by sort_marked_runs and sort_long_runs.
-int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, CodedList& list)
+// packed: the codes are narrow keys, cut from its stream, of word_syms symbols (and so are the words).
+int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, CodedList& list, const TextSource* packed = nullptr, u32 word_syms = 4)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -1105,6 +1145,12 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
         a.text_n = n;
         a.tail = tail;
         a.own = own_of(h);
+        if (packed) {
+            a.stream = packed->stream;
+            a.stream_words = packed->words;
+            a.sym_bits = packed->sym_bits;
+            a.key_bits = 32;
+        }
         a.shift = 8 * p;
         a.bits = 8;
         a.digit_base = h->digit_base + p * RADIX_BINS;
@@ -1116,7 +1162,9 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
         if (rc)
             return rc;
         rc = launch_pass(L, n, [&] {
-            if (p == 0)
+            if (p == 0 && packed)
+                launch_onesweep32<SRC_PACKED>(h, a, s);
+            else if (p == 0)
                 launch_onesweep32<SRC_CODED>(h, a, s);
             else
                 launch_onesweep32<SRC_PAIRS>(h, a, s);
@@ -1133,6 +1181,11 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
     r.text = d_text;
     r.n = n;
     r.words = words;
+    r.word_syms = word_syms;
+    if (packed) {
+        r.stream = packed->stream;
+        r.sym_bits = packed->sym_bits;
+    }
     r.sufs_out = h->idx[1];
     r.ties = ties_of(h);
     r.marks = code_tables(h).marks;
@@ -1140,7 +1193,11 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
     r.any_long = h->counts + 5;
     r.text_codes = codes_of(h);
     r.tail = tail;
-    hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false>), dim3((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, r);
+    const dim3 resolve_grid((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE));
+    if (packed)
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, true>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, r);
+    else
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, false>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, r);
     HIP_TRY(hipGetLastError());
     return CSA_OK;
 }
@@ -1237,7 +1294,11 @@ int sort_long_runs(Launch& L, CodedList& list)
     a.keys = K[in_out];
     a.sufs = V[in_out];
     a.m = (u32)count;
-    hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true>), dim3((u32)((count + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, a);
+    const dim3 resolve_grid((u32)((count + RESOLVE_TILE - 1) / RESOLVE_TILE));
+    if (a.stream)
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true, true>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, a);
+    else
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true, false>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, a);
     HIP_TRY(hipGetLastError());
     rc = move_table(h->h_pinned + 4, h->counts + 4, 2 * sizeof(u32), s);
     if (rc)
@@ -1376,6 +1437,8 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
             // (several tiles a wave on long lists: fewer additions to the level totals)
             const u32 per_wave = r.tiles >= (1u << 15) ? 8u : 1u, waves = (r.tiles + per_wave - 1) / per_wave;
             hipLaunchKernelGGL((count_ties_kernel<RANK_TILE>), dim3((waves + 3) / 4), dim3(256), 0, s, ra, r.tiles, per_wave);
+            if (ra.levels > 0)
+                hipLaunchKernelGGL(count_code_levels_kernel, dim3(hist_blocks(256 * 16, ra.m)), dim3(256), 0, s, ra, coded->args.codes, ra.levels);
         } else {
             hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, ra);
         }
@@ -1395,7 +1458,7 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
         if ((unordered || second) && (rc = count_and_read()) != CSA_OK)
             return rc;
     }
-    const u32 levels = coded ? coded->words - 1 : ra.levels;
+    const u32 levels = ra.levels + (coded ? coded->words - 1 : 0);
     for (u32 i = 0; i < levels && level_counts; ++i) {
         u64 sv = 0, hd = 0;
         for (u32 slot = 0; slot < LEVEL_SLOTS; ++slot) {
@@ -1484,7 +1547,26 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         HIP_TRY(hipStreamSynchronize(s));
         pp = plan_packed_text(h_bytes, n, h->key_words, (u64)h->cap * sizeof(u32));
     }
-    const u32 ell = pp.enabled ? pp.codes.key_syms : 4u; // symbols the first sort resolves
+    TextSource ps;
+    memset(&ps, 0, sizeof(ps));
+    bool narrow = false; // keys of half as many packed symbols
+    if (pp.enabled) {
+        // the code stream lives in rank[], which nothing uses before the sorted list is ranked
+        u32* const stream = h->rank;
+        ps.stream = stream;
+        ps.sym_bits = pp.codes.bits;
+        ps.key_bits = pp.codes.key_syms * pp.codes.bits;
+        ps.words = ((u64)n * ps.sym_bits + 31) / 32 + 4;
+        if ((rc = move_table(bytehist, nullptr, RADIX_BINS * sizeof(u32), s)) != CSA_OK) // (read back already)
+            return rc;
+        const u64 enc_blocks = (ps.words + ENCODE_BLOCK - 1) / ENCODE_BLOCK;
+        hipLaunchKernelGGL(encode_text_kernel, dim3((u32)(enc_blocks < 4096 ? enc_blocks : 4096)), dim3(ENCODE_BLOCK), 0, s, d_text, n,
+                           pp.codes, stream, ps.words, bytehist);
+        HIP_TRY(hipGetLastError());
+        if (n >= CSA_NARROW_MIN && ps.sym_bits == 2 && ps.key_bits == 64 && pp.skipped > 0 && (rc = narrow_keys_pay(L, ps, n, &narrow)) != CSA_OK)
+            return rc;
+    }
+    const u32 ell = pp.enabled ? (narrow ? pp.codes.key_syms / 2 : pp.codes.key_syms) : 4u; // symbols of a key of the first sort
     int folded = 0; // generations after the first that still belong to the reported generation 0
     for (u64 c = ell; c < wide_ell; c += (c < wide_ell - c ? c : wide_ell - c))
         ++folded;
@@ -1507,25 +1589,20 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     u32* V[2] = {h->idx[0], h->idx[1]};
     int cur = 0; // the (K, V) set that holds the sorted pairs
     CodedList list;
-    TextSource ps;
-    memset(&ps, 0, sizeof(ps));
     if (pp.enabled) {
-        // the code stream lives in rank[], which nothing uses before the sorted list is ranked
-        u32* const stream = h->rank;
-        ps.stream = stream;
-        ps.sym_bits = pp.codes.bits;
-        ps.key_bits = pp.codes.key_syms * pp.codes.bits;
-        ps.words = ((u64)n * ps.sym_bits + 31) / 32 + 4;
-        u32* const gramhist = bytehist; // (read back already)
-        HIP_TRY(hipMemsetAsync(gramhist, 0, RADIX_BINS * sizeof(u32), s));
-        const u64 enc_blocks = (ps.words + ENCODE_BLOCK - 1) / ENCODE_BLOCK;
-        hipLaunchKernelGGL(encode_text_kernel, dim3((u32)(enc_blocks < 4096 ? enc_blocks : 4096)), dim3(ENCODE_BLOCK), 0, s, d_text, n,
-                           pp.codes, stream, ps.words, gramhist);
-        const PassPlan plan = make_plan(0, (int)ps.key_bits);
-        hipLaunchKernelGGL(packed_hist_expand_kernel, dim3(1), dim3(256), 0, s, ps.stream, n, ps.sym_bits, pp.codes.key_syms,
-                           plan.num_passes, gramhist, h->ghist);
+        const PassPlan plan = make_plan(0, narrow ? 32 : (int)ps.key_bits);
+        hipLaunchKernelGGL(packed_hist_expand_kernel, dim3(1), dim3(256), 0, s, ps.stream, n, ps.sym_bits, ell, plan.num_passes, bytehist,
+                           h->ghist);
         HIP_TRY(hipGetLastError());
-        rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, plan, &in_out, &p1, nullptr, 0, 0, &ps);
+        coded = narrow;
+        if (narrow) {
+            HIP_TRY(hipMemsetAsync(code_tables(h).marks, 0, RESOLVE_MARK_WORDS * sizeof(u32), s));
+            rc = sort_by_codes(L, d_text, n, tail, 2u, list, &ps, ell);
+            p1 = CODE_PASSES;
+            in_out = 1;
+        } else {
+            rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, plan, &in_out, &p1, nullptr, 0, 0, &ps);
+        }
     } else if (coded) {
         rc = sort_by_codes(L, d_text, n, tail, h->pack_symbols ? 2u : 1u, list);
         p1 = CODE_PASSES;
@@ -1578,8 +1655,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     u32 level_counts[2 * MAX_LEVELS]; // (survivors, groups) of each
     if (pp.skipped > MAX_LEVELS)
         return fail(CSA_ERR_INTERNAL, "the first sort covers %u generations", pp.skipped);
-    ra.levels = pp.skipped;
-    for (u32 i = 0; i < pp.skipped; ++i) {
+    ra.levels = ra.first_level = pp.skipped - (narrow ? 1u : 0u); // (with narrow keys the last one is that of the first word)
+    for (u32 i = 0; i < ra.levels; ++i) {
         ra.level_ell[i] = (u32)wide_ell << i;
         ra.level_drop[i] = (ell - ra.level_ell[i]) * pp.codes.bits;
     }
@@ -1602,10 +1679,12 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
 
     // ---- generations t >= 1 (reference loop: src/GPU_SACA.cu:1999-2103) ----
     int gen = 1;
-    u64 ctx = ell; // symbols resolved so far; the next generation looks hop symbols ahead
+    const u32 resolved = coded ? ell * list.words : ell;                            // symbols the first sort has resolved
+    const u32 skipped = narrow ? pp.skipped + list.words - 2u : pp.skipped; // generations after the first that it stands for
+    u64 ctx = resolved; // symbols resolved so far; the next generation looks hop symbols ahead
     // A list that was resolved on two words leaves what generation 1 would: that one is reported with the lists it would have had, what
     // the members of its large groups took, and no time of its own.
-    if (coded && list.words == 2) {
+    if (coded && !narrow && list.words == 2) {
         if (level_counts[0] > 0) {
             st->active[1] = level_counts[0];
             st->groups[1] = level_counts[1];
@@ -1613,7 +1692,6 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             st->passes[1] = list.long_passes;
             gen = 2;
         }
-        ctx = 2 * ell;
     } else if (coded) {
         st->passes[0] += list.long_passes;
     }
@@ -1971,10 +2049,10 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     }
     // packed keys: the first sort stands for generations 0 .. skipped of the reference; those after the first are reported
     // with the lists they would have had and no time or passes of their own
-    st->key_symbols = ell;
-    st->first_sort_generations = 1 + pp.skipped;
-    if (pp.skipped > 0) {
-        const int sk = (int)pp.skipped;
+    st->key_symbols = pp.enabled ? resolved : ell;
+    st->first_sort_generations = 1 + (int)skipped;
+    if (skipped > 0) {
+        const int sk = (int)skipped;
         if (gen + sk > CSA_MAX_GENERATIONS)
             return fail(CSA_ERR_INTERNAL, "%d generations do not fit the statistics", gen + sk);
         for (int g = gen - 1; g >= 1; --g) {

@@ -173,6 +173,8 @@ struct ProbeArgs {
     u32 table_log2;
     u32 long_from;
     ProbeCounts* counts; // zeroed
+    const u32* stream;   // non-null: the codes are the narrow keys of a packed text, sym_bits bits a symbol; `crowded` counts whoever
+    u32 sym_bits;        // finds its code taken by long_from others or more, its own string as they are
 };
 
 // An entry of the table is a code (high half), eight bits of the first string's hash and the number of suffixes that came.
@@ -190,16 +192,22 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
     if (i < a.taken) {
         const u64 x = sampled_chunk(i, a.n, a.taken, PROBE_START);
         u32 lo[4], width[4], hash = 0, code;
+        bool alone = false;
+        if (a.stream) {
+            code = (u32)packed_window(a.stream, x * a.sym_bits, 32u);
+        } else {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const u32 s = x + k < a.n ? a.text[x + k] : 0u;
-            u32 pair[2];
-            __builtin_memcpy(pair, a.cum + s, 8); // entries s and s + 1 (4-byte aligned)
-            lo[k] = pair[0];
-            width[k] = pair[1] - pair[0];
-            hash = (hash + s + 1u) * 0x9E3779B1u;
+            for (int k = 0; k < 4; ++k) {
+                const u32 s = x + k < a.n ? a.text[x + k] : 0u;
+                u32 pair[2];
+                __builtin_memcpy(pair, a.cum + s, 8); // entries s and s + 1 (4-byte aligned)
+                lo[k] = pair[0];
+                width[k] = pair[1] - pair[0];
+                hash = (hash + s + 1u) * 0x9E3779B1u;
+            }
+            alone = string_code(lo, width, code);
         }
-        if (!string_code(lo, width, code)) {
+        if (!alone) {
             const unsigned long long entry = ((unsigned long long)code << 32) | (hash >> 24 << 24) | 1u;
             const u32 mask = (1u << a.table_log2) - 1u;
             u32 slot = (code * 0x9E3779B1u) >> (32 - a.table_log2);
@@ -214,7 +222,7 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
                 const bool other = (((u32)seen ^ (u32)entry) >> 24) != 0;
                 pairs = before;
                 flags = 1u | (before == 1u ? 2u : 0u) | (before == 2u ? 4u : 0u) | (before == 3u ? 8u : 0u) | (other ? 16u : 0u) |
-                        (other && before >= a.long_from ? 32u : 0u);
+                        ((other || a.stream) && before >= a.long_from ? 32u : 0u);
                 break;
             }
         }
@@ -347,7 +355,10 @@ struct ResolveArgs {
     u32 m;            // entries of the list
     const u16* text;
     u32 n;
-    u32 words; // 1: the list is resolved on the four symbols of the codes; 2: on the four after them, too
+    u32 words; // 1: the list is resolved on the symbols of the codes; 2: on as many after them, too
+    u32 word_syms;     // symbols of a word: four, or 32 bits of the code stream of a packed text, where every code is its string's own:
+    const u32* stream; // non-null
+    u32 sym_bits;
     u32* sufs_out; // the list in order (the whole one: members of long runs go back to their places in it)
     u8* ties;      // of every entry, TIE_LONG and on how many words it ties with its left neighbour (doubling.hpp)
     u32* marks;    // [RESOLVE_MARK_WORDS], zeroed: codes of long runs that are not in order
@@ -366,8 +377,18 @@ struct ResolveArgs {
     u32 slab;
 };
 
+// The second word of suffix x, of which the text or the stream has the end at least.
+template <bool PACKED>
+__device__ __forceinline__ u64 second_word(const ResolveArgs& a, u32 x)
+{
+    if constexpr (!PACKED)
+        return load_kgram(a.text, a.n, x, 1);
+    const u64 y = (u64)x + a.word_syms;
+    return y < a.n ? packed_window(a.stream, y * a.sym_bits, 32u) : 0ull;
+}
+
 // The runs of equal codes (KEYS = false: the list of all suffixes) or of equal keys (KEYS = true: the members of the long runs, sorted
-// once more by the code of the next four symbols) of one tile and the halo its first and last run reach into, refined word by word:
+// once more by the code of the next word) of one tile and the halo its first and last run reach into, refined word by word:
 // every member of a run of at most H counts those with a smaller word, which gives its place and
 // the sub-run it belongs to, and the next word is compared among the members of a sub-run only. A string and its follower lie in
 // one line of the text as a rule, so the second word costs one more line for one suffix in nine and saves a generation: its gather
@@ -375,7 +396,9 @@ struct ResolveArgs {
 // generation 1).
 // The halo's members are refined too (by both tiles their run lies in, with the same result), so that a tile knows
 // all of its own places and writes them in order.
-template <int H, bool KEYS> // H: the longest run that is sorted inside its tile
+// PACKED: the words are cut from the code stream of the text, 16 bytes of which hold what 128 bytes of the text do; it fits the last-level
+// cache up to 10^9 symbols of two bits.
+template <int H, bool KEYS, bool PACKED> // H: the longest run that is sorted inside its tile
 __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs a)
 {
     constexpr int SPAN = RESOLVE_TILE + 2 * H;
@@ -437,6 +460,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     int at[ITEMS], first[ITEMS], last[ITEMS]; // last - first = 1: alone
     u64 w0[ITEMS], w1[ITEMS];
     const bool two = KEYS || a.words == 2; // (keys come with two words)
+    const u32 word_syms = PACKED ? a.word_syms : 4u;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         const bool halo = k == RESOLVE_ITEMS;
@@ -468,11 +492,11 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
             longs |= 1u << k;
         }
         const bool own = (owners >> k) & 1u;
-        if (!KEYS && !own)
+        if (!KEYS && !PACKED && !own)
             w0[k] = load_kgram(a.text, a.n, x[k], 0);
         if (two && (KEYS || is_short)) // (the members of long runs of codes get their second word when they are sorted by it)
-            w1[k] = load_kgram(a.text, a.n, x[k], 1);
-        if ((u64)x[k] + 4u * a.words >= n)
+            w1[k] = second_word<PACKED>(a, x[k]);
+        if ((u64)x[k] + (u64)word_syms * a.words >= n)
             s_ends = 1;
         if (is_short && l - f > FEW) {
             s_many[0] = 1;
@@ -503,7 +527,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
             }
             __syncthreads();
         }
-        const u64 ctx = 4u * (u32)(w + 1);
+        const u64 ctx = word_syms * (u32)(w + 1);
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k) {
             const int f = first[k], l = last[k], j = at[k];
@@ -646,6 +670,63 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         }
 }
 
+// What a list sorted by the narrow keys of a packed text would leave at contexts shorter than a key (RerankArgs::level_drop, level_ell; the
+// sums at level_totals[slot * 8 + 2 i] and [.. + 1]): an entry ties with a neighbour if neither runs off the text inside the context.
+// Reads 8 bytes a suffix.
+__global__ __launch_bounds__(256) void count_code_levels_kernel(RerankArgs a, const u32* __restrict__ codes, u32 levels)
+{
+    constexpr int ITEMS = 4;
+    const u32 lane = threadIdx.x & 63u;
+    u32 sums[2 * MAX_LEVELS] = {};
+    const u64 stride = (u64)gridDim.x * 256 * ITEMS;
+    for (u64 base = ((u64)blockIdx.x * 256 + threadIdx.x) * ITEMS; base < a.m; base += stride) {
+        u32 code[ITEMS + 2] = {}, suf[ITEMS + 2] = {}; // entries base - 1 .. base + ITEMS
+        if (base + ITEMS <= a.m) { // (the arrays are 16-byte aligned)
+            const uint4 c = *reinterpret_cast<const uint4*>(codes + base), x = *reinterpret_cast<const uint4*>(a.sufs + base);
+            code[1] = c.x, code[2] = c.y, code[3] = c.z, code[4] = c.w;
+            suf[1] = x.x, suf[2] = x.y, suf[3] = x.z, suf[4] = x.w;
+        } else {
+#pragma unroll
+            for (int k = 1; k <= ITEMS; ++k)
+                if (base + k - 1 < a.m) {
+                    code[k] = codes[base + k - 1];
+                    suf[k] = a.sufs[base + k - 1];
+                }
+        }
+        if (base > 0) {
+            code[0] = codes[base - 1];
+            suf[0] = a.sufs[base - 1];
+        }
+        if (base + ITEMS < a.m) {
+            code[ITEMS + 1] = codes[base + ITEMS];
+            suf[ITEMS + 1] = a.sufs[base + ITEMS];
+        }
+#pragma unroll
+        for (u32 i = 0; i < MAX_LEVELS; ++i) {
+            if (i >= levels)
+                break;
+            u32 ties = 0; // bit k: entries base + k - 1 and base + k
+#pragma unroll
+            for (int k = 0; k <= ITEMS; ++k) {
+                const bool there = base + k > 0 && base + k < a.m;
+                const u32 last = suf[k] > suf[k + 1] ? suf[k] : suf[k + 1];
+                ties |= (there && ((code[k] ^ code[k + 1]) >> a.level_drop[i]) == 0 && (u64)last + a.level_ell[i] < a.n ? 1u : 0u) << k;
+            }
+            const u32 whole = (1u << ITEMS) - 1u;
+            sums[2 * i] += (u32)__popc((ties | (ties >> 1)) & whole);
+            sums[2 * i + 1] += (u32)__popc(~ties & (ties >> 1) & whole);
+        }
+    }
+#pragma unroll
+    for (u32 i = 0; i < 2 * MAX_LEVELS; ++i) {
+        if (i >= 2 * levels)
+            break;
+        const u32 v = wave_reduce_sum(sums[i]);
+        if (lane == 0 && v)
+            atomicAdd(a.level_totals + (u64)((blockIdx.x * 4 + threadIdx.x / WAVE) % LEVEL_SLOTS) * 8 + i, (unsigned long long)v);
+    }
+}
+
 // Members of long runs, in list order: APPLY = false counts them and the strings they begin per tile, APPLY = true (after
 // rerank_scan_kernel) writes what they are to be sorted by, their suffixes and their list places. MARKED: those of runs that are out of
 // order alone, by their strings; a run is marked as a whole, so the list of them sorted by string, which is also the order
@@ -724,8 +805,8 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_runs_kernel(ResolveArgs
             if constexpr (MARKED) {
                 key[k] = load_kgram(a.text, a.n, x[k], 0);
             } else {
-                const u64 y = (u64)x[k] + 4u; // (a suffix that has none there is a string of its own)
-                key[k] = y >= a.n ? 0u : a.text_codes[y + a.tail >= a.n ? a.n - 1 - y : y + a.tail];
+                const u64 y = (u64)x[k] + a.word_syms; // (a suffix that has none there is a string of its own)
+                key[k] = y >= a.n ? 0u : a.stream ? (u32)packed_window(a.stream, y * a.sym_bits, 32u) : a.text_codes[y + a.tail >= a.n ? a.n - 1 - y : y + a.tail];
             }
         }
     }

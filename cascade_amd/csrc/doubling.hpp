@@ -76,6 +76,7 @@ struct RerankArgs {
     u32 levels; // <= MAX_LEVELS
     u32 level_drop[4];
     u32 level_ell[4];
+    u32 first_level; // TIED: the level that the first word of the list stands for
     unsigned long long* level_totals;
     u32* rank; // [n] by text position; null (and no rank_recs): the list is compacted and nothing is ranked
     // Deferred rank update: instead of the scattered write rank[x] = r, the suffix at sorted index c leaves the record
@@ -330,7 +331,7 @@ __global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles
 #pragma unroll
     for (u32 i = 0; i < TIE_MOST_WORDS; ++i) {
         const u32 sv = wave_reduce_sum(sum_surv[i]), hd = wave_reduce_sum(sum_heads[i]);
-        unsigned long long* const slot = a.level_totals + (u64)(wave % LEVEL_SLOTS) * 8 + 2 * i;
+        unsigned long long* const slot = a.level_totals + (u64)(wave % LEVEL_SLOTS) * 8 + 2 * (a.first_level + i);
         if (lane == 0 && sv) {
             atomicAdd(slot, (unsigned long long)sv);
             atomicAdd(slot + 1, (unsigned long long)hd);

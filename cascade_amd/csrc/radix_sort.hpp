@@ -29,7 +29,8 @@ enum : int {
     SRC_PAIRS = 0, // keys_in[i], vals_in[i]
     SRC_CODED = 1, // generation 0, first pass: keys_in holds the codes of virtual positions (coded_keys.hpp), the suffixes follow from them
     SRC_RANKS = 2, // a dense later generation, first pass: pair i = ((rank[i], rank[i + hop]), i), built from rank[]
-    SRC_PACKED = 3, // generation 0 over a small alphabet, first pass: the key of virtual position i is cut from the code stream
+    SRC_PACKED = 3, // generation 0 over a small alphabet, first pass: the key of virtual position i is cut from the code stream (a narrow
+                    // one is the code of its symbols and of no others: OWN_CODE)
     SRC_TEXT = 4   // generation 0 on K-gram keys, first pass: the pair of virtual position i is built from the text
 };
 
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
     constexpr int TILE = BLOCK * ITEMS;
     constexpr int WAVES = BLOCK / WAVE;
     static_assert(BLOCK >= RADIX_BINS, "one thread per digit is assumed");
-    static_assert(sizeof(KeyT) == 8 || ((SRC == SRC_PAIRS || SRC == SRC_CODED) && HI == 0), "narrow keys are read from an array");
+    static_assert(sizeof(KeyT) == 8 || ((SRC == SRC_PAIRS || SRC == SRC_CODED || SRC == SRC_PACKED) && HI == 0), "narrow keys are read from an array, or cut from the code stream");
     constexpr bool KEYS_IN = SRC == SRC_PAIRS || SRC == SRC_CODED;
     auto rank_key = [&](u32 i) -> u64 { return rank_pair_key(a.rank, a.n, a.hop, i, a.radix); }; // SRC_RANKS: pair i is text position i
     const KeyT* __restrict__ keys_in = static_cast<const KeyT*>(a.keys_in);
@@ -554,7 +555,8 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
                 val[k] = x | ((a.own[x >> 3] >> (x & 7u)) & 1u ? OWN_CODE : 0u);
             }
         } else if (VALS && local < valid)
-            val[k] = (SRC == SRC_TEXT || SRC == SRC_PACKED) ? virtual_to_suffix((u32)(base + local), a.text_n, a.tail)
+            val[k] = SRC == SRC_TEXT                        ? virtual_to_suffix((u32)(base + local), a.text_n, a.tail)
+                     : SRC == SRC_PACKED                    ? virtual_to_suffix((u32)(base + local), a.text_n, a.tail) | (sizeof(KeyT) == 4 ? OWN_CODE : 0u)
                      : SRC == SRC_RANKS                     ? (u32)(base + local)
                                                             : a.vals_in[base + local];
     }

@@ -318,6 +318,37 @@ def test_small_alphabets_start_from_keys_of_many_symbols(emu, name):
         assert np.array_equal(got2, got) and active2 == counts and emu_sort.first_sort_generations == 1
 
 
+@pytest.mark.parametrize("kind", ["copy", "run", "zeros", "skew"])
+@pytest.mark.parametrize("key_words", [1, 2, 4])
+def test_narrow_keys_of_four_letters(emu, kind, key_words):
+    """Texts of two-bit symbols above the length from which the first sort takes 32 bits of the code stream (2000 here) and
+    reads the next 32 for the tied: copies, long runs that are collected or send the text back to wide keys, zeros that tie with the
+    padding. The array and every generation's active count are the oracle's."""
+    rng = np.random.default_rng(key_words)
+    for n in (2000, 2047, 4100):
+        T = rng.integers(0, 4, n).astype(np.uint16)
+        if kind == "copy":
+            T[n // 2:n // 2 + n // 4] = T[:n // 4]
+        elif kind == "run":
+            T[n // 4:n // 4 + n // 9] = 1
+            T[n // 2:n // 2 + n // 20] = np.resize(rng.integers(0, 4, 7), n // 20)
+        elif kind == "zeros":
+            T[-40:] = 0
+        else:
+            T = ((rng.random(n) < 0.03) * 2).astype(np.uint16)
+        got, active, _ = emu_sort(emu, T, key_words)
+        sa, counts = oracle_lib.prefix_doubling(T, key_words)
+        assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)), n
+        assert active == counts, n
+        assert emu_sort.key_symbols == 64 // emu_sort_bits(T)
+        if kind in ("copy", "zeros"):
+            assert emu_sort.passes[0] == 4
+
+
+def emu_sort_bits(T):
+    return 1 if np.unique(np.append(T, 0)).size <= 2 else 2
+
+
 def test_emulated_radix_sort_matches_stable_sort(emu):
     rng = np.random.default_rng(1)
     n = 5000

@@ -360,6 +360,38 @@ def test_four_letters_start_from_keys_of_32_symbols(torch_mod, key_words, exclus
     assert small_stats["first_sort_generations"] == first
 
 
+@pytest.mark.parametrize("n,kind,key_words", [(1 << 24, "copy", 1), ((1 << 24) + 1, "copy", 1), ((1 << 25) + 5, "copy", 4),
+                                              ((1 << 24) + 5, "longs", 1), ((1 << 25) + 64, "longs", 2)])
+def test_narrow_keys_of_four_letters(torch_mod, n, kind, key_words):
+    """Past 2^24 symbols four letters are sorted by 16 of them and by the next 16 where those tie: a long copy, and a string that is in
+    the text ten thousand times, against the sort from K-gram words, generation sizes included."""
+    from cascade_amd import PartitionSorter, _native
+    gen = torch_mod.Generator(device="cuda").manual_seed(n)
+    T = torch_mod.randint(0, 4, (n,), generator=gen, device="cuda", dtype=torch_mod.int32).to(torch_mod.int16)
+    if kind == "copy":
+        T[n // 2:n // 2 + n // 5] = T[:n // 5]
+    else:
+        word = torch_mod.randint(0, 4, (20,), generator=gen, device="cuda", dtype=torch_mod.int32).to(torch_mod.int16)
+        at = torch_mod.randperm(n // 20 - 1, generator=gen, device="cuda")[:10000] * 20
+        for q in range(20):
+            T[at + q] = word[q]
+        T[-30:] = 0
+    print(f"  narrow keys n={n} {kind} key_words={key_words}", flush=True)
+    with PartitionSorter(n, key_words=key_words) as s:
+        out = s.sort(T)
+        assert s.verify(T, out)
+        narrow = s.last_stats
+        s.set_tuning(_native.CSA_TUNE_PACK_SYMBOLS, 0)
+        assert torch_mod.equal(out, s.sort(T))
+        plain = s.last_stats
+    assert narrow["active"] == plain["active"] and narrow["groups"][1:] == plain["groups"][1:]
+    assert narrow["key_symbols"] == 32
+    if kind == "copy":
+        assert narrow["passes"][0] == (8 if n <= 1 << 24 else 4)
+    else:
+        assert narrow["passes"][0] > 4  # the members of the long run were collected
+
+
 def test_a_dense_generation_after_one_that_was_not(torch_mod):
     """A run of 110 000 equal tokens between two stretches whose K-grams collide in some 1500 pairs: generation 1 (one long
     group, many pairs: short groups on average) gathers and leaves ranks in rank[]; the pairs dissolve, generation 2 holds
