@@ -11,6 +11,7 @@
 #include "partition_ids.hpp"
 #include "pipeline_steps.hpp"
 #include "radix_sort.hpp"
+#include "short_text.hpp"
 
 #include <cmath>
 #include <cstdarg>
@@ -1504,12 +1505,93 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
     return CSA_OK;
 }
 
+// Texts of up to this many symbols are ranked by counting (short_text.hpp).
+#ifndef CSA_SHORT_TEXT
+#define CSA_SHORT_TEXT SHORT_MAX
+#endif
+
+// The whole sort of a short text: one round trip, and a second one where many suffixes are tied on four symbols. Works in gid, rank and
+// the symbol counts.
+int sort_short_text(Launch& L, const u16* d_text, u32 n, u64 index_base, u8* d_sa40)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    csa_stats* st = L.stats;
+    RangeScope range("sort_short_text n=%u", n);
+    u32* const ranks[2] = {h->gid, h->rank};
+    ShortArgs a;
+    memset(&a, 0, sizeof(a));
+    a.text = d_text;
+    a.n = n;
+    a.index_base = index_base;
+    a.out = d_sa40;
+    a.rank_out = ranks[0];
+    a.counters = code_tables(h).counts;
+    const u64 wide_ell = 4ull * (u64)h->key_words;
+    u32 last = 0; // generation
+    for (u64 ctx = 4; ctx < n && last + 1 < SHORT_GENERATIONS - 1;) {
+        const u64 hop = ctx < wide_ell ? (ctx < wide_ell - ctx ? ctx : wide_ell - ctx) : ctx;
+        a.hops[++last] = (u32)hop;
+        ctx += hop;
+    }
+    const dim3 grid((n + SHORT_X - 1) / SHORT_X);
+    HIP_TRY(hipEventRecord(h->ev_gen[0], s));
+    int rc = move_table(a.counters, nullptr, SHORT_COUNTERS * sizeof(u32), s);
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(short_first_kernel, grid, dim3(SHORT_BLOCK), 0, s, a);
+    a.generation = 1;
+    a.rank_in = ranks[0];
+    hipLaunchKernelGGL(short_rest_kernel, dim3(1), dim3(SHORT_BLOCK), 0, s, a);
+    u32* const seen = h->h_pinned + PINNED_HIST;
+    static_assert(SHORT_COUNTERS <= MAX_PASSES * RADIX_BINS && SHORT_COUNTERS <= SYMBOLS, "the counters fit the tables they are kept in");
+    if ((rc = move_table(seen, a.counters, SHORT_COUNTERS * sizeof(u32), s)) != CSA_OK)
+        return rc;
+    HIP_TRY(hipEventRecord(h->ev_gen[1], s));
+    HIP_TRY(hipStreamSynchronize(s));
+    if (seen[SHORT_LEFT] != 0) {
+        for (u32 g = 1; g <= last; ++g) {
+            a.generation = g;
+            a.rank_in = ranks[(g - 1) & 1];
+            a.rank_out = ranks[g & 1];
+            hipLaunchKernelGGL(short_next_kernel, grid, dim3(SHORT_BLOCK), 0, s, a);
+        }
+        if ((rc = move_table(seen, a.counters, SHORT_COUNTERS * sizeof(u32), s)) != CSA_OK)
+            return rc;
+        HIP_TRY(hipEventRecord(h->ev_gen[1], s));
+        HIP_TRY(hipStreamSynchronize(s));
+    }
+    // the generations of the caller's key width: those before it has been reached belong to generation 0
+    u32 folded = 0, generations = 1;
+    for (u64 c = 4; c < wide_ell; c += (c < wide_ell - c ? c : wide_ell - c))
+        ++folded;
+    while (generations < SHORT_GENERATIONS && seen[2 * generations] != 0)
+        ++generations;
+    if (generations > last + 1)
+        return fail(CSA_ERR_INTERNAL, "%u suffixes of a short text are tied after the last generation", seen[2 * (generations - 1)]);
+    folded = folded < generations - 1 ? folded : generations - 1;
+    st->generations = (int)(generations - folded);
+    st->active[0] = n;
+    for (u32 g = 1; g + folded < generations; ++g) {
+        st->active[g] = seen[2 * (g + folded)];
+        st->groups[g] = seen[2 * (g + folded) + 1];
+    }
+    st->key_symbols = 4;
+    st->first_sort_generations = 1;
+    HIP_TRY(hipEventElapsedTime(&st->ms[0], h->ev_gen[0], h->ev_gen[1]));
+    st->ms_total = st->ms[0];
+    return CSA_OK;
+}
+
 int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_sa40)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
     csa_stats* st = L.stats;
     const u32 n = (u32)n64;
+    // (a caller who has set thresholds of the large sort, or asks for the times of its passes, gets that one)
+    if (n <= CSA_SHORT_TEXT && h->pack_symbols && h->settle && !h->expect_presorted && !(L.flags & CSA_FLAG_KERNEL_TIMING))
+        return sort_short_text(L, d_text, n, index_base, d_sa40);
     // Wide keys are not sorted word by word. A generation 0 that resolves 4 W symbols is what doubling on one-word keys
     // reaches after one or two more generations (4 -> 8 -> 16 symbols; 4 -> 8 -> 12 with the second step looking only 4
     // symbols ahead; the order of suffixes that run off the text is the same: the shorter first). So the sort always

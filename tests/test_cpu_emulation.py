@@ -349,6 +349,15 @@ def emu_sort_bits(T):
     return 1 if np.unique(np.append(T, 0)).size <= 2 else 2
 
 
+@pytest.mark.parametrize("n,sigma,key_words", texts.SHORT_TEXTS)
+def test_short_texts_by_counting(emu_dev, n, sigma, key_words):
+    """Texts that are ranked by counting, few and many suffixes tied, against the oracle, generation sizes included."""
+    T = texts.short_text(n, sigma)
+    got, active, _ = emu_sort(emu_dev, T, key_words)
+    sa, counts = oracle_lib.prefix_doubling(T, key_words)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
 def test_emulated_radix_sort_matches_stable_sort(emu):
     rng = np.random.default_rng(1)
     n = 5000

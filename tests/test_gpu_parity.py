@@ -392,6 +392,19 @@ def test_narrow_keys_of_four_letters(torch_mod, n, kind, key_words):
         assert narrow["passes"][0] > 4  # the members of the long run were collected
 
 
+@pytest.mark.parametrize("n,sigma,key_words", texts.SHORT_TEXTS + [(8191, 60000, 1), (8192, 2, 1), (8192, 1, 4), (8193, 60000, 1)])
+def test_short_texts_by_counting(torch_mod, n, sigma, key_words):
+    """Texts of up to 8192 symbols are ranked by counting; one more, and the large sort takes over."""
+    from cascade_amd import PartitionSorter
+    T = texts.short_text(n, sigma)
+    print(f"  short text n={n} sigma={sigma} key_words={key_words}", flush=True)
+    with PartitionSorter(n, key_words=key_words) as s:
+        got = s.sort(to_dev(torch_mod, T)).cpu().numpy()
+        stats = s.last_stats
+    sa, counts = oracle_lib.prefix_doubling(T, key_words)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
+
+
 def test_a_dense_generation_after_one_that_was_not(torch_mod):
     """A run of 110 000 equal tokens between two stretches whose K-grams collide in some 1500 pairs: generation 1 (one long
     group, many pairs: short groups on average) gathers and leaves ranks in rank[]; the pairs dissolve, generation 2 holds

@@ -150,3 +150,17 @@ def text_of_copies(n, symbols, seed):
     elif seed % 3 == 1:
         T[n - n // 5:] = T[:n // 5]
     return T
+
+
+SHORT_TEXTS = [(1, 1, 1), (5, 2, 1), (16, 60000, 4), (17, 2, 3), (513, 1, 2), (700, 60000, 1), (1025, 1, 1), (1025, 2, 4), (1500, 60000, 3)]
+
+
+def short_text(n, sigma):
+    """A text for the sort of short texts: a repeat and a run, so that more suffixes are tied than one workgroup takes to the end where
+    n > 1000 (and all of them where sigma = 1), zeros at the end."""
+    rng = np.random.default_rng(n + sigma)
+    T = rng.integers(0, sigma, n).astype(np.uint16)
+    T[n // 2:n // 2 + n // 4] = T[:n // 4]
+    T[n // 8:n // 8 + n // 3] = T[0]
+    T[n - n // 40:] = 0
+    return T
