@@ -2,6 +2,7 @@
 // declared in include/cascade_hip.h. gfx950 only.
 #include "../../include/cascade_hip.h"
 
+#include "chains.hpp"
 #include "coded_keys.hpp"
 #include "copies.hpp"
 #include "device_pool.hpp"
@@ -1408,6 +1409,76 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     return CSA_OK;
 }
 
+// Settles a list whose groups are runs and periods (chains.hpp): num generations of the doubling from the one about to begin, with the
+// sizes that they would have had.
+struct Chains {
+    bool settled;
+    u32 num;
+    u32 active[SETTLE_CONTEXTS], groups[SETTLE_CONTEXTS], big[SETTLE_CONTEXTS];
+    bool small_only[SETTLE_CONTEXTS];
+};
+constexpr u32 CHAIN_TRIES = 2; // failed attempts (two passes over the list and a round trip; a generation costs five times as much)
+
+// Works in `scratch` ([groups]) and the symbol counts of the first sort.
+int settle_chains(Launch& L, Chains& ch, const u16* d_text, u32 n, u64 ctx, u64 wide_ell, const u32* sufs, const u32* gids, const u32* gstart,
+                  const u32* gprim, u32 m, u32 groups, u32* scratch, u32* sa32)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    ChainArgs a;
+    memset(&a, 0, sizeof(a));
+    memset(&ch, 0, sizeof(ch));
+    a.text = d_text;
+    a.n = n;
+    a.ctx = (u32)ctx;
+    a.sufs = sufs;
+    a.gids = gids;
+    a.gstart = gstart;
+    a.gprim = gprim;
+    a.m = m;
+    a.groups = groups;
+    a.sa32 = sa32;
+    a.backwards = scratch;
+    a.limit_lo = SMALL_MAXG;
+    a.limit_hi = SMALL_MAXG_HI;
+    u64 c = ctx;
+    do {
+        a.contexts[a.num_contexts++] = (u32)c;
+        c += c < wide_ell ? (c < wide_ell - c ? c : wide_ell - c) : c;
+    } while (c < n && a.num_contexts < SETTLE_CONTEXTS);
+    a.tallies = code_tables(h).counts;
+    a.failed = h->counts + 4;
+    a.err = h->counts + 2;
+    constexpr u32 TALLIES = SETTLE_CONTEXTS * CHAIN_TALLIES;
+    static_assert(TALLIES <= SYMBOLS && TALLIES <= MAX_PASSES * RADIX_BINS, "the tallies take the symbol counts' place, and the histograms' on the host");
+    TableGroup zeros = {}, seen = {};
+    add_table(zeros, a.failed, nullptr, sizeof(u32));
+    add_table(zeros, a.tallies, nullptr, TALLIES * sizeof(u32));
+    int rc = move_tables(zeros, s);
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(chain_groups_kernel, dim3((groups + 255) / 256), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(chain_place_kernel, dim3((u32)(((u64)m + 255) / 256)), dim3(256), 0, s, a);
+    HIP_TRY(hipGetLastError());
+    u32* const tallies = h->h_pinned + PINNED_HIST;
+    add_table(seen, tallies, a.tallies, TALLIES * sizeof(u32));
+    u32 failed = 0;
+    rc = read_counts(L, &failed, seen);
+    if (rc || failed)
+        return rc;
+    bool all_small = false;
+    for (; ch.num < a.num_contexts && tallies[ch.num * CHAIN_TALLIES] > 0; ++ch.num) {
+        const u32* const w = tallies + ch.num * CHAIN_TALLIES;
+        ch.active[ch.num] = w[0];
+        ch.groups[ch.num] = w[1];
+        ch.small_only[ch.num] = all_small;
+        ch.big[ch.num] = all_small ? 0u : (u64)w[0] <= (u64)w[1] * SMALL_AVG_LIMIT ? w[3] : w[2];
+        all_small = all_small || ch.big[ch.num] == 0;
+    }
+    ch.settled = true;
+    return CSA_OK;
+}
+
 // Generation 0: ranks the sorted list described by `ra`: counts per tile, scans the counts, reads the totals back, then
 // applies them and brings rank[] up to date, directly from the kernel or through the two-pass bucketed update.
 // coded: the list comes from sort_by_codes and carries its ties. settle: the ties of a list of short groups are settled at once if possible; the
@@ -1792,6 +1863,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     int gp = 0; // gprim[gp] / gstart[gp] describe the current groups
     bool all_small = false; // no group of the current list exceeds the limit of the generation that found it so
     bool presorted_before = false; // every large group of the generation before was in order as it stood
+    int chained = 0;               // the generation from which on the list was settled by settle_chains: the time is all that one's
+    u32 chain_tries = 0;           // attempts at settle_chains that came to nothing
     bool high_limit = false; // that generation's limit was SMALL_MAXG_HI (groups only split: the limit stays from there on)
     const int sec_bits = bit_length(n > 1 ? n - 1 : 1);
     while (m > 0) {
@@ -1871,6 +1944,29 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             gen++;
             ctx += hop;
             continue;
+        }
+        // Every member of the list before was one of a long group in order: runs and periods, as a rule.
+        if (h->pack_symbols && h->settle && !ordinals_in_rank && gen > untimed + 1 && st->presorted[gen - 1] == st->active[gen - 1] &&
+            chain_tries < CHAIN_TRIES) {
+            Chains ch;
+            rc = settle_chains(L, ch, d_text, n, ctx, wide_ell, ax, agid, h->gstart[gp], h->gprim[gp], m_in, groups, h->gprim[gp ^ 1], sa32);
+            if (rc)
+                return rc;
+            if (ch.settled) {
+                if (gen + ch.num > CSA_MAX_GENERATIONS)
+                    return fail(CSA_ERR_INTERNAL, "%u generations do not fit the statistics", gen + ch.num);
+                for (u32 i = 0; i < ch.num; ++i) {
+                    st->active[gen + i] = ch.active[i];
+                    st->groups[gen + i] = ch.groups[i];
+                    st->big[gen + i] = st->presorted[gen + i] = ch.big[i];
+                    st->small_only[gen + i] = ch.small_only[i];
+                }
+                chained = gen;
+                gen += (int)ch.num;
+                HIP_TRY(hipEventRecord(h->ev_gen[gen], s));
+                break;
+            }
+            ++chain_tries;
         }
         if (ordinals_in_rank)
             return fail(CSA_ERR_INTERNAL, "generation %d reads ranks but the one before it left ordinals", gen);
@@ -2091,9 +2187,9 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         return rc;
 
     for (int g = 0; g < gen; ++g) {
-        if (g >= 1 && g <= untimed)
+        if ((g >= 1 && g <= untimed) || (chained && g > chained))
             continue;
-        HIP_TRY(hipEventElapsedTime(&st->ms[g], h->ev_gen[g], h->ev_gen[g == 0 ? untimed + 1 : g + 1]));
+        HIP_TRY(hipEventElapsedTime(&st->ms[g], h->ev_gen[g], h->ev_gen[g == 0 ? untimed + 1 : chained && g == chained ? gen : g + 1]));
     }
     HIP_TRY(hipEventElapsedTime(&st->ms_output, h->ev_gen[gen], h->ev_gen[gen + 1]));
     HIP_TRY(hipEventElapsedTime(&st->ms_total, h->ev_gen[0], h->ev_gen[gen + 1]));

@@ -71,7 +71,7 @@ def steps_handle(lib, key_words):
     return make
 
 
-def emu_sort(lib, T, key_words, pack=True, expect_presorted=False):
+def emu_sort(lib, T, key_words, pack=True, expect_presorted=False, defer_min=None):
     """pack=False: the first sort takes one K-gram word even when the alphabet is small (CSA_TUNE_PACK_SYMBOLS 0), for the
     tests that aim at what the generations after it do on such texts. expect_presorted: CSA_TUNE_EXPECT_PRESORTED 1."""
     T = np.ascontiguousarray(T, dtype=np.uint16)
@@ -82,6 +82,8 @@ def emu_sort(lib, T, key_words, pack=True, expect_presorted=False):
         assert lib.csa_set_tuning(h, _native.CSA_TUNE_PACK_SYMBOLS, 0) == 0
     if expect_presorted:
         assert lib.csa_set_tuning(h, _native.CSA_TUNE_EXPECT_PRESORTED, 1) == 0
+    if defer_min is not None:
+        assert lib.csa_set_tuning(h, _native.CSA_TUNE_DEFER_MIN, defer_min) == 0
     out = np.zeros(5 * n + 8, dtype=np.uint8)
     st = _native.CsaStats()
     rc = lib.csa_sort_partition_u16_dev(h, T.ctypes.data, n, 0, out.ctypes.data, None, 0, C.byref(st))
@@ -237,6 +239,21 @@ def test_large_groups_that_are_in_order_already_skip_the_sort(emu, after_run):
     # do sort take the second gather, and nothing else changes
     got2, active2, big2 = emu_sort(emu, T, 1, pack=False, expect_presorted=True)
     assert np.array_equal(got2, got) and (active2, big2, emu_sort.presorted) == (active, big, presorted)
+
+
+@pytest.mark.parametrize("kind", texts.CHAINS)
+def test_runs_and_periods_settled_at_once(emu, kind):
+    """Lists of runs and periods are finished without the generations that the doubling would need: the array is the oracle's, and the
+    statistics are those of a sort that goes through them all (any threshold of the rank updates turns the short cut off)."""
+    for n, key_words in ((6000, 1), (9001, 1), (6000, 3), (9001, 4)):
+        T = texts.chains_text(kind, n)
+        seen = []
+        for tuned in (False, True):
+            got, active, big = emu_sort(emu, T, key_words, defer_min=1500 if tuned else None)
+            seen.append((active, big, emu_sort.presorted, emu_sort.small_only))
+            sa, counts = oracle_lib.prefix_doubling(T, key_words)
+            assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts, (n, key_words, tuned)
+        assert seen[0] == seen[1], (n, key_words)
 
 
 def test_small_and_large_groups_take_both_paths(emu):

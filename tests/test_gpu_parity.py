@@ -450,6 +450,26 @@ def test_generations_that_expect_their_large_groups_in_order(torch_mod):
             assert any(p > 0 for p in plain["presorted"])
 
 
+@pytest.mark.parametrize("kind", texts.CHAINS)
+def test_runs_and_periods_settled_at_once(torch_mod, kind):
+    """Lists of runs and periods are finished at once; a sort with a tuned threshold goes through all generations and has the same
+    array and sizes, and the oracle's."""
+    from cascade_amd import PartitionSorter, _native
+    T = texts.chains_text(kind, 300007)
+    d = to_dev(torch_mod, T)
+    print(f"  chains: {kind}", flush=True)
+    with PartitionSorter(T.size, key_words=1) as s:
+        out = s.sort(d)
+        at_once = s.last_stats
+        s.set_tuning(_native.CSA_TUNE_DEFER_MIN, 1 << 30)
+        assert torch_mod.equal(out, s.sort(d))
+        doubled = s.last_stats
+        got = out.cpu().numpy()
+    assert oracle_lib.is_correct_sa40(got, T)
+    for key in ("active", "groups", "big", "presorted", "small_only"):
+        assert at_once[key] == doubled[key], key
+
+
 def test_byte_texts_start_from_keys_of_8_symbols(torch_mod):
     """A text of byte values (every value 0..255 occurs): codes of 8 bits, 8 symbols in the first key, which covers
     generations 0-1 of one-word keys. A million symbols with long repeats and a tail of zeros, against the oracle."""

@@ -164,3 +164,28 @@ def short_text(n, sigma):
     T[n // 8:n // 8 + n // 3] = T[0]
     T[n - n // 40:] = 0
     return T
+
+
+def chains_text(kind, n):
+    """Independent symbols around runs and stretches of one period, whose suffixes are all that is tied after a generation or two."""
+    rng = np.random.default_rng(n)
+    T = rng.integers(20, 60000, n).astype(np.uint16)
+    if kind in ("rising", "falling", "two runs", "mixed"):
+        T[n // 8:n // 8 + n // 6] = 17
+        T[n // 8 + n // 6] = 1 if kind == "falling" else 50000
+    if kind == "two runs":  # of one token: a group of two stretches, which the doubling goes on with
+        T[n // 2:n // 2 + n // 7] = 17
+    if kind in ("period", "mixed"):
+        T[n // 2:n // 2 + n // 4] = np.resize(rng.integers(20, 60000, 7), n // 4)
+    if kind == "mixed":
+        T[9 * n // 10:9 * n // 10 + n // 20] = np.resize(rng.integers(20, 60000, 3), n // 20)
+    if kind == "long period":  # looked at once ctx has reached it
+        T[n // 4:n // 4 + n // 3] = np.resize(rng.integers(20, 60000, 30), n // 3)
+    if kind == "end":  # the text ends inside the run
+        T[-(n // 5):] = 30
+    if kind == "period at the end":
+        T[-(n // 5):] = np.resize(rng.integers(20, 60000, 7), n // 5)
+    return T
+
+
+CHAINS = ["rising", "falling", "two runs", "period", "mixed", "long period", "end", "period at the end"]
