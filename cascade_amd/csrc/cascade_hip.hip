@@ -1581,7 +1581,7 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
 #define CSA_SHORT_TEXT SHORT_MAX
 #endif
 
-// The whole sort of a short text: one round trip, and a second one where many suffixes are tied on four symbols. Works in gid, rank and
+// The whole sort of a short text: one round trip, and a second one where a group of suffixes that are tied on four symbols is long. Works in gid, rank and
 // the symbol counts.
 int sort_short_text(Launch& L, const u16* d_text, u32 n, u64 index_base, u8* d_sa40)
 {
@@ -1620,7 +1620,7 @@ int sort_short_text(Launch& L, const u16* d_text, u32 n, u64 index_base, u8* d_s
         return rc;
     HIP_TRY(hipEventRecord(h->ev_gen[1], s));
     HIP_TRY(hipStreamSynchronize(s));
-    if (seen[SHORT_LEFT] != 0) {
+    if (seen[SHORT_LONG] != 0) {
         for (u32 g = 1; g <= last; ++g) {
             a.generation = g;
             a.rank_in = ranks[(g - 1) & 1];

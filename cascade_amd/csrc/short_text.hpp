@@ -6,7 +6,7 @@
 // to the length below. Generation 0 compares four symbols, generation t the ranks of the generation before at x and x + h,
 // so every rank, active set and group is that of the prefix doubling of large texts.
 //   short_first_kernel   generation 0
-//   short_rest_kernel    all later ones, in one workgroup, if few suffixes are tied (nearly every text)
+//   short_rest_kernel    all later ones, in one workgroup, if no group is long (nearly every text)
 //   short_next_kernel    one later generation, over the whole device, otherwise
 // A suffix leaves for its place in the output in the generation that finds it alone.
 // 4096 Zipf tokens: 39 us a sort, 158 the long way.
@@ -22,11 +22,13 @@ constexpr u32 SHORT_MAX = 8192;  // the keys of a text take 64 KB of LDS (us a s
                                  // bytes 172 and 302, four letters 268 and 375)
 constexpr u32 SHORT_X = 16;      // suffixes of a workgroup, each compared with the others by ...
 constexpr u32 SHORT_SLICES = SHORT_BLOCK / SHORT_X; // ... so many threads
-constexpr u32 SHORT_FEW = 512;   // tied suffixes that one workgroup takes to the end
-constexpr u32 SHORT_TIED = 0x80000000u; // of a rank: others have it too
+constexpr u32 SHORT_GROUP = 256; // members of the longest group that one workgroup takes to the end (each looks at all others)
+constexpr u32 SHORT_TIED = 0x80000000u; // of a rank: others have it too ...
+constexpr u32 SHORT_RANK_BITS = 13, SHORT_RANK = (1u << SHORT_RANK_BITS) - 1; // ... and how many of them are earlier in the text, above the rank
+static_assert(SHORT_MAX <= 1u << SHORT_RANK_BITS, "a rank and a place in a group take 26 bits");
 constexpr u32 SHORT_GENERATIONS = 16;   // 4, 8, ... symbols: more than SHORT_MAX after 12, one more with keys of three words
-constexpr u32 SHORT_LEFT = 2 * SHORT_GENERATIONS; // counter: the number of suffixes that were too many for short_rest_kernel
-constexpr u32 SHORT_COUNTERS = SHORT_LEFT + 1;
+constexpr u32 SHORT_LONG = 2 * SHORT_GENERATIONS; // counter: not zero if a group of generation 1 is longer than that
+constexpr u32 SHORT_COUNTERS = SHORT_LONG + 1;
 
 struct ShortArgs {
     const u16* text;
@@ -72,9 +74,11 @@ __device__ __forceinline__ void short_settle(const ShortArgs& a, u32 x, bool the
         const u32 rank = base + sums[t][0];
         tied = sums[t][1] != 0;
         head = tied && sums[t][2] == 0;
-        a.rank_out[x] = rank | (tied ? SHORT_TIED : 0u);
+        a.rank_out[x] = rank | (tied ? SHORT_TIED | sums[t][2] << SHORT_RANK_BITS : 0u);
         if (!tied)
             short_emit(a, rank, x);
+        if (head && a.generation == 0 && sums[t][1] + 1 > SHORT_GROUP)
+            a.counters[SHORT_LONG] = 1u;
     }
     const u64 all = __ballot(tied), heads = __ballot(head);
     if (t == 0 && all) {
@@ -135,9 +139,9 @@ __global__ __launch_bounds__(SHORT_BLOCK) void short_next_kernel(ShortArgs a)
     if (t < SHORT_X * 3)
         s_sums[t / 3][t % 3] = 0;
     for (u32 y = t; y < a.n; y += SHORT_BLOCK)
-        s_rank[y] = (u16)a.rank_in[y];
+        s_rank[y] = (u16)(a.rank_in[y] & SHORT_RANK);
     __syncthreads();
-    const u32 hop = a.hops[a.generation], rank = own & ~SHORT_TIED;
+    const u32 hop = a.hops[a.generation], rank = own & SHORT_RANK;
     u32 less = 0, equal = 0, before = 0;
     if (there && x + hop < a.n) {
         const u32 next = s_rank[x + hop];
@@ -153,72 +157,108 @@ __global__ __launch_bounds__(SHORT_BLOCK) void short_next_kernel(ShortArgs a)
     short_settle(a, x, there, rank, less, equal, before, s_sums);
 }
 
-// All generations from a.generation on, if at most SHORT_FEW suffixes are tied: one thread for each.
+// All generations from a.generation on, unless a group is longer than SHORT_GROUP. The members of a group stand side by side, at the places
+// that are theirs in the end: a thread owns every SHORT_BLOCK-th place and compares who stands there with the others of the group.
 __global__ __launch_bounds__(SHORT_BLOCK) void short_rest_kernel(ShortArgs a)
 {
+    constexpr int ITEMS = SHORT_MAX / SHORT_BLOCK;
+    constexpr u16 NOBODY = 0xFFFFu;
     __shared__ u16 s_rank[SHORT_MAX];
-    __shared__ u32 s_member[SHORT_FEW];
-    __shared__ __align__(16) u32 s_key[SHORT_FEW];
-    __shared__ u32 s_count, s_tied[2];
-    const u32 t = threadIdx.x, m = a.counters[2 * a.generation];
-    if (m == 0 || m > SHORT_FEW) {
-        if (t == 0)
-            a.counters[SHORT_LEFT] = m;
+    __shared__ u16 s_member[SHORT_MAX];
+    __shared__ u16 s_next[SHORT_MAX]; // the rank that is compared
+    __shared__ u16 s_end[SHORT_MAX];  // of the group that stands here
+    __shared__ u32 s_tied[2];
+    const u32 t = threadIdx.x;
+    if (a.counters[2 * a.generation] == 0 || a.counters[SHORT_LONG] != 0)
         return;
+    for (u32 y = t; y < a.n; y += SHORT_BLOCK) {
+        s_member[y] = NOBODY;
+        s_end[y] = 0;
     }
-    if (t == 0)
-        s_count = 0;
     __syncthreads();
     for (u32 y = t; y < a.n; y += SHORT_BLOCK) {
-        const u32 r = a.rank_in[y];
-        s_rank[y] = (u16)r;
-        if (r & SHORT_TIED) {
-            const u32 at = atomicAdd(&s_count, 1u);
-            if (at < SHORT_FEW)
-                s_member[at] = y;
-        }
+        const u32 v = a.rank_in[y], rank = v & SHORT_RANK, before = (v >> SHORT_RANK_BITS) & SHORT_RANK;
+        s_rank[y] = (u16)rank;
+        if ((v & SHORT_TIED) && rank + before < a.n)
+            s_member[rank + before] = (u16)y;
     }
     __syncthreads();
-    const bool member = t < m && t < s_count;
-    const u32 x = member ? s_member[t] : 0u;
-    u32 rank = member ? s_rank[x] : 0u;
-    bool tied = member;
+    // ends of the groups: the place behind a member whose right neighbour is of another group, or nobody
+    for (u32 j = t; j < a.n; j += SHORT_BLOCK) {
+        const u32 x = s_member[j];
+        if (x == NOBODY)
+            continue;
+        u32 end = j + 1;
+        while (end < a.n && s_member[end] != NOBODY && s_rank[s_member[end]] == s_rank[x])
+            ++end;
+        s_end[j] = (u16)end;
+    }
     for (u32 g = a.generation; g < SHORT_GENERATIONS - 1 && a.hops[g] != 0; ++g) {
         const u32 hop = a.hops[g];
-        // (ranks are below 2^13: no key of a tied suffix is all ones)
-        if (t < SHORT_FEW)
-            s_key[t] = tied && x + hop < a.n ? rank << 16 | s_rank[x + hop] : 0xFFFFFFFFu;
+        u32 x[ITEMS], to[ITEMS], end[ITEMS]; // who stands at the thread's places; the new place and end of group
+        __syncthreads();
         if (t < 2)
             s_tied[t] = 0;
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const u32 j = k * SHORT_BLOCK + t;
+            x[k] = j < a.n ? s_member[j] : (u32)NOBODY;
+            to[k] = end[k] = 0;
+            if (x[k] != NOBODY && x[k] + hop < a.n) // (nobody who is tied runs off the text)
+                s_next[j] = s_rank[x[k] + hop];
+        }
         __syncthreads();
-        u32 less = 0, equal = 0, before = 0;
-        if (tied) {
-            const u32 key = s_key[t], first = rank << 16;
-            for (u32 i = 0; i < m; ++i) {
-                const u32 v = s_key[i];
-                less += v >= first && v < key ? 1u : 0u;
-                equal += v == key ? 1u : 0u;
-                before += v == key && i < t ? 1u : 0u;
+        u32 tied = 0, heads = 0;
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            if (x[k] == NOBODY)
+                continue;
+            const u32 j = k * SHORT_BLOCK + t, first = s_rank[x[k]], last = s_end[j], mine = s_next[j];
+            u32 less = 0, equal = 0, before = 0;
+            for (u32 i = first; i < last; ++i) {
+                const u32 v = s_next[i];
+                less += v < mine ? 1u : 0u;
+                equal += v == mine ? 1u : 0u;
+                before += v == mine && i < j ? 1u : 0u;
             }
-            rank += less;
-            tied = equal > 1;
-            if (!tied)
-                short_emit(a, rank, x);
+            to[k] = first + less + before;
+            end[k] = first + less + equal;
+            tied += equal > 1 ? 1u : 0u;
+            heads += equal > 1 && before == 0 ? 1u : 0u;
+            if (equal == 1)
+                short_emit(a, to[k], x[k]);
+            x[k] |= (first + less) << 16; // the new rank
+            end[k] |= equal > 1 ? 0u : 0x10000u;
         }
-        const u64 all = __ballot(tied), heads = __ballot(tied && before == 0);
-        if ((t & 63u) == 0 && all) {
-            atomicAdd(&s_tied[0], (u32)__popcll(all));
-            atomicAdd(&s_tied[1], (u32)__popcll(heads));
+        const u32 all_tied = wave_reduce_sum(tied), all_heads = wave_reduce_sum(heads);
+        if ((t & 63u) == 0 && all_tied) {
+            atomicAdd(&s_tied[0], all_tied);
+            atomicAdd(&s_tied[1], all_heads);
         }
-        if (member)
-            s_rank[x] = (u16)rank; // (all ranks at x + hop have been read)
         __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const u32 j = k * SHORT_BLOCK + t;
+            if (x[k] != NOBODY)
+                s_member[j] = NOBODY;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            if (x[k] == NOBODY)
+                continue;
+            const u32 who = x[k] & 0xFFFFu;
+            s_rank[who] = (u16)(x[k] >> 16);
+            if (!(end[k] & 0x10000u)) {
+                s_member[to[k]] = (u16)who;
+                s_end[to[k]] = (u16)end[k];
+            }
+        }
         const u32 left = s_tied[0];
         if (t < 2)
             a.counters[2 * (g + 1) + t] = s_tied[t];
         if (left == 0)
             break;
-        __syncthreads(); // (the sums are cleared by the next round)
     }
 }
 
