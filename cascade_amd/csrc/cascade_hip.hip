@@ -909,6 +909,7 @@ bool dense_generation(u32 m, u32 groups, u32 n)
 struct PackedPlan {
     bool enabled;
     bool byte_wide; // the symbols differ in one of their bytes only: half the passes over K-gram keys have nothing to do
+    bool few;       // few_symbols
     SymbolCodes codes;
     u32 skipped; // j
 };
@@ -926,6 +927,7 @@ PackedPlan plan_packed_text(const u32* bytehist, u32 n, int key_words, u64 room_
     }
     const u32 codes = nlo * nhi;
     pp.byte_wide = nlo == 1 || nhi == 1;
+    pp.few = few_symbols(nlo, nhi);
     if (codes > 256)
         return pp;
     const u32 b = codes <= 2 ? 1u : codes <= 4 ? 2u : codes <= 16 ? 4u : 8u;
@@ -976,7 +978,8 @@ CodeTables code_tables(const csa_handle* h)
 // What a sort by codes starts from: the shares of the symbols, and for texts of PROBE_MIN symbols or more what a sample of the suffixes
 // (probed_suffixes) shows about shared codes, on its way to *seen; ev_gen[1] tells that it is there. A large sample's table is
 // key[0], which holds nothing yet.
-int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
+// bytehist: see sample_symbols_kernel. counts[5], zeroed, says that the text was left alone.
+int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen, const u32* bytehist)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -995,6 +998,7 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
         const u32 long_run = RESOLVE_MAX * 9 / 8 / (n / a.taken);
         a.long_from = long_run > 2 ? long_run : 2;
         a.counts = c.probe;
+        a.skipped = h->counts + 5;
         const bool few = a.taken <= PROBE_FEW;
         a.table = few ? c.table : reinterpret_cast<unsigned long long*>(h->key[0]);
         zeros += sizeof(ProbeCounts);
@@ -1011,10 +1015,10 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen)
     const u64 sampled = (u64)taken * SAMPLE_CHUNK < n ? (u64)taken * SAMPLE_CHUNK : (u64)n;
     const u32 per_block = sample_chunks_per_block(taken);
     hipLaunchKernelGGL(sample_symbols_kernel, dim3((taken + per_block - 1) / per_block), dim3(SAMPLE_BLOCK), 0, s, d_text, n, chunks, taken,
-                       c.counts);
+                       c.counts, bytehist, h->counts + 5);
     const int weight_log2 = SAMPLE_LOG2 - bit_length(sampled - 1);
     hipLaunchKernelGGL(symbol_shares_kernel, dim3(SYMBOLS / SHARES_TILE), dim3(SHARES_TILE), 0, s, (const u32*)c.counts, weight_log2,
-                       (u32)((sampled << weight_log2) + SYMBOLS), c.cum);
+                       (u32)((sampled << weight_log2) + SYMBOLS), c.cum, (const u32*)(h->counts + 5));
     if (n >= PROBE_MIN) {
         hipLaunchKernelGGL(probe_codes_kernel, dim3((a.taken + PROBE_BLOCK - 1) / PROBE_BLOCK), dim3(PROBE_BLOCK), 0, s, a);
         const int rc = move_table(seen, a.counts, sizeof(ProbeCounts), s);
@@ -1689,15 +1693,27 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     u32* const bytehist = h->ghist + MAX_PASSES * RADIX_BINS;
     PackedPlan pp;
     memset(&pp, 0, sizeof(pp));
+    // A workgroup for every 8 K symbols until there is one per CU (10^6 symbols: 12.5 us with 31 of them, 7.3 with 123), then for every
+    // 32 K: more of them add the same counters more often (2 * 10^7 symbols: 1 % of the sort).
+    u32 count_blocks = hist_blocks(256 * 2 * 16, n);
+    count_blocks = count_blocks < 256u ? count_blocks : 256u;
+    if (hist_blocks(256 * 8 * 16, n) > count_blocks)
+        count_blocks = hist_blocks(256 * 8 * 16, n);
     auto count_bytes = [&] {
-        hipLaunchKernelGGL(text_byte_hist_kernel, dim3(hist_blocks(256 * 8 * 16, n)), dim3(256), 0, s, d_text, n, bytehist);
+        hipLaunchKernelGGL(text_byte_hist_kernel, dim3(count_blocks), dim3(256), 0, s, d_text, n, bytehist);
     };
+    ProbeCounts* const seen = reinterpret_cast<ProbeCounts*>(h->h_pinned + PINNED_HIST + 2 * RADIX_BINS); // (behind the byte counts)
     if (h->pack_symbols) {
         count_bytes();
         u32* h_bytes = h->h_pinned + PINNED_HIST;
         if ((rc = move_table(h_bytes, bytehist, 2 * RADIX_BINS * sizeof(u32), s)) != CSA_OK)
             return rc;
-        HIP_TRY(hipStreamSynchronize(s));
+        // The symbols are sampled meanwhile: the device would stand still until the host has seen the counts, and then start with that.
+        // (10^6 independent ids: 238 us with a wait in between, 226 without.)
+        HIP_TRY(hipEventRecord(h->ev_gen[2], s)); // (recorded again when a generation ends)
+        if ((rc = share_symbols(L, d_text, n, seen, bytehist)) != CSA_OK)
+            return rc;
+        HIP_TRY(hipEventSynchronize(h->ev_gen[2]));
         pp = plan_packed_text(h_bytes, n, h->key_words, (u64)h->cap * sizeof(u32));
     }
     TextSource ps;
@@ -1727,8 +1743,11 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     bool coded = !pp.enabled && !pp.byte_wide;
     if (coded) {
         const bool probed = n >= PROBE_MIN, ahead = !probed || n < CODE_AHEAD_MAX;
-        ProbeCounts* const seen = reinterpret_cast<ProbeCounts*>(h->h_pinned + PINNED_HIST);
-        if ((rc = share_symbols(L, d_text, n, seen)) != CSA_OK || (ahead && (rc = code_suffixes(L, d_text, n, tail)) != CSA_OK))
+        if (!h->pack_symbols || pp.few) { // (few symbols, and no packed keys for them)
+            if ((rc = move_table(h->counts + 5, nullptr, sizeof(u32), s)) != CSA_OK || (rc = share_symbols(L, d_text, n, seen, nullptr)) != CSA_OK)
+                return rc;
+        }
+        if (ahead && (rc = code_suffixes(L, d_text, n, tail)) != CSA_OK)
             return rc;
         if (probed) {
             HIP_TRY(hipEventSynchronize(h->ev_gen[1]));
@@ -1749,7 +1768,11 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         HIP_TRY(hipGetLastError());
         coded = narrow;
         if (narrow) {
-            HIP_TRY(hipMemsetAsync(code_tables(h).marks, 0, RESOLVE_MARK_WORDS * sizeof(u32), s));
+            TableGroup cleared = {};
+            add_table(cleared, code_tables(h).marks, nullptr, RESOLVE_MARK_WORDS * sizeof(u32));
+            add_table(cleared, h->counts + 5, nullptr, sizeof(u32)); // (the sampling of the symbols has been called off with it)
+            if ((rc = move_tables(cleared, s)) != CSA_OK)
+                return rc;
             rc = sort_by_codes(L, d_text, n, tail, 2u, list, &ps, ell);
             p1 = CODE_PASSES;
             in_out = 1;

@@ -63,11 +63,43 @@ __device__ __forceinline__ u32 sampled_chunk(u32 c, u32 chunks, u32 taken, u32 s
 // 11, 14, 18, 2^23 17, 17, 20, 2^25 24, 23, 32; independent ids 2^20 12, 15, 18, 2^23 36, 31, 29, 2^25 54, 44, 40.
 __host__ __device__ __forceinline__ u32 sample_chunks_per_block(u32 taken) { return taken < SAMPLE_CHUNKS_WIDE ? 64u : 128u; }
 
-// counts[s] += occurrences of symbol s in the sample: `taken` chunks (all of them when the text is short).
+// Whether a text with these byte counts is one that codes are not for: few enough symbols for packed keys, or symbols that differ in one
+// byte alone (plan_packed_text has the last word).
+__host__ __device__ __forceinline__ bool few_symbols(u32 nlo, u32 nhi) { return nlo * nhi <= 256u || nlo == 1u || nhi == 1u; }
+
+// The different low and high bytes of a text (zero, the padding, counted in) for every thread of a workgroup of 512 or more.
+__device__ __forceinline__ void count_different_bytes(const u32* __restrict__ bytehist, u32 (&s_different)[2], u32& nlo, u32& nhi)
+{
+    const u32 t = threadIdx.x;
+    if (t < 2)
+        s_different[t] = 0;
+    __syncthreads();
+    if (t < 512) {
+        const u64 b = __ballot((t & 255u) == 0 || bytehist[t] != 0);
+        if ((t & 63u) == 0)
+            atomicAdd(&s_different[t / 256u], (u32)__popcll(b));
+    }
+    __syncthreads();
+    nlo = s_different[0];
+    nhi = s_different[1];
+}
+
+// counts[s] += occurrences of symbol s in the sample: `taken` chunks (all of them when the text is short). bytehist: non-null if the host has
+// not seen the byte counts yet; a text that will not be sorted by codes is left alone then, and *skipped is set.
 __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16* __restrict__ text, u32 n, u32 chunks, u32 taken,
-                                                                      u32* __restrict__ counts)
+                                                                      u32* __restrict__ counts, const u32* __restrict__ bytehist, u32* skipped)
 {
     __shared__ u32 s_cnt[SYMBOLS / 2]; // two 16-bit counters per word
+    __shared__ u32 s_different[2];
+    if (bytehist) {
+        u32 nlo, nhi;
+        count_different_bytes(bytehist, s_different, nlo, nhi);
+        if (few_symbols(nlo, nhi)) {
+            if (blockIdx.x == 0 && threadIdx.x == 0)
+                *skipped = 1u;
+            return;
+        }
+    }
     const u32 t = threadIdx.x;
     for (u32 i = t; i < (u32)SYMBOLS / 2; i += SAMPLE_BLOCK)
         s_cnt[i] = 0;
@@ -101,9 +133,12 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_symbols_kernel(const u16*
 // coalesced rounds over a table in the L2), which takes a third of the time of one workgroup that scans them all (18 us).
 constexpr int SHARES_TILE = 1024;
 
-__global__ __launch_bounds__(SHARES_TILE) void symbol_shares_kernel(const u32* __restrict__ counts, int weight_log2, u32 total, u32* __restrict__ cum)
+__global__ __launch_bounds__(SHARES_TILE) void symbol_shares_kernel(const u32* __restrict__ counts, int weight_log2, u32 total, u32* __restrict__ cum,
+                                                                    const u32* __restrict__ skipped)
 {
     __shared__ u32 s_sum[16], s_own[16];
+    if (*skipped)
+        return;
     const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6;
     const u32 first = blockIdx.x * SHARES_TILE;
     u32 earlier = 0;
@@ -175,6 +210,7 @@ struct ProbeArgs {
     ProbeCounts* counts; // zeroed
     const u32* stream;   // non-null: the codes are the narrow keys of a packed text, sym_bits bits a symbol; `crowded` counts whoever
     u32 sym_bits;        // finds its code taken by long_from others or more, its own string as they are
+    const u32* skipped;  // non-null: nothing is looked at if it is set
 };
 
 // An entry of the table is a code (high half), eight bits of the first string's hash and the number of suffixes that came.
@@ -183,6 +219,8 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
 {
     __shared__ unsigned long long s_pairs[PROBE_BLOCK / WAVE];
     __shared__ u32 s_cnt[6];
+    if (a.skipped && *a.skipped)
+        return;
     const u32 t = threadIdx.x;
     if (t < 6)
         s_cnt[t] = 0;

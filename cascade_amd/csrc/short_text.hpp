@@ -9,7 +9,7 @@
 //   short_rest_kernel    all later ones, in one workgroup, if no group is long (nearly every text)
 //   short_next_kernel    one later generation, over the whole device, otherwise
 // A suffix leaves for its place in the output in the generation that finds it alone.
-// 4096 Zipf tokens: 39 us a sort, 158 the long way.
+// 4096 Zipf tokens, no copies among them: 39 us a sort, 158 the long way; with copies 76 and 447.
 #pragma once
 
 #include "device_utils.hpp"
@@ -18,8 +18,8 @@
 namespace csa {
 
 constexpr int SHORT_BLOCK = 1024;
-constexpr u32 SHORT_MAX = 8192;  // the keys of a text take 64 KB of LDS (us a sort of that length, and the long way: tokens 218 and 399, runs 265 and 746,
-                                 // bytes 172 and 302, four letters 268 and 375)
+constexpr u32 SHORT_MAX = 8192;  // the keys of a text take 64 KB of LDS (us a sort of that length, and the long way: tokens 103 and 427, runs 336 and 776,
+                                 // bytes 174 and 314, four letters 171 and 391)
 constexpr u32 SHORT_X = 16;      // suffixes of a workgroup, each compared with the others by ...
 constexpr u32 SHORT_SLICES = SHORT_BLOCK / SHORT_X; // ... so many threads
 constexpr u32 SHORT_GROUP = 256; // members of the longest group that one workgroup takes to the end (each looks at all others)
