@@ -710,6 +710,51 @@ __global__ __launch_bounds__(256) void scatter_ranks_kernel(const u32* __restric
     }
 }
 
+// Where the pairs of each window of 1 << window_log2 positions start in a list sorted by window: starts[0 .. windows].
+__global__ __launch_bounds__(256) void window_starts_kernel(const u32* __restrict__ pos, u32 m, int window_log2, u32 windows, u32* __restrict__ starts)
+{
+    const u64 c = (u64)blockIdx.x * 256 + threadIdx.x;
+    if (c >= m)
+        return;
+    const u32 own = pos[c] >> window_log2, mine = own < windows ? own : windows - 1;
+    const u32 next = c == 0 ? 0u : (pos[c - 1] >> window_log2) + 1u; // the first window that has not started before
+    for (u32 w = next; w <= mine; ++w)
+        starts[w] = (u32)c;
+    if (c + 1 == m)
+        for (u32 w = mine + 1; w <= windows; ++w)
+            starts[w] = m;
+}
+
+// A window of rank[] brought up to date: read into LDS, overwritten by the window's pairs in any order, and written back in full lines.
+template <int MAX_LOG2>
+__global__ __launch_bounds__(1024) void place_window_kernel(const u32* __restrict__ pos, const u32* __restrict__ val, const u32* __restrict__ starts,
+                                                            u32 n, int window_log2, u32* __restrict__ rank, u32* err)
+{
+    __shared__ u32 s_win[1 << MAX_LOG2];
+    const u32 from = starts[blockIdx.x], to = starts[blockIdx.x + 1];
+    if (from >= to)
+        return;
+    const u32 S = 1u << window_log2;
+    const u64 first = (u64)blockIdx.x << window_log2;
+    const u32 count = (u32)((u64)n - first < S ? (u64)n - first : S);
+    for (u32 i = threadIdx.x; i < count; i += 1024)
+        s_win[i] = rank[first + i];
+    __syncthreads();
+    for (u32 i = from + threadIdx.x; i < to; i += 1024) {
+        const u32 v = val[i];
+        if (v != NO_RANK) {
+            const u32 off = pos[i] - (u32)first;
+            if (off < count && v < n)
+                s_win[off] = v;
+            else
+                atomicExch(err, DEV_ERR_RERANK_RANGE);
+        }
+    }
+    __syncthreads();
+    for (u32 i = threadIdx.x; i < count; i += 1024)
+        rank[first + i] = s_win[i];
+}
+
 // ---------------------------------------------------------------------------------------------
 // Generation t >= 1: gather rank[x + h], and sort inside every small group in the same pass.
 //
