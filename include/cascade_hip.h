@@ -71,11 +71,16 @@ typedef struct csa_stats {
                                                 list, as in runs of one token and periodic stretches) */
     uint32_t key_symbols;            /* symbols in the keys of the first sort: 4 (by 32-bit codes of them, or by K-gram words where
                                         too many suffixes would share a code), or up to 64 when the text's alphabet is small
-                                        enough for packed codes of 1, 2, 4 or 8 bits. A sort by codes goes on to resolve the
+                                        enough for packed codes of 1, 2, 4 or 8 bits (more than 2^24 symbols of two bits are sorted
+                                        by 16 of them, with the next 16 read where those tie: 32 all the same, or 16 where
+                                        runs were too long for it). A sort by codes goes on to resolve the
                                         next four symbols from the text: generation 1 is then reported with the list it would
                                         have had, the members of long runs in big[1], their passes in passes[1], and no time.
                                         So are the generations of a list of short groups whose ties come from copied passages,
-                                        which are settled at once without ranks (rank_update[0] is 0 then) */
+                                        which are settled at once without ranks (rank_update[0] is 0 then), and those after the
+                                        first of a list of runs and periods, which is settled at once as well (big[] and presorted[]
+                                        as the generations would have had them). Texts of up to 8192 symbols are ranked by counting:
+                                        no passes, all time in ms[0], and 4 here whatever the alphabet */
     uint32_t first_sort_generations; /* generations of the reference that sort stands for: 1, or 1 + j when its keys held
                                         4 * key_words * 2^j symbols. Generations 1 .. j are then reported with the lists
                                         they would have had (active[], groups[]) and with no time or passes of their own */
@@ -143,7 +148,8 @@ int csa_set_device_exclusive(csa_handle* h, int exclusive);
  *                                (default 2^23 suffixes)
  *   CSA_TUNE_WINDOW_MIN_CHANGED  fewest changed ranks for the windowed update of later generations (default 2^22;
  *                                0xFFFFFFFF: never)
- *                                Setting either threshold also keeps lists of short groups from being settled without ranks
+ *                                Setting either threshold also keeps lists of short groups, and of runs and periods, from being
+ *                                settled without ranks, and short texts from being ranked by counting
  *   CSA_TUNE_XCD_CHUNK           tiles (of 8192 pairs) that one XCD takes in a row under csa_set_device_exclusive
  *                                (default 16; 0: the exclusive order is the default order); call before
  *                                csa_set_device_exclusive. 8 chunks of that many workgroups must be resident
@@ -151,12 +157,13 @@ int csa_set_device_exclusive(csa_handle* h, int exclusive);
  *   CSA_TUNE_PACK_SYMBOLS        1 (default): a text whose symbols take at most 256 values (by the values its low and its
  *                                high bytes take) is sorted first on keys of as many packed symbols as 64 bits hold, which
  *                                covers the first generations of the doubling (csa_stats.first_sort_generations), and a sort
- *                                by codes resolves eight symbols, and lists of short groups are settled without ranks; 0: the
+ *                                by codes resolves eight symbols, lists of short groups and of runs and periods are settled without
+ *                                ranks, and texts of up to 8192 symbols are ranked by counting; 0: the
  *                                first sort always resolves four symbols, and the doubling does the rest
  *   CSA_TUNE_EXPECT_PRESORTED    0 (default): a generation leaves out the (key, suffix) pairs of its large groups' radix sort
  *                                when every large group of the generation before was in order as it stood (csa_stats.presorted),
  *                                and gathers again with them if this one's are not; 1: every generation starts that way
- *                                (tests of the second gather)
+ *                                (tests of the second gather), and short texts are sorted like long ones
  * No counterpart in the reference. */
 enum {
     CSA_TUNE_DEFER_MIN = 0,
