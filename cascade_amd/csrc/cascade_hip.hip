@@ -1368,8 +1368,13 @@ struct Settle {
 
 // Whether it is tried: a failed attempt costs the comparison of every member with its group's root, which is what a generation of the doubling
 // costs too. A list of copies has two or three members to a group; long groups are runs and periods, whose members agree with
-// their neighbours and not with their group's root, or short strings that are in the text a hundred times.
-constexpr u32 SETTLE_AVG_LIMIT = 4;
+// their neighbours and not with their group's root, or short strings that are in the text a hundred times: members that differ from the root
+// in the same way are compared with each other one by one, and one such group holds up a short text. (Written text, us a sort settled / doubled: 20000
+// symbols, 3.5 members to a group on average, 395 / 381; 33000, 3.9, 665 / 391; 12000 349 / 376. Token and four-letter texts with copies average 2.0 to 2.3.)
+#ifndef CSA_SETTLE_AVG
+#define CSA_SETTLE_AVG 3
+#endif
+constexpr u32 SETTLE_AVG_LIMIT = CSA_SETTLE_AVG;
 
 // Works in key[2] (the anchors' records and bits: two bytes per suffix at most) and the symbol counts of the first sort.
 int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups)
