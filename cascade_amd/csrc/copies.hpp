@@ -19,7 +19,9 @@
 // of their own past that. The agreement of neighbours gives the generation in which the doubling would have told them apart, and
 // with it the sizes of its lists.
 // Every comparison has a limit; a group that runs into it, or is longer than SETTLE_MAX, raises a flag, and the sort goes on by doubling from
-// where it was (nothing it needs has changed but the order inside groups).
+// where it was. All that has changed by then is the order inside the groups of tiles that were settled: a tile with a comparison that came
+// to nothing writes none of its groups. (Comparisons that did and places in the list where they did not are no order together:
+// with y before x by the text, x before z and z before y by their places, all three would go to one place.)
 #pragma once
 
 #include "device_utils.hpp"
@@ -315,9 +317,12 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
     __shared__ u64 s_key[SPAN];
     __shared__ u32 s_suf[SPAN];
     __shared__ u32 s_tally[TALLIES * COPIES];
+    __shared__ u32 s_failed; // some members of the tile could not be told apart
     const u32 t = threadIdx.x;
     for (u32 i = t; i < TALLIES * COPIES; i += BLOCK)
         s_tally[i] = 0;
+    if (t == 0)
+        s_failed = 0;
     const u64 t0 = (u64)blockIdx.x * TILE;
     u32 x[ITEMS], place[ITEMS];
     int from[ITEMS], to[ITEMS]; // the group, by places of the span; to = 0: nothing to do
@@ -373,7 +378,7 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         if (root != x[k]) {
             const Agreement w = agreement(a, root, x[k], a.ctx);
             if (!w.found)
-                *a.failed = 1u;
+                s_failed = 1u;
             const u64 next = (u64)x[k] + w.length;
             const u64 symbol = to[k] - from[k] > 2 && next < a.n ? (u64)a.text[next] + 1u : 0u; // (a pair has nobody else to be told from)
             key[k] = w.larger ? LARGER | ((FAR - w.length) << 17) | symbol : ((u64)w.length << 17) | symbol;
@@ -400,17 +405,19 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
             } else if (w == key[k] && i != j) {
                 const u32 y = s_suf[i];
                 const Agreement v = further(x[k], y, w);
-                if (!v.found) {
-                    *a.failed = 1u;
-                    before += i < j ? 1u : 0u; // (the members stay a permutation of themselves)
-                } else {
-                    before += (y < x[k]) == v.larger ? 1u : 0u;
-                }
+                if (!v.found)
+                    s_failed = 1u;
+                before += (y < x[k]) == v.larger ? 1u : 0u;
             }
         }
         place[k] = (u32)from[k] + before;
     }
     __syncthreads();
+    if (s_failed) { // (the same for all threads: nobody sets it past the barrier)
+        if (t == 0)
+            *a.failed = 1u;
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k)
         if (to[k] != 0) {

@@ -876,3 +876,30 @@ def test_copies_that_cannot_be_settled_are_left_to_the_doubling(symbols, key_wor
     assert emu_sort.rank_update[0] == 1 and len(active) > 3
     sa, counts = oracle_lib.prefix_doubling(T, key_words)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
+@pytest.mark.parametrize("length", [1500, 2500, 4000])
+def test_groups_of_which_some_members_are_told_apart_and_some_are_not(emu_dev, length):
+    """Three copies of a passage whose comparisons run into their limit (from 2500 symbols on) for some pairs of a group, while records
+    tell the others apart: the sort goes on by doubling, from a list that still holds every suffix once."""
+    T = texts.text_of_undecided_copies(length)
+    got, active, _ = emu_sort(emu_dev, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
+@pytest.mark.parametrize("symbols,key_words", [(60000, 1), (60000, 4), (256, 1), (4, 1), (2, 1)])
+def test_copies_of_which_some_are_left_to_the_doubling(symbols, key_words):
+    """A build in which a comparison of copies gives up after two steps: of many texts some are settled and some doubled, and in those that
+    are doubled some pairs of a group had been told apart and others not."""
+    lib = load_emulation("libcascade_emu_few.so")
+    doubled = settled = 0
+    for seed in range(24):
+        T = texts.text_of_copies(1600 + 40 * seed, symbols, 1000 * seed + symbols + key_words)
+        got, active, _ = emu_sort(lib, T, key_words)
+        sa, counts = oracle_lib.prefix_doubling(T, key_words)
+        assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts, seed
+        if len(active) > 1:
+            doubled += emu_sort.rank_update[0] != 0
+            settled += emu_sort.rank_update[0] == 0
+    assert doubled >= 2 and settled >= 2, (doubled, settled)

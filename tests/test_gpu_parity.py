@@ -837,3 +837,17 @@ def test_ties_of_copied_passages_are_settled_by_where_the_copies_end(torch_mod, 
         s.set_tuning(_native.CSA_TUNE_WINDOW_MIN_CHANGED, 1 << 22)
         assert torch_mod.equal(s.sort(d), out)
         assert settled["active"] == s.last_stats["active"] and settled["groups"] == s.last_stats["groups"]
+
+
+@pytest.mark.parametrize("length", [1500, 4000])
+def test_groups_of_which_some_members_are_told_apart_and_some_are_not(torch_mod, length):
+    """Three copies of a passage some pairs of which take more steps to compare than one comparison is given (from 2500 symbols on), while
+    records tell the others apart: such a tile writes nothing, and the sort goes on by doubling. Suffix array and generation sizes are the oracle's."""
+    from cascade_amd import PartitionSorter
+    T = texts.text_of_undecided_copies(length)
+    with PartitionSorter(T.size, key_words=1) as s:
+        print(f"  undecided copies {length}", flush=True)
+        got = gpu_sa40(torch_mod, s, T)
+        stats = s.last_stats
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts

@@ -189,3 +189,24 @@ def chains_text(kind, n):
 
 
 CHAINS = ["rising", "falling", "two runs", "period", "mixed", "long period", "end", "period at the end"]
+
+
+def text_of_undecided_copies(length):
+    """A passage of `length` symbols three times, at residues 0, 4 and 0 modulo 8, the first eight symbols from each of its places 4, 12, 20, ...
+    on once more in front of it, and an unrelated passage twice (so that groups have fewer than three members on average).
+    In a sort that settles copies from anchors eight symbols apart, some pairs of the passage's copies are told apart by one record;
+    for others every anchor says eight symbols and no more, and a comparison goes through the whole passage step by step."""
+    rng = np.random.default_rng(length)
+    M = rng.integers(100, 60000, length).astype(np.uint16)
+    twice = rng.integers(100, 60000, 4000).astype(np.uint16)
+    parts = []
+    for o in range(4, length - 8, 8):
+        parts += [M[o:o + 8], rng.integers(100, 60000, 3).astype(np.uint16)]
+    at = sum(p.size for p in parts)
+    for residue, end in ((0, 50), (4, 40), (0, 30)):
+        gap = rng.integers(100, 60000, (residue - at) % 8).astype(np.uint16)
+        parts += [gap, M, np.array([end], dtype=np.uint16)]
+        at += gap.size + length + 1
+    for _ in range(2):
+        parts += [rng.integers(100, 60000, 20).astype(np.uint16), twice]
+    return np.concatenate(parts + [rng.integers(100, 60000, 20).astype(np.uint16)])
