@@ -1366,11 +1366,13 @@ struct Settle {
     u64 active[SETTLE_CONTEXTS], groups[SETTLE_CONTEXTS];
 };
 
-// Whether it is tried: a failed attempt costs the comparison of every member with its group's root, which is what a generation of the doubling
-// costs too. A list of copies has two or three members to a group; long groups are runs and periods, whose members agree with
+// Whether it is tried. A failed attempt costs the list, the anchors' records and as many steps of a member as SETTLE_STEPS lets it take before
+// its tile gives up, and no more for the tiles that start after that: 0.15 to 0.9 ms on texts of 10^4 to 3 * 10^6 symbols made for it.
+// A list of copies has two or three members to a group; long groups are runs and periods, whose members agree with
 // their neighbours and not with their group's root, or short strings that are in the text a hundred times: members that differ from the root
-// in the same way are compared with each other one by one, and one such group holds up a short text. (Written text, us a sort settled / doubled: 20000
-// symbols, 3.5 members to a group on average, 395 / 381; 33000, 3.9, 665 / 391; 12000 349 / 376. Token and four-letter texts with copies average 2.0 to 2.3.)
+// in the same way are compared with each other one by one, and one such group holds up a short text. (Written text, us of
+// the device a sort settled / doubled: 12000 symbols 316 / 288, 20000, 3.5 members to a group on average, 362 / 292, 33000, 3.9, 635 / 307.
+// Token and four-letter texts with copies average 2.0 to 2.3.)
 #ifndef CSA_SETTLE_AVG
 #define CSA_SETTLE_AVG 3
 #endif

@@ -42,9 +42,14 @@ constexpr u64 NO_RECORD = ~0ull, OPEN = 1ull << 63; // (positions are below 2^31
 #endif
 constexpr u32 SETTLE_ENDS = CSA_SETTLE_ENDS; // anchors that an end looks ahead
 #ifndef CSA_SETTLE_STEPS
-#define CSA_SETTLE_STEPS 256
+#define CSA_SETTLE_STEPS 32
 #endif
-constexpr u32 SETTLE_STEPS = CSA_SETTLE_STEPS; // records and stretches between anchors that a comparison goes through
+// Steps (records, and stretches between anchors) of a member's comparison with its root, and of its comparisons with the members of its
+// key past the first two of each, together. Texts with copies take 13 at most (4e8 letters, a fifth of them copies), and groups of 250
+// members, a hundred of which go on alike, one or two a comparison. Passages whose anchors say little take as many as they are long: ms a
+// sort with 256 steps for every comparison, with these limits, and doubled: 12437 symbols, 125 steps, 1.97, 0.68, 0.50; 2.9 M symbols, 187
+// steps, 4.0, 1.5, 1.1; a group of 250, 20 steps a comparison, 174304 symbols, 8.5, 2.0, 1.1, and worse the longer the passage.
+constexpr u32 SETTLE_STEPS = CSA_SETTLE_STEPS;
 constexpr int LINK_TILE = 64 * 64;           // anchors of a workgroup of the link kernel: one word of the first summary
 
 struct SettleArgs {
@@ -151,13 +156,14 @@ __device__ __forceinline__ u32 chain_end(const SettleArgs& a, u32 i)
 __device__ __forceinline__ u32 root_of(u64 record) { return (u32)(record >> 32) & 0x7FFFFFFFu; }
 __device__ __forceinline__ u32 length_of(u64 record) { return (u32)record >> 1; }
 
-// How far suffixes r < y agree, which are tied on their first `tied` >= ctx symbols.
-__device__ __forceinline__ Agreement agreement(const SettleArgs& a, u32 r, u32 y, u32 tied)
+// How far suffixes r < y agree, which are tied on their first `tied` >= ctx symbols; takes its steps from steps_left.
+__device__ __forceinline__ Agreement agreement(const SettleArgs& a, u32 r, u32 y, u32 tied, u32& steps_left)
 {
     Agreement out = {tied, false, false};
     u64 off = tied;
     const u32 gap = 1u << a.log2_gap;
-    for (u32 step = 0; step < SETTLE_STEPS; ++step) {
+    while (steps_left > 0) {
+        --steps_left;
         const u64 reach = (u64)y + off;
         const u32 i = (u32)((reach < a.n ? reach : (u64)a.n) >> a.log2_gap); // the last anchor up to which they are known to agree
         u32 shift = (i << a.log2_gap) - y;                                  // (tied >= ctx >= gap: it lies at y or after it)
@@ -240,6 +246,8 @@ __global__ __launch_bounds__(1024) void copy_links_kernel(SettleArgs a)
     __shared__ unsigned long long s_word[LINK_TILE / 64];
     const u32 t = threadIdx.x, gap = 1u << a.log2_gap;
     const u32 first = blockIdx.x * LINK_TILE;
+    if (*a.failed) // (set by the kernel before, if at all)
+        return;
     for (u32 k = 0; k < LINK_TILE; k += 1024) {
         const u32 i = first + k + t;
         // (an end only ever changes the lower half of a record, so the roots can be read meanwhile)
@@ -296,7 +304,7 @@ __global__ __launch_bounds__(256) void copy_links_top_kernel(SettleArgs a)
 __global__ __launch_bounds__(256) void copy_spread_kernel(SettleArgs a)
 {
     const u32 i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= a.anchors || !((a.links[0][i / 64] >> (i & 63u)) & 1ull))
+    if (i >= a.anchors || *a.failed || !((a.links[0][i / 64] >> (i & 63u)) & 1ull))
         return;
     const u32 end = chain_end(a, i);
     const u64 record = a.records[end];
@@ -317,12 +325,15 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
     __shared__ u64 s_key[SPAN];
     __shared__ u32 s_suf[SPAN];
     __shared__ u32 s_tally[TALLIES * COPIES];
-    __shared__ u32 s_failed; // some members of the tile could not be told apart
+    __shared__ u32 s_over;   // a tile before has given up
+    __shared__ u32 s_lost[2]; // some member of the tile could not be compared with its root; two members with each other
     const u32 t = threadIdx.x;
     for (u32 i = t; i < TALLIES * COPIES; i += BLOCK)
         s_tally[i] = 0;
-    if (t == 0)
-        s_failed = 0;
+    if (t == 0) {
+        s_over = *a.failed;
+        s_lost[0] = s_lost[1] = 0;
+    }
     const u64 t0 = (u64)blockIdx.x * TILE;
     u32 x[ITEMS], place[ITEMS];
     int from[ITEMS], to[ITEMS]; // the group, by places of the span; to = 0: nothing to do
@@ -360,6 +371,8 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         }
     }
     __syncthreads();
+    if (s_over)
+        return;
     // A member's key: which side of the root it is on, how far it agrees with it (the closer the longer), the symbol after that (0: none).
     // 2 + 31 + 17 bits.
     constexpr u64 ROOT = 1ull << 48, LARGER = 2ull << 48, FAR = 0x7FFFFFFFull;
@@ -376,9 +389,10 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         for (int i = from[k]; i < to[k]; ++i)
             root = s_suf[i] < root ? s_suf[i] : root;
         if (root != x[k]) {
-            const Agreement w = agreement(a, root, x[k], a.ctx);
+            u32 steps_left = SETTLE_STEPS;
+            const Agreement w = agreement(a, root, x[k], a.ctx, steps_left);
             if (!w.found)
-                s_failed = 1u;
+                s_lost[0] = 1u;
             const u64 next = (u64)x[k] + w.length;
             const u64 symbol = to[k] - from[k] > 2 && next < a.n ? (u64)a.text[next] + 1u : 0u; // (a pair has nobody else to be told from)
             key[k] = w.larger ? LARGER | ((FAR - w.length) << 17) | symbol : ((u64)w.length << 17) | symbol;
@@ -386,34 +400,46 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         s_key[k * BLOCK + t] = key[k];
     }
     __syncthreads();
+    if (s_lost[0]) {
+        if (t == 0)
+            *a.failed = 1u;
+        return;
+    }
     // does suffix y go before suffix z of the same key: their agreement from the symbol after the one that tells them from their root
-    auto further = [&](u32 y, u32 z, u64 w) -> Agreement {
+    // (more_left: steps that comparisons may take past their first two)
+    auto further = [&](u32 y, u32 z, u64 w, u32& more_left) -> Agreement {
         const u32 r = y < z ? y : z, o = y < z ? z : y;
-        return agreement(a, r, o, agreement_of(w) + 1u);
+        u32 steps_left = more_left + 2u;
+        const Agreement v = agreement(a, r, o, agreement_of(w) + 1u, steps_left);
+        more_left = steps_left < more_left ? steps_left : more_left;
+        return v;
     };
+    volatile u32* const lost = &s_lost[1];
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         place[k] = (u32)(k * BLOCK) + t;
         if (to[k] == 0)
             continue;
         const int j = k * BLOCK + (int)t;
-        u32 before = 0;
+        u32 before = 0, more_left = SETTLE_STEPS;
         for (int i = from[k]; i < to[k]; ++i) {
             const u64 w = s_key[i];
             if (w < key[k]) {
                 ++before;
             } else if (w == key[k] && i != j) {
+                if (*lost) // (of whatever group: the tile writes nothing)
+                    break;
                 const u32 y = s_suf[i];
-                const Agreement v = further(x[k], y, w);
+                const Agreement v = further(x[k], y, w, more_left);
                 if (!v.found)
-                    s_failed = 1u;
+                    *lost = 1u;
                 before += (y < x[k]) == v.larger ? 1u : 0u;
             }
         }
         place[k] = (u32)from[k] + before;
     }
     __syncthreads();
-    if (s_failed) { // (the same for all threads: nobody sets it past the barrier)
+    if (s_lost[1]) { // (the same for all threads: nobody sets it past the barrier)
         if (t == 0)
             *a.failed = 1u;
         return;
@@ -431,8 +457,10 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         const u32 y = s_suf[right - 1], z = s_suf[right];
         const u32 of_v = agreement_of(v), of_w = agreement_of(w);
         u32 agree = of_v < of_w ? of_v : of_w;
-        if (v == w)
-            agree = further(y, z, w).length;
+        if (v == w) {
+            u32 more_left = SETTLE_STEPS; // (enough: the two have been compared before)
+            agree = further(y, z, w, more_left).length;
+        }
         const u32 room = a.n - 1u - (y > z ? y : z); // (whoever runs off the text within a context is tied with nobody on it)
         agree = agree < room ? agree : room;
         u32 c = 0;

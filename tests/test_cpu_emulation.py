@@ -903,3 +903,15 @@ def test_copies_of_which_some_are_left_to_the_doubling(symbols, key_words):
             doubled += emu_sort.rank_update[0] != 0
             settled += emu_sort.rank_update[0] == 0
     assert doubled >= 2 and settled >= 2, (doubled, settled)
+
+
+@pytest.mark.parametrize("text,size,doubled", [(texts.text_of_undecided_copies, 100, False), (texts.text_of_undecided_copies, 500, True),
+                                               (texts.text_of_an_undecided_group, 2, False), (texts.text_of_an_undecided_group, 30, True)])
+def test_what_settling_copies_may_cost(emu, text, size, doubled):
+    """A member that would take more than 32 steps to be compared with its group's root (every eight symbols of the long passage are one), or
+    more than 32 past the first two of each with all others that differ from the root like itself, is not compared to the end: the list is doubled."""
+    T = text(size)
+    got, active, _ = emu_sort(emu, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    assert (emu_sort.rank_update[0] != 0) == doubled

@@ -210,3 +210,23 @@ def text_of_undecided_copies(length):
     for _ in range(2):
         parts += [rng.integers(100, 60000, 20).astype(np.uint16), twice]
     return np.concatenate(parts + [rng.integers(100, 60000, 20).astype(np.uint16)])
+
+
+def text_of_an_undecided_group(copies):
+    """A passage of 24 symbols once on its own and `copies` times in front of another one of 160, the blocks of which (the first eight symbols from
+    each of its places 4, 12, 20, ... on) stand in the text once more; and an unrelated passage twice. The members of a group of the short
+    passage that go on with the long one differ from the first in the same way, and it takes two of them a step for every eight symbols of the
+    long one to be told apart."""
+    rng = np.random.default_rng(copies)
+    short, long, twice = (rng.integers(100, 60000, k).astype(np.uint16) for k in (24, 160, 250 * copies))
+    parts = [short, rng.integers(100, 60000, 8).astype(np.uint16)]
+    for o in range(4, long.size - 8, 8):
+        parts += [long[o:o + 8], rng.integers(100, 60000, 3).astype(np.uint16)]
+    at = sum(p.size for p in parts)
+    for c in range(copies):
+        gap = rng.integers(100, 60000, 8 + (4 * c - at) % 8).astype(np.uint16)
+        parts += [gap, short, long]
+        at += gap.size + short.size + long.size
+    for _ in range(2):
+        parts += [rng.integers(100, 60000, 20).astype(np.uint16), twice]
+    return np.concatenate(parts + [rng.integers(100, 60000, 20).astype(np.uint16)])
