@@ -47,8 +47,8 @@ constexpr u32 SETTLE_ENDS = CSA_SETTLE_ENDS; // anchors that an end looks ahead
 // Steps (records, and stretches between anchors) of a member's comparison with its root, and of its comparisons with the members of its
 // key past the first two of each, together. Texts with copies take 13 at most (4e8 letters, a fifth of them copies), and groups of 250
 // members, a hundred of which go on alike, one or two a comparison. Passages whose anchors say little take as many as they are long: ms a
-// sort with 256 steps for every comparison, with these limits, and doubled: 12437 symbols, 125 steps, 1.97, 0.68, 0.50; 2.9 M symbols, 187
-// steps, 4.0, 1.5, 1.1; a group of 250, 20 steps a comparison, 174304 symbols, 8.5, 2.0, 1.1, and worse the longer the passage.
+// sort with 256 steps for every comparison, with these limits, and doubled: 12437 symbols, 125 steps, 1.97, 0.63, 0.52; 2.9 M symbols, 187
+// steps, 4.0, 1.3, 1.1; a group of 250, 20 steps a comparison, 174304 symbols, 8.5, 2.0, 1.1, and worse the longer the passage.
 constexpr u32 SETTLE_STEPS = CSA_SETTLE_STEPS;
 constexpr int LINK_TILE = 64 * 64;           // anchors of a workgroup of the link kernel: one word of the first summary
 
@@ -380,10 +380,11 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         const u32 v = (u32)(w >> 17) & (u32)FAR;
         return (w >> 48) == 0 ? v : (w >> 48) == 1 ? (u32)FAR : (u32)FAR - v;
     };
+    volatile u32* const lost = s_lost;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         key[k] = ROOT;
-        if (to[k] == 0)
+        if (to[k] == 0 || lost[0]) // (a tile that has lost a member writes nothing)
             continue;
         u32 root = x[k];
         for (int i = from[k]; i < to[k]; ++i)
@@ -392,7 +393,7 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
             u32 steps_left = SETTLE_STEPS;
             const Agreement w = agreement(a, root, x[k], a.ctx, steps_left);
             if (!w.found)
-                s_lost[0] = 1u;
+                lost[0] = 1u;
             const u64 next = (u64)x[k] + w.length;
             const u64 symbol = to[k] - from[k] > 2 && next < a.n ? (u64)a.text[next] + 1u : 0u; // (a pair has nobody else to be told from)
             key[k] = w.larger ? LARGER | ((FAR - w.length) << 17) | symbol : ((u64)w.length << 17) | symbol;
@@ -414,7 +415,6 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         more_left = steps_left < more_left ? steps_left : more_left;
         return v;
     };
-    volatile u32* const lost = &s_lost[1];
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         place[k] = (u32)(k * BLOCK) + t;
@@ -427,12 +427,12 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
             if (w < key[k]) {
                 ++before;
             } else if (w == key[k] && i != j) {
-                if (*lost) // (of whatever group: the tile writes nothing)
+                if (lost[1])
                     break;
                 const u32 y = s_suf[i];
                 const Agreement v = further(x[k], y, w, more_left);
                 if (!v.found)
-                    *lost = 1u;
+                    lost[1] = 1u;
                 before += (y < x[k]) == v.larger ? 1u : 0u;
             }
         }
