@@ -447,6 +447,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     __shared__ u64 s_diff[SPAN / 64]; // ... or another one
     __shared__ u32 s_many[2];         // some run of the tile has more members, by word
     __shared__ u32 s_ends;            // some member of a run runs off the text inside its words
+    __shared__ u32 s_off[2][SPAN / 32]; // bit j, by word: one of the run that starts at place j does
     __shared__ __align__(16) u64 s_key[SPAN];
     __shared__ __align__(16) u32 s_suf[SPAN];
     __shared__ __align__(16) u8 s_tie[SPAN];
@@ -455,6 +456,8 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         s_many[t] = 0;
     if (t == 2)
         s_ends = 0;
+    for (int j = t; j < 2 * SPAN / 32; j += RESOLVE_BLOCK)
+        s_off[j / (SPAN / 32)][j % (SPAN / 32)] = 0;
     const long long t0 = (long long)blockIdx.x * RESOLVE_TILE, lo = t0 - H, m = a.m;
     const u64 n = a.n;
     // whole waves take consecutive places: one ballot per wave and round gives 64 bits of s_head
@@ -544,17 +547,22 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     __syncthreads();
     const bool ends = s_ends != 0;
     // One word of all elements that still have company: refines their runs. Whoever runs off the text inside the word ties with
-    // nobody and comes before those with the same padded word, shortest first.
+    // nobody and comes before those with the same padded word, shortest first. (Only the runs with such a member are looked at that way: a tile
+    // is as slow as its slowest run, and a short text as its slowest tile. 10^5 symbols of phrases: 168 us with all runs of a tile that
+    // holds one of the last suffixes, 55 without.)
     auto refine = [&](int w) {
+        const u64 ctx = word_syms * (u32)(w + 1);
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k)
             if (last[k] - first[k] > 1 || ((longs >> k) & 1u)) {
                 s_suf[at[k]] = x[k];
                 if (w == 1 || !((owners >> k) & 1u))
                     s_key[at[k]] = w == 0 ? w0[k] : w1[k];
+                if (ends && (u64)x[k] + ctx >= n && !((longs >> k) & 1u))
+                    atomicOr(&s_off[w][first[k] / 32], 1u << (first[k] & 31));
             }
         __syncthreads();
-        const bool many = s_many[w] != 0 && !ends;
+        const bool many = s_many[w] != 0;
         if (many) {
             for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (places whose words were not wanted hold anything: no run looked at below has any)
                 const u64 down = __ballot(j > 0 && s_key[j] < s_key[j - 1]), diff = __ballot(j > 0 && s_key[j] != s_key[j - 1]);
@@ -565,16 +573,15 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
             }
             __syncthreads();
         }
-        const u64 ctx = word_syms * (u32)(w + 1);
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k) {
             const int f = first[k], l = last[k], j = at[k];
             if ((longs >> k) & 1u || l - f <= 1)
                 continue;
-            const bool own = w == 0 && ((owners >> k) & 1u);
+            const bool own = w == 0 && ((owners >> k) & 1u), off = ends && ((s_off[w][f / 32] >> (f & 31)) & 1u);
             int nf = f, nl = l, place = j;
             if (own) { // one string: those that run off the text come first as they stand
-                if (ends) {
+                if (off) {
                     while (nf < l && (u64)s_suf[nf] + ctx >= n)
                         ++nf;
                     if (j < nf) {
@@ -584,7 +591,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
                 }
             } else {
                 bool counted = true;
-                if (many && l - f > FEW) {
+                if (many && l - f > FEW && !off) {
                     // A run that is one string repeated, or several in order, stays as it is: its members need not be compared with
                     // each other. (In a short text the kernel takes as long as the longest run of a tile: generation 0 of 2^18
                     // symbols of phrases 221 us with all comparisons, 191 without these.)
@@ -616,7 +623,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
                 if (counted) {
                     const u64 mine = s_key[j];
                     int less = 0, equal = 0, before = 0; // equal: itself included
-                    if (!ends) {
+                    if (!off) {
                         for (int i = f; i < l; ++i) {
                             const u64 v = s_key[i];
                             less += v < mine ? 1 : 0;
