@@ -1164,14 +1164,15 @@ int code_suffixes(Launch& L, const u16* d_text, u32 n, u32 tail)
 // A list sorted by codes on its way to being ranked.
 struct CodedList {
     ResolveArgs args;
-    u32 words;        // words of four symbols that its order and its ties stand for, at most 2
+    u32 words;        // words of four symbols that its order and its ties stand for, at most 2 ...
+    bool told;        // ... as the device has decided (many_in_long_runs)
     u64 long_members; // suffixes in runs that were too long for their tile, sorted by their second word in ...
     int long_passes;  // ... so many radix passes
     bool long_left;   // there are runs that are too long for a tile on both words
 };
 
-// Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their first `words` words of four symbols, with
-// their ties beside them; code_suffixes ran before. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into
+// Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their first `words` words of four symbols (0: two, or one
+// if many lie in long runs), with their ties beside them; code_suffixes ran before. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into
 // idx[1]; the codes live in the halves of key[0]. What long runs leave open is finished by sort_marked_runs and sort_long_runs.
 // packed: the codes are narrow keys, cut from its stream, of word_syms symbols (and so are the words).
 int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, CodedList& list, const TextSource* packed = nullptr, u32 word_syms = 4)
@@ -1237,9 +1238,12 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
     r.marks = code_tables(h).marks;
     r.unordered = h->counts + 4;
     r.any_long = h->counts + 5;
+    r.words_out = h->counts + 6;
     r.text_codes = codes_of(h);
     r.tail = tail;
     const dim3 resolve_grid((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE));
+    if (words == 0 && n >= WORDS_AHEAD)
+        hipLaunchKernelGGL(choose_words_kernel, dim3(1), dim3(64), 0, s, r.codes, n, r.words_out);
     if (packed)
         hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, true>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, r);
     else
@@ -1558,6 +1562,7 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
         TableGroup beside = {};
         if (coded) {
             ra.words = coded->words;
+            ra.words_known = coded->told ? nullptr : coded->args.words_out;
             // (several tiles a wave on long lists: fewer additions to the level totals)
             const u32 per_wave = r.tiles >= (1u << 15) ? 8u : 1u, waves = (r.tiles + per_wave - 1) / per_wave;
             hipLaunchKernelGGL((count_ties_kernel<RANK_TILE>), dim3((waves + 3) / 4), dim3(256), 0, s, ra, r.tiles, per_wave);
@@ -1574,6 +1579,8 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
     if (rc)
         return rc;
     if (coded) {
+        coded->words = ra.words = h->h_pinned[6];
+        coded->told = true;
         const bool unordered = h->h_pinned[4] != 0, second = h->h_pinned[5] != 0 && coded->words == 2;
         if (unordered && (rc = sort_marked_runs(L, coded->args, passes)) != CSA_OK) // long runs of one code are out of order: they are sorted now
             return rc;
@@ -1828,7 +1835,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, plan, &in_out, &p1, nullptr, 0, 0, &ps);
         }
     } else if (coded) {
-        rc = sort_by_codes(L, d_text, n, tail, h->pack_symbols ? 2u : 1u, list);
+        rc = sort_by_codes(L, d_text, n, tail, h->pack_symbols ? 0u : 1u, list);
         p1 = CODE_PASSES;
         in_out = 1; // idx[1] holds the list, key[0] and key[1] what the sort has left behind
     } else {

@@ -18,7 +18,7 @@
 // run of up to RESOLVE_MAX suffixes in order inside its tile, and notes beside every suffix on how many words of four symbols it
 // ties with its left neighbour, which is all the rank step needs to know: the list is that of generation 1, and what that generation
 // cost (a gathered line for every suffix that is tied on four symbols, a sort of its large groups, an update of the ranks) is not
-// paid. Longer runs that are one string repeated are in order as they stand; those that are not are collected and radix sorted by the
+// paid (a list with many suffixes in long runs is resolved on one word: many_in_long_runs). Longer runs that are one string repeated are in order as they stand; those that are not are collected and radix sorted by the
 // string itself. Then all members of long runs are sorted by the code of the next four symbols and resolved like the rest.
 // Time of whole sorts when the first sort resolves four symbols and eight: 1e9 Zipf tokens 73.2 and 65.4 ms, 2^28 18.6 and 16.9, 4096
 // 0.37 and 0.31; the kernel itself 8.1 and 13.8 ms on 1e9.
@@ -377,6 +377,9 @@ constexpr int RESOLVE_TILE = RESOLVE_BLOCK * RESOLVE_ITEMS;
 #ifndef CSA_RESOLVE_MAX
 #define CSA_RESOLVE_MAX 256
 #endif
+#ifndef CSA_WORDS_AHEAD
+#define CSA_WORDS_AHEAD (1u << 22)
+#endif
 constexpr int RESOLVE_MAX = CSA_RESOLVE_MAX; // longest run that is sorted inside its tile
 static_assert(CODE_ITEMS == 8, "a thread of the coding kernel writes one byte of flags");
 static_assert(RESOLVE_MAX % 64 == 0 && 2 * RESOLVE_MAX <= RESOLVE_BLOCK, "the halo is read in whole waves, one element per thread");
@@ -393,7 +396,8 @@ struct ResolveArgs {
     u32 m;            // entries of the list
     const u16* text;
     u32 n;
-    u32 words; // 1: the list is resolved on the symbols of the codes; 2: on as many after them, too
+    u32 words; // 1: the list is resolved on the symbols of the codes; 2: on as many after them, too; 0: as many_in_long_runs says ...
+    u32* words_out; // ... which stands here already for long lists, and is written here for short ones
     u32 word_syms;     // symbols of a word: four, or 32 bits of the code stream of a packed text, where every code is its string's own:
     const u32* stream; // non-null
     u32 sym_bits;
@@ -425,6 +429,33 @@ __device__ __forceinline__ u64 second_word(const ResolveArgs& a, u32 x)
     return y < a.n ? packed_window(a.stream, y * a.sym_bits, 32u) : 0ull;
 }
 
+// Whether many of a list's suffixes lie in long runs, by 64 of its places (one wave): more than 12 in runs of HALF_LONG or more, which are found
+// where they have HALF_LONG others at one side. Such a list is resolved on one word. Members of runs that are too long for a tile would have to be
+// sorted by the second one, those of others long for a tile compared by it one by one, and the generation after, with the
+// ranks of all, costs no more. (Sorts, ms, by two words, one, and before there were two: 33000 symbols of ten phrases 0.83, 0.60, 0.65; 130000 of
+// a hundred 1.01, 0.85, 0.92; 400000 of 300 1.33, 1.12, 1.09; 400000 symbols Zipf(2) 0.80, 0.69, 0.73; 4 M of written text in 16-bit symbols
+// 1.50, 1.38, 1.43. With 20 places of 64 as the limit the third stays at 1.35. Token texts have 4 to 6 places.)
+constexpr u32 HALF_LONG = RESOLVE_MAX / 2, MANY_LONG = 12;
+
+__device__ __forceinline__ bool many_in_long_runs(const u32* __restrict__ codes, u32 m)
+{
+    const u32 e = (u32)((u64)m * (threadIdx.x & 63u) / 64u);
+    const u32 c = codes[e];
+    const bool in = (e >= HALF_LONG && codes[e - HALF_LONG] == c) || (e + HALF_LONG < m && codes[e + HALF_LONG] == c);
+    return (u32)__popcll(__ballot(in)) > MANY_LONG;
+}
+
+// Lists of WORDS_AHEAD suffixes or more are looked at by a wave of its own: a launch costs 3 us, and the look of every tile 2 % of the sort of 2^28
+// tokens (11.35 -> 11.6 ms).
+constexpr u32 WORDS_AHEAD = CSA_WORDS_AHEAD;
+
+__global__ __launch_bounds__(64) void choose_words_kernel(const u32* __restrict__ codes, u32 m, u32* words_out)
+{
+    const bool one = many_in_long_runs(codes, m);
+    if (threadIdx.x == 0)
+        *words_out = one ? 1u : 2u;
+}
+
 // The runs of equal codes (KEYS = false: the list of all suffixes) or of equal keys (KEYS = true: the members of the long runs, sorted
 // once more by the code of the next word) of one tile and the halo its first and last run reach into, refined word by word:
 // every member of a run of at most H counts those with a smaller word, which gives its place and
@@ -447,6 +478,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     __shared__ u64 s_diff[SPAN / 64]; // ... or another one
     __shared__ u32 s_many[2];         // some run of the tile has more members, by word
     __shared__ u32 s_ends;            // some member of a run runs off the text inside its words
+    __shared__ u32 s_words;
     __shared__ u32 s_off[2][SPAN / 32]; // bit j, by word: one of the run that starts at place j does
     __shared__ __align__(16) u64 s_key[SPAN];
     __shared__ __align__(16) u32 s_suf[SPAN];
@@ -456,8 +488,14 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         s_many[t] = 0;
     if (t == 2)
         s_ends = 0;
-    for (int j = t; j < 2 * SPAN / 32; j += RESOLVE_BLOCK)
-        s_off[j / (SPAN / 32)][j % (SPAN / 32)] = 0;
+    if (!KEYS && t < 64u) {
+        const u32 w = a.words ? a.words : a.m >= WORDS_AHEAD ? *a.words_out : many_in_long_runs(a.codes, a.m) ? 1u : 2u;
+        if (t == 0) {
+            s_words = w;
+            if (blockIdx.x == 0)
+                *a.words_out = w;
+        }
+    }
     const long long t0 = (long long)blockIdx.x * RESOLVE_TILE, lo = t0 - H, m = a.m;
     const u64 n = a.n;
     // whole waves take consecutive places: one ballot per wave and round gives 64 bits of s_head
@@ -474,12 +512,16 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
                 head = a.codes[e] != a.codes[e - 1];
             }
         }
-        s_tie[j] = head ? tie : (u8)a.words;
+        s_tie[j] = head ? tie : (u8)TIE_MOST_WORDS;
         const u64 b = __ballot(head);
         if ((t & 63u) == 0)
             s_head[j / 64] = b;
     }
     __syncthreads();
+    const u32 words = KEYS ? TIE_MOST_WORDS : s_words;
+    if (words < TIE_MOST_WORDS)
+        for (int j = t; j < SPAN; j += RESOLVE_BLOCK) // (the thread's own places)
+            s_tie[j] = s_tie[j] ? (u8)words : (u8)0;
     // the run around place j: first place and first place behind it; false if it has more than H members
     auto run_of = [&](int j, int& first, int& last) -> bool {
         int wd = j / 64;
@@ -500,7 +542,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     u32 x[ITEMS], owners = 0, longs = 0; // bit k: element k has OWN_CODE; is one of a long run
     int at[ITEMS], first[ITEMS], last[ITEMS]; // last - first = 1: alone
     u64 w0[ITEMS], w1[ITEMS];
-    const bool two = KEYS || a.words == 2; // (keys come with two words)
+    const bool two = KEYS || words == 2; // (keys come with two words)
     const u32 word_syms = PACKED ? a.word_syms : 4u;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
@@ -537,7 +579,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
             w0[k] = load_kgram(a.text, a.n, x[k], 0);
         if (two && (KEYS || is_short)) // (the members of long runs of codes get their second word when they are sorted by it)
             w1[k] = second_word<PACKED>(a, x[k]);
-        if ((u64)x[k] + (u64)word_syms * a.words >= n)
+        if ((u64)x[k] + (u64)word_syms * words >= n)
             s_ends = 1;
         if (is_short && l - f > FEW) {
             s_many[0] = 1;
@@ -546,6 +588,11 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     }
     __syncthreads();
     const bool ends = s_ends != 0;
+    if (ends) {
+        for (int j = t; j < 2 * SPAN / 32; j += RESOLVE_BLOCK)
+            s_off[j / (SPAN / 32)][j % (SPAN / 32)] = 0;
+        __syncthreads();
+    }
     // One word of all elements that still have company: refines their runs. Whoever runs off the text inside the word ties with
     // nobody and comes before those with the same padded word, shortest first. (Only the runs with such a member are looked at that way: a tile
     // is as slow as its slowest run, and a short text as its slowest tile. 10^5 symbols of phrases: 168 us with all runs of a tile that

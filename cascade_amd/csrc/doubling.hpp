@@ -66,6 +66,7 @@ struct RerankArgs {
     const u32* sufs;
     const u8* ties;  // TIED: the bytes of the list's entries, and the words that the list is ranked on: neighbours belong to one
     u32 words;       // run if they share as many
+    const u32* words_known; // count_ties_kernel, non-null: the same, where the host has yet to see it
     u32 m;         // = n: generation 0 ranks every suffix
     u32 n;         // partition size
     u32 ell;       // symbols in the generation-0 key
@@ -299,6 +300,7 @@ __global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles
 {
     const u32 lane = threadIdx.x & 63u;
     const u32 wave = blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
+    const u32 words = a.words_known ? *a.words_known : a.words;
     u32 sum_surv[TIE_MOST_WORDS] = {}, sum_heads[TIE_MOST_WORDS] = {};
     for (u32 r = 0; r < per_wave; ++r) {
         const u64 tile = (u64)wave * per_wave + r;
@@ -311,7 +313,7 @@ __global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles
             const u32 surv = (u32)__popc((v.tie[i] | v.right[i]) & v.valid), heads = (u32)__popc(~v.tie[i] & v.right[i] & v.valid);
             sum_surv[i] += surv;
             sum_heads[i] += heads;
-            if (i + 1 == a.words) {
+            if (i + 1 == words) {
                 const u32 begin = ~v.tie[i] & v.valid; // (1-based: 0 means no head in the tile)
                 const u32 last = begin ? (u32)base + 32u - (u32)__builtin_clz(begin) : 0u;
                 u32 most = last, packed = surv | (heads << 16);

@@ -74,7 +74,8 @@ typedef struct csa_stats {
                                         enough for packed codes of 1, 2, 4 or 8 bits (more than 2^24 symbols of two bits are sorted
                                         by 16 of them, with the next 16 read where those tie: 32 all the same, or 16 where
                                         runs were too long for it). A sort by codes goes on to resolve the
-                                        next four symbols from the text: generation 1 is then reported with the list it would
+                                        next four symbols from the text, unless many suffixes share their first four with hundreds
+                                        of others: generation 1 is then reported with the list it would
                                         have had, the members of long runs in big[1], their passes in passes[1], and no time.
                                         So are the generations of a list of short groups whose ties come from copied passages,
                                         which are settled at once without ranks (rank_update[0] is 0 then), and those after the

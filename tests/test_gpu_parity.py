@@ -851,3 +851,17 @@ def test_groups_of_which_some_members_are_told_apart_and_some_are_not(torch_mod,
         stats = s.last_stats
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
+
+
+@pytest.mark.parametrize("n,phrases,lo,hi", [(33000, 10, 2, 6), (130000, 100, 4, 20), ((1 << 22) - 1, 300, 4, 20), (1 << 22, 10, 2, 6), ((1 << 22) + 5, 0, 0, 0)])
+def test_lists_with_many_suffixes_in_long_runs(torch_mod, n, phrases, lo, hi):
+    """Texts of few phrases, and of 1000 symbols (phrases = 0) that have none: most suffixes of the former share their first four symbols with hundreds
+    of others, and the first sort stops at those. From 2^22 symbols on a kernel of its own looks for that."""
+    from cascade_amd import PartitionSorter
+    T = texts.text_of_phrases(n, phrases, lo, hi, 1) if phrases else np.random.default_rng(n).integers(1, 1000, n).astype(np.uint16)
+    with PartitionSorter(T.size, key_words=1) as s:
+        print(f"  {n} symbols of {phrases} phrases", flush=True)
+        got = gpu_sa40(torch_mod, s, T)
+        stats = s.last_stats
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
