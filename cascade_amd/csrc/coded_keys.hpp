@@ -429,21 +429,12 @@ __device__ __forceinline__ u64 second_word(const ResolveArgs& a, u32 x)
     return y < a.n ? packed_window(a.stream, y * a.sym_bits, 32u) : 0ull;
 }
 
-// Whether many of a list's suffixes lie in long runs, by 64 of its places (one wave): more than 12 in runs of HALF_LONG or more, which are found
-// where they have HALF_LONG others at one side. Such a list is resolved on one word. Members of runs that are too long for a tile would have to be
+// A list many of whose suffixes lie in runs of RESOLVE_MAX / 2 or more is resolved on one word. Members of runs that are too long for a tile would have to be
 // sorted by the second one, those of others long for a tile compared by it one by one, and the generation after, with the
 // ranks of all, costs no more. (Sorts, ms, by two words, one, and before there were two: 33000 symbols of ten phrases 0.83, 0.60, 0.65; 130000 of
 // a hundred 1.01, 0.85, 0.92; 400000 of 300 1.33, 1.12, 1.09; 400000 symbols Zipf(2) 0.80, 0.69, 0.73; 4 M of written text in 16-bit symbols
 // 1.50, 1.38, 1.43. With 20 places of 64 as the limit the third stays at 1.35. Token texts have 4 to 6 places.)
-constexpr u32 HALF_LONG = RESOLVE_MAX / 2, MANY_LONG = 12;
-
-__device__ __forceinline__ bool many_in_long_runs(const u32* __restrict__ codes, u32 m)
-{
-    const u32 e = (u32)((u64)m * (threadIdx.x & 63u) / 64u);
-    const u32 c = codes[e];
-    const bool in = (e >= HALF_LONG && codes[e - HALF_LONG] == c) || (e + HALF_LONG < m && codes[e + HALF_LONG] == c);
-    return (u32)__popcll(__ballot(in)) > MANY_LONG;
-}
+constexpr u32 HALF_LONG = RESOLVE_MAX / 2;
 
 // Lists of WORDS_AHEAD suffixes or more are looked at by a wave of its own: a launch costs 3 us, and the look of every tile 2 % of the sort of 2^28
 // tokens (11.35 -> 11.6 ms).
@@ -451,7 +442,7 @@ constexpr u32 WORDS_AHEAD = CSA_WORDS_AHEAD;
 
 __global__ __launch_bounds__(64) void choose_words_kernel(const u32* __restrict__ codes, u32 m, u32* words_out)
 {
-    const bool one = many_in_long_runs(codes, m);
+    const bool one = many_in_long_runs(codes, m, HALF_LONG);
     if (threadIdx.x == 0)
         *words_out = one ? 1u : 2u;
 }
@@ -489,7 +480,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     if (t == 2)
         s_ends = 0;
     if (!KEYS && t < 64u) {
-        const u32 w = a.words ? a.words : a.m >= WORDS_AHEAD ? *a.words_out : many_in_long_runs(a.codes, a.m) ? 1u : 2u;
+        const u32 w = a.words ? a.words : a.m >= WORDS_AHEAD ? *a.words_out : many_in_long_runs(a.codes, a.m, HALF_LONG) ? 1u : 2u;
         if (t == 0) {
             s_words = w;
             if (blockIdx.x == 0)

@@ -73,8 +73,8 @@ __global__ __launch_bounds__(256) void scatter_u32_kernel(const u32* __restrict_
         atomicExch(err, DEV_ERR_RERANK_RANGE);
 }
 
-// Runs of one first word in a list sorted by it: members can still change places, and only inside their run. Those of up to ORDER_MAX
-// members are put in order by their other words and the forward tag where they stand; bits of the members of longer ones are
+// Runs of one first word in a list sorted by it: members can still change places, and only inside their run. Those of up to ORDER_MAX (or
+// ORDER_FEW) members are put in order by their other words and the forward tag where they stand; bits of the members of longer ones are
 // left for the passes over them (tie_kernel).
 // A tile orders the runs that start in it. What bounds it is the random reads of a tied suffix, a line of its key and one of its tags,
 // where the passes over all tied suffixes moved 24 bytes a pass, 34 times with keys of four words (the whole step on 16.8 M suffixes of
@@ -84,6 +84,13 @@ constexpr int ORDER_ITEMS = 4;
 constexpr int ORDER_TILE = ORDER_BLOCK * ORDER_ITEMS;
 constexpr int ORDER_MAX = 256;
 static_assert(ORDER_MAX == ORDER_BLOCK && ORDER_TILE % 64 == 0, "the halo behind a tile is one element per thread, bits leave in whole words");
+
+// In a list of fewer than ORDER_LOOK_MAX suffixes many of which lie in long runs, runs of up to ORDER_FEW members are ordered here and longer ones
+// are left: the passes over the members of long runs take about as long for them too, and the tile with the longest run holds up the
+// kernel. (ms a step with two words, runs of up to 256, of up to 32, and all of them left to the passes: a third of 200000 bytes of text 0.44,
+// 0.39, 0.37; of 2 M 0.58, 0.53, 0.52; of 6 M 0.85, 0.81, 0.80; of 16 M 1.71, 1.73, 1.78. Where no run is long, it is the passes that are
+// saved: tokens, 200000, four words, 0.23, 0.62 and 0.72.)
+constexpr u32 ORDER_LOOK_MAX = 1u << 22, ORDER_FEW = 32;
 
 struct OrderRunsArgs {
     const u64* first_words; // sorted
@@ -100,10 +107,16 @@ __global__ __launch_bounds__(ORDER_BLOCK) void order_runs_kernel(OrderRunsArgs a
 {
     constexpr int H = ORDER_MAX, SPAN = ORDER_TILE + 2 * H, ITEMS = ORDER_ITEMS + 1;
     __shared__ u64 s_head[SPAN / 64]; // bit j: the entry at span place j starts a run (places outside the list count as starts)
+    __shared__ u32 s_most;
     __shared__ u64 s_word[(W - 1) * (ORDER_TILE + H)];
     __shared__ u16 s_tag[ORDER_TILE + H];
     const u32 t = threadIdx.x;
     const long long t0 = (long long)blockIdx.x * ORDER_TILE, lo = t0 - H, m = (long long)a.m;
+    if (t < 64u) {
+        const u32 most = a.m < ORDER_LOOK_MAX && many_in_long_runs(a.first_words, (u32)a.m, H / 2) ? ORDER_FEW : (u32)H;
+        if (t == 0)
+            s_most = most;
+    }
     for (int j = t; j < SPAN; j += ORDER_BLOCK) {
         const long long e = lo + j;
         const u64 b = __ballot(e <= 0 || e >= m || a.first_words[e] != a.first_words[e - 1]);
@@ -111,7 +124,8 @@ __global__ __launch_bounds__(ORDER_BLOCK) void order_runs_kernel(OrderRunsArgs a
             s_head[j / 64] = b;
     }
     __syncthreads();
-    // the run around place j: first place and first place behind it; false if it has more than H members
+    const int most = (int)s_most;
+    // the run around place j: first place and first place behind it; false if it has more than `most` members
     auto run_of = [&](int j, int& first, int& last) -> bool {
         int wd = j / 64;
         u64 b = s_head[wd] & (~0ull >> (63 - (j & 63)));
@@ -125,7 +139,7 @@ __global__ __launch_bounds__(ORDER_BLOCK) void order_runs_kernel(OrderRunsArgs a
         while (b == 0 && wd + 1 < SPAN / 64 && (wd + 1) * 64 <= j + H)
             b = s_head[++wd];
         last = b ? wd * 64 + __builtin_ctzll(b) : SPAN + H;
-        return last - first <= H;
+        return last - first <= most;
     };
     u32 x[ITEMS];
     int first[ITEMS], last[ITEMS]; // last = 0: nothing to do

@@ -36,10 +36,15 @@ def groups(target, rank, end, p):
 
 def runs_of_first_words(key_words, long_runs, seed):
     """Keys of generation 0 with runs of one first word as long as a tile sorts in place (256), one shorter and one longer, and across
-    the ends of tiles of 1024; the other words and the forward tags differ, or only the last of them does, or nothing does."""
+    the ends of tiles of 1024; the other words and the forward tags differ, or only the last of them does, or nothing does. long_runs: "few", of a list that goes on with
+    short ones, or "many", when runs of up to 32 are sorted in place, with some on both sides of that."""
     rng = np.random.default_rng(seed)
     lengths = [1, 2, 255, 256, 3, 1, 500 - (1 + 2 + 255 + 256 + 3 + 1) % 500, 256, 255, 2, 17] + rng.integers(1, 6, 900).tolist()
-    if long_runs:
+    if long_runs == "few":
+        lengths += [257, 300, 2] + rng.integers(1, 6, 6000).tolist()
+    elif long_runs == "many":
+        lengths += [31, 32, 33, 34, 1] * 5 + [900, 64, 128] * 6
+    elif long_runs:
         lengths += [257, 1, 700, 2500, 2, 256]
     first = np.repeat(np.cumsum(rng.integers(1, 1 << 40, len(lengths))).astype(np.uint64), lengths)
     if not long_runs:  # (one of the lengths above is longer than a tile sorts)

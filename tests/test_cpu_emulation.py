@@ -482,7 +482,7 @@ class HostArray:
         self.ptr = a.ctypes.data
 
 
-@pytest.mark.parametrize("key_words,long_runs", [(1, True), (2, False), (2, True), (3, True), (4, False), (4, True)])
+@pytest.mark.parametrize("key_words,long_runs", [(1, True), (2, False), (2, True), (3, True), (4, False), (4, True), (2, "few"), (4, "few"), (2, "many"), (3, "many")])
 def test_emulated_runs_of_one_first_word_in_order(emu, key_words, long_runs):
     """The first partition step with wide keys: runs of one first word, short ones sorted where they stand and long ones taken out."""
     import message_cases

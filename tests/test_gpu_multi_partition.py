@@ -207,7 +207,7 @@ def test_the_references_own_predictor_gives_the_cohorts_and_pill_receipts_of_the
     assert len(ours["cohorts"]) >= 10 and sum(ours["pill_receipts"]) > 0
 
 
-@pytest.mark.parametrize("key_words,long_runs", [(1, True), (2, False), (2, True), (3, True), (4, False), (4, True)])
+@pytest.mark.parametrize("key_words,long_runs", [(1, True), (2, False), (2, True), (3, True), (4, False), (4, True), (2, "few"), (4, "few"), (2, "many"), (4, "many")])
 def test_runs_of_one_first_word_in_order(gpu, key_words, long_runs):
     """csa_sort_init_dev with runs of one first word at the edges of what is sorted in place, against a sort of whole keys."""
     import message_cases
