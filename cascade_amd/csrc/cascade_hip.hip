@@ -336,7 +336,7 @@ struct csa_handle {
     u32 defer_min = DEFER_MIN; // lists at least this long use the bucketed rank update (csa_set_tuning)
     u32 window_min_changed = WINDOW_MIN_CHANGED; // csa_set_tuning (0xFFFFFFFF: never)
     u32 expect_presorted = 0; // csa_set_tuning: 1 = every generation first runs as if its large groups were in order already
-    u32 settle = 1;       // csa_set_tuning: 0 once a threshold of the rank updates has been set
+    u32 settle = 1;       // csa_set_tuning: lists are settled without ranks, short texts ranked by counting; 0 once a threshold of the rank updates has been set
     u32 pack_symbols = 1; // csa_set_tuning: texts over small alphabets start from keys of many symbols (packed_text.hpp)
     csa_step_result last_step = {};              // counters of the last partition step (csa_last_step_result)
     std::vector<hipEvent_t> events;
@@ -2866,6 +2866,7 @@ int csa_set_tuning(csa_handle* h, int knob, uint32_t value)
     case CSA_TUNE_WINDOW_MIN_CHANGED: h->window_min_changed = value, h->settle = 0; break;
     case CSA_TUNE_PACK_SYMBOLS: h->pack_symbols = value ? 1u : 0u; break;
     case CSA_TUNE_EXPECT_PRESORTED: h->expect_presorted = value ? 1u : 0u; break;
+    case CSA_TUNE_SETTLE: h->settle = value ? 1u : 0u; break;
     case CSA_TUNE_XCD_CHUNK:
         // the chunked order waits for workgroups that are dispatched later: 8 * chunk workgroups of a pass must be able
         // to be resident together, and the device must have room for twice that many (the condition csa_create applies)

@@ -149,8 +149,7 @@ int csa_set_device_exclusive(csa_handle* h, int exclusive);
  *                                (default 2^23 suffixes)
  *   CSA_TUNE_WINDOW_MIN_CHANGED  fewest changed ranks for the windowed update of later generations (default 2^22;
  *                                0xFFFFFFFF: never)
- *                                Setting either threshold also keeps lists of short groups, and of runs and periods, from being
- *                                settled without ranks, and short texts from being ranked by counting
+ *                                Setting either threshold, to whatever value, also sets CSA_TUNE_SETTLE to 0
  *   CSA_TUNE_XCD_CHUNK           tiles (of 8192 pairs) that one XCD takes in a row under csa_set_device_exclusive
  *                                (default 16; 0: the exclusive order is the default order); call before
  *                                csa_set_device_exclusive. 8 chunks of that many workgroups must be resident
@@ -165,13 +164,17 @@ int csa_set_device_exclusive(csa_handle* h, int exclusive);
  *                                when every large group of the generation before was in order as it stood (csa_stats.presorted),
  *                                and gathers again with them if this one's are not; 1: every generation starts that way
  *                                (tests of the second gather), and short texts are sorted like long ones
+ *   CSA_TUNE_SETTLE              1 (default): lists of short groups, and of runs and periods, are settled without ranks, and short texts
+ *                                are ranked by counting; 0: they go through the generations whose thresholds the first two
+ *                                knobs set. To have both, set this after them
  * No counterpart in the reference. */
 enum {
     CSA_TUNE_DEFER_MIN = 0,
     CSA_TUNE_WINDOW_MIN_CHANGED = 1,
     CSA_TUNE_XCD_CHUNK = 2,
     CSA_TUNE_PACK_SYMBOLS = 3,
-    CSA_TUNE_EXPECT_PRESORTED = 4
+    CSA_TUNE_EXPECT_PRESORTED = 4,
+    CSA_TUNE_SETTLE = 5
 };
 int csa_set_tuning(csa_handle* h, int knob, uint32_t value);
 

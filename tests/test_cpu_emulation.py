@@ -929,3 +929,21 @@ def test_lists_with_many_suffixes_in_long_runs_are_resolved_on_one_word(emu, n, 
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
     if key_words == 1:
         assert emu_sort.passes[0] == 4 and (big[1] > 0) == (words == 2)
+
+
+def test_the_knob_of_the_settling(emu):
+    """A threshold of the rank updates turns the settling of copies off, whatever its value, CSA_TUNE_SETTLE on again with the threshold kept, and off by
+    itself; the array is the same each time."""
+    T = texts.text_of_copies(5000, 60000, 3)
+    seen = []
+    for knobs in ([], [(_native.CSA_TUNE_DEFER_MIN, 1000)], [(_native.CSA_TUNE_DEFER_MIN, 1000), (_native.CSA_TUNE_SETTLE, 1)], [(_native.CSA_TUNE_SETTLE, 0)],
+                  [(_native.CSA_TUNE_SETTLE, 0), (_native.CSA_TUNE_SETTLE, 1)]):
+        h = C.c_void_p()
+        assert emu.csa_create(T.size, 1, C.byref(h)) == 0
+        for knob, value in knobs:
+            assert emu.csa_set_tuning(h, knob, value) == 0
+        out, st = np.zeros(5 * T.size + 8, dtype=np.uint8), _native.CsaStats()
+        assert emu.csa_sort_partition_u16_dev(h, T.ctypes.data, T.size, 0, out.ctypes.data, None, 0, C.byref(st)) == 0
+        emu.csa_destroy(h)
+        seen.append((int(st.rank_update[0]), out.tobytes()))
+    assert [s[0] != 0 for s in seen] == [False, True, False, True, False] and len({s[1] for s in seen}) == 1
