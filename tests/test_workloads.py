@@ -51,3 +51,12 @@ def test_shapes():
     assert len(np.unique(c5[:run])) == 1
     assert np.array_equal(c5[run:run + per - 7], c5[run + 7:run + per])
     assert c5[run + per] == SEP
+
+
+def test_the_bench_line_tells_covered_generations_from_settled_ones():
+    import bench
+    codes = {"first_sort_generations": 1, "key_symbols": 4, "key_words": 1}
+    assert [bench.untimed_as(codes, g) for g in (1, 2, 14)] == ["covered_by_first_sort", "settled_at_once", "settled_at_once"]
+    assert bench.untimed_as(dict(codes, key_words=4), 1) == "settled_at_once"  # (generation 0 of wide keys takes the eight symbols)
+    packed = {"first_sort_generations": 4, "key_symbols": 32, "key_words": 1}
+    assert [bench.untimed_as(packed, g) for g in (1, 3, 4)] == ["covered_by_first_sort", "covered_by_first_sort", "settled_at_once"]
