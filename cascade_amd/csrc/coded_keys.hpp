@@ -433,8 +433,10 @@ __device__ __forceinline__ u64 second_word(const ResolveArgs& a, u32 x)
 // sorted by the second one, those of others long for a tile compared by it one by one, and the generation after, with the
 // ranks of all, costs no more. (Sorts, ms, by two words, one, and before there were two: 33000 symbols of ten phrases 0.83, 0.60, 0.65; 130000 of
 // a hundred 1.01, 0.85, 0.92; 400000 of 300 1.33, 1.12, 1.09; 400000 symbols Zipf(2) 0.80, 0.69, 0.73; 4 M of written text in 16-bit symbols
-// 1.50, 1.38, 1.43. With 20 places of 64 as the limit the third stays at 1.35. Token texts have 4 to 6 places.)
-constexpr u32 HALF_LONG = RESOLVE_MAX / 2;
+// 1.50, 1.38, 1.43.) The line lies at 12 of 64 places in short lists (with 20 the third of these stays at 1.35) and at 24 in long ones, whose second
+// words are lines of the text, which generation 1 would read as lines of ranks: 2^26 symbols of runs and Zipf(1.3), 12 places 7.4 ms, 24 to 64
+// 6.4; 2^26 Zipf(1.3) alone 6.0 and 5.0; 2 * 10^7 Zipf(1.5) 2.9 with 24, 4.0 with 36. Token texts have 4 to 6 places.
+constexpr u32 HALF_LONG = RESOLVE_MAX / 2, SHORT_LIST_FEW = 12, LONG_LIST_FEW = 24;
 
 // Lists of WORDS_AHEAD suffixes or more are looked at by a wave of its own: a launch costs 3 us, and the look of every tile 2 % of the sort of 2^28
 // tokens (11.35 -> 11.6 ms).
@@ -442,7 +444,7 @@ constexpr u32 WORDS_AHEAD = CSA_WORDS_AHEAD;
 
 __global__ __launch_bounds__(64) void choose_words_kernel(const u32* __restrict__ codes, u32 m, u32* words_out)
 {
-    const bool one = many_in_long_runs(codes, m, HALF_LONG);
+    const bool one = many_in_long_runs(codes, m, HALF_LONG, LONG_LIST_FEW);
     if (threadIdx.x == 0)
         *words_out = one ? 1u : 2u;
 }
@@ -480,7 +482,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     if (t == 2)
         s_ends = 0;
     if (!KEYS && t < 64u) {
-        const u32 w = a.words ? a.words : a.m >= WORDS_AHEAD ? *a.words_out : many_in_long_runs(a.codes, a.m, HALF_LONG) ? 1u : 2u;
+        const u32 w = a.words ? a.words : a.m >= WORDS_AHEAD ? *a.words_out : many_in_long_runs(a.codes, a.m, HALF_LONG, SHORT_LIST_FEW) ? 1u : 2u;
         if (t == 0) {
             s_words = w;
             if (blockIdx.x == 0)

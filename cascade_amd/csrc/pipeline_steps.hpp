@@ -85,12 +85,12 @@ constexpr int ORDER_TILE = ORDER_BLOCK * ORDER_ITEMS;
 constexpr int ORDER_MAX = 256;
 static_assert(ORDER_MAX == ORDER_BLOCK && ORDER_TILE % 64 == 0, "the halo behind a tile is one element per thread, bits leave in whole words");
 
-// In a list of fewer than ORDER_LOOK_MAX suffixes many of which lie in long runs, runs of up to ORDER_FEW members are ordered here and longer ones
+// In a list of fewer than ORDER_LOOK_MAX suffixes many of which lie in long runs (more than 12 of 64 places), runs of up to ORDER_FEW members are ordered here and longer ones
 // are left: the passes over the members of long runs take about as long for them too, and the tile with the longest run holds up the
 // kernel. (ms a step with two words, runs of up to 256, of up to 32, and all of them left to the passes: a third of 200000 bytes of text 0.44,
 // 0.39, 0.37; of 2 M 0.58, 0.53, 0.52; of 6 M 0.85, 0.81, 0.80; of 16 M 1.71, 1.73, 1.78. Where no run is long, it is the passes that are
 // saved: tokens, 200000, four words, 0.23, 0.62 and 0.72.)
-constexpr u32 ORDER_LOOK_MAX = 1u << 22, ORDER_FEW = 32;
+constexpr u32 ORDER_LOOK_MAX = 1u << 22, ORDER_FEW = 32, ORDER_FEW_PLACES = 12;
 
 struct OrderRunsArgs {
     const u64* first_words; // sorted
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(ORDER_BLOCK) void order_runs_kernel(OrderRunsArgs a
     const u32 t = threadIdx.x;
     const long long t0 = (long long)blockIdx.x * ORDER_TILE, lo = t0 - H, m = (long long)a.m;
     if (t < 64u) {
-        const u32 most = a.m < ORDER_LOOK_MAX && many_in_long_runs(a.first_words, (u32)a.m, H / 2) ? ORDER_FEW : (u32)H;
+        const u32 most = a.m < ORDER_LOOK_MAX && many_in_long_runs(a.first_words, (u32)a.m, H / 2, ORDER_FEW_PLACES) ? ORDER_FEW : (u32)H;
         if (t == 0)
             s_most = most;
     }

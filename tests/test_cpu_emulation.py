@@ -917,18 +917,19 @@ def test_what_settling_copies_may_cost(emu, text, size, doubled):
     assert (emu_sort.rank_update[0] != 0) == doubled
 
 
-@pytest.mark.parametrize("n,repeats,words", [(2900, [70], 2), (2900, [100] * 3, 1), (3900, [90], 2), (3900, [100] * 4, 1)])
+@pytest.mark.parametrize("n,repeats,followers,words", [(2900, [70], 40, 2), (2900, [100] * 3, 40, 1), (3900, [100] * 2, 40, 2), (3900, [100] * 4, 2, 1)])
 @pytest.mark.parametrize("key_words", [1, 2, 4])
-def test_lists_with_many_suffixes_in_long_runs_are_resolved_on_one_word(emu, n, repeats, words, key_words):
-    """Where more than 12 of 64 places of the sorted list lie in runs of half the in-tile limit (32 of 64 members in this build) or more,
-    the first sort resolves four symbols, and the groups of a hundred are small ones of generation 1; otherwise it resolves eight, and they
-    are long runs. (From 3000 symbols on a kernel of its own looks, in this build.) Suffix array and generation sizes are the oracle's."""
-    T = texts.text_with_repeated_strings(n, repeats, 40, 4, n)
+def test_lists_with_many_suffixes_in_long_runs_are_resolved_on_one_word(emu, n, repeats, followers, words, key_words):
+    """Where more than 12 of 64 places of the sorted list (24 in a long one, which a kernel of its own looks at, from 3000 symbols on in this build) lie
+    in runs of half the in-tile limit or more, the first sort resolves four symbols; otherwise eight, the members of long runs by five
+    passes over their string's number and the code of the next four. Suffix array and generation sizes are the oracle's."""
+    T = texts.text_with_repeated_strings(n, repeats, followers, 4, n)
     got, active, big = emu_sort(emu, T, key_words)
     sa, counts = oracle_lib.prefix_doubling(T, key_words)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
     if key_words == 1:
-        assert emu_sort.passes[0] == 4 and (big[1] > 0) == (words == 2)
+        assert emu_sort.passes[0] == 4 and (emu_sort.passes[1] == 5) == (words == 2)
+
 
 
 def test_the_knob_of_the_settling(emu):
