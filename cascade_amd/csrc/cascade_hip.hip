@@ -1245,9 +1245,11 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
     if (words == 0 && n >= WORDS_AHEAD)
         hipLaunchKernelGGL(choose_words_kernel, dim3(1), dim3(64), 0, s, r.codes, n, r.words_out);
     if (packed)
-        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, true>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, r);
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, true, false>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, r);
+    else if (n < WORDS_AHEAD)
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, false, true>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, r);
     else
-        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, false>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, r);
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, false, false>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, r);
     HIP_TRY(hipGetLastError());
     return CSA_OK;
 }
@@ -1346,9 +1348,9 @@ int sort_long_runs(Launch& L, CodedList& list)
     a.m = (u32)count;
     const dim3 resolve_grid((u32)((count + RESOLVE_TILE - 1) / RESOLVE_TILE));
     if (a.stream)
-        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true, true>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, a);
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true, true, true>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, a);
     else
-        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true, false>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, a);
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, true, false, true>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, a);
     HIP_TRY(hipGetLastError());
     rc = move_table(h->h_pinned + 4, h->counts + 4, 2 * sizeof(u32), s);
     if (rc)

@@ -460,7 +460,8 @@ __global__ __launch_bounds__(64) void choose_words_kernel(const u32* __restrict_
 // all of its own places and writes them in order.
 // PACKED: the words are cut from the code stream of the text, 16 bytes of which hold what 128 bytes of the text do; it fits the last-level
 // cache up to 10^9 symbols of two bits.
-template <int H, bool KEYS, bool PACKED> // H: the longest run that is sorted inside its tile
+// SHORT: lists of fewer than WORDS_AHEAD suffixes, where the slowest tile counts; what that takes costs others 1.5 % of the kernel.
+template <int H, bool KEYS, bool PACKED, bool SHORT> // H: the longest run that is sorted inside its tile
 __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs a)
 {
     constexpr int SPAN = RESOLVE_TILE + 2 * H;
@@ -472,7 +473,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     __shared__ u32 s_many[2];         // some run of the tile has more members, by word
     __shared__ u32 s_ends;            // some member of a run runs off the text inside its words
     __shared__ u32 s_words;
-    __shared__ u32 s_off[2][SPAN / 32]; // bit j, by word: one of the run that starts at place j does
+    __shared__ u32 s_off[SHORT ? 2 : 1][SHORT ? SPAN / 32 : 1]; // bit j, by word: one of the run that starts at place j does
     __shared__ __align__(16) u64 s_key[SPAN];
     __shared__ __align__(16) u32 s_suf[SPAN];
     __shared__ __align__(16) u8 s_tie[SPAN];
@@ -481,10 +482,12 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
         s_many[t] = 0;
     if (t == 2)
         s_ends = 0;
+    const u32 told = KEYS ? TIE_MOST_WORDS : SHORT || a.words ? a.words : *a.words_out;
     if (!KEYS && t < 64u) {
-        const u32 w = a.words ? a.words : a.m >= WORDS_AHEAD ? *a.words_out : many_in_long_runs(a.codes, a.m, HALF_LONG, SHORT_LIST_FEW) ? 1u : 2u;
+        const u32 w = SHORT && told == 0 ? (many_in_long_runs(a.codes, a.m, HALF_LONG, SHORT_LIST_FEW) ? 1u : 2u) : told;
         if (t == 0) {
-            s_words = w;
+            if (SHORT)
+                s_words = w;
             if (blockIdx.x == 0)
                 *a.words_out = w;
         }
@@ -511,7 +514,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
             s_head[j / 64] = b;
     }
     __syncthreads();
-    const u32 words = KEYS ? TIE_MOST_WORDS : s_words;
+    const u32 words = SHORT && !KEYS ? s_words : told;
     if (words < TIE_MOST_WORDS)
         for (int j = t; j < SPAN; j += RESOLVE_BLOCK) // (the thread's own places)
             s_tie[j] = s_tie[j] ? (u8)words : (u8)0;
@@ -581,13 +584,13 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
     }
     __syncthreads();
     const bool ends = s_ends != 0;
-    if (ends) {
+    if (SHORT && ends) {
         for (int j = t; j < 2 * SPAN / 32; j += RESOLVE_BLOCK)
             s_off[j / (SPAN / 32)][j % (SPAN / 32)] = 0;
         __syncthreads();
     }
     // One word of all elements that still have company: refines their runs. Whoever runs off the text inside the word ties with
-    // nobody and comes before those with the same padded word, shortest first. (Only the runs with such a member are looked at that way: a tile
+    // nobody and comes before those with the same padded word, shortest first. (SHORT: only the runs with such a member are looked at that way: a tile
     // is as slow as its slowest run, and a short text as its slowest tile. 10^5 symbols of phrases: 168 us with all runs of a tile that
     // holds one of the last suffixes, 55 without.)
     auto refine = [&](int w) {
@@ -598,11 +601,11 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
                 s_suf[at[k]] = x[k];
                 if (w == 1 || !((owners >> k) & 1u))
                     s_key[at[k]] = w == 0 ? w0[k] : w1[k];
-                if (ends && (u64)x[k] + ctx >= n && !((longs >> k) & 1u))
+                if (SHORT && ends && (u64)x[k] + ctx >= n && !((longs >> k) & 1u))
                     atomicOr(&s_off[w][first[k] / 32], 1u << (first[k] & 31));
             }
         __syncthreads();
-        const bool many = s_many[w] != 0;
+        const bool many = s_many[w] != 0 && (SHORT || !ends);
         if (many) {
             for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (places whose words were not wanted hold anything: no run looked at below has any)
                 const u64 down = __ballot(j > 0 && s_key[j] < s_key[j - 1]), diff = __ballot(j > 0 && s_key[j] != s_key[j - 1]);
@@ -618,7 +621,7 @@ __global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs
             const int f = first[k], l = last[k], j = at[k];
             if ((longs >> k) & 1u || l - f <= 1)
                 continue;
-            const bool own = w == 0 && ((owners >> k) & 1u), off = ends && ((s_off[w][f / 32] >> (f & 31)) & 1u);
+            const bool own = w == 0 && ((owners >> k) & 1u), off = ends && (!SHORT || ((s_off[w][f / 32] >> (f & 31)) & 1u));
             int nf = f, nl = l, place = j;
             if (own) { // one string: those that run off the text come first as they stand
                 if (off) {
