@@ -781,8 +781,8 @@ int deferred_rank_update(Launch& L, const DeferBuffers& buf, u32 n)
 // A list of an eighth of the partition or more goes through two radix passes on the position bits above a window that fits LDS; the windows are
 // read, brought up to date and written back whole. A shorter one goes through one pass and a plain scatter that stays inside one
 // window of 1 << WINDOW_LOG2 ranks at a time. Per pair the scatter costs 19 ps, the second pass and the placing 8, and reading and writing
-// every rank of the partition 1.8 (10^8 bytes of text, two such updates of 88.2 and 24.0 M pairs: the sort 16.4 ms with the scatter,
-// 15.7 with the windows).
+// every rank of the partition 1.8 (10^8 bytes of text, two such updates of 88.2 and 24.0 M pairs: device time of the sort 15.45 ms with
+// the scatter, 14.82 with the windows, three processes of each in turn within 0.03).
 int windowed_rank_update(Launch& L, const u32* pos, const DeferBuffers& buf, u32 m, u32 n)
 {
     csa_handle* h = L.h;
@@ -1070,9 +1070,10 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen, const 
     return CSA_OK;
 }
 
-// Texts of two-bit symbols from this length on may start from narrow keys. (They gain at every length measured: 2^25 + 5 independent letters
-// 2.0 -> 1.2 ms, 4 * 10^8, a fifth of them copies, 28.4 -> 21.4. Up to 2^24 the first sort keeps the eight passes that its statistics
-// have always shown.)
+// Texts of two-bit symbols from this length on may start from narrow keys: 2^25 + 5 independent letters 2.0 -> 1.2 ms, 4 * 10^8, a fifth of
+// them copies, 28.4 -> 21.4. The line is not where they begin to pay: they gain at every length measured (ms, wide and narrow: 20000 letters
+// with copies 0.27, 0.26; 2^17 0.29, 0.27; 2^20 0.40, 0.35; 2^22 0.56, 0.48; 2^24 1.50, 1.14), and shorter texts keep wide ones
+// because callers have been told of eight passes for them. Texts of symbols of one or four bits, and keys of 48, have not been tried.
 #ifndef CSA_NARROW_MIN
 #define CSA_NARROW_MIN ((1u << 24) + 1)
 #endif
