@@ -1244,7 +1244,7 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
     r.tail = tail;
     const dim3 resolve_grid((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE));
     if (words == 0 && n >= WORDS_AHEAD)
-        hipLaunchKernelGGL(choose_words_kernel, dim3(1), dim3(64), 0, s, r.codes, n, r.words_out);
+        hipLaunchKernelGGL(choose_words_kernel, dim3(1), dim3(LONG_LIST_PLACES), 0, s, r.codes, n, r.words_out);
     if (packed)
         hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, true, false>), resolve_grid, dim3(RESOLVE_BLOCK), 0, s, r);
     else if (n < WORDS_AHEAD)

@@ -429,24 +429,33 @@ __device__ __forceinline__ u64 second_word(const ResolveArgs& a, u32 x)
     return y < a.n ? packed_window(a.stream, y * a.sym_bits, 32u) : 0ull;
 }
 
-// A list many of whose suffixes lie in runs of RESOLVE_MAX / 2 or more is resolved on one word. Members of runs that are too long for a tile would have to be
-// sorted by the second one, those of others long for a tile compared by it one by one, and the generation after, with the
-// ranks of all, costs no more. (Sorts, ms, by two words, one, and before there were two: 33000 symbols of ten phrases 0.83, 0.60, 0.65; 130000 of
-// a hundred 1.01, 0.85, 0.92; 400000 of 300 1.33, 1.12, 1.09; 400000 symbols Zipf(2) 0.80, 0.69, 0.73; 4 M of written text in 16-bit symbols
-// 1.50, 1.38, 1.43.) The line lies at 12 of 64 places in short lists (with 20 the third of these stays at 1.35) and at 24 in long ones, whose second
-// words are lines of the text, which generation 1 would read as lines of ranks: 2^26 symbols of runs and Zipf(1.3), 12 places 7.4 ms, 24 to 64
-// 6.4; 2^26 Zipf(1.3) alone 6.0 and 5.0; 2 * 10^7 Zipf(1.5) 2.9 with 24, 4.0 with 36. Token texts have 4 to 6 places.
-constexpr u32 HALF_LONG = RESOLVE_MAX / 2, SHORT_LIST_FEW = 12, LONG_LIST_FEW = 24;
+// A list many of whose suffixes lie in runs of RESOLVE_MAX / 2 or more is resolved on one word.
+// Short lists, 12 of 64 places: members of runs that are too long for a tile would have to be sorted by the second word, those of others long for a
+// tile compared by it one by one, and the generation after, with the ranks of all, costs no more. (Sorts, ms, by two words, by one,
+// and before there were two: 33000 symbols of ten phrases 0.83, 0.60, 0.65; 130000 of a hundred 1.01, 0.85, 0.92; 400000 of 300 1.33, 1.12, 1.09,
+// which a limit of 20 leaves at 1.35; 400000 symbols Zipf(2) 0.80, 0.69, 0.73.)
+// Long lists, 543 of 1024 places, which is about where half of the list is in runs of more than RESOLVE_MAX and sort_long_runs gives it up; up to there the
+// second word pays, since generation 1 would read as many lines. (ms by two words and by one, and the share of the places: 2^28 symbols
+// Zipf(1.4) 0.51 25.4, 30.3; 2^29 of runs and Zipf(1.3) 0.45 52.0, 59.8; 2^26 Zipf(1.5) 0.58 9.2, 8.6; 2^28 0.66 37.9, 34.4; 2^26 Zipf(2) 0.93 14.2, 13.9;
+// 5 * 10^6 of written text in 16-bit symbols 0.65 1.80, 1.63. Token texts have 0.04.)
+constexpr u32 HALF_LONG = RESOLVE_MAX / 2, SHORT_LIST_FEW = 12, LONG_LIST_PLACES = 1024, LONG_LIST_FEW = 543;
 
-// Lists of WORDS_AHEAD suffixes or more are looked at by a wave of its own: a launch costs 3 us, and the look of every tile 2 % of the sort of 2^28
+// Lists of WORDS_AHEAD suffixes or more are looked at by a workgroup of its own: a launch costs 4 us, and the look of every tile 2 % of the sort of 2^28
 // tokens (11.35 -> 11.6 ms).
 constexpr u32 WORDS_AHEAD = CSA_WORDS_AHEAD;
 
-__global__ __launch_bounds__(64) void choose_words_kernel(const u32* __restrict__ codes, u32 m, u32* words_out)
+__global__ __launch_bounds__(LONG_LIST_PLACES) void choose_words_kernel(const u32* __restrict__ codes, u32 m, u32* words_out)
 {
-    const bool one = many_in_long_runs(codes, m, HALF_LONG, LONG_LIST_FEW);
+    __shared__ u32 s_in;
     if (threadIdx.x == 0)
-        *words_out = one ? 1u : 2u;
+        s_in = 0;
+    __syncthreads();
+    const u64 b = __ballot(in_long_run(codes, m, HALF_LONG, threadIdx.x, LONG_LIST_PLACES));
+    if ((threadIdx.x & 63u) == 0 && b)
+        atomicAdd(&s_in, (u32)__popcll(b));
+    __syncthreads();
+    if (threadIdx.x == 0)
+        *words_out = s_in > LONG_LIST_FEW ? 1u : 2u;
 }
 
 // The runs of equal codes (KEYS = false: the list of all suffixes) or of equal keys (KEYS = true: the members of the long runs, sorted

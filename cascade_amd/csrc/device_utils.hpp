@@ -213,15 +213,21 @@ __global__ __launch_bounds__(256) void move_tables_kernel(TableGroup g)
 
 // ---- long runs in a sorted list ----
 
-// Whether many entries of a sorted list lie in long runs of equal ones: more than `few` of 64 of its places (one wave looks; the answer is
-// the same for every wave) have an equal one `half` places on at one side.
+// Whether place `at` of `places` evenly spread ones of a sorted list lies in a long run of equal entries: one that reaches `half` places on at one
+// side of it.
+template <typename T>
+__device__ __forceinline__ bool in_long_run(const T* __restrict__ sorted, u32 m, u32 half, u32 at, u32 places)
+{
+    const u32 e = (u32)((u64)m * at / places);
+    const T c = sorted[e];
+    return (e >= half && sorted[e - half] == c) || ((u64)e + half < m && sorted[e + half] == c);
+}
+
+// Whether more than `few` of 64 places do. One wave looks; the answer is the same for every wave.
 template <typename T>
 __device__ __forceinline__ bool many_in_long_runs(const T* __restrict__ sorted, u32 m, u32 half, u32 few)
 {
-    const u32 e = (u32)((u64)m * (threadIdx.x & 63u) / 64u);
-    const T c = sorted[e];
-    const bool in = (e >= half && sorted[e - half] == c) || ((u64)e + half < m && sorted[e + half] == c);
-    return (u32)__popcll(__ballot(in)) > few;
+    return (u32)__popcll(__ballot(in_long_run(sorted, m, half, threadIdx.x & 63u, 64u))) > few;
 }
 
 // ---- wave-wide reduction ----

@@ -917,10 +917,10 @@ def test_what_settling_copies_may_cost(emu, text, size, doubled):
     assert (emu_sort.rank_update[0] != 0) == doubled
 
 
-@pytest.mark.parametrize("n,repeats,followers,words", [(2900, [70], 40, 2), (2900, [100] * 3, 40, 1), (3900, [100] * 2, 40, 2), (3900, [100] * 4, 2, 1)])
+@pytest.mark.parametrize("n,repeats,followers,words", [(2900, [70], 40, 2), (2900, [100] * 3, 40, 1), (3900, [100] * 2, 40, 2), (3900, [107] * 4, 2, 1)])
 @pytest.mark.parametrize("key_words", [1, 2, 4])
 def test_lists_with_many_suffixes_in_long_runs_are_resolved_on_one_word(emu, n, repeats, followers, words, key_words):
-    """Where more than 12 of 64 places of the sorted list (24 in a long one, which a kernel of its own looks at, from 3000 symbols on in this build) lie
+    """Where more than 12 of 64 places of the sorted list (543 of 1024 of a long one, which a kernel of its own looks at, from 3000 symbols on in this build) lie
     in runs of half the in-tile limit or more, the first sort resolves four symbols; otherwise eight, the members of long runs by five
     passes over their string's number and the code of the next four. Suffix array and generation sizes are the oracle's."""
     T = texts.text_with_repeated_strings(n, repeats, followers, 4, n)
