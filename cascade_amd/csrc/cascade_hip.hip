@@ -1141,11 +1141,12 @@ bool codes_pay(const ProbeCounts& c, u32 n)
     return cost < 18.0 + 2.5e7 / n;
 }
 
-// Where the codes live until the first pass has read them: by virtual position, with the flags by text position behind them.
+// key[1] until the list is ranked: the codes by virtual position, which the first pass reads, the flags by text position behind them, and the
+// ties of the sorted list behind those. Each starts at a multiple of 16 bytes, for the loads that wide; 5.125 bytes a suffix and 31 are fewer than 8 a
+// suffix rounded up to 256.
 u32* codes_of(const csa_handle* h) { return reinterpret_cast<u32*>(h->key[1]); }
-u8* own_of(const csa_handle* h) { return reinterpret_cast<u8*>(h->key[1]) + 4 * h->cap; }
-// The ties of the sorted list live behind them, until it is ranked (cap is a multiple of 256).
-u8* ties_of(const csa_handle* h) { return own_of(h) + (h->cap / 8 + 255) / 256 * 256; }
+u8* own_of(const csa_handle* h) { return reinterpret_cast<u8*>(h->key[1]) + (4 * h->cap + 15) / 16 * 16; }
+u8* ties_of(const csa_handle* h) { return own_of(h) + ((h->cap + 7) / 8 + 15) / 16 * 16; }
 
 int code_suffixes(Launch& L, const u16* d_text, u32 n, u32 tail)
 {

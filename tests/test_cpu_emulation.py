@@ -948,3 +948,21 @@ def test_the_knob_of_the_settling(emu):
         emu.csa_destroy(h)
         seen.append((int(st.rank_update[0]), out.tobytes()))
     assert [s[0] != 0 for s in seen] == [False, True, False, True, False] and len({s[1] for s in seen}) == 1
+
+
+def test_wide_loads_are_aligned_for_every_capacity():
+    """Handles of every size modulo 16, the smallest among them: the columns that share an array start where 16-byte loads may. (A build that traps at an
+    access which is not aligned as its type says, in a process of its own.)"""
+    import sys
+    code = ("import sys; sys.path[:0] = [%r, %r]\n"
+            "import numpy as np, oracle_lib, texts, test_cpu_emulation as t\n"
+            "lib = t.load_emulation('libcascade_emu_align.so')\n"
+            "for n in list(range(1, 40)) + list(range(2041, 2058)) + [4099, 7001]:\n"
+            "    for symbols in (60000, 3):\n"
+            "        T = texts.text_of_copies(n, symbols, n) if n > 30 else np.arange(n, dtype=np.uint16) %% symbols * 300\n"
+            "        got, active, _ = t.emu_sort(lib, T, 1)\n"
+            "        sa, counts = oracle_lib.prefix_doubling(T, 1)\n"
+            "        assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts, n\n"
+            % (os.path.dirname(os.path.abspath(__file__)), os.path.dirname(os.path.dirname(os.path.abspath(__file__)))))
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert run.returncode == 0, (run.returncode, run.stderr[-2000:])
