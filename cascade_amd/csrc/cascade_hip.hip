@@ -2,6 +2,7 @@
 // declared in include/cascade_hip.h. gfx950 only.
 #include "../../include/cascade_hip.h"
 
+#include "bucket_sort.hpp"
 #include "chains.hpp"
 #include "coded_keys.hpp"
 #include "copies.hpp"
@@ -184,7 +185,7 @@ static_assert(SMALL_MAXG_HI >= SMALL_MAXG, "the higher group limit is the higher
 constexpr u32 TICKET_POOL = 4096;
 constexpr u32 PROBE_FEW = 1u << 15;           // suffixes that are probed, whose table ...
 constexpr u64 PROBE_TABLE = 2ull * PROBE_FEW; // ... is one of the handle's own
-constexpr u64 CODE_TABLE_WORDS = SYMBOLS + RESOLVE_MARK_WORDS + 8 + 2 * PROBE_TABLE + SYMBOLS + 4; // symbol counts, marks, ProbeCounts, its table, shares (and entry [SYMBOLS])
+constexpr u64 CODE_TABLE_WORDS = SYMBOLS + RESOLVE_MARK_WORDS + PROBE_WORDS + 2 * PROBE_TABLE + SYMBOLS + 4; // symbol counts, marks, ProbeCounts, its table, shares (and entry [SYMBOLS])
 // Texts of at least this many symbols are probed before they are sorted by codes (probe_codes_kernel, 12 us with its round trip). Shorter
 // ones have no runs of one code that are too long for a tile, out of order and not planted: strings of four symbols that are
 // rare enough to share a code with others can come up 256 times from there on. Generation 0 of records of four symbols, one of
@@ -451,11 +452,15 @@ void launch_onesweep(const csa_handle* h, OnesweepArgs& a, hipStream_t s)
         launch_onesweep_shape<SRC, SORT_BLOCK, VALS>(tile_order_of(h), a, s);
 }
 
+// a.bits > RADIX_BITS: wide workgroups only (the look-back words are sized for RADIX_BINS a tile of half the size)
 template <int SRC>
 void launch_onesweep32(const csa_handle* hh, OnesweepArgs& a, hipStream_t s)
 {
     const TileOrder h = tile_order_of(hh);
-    if (wide_workgroups(a)) {
+    if (a.bits > RADIX_BITS) {
+        set_tile_order(h, a, SORT_WIDE_BLOCK * SORT32_ITEMS);
+        hipLaunchKernelGGL((onesweep_kernel<u32, SORT_WIDE_BLOCK, SORT32_ITEMS, SRC, 0, true, RADIX_BITS + 1>), dim3(a.tiles), dim3(SORT_WIDE_BLOCK), 0, s, a);
+    } else if (wide_workgroups(a)) {
         set_tile_order(h, a, SORT_WIDE_BLOCK * SORT32_ITEMS);
         hipLaunchKernelGGL((onesweep_kernel<u32, SORT_WIDE_BLOCK, SORT32_ITEMS, SRC, 0>), dim3(a.tiles), dim3(SORT_WIDE_BLOCK), 0, s, a);
     } else {
@@ -551,7 +556,7 @@ int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64
             hipLaunchKernelGGL(radix_hist_kernel, dim3(hist_blocks(256 * 16, n)), dim3(256), 0, s, ha);
         }
     }
-    hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, plan.num_passes);
+    hipLaunchKernelGGL(radix_scan_hist_kernel<RADIX_BINS>, dim3(1), dim3(RADIX_BINS), 0, s, h->ghist, h->digit_base, plan.num_passes);
     HIP_TRY(hipGetLastError());
     // (the digits of K-gram keys are the two bytes of a symbol, four times: where both take several values no pass is skipped)
     const bool all_run = src == SRC_TEXT && !source->byte_wide;
@@ -744,7 +749,7 @@ int deferred_rank_update(Launch& L, const DeferBuffers& buf, u32 n)
             }
         }
         HIP_TRY(hipMemcpyAsync(h->ghist, h_hist, n_pass * RADIX_BINS * sizeof(u32), hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, n_pass);
+        hipLaunchKernelGGL(radix_scan_hist_kernel<RADIX_BINS>, dim3(1), dim3(RADIX_BINS), 0, s, h->ghist, h->digit_base, n_pass);
         for (int p = 0; p < n_pass; ++p) {
             OnesweepArgs a;
             a.keys_in = in_recs;
@@ -818,7 +823,7 @@ int windowed_rank_update(Launch& L, const u32* pos, const DeferBuffers& buf, u32
         for (int p = 0; p < passes; ++p)
             hipLaunchKernelGGL(position_hist_kernel, dim3(hist_blocks(256 * 16, m)), dim3(256), 0, s, pos, m, shift[p], bits[p],
                                h->ghist + p * RADIX_BINS);
-        hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, passes);
+        hipLaunchKernelGGL(radix_scan_hist_kernel<RADIX_BINS>, dim3(1), dim3(RADIX_BINS), 0, s, h->ghist, h->digit_base, passes);
         u32* const out_pos[2] = {buf.t1_pos, buf.t2_pos};
         u32* const out_val[2] = {buf.t1_val, buf.t2_val};
         for (int p = 0; p < passes; ++p) {
@@ -1015,6 +1020,63 @@ CodeTables code_tables(const csa_handle* h)
     return c;
 }
 
+// Digits of a sort by codes whose lower bits are sorted in buckets (bucket_sort.hpp): as many upper bits as leave BUCKET_AVERAGE suffixes a bucket or
+// fewer, by two passes of eight bits or two of nine. Longer texts take all digits.
+#ifndef CSA_BUCKETS_MIN
+#define CSA_BUCKETS_MIN ((1u << 24) + 1)
+#endif
+#ifndef CSA_TWO_PASS_LOG2
+#define CSA_TWO_PASS_LOG2 16
+#endif
+#ifndef CSA_BUCKET_AVERAGE
+#define CSA_BUCKET_AVERAGE 4096
+#endif
+constexpr u32 BUCKET_AVERAGE = CSA_BUCKET_AVERAGE;
+constexpr CodeDigits ALL_DIGITS = {CODE_PASSES, RADIX_BITS, {0, 8, 16, 24}, 0};
+
+CodeDigits bucket_digits(u32 n, bool packed)
+{
+    u32 log2 = 1;
+    while ((n >> log2) > BUCKET_AVERAGE)
+        ++log2;
+    // (the digits of packed keys are counted by eight bits: up to nine tenths of BUCKET_MAX)
+    if (packed && log2 == CSA_TWO_PASS_LOG2 + 1 && (n >> CSA_TWO_PASS_LOG2) <= BUCKET_MAX / 10 * 9)
+        log2 = CSA_TWO_PASS_LOG2;
+    if (log2 <= CSA_TWO_PASS_LOG2)
+        return CodeDigits{2, RADIX_BITS, {16, 24}, log2};
+    if (log2 <= 18 && !packed && n >= SORT_WIDE_MIN && n >= CODE_AHEAD_MAX) // (codes that are made ahead have their digits counted by eight bits)
+        return CodeDigits{2, RADIX_BITS + 1, {14, 23}, log2};
+    return ALL_DIGITS;
+}
+
+// Of the suffixes that are probed, one in so many (and one less here) is counted by its bucket: 16 to 31 a bucket on average where there are more (all of
+// 62500 on 256 counters: 30 us instead of 14).
+u32 bucket_skip(u32 n, const CodeDigits& digits)
+{
+    u32 skip = 1;
+    while ((probed_suffixes(n) >> digits.buckets_log2) / skip >= 32)
+        skip *= 2;
+    return skip - 1u;
+}
+
+// The buckets of a sample of the suffixes are counted too where the lower digits may be sorted in them, in `room` (zeroed by the caller).
+void probe_buckets(ProbeArgs& a, const CodeDigits& digits, u32* room)
+{
+    if (digits.buckets_log2 == 0)
+        return;
+    a.buckets = room;
+    a.bucket_shift = 32u - digits.buckets_log2;
+    a.bucket_skip = bucket_skip(a.n, digits);
+    const u32 full = BUCKET_MAX / 16 * 18 / (a.n / a.taken * (a.bucket_skip + 1u)); // (the average bucket shows half of that)
+    a.full_from = full > 2 ? full : 2;
+}
+
+// Buckets that do not fit are sorted by radix passes after all: from a tenth of the suffixes on all passes are made at once.
+bool buckets_fit(const ProbeCounts& c, u32 n, const CodeDigits& digits)
+{
+    return (u64)c.packed * 10 * (bucket_skip(n, digits) + 1u) <= probed_suffixes(n);
+}
+
 // What a sort by codes starts from: the shares of the symbols, and for texts of PROBE_MIN symbols or more what a sample of the suffixes
 // (probed_suffixes) shows about shared codes, on its way to *seen; ev_gen[1] tells that it is there. A large sample's table is
 // key[0], which holds nothing yet.
@@ -1042,10 +1104,15 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen, const 
         const bool few = a.taken <= PROBE_FEW;
         a.table = few ? c.table : reinterpret_cast<unsigned long long*>(h->key[0]);
         zeros += sizeof(ProbeCounts);
-        if (few)
-            zeros += sizeof(u64) << a.table_log2;
-        else
-            HIP_TRY(hipMemsetAsync(a.table, 0, sizeof(u64) << a.table_log2, s));
+        u64 large_zeros = 0;
+        (few ? zeros : large_zeros) += sizeof(u64) << a.table_log2;
+        if (n >= CSA_BUCKETS_MIN) {
+            const CodeDigits digits = bucket_digits(n, false);
+            probe_buckets(a, digits, reinterpret_cast<u32*>(reinterpret_cast<unsigned char*>(h->key[0]) + large_zeros));
+            large_zeros += sizeof(u32) << digits.buckets_log2;
+        }
+        if (large_zeros)
+            HIP_TRY(hipMemsetAsync(h->key[0], 0, large_zeros, s));
     }
     HIP_TRY(hipMemsetAsync(c.counts, 0, zeros, s));
     // one chunk in 16, at least SAMPLE_CHUNKS_MIN of them (or all there are) and at most SAMPLE_CHUNKS_MAX
@@ -1081,7 +1148,8 @@ int share_symbols(Launch& L, const u16* d_text, u32 n, ProbeCounts* seen, const 
 // Whether the first sort of a packed text takes narrow keys, 32 bits of the code stream, and reads the next 32 for the suffixes that tie
 // on them (sort_by_codes): four passes over 8-byte pairs instead of eight over 12-byte ones save 27 ps a suffix, less 8 for the second half; a member of a
 // run that is too long for a tile costs 100 (it is collected and sorted again), and a sample of the suffixes shows how many there are.
-int narrow_keys_pay(Launch& L, const TextSource& ps, u32 n, bool* pay)
+// *digits: the radix passes that they take.
+int narrow_keys_pay(Launch& L, const TextSource& ps, u32 n, bool* pay, CodeDigits* digits)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -1098,7 +1166,9 @@ int narrow_keys_pay(Launch& L, const TextSource& ps, u32 n, bool* pay)
     a.counts = c.probe;
     a.stream = ps.stream;
     a.sym_bits = ps.sym_bits;
-    HIP_TRY(hipMemsetAsync(a.table, 0, sizeof(u64) << a.table_log2, s));
+    const CodeDigits in_buckets = bucket_digits(n, true);
+    probe_buckets(a, in_buckets, reinterpret_cast<u32*>(a.table + (1ull << a.table_log2)));
+    HIP_TRY(hipMemsetAsync(a.table, 0, (sizeof(u64) << a.table_log2) + (sizeof(u32) << in_buckets.buckets_log2), s));
     int rc = move_table(c.probe, nullptr, sizeof(ProbeCounts), s);
     if (rc)
         return rc;
@@ -1107,6 +1177,7 @@ int narrow_keys_pay(Launch& L, const TextSource& ps, u32 n, bool* pay)
         return rc;
     HIP_TRY(hipStreamSynchronize(s));
     *pay = (u64)seen->crowded * 6 <= a.taken;
+    *digits = buckets_fit(*seen, n, in_buckets) ? in_buckets : ALL_DIGITS;
     return CSA_OK;
 }
 
@@ -1148,17 +1219,20 @@ u32* codes_of(const csa_handle* h) { return reinterpret_cast<u32*>(h->key[1]); }
 u8* own_of(const csa_handle* h) { return reinterpret_cast<u8*>(h->key[1]) + (4 * h->cap + 15) / 16 * 16; }
 u8* ties_of(const csa_handle* h) { return own_of(h) + ((h->cap + 7) / 8 + 15) / 16 * 16; }
 
-int code_suffixes(Launch& L, const u16* d_text, u32 n, u32 tail)
+int code_suffixes(Launch& L, const u16* d_text, u32 n, u32 tail, const CodeDigits& digits)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
     const u32* const cum = code_tables(h).cum;
-    if (n >= SORT_WIDE_MIN) // 2048 tiles of the wide workgroups: four for each of those a device holds at a time
-        hipLaunchKernelGGL(code_suffixes_kernel<CODE_WIDE_BLOCK>, dim3(hist_blocks(CODE_WIDE_BLOCK * CODE_ITEMS, n)), dim3(CODE_WIDE_BLOCK), 0,
-                           s, d_text, n, tail, cum, codes_of(h), own_of(h), h->ghist);
+    auto launch = [&](auto kernel, int block) {
+        hipLaunchKernelGGL(kernel, dim3(hist_blocks(block * CODE_ITEMS, n)), dim3(block), 0, s, d_text, n, tail, cum, codes_of(h), own_of(h), digits, h->ghist);
+    };
+    if (digits.passes == 2)
+        launch(code_suffixes_kernel<CODE_WIDE_BLOCK, 2>, CODE_WIDE_BLOCK);
+    else if (n >= SORT_WIDE_MIN) // 2048 tiles of the wide workgroups: four for each of those a device holds at a time
+        launch(code_suffixes_kernel<CODE_WIDE_BLOCK, CODE_PASSES>, CODE_WIDE_BLOCK);
     else
-        hipLaunchKernelGGL(code_suffixes_kernel<CODE_BLOCK>, dim3(hist_blocks(CODE_BLOCK * CODE_ITEMS, n)), dim3(CODE_BLOCK), 0, s, d_text, n,
-                           tail, cum, codes_of(h), own_of(h), h->ghist);
+        launch(code_suffixes_kernel<CODE_BLOCK, CODE_PASSES>, CODE_BLOCK);
     HIP_TRY(hipGetLastError());
     return CSA_OK;
 }
@@ -1173,23 +1247,83 @@ struct CodedList {
     bool long_left;   // there are runs that are too long for a tile on both words
 };
 
+// The bits of the codes below the passes of `digits`, in place (bucket_sort.hpp). *finished = false: too many suffixes are in buckets that do
+// not fit, and nothing that is used has changed. Works in the group tables, and in key[2], idx[3] and idx[4].
+int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* codes, u32* sufs, const u32* top_base, int* passes, bool* finished)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    BucketArgs a;
+    memset(&a, 0, sizeof(a));
+    a.codes = codes;
+    a.sufs = sufs;
+    a.n = n;
+    a.low_bits = 32u - digits.buckets_log2;
+    a.buckets = 1u << digits.buckets_log2;
+    a.starts = h->gprim[0];
+    a.top_base = top_base;
+    a.top_shift = digits.shift[digits.passes - 1];
+    a.over = h->counts + 8;
+    a.over_list = h->gprim[1];
+    a.tail = tail;
+    a.crowded = h->counts + 10;
+    a.crowded_list = h->gstart[0]; // (done with before over_before)
+    a.over_before = h->gstart[0];
+    a.over_tiles = h->gstart[1];
+    hipLaunchKernelGGL(bucket_starts_kernel, dim3(a.buckets / (STARTS_BLOCK - 1) + 1), dim3(STARTS_BLOCK), 0, s, a);
+    int rc = move_table(h->h_pinned + 8, a.over, 2 * sizeof(u32), s);
+    if (rc)
+        return rc;
+    HIP_TRY(hipEventRecord(h->ev_gen[2], s)); // (recorded again when a generation ends)
+    hipLaunchKernelGGL(finish_buckets_kernel, dim3(a.buckets), dim3(BUCKET_BLOCK), 0, s, a);
+    hipLaunchKernelGGL(finish_crowded_kernel, dim3(a.buckets < CROWDED_BLOCKS ? a.buckets : CROWDED_BLOCKS), dim3(BUCKET_BLOCK), 0, s, a);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipEventSynchronize(h->ev_gen[2]));
+    const u32 over = h->h_pinned[8], over_buckets = h->h_pinned[9];
+    *finished = over <= n / 4 && over <= h->cap / 2;
+    if (over == 0 || !*finished)
+        return CSA_OK;
+    u64* const K[2] = {h->key[2], h->key[2] + h->cap / 2};
+    u32* const V[2] = {h->idx[3], h->idx[4]};
+    a.over_keys = K[0];
+    a.over_sufs = V[0];
+    hipLaunchKernelGGL(over_before_kernel, dim3((a.buckets + OVER_TILE - 1) / OVER_TILE), dim3(OVER_TILE), 0, s, a);
+    hipLaunchKernelGGL(over_move_kernel<false>, dim3(over_buckets * OVER_SLICES), dim3(256), 0, s, a);
+    int in_out = 0, run = 0;
+    rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], V[0], K[1], V[1], over, make_plan(0, 32), &in_out, &run);
+    if (rc)
+        return rc;
+    *passes += run;
+    a.over_keys = K[in_out];
+    a.over_sufs = V[in_out];
+    hipLaunchKernelGGL(over_move_kernel<true>, dim3(over_buckets * OVER_SLICES), dim3(256), 0, s, a);
+    HIP_TRY(hipGetLastError());
+    return CSA_OK;
+}
+
 // Generation 0 on codes (coded_keys.hpp): the suffixes of the text in the order of their first `words` words of four symbols (0: two, or one
 // if many lie in long runs), with their ties beside them; code_suffixes ran before. Sorts (codes, idx[0]) <-> (codes', idx[1]) and resolves the runs of equal codes into
 // idx[1]; the codes live in the halves of key[0]. What long runs leave open is finished by sort_marked_runs and sort_long_runs.
 // packed: the codes are narrow keys, cut from its stream, of word_syms symbols (and so are the words).
-int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, CodedList& list, const TextSource* packed = nullptr, u32 word_syms = 4)
+// digits: the radix passes; `counted` says whose counts ghist holds, theirs or those of all digits.
+int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, CodedList& list, const CodeDigits& counted, const CodeDigits& digits,
+                  int* passes, const TextSource* packed = nullptr, u32 word_syms = 4)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
-    hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, h->ghist, h->digit_base, CODE_PASSES);
+    if (counted.bits == RADIX_BITS)
+        hipLaunchKernelGGL(radix_scan_hist_kernel<RADIX_BINS>, dim3(1), dim3(RADIX_BINS), 0, s, h->ghist, h->digit_base, (int)counted.passes);
+    else
+        hipLaunchKernelGGL(radix_scan_hist_kernel<2 * RADIX_BINS>, dim3(1), dim3(2 * RADIX_BINS), 0, s, h->ghist, h->digit_base, (int)counted.passes);
     u32* const sorted[2] = {reinterpret_cast<u32*>(h->key[0]), reinterpret_cast<u32*>(h->key[0]) + h->cap};
-    static_assert(CODE_PASSES % 2 == 0, "the sorted codes end in the first half of key[0], their suffixes in idx[0]");
-    for (int p = 0; p < CODE_PASSES; ++p) {
+    const u32* top_base = nullptr;
+    for (u32 p = 0; p < digits.passes; ++p) {
+        const u32 out = (digits.passes - 1 - p) & 1, in = out ^ 1; // the sorted codes end in the first half of key[0], their suffixes in idx[0]
         OnesweepArgs a;
-        a.keys_in = p == 0 ? codes_of(h) : sorted[p & 1];
-        a.vals_in = h->idx[p & 1];
-        a.keys_out = sorted[(p + 1) & 1];
-        a.vals_out = h->idx[(p + 1) & 1];
+        a.keys_in = p == 0 ? codes_of(h) : sorted[in];
+        a.vals_in = h->idx[in];
+        a.keys_out = sorted[out];
+        a.vals_out = h->idx[out];
         a.n = n;
         a.text_n = n;
         a.tail = tail;
@@ -1200,9 +1334,10 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
             a.sym_bits = packed->sym_bits;
             a.key_bits = 32;
         }
-        a.shift = 8 * p;
-        a.bits = 8;
-        a.digit_base = h->digit_base + p * RADIX_BINS;
+        a.shift = (int)digits.shift[p];
+        a.bits = (int)digits.bits;
+        top_base = h->digit_base + ((counted.buckets_log2 ? p : digits.shift[p] / RADIX_BITS) << digits.bits);
+        a.digit_base = top_base;
         a.lookback = h->lookback;
         a.lookback_groups = h->lookback + h->lookback_tile_words;
         a.epoch = next_epoch(h);
@@ -1220,6 +1355,21 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
         });
         if (rc)
             return rc;
+    }
+    *passes = CODE_PASSES; // (the digits that are sorted in buckets among them)
+    if (digits.buckets_log2) {
+        bool finished = false;
+        int rc = finish_buckets(L, digits, n, tail, sorted[0], h->idx[0], top_base, passes, &finished);
+        if (rc)
+            return rc;
+        if (!finished) { // (a sample had shown fewer suffixes in buckets that do not fit)
+            if (counted.buckets_log2) {
+                HIP_TRY(hipMemsetAsync(h->ghist, 0, CODE_BINS * sizeof(u32), s));
+                if ((rc = code_suffixes(L, d_text, n, tail, ALL_DIGITS)) != CSA_OK)
+                    return rc;
+            }
+            return sort_by_codes(L, d_text, n, tail, words, list, ALL_DIGITS, ALL_DIGITS, passes, packed, word_syms);
+        }
     }
     memset(&list, 0, sizeof(list));
     list.words = words;
@@ -1744,7 +1894,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     // The byte histograms of the text come first: they tell whether the alphabet is small enough for keys of more than four
     // symbols. (The digit counts are zeroed with them.)
     TableGroup zeros = {};
-    add_table(zeros, h->counts, nullptr, 6 * sizeof(u32));
+    add_table(zeros, h->counts, nullptr, 11 * sizeof(u32));
     add_table(zeros, h->ghist, nullptr, (MAX_PASSES + 2) * RADIX_BINS * sizeof(u32));
     int rc = move_tables(zeros, s);
     if (rc)
@@ -1778,6 +1928,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     TextSource ps;
     memset(&ps, 0, sizeof(ps));
     bool narrow = false; // keys of half as many packed symbols
+    const bool in_buckets = n >= CSA_BUCKETS_MIN && h->pack_symbols;
+    CodeDigits digits = ALL_DIGITS, counted = ALL_DIGITS;
     if (pp.enabled) {
         // the code stream lives in rank[], which nothing uses before the sorted list is ranked
         u32* const stream = h->rank;
@@ -1791,7 +1943,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         hipLaunchKernelGGL(encode_text_kernel, dim3((u32)(enc_blocks < 4096 ? enc_blocks : 4096)), dim3(ENCODE_BLOCK), 0, s, d_text, n,
                            pp.codes, stream, ps.words, bytehist);
         HIP_TRY(hipGetLastError());
-        if (n >= CSA_NARROW_MIN && ps.sym_bits == 2 && ps.key_bits == 64 && pp.skipped > 0 && (rc = narrow_keys_pay(L, ps, n, &narrow)) != CSA_OK)
+        if (n >= CSA_NARROW_MIN && ps.sym_bits == 2 && ps.key_bits == 64 && pp.skipped > 0 && (rc = narrow_keys_pay(L, ps, n, &narrow, &digits)) != CSA_OK)
             return rc;
     }
     const u32 ell = pp.enabled ? (narrow ? pp.codes.key_syms / 2 : pp.codes.key_syms) : 4u; // symbols of a key of the first sort
@@ -1806,13 +1958,15 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             if ((rc = move_table(h->counts + 5, nullptr, sizeof(u32), s)) != CSA_OK || (rc = share_symbols(L, d_text, n, seen, nullptr)) != CSA_OK)
                 return rc;
         }
-        if (ahead && (rc = code_suffixes(L, d_text, n, tail)) != CSA_OK)
+        if (ahead && (rc = code_suffixes(L, d_text, n, tail, counted)) != CSA_OK)
             return rc;
         if (probed) {
             HIP_TRY(hipEventSynchronize(h->ev_gen[1]));
             coded = codes_pay(*seen, n);
+            if (coded && in_buckets && buckets_fit(*seen, n, bucket_digits(n, false)))
+                digits = bucket_digits(n, false);
         }
-        if (coded && !ahead && (rc = code_suffixes(L, d_text, n, tail)) != CSA_OK)
+        if (coded && !ahead && (rc = code_suffixes(L, d_text, n, tail, counted = digits)) != CSA_OK)
             return rc;
     }
     int passes = 0, p1 = 0, in_out = 0;
@@ -1832,15 +1986,13 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             add_table(cleared, h->counts + 5, nullptr, sizeof(u32)); // (the sampling of the symbols has been called off with it)
             if ((rc = move_tables(cleared, s)) != CSA_OK)
                 return rc;
-            rc = sort_by_codes(L, d_text, n, tail, 2u, list, &ps, ell);
-            p1 = CODE_PASSES;
+            rc = sort_by_codes(L, d_text, n, tail, 2u, list, ALL_DIGITS, digits, &p1, &ps, ell);
             in_out = 1;
         } else {
             rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, plan, &in_out, &p1, nullptr, 0, 0, &ps);
         }
     } else if (coded) {
-        rc = sort_by_codes(L, d_text, n, tail, h->pack_symbols ? 0u : 1u, list);
-        p1 = CODE_PASSES;
+        rc = sort_by_codes(L, d_text, n, tail, h->pack_symbols ? 0u : 1u, list, counted, digits, &p1);
         in_out = 1; // idx[1] holds the list, key[0] and key[1] what the sort has left behind
     } else {
         if (!h->pack_symbols)
@@ -2745,8 +2897,10 @@ WorkspaceSizes workspace_sizes(u64 cap)
     WorkspaceSizes w;
     const u64 sort_tiles = (cap + SORT_TILE - 1) / SORT_TILE;
     const u64 rank_tiles = (cap + TABLE_TILE - 1) / TABLE_TILE;
-    w.lookback_tile_words = sort_tiles * RADIX_BINS; // the group words of the radix pass follow the tile words
-    w.lookback_words = w.lookback_tile_words + (sort_tiles / LB_GROUP + 1) * RADIX_BINS;
+    // the group words of the radix pass follow the tile words (passes over nine bits have twice the words for a tile of twice the size: the last one
+    // and its group may have no second half)
+    w.lookback_tile_words = (sort_tiles + 1) * RADIX_BINS;
+    w.lookback_words = w.lookback_tile_words + (sort_tiles / LB_GROUP + 2) * RADIX_BINS;
     if (rank_tiles * 4 > w.lookback_words)
         w.lookback_words = rank_tiles * 4;
     w.rank_tiles_cap = rank_tiles + 1;
@@ -3077,7 +3231,7 @@ int csa_radix_sort_pairs_static_dev(uint64_t* d_keys, uint32_t* d_vals, uint64_t
     ha.plan = plan;
     ha.ghist = ghist;
     hipLaunchKernelGGL(radix_hist_kernel, dim3(hist_blocks(256 * 16, n)), dim3(256), 0, s, ha);
-    hipLaunchKernelGGL(radix_scan_hist_kernel, dim3(1), dim3(256), 0, s, ghist, digit_base, plan.num_passes);
+    hipLaunchKernelGGL(radix_scan_hist_kernel<RADIX_BINS>, dim3(1), dim3(RADIX_BINS), 0, s, ghist, digit_base, plan.num_passes);
     // every pass runs (skipping the passes whose digit is constant would need the counts on the host: a round trip)
     const TileOrder by_arrival = {TILES_BY_ARRIVAL, XCD_CHUNK};
     int where = 0; // 0: the pairs are in the caller's arrays, 1: in the scratch

@@ -195,9 +195,13 @@ struct ProbeCounts {
     u32 second, third, fourth; // ... by one, by two, by three others
     u32 other;  // of `again`: whose string is not that of the first one there
     u32 crowded; // of `other`: by `long_from` others or more
+    u32 packed;  // suffixes, of one in bucket_skip + 1, that find `full_from` others or more in the bucket of their code (bucket_sort.hpp)
+    u32 unused[3]; // (a multiple of 16 bytes is cleared by one launch)
     unsigned long long pairs; // pairs of suffixes with one code
 };
-static_assert(sizeof(ProbeCounts) == 8 * sizeof(u32), "the counters take eight words of the tables");
+constexpr u32 PROBE_FLAGS = 7; // counters before `unused`
+constexpr u32 PROBE_WORDS = sizeof(ProbeCounts) / sizeof(u32);
+static_assert(PROBE_WORDS % 4 == 0, "what follows the counters in the tables holds 64-bit words, and they are cleared with it");
 
 struct ProbeArgs {
     const u16* text;
@@ -211,6 +215,10 @@ struct ProbeArgs {
     const u32* stream;   // non-null: the codes are the narrow keys of a packed text, sym_bits bits a symbol; `crowded` counts whoever
     u32 sym_bits;        // finds its code taken by long_from others or more, its own string as they are
     const u32* skipped;  // non-null: nothing is looked at if it is set
+    u32* buckets;        // non-null, zeroed: suffixes that came, by the bits of their code from bucket_shift on
+    u32 bucket_shift;
+    u32 full_from;
+    u32 bucket_skip; // one suffix of so many, a power of two, and one less here
 };
 
 // An entry of the table is a code (high half), eight bits of the first string's hash and the number of suffixes that came.
@@ -218,11 +226,11 @@ struct ProbeArgs {
 __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
 {
     __shared__ unsigned long long s_pairs[PROBE_BLOCK / WAVE];
-    __shared__ u32 s_cnt[6];
+    __shared__ u32 s_cnt[PROBE_FLAGS];
     if (a.skipped && *a.skipped)
         return;
     const u32 t = threadIdx.x;
-    if (t < 6)
+    if (t < PROBE_FLAGS)
         s_cnt[t] = 0;
     __syncthreads();
     u32 pairs = 0, flags = 0;
@@ -245,6 +253,12 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
             }
             alone = string_code(lo, width, code);
         }
+        const bool placed = a.buckets && (i & a.bucket_skip) == 0;
+        // (a full one is not counted any further: additions to one address queue, 54 us instead of 10 for a text of runs)
+        u32* const bucket = placed ? a.buckets + (code >> a.bucket_shift) : nullptr;
+        u32 company = placed ? __hip_atomic_load(bucket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+        if (placed && company < a.full_from)
+            company = atomicAdd(bucket, 1u);
         if (!alone) {
             const unsigned long long entry = ((unsigned long long)code << 32) | (hash >> 24 << 24) | 1u;
             const u32 mask = (1u << a.table_log2) - 1u;
@@ -264,9 +278,11 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
                 break;
             }
         }
+        if (placed && company >= a.full_from)
+            flags |= 64u;
     }
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
+    for (u32 k = 0; k < PROBE_FLAGS; ++k) {
         const u64 b = __ballot((flags >> k) & 1u);
         if ((t & 63u) == 0 && b)
             atomicAdd(&s_cnt[k], (u32)__popcll(b));
@@ -275,7 +291,7 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
     if ((t & 63u) == 0)
         s_pairs[t / WAVE] = sum;
     __syncthreads();
-    if (t < 6 && s_cnt[t])
+    if (t < PROBE_FLAGS && s_cnt[t])
         atomicAdd(reinterpret_cast<u32*>(a.counts) + t, s_cnt[t]);
     if (t == 0) {
         unsigned long long all = 0;
@@ -294,21 +310,33 @@ constexpr int CODE_ITEMS = 8;
 constexpr int CODE_PASSES = 4;
 constexpr int CODE_COPIES = 8;
 
+// The radix passes over the codes: all four digits of eight bits, or those above the buckets (bucket_sort.hpp).
+struct CodeDigits {
+    u32 passes;
+    u32 bits; // of a digit, 8 or 9
+    u32 shift[CODE_PASSES];
+    u32 buckets_log2; // upper bits of a code that number its bucket; 0: the passes take all bits
+};
+constexpr u32 CODE_BINS = CODE_PASSES * RADIX_BINS; // digit counts of all passes: four of 256, or two of 512 at most
+
 // codes[v] = code of the suffix at virtual position v (virtual_to_suffix with `tail` = min(n, 4)); bit x & 7 of own[x >> 3]: the
 // suffix at text position x has a code that only its string can have (string_code). Bounded by the lookups
 // of cum[]: one 8-byte gather per symbol (the table is 256 KB: it lives in the L2s), shared by the four suffixes it appears in.
 // BLOCK: the 32 KB of digit counters decide how many waves a CU holds, 16 in workgroups of 256 and 32 in workgroups of 1024,
 // which code 1e9 tokens in 2.27 instead of 3.06 ms and 2^28 in 0.58 instead of 0.78 (512: 2.69, 0.66; 256 with half the
 // counters: 2.92, 0.75). Short texts take 256, so that there are workgroups for every CU.
-template <int BLOCK>
+// PASSES: of `digits`.
+template <int BLOCK, u32 PASSES>
 __global__ __launch_bounds__(BLOCK) void code_suffixes_kernel(const u16* __restrict__ text, u32 n, u32 tail, const u32* __restrict__ cum,
-                                                              u32* __restrict__ codes, u8* __restrict__ own, u32* __restrict__ ghist)
+                                                              u32* __restrict__ codes, u8* __restrict__ own, CodeDigits digits,
+                                                              u32* __restrict__ ghist)
 {
     constexpr u32 TILE = BLOCK * CODE_ITEMS;
     __shared__ u64 s_text[(TILE + 3 + 6) / 4 + 2];
-    __shared__ u32 s_hist[CODE_PASSES * RADIX_BINS * CODE_COPIES];
+    __shared__ u32 s_hist[CODE_BINS * CODE_COPIES];
     const u32 t = threadIdx.x;
-    for (u32 i = t; i < CODE_PASSES * RADIX_BINS * CODE_COPIES; i += BLOCK)
+    const u32 bits = PASSES == CODE_PASSES ? (u32)RADIX_BITS : digits.bits, bins = PASSES << bits;
+    for (u32 i = t; i < bins * CODE_COPIES; i += BLOCK)
         s_hist[i] = 0;
     const u32 copy = t & (CODE_COPIES - 1);
     const u64 tiles = ((u64)n + TILE - 1) / TILE;
@@ -354,12 +382,14 @@ __global__ __launch_bounds__(BLOCK) void code_suffixes_kernel(const u16* __restr
         for (int k = 0; k < CODE_ITEMS; ++k)
             if (x0 + k < n) {
 #pragma unroll
-                for (int p = 0; p < CODE_PASSES; ++p)
-                    atomicAdd(&s_hist[(p * RADIX_BINS + ((code[k] >> (8 * p)) & 0xFFu)) * CODE_COPIES + copy], 1u);
+                for (u32 p = 0; p < PASSES; ++p) {
+                    const u32 shift = PASSES == CODE_PASSES ? RADIX_BITS * p : digits.shift[p];
+                    atomicAdd(&s_hist[((p << bits) + __builtin_amdgcn_ubfe(code[k], shift, bits)) * CODE_COPIES + copy], 1u);
+                }
             }
     }
     __syncthreads();
-    for (u32 i = t; i < CODE_PASSES * RADIX_BINS; i += BLOCK) {
+    for (u32 i = t; i < bins; i += BLOCK) {
         u32 v = 0;
 #pragma unroll
         for (int c = 0; c < CODE_COPIES; ++c)

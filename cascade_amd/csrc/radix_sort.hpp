@@ -255,12 +255,13 @@ __global__ __launch_bounds__(256) void text_hist_expand_kernel(const u16* __rest
 }
 
 // digit_base[p][d] = number of pairs whose pass-p digit is < d.
-__global__ __launch_bounds__(256) void radix_scan_hist_kernel(const u32* ghist, u32* digit_base, int num_passes)
+template <int BINS>
+__global__ __launch_bounds__(BINS) void radix_scan_hist_kernel(const u32* ghist, u32* digit_base, int num_passes)
 {
-    __shared__ u32 s_wave[4];
+    __shared__ u32 s_wave[BINS / WAVE];
     const u32 t = threadIdx.x;
     for (int p = 0; p < num_passes; ++p) {
-        const u32 c = ghist[p * RADIX_BINS + t];
+        const u32 c = ghist[p * BINS + t];
         const u32 incl = wave_incl_sum(c);
         if ((t & 63u) == 63u)
             s_wave[t >> 6] = incl;
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(256) void radix_scan_hist_kernel(const u32* ghist, 
         u32 prefix = 0;
         for (u32 w = 0; w < (t >> 6); ++w)
             prefix += s_wave[w];
-        digit_base[p * RADIX_BINS + t] = prefix + incl - c;
+        digit_base[p * BINS + t] = prefix + incl - c;
         __syncthreads();
     }
 }
@@ -283,9 +284,9 @@ struct OnesweepArgs {
     u32 tail;   // suffixes that run off the text inside their key (SRC_CODED, SRC_PACKED, SRC_TEXT)
     int shift;
     int bits;
-    const u32* digit_base; // [256] for this pass
-    u64* lookback;         // [tiles][256]
-    u64* lookback_groups;  // [ceil(tiles / LB_GROUP)][256]
+    const u32* digit_base; // [bins] for this pass, 256 or 512
+    u64* lookback;         // [tiles][bins]
+    u64* lookback_groups;  // [ceil(tiles / LB_GROUP)][bins]
     u32* ticket;           // zero before the launch (TILES_BY_ARRIVAL)
     u32 order;             // TILES_BY_ARRIVAL or TILES_STATIC_CHUNKS
     u32 xcd_chunk;         // TILES_STATIC_CHUNKS: consecutive tiles given to one XCD
@@ -348,17 +349,59 @@ __device__ __forceinline__ u32 onesweep_tile_number(const OnesweepArgs& a)
 #define CSA_SORT_MIN_WAVES 1
 #endif
 
+#ifdef __HIP_DEVICE_COMPILE__
+#define CSA_LDS_ORDER() asm volatile("" ::: "memory")
+#define CSA_OPAQUE(x) asm volatile("" : "+v"(x))
+#else
+#define CSA_LDS_ORDER() __builtin_amdgcn_wave_barrier() /* CPU emulation: lanes are threads, order them for real */
+#define CSA_OPAQUE(x) ((void)0)
+#endif
+
+// The place of a lane's item among the items of its wave so far that have digit d (DB bits), those of this call in lane order; whist[d] counts
+// them. Call with all 64 lanes.
+// For every digit bit, (ballot of "bit set") XOR (all-ones if my own bit is set) has a 0 exactly at the lanes
+// that agree with me on that bit; `same` keeps the lanes that agree on every bit, i.e. whose digit is mine.
+// The per-wave counters are plain LDS words: a wave executes its LDS instructions in order, so the counter
+// update of one item is seen by the next item's read; the empty asm statements only keep the compiler from
+// moving those accesses across each other.
+template <int DB>
+__device__ __forceinline__ u32 rank_in_wave(u32 d, u32* whist)
+{
+    u32 same_lo = ~0u, same_hi = ~0u;
+#pragma unroll
+    for (int b = 0; b < DB; ++b) {
+        u32 mine = (u32)__builtin_amdgcn_sbfe(d, b, 1); // 0 or 0xFFFFFFFF
+        CSA_OPAQUE(mine); // the ballot tests this register (one compare), not a second extraction of the bit
+        const u64 bal = __ballot((int)mine < 0);
+        // same &= ~(bal ^ mine): one three-input bit operation per half (table of a & ~(b ^ c): 0x90)
+        same_lo = __builtin_amdgcn_bitop3_b32(same_lo, (u32)bal, mine, 0x90);
+        same_hi = __builtin_amdgcn_bitop3_b32(same_hi, (u32)(bal >> 32), mine, 0x90);
+    }
+    const u32 before = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
+    const u32 prev = whist[d];
+    CSA_LDS_ORDER();
+    if (before == 0)
+        whist[d] = prev + __popc(same_lo) + __popc(same_hi);
+    CSA_LDS_ORDER();
+    return prev + before;
+}
+
+#undef CSA_LDS_ORDER
+#undef CSA_OPAQUE
+
 // KeyT is u64 (the suffix-sort keys) or u32 (the (text position, rank) pairs of the bucketed rank update).
 // HI selects the 32-bit half of a 64-bit key that holds this pass's digit (digits never straddle the halves),
 // so that the digit is one bit-field extract of a 32-bit register.
 // VALS = false: the keys travel alone (records whose payload sits in the key bits that are not sorted on).
-template <typename KeyT, int BLOCK, int ITEMS, int SRC, int HI, bool VALS = true>
+// DB: bits of the widest digit.
+template <typename KeyT, int BLOCK, int ITEMS, int SRC, int HI, bool VALS = true, int DB = RADIX_BITS>
 __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(OnesweepArgs a)
 {
     static_assert(VALS || SRC == SRC_PAIRS, "the passes that build their keys make the suffix indices");
     constexpr int TILE = BLOCK * ITEMS;
     constexpr int WAVES = BLOCK / WAVE;
-    static_assert(BLOCK >= RADIX_BINS, "one thread per digit is assumed");
+    constexpr int BINS = 1 << DB;
+    static_assert(BLOCK >= BINS, "one thread per digit is assumed");
     static_assert(sizeof(KeyT) == 8 || ((SRC == SRC_PAIRS || SRC == SRC_CODED || SRC == SRC_PACKED) && HI == 0), "narrow keys are read from an array, or cut from the code stream");
     constexpr bool KEYS_IN = SRC == SRC_PAIRS || SRC == SRC_CODED;
     auto rank_key = [&](u32 i) -> u64 { return rank_pair_key(a.rank, a.n, a.hop, i, a.radix); }; // SRC_RANKS: pair i is text position i
@@ -366,9 +409,9 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
     KeyT* __restrict__ keys_out = static_cast<KeyT*>(a.keys_out);
 
     __shared__ KeyT s_keys[TILE];
-    __shared__ u32 s_whist[WAVES * RADIX_BINS];
-    __shared__ u32 s_binstart[RADIX_BINS];
-    __shared__ u32 s_delta[RADIX_BINS];
+    __shared__ u32 s_whist[WAVES * BINS];
+    __shared__ u32 s_binstart[BINS];
+    __shared__ u32 s_delta[BINS];
     __shared__ u32 s_wsum[WAVES];
     __shared__ u32 s_tile;
 
@@ -378,7 +421,7 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
 
     if (t == 0)
         s_tile = onesweep_tile_number(a);
-    for (int i = t; i < WAVES * RADIX_BINS; i += BLOCK)
+    for (int i = t; i < WAVES * BINS; i += BLOCK)
         s_whist[i] = 0;
     __syncthreads();
     const u32 tile = s_tile;
@@ -390,13 +433,6 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
     const u32 bits = (u32)a.bits;
     const u32 mask = (1u << bits) - 1u;
 #define CSA_DIGIT(kk) __builtin_amdgcn_ubfe(HI ? (u32)((u64)(kk) >> 32) : (u32)(kk), sh, bits)
-#ifdef __HIP_DEVICE_COMPILE__
-#define CSA_LDS_ORDER() asm volatile("" ::: "memory")
-#define CSA_OPAQUE(x) asm volatile("" : "+v"(x))
-#else
-#define CSA_LDS_ORDER() __builtin_amdgcn_wave_barrier() /* CPU emulation: lanes are threads, order them for real */
-#define CSA_OPAQUE(x) ((void)0)
-#endif
     // ---- first pass of generation 0 on K-gram keys: stage the tile's stretch of the text in LDS ----
     // The tile covers consecutive virtual positions, i.e. (after the few tail suffixes of tile 0) consecutive text
     // positions j0, j0 + 1, ...; the (still unused) reorder buffer holds the stretch, and each key is assembled
@@ -468,58 +504,35 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
     }
 
     // ---- rank each pair among the pairs of its wave that share its digit ----
-    // For every digit bit, (ballot of "bit set") XOR (all-ones if my own bit is set) has a 0 exactly at the lanes
-    // that agree with me on that bit; `same` keeps the lanes that agree on every bit, i.e. whose digit is mine.
-    // The per-wave counters are plain LDS words: a wave executes its LDS instructions in order, so the counter
-    // update of one item is seen by the next item's read; the empty asm statements only keep the compiler from
-    // moving those accesses across each other.
-    u32* whist = s_whist + w * RADIX_BINS;
+    u32* whist = s_whist + w * BINS;
     u32 pos[ITEMS];
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-        const u32 d = CSA_DIGIT(key[k]);
-        u32 same_lo = ~0u, same_hi = ~0u;
-#pragma unroll
-        for (int b = 0; b < RADIX_BITS; ++b) {
-            u32 mine = (u32)__builtin_amdgcn_sbfe(d, b, 1); // 0 or 0xFFFFFFFF
-            CSA_OPAQUE(mine); // the ballot tests this register (one compare), not a second extraction of the bit
-            const u64 bal = __ballot((int)mine < 0);
-            // same &= ~(bal ^ mine): one three-input bit operation per half (table of a & ~(b ^ c): 0x90)
-            same_lo = __builtin_amdgcn_bitop3_b32(same_lo, (u32)bal, mine, 0x90);
-            same_hi = __builtin_amdgcn_bitop3_b32(same_hi, (u32)(bal >> 32), mine, 0x90);
-        }
-        const u32 before = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
-        const u32 prev = whist[d];
-        CSA_LDS_ORDER();
-        if (before == 0)
-            whist[d] = prev + __popc(same_lo) + __popc(same_hi);
-        CSA_LDS_ORDER();
-        pos[k] = prev + before;
-    }
+    for (int k = 0; k < ITEMS; ++k)
+        pos[k] = rank_in_wave<DB>(CSA_DIGIT(key[k]), whist);
     __syncthreads();
 
     // ---- one thread per digit: offsets of the waves inside the tile, tile totals; publish them at once ----
     u32 total = 0, real = 0;
-    if (t < RADIX_BINS) {
+    if (t < BINS) {
 #pragma unroll
         for (int ww = 0; ww < WAVES; ++ww) {
-            const u32 c = s_whist[ww * RADIX_BINS + t];
-            s_whist[ww * RADIX_BINS + t] = total;
+            const u32 c = s_whist[ww * BINS + t];
+            s_whist[ww * BINS + t] = total;
             total += c;
         }
         real = total;
         if (t == mask)
             real -= (u32)TILE - valid; // padding pairs all carry the largest digit
-        lb2_publish(a.lookback + t, RADIX_BINS, tile, a.epoch, real);
+        lb2_publish(a.lookback + t, BINS, tile, a.epoch, real);
     }
-    // exclusive scan of the 256 totals (padding included: it occupies LDS slots too)
+    // exclusive scan of the totals (padding included: it occupies LDS slots too)
     u32 binstart = 0;
     {
         const u32 incl = wave_incl_sum(total);
-        if (t < RADIX_BINS && lane == 63u)
+        if (t < BINS && lane == 63u)
             s_wsum[w] = incl;
         __syncthreads();
-        if (t < RADIX_BINS) {
+        if (t < BINS) {
             u32 prefix = 0;
             for (u32 ww = 0; ww < w; ++ww)
                 prefix += s_wsum[ww];
@@ -533,11 +546,11 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         const u32 d = CSA_DIGIT(key[k]);
-        pos[k] += s_binstart[d] + s_whist[w * RADIX_BINS + d];
+        pos[k] += s_binstart[d] + s_whist[w * BINS + d];
         s_keys[pos[k]] = key[k];
     }
-    if (t < RADIX_BINS) {
-        const u32 excl = lb2_wait_exclusive(a.lookback + t, a.lookback_groups + t, RADIX_BINS, tile, a.epoch, real, a.err);
+    if (t < BINS) {
+        const u32 excl = lb2_wait_exclusive(a.lookback + t, a.lookback_groups + t, BINS, tile, a.epoch, real, a.err);
         s_delta[t] = a.digit_base[t] + excl - binstart; // wraps; added back to an LDS slot below
     }
     __syncthreads();
@@ -586,8 +599,6 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
             a.vals_out[dst[k]] = s_vals[q];
     }
 #undef CSA_DIGIT
-#undef CSA_LDS_ORDER
-#undef CSA_OPAQUE
 }
 
 // Sorted pairs that ended in the ping-pong partner go back to the caller's arrays (a kernel rather than a copy call,

@@ -966,3 +966,21 @@ def test_wide_loads_are_aligned_for_every_capacity():
             % (os.path.dirname(os.path.abspath(__file__)), os.path.dirname(os.path.dirname(os.path.abspath(__file__)))))
     run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
     assert run.returncode == 0, (run.returncode, run.stderr[-2000:])
+
+
+@pytest.mark.parametrize("n", [17000, 33000, 41000])
+@pytest.mark.parametrize("kind", ["even", "heavy", "crowded", "copies", "letters"])
+def test_lower_digits_are_sorted_in_buckets(n, kind):
+    """A build with buckets of up to 256 suffixes, 512 cells of up to 20 members that are compared, and two passes of eight bits below 2^15 symbols, of
+    nine above: even codes, strings that fill a bucket and more (they are collected and radix sorted) or a cell (passes in LDS), copies, packed symbols of
+    two bits. Suffix array and generation sizes are the oracle's."""
+    lib = load_emulation("libcascade_emu_buckets.so")
+    rng = np.random.default_rng(n)
+    T = texts.text_of_copies(n, 4 if kind == "letters" else 60000, n) if kind in ("copies", "letters") else rng.integers(1, 60000, n).astype(np.uint16)
+    if kind in ("heavy", "crowded"):
+        for string, times in enumerate([400, 257, 90] if kind == "heavy" else [120, 64, 21, 22]):
+            for at in rng.permutation(n // 8 - 1)[:times]:
+                T[8 * at:8 * at + 4] = [7, 8, 9, 100 * string]
+    got, active, _ = emu_sort(lib, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts

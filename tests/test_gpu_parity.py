@@ -865,3 +865,29 @@ def test_lists_with_many_suffixes_in_long_runs(torch_mod, n, phrases, lo, hi):
         stats = s.last_stats
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
+
+
+@pytest.mark.parametrize("n,letters", [((1 << 24) + 1, 50000), ((1 << 24) + 4099, 50000), (30000001, 4)])
+def test_lower_digits_are_sorted_in_buckets(torch_mod, n, letters):
+    """Texts of more than 2^24 symbols: two passes over the upper digits, then buckets in LDS, with strings that come 300 times (a crowded cell) and 20000
+    times (a bucket that does not fit) among independent ones, and four-letter texts with copies. The device verifier judges, and the generation
+    sizes are those of the sort with K-gram keys."""
+    from cascade_amd import PartitionSorter, _native
+    rng = np.random.default_rng(n)
+    T = rng.integers(1, letters + 1, n).astype(np.uint16)
+    if letters > 4:
+        for string, times in enumerate([300, 20000, 7300, 256, 258]):
+            at = 8 * rng.permutation(n // 8 - 1)[:times]
+            for k in range(4):
+                T[at + k] = [7, 8, 9, 100 * string + 1][k]
+    T[n // 2:n // 2 + 70000] = T[1000:71000]
+    d = to_dev(torch_mod, T)
+    seen = []
+    with PartitionSorter(n, key_words=1) as s:
+        for pack in (1, 0):
+            print(f"  buckets {n} {letters} {pack}", flush=True)
+            s.set_tuning(_native.CSA_TUNE_PACK_SYMBOLS, pack)
+            out = s.sort(d)
+            assert s.verify(d, out)
+            seen.append(s.last_stats["active"])
+    assert seen[0] == seen[1]
