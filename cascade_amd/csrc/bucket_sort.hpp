@@ -22,7 +22,7 @@ namespace csa {
 #define CSA_CELLS_LOG2 13
 #endif
 #ifndef CSA_CELL_MAX
-#define CSA_CELL_MAX 256
+#define CSA_CELL_MAX 512
 #endif
 constexpr int BUCKET_BLOCK = CSA_BUCKET_BLOCK;
 constexpr int BUCKET_ITEMS = CSA_BUCKET_ITEMS;
@@ -45,11 +45,20 @@ struct BucketArgs {
     u32* over_list;      // [n / BUCKET_MAX]: them, in any order
     u32* crowded;        // zeroed: buckets with a cell of more than CELL_MAX ...
     u32* crowded_list;   // ... [buckets]: them, in any order
+    // EXT: sixteen bits more of every suffix (code_suffixes_kernel); the list in order goes elsewhere, with its ties
+    const u16* ext;
+    u32 ext_bits; // that are sorted with the lower bits of the code: 32 in all at most
+    u32* sufs_out;
+    u8* ties;
+    u32* open_count; // zeroed: suffixes in runs of one code and one ext, which are left open (resolve_runs_kernel) ...
+    u32* open_sufs;  // ... them, run after run, with OWN_CODE ...
+    u32* open_places; // ... and their places in the list, with RUN_START
     // the suffixes of buckets that do not fit, collected in list order
     u32* over_before; // [buckets]: of the buckets before this one whose number is the same in its upper bits (OVER_TILE buckets) ...
     u32* over_tiles;  // ... and of all that differ in those, by them
     u64* over_keys;
     u32* over_sufs;
+    u32* over_open; // EXT: where they start in the list of open runs
 };
 
 constexpr int STARTS_BLOCK = 256;
@@ -87,10 +96,84 @@ __global__ __launch_bounds__(STARTS_BLOCK) void bucket_starts_kernel(BucketArgs 
     }
 }
 
+// EXT: what the members of a bucket are sorted by, the lower bits of the code and the upper ones of ext.
+__device__ __forceinline__ u32 bucket_key(const BucketArgs& a, u32 code, u32 ext)
+{
+    return (code & ((1u << a.low_bits) - 1u)) << a.ext_bits | ext >> (16u - a.ext_bits);
+}
+
+// How an entry ties with its left neighbour, whose key is another one: suffixes that own one code have one string. The last `tail` suffixes, which run off
+// the text inside it, come first in virtual order and tie with nobody.
+__device__ __forceinline__ u32 tie_of_strings(bool same_code, u32 mine, u32 left, u32 tail)
+{
+    return same_code && (mine & OWN_CODE) && (mine & ~OWN_CODE) >= tail && (left & ~OWN_CODE) >= tail ? 1u : 0u;
+}
+
+// EXT: writes a bucket whose pairs (key, virtual position and OWN_CODE) pair_of(j) gives in order, and adds the runs of one key to the open ones.
+constexpr u32 BUCKET_WAVES = BUCKET_ITEMS * BUCKET_BLOCK / WAVE;
+static_assert(BUCKET_WAVES <= 2 * WAVE, "one wave scans them, two a lane");
+
+template <typename Pairs>
+__device__ __forceinline__ void write_bucket(const BucketArgs& a, u32 start, u32 size, u32* s_open, Pairs pair_of)
+{
+    constexpr int BLOCK = BUCKET_BLOCK, ITEMS = BUCKET_ITEMS;
+    const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    const u32 rounds = (size + BLOCK - 1) / BLOCK;
+    u32 suf[ITEMS], member = 0, begins = 0; // bit k: the entry of round k is one of a run; begins one
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+        if ((u32)k < rounds) {
+            const u32 j = k * BLOCK + t, from = j < size ? j : size - 1u;
+            const u64 pair = pair_of(from), left = pair_of(from > 0 ? from - 1u : 0u), right = pair_of(from + 1u < size ? from + 1u : from);
+            const u32 key = (u32)(pair >> 32), before = (u32)(left >> 32);
+            const bool follows = from > 0 && key == before, precedes = from + 1u < size && key == (u32)(right >> 32);
+            const bool same_code = from > 0 && (key ^ before) >> a.ext_bits == 0;
+            const bool in = j < size && (follows || precedes);
+            const u32 x = virtual_to_suffix((u32)pair & ~OWN_CODE, a.n, a.tail);
+            suf[k] = x | ((u32)pair & OWN_CODE);
+            member |= (in ? 1u : 0u) << k;
+            begins |= (follows ? 0u : 1u) << k;
+            if (j < size) {
+                a.sufs_out[start + j] = x;
+                a.ties[start + j] = (u8)tie_of_strings(same_code, (u32)pair, (u32)left, a.tail);
+            }
+            const u64 b = __ballot(in);
+            if (lane == 0)
+                s_open[k * (BLOCK / WAVE) + w] = (u32)__popcll(b);
+        }
+    __syncthreads();
+    if (w == 0) {
+        const u32 used = rounds * (BLOCK / WAVE);
+        const u32 c0 = 2 * lane < used ? s_open[2 * lane] : 0u, c1 = 2 * lane + 1 < used ? s_open[2 * lane + 1] : 0u;
+        const u32 incl = wave_incl_sum(c0 + c1), total = __shfl(incl, 63);
+        u32 base = 0;
+        if (lane == 0 && total)
+            base = atomicAdd(a.open_count, total);
+        base = __shfl(base, 0) + incl - c0 - c1;
+        if (2 * lane < used)
+            s_open[2 * lane] = base;
+        if (2 * lane + 1 < used)
+            s_open[2 * lane + 1] = base + c0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+        if ((u32)k < rounds) {
+            const bool in = (member >> k) & 1u;
+            const u64 b = __ballot(in);
+            if (in) {
+                const u32 slot = s_open[k * (BLOCK / WAVE) + w] + (u32)__popcll(b & ((1ull << lane) - 1ull));
+                a.open_sufs[slot] = suf[k];
+                a.open_places[slot] = (start + k * BLOCK + t) | ((begins >> k) & 1u ? RUN_START : 0u);
+            }
+        }
+}
+
 // One bucket a workgroup. Its suffixes go to 8192 cells by the next bits of their codes, in whatever order they arrive, and everyone is compared with the
 // others in its cell, of which there are one or two, by the whole code and its place in the order of the text. What bounds it are vector
 // instructions: all threads do the same for whole rounds, what is past the end of the bucket going to a cell of its own. Buckets with a long
 // cell, one string hundreds of times, are left to finish_crowded_kernel.
+template <bool EXT>
 __global__ __launch_bounds__(BUCKET_BLOCK, 8) void finish_buckets_kernel(BucketArgs a)
 {
     constexpr int BLOCK = BUCKET_BLOCK, ITEMS = BUCKET_ITEMS, CAP = BUCKET_MAX, CELLS = 1 << CELLS_LOG2;
@@ -100,12 +183,14 @@ __global__ __launch_bounds__(BUCKET_BLOCK, 8) void finish_buckets_kernel(BucketA
     __shared__ __align__(16) u32 s_cell[CELLS / 2 + 4]; // two to a word: members of a cell, then where they start
     __shared__ u32 s_sum[BLOCK / WAVE];
     __shared__ u32 s_crowded;
+    __shared__ u32 s_open[EXT ? BUCKET_WAVES : 1];
     const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6;
     const u32 start = a.starts[blockIdx.x], size = a.starts[blockIdx.x + 1] - start;
-    if (size < 2 || size > (u32)CAP)
+    if (size < (EXT ? 1u : 2u) || size > (u32)CAP)
         return;
     const u32 rounds = (size + BLOCK - 1) / BLOCK;
-    const u32 drop = a.low_bits > (u32)CELLS_LOG2 ? a.low_bits - CELLS_LOG2 : 0u;
+    const u32 key_bits = a.low_bits + (EXT ? a.ext_bits : 0u);
+    const u32 drop = key_bits > (u32)CELLS_LOG2 ? key_bits - CELLS_LOG2 : 0u;
     const u32* const codes = a.codes + start;
     const u32* const sufs = a.sufs + start;
     u32 key[ITEMS], val[ITEMS], cell[ITEMS];
@@ -115,6 +200,8 @@ __global__ __launch_bounds__(BUCKET_BLOCK, 8) void finish_buckets_kernel(BucketA
             const u32 i = k * BLOCK + t, from = i < size ? i : size - 1u;
             key[k] = codes[from];
             val[k] = sufs[from];
+            if constexpr (EXT)
+                key[k] = bucket_key(a, key[k], a.ext[start + from]);
         }
     for (int i = t; i < CELLS / 2 + 1; i += BLOCK)
         s_cell[i] = 0;
@@ -166,31 +253,48 @@ __global__ __launch_bounds__(BUCKET_BLOCK, 8) void finish_buckets_kernel(BucketA
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k)
         if ((u32)k < rounds) {
-            const u32 x = val[k] & ~OWN_CODE, virt = x + a.tail >= a.n ? a.n - 1u - x : x + a.tail;
+            const u32 virt = suffix_to_virtual(val[k] & ~OWN_CODE, a.n, a.tail);
             const u32 to = starts[cell[k]] + ((at[k] >> (cell[k] & 1u) * 16u) & 0xFFFFu);
             s_pair[cell[k] == (u32)CELLS ? CAP + lane : to] = (u64)key[k] << 32 | virt | (val[k] & OWN_CODE);
         }
     __syncthreads();
+    u64 pair[EXT ? ITEMS : 1];
+    u32 to_place[EXT ? ITEMS : 1];
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         const u32 j = k * BLOCK + t;
         if (j < size) {
-            const u64 pair = s_pair[j];
-            const u32 code = (u32)(pair >> 32), c = (code >> drop) & (u32)(CELLS - 1), virt = (u32)pair & ~OWN_CODE;
+            const u64 mine_pair = s_pair[j];
+            const u32 code = (u32)(mine_pair >> 32), c = (code >> drop) & (u32)(CELLS - 1);
             const u32 from = starts[c], to = starts[c + 1];
             u32 place = from;
             if (to - from > 1u)
                 for (u32 i = from; i < to; ++i)
-                    place += s_pair[i] < pair ? 1u : 0u;
-            a.codes[start + place] = code;
-            a.sufs[start + place] = virtual_to_suffix(virt, a.n, a.tail) | ((u32)pair & OWN_CODE);
+                    place += s_pair[i] < mine_pair ? 1u : 0u;
+            if constexpr (EXT) {
+                pair[k] = mine_pair;
+                to_place[k] = place;
+            } else {
+                a.codes[start + place] = code;
+                a.sufs[start + place] = virtual_to_suffix((u32)mine_pair & ~OWN_CODE, a.n, a.tail) | ((u32)mine_pair & OWN_CODE);
+            }
         }
+    }
+    if constexpr (EXT) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k)
+            if (k * BLOCK + t < size)
+                s_pair[to_place[k]] = pair[k];
+        __syncthreads();
+        write_bucket(a, start, size, s_open, [&](u32 j) { return s_pair[j]; });
     }
 }
 
 // The crowded buckets, one at a time a workgroup: stable LSD passes over digits of eight bits, ranked as in onesweep_kernel, whose tile the bucket is.
 constexpr u32 CROWDED_BLOCKS = 1024;
 
+template <bool EXT>
 __global__ __launch_bounds__(BUCKET_BLOCK) void finish_crowded_kernel(BucketArgs a)
 {
     constexpr int DB = RADIX_BITS, BLOCK = BUCKET_BLOCK, ITEMS = BUCKET_ITEMS, CAP = BUCKET_MAX, WAVES = BLOCK / WAVE, BINS = 1 << DB;
@@ -199,6 +303,7 @@ __global__ __launch_bounds__(BUCKET_BLOCK) void finish_crowded_kernel(BucketArgs
     static_assert(BINS <= BLOCK * PER, "the bins are scanned at once");
     __shared__ __align__(16) u32 s_mem[WORDS]; // the counters of a pass, [wave][bin]; then the pairs in the order of it
     __shared__ u32 s_carry[WAVES];
+    __shared__ u32 s_open[EXT ? BUCKET_WAVES : 1];
     const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6;
     const u32 crowded = *a.crowded;
     for (u32 at = blockIdx.x; at < crowded; at += gridDim.x) {
@@ -215,10 +320,13 @@ __global__ __launch_bounds__(BUCKET_BLOCK) void finish_crowded_kernel(BucketArgs
                 if (i < size) {
                     key[k] = a.codes[start + i];
                     val[k] = a.sufs[start + i];
+                    if constexpr (EXT)
+                        key[k] = bucket_key(a, key[k], a.ext[start + i]);
                 }
             }
-        for (u32 shift = 0; shift < a.low_bits; shift += DB) {
-            const u32 bits = a.low_bits - shift < (u32)DB ? a.low_bits - shift : (u32)DB;
+        const u32 key_bits = a.low_bits + (EXT ? a.ext_bits : 0u);
+        for (u32 shift = 0; shift < key_bits; shift += DB) {
+            const u32 bits = key_bits - shift < (u32)DB ? key_bits - shift : (u32)DB;
             for (int i = t; i < WAVES * BINS / 4; i += BLOCK)
                 reinterpret_cast<uint4*>(s_mem)[i] = make_uint4(0u, 0u, 0u, 0u);
             __syncthreads();
@@ -274,7 +382,15 @@ __global__ __launch_bounds__(BUCKET_BLOCK) void finish_crowded_kernel(BucketArgs
                     s_mem[CAP + pos[k]] = val[k];
                 }
             __syncthreads();
-            const bool last = shift + DB >= a.low_bits;
+            const bool last = shift + DB >= key_bits;
+            if (EXT && last) {
+                write_bucket(a, start, size, s_open, [&](u32 j) {
+                    const u32 v = s_mem[CAP + j];
+                    return (u64)s_mem[j] << 32 | suffix_to_virtual(v & ~OWN_CODE, a.n, a.tail) | (v & OWN_CODE);
+                });
+                __syncthreads();
+                break;
+            }
 #pragma unroll
             for (int k = 0; k < ITEMS; ++k)
                 if ((u32)k < rounds) {
@@ -315,10 +431,13 @@ __global__ __launch_bounds__(OVER_TILE) void over_before_kernel(BucketArgs a)
         a.over_before[b] = before;
     if (t == 0)
         a.over_tiles[blockIdx.x] = all;
+    if (a.over_open && blockIdx.x == 0 && t == 0)
+        *a.over_open = atomicAdd(a.open_count, a.over[0]);
 }
 
 // The suffixes of the buckets in over_list to their places in over_keys and over_sufs, or back from there (BACK), OVER_SLICES workgroups a bucket.
-template <bool BACK>
+// EXT: by the code and ext; on the way back the ties follow from those.
+template <bool BACK, bool EXT>
 __global__ __launch_bounds__(256) void over_move_kernel(BucketArgs a)
 {
     __shared__ u32 s_sum[256 / WAVE];
@@ -336,11 +455,24 @@ __global__ __launch_bounds__(256) void over_move_kernel(BucketArgs a)
     const u32 start = a.starts[b], size = a.starts[b + 1] - start;
     for (u32 i = blockIdx.x % OVER_SLICES * 256 + t; i < size; i += OVER_SLICES * 256) {
         if constexpr (!BACK) {
-            a.over_keys[to + i] = a.codes[start + i];
+            a.over_keys[to + i] = EXT ? (u64)a.codes[start + i] << 16 | a.ext[start + i] : (u64)a.codes[start + i];
             a.over_sufs[to + i] = a.sufs[start + i];
-        } else {
+        } else if constexpr (!EXT) {
             a.codes[start + i] = (u32)a.over_keys[to + i];
             a.sufs[start + i] = a.over_sufs[to + i];
+        } else {
+            const u64 key = a.over_keys[to + i];
+            const u32 v = a.over_sufs[to + i], x = v & ~OWN_CODE;
+            const bool follows = i > 0 && a.over_keys[to + i - 1] == key;
+            u32 tie = 0;
+            if (i > 0 && a.over_keys[to + i - 1] >> 16 == key >> 16) {
+                const u32 left = a.over_sufs[to + i - 1] & ~OWN_CODE;
+                tie = tie_of_strings(true, suffix_to_virtual(x, a.n, a.tail) | (v & OWN_CODE), suffix_to_virtual(left, a.n, a.tail), a.tail);
+            }
+            a.ties[start + i] = (u8)tie;
+            const u32 slot = *a.over_open + to + i; // (all of them are listed, runs or not)
+            a.open_sufs[slot] = v;
+            a.open_places[slot] = (start + i) | (follows ? 0u : RUN_START);
         }
     }
 }

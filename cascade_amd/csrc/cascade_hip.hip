@@ -453,13 +453,17 @@ void launch_onesweep(const csa_handle* h, OnesweepArgs& a, hipStream_t s)
 }
 
 // a.bits > RADIX_BITS: wide workgroups only (the look-back words are sized for RADIX_BINS a tile of half the size)
-template <int SRC>
+// EXT: wide workgroups
+template <int SRC, bool EXT = false>
 void launch_onesweep32(const csa_handle* hh, OnesweepArgs& a, hipStream_t s)
 {
     const TileOrder h = tile_order_of(hh);
     if (a.bits > RADIX_BITS) {
         set_tile_order(h, a, SORT_WIDE_BLOCK * SORT32_ITEMS);
-        hipLaunchKernelGGL((onesweep_kernel<u32, SORT_WIDE_BLOCK, SORT32_ITEMS, SRC, 0, true, RADIX_BITS + 1>), dim3(a.tiles), dim3(SORT_WIDE_BLOCK), 0, s, a);
+        hipLaunchKernelGGL((onesweep_kernel<u32, SORT_WIDE_BLOCK, SORT32_ITEMS, SRC, 0, true, RADIX_BITS + 1, EXT>), dim3(a.tiles), dim3(SORT_WIDE_BLOCK), 0, s, a);
+    } else if (EXT) {
+        set_tile_order(h, a, SORT_WIDE_BLOCK * SORT32_ITEMS);
+        hipLaunchKernelGGL((onesweep_kernel<u32, SORT_WIDE_BLOCK, SORT32_ITEMS, SRC, 0, true, RADIX_BITS, EXT>), dim3(a.tiles), dim3(SORT_WIDE_BLOCK), 0, s, a);
     } else if (wide_workgroups(a)) {
         set_tile_order(h, a, SORT_WIDE_BLOCK * SORT32_ITEMS);
         hipLaunchKernelGGL((onesweep_kernel<u32, SORT_WIDE_BLOCK, SORT32_ITEMS, SRC, 0>), dim3(a.tiles), dim3(SORT_WIDE_BLOCK), 0, s, a);
@@ -1044,7 +1048,7 @@ CodeDigits bucket_digits(u32 n, bool packed)
         log2 = CSA_TWO_PASS_LOG2;
     if (log2 <= CSA_TWO_PASS_LOG2)
         return CodeDigits{2, RADIX_BITS, {16, 24}, log2};
-    if (log2 <= 18 && !packed && n >= SORT_WIDE_MIN && n >= CODE_AHEAD_MAX) // (codes that are made ahead have their digits counted by eight bits)
+    if (log2 <= 18 && !packed)
         return CodeDigits{2, RADIX_BITS + 1, {14, 23}, log2};
     return ALL_DIGITS;
 }
@@ -1219,23 +1223,27 @@ u32* codes_of(const csa_handle* h) { return reinterpret_cast<u32*>(h->key[1]); }
 u8* own_of(const csa_handle* h) { return reinterpret_cast<u8*>(h->key[1]) + (4 * h->cap + 15) / 16 * 16; }
 u8* ties_of(const csa_handle* h) { return own_of(h) + ((h->cap + 7) / 8 + 15) / 16 * 16; }
 
+u16* ext_of(const csa_handle* h) { return reinterpret_cast<u16*>(ties_of(h) + (h->cap + 15) / 16 * 16); } // (of texts that are sorted in buckets: 7.125 bytes a suffix)
+
 int code_suffixes(Launch& L, const u16* d_text, u32 n, u32 tail, const CodeDigits& digits)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
     const u32* const cum = code_tables(h).cum;
     auto launch = [&](auto kernel, int block) {
-        hipLaunchKernelGGL(kernel, dim3(hist_blocks(block * CODE_ITEMS, n)), dim3(block), 0, s, d_text, n, tail, cum, codes_of(h), own_of(h), digits, h->ghist);
+        hipLaunchKernelGGL(kernel, dim3(hist_blocks(block * CODE_ITEMS, n)), dim3(block), 0, s, d_text, n, tail, cum, codes_of(h), own_of(h), digits, h->ghist, ext_of(h));
     };
     if (digits.passes == 2)
-        launch(code_suffixes_kernel<CODE_WIDE_BLOCK, 2>, CODE_WIDE_BLOCK);
+        launch(code_suffixes_kernel<CODE_WIDE_BLOCK, 2, true>, CODE_WIDE_BLOCK);
     else if (n >= SORT_WIDE_MIN) // 2048 tiles of the wide workgroups: four for each of those a device holds at a time
-        launch(code_suffixes_kernel<CODE_WIDE_BLOCK, CODE_PASSES>, CODE_WIDE_BLOCK);
+        launch(code_suffixes_kernel<CODE_WIDE_BLOCK, CODE_PASSES, false>, CODE_WIDE_BLOCK);
     else
-        launch(code_suffixes_kernel<CODE_BLOCK, CODE_PASSES>, CODE_BLOCK);
+        launch(code_suffixes_kernel<CODE_BLOCK, CODE_PASSES, false>, CODE_BLOCK);
     HIP_TRY(hipGetLastError());
     return CSA_OK;
 }
+
+constexpr u32 OPEN_BLOCKS = 2048; // workgroups that resolve open runs: twice as many as a device of 256 compute units holds at a time
 
 // A list sorted by codes on its way to being ranked.
 struct CodedList {
@@ -1247,9 +1255,14 @@ struct CodedList {
     bool long_left;   // there are runs that are too long for a tile on both words
 };
 
-// The bits of the codes below the passes of `digits`, in place (bucket_sort.hpp). *finished = false: too many suffixes are in buckets that do
+// The list of open runs: where the passes of a sort by codes in buckets had their pairs, and in an array that is not used before its long runs are.
+u32* open_sufs_of(const csa_handle* h) { return reinterpret_cast<u32*>(h->key[0]) + h->cap; }
+u32* open_places_of(const csa_handle* h) { return h->idx[2]; }
+
+// The bits of the codes below the passes of `digits`, in place, or with those of ext, if non-null, into idx[1] (bucket_sort.hpp). *finished = false: too many suffixes are in buckets that do
 // not fit, and nothing that is used has changed. Works in the group tables, and in key[2], idx[3] and idx[4].
-int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* codes, u32* sufs, const u32* top_base, int* passes, bool* finished)
+int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* codes, u32* sufs, const u16* ext, const u32* top_base, int* passes,
+                   bool* finished)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -1268,6 +1281,16 @@ int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* co
     a.tail = tail;
     a.crowded = h->counts + 10;
     a.crowded_list = h->gstart[0]; // (done with before over_before)
+    if (ext) {
+        a.ext = ext;
+        a.ext_bits = digits.buckets_log2 < 16u ? digits.buckets_log2 : 16u;
+        a.sufs_out = h->idx[1];
+        a.ties = ties_of(h);
+        a.open_count = h->counts + 11;
+        a.open_sufs = open_sufs_of(h);
+        a.open_places = open_places_of(h);
+        a.over_open = h->counts + 12;
+    }
     a.over_before = h->gstart[0];
     a.over_tiles = h->gstart[1];
     hipLaunchKernelGGL(bucket_starts_kernel, dim3(a.buckets / (STARTS_BLOCK - 1) + 1), dim3(STARTS_BLOCK), 0, s, a);
@@ -1275,8 +1298,14 @@ int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* co
     if (rc)
         return rc;
     HIP_TRY(hipEventRecord(h->ev_gen[2], s)); // (recorded again when a generation ends)
-    hipLaunchKernelGGL(finish_buckets_kernel, dim3(a.buckets), dim3(BUCKET_BLOCK), 0, s, a);
-    hipLaunchKernelGGL(finish_crowded_kernel, dim3(a.buckets < CROWDED_BLOCKS ? a.buckets : CROWDED_BLOCKS), dim3(BUCKET_BLOCK), 0, s, a);
+    const dim3 crowded_grid(a.buckets < CROWDED_BLOCKS ? a.buckets : CROWDED_BLOCKS);
+    if (ext) {
+        hipLaunchKernelGGL(finish_buckets_kernel<true>, dim3(a.buckets), dim3(BUCKET_BLOCK), 0, s, a);
+        hipLaunchKernelGGL(finish_crowded_kernel<true>, crowded_grid, dim3(BUCKET_BLOCK), 0, s, a);
+    } else {
+        hipLaunchKernelGGL(finish_buckets_kernel<false>, dim3(a.buckets), dim3(BUCKET_BLOCK), 0, s, a);
+        hipLaunchKernelGGL(finish_crowded_kernel<false>, crowded_grid, dim3(BUCKET_BLOCK), 0, s, a);
+    }
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventSynchronize(h->ev_gen[2]));
     const u32 over = h->h_pinned[8], over_buckets = h->h_pinned[9];
@@ -1288,15 +1317,22 @@ int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* co
     a.over_keys = K[0];
     a.over_sufs = V[0];
     hipLaunchKernelGGL(over_before_kernel, dim3((a.buckets + OVER_TILE - 1) / OVER_TILE), dim3(OVER_TILE), 0, s, a);
-    hipLaunchKernelGGL(over_move_kernel<false>, dim3(over_buckets * OVER_SLICES), dim3(256), 0, s, a);
+    const dim3 over_grid(over_buckets * OVER_SLICES);
+    if (ext)
+        hipLaunchKernelGGL((over_move_kernel<false, true>), over_grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((over_move_kernel<false, false>), over_grid, dim3(256), 0, s, a);
     int in_out = 0, run = 0;
-    rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], V[0], K[1], V[1], over, make_plan(0, 32), &in_out, &run);
+    rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], V[0], K[1], V[1], over, make_plan(0, ext ? 48 : 32), &in_out, &run);
     if (rc)
         return rc;
     *passes += run;
     a.over_keys = K[in_out];
     a.over_sufs = V[in_out];
-    hipLaunchKernelGGL(over_move_kernel<true>, dim3(over_buckets * OVER_SLICES), dim3(256), 0, s, a);
+    if (ext)
+        hipLaunchKernelGGL((over_move_kernel<true, true>), over_grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((over_move_kernel<true, false>), over_grid, dim3(256), 0, s, a);
     HIP_TRY(hipGetLastError());
     return CSA_OK;
 }
@@ -1316,6 +1352,7 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
     else
         hipLaunchKernelGGL(radix_scan_hist_kernel<2 * RADIX_BINS>, dim3(1), dim3(2 * RADIX_BINS), 0, s, h->ghist, h->digit_base, (int)counted.passes);
     u32* const sorted[2] = {reinterpret_cast<u32*>(h->key[0]), reinterpret_cast<u32*>(h->key[0]) + h->cap};
+    u16* const ext[2] = {reinterpret_cast<u16*>(h->gid), reinterpret_cast<u16*>(h->gid) + h->cap}; // (no groups yet)
     const u32* top_base = nullptr;
     for (u32 p = 0; p < digits.passes; ++p) {
         const u32 out = (digits.passes - 1 - p) & 1, in = out ^ 1; // the sorted codes end in the first half of key[0], their suffixes in idx[0]
@@ -1346,7 +1383,14 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
         if (rc)
             return rc;
         rc = launch_pass(L, n, [&] {
-            if (p == 0 && packed)
+            if (digits.buckets_log2 && !packed) {
+                a.ext_in = p == 0 ? ext_of(h) : ext[in];
+                a.ext_out = ext[out];
+                if (p == 0)
+                    launch_onesweep32<SRC_CODED, true>(h, a, s);
+                else
+                    launch_onesweep32<SRC_PAIRS, true>(h, a, s);
+            } else if (p == 0 && packed)
                 launch_onesweep32<SRC_PACKED>(h, a, s);
             else if (p == 0)
                 launch_onesweep32<SRC_CODED>(h, a, s);
@@ -1359,7 +1403,7 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
     *passes = CODE_PASSES; // (the digits that are sorted in buckets among them)
     if (digits.buckets_log2) {
         bool finished = false;
-        int rc = finish_buckets(L, digits, n, tail, sorted[0], h->idx[0], top_base, passes, &finished);
+        int rc = finish_buckets(L, digits, n, tail, sorted[0], h->idx[0], packed ? nullptr : ext[0], top_base, passes, &finished);
         if (rc)
             return rc;
         if (!finished) { // (a sample had shown fewer suffixes in buckets that do not fit)
@@ -1394,6 +1438,16 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
     r.text_codes = codes_of(h);
     r.tail = tail;
     const dim3 resolve_grid((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE));
+    if (digits.buckets_log2 && !packed) { // the list stands in idx[1] already, but for its open runs
+        r.codes = nullptr;
+        r.open_count = h->counts + 11;
+        r.sufs = open_sufs_of(h);
+        r.places = open_places_of(h);
+        hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, false, false, true>), dim3(resolve_grid.x < OPEN_BLOCKS ? resolve_grid.x : OPEN_BLOCKS),
+                           dim3(RESOLVE_BLOCK), 0, s, r);
+        HIP_TRY(hipGetLastError());
+        return CSA_OK;
+    }
     if (words == 0 && n >= WORDS_AHEAD)
         hipLaunchKernelGGL(choose_words_kernel, dim3(1), dim3(LONG_LIST_PLACES), 0, s, r.codes, n, r.words_out);
     if (packed)
@@ -1894,7 +1948,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     // The byte histograms of the text come first: they tell whether the alphabet is small enough for keys of more than four
     // symbols. (The digit counts are zeroed with them.)
     TableGroup zeros = {};
-    add_table(zeros, h->counts, nullptr, 11 * sizeof(u32));
+    add_table(zeros, h->counts, nullptr, 13 * sizeof(u32));
     add_table(zeros, h->ghist, nullptr, (MAX_PASSES + 2) * RADIX_BINS * sizeof(u32));
     int rc = move_tables(zeros, s);
     if (rc)
@@ -1963,7 +2017,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         if (probed) {
             HIP_TRY(hipEventSynchronize(h->ev_gen[1]));
             coded = codes_pay(*seen, n);
-            if (coded && in_buckets && buckets_fit(*seen, n, bucket_digits(n, false)))
+            if (coded && in_buckets && !ahead && buckets_fit(*seen, n, bucket_digits(n, false)))
                 digits = bucket_digits(n, false);
         }
         if (coded && !ahead && (rc = code_suffixes(L, d_text, n, tail, counted = digits)) != CSA_OK)

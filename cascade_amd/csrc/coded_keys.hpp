@@ -184,6 +184,23 @@ __device__ __forceinline__ bool string_code(const u32 (&lo)[4], const u32 (&widt
     return alone;
 }
 
+// The same with 32 bits more, where the string does not take a code of its own: the place of the string inside its code's values, of which the upper
+// 16 are kept. (`low` is the upper half of the longer product, which may lie above `high`, cut at every step, where the interval is short.)
+__device__ __forceinline__ bool string_code(const u32 (&lo)[4], const u32 (&width)[4], u32& code, u32& within)
+{
+    u64 low = (u64)lo[3] << 32;
+    u32 high = lo[3] + width[3];
+#pragma unroll
+    for (int q = 2; q >= 0; --q) {
+        low = ((u64)lo[q] << 32) + (u64)width[q] * (u32)(low >> 32) + (((u64)width[q] * (u32)low) >> 32);
+        high = lo[q] + (u32)(((u64)width[q] * high) >> 32);
+    }
+    const bool alone = (int)(high - (u32)(low >> 32)) >= 2;
+    code = (u32)(low >> 32) + (alone ? 1u : 0u);
+    within = (u32)low >> 16;
+    return alone;
+}
+
 constexpr int PROBE_BLOCK = 256;
 constexpr u32 PROBE_START = 0x55555555u; // (the sample of the symbols is taken elsewhere: what its own places show is too good)
 constexpr u32 PROBE_MOST_LOG2 = 20;      // suffixes that are looked at
@@ -325,14 +342,16 @@ constexpr u32 CODE_BINS = CODE_PASSES * RADIX_BINS; // digit counts of all passe
 // BLOCK: the 32 KB of digit counters decide how many waves a CU holds, 16 in workgroups of 256 and 32 in workgroups of 1024,
 // which code 1e9 tokens in 2.27 instead of 3.06 ms and 2^28 in 0.58 instead of 0.78 (512: 2.69, 0.66; 256 with half the
 // counters: 2.92, 0.75). Short texts take 256, so that there are workgroups for every CU.
-// PASSES: of `digits`.
-template <int BLOCK, u32 PASSES>
+// PASSES: of `digits`. EXT: ext[v] = 16 bits that tell suffixes of one code apart, or come from equal symbols: of those that own it by their
+// next four symbols (of three alone there are runs a thousand long among 1e9 tokens), of others by the rest of their string's place. Larger for none that goes before another
+// suffix of the code.
+template <int BLOCK, u32 PASSES, bool EXT>
 __global__ __launch_bounds__(BLOCK) void code_suffixes_kernel(const u16* __restrict__ text, u32 n, u32 tail, const u32* __restrict__ cum,
                                                               u32* __restrict__ codes, u8* __restrict__ own, CodeDigits digits,
-                                                              u32* __restrict__ ghist)
+                                                              u32* __restrict__ ghist, u16* __restrict__ ext)
 {
-    constexpr u32 TILE = BLOCK * CODE_ITEMS;
-    __shared__ u64 s_text[(TILE + 3 + 6) / 4 + 2];
+    constexpr u32 TILE = BLOCK * CODE_ITEMS, AHEAD = EXT ? 7 : 3;
+    __shared__ u64 s_text[(TILE + AHEAD + 6) / 4 + 2];
     __shared__ u32 s_hist[CODE_BINS * CODE_COPIES];
     const u32 t = threadIdx.x;
     const u32 bits = PASSES == CODE_PASSES ? (u32)RADIX_BITS : digits.bits, bins = PASSES << bits;
@@ -343,24 +362,34 @@ __global__ __launch_bounds__(BLOCK) void code_suffixes_kernel(const u16* __restr
     for (u64 tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const u64 p0 = tile * TILE;
         __syncthreads(); // the counters are cleared; the stretch of the round before has been read
-        const u32 sym_off = stage_text(text, n, p0, TILE + 3u, s_text, t, BLOCK);
+        const u32 sym_off = stage_text(text, n, p0, TILE + AHEAD, s_text, t, BLOCK);
         __syncthreads();
         const u16* s16 = reinterpret_cast<const u16*>(s_text) + sym_off + t * CODE_ITEMS;
-        u32 lo[CODE_ITEMS + 3], width[CODE_ITEMS + 3];
+        u32 lo[CODE_ITEMS + AHEAD], width[CODE_ITEMS + AHEAD];
 #pragma unroll
-        for (int k = 0; k < CODE_ITEMS + 3; ++k) {
+        for (int k = 0; k < CODE_ITEMS + (int)AHEAD; ++k) {
             const u32 s = s16[k];
             u32 pair[2];
             __builtin_memcpy(pair, cum + s, 8); // entries s and s + 1 (4-byte aligned)
             lo[k] = pair[0];
             width[k] = pair[1] - pair[0];
         }
-        u32 code[CODE_ITEMS], owners = 0;
+        u32 code[CODE_ITEMS], more[CODE_ITEMS], owners = 0;
 #pragma unroll
         for (int k = 0; k < CODE_ITEMS; ++k) {
             const u32 lo4[4] = {lo[k], lo[k + 1], lo[k + 2], lo[k + 3]};
             const u32 width4[4] = {width[k], width[k + 1], width[k + 2], width[k + 3]};
-            owners |= (string_code(lo4, width4, code[k]) ? 1u : 0u) << k;
+            if constexpr (EXT) {
+                const bool alone = string_code(lo4, width4, code[k], more[k]);
+                u32 next = lo[k + 7];
+#pragma unroll
+                for (int q = 6; q >= 4; --q)
+                    next = lo[k + q] + (u32)(((u64)width[k + q] * next) >> 32);
+                more[k] = alone ? next >> 16 : more[k];
+                owners |= (alone ? 1u : 0u) << k;
+            } else {
+                owners |= (string_code(lo4, width4, code[k]) ? 1u : 0u) << k;
+            }
         }
         const u64 x0 = p0 + (u64)t * CODE_ITEMS;
         if (x0 < n)
@@ -370,12 +399,22 @@ __global__ __launch_bounds__(BLOCK) void code_suffixes_kernel(const u16* __restr
 #pragma unroll
             for (int k = 0; k < CODE_ITEMS; k += 4)
                 out[k / 4] = make_uint4(code[k], code[k + 1], code[k + 2], code[k + 3]);
+            if constexpr (EXT) { // (x0 is a multiple of eight, ext 16-byte aligned)
+                u64* const wide = reinterpret_cast<u64*>(ext + x0 + 4);
+#pragma unroll
+                for (int k = 0; k < CODE_ITEMS; k += 4)
+                    wide[k / 4] = (u64)(more[k] | more[k + 1] << 16) | (u64)(more[k + 2] | more[k + 3] << 16) << 32;
+            }
         } else {
 #pragma unroll
             for (int k = 0; k < CODE_ITEMS; ++k) {
                 const u64 x = x0 + k;
-                if (x < n)
-                    codes[x + tail >= n ? n - 1 - x : x + tail] = code[k];
+                if (x < n) {
+                    const u64 v = x + tail >= n ? n - 1 - x : x + tail;
+                    codes[v] = code[k];
+                    if constexpr (EXT)
+                        ext[v] = (u16)more[k];
+                }
             }
         }
 #pragma unroll
@@ -420,10 +459,11 @@ constexpr u32 RESOLVE_MARK_WORDS = 1u << (RESOLVE_MARK_BITS - 5);
 __device__ __forceinline__ u32 resolve_mark(u32 code) { return (code * 0x9E3779B1u) >> (32 - RESOLVE_MARK_BITS); }
 
 struct ResolveArgs {
-    const u32* codes; // sorted by code: the codes ...
+    const u32* codes; // sorted by code: the codes (null where they have not been kept) ...
     const u64* keys;  // ... or, of the members of long runs, (ordinal of the run's string << 32 | code of the four symbols after it)
     const u32* sufs;  // OWN_CODE (with codes): no other string has this suffix's code
-    u32 m;            // entries of the list
+    u32 m;            // entries of the list ...
+    const u32* open_count; // ... of open runs (OPEN), as the device has counted them; those start where bit 31 of their places is set
     const u16* text;
     u32 n;
     u32 words; // 1: the list is resolved on the symbols of the codes; 2: on as many after them, too; 0: as many_in_long_runs says ...
@@ -500,301 +540,321 @@ __global__ __launch_bounds__(LONG_LIST_PLACES) void choose_words_kernel(const u3
 // PACKED: the words are cut from the code stream of the text, 16 bytes of which hold what 128 bytes of the text do; it fits the last-level
 // cache up to 10^9 symbols of two bits.
 // SHORT: lists of fewer than WORDS_AHEAD suffixes, where the slowest tile counts; what that takes costs others 1.5 % of the kernel.
-template <int H, bool KEYS, bool PACKED, bool SHORT> // H: the longest run that is sorted inside its tile
-__global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_runs_kernel(ResolveArgs a)
+// OPEN: the list is that of runs that buckets have left open (finish_buckets_kernel), wherever they stand; a workgroup takes one tile after the other.
+template <int H, bool KEYS, bool PACKED, bool SHORT, bool OPEN = false> // H: the longest run that is sorted inside its tile
+__global__ __launch_bounds__(RESOLVE_BLOCK, OPEN ? 8 : 1) void resolve_runs_kernel(ResolveArgs a)
 {
-    constexpr int SPAN = RESOLVE_TILE + 2 * H;
-    constexpr int ITEMS = RESOLVE_ITEMS + 1; // the last one is the thread's element of the halo
-    constexpr int FEW = 16; // (sub-)runs of up to this many members are sorted without a look whether they are in order
-    __shared__ u64 s_head[SPAN / 64]; // bit j: the element at span place j starts a run (places outside the list count as starts)
-    __shared__ u64 s_down[SPAN / 64]; // bit j: its word is smaller than that of the element before it ...
-    __shared__ u64 s_diff[SPAN / 64]; // ... or another one
-    __shared__ u32 s_many[2];         // some run of the tile has more members, by word
-    __shared__ u32 s_ends;            // some member of a run runs off the text inside its words
-    __shared__ u32 s_words;
-    __shared__ u32 s_off[SHORT ? 2 : 1][SHORT ? SPAN / 32 : 1]; // bit j, by word: one of the run that starts at place j does
-    __shared__ __align__(16) u64 s_key[SPAN];
-    __shared__ __align__(16) u32 s_suf[SPAN];
-    __shared__ __align__(16) u8 s_tie[SPAN];
-    const u32 t = threadIdx.x;
-    if (t < 2)
-        s_many[t] = 0;
-    if (t == 2)
-        s_ends = 0;
-    const u32 told = KEYS ? TIE_MOST_WORDS : SHORT || a.words ? a.words : *a.words_out;
-    if (!KEYS && t < 64u) {
-        const u32 w = SHORT && told == 0 ? (many_in_long_runs(a.codes, a.m, HALF_LONG, SHORT_LIST_FEW) ? 1u : 2u) : told;
-        if (t == 0) {
-            if (SHORT)
-                s_words = w;
-            if (blockIdx.x == 0)
-                *a.words_out = w;
-        }
-    }
-    const long long t0 = (long long)blockIdx.x * RESOLVE_TILE, lo = t0 - H, m = a.m;
-    const u64 n = a.n;
-    // whole waves take consecutive places: one ballot per wave and round gives 64 bits of s_head
-    for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (the same rounds for every lane of a wave: SPAN is a multiple of 64)
-        const long long e = lo + j;
-        bool head = e <= 0 || e >= m;
-        u8 tie = 0;
-        if (!head) {
-            if constexpr (KEYS) {
-                const u64 mine = a.keys[e], before = a.keys[e - 1];
-                head = mine != before;
-                tie = (mine >> 32) == (before >> 32) ? 1 : 0; // (members of one string that do not run off the text inside it)
-            } else {
-                head = a.codes[e] != a.codes[e - 1];
+    static_assert(!OPEN || (!KEYS && !PACKED && !SHORT), "open runs are those of codes, in long lists");
+    constexpr bool PLACED = KEYS || OPEN; // the entries go to places of their own, where the ties of what starts a run are known
+    constexpr u8 TIE_KNOWN = 0x20;
+    const u32 entries = OPEN ? *a.open_count : a.m;
+    if (OPEN && blockIdx.x == 0 && threadIdx.x == 0)
+        *a.words_out = TIE_MOST_WORDS;
+    for (u32 tile = blockIdx.x; !OPEN || (u64)tile * RESOLVE_TILE < entries; tile += gridDim.x) {
+        constexpr int SPAN = RESOLVE_TILE + 2 * H;
+        constexpr int ITEMS = RESOLVE_ITEMS + 1; // the last one is the thread's element of the halo
+        constexpr int FEW = 16; // (sub-)runs of up to this many members are sorted without a look whether they are in order
+        __shared__ u64 s_head[SPAN / 64]; // bit j: the element at span place j starts a run (places outside the list count as starts)
+        __shared__ u64 s_down[SPAN / 64]; // bit j: its word is smaller than that of the element before it ...
+        __shared__ u64 s_diff[SPAN / 64]; // ... or another one
+        __shared__ u32 s_many[2];         // some run of the tile has more members, by word
+        __shared__ u32 s_ends;            // some member of a run runs off the text inside its words
+        __shared__ u32 s_words;
+        __shared__ u32 s_off[SHORT ? 2 : 1][SHORT ? SPAN / 32 : 1]; // bit j, by word: one of the run that starts at place j does
+        __shared__ __align__(16) u64 s_key[SPAN];
+        __shared__ __align__(16) u32 s_suf[SPAN];
+        __shared__ __align__(16) u8 s_tie[SPAN];
+        u32 t = threadIdx.x;
+        if (OPEN)
+            opaque(t); // (what follows from it is not kept from tile to tile: 152 registers, a workgroup a SIMD)
+        if (t < 2)
+            s_many[t] = 0;
+        if (t == 2)
+            s_ends = 0;
+        const u32 told = PLACED ? TIE_MOST_WORDS : SHORT || a.words ? a.words : *a.words_out;
+        if (!PLACED && t < 64u) {
+            const u32 w = SHORT && told == 0 ? (many_in_long_runs(a.codes, a.m, HALF_LONG, SHORT_LIST_FEW) ? 1u : 2u) : told;
+            if (t == 0) {
+                if (SHORT)
+                    s_words = w;
+                if (blockIdx.x == 0)
+                    *a.words_out = w;
             }
         }
-        s_tie[j] = head ? tie : (u8)TIE_MOST_WORDS;
-        const u64 b = __ballot(head);
-        if ((t & 63u) == 0)
-            s_head[j / 64] = b;
-    }
-    __syncthreads();
-    const u32 words = SHORT && !KEYS ? s_words : told;
-    if (words < TIE_MOST_WORDS)
-        for (int j = t; j < SPAN; j += RESOLVE_BLOCK) // (the thread's own places)
-            s_tie[j] = s_tie[j] ? (u8)words : (u8)0;
-    // the run around place j: first place and first place behind it; false if it has more than H members
-    auto run_of = [&](int j, int& first, int& last) -> bool {
-        int wd = j / 64;
-        u64 b = s_head[wd] & (~0ull >> (63 - (j & 63))); // starts at or before j
-        while (b == 0 && wd > 0 && wd * 64 > j - H)
-            b = s_head[--wd];
-        first = b ? wd * 64 + 63 - __builtin_clzll(b) : -1;
-        if (first < 0 || j - first > H)
-            return false;
-        wd = j / 64;
-        b = (j & 63) == 63 ? 0ull : s_head[wd] & (~0ull << ((j & 63) + 1)); // starts behind j
-        while (b == 0 && wd + 1 < SPAN / 64 && (wd + 1) * 64 <= j + H)
-            b = s_head[++wd];
-        last = b ? wd * 64 + __builtin_ctzll(b) : SPAN + H;
-        return last - first <= H;
-    };
-    // the elements: suffix, place, run, and the words where there is company
-    u32 x[ITEMS], owners = 0, longs = 0; // bit k: element k has OWN_CODE; is one of a long run
-    int at[ITEMS], first[ITEMS], last[ITEMS]; // last - first = 1: alone
-    u64 w0[ITEMS], w1[ITEMS];
-    const bool two = KEYS || words == 2; // (keys come with two words)
-    const u32 word_syms = PACKED ? a.word_syms : 4u;
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-        const bool halo = k == RESOLVE_ITEMS;
-        const int j = !halo ? H + k * RESOLVE_BLOCK + (int)t : (int)t < H ? (int)t : RESOLVE_TILE + (int)t;
-        const long long e = lo + j;
-        x[k] = 0;
-        at[k] = first[k] = j;
-        last[k] = j + 1;
-        w0[k] = w1[k] = 0;
-        if (e < 0 || e >= m || (halo && (int)t >= 2 * H))
-            continue;
-        int f, l;
-        const bool is_short = run_of(j, f, l);
-        if (halo) { // members of runs that reach into the tile; of a long run the left neighbour of the tile's first element alone
-            const bool left = (int)t < H;
-            if (is_short ? (left ? l <= H : f >= H + RESOLVE_TILE) : j != H - 1)
-                continue;
-        }
-        x[k] = a.sufs[e]; // (asked for before the runs are known, for all elements: no faster, 14.4 and 15.0 ms on 1e9 tokens)
-        if (!KEYS && (x[k] & OWN_CODE))
-            owners |= 1u << k;
-        x[k] &= ~OWN_CODE;
-        if (is_short) {
-            first[k] = f;
-            last[k] = l;
-            if (l - f == 1)
-                continue;
-        } else {
-            longs |= 1u << k;
-        }
-        const bool own = (owners >> k) & 1u;
-        if (!KEYS && !PACKED && !own)
-            w0[k] = load_kgram(a.text, a.n, x[k], 0);
-        if (two && (KEYS || is_short)) // (the members of long runs of codes get their second word when they are sorted by it)
-            w1[k] = second_word<PACKED>(a, x[k]);
-        if ((u64)x[k] + (u64)word_syms * words >= n)
-            s_ends = 1;
-        if (is_short && l - f > FEW) {
-            s_many[0] = 1;
-            s_many[1] = 1;
-        }
-    }
-    __syncthreads();
-    const bool ends = s_ends != 0;
-    if (SHORT && ends) {
-        for (int j = t; j < 2 * SPAN / 32; j += RESOLVE_BLOCK)
-            s_off[j / (SPAN / 32)][j % (SPAN / 32)] = 0;
-        __syncthreads();
-    }
-    // One word of all elements that still have company: refines their runs. Whoever runs off the text inside the word ties with
-    // nobody and comes before those with the same padded word, shortest first. (SHORT: only the runs with such a member are looked at that way: a tile
-    // is as slow as its slowest run, and a short text as its slowest tile. 10^5 symbols of phrases: 168 us with all runs of a tile that
-    // holds one of the last suffixes, 55 without.)
-    auto refine = [&](int w) {
-        const u64 ctx = word_syms * (u32)(w + 1);
-#pragma unroll
-        for (int k = 0; k < ITEMS; ++k)
-            if (last[k] - first[k] > 1 || ((longs >> k) & 1u)) {
-                s_suf[at[k]] = x[k];
-                if (w == 1 || !((owners >> k) & 1u))
-                    s_key[at[k]] = w == 0 ? w0[k] : w1[k];
-                if (SHORT && ends && (u64)x[k] + ctx >= n && !((longs >> k) & 1u))
-                    atomicOr(&s_off[w][first[k] / 32], 1u << (first[k] & 31));
-            }
-        __syncthreads();
-        const bool many = s_many[w] != 0 && (SHORT || !ends);
-        if (many) {
-            for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (places whose words were not wanted hold anything: no run looked at below has any)
-                const u64 down = __ballot(j > 0 && s_key[j] < s_key[j - 1]), diff = __ballot(j > 0 && s_key[j] != s_key[j - 1]);
-                if ((t & 63u) == 0) {
-                    s_down[j / 64] = down;
-                    s_diff[j / 64] = diff;
+        const long long t0 = (long long)tile * RESOLVE_TILE, lo = t0 - H, m = entries;
+        const u64 n = a.n;
+        // whole waves take consecutive places: one ballot per wave and round gives 64 bits of s_head
+        for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (the same rounds for every lane of a wave: SPAN is a multiple of 64)
+            const long long e = lo + j;
+            bool head = e <= 0 || e >= m;
+            u8 tie = 0;
+            if (!head) {
+                if constexpr (OPEN) {
+                    head = (a.places[e] & RUN_START) != 0;
+                } else if constexpr (KEYS) {
+                    const u64 mine = a.keys[e], before = a.keys[e - 1];
+                    head = mine != before;
+                    tie = (mine >> 32) == (before >> 32) ? 1 : TIE_KNOWN; // (members of one string that do not run off the text inside it)
+                } else {
+                    head = a.codes[e] != a.codes[e - 1];
                 }
             }
-            __syncthreads();
+            s_tie[j] = !head ? (u8)TIE_MOST_WORDS : OPEN || (KEYS && e <= 0) ? TIE_KNOWN : tie;
+            const u64 b = __ballot(head);
+            if ((t & 63u) == 0)
+                s_head[j / 64] = b;
         }
+        __syncthreads();
+        const u32 words = SHORT && !KEYS ? s_words : told;
+        if (words < TIE_MOST_WORDS)
+            for (int j = t; j < SPAN; j += RESOLVE_BLOCK) // (the thread's own places)
+                s_tie[j] = s_tie[j] ? (u8)words : (u8)0;
+        // the run around place j: first place and first place behind it; false if it has more than H members
+        auto run_of = [&](int j, int& first, int& last) -> bool {
+            int wd = j / 64;
+            u64 b = s_head[wd] & (~0ull >> (63 - (j & 63))); // starts at or before j
+            while (b == 0 && wd > 0 && wd * 64 > j - H)
+                b = s_head[--wd];
+            first = b ? wd * 64 + 63 - __builtin_clzll(b) : -1;
+            if (first < 0 || j - first > H)
+                return false;
+            wd = j / 64;
+            b = (j & 63) == 63 ? 0ull : s_head[wd] & (~0ull << ((j & 63) + 1)); // starts behind j
+            while (b == 0 && wd + 1 < SPAN / 64 && (wd + 1) * 64 <= j + H)
+                b = s_head[++wd];
+            last = b ? wd * 64 + __builtin_ctzll(b) : SPAN + H;
+            return last - first <= H;
+        };
+        // the elements: suffix, place, run, and the words where there is company
+        u32 x[ITEMS], owners = 0, longs = 0; // bit k: element k has OWN_CODE; is one of a long run
+        int at[ITEMS], first[ITEMS], last[ITEMS]; // last - first = 1: alone
+        u64 w0[ITEMS], w1[ITEMS];
+        const bool two = PLACED || words == 2; // (keys come with two words)
+        const u32 word_syms = PACKED ? a.word_syms : 4u;
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k) {
-            const int f = first[k], l = last[k], j = at[k];
-            if ((longs >> k) & 1u || l - f <= 1)
+            const bool halo = k == RESOLVE_ITEMS;
+            const int j = !halo ? H + k * RESOLVE_BLOCK + (int)t : (int)t < H ? (int)t : RESOLVE_TILE + (int)t;
+            const long long e = lo + j;
+            x[k] = 0;
+            at[k] = first[k] = j;
+            last[k] = j + 1;
+            w0[k] = w1[k] = 0;
+            if (e < 0 || e >= m || (halo && (int)t >= 2 * H))
                 continue;
-            const bool own = w == 0 && ((owners >> k) & 1u), off = ends && (!SHORT || ((s_off[w][f / 32] >> (f & 31)) & 1u));
-            int nf = f, nl = l, place = j;
-            if (own) { // one string: those that run off the text come first as they stand
-                if (off) {
-                    while (nf < l && (u64)s_suf[nf] + ctx >= n)
-                        ++nf;
-                    if (j < nf) {
-                        nf = j;
-                        nl = j + 1;
-                    }
-                }
-            } else {
-                bool counted = true;
-                if (many && l - f > FEW && !off) {
-                    // A run that is one string repeated, or several in order, stays as it is: its members need not be compared with
-                    // each other. (In a short text the kernel takes as long as the longest run of a tile: generation 0 of 2^18
-                    // symbols of phrases 221 us with all comparisons, 191 without these.)
-                    u64 seen = 0;
-                    for (int wd = (f + 1) / 64; wd <= (l - 1) / 64; ++wd) { // places f + 1 .. l - 1
-                        u64 b = s_down[wd];
-                        if (wd == (f + 1) / 64)
-                            b &= ~0ull << ((f + 1) & 63);
-                        if (wd == (l - 1) / 64)
-                            b &= ~0ull >> (63 - ((l - 1) & 63));
-                        seen |= b;
-                    }
-                    if (seen == 0) {
-                        counted = false;
-                        int wd = j / 64; // the last other word at or before j, the first behind it
-                        u64 b = s_diff[wd] & (~0ull >> (63 - (j & 63)));
-                        while (b == 0 && wd > f / 64)
-                            b = s_diff[--wd];
-                        const int start = b ? wd * 64 + 63 - __builtin_clzll(b) : f;
-                        nf = start > f ? start : f;
-                        wd = j / 64;
-                        b = (j & 63) == 63 ? 0ull : s_diff[wd] & (~0ull << ((j & 63) + 1));
-                        while (b == 0 && wd < (l - 1) / 64)
-                            b = s_diff[++wd];
-                        const int stop = b ? wd * 64 + __builtin_ctzll(b) : l;
-                        nl = stop < l ? stop : l;
-                    }
-                }
-                if (counted) {
-                    const u64 mine = s_key[j];
-                    int less = 0, equal = 0, before = 0; // equal: itself included
-                    if (!off) {
-                        for (int i = f; i < l; ++i) {
-                            const u64 v = s_key[i];
-                            less += v < mine ? 1 : 0;
-                            equal += v == mine ? 1 : 0;
-                            before += v == mine && i < j ? 1 : 0;
-                        }
-                    } else {
-                        const bool whole = (u64)x[k] + ctx < n;
-                        for (int i = f; i < l; ++i) {
-                            const u64 v = s_key[i];
-                            if (v < mine) {
-                                ++less;
-                            } else if (v == mine) {
-                                const u32 y = s_suf[i];
-                                const bool y_whole = (u64)y + ctx < n;
-                                if (whole != y_whole)
-                                    less += whole ? 1 : 0;
-                                else if (!whole)
-                                    less += y > x[k] ? 1 : 0;
-                                else
-                                    ++equal, before += i < j ? 1 : 0;
-                            }
-                        }
-                        equal = whole ? equal : 1;
-                    }
-                    nf = f + less;
-                    nl = nf + equal;
-                    place = nf + before;
-                }
+            int f, l;
+            const bool is_short = run_of(j, f, l);
+            if (halo) { // members of runs that reach into the tile; of a long run the left neighbour of the tile's first element alone
+                const bool left = (int)t < H;
+                if (is_short ? (left ? l <= H : f >= H + RESOLVE_TILE) : j != H - 1)
+                    continue;
             }
-            if (place == nf && nf != f)
-                s_tie[nf] = (u8)w;
-            first[k] = nf;
-            last[k] = nl;
-            at[k] = place;
+            x[k] = a.sufs[e]; // (asked for before the runs are known, for all elements: no faster, 14.4 and 15.0 ms on 1e9 tokens)
+            if (!KEYS && (x[k] & OWN_CODE))
+                owners |= 1u << k;
+            x[k] &= ~OWN_CODE;
+            if (is_short) {
+                first[k] = f;
+                last[k] = l;
+                if (l - f == 1)
+                    continue;
+            } else {
+                longs |= 1u << k;
+            }
+            const bool own = (owners >> k) & 1u;
+            if (!KEYS && !PACKED && !own)
+                w0[k] = load_kgram(a.text, a.n, x[k], 0);
+            if (two && (KEYS || is_short)) // (the members of long runs of codes get their second word when they are sorted by it)
+                w1[k] = second_word<PACKED>(a, x[k]);
+            if ((u64)x[k] + (u64)word_syms * words >= n)
+                s_ends = 1;
+            if (is_short && l - f > FEW) {
+                s_many[0] = 1;
+                s_many[1] = 1;
+            }
         }
-        // the members of long runs stay where they are: do they tie with their left neighbours, are they in order?
+        __syncthreads();
+        const bool ends = s_ends != 0;
+        if (SHORT && ends) {
+            for (int j = t; j < 2 * SPAN / 32; j += RESOLVE_BLOCK)
+                s_off[j / (SPAN / 32)][j % (SPAN / 32)] = 0;
+            __syncthreads();
+        }
+        // One word of all elements that still have company: refines their runs. Whoever runs off the text inside the word ties with
+        // nobody and comes before those with the same padded word, shortest first. (SHORT: only the runs with such a member are looked at that way: a tile
+        // is as slow as its slowest run, and a short text as its slowest tile. 10^5 symbols of phrases: 168 us with all runs of a tile that
+        // holds one of the last suffixes, 55 without.)
+        auto refine = [&](int w) {
+            const u64 ctx = word_syms * (u32)(w + 1);
 #pragma unroll
-        for (int k = 0; k < RESOLVE_ITEMS; ++k)
-            if ((longs >> k) & 1u && w == (KEYS ? 1 : 0)) {
-                const int j = at[k];
-                u8 tie = s_tie[j];
-                if (!((s_head[j / 64] >> (j & 63)) & 1ull)) {
-                    const bool whole = (u64)x[k] + ctx < n && (u64)s_suf[j - 1] + ctx < n;
-                    const bool own = w == 0 && ((owners >> k) & 1u);
-                    const u64 mine = own ? 0 : s_key[j], left = own ? 0 : s_key[j - 1];
-                    tie = (u8)(w + (mine == left && whole ? 1 : 0));
-                    if constexpr (KEYS) {
-                        if (mine < left || !whole)
-                            *a.unordered = 1u;
-                    } else if (mine < left) {
-                        const u32 mark = resolve_mark(a.codes[lo + j]), bit = 1u << (mark & 31u);
-                        if (!(a.marks[mark >> 5] & bit)) // (soon set for all to see: few of a run's members get to the atomic)
-                            atomicOr(&a.marks[mark >> 5], bit);
-                        *a.unordered = 1u;
+            for (int k = 0; k < ITEMS; ++k)
+                if (last[k] - first[k] > 1 || ((longs >> k) & 1u)) {
+                    s_suf[at[k]] = x[k];
+                    if (w == 1 || !((owners >> k) & 1u))
+                        s_key[at[k]] = w == 0 ? w0[k] : w1[k];
+                    if (SHORT && ends && (u64)x[k] + ctx >= n && !((longs >> k) & 1u))
+                        atomicOr(&s_off[w][first[k] / 32], 1u << (first[k] & 31));
+                }
+            __syncthreads();
+            const bool many = s_many[w] != 0 && (SHORT || !ends);
+            if (many) {
+                for (int j = t; j < SPAN; j += RESOLVE_BLOCK) { // (places whose words were not wanted hold anything: no run looked at below has any)
+                    const u64 down = __ballot(j > 0 && s_key[j] < s_key[j - 1]), diff = __ballot(j > 0 && s_key[j] != s_key[j - 1]);
+                    if ((t & 63u) == 0) {
+                        s_down[j / 64] = down;
+                        s_diff[j / 64] = diff;
+                    }
+                }
+                __syncthreads();
+            }
+#pragma unroll
+            for (int k = 0; k < ITEMS; ++k) {
+                const int f = first[k], l = last[k], j = at[k];
+                if ((longs >> k) & 1u || l - f <= 1)
+                    continue;
+                const bool own = w == 0 && ((owners >> k) & 1u), off = ends && (!SHORT || ((s_off[w][f / 32] >> (f & 31)) & 1u));
+                int nf = f, nl = l, place = j;
+                if (own) { // one string: those that run off the text come first as they stand
+                    if (off) {
+                        while (nf < l && (u64)s_suf[nf] + ctx >= n)
+                            ++nf;
+                        if (j < nf) {
+                            nf = j;
+                            nl = j + 1;
+                        }
                     }
                 } else {
-                    *a.any_long = 1u;
+                    bool counted = true;
+                    if (many && l - f > FEW && !off) {
+                        // A run that is one string repeated, or several in order, stays as it is: its members need not be compared with
+                        // each other. (In a short text the kernel takes as long as the longest run of a tile: generation 0 of 2^18
+                        // symbols of phrases 221 us with all comparisons, 191 without these.)
+                        u64 seen = 0;
+                        for (int wd = (f + 1) / 64; wd <= (l - 1) / 64; ++wd) { // places f + 1 .. l - 1
+                            u64 b = s_down[wd];
+                            if (wd == (f + 1) / 64)
+                                b &= ~0ull << ((f + 1) & 63);
+                            if (wd == (l - 1) / 64)
+                                b &= ~0ull >> (63 - ((l - 1) & 63));
+                            seen |= b;
+                        }
+                        if (seen == 0) {
+                            counted = false;
+                            int wd = j / 64; // the last other word at or before j, the first behind it
+                            u64 b = s_diff[wd] & (~0ull >> (63 - (j & 63)));
+                            while (b == 0 && wd > f / 64)
+                                b = s_diff[--wd];
+                            const int start = b ? wd * 64 + 63 - __builtin_clzll(b) : f;
+                            nf = start > f ? start : f;
+                            wd = j / 64;
+                            b = (j & 63) == 63 ? 0ull : s_diff[wd] & (~0ull << ((j & 63) + 1));
+                            while (b == 0 && wd < (l - 1) / 64)
+                                b = s_diff[++wd];
+                            const int stop = b ? wd * 64 + __builtin_ctzll(b) : l;
+                            nl = stop < l ? stop : l;
+                        }
+                    }
+                    if (counted) {
+                        const u64 mine = s_key[j];
+                        int less = 0, equal = 0, before = 0; // equal: itself included
+                        if (!off) {
+                            for (int i = f; i < l; ++i) {
+                                const u64 v = s_key[i];
+                                less += v < mine ? 1 : 0;
+                                equal += v == mine ? 1 : 0;
+                                before += v == mine && i < j ? 1 : 0;
+                            }
+                        } else {
+                            const bool whole = (u64)x[k] + ctx < n;
+                            for (int i = f; i < l; ++i) {
+                                const u64 v = s_key[i];
+                                if (v < mine) {
+                                    ++less;
+                                } else if (v == mine) {
+                                    const u32 y = s_suf[i];
+                                    const bool y_whole = (u64)y + ctx < n;
+                                    if (whole != y_whole)
+                                        less += whole ? 1 : 0;
+                                    else if (!whole)
+                                        less += y > x[k] ? 1 : 0;
+                                    else
+                                        ++equal, before += i < j ? 1 : 0;
+                                }
+                            }
+                            equal = whole ? equal : 1;
+                        }
+                        nf = f + less;
+                        nl = nf + equal;
+                        place = nf + before;
+                    }
                 }
-                s_tie[j] = tie | TIE_LONG;
+                if (place == nf && nf != f)
+                    s_tie[nf] = (u8)w;
+                first[k] = nf;
+                last[k] = nl;
+                at[k] = place;
             }
+            // the members of long runs stay where they are: do they tie with their left neighbours, are they in order?
+#pragma unroll
+            for (int k = 0; k < RESOLVE_ITEMS; ++k)
+                if ((longs >> k) & 1u && w == (KEYS ? 1 : 0)) {
+                    const int j = at[k];
+                    u8 tie = s_tie[j];
+                    if (!((s_head[j / 64] >> (j & 63)) & 1ull)) {
+                        const bool whole = (u64)x[k] + ctx < n && (u64)s_suf[j - 1] + ctx < n;
+                        const bool own = w == 0 && ((owners >> k) & 1u);
+                        const u64 mine = own ? 0 : s_key[j], left = own ? 0 : s_key[j - 1];
+                        tie = (u8)(w + (mine == left && whole ? 1 : 0));
+                        if constexpr (KEYS) {
+                            if (mine < left || !whole)
+                                *a.unordered = 1u;
+                        } else if (mine < left) {
+                            const u32 mark = resolve_mark(OPEN ? a.text_codes[suffix_to_virtual(x[k], a.n, a.tail)] : a.codes[lo + j]), bit = 1u << (mark & 31u);
+                            if (!(a.marks[mark >> 5] & bit)) // (soon set for all to see: few of a run's members get to the atomic)
+                                atomicOr(&a.marks[mark >> 5], bit);
+                            *a.unordered = 1u;
+                        }
+                    } else {
+                        *a.any_long = 1u;
+                        tie |= OPEN ? TIE_HEAD : 0;
+                    }
+                    s_tie[j] = tie | TIE_LONG;
+                }
+            __syncthreads();
+        };
+        if constexpr (!KEYS)
+            refine(0);
+        if (two)
+            refine(1);
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k)
+            if (k < RESOLVE_ITEMS || (int)t < 2 * H)
+                s_suf[at[k]] = x[k];
         __syncthreads();
-    };
-    if constexpr (!KEYS)
-        refine(0);
-    if (two)
-        refine(1);
+        const int j = H + (int)t * RESOLVE_ITEMS;
+        const long long e = lo + j;
+        if constexpr (!PLACED) {
+            if (e + RESOLVE_ITEMS <= m) { // (e is a multiple of RESOLVE_ITEMS, and the arrays are 16-byte aligned)
+                static_assert(RESOLVE_ITEMS == 4 && H % 4 == 0, "four suffixes leave in one 16-byte store");
+                *reinterpret_cast<uint4*>(a.sufs_out + e) = *reinterpret_cast<const uint4*>(s_suf + j);
+                *reinterpret_cast<u32*>(a.ties + e) = *reinterpret_cast<const u32*>(s_tie + j);
+                return;
+            }
+        }
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k)
-        if (k < RESOLVE_ITEMS || (int)t < 2 * H)
-            s_suf[at[k]] = x[k];
-    __syncthreads();
-    const int j = H + (int)t * RESOLVE_ITEMS;
-    const long long e = lo + j;
-    if constexpr (!KEYS) {
-        if (e + RESOLVE_ITEMS <= m) { // (e is a multiple of RESOLVE_ITEMS, and the arrays are 16-byte aligned)
-            static_assert(RESOLVE_ITEMS == 4 && H % 4 == 0, "four suffixes leave in one 16-byte store");
-            *reinterpret_cast<uint4*>(a.sufs_out + e) = *reinterpret_cast<const uint4*>(s_suf + j);
-            *reinterpret_cast<u32*>(a.ties + e) = *reinterpret_cast<const u32*>(s_tie + j);
+        for (int k = 0; k < RESOLVE_ITEMS; ++k)
+            if (e + k < m) {
+                const u64 to = OPEN ? (u64)(a.places[e + k] & ~RUN_START) : KEYS ? (u64)a.places[e + k] : (u64)(e + k);
+                u8 tie = s_tie[j + k];
+                if (PLACED && (tie & TIE_KNOWN))
+                    tie = (u8)((tie & ~TIE_KNOWN) | (a.ties[to] & TIE_WORDS));
+                a.sufs_out[to] = s_suf[j + k];
+                a.ties[to] = tie;
+            }
+        if (!OPEN)
             return;
-        }
+        __syncthreads();
     }
-#pragma unroll
-    for (int k = 0; k < RESOLVE_ITEMS; ++k)
-        if (e + k < m) {
-            const u64 to = KEYS ? (u64)a.places[e + k] : (u64)(e + k);
-            a.sufs_out[to] = s_suf[j + k];
-            a.ties[to] = s_tie[j + k];
-        }
 }
 
 // What a list sorted by the narrow keys of a packed text would leave at contexts shorter than a key (RerankArgs::level_drop, level_ell; the
@@ -863,6 +923,9 @@ constexpr int COLLECT_BLOCK = 256;
 constexpr int COLLECT_ITEMS = 4;
 constexpr int COLLECT_TILE = COLLECT_BLOCK * COLLECT_ITEMS;
 
+// Does this entry of a long run start a string (or, of a run that is a string's with 16 bits of what follows, the run)?
+__device__ __forceinline__ bool starts_string(u32 tie) { return (tie & TIE_WORDS) == 0 || (tie & TIE_HEAD); }
+
 template <bool MARKED, bool APPLY>
 __global__ __launch_bounds__(COLLECT_BLOCK) void collect_runs_kernel(ResolveArgs a)
 {
@@ -890,12 +953,13 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_runs_kernel(ResolveArgs
         if ((ties >> (8 * k)) & TIE_LONG) {
             u32 in = 1u;
             if constexpr (MARKED) {
-                const u32 mark = resolve_mark(a.codes[base + k]);
+                const u32 code = a.codes ? a.codes[base + k] : a.text_codes[suffix_to_virtual(a.sufs_out[base + k], a.n, a.tail)];
+                const u32 mark = resolve_mark(code);
                 in = (a.marks[mark >> 5] >> (mark & 31u)) & 1u;
             }
             flags |= in << k;
             mine += in;
-            heads += in && ((ties >> (8 * k)) & TIE_WORDS) == 0 ? 1u : 0u;
+            heads += in && starts_string(ties >> (8 * k)) ? 1u : 0u;
         }
     const u32 incl = wave_incl_sum(mine), incl_heads = wave_incl_sum(heads);
     if (lane == 63u) {
@@ -944,7 +1008,7 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_runs_kernel(ResolveArgs
     for (int k = 0; k < COLLECT_ITEMS; ++k)
         if ((flags >> k) & 1u) {
             if constexpr (!MARKED) {
-                ordinal += ((ties >> (8 * k)) & TIE_WORDS) == 0 ? 1u : 0u;
+                ordinal += starts_string(ties >> (8 * k)) ? 1u : 0u;
                 key[k] |= (u64)(ordinal - 1u) << 32;
             }
             a.run_keys[slot] = key[k];
@@ -963,7 +1027,8 @@ __global__ __launch_bounds__(256) void place_marked_kernel(ResolveArgs a, u32 co
     const u32 x = a.members[i];
     const bool tied = i > 0 && a.run_keys[i] == a.run_keys[i - 1] && (u64)x + 4 < a.n && (u64)a.members[i - 1] + 4 < a.n;
     a.sufs_out[a.places[i]] = x;
-    a.ties[a.places[i]] = (u8)(TIE_LONG | (tied ? 1u : 0u));
+    if (!(a.ties[a.places[i]] & TIE_HEAD)) // (whose left neighbour is none of these)
+        a.ties[a.places[i]] = (u8)(TIE_LONG | (tied ? 1u : 0u));
 }
 
 } // namespace csa

@@ -23,6 +23,16 @@ constexpr unsigned DEV_ERR_RERANK_RANGE = 4;
 constexpr unsigned DEV_ERR_UNEXPECTED_LARGE_GROUP = 5;
 constexpr unsigned DEV_ERR_JOIN_TABLE_FULL = 6;
 
+// The compiler takes v for a value that it knows nothing about.
+__device__ __forceinline__ void opaque(u32& v)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+v"(v));
+#else
+    (void)v;
+#endif
+}
+
 __device__ __forceinline__ u32 lane_id() { return __lane_id(); }
 
 // ---- wave64 inclusive scans by shuffles ----

@@ -59,6 +59,11 @@ __device__ __forceinline__ u32 virtual_to_suffix(u32 i, u32 n, u32 tail)
     return i < tail ? n - 1 - i : i - tail;
 }
 
+__device__ __forceinline__ u32 suffix_to_virtual(u32 x, u32 n, u32 tail)
+{
+    return x + tail >= n ? n - 1 - x : x + tail;
+}
+
 struct HistArgs {
     const u64* keys;
     u32 n; // pairs
@@ -295,6 +300,8 @@ struct OnesweepArgs {
     u32* err;
     const u16* text = nullptr; // SRC_TEXT
     const u8* own = nullptr;   // SRC_CODED: flags by text position, 8 to a byte
+    const u16* ext_in = nullptr; // EXT: by virtual position, or of the pairs
+    u16* ext_out = nullptr;
     const u32* rank = nullptr; // SRC_RANKS: rank[] by text position ...
     u32 hop = 0;               // ... the distance to the second rank of a key ...
     u32 radix = 0;             // ... and how the two make the key (rank_pair_key)
@@ -351,10 +358,8 @@ __device__ __forceinline__ u32 onesweep_tile_number(const OnesweepArgs& a)
 
 #ifdef __HIP_DEVICE_COMPILE__
 #define CSA_LDS_ORDER() asm volatile("" ::: "memory")
-#define CSA_OPAQUE(x) asm volatile("" : "+v"(x))
 #else
 #define CSA_LDS_ORDER() __builtin_amdgcn_wave_barrier() /* CPU emulation: lanes are threads, order them for real */
-#define CSA_OPAQUE(x) ((void)0)
 #endif
 
 // The place of a lane's item among the items of its wave so far that have digit d (DB bits), those of this call in lane order; whist[d] counts
@@ -371,7 +376,7 @@ __device__ __forceinline__ u32 rank_in_wave(u32 d, u32* whist)
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
         u32 mine = (u32)__builtin_amdgcn_sbfe(d, b, 1); // 0 or 0xFFFFFFFF
-        CSA_OPAQUE(mine); // the ballot tests this register (one compare), not a second extraction of the bit
+        opaque(mine); // the ballot tests this register (one compare), not a second extraction of the bit
         const u64 bal = __ballot((int)mine < 0);
         // same &= ~(bal ^ mine): one three-input bit operation per half (table of a & ~(b ^ c): 0x90)
         same_lo = __builtin_amdgcn_bitop3_b32(same_lo, (u32)bal, mine, 0x90);
@@ -387,14 +392,13 @@ __device__ __forceinline__ u32 rank_in_wave(u32 d, u32* whist)
 }
 
 #undef CSA_LDS_ORDER
-#undef CSA_OPAQUE
 
 // KeyT is u64 (the suffix-sort keys) or u32 (the (text position, rank) pairs of the bucketed rank update).
 // HI selects the 32-bit half of a 64-bit key that holds this pass's digit (digits never straddle the halves),
 // so that the digit is one bit-field extract of a 32-bit register.
 // VALS = false: the keys travel alone (records whose payload sits in the key bits that are not sorted on).
-// DB: bits of the widest digit.
-template <typename KeyT, int BLOCK, int ITEMS, int SRC, int HI, bool VALS = true, int DB = RADIX_BITS>
+// DB: bits of the widest digit. EXT: sixteen bits more travel beside the values.
+template <typename KeyT, int BLOCK, int ITEMS, int SRC, int HI, bool VALS = true, int DB = RADIX_BITS, bool EXT = false>
 __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(OnesweepArgs a)
 {
     static_assert(VALS || SRC == SRC_PAIRS, "the passes that build their keys make the suffix indices");
@@ -597,6 +601,25 @@ __global__ __launch_bounds__(BLOCK, CSA_SORT_MIN_WAVES) void onesweep_kernel(One
         const u32 q = k * BLOCK + t;
         if (q < valid)
             a.vals_out[dst[k]] = s_vals[q];
+    }
+    if constexpr (EXT) {
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const u32 local = first_local + k * WAVE;
+            val[k] = local < valid ? a.ext_in[base + local] : 0u;
+        }
+        __syncthreads();
+        u16* s_ext = reinterpret_cast<u16*>(s_keys);
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k)
+            s_ext[pos[k]] = (u16)val[k];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const u32 q = k * BLOCK + t;
+            if (q < valid)
+                a.ext_out[dst[k]] = s_ext[q];
+        }
     }
 #undef CSA_DIGIT
 }

@@ -969,18 +969,28 @@ def test_wide_loads_are_aligned_for_every_capacity():
 
 
 @pytest.mark.parametrize("n", [17000, 33000, 41000])
-@pytest.mark.parametrize("kind", ["even", "heavy", "crowded", "copies", "letters"])
+@pytest.mark.parametrize("kind", ["even", "heavy", "crowded", "copies", "letters", "shared", "repeated", "end"])
 def test_lower_digits_are_sorted_in_buckets(n, kind):
     """A build with buckets of up to 256 suffixes, 512 cells of up to 20 members that are compared, and two passes of eight bits below 2^15 symbols, of
-    nine above: even codes, strings that fill a bucket and more (they are collected and radix sorted) or a cell (passes in LDS), copies, packed symbols of
-    two bits. Suffix array and generation sizes are the oracle's."""
+    nine above; the sixteen bits that travel with a code tell suffixes apart that share it, the rest is left open and resolved from the text. Even codes, strings that fill
+    a bucket and more (they are collected and radix sorted) or a cell (passes in LDS), copies, packed symbols of two bits, strings that share a code without owning it, runs of
+    one string past the in-tile limit, a string that ends the text. Suffix array and generation sizes are the oracle's."""
     lib = load_emulation("libcascade_emu_buckets.so")
     rng = np.random.default_rng(n)
-    T = texts.text_of_copies(n, 4 if kind == "letters" else 60000, n) if kind in ("copies", "letters") else rng.integers(1, 60000, n).astype(np.uint16)
-    if kind in ("heavy", "crowded"):
-        for string, times in enumerate([400, 257, 90] if kind == "heavy" else [120, 64, 21, 22]):
+    if kind in ("copies", "letters"):
+        T = texts.text_of_copies(n, 4 if kind == "letters" else 60000, n)
+    elif kind == "shared":
+        T = texts.text_with_shared_codes(n, [2, 5, 63, 64, 65, 70, 90], n)
+    elif kind == "repeated":
+        T = texts.text_with_repeated_strings(n, [64, 65, 300, 400], 3, 5, n)
+    else:
+        T = rng.integers(1, 60000, n).astype(np.uint16)
+        for string, times in enumerate({"heavy": [400, 257, 90], "crowded": [120, 64, 21, 22], "end": [30]}.get(kind, [])):
             for at in rng.permutation(n // 8 - 1)[:times]:
                 T[8 * at:8 * at + 4] = [7, 8, 9, 100 * string]
-    got, active, _ = emu_sort(lib, T, 1)
-    sa, counts = oracle_lib.prefix_doubling(T, 1)
-    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+        if kind == "end":
+            T[-9:] = [0, 0, 7, 8, 9, 0, 7, 8, 9]
+    for key_words in (1, 4):
+        got, active, _ = emu_sort(lib, T, key_words)
+        sa, counts = oracle_lib.prefix_doubling(T, key_words)
+        assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
