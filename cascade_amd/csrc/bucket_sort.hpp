@@ -19,7 +19,7 @@ namespace csa {
 #define CSA_BUCKET_ITEMS 7
 #endif
 #ifndef CSA_CELLS_LOG2
-#define CSA_CELLS_LOG2 13
+#define CSA_CELLS_LOG2 12
 #endif
 #ifndef CSA_CELL_MAX
 #define CSA_CELL_MAX 512
@@ -52,7 +52,7 @@ struct BucketArgs {
     u8* ties;
     u32* open_count; // zeroed: suffixes in runs of one code and one ext, which are left open (resolve_runs_kernel) ...
     u32* open_sufs;  // ... them, run after run, with OWN_CODE ...
-    u32* open_places; // ... and their places in the list, with RUN_START
+    u32* open_places; // ... and their places in the list, with RUN_START and RUN_TIED
     // the suffixes of buckets that do not fit, collected in list order
     u32* over_before; // [buckets]: of the buckets before this one whose number is the same in its upper bits (OVER_TILE buckets) ...
     u32* over_tiles;  // ... and of all that differ in those, by them
@@ -119,7 +119,9 @@ __device__ __forceinline__ void write_bucket(const BucketArgs& a, u32 start, u32
     constexpr int BLOCK = BUCKET_BLOCK, ITEMS = BUCKET_ITEMS;
     const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6;
     const u32 rounds = (size + BLOCK - 1) / BLOCK;
-    u32 suf[ITEMS], member = 0, begins = 0; // bit k: the entry of round k is one of a run; begins one
+    u32* const sufs_out = a.sufs_out + start;
+    u8* const ties = a.ties + start;
+    u32 suf[ITEMS], member = 0, begins = 0, tied = 0; // bit k: the entry of round k is one of a run; begins one; ties with its left neighbour on one word
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k)
         if ((u32)k < rounds) {
@@ -133,10 +135,12 @@ __device__ __forceinline__ void write_bucket(const BucketArgs& a, u32 start, u32
             suf[k] = x | ((u32)pair & OWN_CODE);
             member |= (in ? 1u : 0u) << k;
             begins |= (follows ? 0u : 1u) << k;
-            if (j < size) {
-                a.sufs_out[start + j] = x;
-                a.ties[start + j] = (u8)tie_of_strings(same_code, (u32)pair, (u32)left, a.tail);
+            const u32 tie = tie_of_strings(same_code, (u32)pair, (u32)left, a.tail);
+            if (j < size) { // (most of a run are copies, tied on both words, and stay as they stand: what is to be resolved is written as if they were)
+                sufs_out[j] = x;
+                ties[j] = (u8)(follows ? TIE_MOST_WORDS : tie);
             }
+            tied |= tie << k;
             const u64 b = __ballot(in);
             if (lane == 0)
                 s_open[k * (BLOCK / WAVE) + w] = (u32)__popcll(b);
@@ -164,17 +168,17 @@ __device__ __forceinline__ void write_bucket(const BucketArgs& a, u32 start, u32
             if (in) {
                 const u32 slot = s_open[k * (BLOCK / WAVE) + w] + (u32)__popcll(b & ((1ull << lane) - 1ull));
                 a.open_sufs[slot] = suf[k];
-                a.open_places[slot] = (start + k * BLOCK + t) | ((begins >> k) & 1u ? RUN_START : 0u);
+                a.open_places[slot] = (start + k * BLOCK + t) | ((begins >> k) & 1u ? RUN_START | ((tied >> k) & 1u ? RUN_TIED : 0u) : 0u);
             }
         }
 }
 
-// One bucket a workgroup. Its suffixes go to 8192 cells by the next bits of their codes, in whatever order they arrive, and everyone is compared with the
+// One bucket a workgroup. Its suffixes go to 4096 cells by the next bits of their codes, in whatever order they arrive, and everyone is compared with the
 // others in its cell, of which there are one or two, by the whole code and its place in the order of the text. What bounds it are vector
 // instructions: all threads do the same for whole rounds, what is past the end of the bucket going to a cell of its own. Buckets with a long
 // cell, one string hundreds of times, are left to finish_crowded_kernel.
 template <bool EXT>
-__global__ __launch_bounds__(BUCKET_BLOCK, 8) void finish_buckets_kernel(BucketArgs a)
+__global__ __launch_bounds__(BUCKET_BLOCK, 2 * BUCKET_BLOCK / 256) void finish_buckets_kernel(BucketArgs a)
 {
     constexpr int BLOCK = BUCKET_BLOCK, ITEMS = BUCKET_ITEMS, CAP = BUCKET_MAX, CELLS = 1 << CELLS_LOG2;
     constexpr int PER = CELLS / BLOCK; // cells of a thread in the scan
@@ -469,10 +473,11 @@ __global__ __launch_bounds__(256) void over_move_kernel(BucketArgs a)
                 const u32 left = a.over_sufs[to + i - 1] & ~OWN_CODE;
                 tie = tie_of_strings(true, suffix_to_virtual(x, a.n, a.tail) | (v & OWN_CODE), suffix_to_virtual(left, a.n, a.tail), a.tail);
             }
-            a.ties[start + i] = (u8)tie;
+            a.sufs_out[start + i] = x;
+            a.ties[start + i] = (u8)(follows ? TIE_MOST_WORDS : tie);
             const u32 slot = *a.over_open + to + i; // (all of them are listed, runs or not)
             a.open_sufs[slot] = v;
-            a.open_places[slot] = (start + i) | (follows ? 0u : RUN_START);
+            a.open_places[slot] = (start + i) | (follows ? 0u : RUN_START | (tie ? RUN_TIED : 0u));
         }
     }
 }

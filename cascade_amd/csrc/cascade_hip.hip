@@ -1033,7 +1033,7 @@ CodeTables code_tables(const csa_handle* h)
 #define CSA_TWO_PASS_LOG2 16
 #endif
 #ifndef CSA_BUCKET_AVERAGE
-#define CSA_BUCKET_AVERAGE 4096
+#define CSA_BUCKET_AVERAGE 5000
 #endif
 constexpr u32 BUCKET_AVERAGE = CSA_BUCKET_AVERAGE;
 constexpr CodeDigits ALL_DIGITS = {CODE_PASSES, RADIX_BITS, {0, 8, 16, 24}, 0};
@@ -1048,7 +1048,7 @@ CodeDigits bucket_digits(u32 n, bool packed)
         log2 = CSA_TWO_PASS_LOG2;
     if (log2 <= CSA_TWO_PASS_LOG2)
         return CodeDigits{2, RADIX_BITS, {16, 24}, log2};
-    if (log2 <= 18 && !packed)
+    if (log2 <= 18 && !packed && n <= RUN_PLACE)
         return CodeDigits{2, RADIX_BITS + 1, {14, 23}, log2};
     return ALL_DIGITS;
 }

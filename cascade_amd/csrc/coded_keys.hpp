@@ -244,13 +244,16 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
 {
     __shared__ unsigned long long s_pairs[PROBE_BLOCK / WAVE];
     __shared__ u32 s_cnt[PROBE_FLAGS];
+    __shared__ u32 s_bucket[PROBE_BLOCK], s_members[PROBE_BLOCK], s_before[PROBE_BLOCK];
     if (a.skipped && *a.skipped)
         return;
     const u32 t = threadIdx.x;
     if (t < PROBE_FLAGS)
         s_cnt[t] = 0;
+    s_bucket[t] = ~0u;
+    s_members[t] = 0;
     __syncthreads();
-    u32 pairs = 0, flags = 0;
+    u32 pairs = 0, flags = 0, bucket = ~0u, in_bucket = ~0u;
     const u32 i = blockIdx.x * PROBE_BLOCK + t;
     if (i < a.taken) {
         const u64 x = sampled_chunk(i, a.n, a.taken, PROBE_START);
@@ -270,12 +273,12 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
             }
             alone = string_code(lo, width, code);
         }
-        const bool placed = a.buckets && (i & a.bucket_skip) == 0;
-        // (a full one is not counted any further: additions to one address queue, 54 us instead of 10 for a text of runs)
-        u32* const bucket = placed ? a.buckets + (code >> a.bucket_shift) : nullptr;
-        u32 company = placed ? __hip_atomic_load(bucket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-        if (placed && company < a.full_from)
-            company = atomicAdd(bucket, 1u);
+        if (a.buckets && (i & a.bucket_skip) == 0) {
+            bucket = code >> a.bucket_shift;
+            const u32 seen = atomicCAS(&s_bucket[bucket % PROBE_BLOCK], ~0u, bucket);
+            if (seen == ~0u || seen == bucket)
+                in_bucket = atomicAdd(&s_members[bucket % PROBE_BLOCK], 1u);
+        }
         if (!alone) {
             const unsigned long long entry = ((unsigned long long)code << 32) | (hash >> 24 << 24) | 1u;
             const u32 mask = (1u << a.table_log2) - 1u;
@@ -295,8 +298,19 @@ __global__ __launch_bounds__(PROBE_BLOCK) void probe_codes_kernel(ProbeArgs a)
                 break;
             }
         }
-        if (placed && company >= a.full_from)
-            flags |= 64u;
+    }
+    // The members of a bucket are added by one of the workgroup's: additions to one address queue (a text of runs: 54 us, 10 without).
+    if (a.buckets) {
+        __syncthreads();
+        u32 before = 0;
+        if (in_bucket == 0)
+            s_before[bucket % PROBE_BLOCK] = atomicAdd(&a.buckets[bucket], s_members[bucket % PROBE_BLOCK]);
+        else if (in_bucket == ~0u && bucket != ~0u) // (its place is another bucket's)
+            before = atomicAdd(&a.buckets[bucket], 1u);
+        __syncthreads();
+        if (in_bucket != ~0u)
+            before = s_before[bucket % PROBE_BLOCK] + in_bucket;
+        flags |= bucket != ~0u && before >= a.full_from ? 64u : 0u;
     }
 #pragma unroll
     for (u32 k = 0; k < PROBE_FLAGS; ++k) {
@@ -844,9 +858,19 @@ __global__ __launch_bounds__(RESOLVE_BLOCK, OPEN ? 8 : 1) void resolve_runs_kern
 #pragma unroll
         for (int k = 0; k < RESOLVE_ITEMS; ++k)
             if (e + k < m) {
-                const u64 to = OPEN ? (u64)(a.places[e + k] & ~RUN_START) : KEYS ? (u64)a.places[e + k] : (u64)(e + k);
+                if constexpr (OPEN) { // what is as the buckets have left it is not written again (a line each)
+                    const u32 place = a.places[e + k], before = place & RUN_START ? (place & RUN_TIED ? 1u : 0u) : TIE_MOST_WORDS;
+                    const u32 known = s_tie[j + k], tie = known & TIE_KNOWN ? (known & ~TIE_KNOWN) | before : known;
+                    const u64 to = place & RUN_PLACE;
+                    if (s_suf[j + k] != (a.sufs[e + k] & ~OWN_CODE))
+                        a.sufs_out[to] = s_suf[j + k];
+                    if (tie != before)
+                        a.ties[to] = (u8)tie;
+                    continue;
+                }
+                const u64 to = KEYS ? (u64)a.places[e + k] : (u64)(e + k);
                 u8 tie = s_tie[j + k];
-                if (PLACED && (tie & TIE_KNOWN))
+                if (KEYS && (tie & TIE_KNOWN))
                     tie = (u8)((tie & ~TIE_KNOWN) | (a.ties[to] & TIE_WORDS));
                 a.sufs_out[to] = s_suf[j + k];
                 a.ties[to] = tie;

@@ -26,7 +26,8 @@ constexpr u32 NO_RANK = 0xFFFFFFFFu; // ranks are below 2^31
 // run that was too long to be resolved in its tile.
 constexpr u32 TIE_LONG = 0x80u, TIE_HEAD = 0x40u, TIE_WORDS = 0x1Fu; // (TIE_HEAD: of a long run that buckets had left open, its first one)
 constexpr u32 TIE_MOST_WORDS = 2;
-constexpr u32 RUN_START = 0x80000000u; // of the place (below 2^31) of an open run's first entry (bucket_sort.hpp)
+// Of the place (below 2^30) of an open run's first entry (bucket_sort.hpp): that it is one; that it ties with its left neighbour on one word.
+constexpr u32 RUN_START = 0x80000000u, RUN_TIED = 0x40000000u, RUN_PLACE = 0x3FFFFFFFu;
 
 // The tiles of a rank step are scanned in RERANK_SLABS slabs (rerank_scan_kernel): a tile's prefix is its prefix inside
 // its slab combined with the totals (max, max, sum, sum, -) of the slabs before. One slab per lane: a wave fetches the

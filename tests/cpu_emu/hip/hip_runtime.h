@@ -277,6 +277,17 @@ inline T __shfl_up(T var, unsigned delta)
 }
 
 template <typename T>
+inline T __shfl_down(T var, unsigned delta)
+{
+    hipemu::Wave* w = hipemu::wave;
+    w->buf[hipemu::lane] = (uint64_t)var;
+    hipemu::wave_sync(w);
+    const T r = hipemu::lane + delta < 64u ? (T)w->buf[hipemu::lane + delta] : var;
+    hipemu::wave_sync(w);
+    return r;
+}
+
+template <typename T>
 inline T __shfl_xor(T var, unsigned mask)
 {
     hipemu::Wave* w = hipemu::wave;
@@ -346,6 +357,11 @@ inline unsigned long long atomicCAS(unsigned long long* p, unsigned long long ex
 {
     __atomic_compare_exchange_n(p, &expected, desired, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);
     return expected; // the value found, as the device function returns it
+}
+inline unsigned atomicCAS(unsigned* p, unsigned expected, unsigned desired)
+{
+    __atomic_compare_exchange_n(p, &expected, desired, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);
+    return expected;
 }
 inline unsigned long long __umul64hi(unsigned long long a, unsigned long long b) { return (unsigned long long)(((unsigned __int128)a * b) >> 64); }
 
