@@ -379,14 +379,27 @@ __global__ __launch_bounds__(BLOCK) void code_suffixes_kernel(const u16* __restr
         const u32 sym_off = stage_text(text, n, p0, TILE + AHEAD, s_text, t, BLOCK);
         __syncthreads();
         const u16* s16 = reinterpret_cast<const u16*>(s_text) + sym_off + t * CODE_ITEMS;
+        // A thread looks its own symbols up, and has those after them from the lane after it; the last lane of a wave looks them up as well. (A gather from the
+        // table takes a cycle a lane, which bounded the kernel when every thread looked up all it needs.)
         u32 lo[CODE_ITEMS + AHEAD], width[CODE_ITEMS + AHEAD];
-#pragma unroll
-        for (int k = 0; k < CODE_ITEMS + (int)AHEAD; ++k) {
-            const u32 s = s16[k];
+        auto look_up = [&](int k) {
             u32 pair[2];
-            __builtin_memcpy(pair, cum + s, 8); // entries s and s + 1 (4-byte aligned)
+            __builtin_memcpy(pair, cum + s16[k], 8); // entries s and s + 1 (4-byte aligned)
             lo[k] = pair[0];
             width[k] = pair[1] - pair[0];
+        };
+#pragma unroll
+        for (int k = 0; k < CODE_ITEMS; ++k)
+            look_up(k);
+#pragma unroll
+        for (int k = CODE_ITEMS; k < CODE_ITEMS + (int)AHEAD; ++k) {
+            lo[k] = __shfl_down(lo[k - CODE_ITEMS], 1);
+            width[k] = __shfl_down(width[k - CODE_ITEMS], 1);
+        }
+        if ((t & 63u) == 63u) {
+#pragma unroll
+            for (int k = CODE_ITEMS; k < CODE_ITEMS + (int)AHEAD; ++k)
+                look_up(k);
         }
         u32 code[CODE_ITEMS], more[CODE_ITEMS], owners = 0;
 #pragma unroll
