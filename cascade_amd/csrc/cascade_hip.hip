@@ -1843,6 +1843,12 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
     return CSA_OK;
 }
 
+// Texts of this length on are looked at before their bytes are counted (text_byte_hist_kernel): a look takes 4 us, and so does counting half as many.
+#ifndef CSA_BYTE_LOOK_MIN
+#define CSA_BYTE_LOOK_MIN 1000000u
+#endif
+constexpr u32 BYTE_LOOK_MIN = CSA_BYTE_LOOK_MIN;
+
 // Texts of up to this many symbols are ranked by counting (short_text.hpp).
 #ifndef CSA_SHORT_TEXT
 #define CSA_SHORT_TEXT SHORT_MAX
@@ -1962,12 +1968,16 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     count_blocks = count_blocks < 256u ? count_blocks : 256u;
     if (hist_blocks(256 * 8 * 16, n) > count_blocks)
         count_blocks = hist_blocks(256 * 8 * 16, n);
-    auto count_bytes = [&] {
-        hipLaunchKernelGGL(text_byte_hist_kernel, dim3(count_blocks), dim3(256), 0, s, d_text, n, bytehist);
+    auto count_bytes = [&](bool look) {
+        if (look)
+            hipLaunchKernelGGL(text_byte_hist_kernel<true>, dim3(count_blocks), dim3(256), 0, s, d_text, n, bytehist);
+        else
+            hipLaunchKernelGGL(text_byte_hist_kernel<false>, dim3(count_blocks), dim3(256), 0, s, d_text, n, bytehist);
     };
+    bool bytes_counted = false;
     ProbeCounts* const seen = reinterpret_cast<ProbeCounts*>(h->h_pinned + PINNED_HIST + 2 * RADIX_BINS); // (behind the byte counts)
     if (h->pack_symbols) {
-        count_bytes();
+        count_bytes(n >= BYTE_LOOK_MIN);
         u32* h_bytes = h->h_pinned + PINNED_HIST;
         if ((rc = move_table(h_bytes, bytehist, 2 * RADIX_BINS * sizeof(u32), s)) != CSA_OK)
             return rc;
@@ -1978,6 +1988,10 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             return rc;
         HIP_TRY(hipEventSynchronize(h->ev_gen[2]));
         pp = plan_packed_text(h_bytes, n, h->key_words, (u64)h->cap * sizeof(u32));
+        u64 counted_symbols = 0;
+        for (u32 d = 0; d < RADIX_BINS; ++d)
+            counted_symbols += h_bytes[d];
+        bytes_counted = counted_symbols == n;
     }
     TextSource ps;
     memset(&ps, 0, sizeof(ps));
@@ -2049,8 +2063,11 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         rc = sort_by_codes(L, d_text, n, tail, h->pack_symbols ? 0u : 1u, list, counted, digits, &p1);
         in_out = 1; // idx[1] holds the list, key[0] and key[1] what the sort has left behind
     } else {
-        if (!h->pack_symbols)
-            count_bytes();
+        if (!bytes_counted) {
+            if (h->pack_symbols && (rc = move_table(bytehist, nullptr, 2 * RADIX_BINS * sizeof(u32), s)) != CSA_OK)
+                return rc;
+            count_bytes(false);
+        }
         ps.text = d_text;
         ps.byte_wide = pp.byte_wide || !h->pack_symbols;
         hipLaunchKernelGGL(text_hist_expand_kernel, dim3(1), dim3(256), 0, s, d_text, n, (const u32*)bytehist, h->ghist);
