@@ -14,6 +14,7 @@
 #include "pipeline_steps.hpp"
 #include "radix_sort.hpp"
 #include "short_text.hpp"
+#include "word_keys.hpp"
 
 #include <cmath>
 #include <cstdarg>
@@ -961,6 +962,7 @@ struct PackedPlan {
     bool few;       // few_symbols
     SymbolCodes codes;
     u32 skipped; // j
+    u32 values;  // codes, 256 at most; 0: too many
 };
 
 PackedPlan plan_packed_text(const u32* bytehist, u32 n, int key_words, u64 room_bytes)
@@ -979,6 +981,8 @@ PackedPlan plan_packed_text(const u32* bytehist, u32 n, int key_words, u64 room_
     pp.few = few_symbols(nlo, nhi);
     if (codes > 256)
         return pp;
+    pp.values = codes;
+    pp.codes.nlo = nlo;
     const u32 b = codes <= 2 ? 1u : codes <= 4 ? 2u : codes <= 16 ? 4u : 8u;
     u32 S = 4u * (u32)key_words;
     if (S * b > 64)
@@ -991,7 +995,6 @@ PackedPlan plan_packed_text(const u32* bytehist, u32 n, int key_words, u64 room_
     const u64 words = ((u64)n * b + 31) / 32 + 4;
     if (words * 4 > room_bytes)
         return pp;
-    pp.codes.nlo = nlo;
     pp.codes.bits = b;
     pp.codes.key_syms = S;
     pp.skipped = j;
@@ -1253,6 +1256,7 @@ struct CodedList {
     u64 long_members; // suffixes in runs that were too long for their tile, sorted by their second word in ...
     int long_passes;  // ... so many radix passes
     bool long_left;   // there are runs that are too long for a tile on both words
+    bool by_levels;   // the ties are those of sort_by_words: `words` of its levels, and nothing else to be done
 };
 
 // The list of open runs: where the passes of a sort by codes in buckets had their pairs, and in an array that is not used before its long runs are.
@@ -1573,6 +1577,8 @@ struct Settle {
     const u16* text;
     u32* sa32;      // the sorted list, whose groups are put in order
     u32 ctx, wide_ell; // symbols the groups are tied on; of the caller's key
+    u64 next;          // 0, or the doubling's first context past ctx, where it has none of ctx
+    bool words;        // the list is tied on words of written text
     bool settled;   // the list is in order, and the doubling would have gone through num generations more, of these sizes
     u32 num;
     u64 active[SETTLE_CONTEXTS], groups[SETTLE_CONTEXTS];
@@ -1609,6 +1615,7 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     a.gprim = ra.gprim_out;
     a.m = m;
     a.groups = groups;
+    a.most = st.words ? SETTLE_MAX_WORDS : SETTLE_MAX;
     a.words[0] = (a.anchors + 63u) / 64u;
     a.words[1] = (a.words[0] + 63u) / 64u;
     a.words[2] = (a.words[1] + 63u) / 64u;
@@ -1625,9 +1632,9 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     if (at > end)
         return CSA_OK; // (a handle of a few hundred suffixes)
     a.sa32 = st.sa32;
-    u64 c = st.ctx;
+    u64 c = st.next ? st.next : st.ctx;
     do {
-        a.contexts[a.num_contexts++] = (u32)c;
+        a.contexts[a.num_contexts++] = (u32)(c < a.n ? c : a.n); // (nobody is tied on that many)
         c += c < st.wide_ell ? (c < st.wide_ell - c ? c : st.wide_ell - c) : c;
     } while (c < a.n && a.num_contexts < SETTLE_CONTEXTS);
     constexpr u32 TALLIES = 2 * (SETTLE_CONTEXTS + 1);
@@ -1646,7 +1653,11 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     hipLaunchKernelGGL(copy_links_kernel, dim3(a.words[1]), dim3(1024), 0, s, a);
     hipLaunchKernelGGL(copy_links_top_kernel, dim3((a.words[1] + 255u) / 256u), dim3(256), 0, s, a);
     hipLaunchKernelGGL(copy_spread_kernel, dim3((u32)(((u64)a.anchors + 255) / 256)), dim3(256), 0, s, a);
-    hipLaunchKernelGGL((settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX>), dim3((u32)(((u64)m + SETTLE_TILE - 1) / SETTLE_TILE)), dim3(SETTLE_BLOCK), 0, s, a);
+    const dim3 settle_grid((u32)(((u64)m + SETTLE_TILE - 1) / SETTLE_TILE));
+    if (st.words)
+        hipLaunchKernelGGL((settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX_WORDS>), settle_grid, dim3(SETTLE_BLOCK), 0, s, a);
+    else
+        hipLaunchKernelGGL((settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX>), settle_grid, dim3(SETTLE_BLOCK), 0, s, a);
     HIP_TRY(hipGetLastError());
     u32* const h_tallies = h->h_pinned + PINNED_HIST;
     add_table(seen, h_tallies, a.tallies, SETTLE_SLOTS * TALLIES * sizeof(u32));
@@ -1773,7 +1784,10 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
             ra.words_known = coded->told ? nullptr : coded->args.words_out;
             // (several tiles a wave on long lists: fewer additions to the level totals)
             const u32 per_wave = r.tiles >= (1u << 15) ? 8u : 1u, waves = (r.tiles + per_wave - 1) / per_wave;
-            hipLaunchKernelGGL((count_ties_kernel<RANK_TILE>), dim3((waves + 3) / 4), dim3(256), 0, s, ra, r.tiles, per_wave);
+            if (coded->by_levels)
+                hipLaunchKernelGGL((count_ties_kernel<RANK_TILE, WORD_LEVELS>), dim3((waves + 3) / 4), dim3(256), 0, s, ra, r.tiles, per_wave);
+            else
+                hipLaunchKernelGGL((count_ties_kernel<RANK_TILE>), dim3((waves + 3) / 4), dim3(256), 0, s, ra, r.tiles, per_wave);
             if (ra.levels > 0)
                 hipLaunchKernelGGL(count_code_levels_kernel, dim3(hist_blocks(256 * 16, ra.m)), dim3(256), 0, s, ra, coded->args.codes, ra.levels);
         } else {
@@ -1786,7 +1800,7 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
     int rc = count_and_read();
     if (rc)
         return rc;
-    if (coded) {
+    if (coded && !coded->by_levels) {
         coded->words = ra.words = h->h_pinned[6];
         coded->told = true;
         const bool unordered = h->h_pinned[4] != 0, second = h->h_pinned[5] != 0 && coded->words == 2;
@@ -1841,6 +1855,166 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
     if (*rank_update == 1)
         return deferred_rank_update(L, buf, ra.n);
     return CSA_OK;
+}
+
+// Written text (word_keys.hpp): texts of at least this many symbols over 17 to 128 values (a symbol of eight bits gains nothing in the first word). Below,
+// its round trips and launches cost as much as they save: 40000 letters of written text take 361 us by the doubling and 364 this way, independent ones of an
+// alphabet of 20 217 and 238; 3 * 10^5 of written text 681 and 416. Texts whose runs of equal first words are long (choose_seconds_kernel) lose the launches that
+// tell: 10^6 symbols of log lines 1203 us and 1210, 3 * 10^7 with long runs of spaces 6.20 ms and 6.30.
+#ifndef CSA_WORD_KEYS_MIN
+#define CSA_WORD_KEYS_MIN (1u << 18)
+#endif
+static_assert(CSA_WORD_KEYS_MIN * sizeof(u64) >= sizeof(u32) << WINDOW_BITS<7>, "the windows are counted in a list of keys");
+
+// What sort_by_words leaves.
+struct WordList {
+    WordLevels levels;      // contexts that the list has been counted on: the doubling's, and the two words
+    u32 survivors[WORD_LEVELS], groups[WORD_LEVELS]; // on each
+    u32 valid;              // levels on which the order and the ties are those of the suffixes
+    u32 members, runs;      // of long runs, sorted by the second word in ...
+    int passes;             // ... so many radix passes
+};
+
+// The sorted first words of a text (syms symbols of ps.sym_bits bits each), resolved on the second ones: keys and sufs -> sufs_out, and the ties. `spare` holds the
+// keys, which are not needed once the tiles are resolved. Works in key[2], idx[2..4] and spare.
+int sort_by_words(Launch& L, u32 n, const TextSource& ps, u32 syms, u64* spare, const u32* sufs, u32* sufs_out, u8* ties, RerankArgs& ra, WordList& list)
+{
+    csa_handle* h = L.h;
+    hipStream_t s = L.stream;
+    WordArgs a;
+    memset(&a, 0, sizeof(a));
+    a.keys = spare;
+    a.sufs = sufs;
+    a.n = n;
+    a.stream = ps.stream;
+    a.bits = ps.sym_bits;
+    a.syms = syms;
+    a.levels = list.levels;
+    a.sufs_out = sufs_out;
+    a.ties = ties;
+    a.at_end = h->counts + 4;
+    a.any_long = h->counts + 5;
+    TableGroup cleared = {};
+    add_table(cleared, h->counts + 4, nullptr, 2 * sizeof(u32));
+    int rc = move_tables(cleared, s);
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(resolve_words_kernel, dim3((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, a);
+    HIP_TRY(hipGetLastError());
+    ra.ties = ties;
+    ra.sufs = sufs_out;
+    ra.words = list.levels.count;
+    ra.words_known = nullptr;
+    ra.first_level = 0;
+    ra.levels = 0;
+    const RankTables r = rank_tables<RANK_TILE>(h, n);
+    unsigned long long* const h_levels = reinterpret_cast<unsigned long long*>(h->h_pinned + PINNED_HIST + 512);
+    auto count_and_read = [&]() -> int {
+        ra.tile_agg = r.tile_agg;
+        ra.tile_prefix = r.tile_prefix;
+        ra.tile_splits = r.tile_splits;
+        ra.slab_total = r.slab_total;
+        ra.slab = r.slab;
+        ra.level_totals = reinterpret_cast<unsigned long long*>(h->ghist);
+        HIP_TRY(hipMemsetAsync(ra.level_totals, 0, LEVEL_SLOTS * 8 * sizeof(unsigned long long), s));
+        const u32 per_wave = r.tiles >= (1u << 15) ? 8u : 1u, waves = (r.tiles + per_wave - 1) / per_wave;
+        hipLaunchKernelGGL((count_ties_kernel<RANK_TILE, WORD_LEVELS>), dim3((waves + 3) / 4), dim3(256), 0, s, ra, r.tiles, per_wave);
+        TableGroup beside = {};
+        add_table(beside, h_levels, ra.level_totals, LEVEL_SLOTS * 8 * sizeof(unsigned long long));
+        u32 survivors = 0, groups = 0;
+        int update = 0;
+        const int read = rank_totals(L, r, true, n, n, false, &survivors, &groups, &update, beside);
+        for (u32 i = 0; i < list.levels.count; ++i) {
+            u64 sv = 0, hd = 0;
+            for (u32 slot = 0; slot < LEVEL_SLOTS; ++slot) {
+                sv += h_levels[slot * 8 + 2 * i];
+                hd += h_levels[slot * 8 + 2 * i + 1];
+            }
+            list.survivors[i] = (u32)sv;
+            list.groups[i] = (u32)hd;
+        }
+        return read;
+    };
+    if ((rc = count_and_read()) != CSA_OK)
+        return rc;
+    list.valid = list.levels.count;
+    if (h->h_pinned[5] == 0)
+        return CSA_OK;
+    // The members of long runs: more than a quarter of the text in them are left to the doubling (runs, padding, few words).
+    list.valid = list.levels.in_first;
+    const RankTables cr = rank_tables<COLLECT_TILE>(h, n);
+    a.tile_agg = cr.tile_agg;
+    a.tile_splits = cr.tile_splits;
+    a.tile_prefix = cr.tile_prefix;
+    a.slab_total = cr.slab_total;
+    a.slab = cr.slab;
+    hipLaunchKernelGGL(collect_words_kernel<false>, dim3(cr.tiles), dim3(COLLECT_BLOCK), 0, s, a);
+    hipLaunchKernelGGL(rerank_scan_kernel, dim3(cr.slabs), dim3(1024), 0, s, cr.tile_agg, cr.tile_prefix, cr.tiles, cr.slab, cr.slab_total, cr.tile_splits);
+    HIP_TRY(hipGetLastError());
+    u32* const h_slabs = h->h_pinned + PINNED_HIST;
+    if ((rc = move_table(h_slabs, cr.slab_total, cr.slabs * 5 * sizeof(u32), s)) != CSA_OK)
+        return rc;
+    HIP_TRY(hipStreamSynchronize(s));
+    u64 members = 0, runs = 0;
+    for (u32 sl = 0; sl < cr.slabs; ++sl) {
+        members += h_slabs[sl * 5 + 2];
+        runs += h_slabs[sl * 5 + 3];
+    }
+    if (members > n / 4 || members > h->cap / 2)
+        return count_and_read(); // (the tables of the tiles have been used)
+    list.members = (u32)members;
+    list.runs = (u32)runs;
+    u64* const K[2] = {h->key[2], h->key[2] + h->cap / 2};
+    u32* const V[2] = {h->idx[3], h->idx[4]};
+    a.run_keys = K[0];
+    a.run_slots = V[0];
+    a.words2 = spare;
+    a.members = reinterpret_cast<u32*>(spare + h->cap / 2);
+    a.ordinals = a.members + h->cap / 2;
+    a.places = h->idx[2];
+    hipLaunchKernelGGL(collect_words_kernel<true>, dim3(cr.tiles), dim3(COLLECT_BLOCK), 0, s, a);
+    HIP_TRY(hipGetLastError());
+    int first = 0, second = 0, run = 0;
+    rc = radix_sort(L, SRC_PAIRS, 0, 0, K[0], V[0], K[1], V[1], list.members, make_plan(0, (int)(ps.sym_bits * syms)), &first, &run);
+    if (rc)
+        return rc;
+    list.passes = run;
+    const dim3 member_grid((u32)((members + 255) / 256));
+    hipLaunchKernelGGL(gather_ordinals_kernel, member_grid, dim3(256), 0, s, (const u32*)a.ordinals, (const u32*)V[first], list.members, K[first]);
+    rc = radix_sort(L, SRC_PAIRS, 0, 0, K[first], V[first], K[first ^ 1], V[first ^ 1], list.members, make_plan(0, bit_length(runs - 1 ? runs - 1 : 1)), &second, &run);
+    if (rc)
+        return rc;
+    list.passes += run;
+    a.run_slots = V[first ^ second];
+    hipLaunchKernelGGL(place_words_kernel, member_grid, dim3(256), 0, s, a, list.members);
+    HIP_TRY(hipGetLastError());
+    if ((rc = count_and_read()) != CSA_OK)
+        return rc;
+    if (h->h_pinned[4] == 0)
+        list.valid = list.levels.count;
+    return CSA_OK;
+}
+
+// The contexts of a list that is resolved on two words of syms symbols: the doubling's from the caller's key on, the last of those before it that the first
+// word holds, from which the doubling may go on, and the two words themselves.
+WordLevels word_levels(u32 syms, u32 bits, u64 wide_ell)
+{
+    WordLevels l;
+    memset(&l, 0, sizeof(l));
+    auto next = [&](u64 c) { return c + (c < wide_ell ? (c < wide_ell - c ? c : wide_ell - c) : c); };
+    auto add = [&](u64 c) {
+        if (l.count < WORD_LEVELS) {
+            l.in_first += c <= syms ? 1u : 0u;
+            l.context[l.count] = (u32)c;
+            l.drop[l.count++] = (u32)(c <= syms ? syms - c : 2 * syms - c) * bits;
+        }
+    };
+    for (u64 c = 4; c <= 2 * syms; c = next(c))
+        if (c >= wide_ell || (c <= syms && next(c) > syms))
+            add(c);
+    if (l.context[l.count - 1] != 2 * syms)
+        add(2 * syms);
+    return l;
 }
 
 // Texts of this length on are looked at before their bytes are counted (text_byte_hist_kernel): a look takes 4 us, and so does counting half as many.
@@ -1956,6 +2130,9 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     TableGroup zeros = {};
     add_table(zeros, h->counts, nullptr, 13 * sizeof(u32));
     add_table(zeros, h->ghist, nullptr, (MAX_PASSES + 2) * RADIX_BINS * sizeof(u32));
+    u32* const windows = reinterpret_cast<u32*>(h->key[1]); // for written text; the first pass of the sort writes it, afterwards
+    if (n >= CSA_WORD_KEYS_MIN)
+        add_table(zeros, windows, nullptr, sizeof(u32) << WINDOW_BITS<7>);
     int rc = move_tables(zeros, s);
     if (rc)
         return rc;
@@ -1995,6 +2172,11 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     }
     TextSource ps;
     memset(&ps, 0, sizeof(ps));
+    const bool by_words = pp.values > 16 && pp.values <= 128 && n >= CSA_WORD_KEYS_MIN && h->pack_symbols && h->settle && !h->expect_presorted;
+    const u32 word_bits = by_words ? (u32)bit_length(pp.values - 1) : 0u, word_syms = by_words ? 64u / word_bits : 0u;
+    const PackedPlan as_reported = pp; // what callers are told of the first sort of such texts
+    if (by_words)
+        pp.enabled = false;
     bool narrow = false; // keys of half as many packed symbols
     const bool in_buckets = n >= CSA_BUCKETS_MIN && h->pack_symbols;
     CodeDigits digits = ALL_DIGITS, counted = ALL_DIGITS;
@@ -2014,12 +2196,13 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         if (n >= CSA_NARROW_MIN && ps.sym_bits == 2 && ps.key_bits == 64 && pp.skipped > 0 && (rc = narrow_keys_pay(L, ps, n, &narrow, &digits)) != CSA_OK)
             return rc;
     }
-    const u32 ell = pp.enabled ? (narrow ? pp.codes.key_syms / 2 : pp.codes.key_syms) : 4u; // symbols of a key of the first sort
+    // symbols of a key of the first sort, or that its list will be taken to be resolved on
+    u32 ell = pp.enabled ? (narrow ? pp.codes.key_syms / 2 : pp.codes.key_syms) : 4u;
     int folded = 0; // generations after the first that still belong to the reported generation 0
     for (u64 c = ell; c < wide_ell; c += (c < wide_ell - c ? c : wide_ell - c))
         ++folded;
-    const u32 tail = n < ell ? n : ell;
-    bool coded = !pp.enabled && !pp.byte_wide;
+    const u32 tail = by_words ? (n < word_syms ? n : word_syms) : n < ell ? n : ell;
+    bool coded = !pp.enabled && !pp.byte_wide && !by_words;
     if (coded) {
         const bool probed = n >= PROBE_MIN, ahead = !probed || n < CODE_AHEAD_MAX;
         if (!h->pack_symbols || pp.few) { // (few symbols, and no packed keys for them)
@@ -2042,7 +2225,22 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     u32* V[2] = {h->idx[0], h->idx[1]};
     int cur = 0; // the (K, V) set that holds the sorted pairs
     CodedList list;
-    if (pp.enabled) {
+    if (by_words) {
+        SymbolCodes codes = pp.codes;
+        codes.bits = word_bits;
+        codes.key_syms = word_syms;
+        ps.stream = h->rank;
+        ps.sym_bits = word_bits;
+        ps.key_bits = word_bits * word_syms;
+        ps.words = ((u64)n * word_bits + 31) / 32 + 4;
+        hipLaunchKernelGGL(encode_words_kernel, dim3((u32)((ps.words + WORD_SPAN - 1) / WORD_SPAN)), dim3(WORD_BLOCK), 0, s, d_text, n, codes, h->rank, ps.words);
+        const u32 blocks = hist_blocks(WINDOW_BLOCK * 4, n);
+        auto* const count = word_bits == 5 ? window_hist_kernel<5> : word_bits == 6 ? window_hist_kernel<6> : window_hist_kernel<7>;
+        hipLaunchKernelGGL(count, dim3(blocks < WINDOW_HIST_BLOCKS ? blocks : WINDOW_HIST_BLOCKS), dim3(WINDOW_BLOCK), 0, s, (const u32*)h->rank, n, windows);
+        hipLaunchKernelGGL(word_digits_kernel, dim3((ps.key_bits + 7) / 8), dim3(WINDOW_BLOCK), 0, s, (const u32*)h->rank, (const u32*)windows, n, word_bits, ps.key_bits, h->ghist);
+        HIP_TRY(hipGetLastError());
+        rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, make_plan(0, (int)ps.key_bits), &in_out, &p1, nullptr, 0, 0, &ps);
+    } else if (pp.enabled) {
         const PassPlan plan = make_plan(0, narrow ? 32 : (int)ps.key_bits);
         hipLaunchKernelGGL(packed_hist_expand_kernel, dim3(1), dim3(256), 0, s, ps.stream, n, ps.sym_bits, ell, plan.num_passes, bytehist,
                            h->ghist);
@@ -2125,8 +2323,157 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     settle.sa32 = sa32;
     settle.ctx = ell;
     settle.wide_ell = (u32)wide_ell;
-    rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], level_counts, coded ? &list : nullptr, &passes,
-                     h->pack_symbols && h->settle ? &settle : nullptr);
+    WordList words;
+    memset(&words, 0, sizeof(words));
+    u32 by_words_settled = 0; // generations of the reference that such a sort has left nothing of, and one
+    if (by_words) {
+        words.levels = word_levels(word_syms, word_bits, wide_ell);
+        const WordLevels& lv = words.levels;
+        const u32 all = lv.count - 1;
+        auto next = [&](u64 c) { return c + (c < wide_ell ? (c < wide_ell - c ? c : wide_ell - c) : c); };
+        auto settle_at = [&](u64 context, u32 tied, u32 in_groups) -> int {
+            settle.ctx = (u32)context;
+            settle.words = true;
+            settle.next = 4;
+            while (settle.next <= context)
+                settle.next = next(settle.next);
+            return settle_copies(L, settle, ra, tied, in_groups);
+        };
+        // A list with few ties on the first word has them counted and settled as they are: nothing is read from the text.
+        const RankTables r = rank_tables<RANK_TILE>(h, n);
+        RerankArgs firsts = ra;
+        firsts.ell = word_syms;
+        firsts.levels = firsts.first_level = 0;
+        for (u32 i = 0; i < lv.in_first; ++i) {
+            firsts.level_ell[firsts.levels] = lv.context[i];
+            firsts.level_drop[firsts.levels++] = lv.drop[i];
+        }
+        firsts.tile_agg = r.tile_agg;
+        firsts.tile_prefix = r.tile_prefix;
+        firsts.tile_splits = r.tile_splits;
+        firsts.slab_total = r.slab_total;
+        firsts.slab = r.slab;
+        firsts.err = h->counts + 2;
+        firsts.level_totals = reinterpret_cast<unsigned long long*>(h->ghist);
+        unsigned long long* const h_levels = reinterpret_cast<unsigned long long*>(h->h_pinned + PINNED_HIST + 512);
+        HIP_TRY(hipMemsetAsync(firsts.level_totals, 0, LEVEL_SLOTS * 8 * sizeof(unsigned long long), s));
+        hipLaunchKernelGGL(choose_seconds_kernel, dim3(1), dim3(WORD_PLACES), 0, s, (const u64*)k_sorted, n, h->counts + 6);
+        firsts.skip = h->counts + 6;
+        hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, firsts);
+        TableGroup beside = {};
+        add_table(beside, h_levels, firsts.level_totals, LEVEL_SLOTS * 8 * sizeof(unsigned long long));
+        u32 tied = 0, in_groups = 0;
+        int update = 0;
+        if ((rc = rank_totals(L, r, true, n, n, false, &tied, &in_groups, &update, beside)) != CSA_OK)
+            return rc;
+        const bool skip = h->h_pinned[6] != 0; // (nothing has been counted then)
+        u32 known = lv.in_first; // levels whose lists are known
+        for (u32 i = 0; i < known; ++i) {
+            u64 sv = 0, hd = 0;
+            for (u32 slot = 0; slot < LEVEL_SLOTS; ++slot) {
+                sv += h_levels[slot * 8 + 2 * i];
+                hd += h_levels[slot * 8 + 2 * i + 1];
+            }
+            words.survivors[i] = (u32)sv;
+            words.groups[i] = (u32)hd;
+        }
+        firsts.skip = nullptr;
+        if (!skip && tied > 0 && tied < n / 8 && (u64)tied <= (u64)in_groups * SETTLE_AVG_LIMIT) {
+            firsts.rank = nullptr;
+            hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS, false>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, firsts);
+            HIP_TRY(hipGetLastError());
+            if ((rc = settle_at(word_syms, tied, in_groups)) != CSA_OK)
+                return rc;
+        }
+        const bool seconds = !skip && tied > 0 && !settle.settled;
+        bool whole = false;
+        if (seconds) {
+            u8* const ties = reinterpret_cast<u8*>(K[cur ^ 1]);
+            if ((rc = sort_by_words(L, n, ps, word_syms, k_sorted, sa32, ax, ties, ra, words)) != CSA_OK)
+                return rc;
+            std::swap(sa32, ax);
+            std::swap(k_sorted, key_out);
+            bkey[1] = k_sorted;
+            settle.sa32 = sa32;
+            ra.keys = k_sorted;
+            ra.sufs_out = ax;
+            passes += words.passes;
+            whole = words.valid == lv.count;
+            known = lv.count;
+            tied = words.survivors[all];
+            in_groups = words.groups[all];
+            if (whole && tied > 0 && (u64)tied <= (u64)in_groups * SETTLE_AVG_LIMIT) {
+                RerankArgs active = ra;
+                active.rank = nullptr;
+                hipLaunchKernelGGL((compact_ties_kernel<RANK_TILE>), dim3((r.tiles + 3) / 4), dim3(256), 0, s, active, r.tiles);
+                HIP_TRY(hipGetLastError());
+                if ((rc = settle_at(lv.context[all], tied, in_groups)) != CSA_OK)
+                    return rc;
+            }
+        }
+        if (!skip && (settle.settled || (tied == 0 && (whole || known == lv.in_first)))) {
+            // the lists of all generations are known: those of the contexts inside the words, and those that were settled
+            u32 gens = 1;
+            auto report = [&](u64 active, u64 groups_of) {
+                if (active == 0 || gens >= (u32)CSA_MAX_GENERATIONS)
+                    return;
+                st->active[gens] = active;
+                st->groups[gens++] = groups_of;
+            };
+            for (u32 i = 0; i < known; ++i) {
+                u64 c = 4;
+                while (c < lv.context[i])
+                    c = next(c);
+                if (c == lv.context[i] && c >= wide_ell)
+                    report(words.survivors[i], words.groups[i]);
+            }
+            for (u32 i = 0; settle.settled && i < settle.num; ++i)
+                report(settle.active[i], settle.groups[i]);
+            by_words_settled = gens;
+        } else {
+            // the doubling goes on from the last of its contexts that the list is resolved on, by the ties or by the first words
+            u32 at = whole ? lv.count : lv.in_first;
+            u64 c = 4;
+            for (; at > 0; --at) {
+                for (c = 4; c < lv.context[at - 1]; c = next(c)) {}
+                if (c == lv.context[at - 1])
+                    break;
+            }
+            if (at == 0)
+                return fail(CSA_ERR_INTERNAL, "a list of words has no context of the doubling");
+            ell = (u32)c;
+            if (seconds) {
+                memset(&list, 0, sizeof(list));
+                list.words = at;
+                list.told = list.by_levels = true;
+                ra.words = at;
+                coded = true;
+            } else {
+                ra.ell = ell;
+                ra.drop = lv.drop[at - 1];
+                ra.levels = ra.first_level = 0;
+                for (u32 i = 0; i + 1 < at; ++i) // (counted with it)
+                    if (lv.context[i] >= wide_ell) {
+                        ra.level_ell[ra.levels] = lv.context[i];
+                        ra.level_drop[ra.levels++] = lv.drop[i];
+                    }
+            }
+            folded = 0;
+            for (u64 f = ell; f < wide_ell; f = next(f))
+                ++folded;
+            pp.skipped = ra.levels;
+            for (u32 i = 0; i + 1 < at && seconds; ++i)
+                if (lv.context[i] >= wide_ell) {
+                    level_counts[2 * pp.skipped] = words.survivors[i];
+                    level_counts[2 * pp.skipped + 1] = words.groups[i];
+                    ++pp.skipped;
+                }
+            settle.settled = false;
+        }
+    }
+    if (by_words_settled == 0) // (a list by levels has had its shorter contexts counted)
+        rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], by_words && coded ? nullptr : level_counts, coded ? &list : nullptr, &passes,
+                         h->pack_symbols && h->settle && !by_words ? &settle : nullptr);
     range_gen0.close();
     if (rc)
         return rc;
@@ -2137,6 +2484,15 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
 
     // ---- generations t >= 1 (reference loop: src/GPU_SACA.cu:1999-2103) ----
     int gen = 1;
+    if (by_words) { // (its list says how far it goes, whatever the words)
+        coded = false;
+        if (by_words_settled) {
+            gen = (int)by_words_settled;
+            settle.settled = false;
+            pp.skipped = 0;
+            folded = 0;
+        }
+    }
     const u32 resolved = coded ? ell * list.words : ell;                            // symbols the first sort has resolved
     const u32 skipped = narrow ? pp.skipped + list.words - 2u : pp.skipped; // generations after the first that it stands for
     u64 ctx = resolved; // symbols resolved so far; the next generation looks hop symbols ahead
@@ -2532,8 +2888,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     }
     // packed keys: the first sort stands for generations 0 .. skipped of the reference; those after the first are reported
     // with the lists they would have had and no time or passes of their own
-    st->key_symbols = pp.enabled ? resolved : ell;
-    st->first_sort_generations = 1 + (int)skipped;
+    st->key_symbols = by_words ? (as_reported.enabled ? as_reported.codes.key_syms : 4u) : pp.enabled ? resolved : ell;
+    st->first_sort_generations = 1 + (int)(by_words ? as_reported.skipped : skipped);
     if (skipped > 0) {
         const int sk = (int)skipped;
         if (gen + sk > CSA_MAX_GENERATIONS)

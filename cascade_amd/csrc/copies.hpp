@@ -31,8 +31,10 @@ namespace csa {
 constexpr int SETTLE_BLOCK = 512;
 constexpr int SETTLE_ITEMS = 4;
 constexpr int SETTLE_TILE = SETTLE_BLOCK * SETTLE_ITEMS;
-constexpr int SETTLE_MAX = 256; // longest group
-static_assert(SETTLE_MAX <= SETTLE_BLOCK, "the halo is one element per thread");
+constexpr int SETTLE_MAX = 256; // longest group ...
+// ... and of lists that are tied on two words of written text, where one phrase may come a thousand times (5 * 10^7 symbols: 434 times on 24
+// letters, the next longest group has 55 members).
+constexpr int SETTLE_MAX_WORDS = 2048;
 constexpr u32 SETTLE_CONTEXTS = 40;  // contexts of the doubling from here on
 constexpr u32 SETTLE_SLOTS = 16;     // copies of the counters, so that the workgroups' additions do not queue on one address
 // A record: root << 32 | agreement past the anchor << 1 | the member is the larger one; with OPEN the agreement is that long at least.
@@ -63,6 +65,7 @@ struct SettleArgs {
     const u32* gstart;
     const u32* gprim;
     u32 m, groups;
+    u32 most;     // members of a group: SETTLE_MAX or SETTLE_MAX_WORDS
     u64* records; // [anchors + 1], NO_RECORD
     unsigned long long* links[3]; // bits of the anchors, of the words of links[0] that are all ones, of those of links[1]
     u32 words[3];
@@ -227,7 +230,7 @@ __global__ __launch_bounds__(256) void copy_roots_kernel(SettleArgs a)
         return;
     }
     const u32 from = a.gstart[g], to = a.gstart[g + 1];
-    if (to - from > (u32)SETTLE_MAX || to > a.m) {
+    if (to - from > a.most || to > a.m) {
         *a.failed = 1u;
         return;
     }
@@ -320,9 +323,13 @@ __global__ __launch_bounds__(256) void copy_spread_kernel(SettleArgs a)
 template <int BLOCK, int MAXG>
 __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
 {
-    constexpr int TILE = BLOCK * SETTLE_ITEMS, SPAN = TILE + MAXG, ITEMS = SETTLE_ITEMS + 1;
+    constexpr int TILE = BLOCK * SETTLE_ITEMS, SPAN = TILE + MAXG, ITEMS = (SPAN + BLOCK - 1) / BLOCK;
     constexpr u32 TALLIES = 2 * (SETTLE_CONTEXTS + 1), COPIES = 4;
     __shared__ u64 s_key[SPAN];
+    // Of groups that may be long, the four symbols after those in the key: members that are told from their root in the same way are told apart by these as a
+    // rule (one tile with a group of a thousand: 3.1 ms when all such pairs were compared by the text).
+    constexpr bool MORE = MAXG > SETTLE_MAX;
+    __shared__ u64 s_more[MORE ? SPAN : 1];
     __shared__ u32 s_suf[SPAN];
     __shared__ u32 s_tally[TALLIES * COPIES];
     __shared__ u32 s_over;   // a tile before has given up
@@ -338,7 +345,7 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
     u32 x[ITEMS], place[ITEMS];
     int from[ITEMS], to[ITEMS]; // the group, by places of the span; to = 0: nothing to do
     u32 prim[ITEMS];
-    u64 key[ITEMS];
+    u64 key[ITEMS], more[MORE ? ITEMS : 1] = {};
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         const u32 j = k * BLOCK + t;
@@ -384,6 +391,8 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         key[k] = ROOT;
+        if constexpr (MORE)
+            more[k] = 0;
         if (to[k] == 0 || lost[0]) // (a tile that has lost a member writes nothing)
             continue;
         u32 root = x[k];
@@ -397,8 +406,12 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
             const u64 next = (u64)x[k] + w.length;
             const u64 symbol = to[k] - from[k] > 2 && next < a.n ? (u64)a.text[next] + 1u : 0u; // (a pair has nobody else to be told from)
             key[k] = w.larger ? LARGER | ((FAR - w.length) << 17) | symbol : ((u64)w.length << 17) | symbol;
+            if constexpr (MORE)
+                more[k] = symbol && next + 1 < a.n ? load_kgram(a.text, a.n, (u32)next + 1u, 0) : 0u;
         }
         s_key[k * BLOCK + t] = key[k];
+        if constexpr (MORE)
+            s_more[k * BLOCK + t] = more[k];
     }
     __syncthreads();
     if (s_lost[0]) {
@@ -424,9 +437,15 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         u32 before = 0, more_left = SETTLE_STEPS;
         for (int i = from[k]; i < to[k]; ++i) {
             const u64 w = s_key[i];
-            if (w < key[k]) {
+            bool smaller = w < key[k], same = w == key[k];
+            if constexpr (MORE)
+                if (same) {
+                    smaller = s_more[i] < more[k];
+                    same = s_more[i] == more[k];
+                }
+            if (smaller) {
                 ++before;
-            } else if (w == key[k] && i != j) {
+            } else if (same && i != j) {
                 if (lost[1])
                     break;
                 const u32 y = s_suf[i];
@@ -449,6 +468,8 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         if (to[k] != 0) {
             s_suf[place[k]] = x[k];
             s_key[place[k]] = key[k];
+            if constexpr (MORE)
+                s_more[place[k]] = more[k];
         }
     __syncthreads();
     // the thread's places from here on: who stands there now, and on how many contexts it is tied with its neighbours
@@ -457,7 +478,10 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         const u32 y = s_suf[right - 1], z = s_suf[right];
         const u32 of_v = agreement_of(v), of_w = agreement_of(w);
         u32 agree = of_v < of_w ? of_v : of_w;
-        if (v == w) {
+        const u64 differ = MORE && v == w ? s_more[MORE ? right - 1 : 0] ^ s_more[MORE ? right : 0] : 0u;
+        if (differ) {
+            agree = of_w + 1u + (u32)__builtin_clzll(differ) / 16u;
+        } else if (v == w) {
             u32 more_left = SETTLE_STEPS; // (enough: the two have been compared before)
             agree = further(y, z, w, more_left).length;
         }

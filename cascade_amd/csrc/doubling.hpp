@@ -71,7 +71,9 @@ struct RerankArgs {
     const u32* words_known; // count_ties_kernel, non-null: the same, where the host has yet to see it
     u32 m;         // = n: generation 0 ranks every suffix
     u32 n;         // partition size
-    u32 ell;       // symbols in the generation-0 key
+    u32 ell;       // symbols in the generation-0 key, or in its bits above the lowest `drop`, which the list is ranked on then
+    u32 drop;
+    const u32* skip; // null, or where a word other than zero says that the list need not be counted
     // Packed keys of many symbols (packed_text.hpp): the counting pass also counts what the list would leave at shorter
     // contexts. Level i looks at the key bits above level_drop[i] and sets apart the suffixes that run off the text inside
     // level_ell[i] symbols; its survivors and groups are added to level_totals[slot * 8 + 2 i] and [.. + 1], slot = tile
@@ -150,7 +152,7 @@ __device__ __forceinline__ void load_with_neighbours(const u64* __restrict__ key
 __device__ __forceinline__ bool same_run(const RerankArgs& a, u64 key_b, u32 suf_b, u64 key_c, u32 suf_c)
 {
     // a suffix that runs off the text inside its key ties with nobody (include/bit-layout.hpp:99-100)
-    return key_b == key_c && (u64)suf_b + a.ell < a.n && (u64)suf_c + a.ell < a.n;
+    return ((key_b ^ key_c) >> a.drop) == 0 && (u64)suf_b + a.ell < a.n && (u64)suf_c + a.ell < a.n;
 }
 
 // The counting pass of generation 0 on its own: the per-tile aggregates need no ordering inside the tile, so every
@@ -168,6 +170,13 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
     const u32 tile = blockIdx.x;
     const u64 base = (u64)tile * TILE + (u64)t * ITEMS;
     const u32 m = a.m;
+    if (a.skip && *a.skip) {
+        if (t < 4)
+            a.tile_agg[(u64)tile * 4 + t] = 0;
+        if (t == 0)
+            a.tile_splits[tile] = 0;
+        return;
+    }
     u64 key[ITEMS + 2] = {}; // elements base - 1 .. base + ITEMS
     u32 suf[ITEMS + 2];
     load_with_neighbours<ITEMS, true>(a.keys, a.sufs, base, m, key, suf);
@@ -253,17 +262,18 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
 
 // The ties of a tile of a list that carries them, for the wave that takes it: PER entries a lane. tie[i], bit k: element base + k shares
 // more than i words with its left neighbour; right[i], bit k: its right neighbour does with it; valid: the entries there are.
-template <int TILE>
+// MOST: numbers of words that are looked at, from `from` + 1 on.
+template <int TILE, u32 MOST = TIE_MOST_WORDS>
 struct TileTies {
     static constexpr int PER = TILE / WAVE;
     static_assert(PER % 16 == 0 && PER <= 32, "a lane's bytes come in 16-byte loads, their ties fit a word");
-    u32 tie[TIE_MOST_WORDS], right[TIE_MOST_WORDS], valid;
-    __device__ __forceinline__ TileTies(const u8* __restrict__ ties, u32 m, u64 tile)
+    u32 tie[MOST], right[MOST], valid;
+    __device__ __forceinline__ TileTies(const u8* __restrict__ ties, u32 m, u64 tile, u32 from = 0)
     {
         const u32 lane = threadIdx.x & 63u;
         const u64 base = tile * TILE + (u64)lane * PER, behind = (tile + 1) * TILE;
 #pragma unroll
-        for (u32 i = 0; i < TIE_MOST_WORDS; ++i)
+        for (u32 i = 0; i < MOST; ++i)
             tie[i] = 0;
         if (base + PER <= m) {
 #pragma unroll
@@ -273,45 +283,45 @@ struct TileTies {
 #pragma unroll
                 for (int k = 0; k < 16; ++k)
 #pragma unroll
-                    for (u32 i = 0; i < TIE_MOST_WORDS; ++i)
-                        tie[i] |= (((word[k / 4] >> (8 * (k % 4))) & TIE_WORDS) > i ? 1u : 0u) << (q + k);
+                    for (u32 i = 0; i < MOST; ++i)
+                        tie[i] |= (((word[k / 4] >> (8 * (k % 4))) & TIE_WORDS) > from + i ? 1u : 0u) << (q + k);
             }
         } else {
             for (int k = 0; k < PER; ++k)
                 if (base + k < m)
-                    for (u32 i = 0; i < TIE_MOST_WORDS; ++i)
-                        tie[i] |= ((ties[base + k] & TIE_WORDS) > i ? 1u : 0u) << k;
+                    for (u32 i = 0; i < MOST; ++i)
+                        tie[i] |= ((ties[base + k] & TIE_WORDS) > from + i ? 1u : 0u) << k;
         }
         const u32 after = behind < m ? ties[behind] & TIE_WORDS : 0u;
         const u32 have = base >= m ? 0u : m - base >= PER ? PER : (u32)(m - base);
         valid = have == 32u ? 0xFFFFFFFFu : (1u << have) - 1u;
 #pragma unroll
-        for (u32 i = 0; i < TIE_MOST_WORDS; ++i) {
+        for (u32 i = 0; i < MOST; ++i) {
             const u64 firsts = __ballot(tie[i] & 1u);
-            const u32 next = lane == 63u ? (after > i ? 1u : 0u) : (u32)(firsts >> (lane + 1)) & 1u;
+            const u32 next = lane == 63u ? (after > from + i ? 1u : 0u) : (u32)(firsts >> (lane + 1)) & 1u;
             right[i] = (tie[i] >> 1) | (next << (PER - 1));
         }
     }
 };
 
-// The same for a list that carries its ties, at every number of words up to TIE_MOST_WORDS at once: one byte read per suffix. A wave takes
+// The same for a list that carries its ties, at every number of words up to MOST at once: one byte read per suffix. A wave takes
 // whole tiles, `per_wave` of them one after the other; the tile aggregates are those at a.words, the
 // survivors and groups at i + 1 words are added to level_totals[.. + 2 i] and [.. + 2 i + 1].
-template <int TILE>
+template <int TILE, u32 MOST = TIE_MOST_WORDS>
 __global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles, u32 per_wave)
 {
     const u32 lane = threadIdx.x & 63u;
     const u32 wave = blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
     const u32 words = a.words_known ? *a.words_known : a.words;
-    u32 sum_surv[TIE_MOST_WORDS] = {}, sum_heads[TIE_MOST_WORDS] = {};
+    u32 sum_surv[MOST] = {}, sum_heads[MOST] = {};
     for (u32 r = 0; r < per_wave; ++r) {
         const u64 tile = (u64)wave * per_wave + r;
         if (tile >= tiles)
             break;
-        const TileTies<TILE> v(a.ties, a.m, tile);
+        const TileTies<TILE, MOST> v(a.ties, a.m, tile);
         const u64 base = tile * TILE + (u64)lane * TileTies<TILE>::PER;
 #pragma unroll
-        for (u32 i = 0; i < TIE_MOST_WORDS; ++i) {
+        for (u32 i = 0; i < MOST; ++i) {
             const u32 surv = (u32)__popc((v.tie[i] | v.right[i]) & v.valid), heads = (u32)__popc(~v.tie[i] & v.right[i] & v.valid);
             sum_surv[i] += surv;
             sum_heads[i] += heads;
@@ -333,7 +343,7 @@ __global__ __launch_bounds__(256) void count_ties_kernel(RerankArgs a, u32 tiles
         }
     }
 #pragma unroll
-    for (u32 i = 0; i < TIE_MOST_WORDS; ++i) {
+    for (u32 i = 0; i < MOST; ++i) {
         const u32 sv = wave_reduce_sum(sum_surv[i]), hd = wave_reduce_sum(sum_heads[i]);
         unsigned long long* const slot = a.level_totals + (u64)(wave % LEVEL_SLOTS) * 8 + 2 * (a.first_level + i);
         if (lane == 0 && sv) {
@@ -353,10 +363,8 @@ __global__ __launch_bounds__(256) void compact_ties_kernel(RerankArgs a, u32 til
     const u64 tile = (u64)blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
     if (tile >= tiles)
         return;
-    const TileTies<TILE> v(a.ties, a.m, tile);
-    const bool two = a.words == 2;
-    const u32 tie = two ? v.tie[1] : v.tie[0], right = two ? v.right[1] : v.right[0];
-    static_assert(TIE_MOST_WORDS == 2, "one word or two");
+    const TileTies<TILE, 1> v(a.ties, a.m, tile, a.words - 1u);
+    const u32 tie = v.tie[0], right = v.right[0];
     u32 surv = (tie | right) & v.valid;
     const u32 heads = ~tie & right & v.valid;
     const u32 mine = (u32)__popc(surv) | ((u32)__popc(heads) << 16); // at most TILE of each in all

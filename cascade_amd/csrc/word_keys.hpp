@@ -1,0 +1,400 @@
+// Texts over 17 to 128 symbols (written text): the first sort on 64 bits of the code stream, and on 64 more where those tie.
+//
+// A symbol takes b = 5 to 7 bits of the stream (packed_text.hpp has codes of a power of two), a word is the L = 64 / b symbols that fit 64 bits: twelve letters.
+// Written text takes about two bits a letter to tell apart, so eight letters leave nine suffixes in ten tied, twelve six in ten and 24 the
+// copies. After the passes over the first words, resolve_words_kernel reads the second word of every suffix that shares its first (a line of the
+// stream), puts runs of up to WORDS_MAX suffixes in order inside its tile and counts, from the words, on how many of the doubling's contexts neighbours
+// tie; longer runs are collected and radix sorted by the second word. What is left are copies as a rule, and settled as such (copies.hpp). The generations that
+// this stands for used to gather a rank for every tied suffix: 10^8 symbols of text 15.4 -> 9.2 to 11.3 ms, with the longest runs of equal words.
+#pragma once
+
+#include "coded_keys.hpp"
+#include "device_utils.hpp"
+#include "doubling.hpp"
+#include "packed_text.hpp"
+
+namespace csa {
+
+constexpr u32 WORD_LEVELS = 4; // contexts that a list is counted on, the two words among them
+
+struct WordLevels {
+    u32 count;
+    u32 in_first;               // of them, those inside the first word
+    u32 context[WORD_LEVELS];   // symbols, rising
+    u32 drop[WORD_LEVELS];      // bits of a word (the first one; the second for contexts past it) behind the context
+};
+
+// ---- the stream, and the digit counts of the passes over its words ----
+
+constexpr int WORD_BLOCK = 256;
+constexpr u32 WORD_SPAN = 256;      // words of a workgroup's stretch
+
+// stream[wd], wd < words: bits 32 wd .. of the codes of all symbols, `bits` each, zero past the text.
+__global__ __launch_bounds__(WORD_BLOCK) void encode_words_kernel(const u16* __restrict__ text, u32 n, SymbolCodes codes, u32* __restrict__ stream, u64 words)
+{
+    constexpr u32 MAX_SYMS = WORD_SPAN * 32 / 5 + 8;
+    __shared__ u64 s_text[(MAX_SYMS + 6) / 4 + 2];
+    __shared__ SymbolCodes s_codes;
+    const u32 t = threadIdx.x, b = codes.bits;
+    for (u32 i = t; i < sizeof(SymbolCodes) / 4; i += WORD_BLOCK)
+        reinterpret_cast<u32*>(&s_codes)[i] = reinterpret_cast<const u32*>(&codes)[i];
+    const u64 w0 = (u64)blockIdx.x * WORD_SPAN, first = w0 * 32 / b;
+    const u32 sym_off = stage_text(text, n, first, WORD_SPAN * 32 / b + 8u, s_text, t, WORD_BLOCK);
+    __syncthreads();
+    const u16* const s16 = reinterpret_cast<const u16*>(s_text) + sym_off;
+    for (u32 i = t; i < WORD_SPAN; i += WORD_BLOCK) {
+        const u64 bit = (w0 + i) * 32, y = bit / b;
+        u32 word = 0, s = (u32)(y - first);
+        int up = 32 + (int)(bit - y * b) - (int)b; // bits of the word behind the symbol (the first one may start before the word)
+        for (; up > -(int)b; up -= (int)b, ++s) {
+            const u32 c = symbol_code(s_codes, s16[s]);
+            word |= up >= 0 ? c << up : c >> -up;
+        }
+        if (w0 + i < words)
+            stream[w0 + i] = word;
+    }
+}
+
+// The digits of a word start inside one of its symbols, `bits` places apart at most: all of them are read off one count of the windows of a symbol and the
+// seven bits behind the next one's first, which every suffix adds to once (eight digits counted one by one took 0.30 ms of 10^8 symbols, bound by LDS
+// atomics; this takes 0.12).
+constexpr int WINDOW_BLOCK = 1024;
+constexpr u32 WINDOW_HIST_BLOCKS = 256;
+
+template <u32 BITS> constexpr u32 WINDOW_BITS = BITS + 7; // of a symbol, a digit of eight bits from any of its places on
+
+// windows[v] += suffixes whose first WINDOW_BITS bits in the stream are v.
+template <u32 BITS>
+__global__ __launch_bounds__(WINDOW_BLOCK) void window_hist_kernel(const u32* __restrict__ stream, u32 n, u32* __restrict__ windows)
+{
+    constexpr u32 BINS = 1u << WINDOW_BITS<BITS>;
+    __shared__ u32 s_hist[BINS];
+    const u32 t = threadIdx.x;
+    for (u32 i = t; i < BINS; i += WINDOW_BLOCK)
+        s_hist[i] = 0;
+    __syncthreads();
+    const u64 stride = (u64)gridDim.x * WINDOW_BLOCK;
+    for (u64 x = (u64)blockIdx.x * WINDOW_BLOCK + t; x < n; x += stride)
+        atomicAdd(&s_hist[(u32)packed_window(stream, x * BITS, WINDOW_BITS<BITS>)], 1u);
+    __syncthreads();
+    for (u32 i = t; i < BINS; i += WINDOW_BLOCK)
+        if (s_hist[i])
+            atomicAdd(&windows[i], s_hist[i]);
+}
+
+// ghist[p][d] = suffixes whose word has digit d at bits 8 p .. of the word (the last digit may be shorter): a workgroup a digit. Digit p is that of the windows
+// k symbols on, so the first k windows are taken out, and k of zeros, past the text, put in.
+__global__ __launch_bounds__(WINDOW_BLOCK) void word_digits_kernel(const u32* __restrict__ stream, const u32* __restrict__ windows, u32 n, u32 bits, u32 word_bits, u32* __restrict__ ghist)
+{
+    __shared__ u32 s_count[RADIX_BINS];
+    const u32 t = threadIdx.x, p = blockIdx.x, size = word_bits - 8 * p < 8 ? word_bits - 8 * p : 8u;
+    const u32 from = word_bits - 8 * p - size, k = from / bits, r = from - k * bits; // the digit starts r bits into symbol k
+    const u32 below = bits + 7 - r - size;                                           // bits of a window behind it
+    if (t < RADIX_BINS)
+        s_count[t] = 0;
+    __syncthreads();
+    // as many threads a digit as there are: each adds up 2^(bits - 3) windows
+    const u32 d = t & ((1u << size) - 1u), first = t >> size, threads = WINDOW_BLOCK >> size;
+    u32 v = 0;
+#pragma unroll 4
+    for (u32 i = 0; i < 1u << (bits - 3); ++i) {
+        const u32 j = first + i * threads; // the window's bits before and behind the digit
+        v += windows[(j >> below << (below + size)) | (d << below) | (j & ((1u << below) - 1u))];
+    }
+    if (v)
+        atomicAdd(&s_count[d], v);
+    if (t < k && t < n) {
+        atomicAdd(&s_count[(u32)packed_window(stream, (u64)t * bits + r, size)], ~0u); // (one less)
+        atomicAdd(&s_count[0], 1u);
+    }
+    __syncthreads();
+    if (t < RADIX_BINS)
+        ghist[p * RADIX_BINS + t] = s_count[t];
+}
+
+// ---- the second words ----
+
+// Texts that the second word does little for: padding, lines that come again and again, few words. Long runs of one first word are sorted again, to find them
+// long and of one second word as well. Looked for at 1024 places of the sorted list: more than 143 in runs of 256 or more, or more than 51 in
+// runs of 2048. (10^8 letters of written text have 10 and 2 % of their suffixes in such, 5 * 10^7 with a fifth in runs of spaces and a
+// period 28 and 22 %: those take 9.3 ms by the doubling and 10.4 when the second words are read first.) Such lists are ranked on the doubling's last
+// context inside the first word.
+constexpr u32 WORD_PLACES = 1024, WORD_LONG = 256, WORD_LONG_FEW = 143, WORD_LONGER = 2048, WORD_LONGER_FEW = 51;
+
+// (Launched before the list is counted, which is then left out: nothing would be done with the counts.)
+__global__ __launch_bounds__(WORD_PLACES) void choose_seconds_kernel(const u64* __restrict__ keys, u32 n, u32* skip)
+{
+    __shared__ u32 s_in[2];
+    const u32 t = threadIdx.x;
+    if (t < 2)
+        s_in[t] = 0;
+    __syncthreads();
+    const u64 in_long = __ballot(in_long_run(keys, n, WORD_LONG, t, WORD_PLACES)), in_longer = __ballot(in_long_run(keys, n, WORD_LONGER, t, WORD_PLACES));
+    if ((t & 63u) == 0) {
+        atomicAdd(&s_in[0], (u32)__popcll(in_long));
+        atomicAdd(&s_in[1], (u32)__popcll(in_longer));
+    }
+    __syncthreads();
+    if (t == 0)
+        *skip = s_in[0] > WORD_LONG_FEW || s_in[1] > WORD_LONGER_FEW ? 1u : 0u;
+}
+
+constexpr int WORDS_MAX = RESOLVE_MAX;
+
+struct WordArgs {
+    const u64* keys; // sorted: the first words
+    const u32* sufs;
+    u32 n; // suffixes, all of which the list holds
+    const u32* stream;
+    u32 bits, syms; // of a symbol; symbols of a word
+    WordLevels levels;
+    u32* sufs_out;
+    u8* ties;      // of every entry, TIE_LONG and on how many of the levels it ties with its left neighbour
+    u32* any_long; // zeroed: set if some run has more than WORDS_MAX members
+    u32* at_end;   // zeroed: set if a member of a long run runs off the text inside its second word, and another has the same padded word: it goes before
+                   // that one and may stand behind it
+    // the members of long runs, in list order
+    u64* run_keys; // second words, and places in the lists below: what is sorted
+    u32* run_slots;
+    u64* words2;
+    u32* members;
+    u32* ordinals; // of their runs
+    u32* places;
+    u32* tile_agg;
+    u32* tile_splits;
+    const u32* tile_prefix;
+    const u32* slab_total;
+    u32 slab;
+};
+
+__device__ __forceinline__ u64 word_after(const WordArgs& a, u32 x)
+{
+    const u64 y = (u64)x + a.syms;
+    return y < a.n ? packed_window(a.stream, y * a.bits, a.bits * a.syms) : 0ull;
+}
+
+// On how many levels two neighbours x and y tie whose first words differ in `diff`, or agree (diff = 0) and whose second words differ in diff2: whoever
+// runs off the text inside a context ties with nobody on it.
+__device__ __forceinline__ u32 levels_of(const WordArgs& a, u64 diff, u64 diff2, u32 x, u32 y)
+{
+    const u64 last = x > y ? x : y;
+    u32 level = 0;
+#pragma unroll
+    for (u32 i = 0; i < WORD_LEVELS; ++i) {
+        const bool inside = i < a.levels.in_first;
+        const u64 left = inside ? diff >> a.levels.drop[i] : diff | (diff2 >> a.levels.drop[i]);
+        level += i < a.levels.count && left == 0 && last + a.levels.context[i] < a.n ? 1u : 0u;
+    }
+    return level;
+}
+
+// The runs of equal first words of one tile and the halo its first and last run reach into (as in resolve_runs_kernel): every member of a run of up to
+// WORDS_MAX suffixes counts those with a smaller second word. Bounded by the lines of the stream.
+__global__ __launch_bounds__(RESOLVE_BLOCK) void resolve_words_kernel(WordArgs a)
+{
+    constexpr int H = WORDS_MAX, SPAN = RESOLVE_TILE + 2 * H;
+    constexpr int ITEMS = RESOLVE_ITEMS + 1; // the last one is the thread's element of the halo
+    __shared__ u64 s_head[SPAN / 64]; // bit j: the element at span place j starts a run (places outside the list count as starts)
+    __shared__ u32 s_ends;            // some member of a run runs off the text inside its words
+    __shared__ u64 s_key[SPAN];       // second words
+    __shared__ u32 s_suf[SPAN];
+    const u32 t = threadIdx.x;
+    if (t == 0)
+        s_ends = 0;
+    const long long t0 = (long long)blockIdx.x * RESOLVE_TILE, lo = t0 - H, m = a.n;
+    for (int j = t; j < SPAN; j += RESOLVE_BLOCK) {
+        const long long e = lo + j;
+        const bool in = e >= 0 && e < m, head = e <= 0 || e >= m || a.keys[e] != a.keys[e - 1];
+        s_suf[j] = in ? a.sufs[e] : 0u;
+        const u64 b = __ballot(head);
+        if ((t & 63u) == 0)
+            s_head[j / 64] = b;
+    }
+    __syncthreads();
+    auto is_head = [&](int j) { return ((s_head[j / 64] >> (j & 63)) & 1ull) != 0; };
+    // the run around place j: first place and first place behind it; false if it has more than H members
+    auto run_of = [&](int j, int& first, int& last) -> bool {
+        int wd = j / 64;
+        u64 b = s_head[wd] & (~0ull >> (63 - (j & 63))); // starts at or before j
+        while (b == 0 && wd > 0 && wd * 64 > j - H)
+            b = s_head[--wd];
+        first = b ? wd * 64 + 63 - __builtin_clzll(b) : -1;
+        if (first < 0 || j - first > H)
+            return false;
+        wd = j / 64;
+        b = (j & 63) == 63 ? 0ull : s_head[wd] & (~0ull << ((j & 63) + 1)); // starts behind j
+        while (b == 0 && wd + 1 < SPAN / 64 && (wd + 1) * 64 <= j + H)
+            b = s_head[++wd];
+        last = b ? wd * 64 + __builtin_ctzll(b) : SPAN + H;
+        return last - first <= H;
+    };
+    u32 x[ITEMS], longs = 0;
+    int first[ITEMS], last[ITEMS]; // last - first = 1: alone, or nothing to do
+    u64 w1[ITEMS];
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        const bool halo = k == RESOLVE_ITEMS;
+        const int j = !halo ? H + k * RESOLVE_BLOCK + (int)t : (int)t < H ? (int)t : RESOLVE_TILE + (int)t;
+        const long long e = lo + j;
+        x[k] = 0;
+        first[k] = j;
+        last[k] = j + 1;
+        w1[k] = 0;
+        if (e < 0 || e >= m || (halo && (int)t >= 2 * H))
+            continue;
+        int f, l;
+        if (!run_of(j, f, l)) {
+            longs |= halo ? 0u : 1u << k;
+            continue;
+        }
+        if (l - f == 1 || (halo && ((int)t < H ? l <= H : f >= H + RESOLVE_TILE)))
+            continue;
+        first[k] = f;
+        last[k] = l;
+        x[k] = s_suf[j];
+        w1[k] = word_after(a, x[k]);
+        if ((u64)x[k] + 2u * a.syms >= a.n)
+            s_ends = 1;
+    }
+    if (longs)
+        *a.any_long = 1u;
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+        if (last[k] - first[k] > 1)
+            s_key[k == RESOLVE_ITEMS ? ((int)t < H ? (int)t : RESOLVE_TILE + (int)t) : H + k * RESOLVE_BLOCK + (int)t] = w1[k];
+    __syncthreads();
+    const bool ends = s_ends != 0;
+    int place[ITEMS];
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        const int f = first[k], l = last[k];
+        const int j = k == RESOLVE_ITEMS ? ((int)t < H ? (int)t : RESOLVE_TILE + (int)t) : H + k * RESOLVE_BLOCK + (int)t;
+        place[k] = j;
+        if (l - f <= 1)
+            continue;
+        int before = 0;
+        if (!ends) {
+            for (int i = f; i < l; ++i)
+                before += s_key[i] < w1[k] || (s_key[i] == w1[k] && i < j) ? 1 : 0;
+        } else {
+            // whoever runs off the text inside the two words comes before those with the same padded words, shortest first
+            const bool off = (u64)x[k] + 2u * a.syms >= a.n;
+            for (int i = f; i < l; ++i) {
+                const u64 v = s_key[i];
+                const u32 y = s_suf[i];
+                const bool y_off = (u64)y + 2u * a.syms >= a.n;
+                const bool y_before = off != y_off ? y_off : off ? y > x[k] : i < j;
+                before += v < w1[k] || (v == w1[k] && y_before) ? 1 : 0;
+            }
+        }
+        place[k] = f + before;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+        if (last[k] - first[k] > 1) {
+            s_suf[place[k]] = x[k];
+            s_key[place[k]] = w1[k];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RESOLVE_ITEMS; ++k) {
+        const int j = H + k * RESOLVE_BLOCK + (int)t;
+        const long long e = lo + j;
+        if (e >= m)
+            continue;
+        const bool is_long = (longs >> k) & 1u;
+        u32 tie = 0;
+        if (e > 0) {
+            const bool head = is_head(j);
+            const u64 diff = head ? a.keys[e] ^ a.keys[e - 1] : 0ull;
+            tie = levels_of(a, diff, head || is_long ? ~0ull : s_key[j] ^ s_key[j - 1], s_suf[j], s_suf[j - 1]);
+        }
+        a.sufs_out[e] = s_suf[j];
+        a.ties[e] = (u8)(tie | (is_long ? TIE_LONG | (is_head(j) ? TIE_HEAD : 0u) : 0u));
+    }
+}
+
+// The members of long runs in list order: APPLY = false counts them and their runs per tile, APPLY = true (after rerank_scan_kernel) lists them.
+template <bool APPLY>
+__global__ __launch_bounds__(COLLECT_BLOCK) void collect_words_kernel(WordArgs a)
+{
+    __shared__ u32 s_w[COLLECT_BLOCK / WAVE][2];
+    const u32 t = threadIdx.x, lane = t & 63u, w = t >> 6, tile = blockIdx.x;
+    const u64 base = (u64)tile * COLLECT_TILE + (u64)t * COLLECT_ITEMS;
+    u32 mine = 0, heads = 0;
+    u8 tie[COLLECT_ITEMS];
+#pragma unroll
+    for (int k = 0; k < COLLECT_ITEMS; ++k) {
+        tie[k] = base + k < a.n ? a.ties[base + k] : (u8)0;
+        mine += (tie[k] & TIE_LONG) ? 1u : 0u;
+        heads += (tie[k] & TIE_HEAD) ? 1u : 0u;
+    }
+    const u32 incl = wave_incl_sum(mine), incl_heads = wave_incl_sum(heads);
+    if (lane == 63u) {
+        s_w[w][0] = incl;
+        s_w[w][1] = incl_heads;
+    }
+    __syncthreads();
+    u32 slot = incl - mine, total = 0, ordinal = incl_heads - heads, total_heads = 0;
+    for (u32 ww = 0; ww < COLLECT_BLOCK / WAVE; ++ww) {
+        if (ww < w) {
+            slot += s_w[ww][0];
+            ordinal += s_w[ww][1];
+        }
+        total += s_w[ww][0];
+        total_heads += s_w[ww][1];
+    }
+    if (!APPLY) {
+        if (t == 0) {
+            *reinterpret_cast<uint4*>(a.tile_agg + (u64)tile * 4) = make_uint4(0u, 0u, total, total_heads);
+            a.tile_splits[tile] = 0;
+        }
+        return;
+    }
+    if (total == 0)
+        return;
+    const SlabPrefix sp = slabs_before(a.slab_total, tile / a.slab);
+    slot += a.tile_prefix[(u64)tile * 4 + 2] + sp.sum2;
+    ordinal += a.tile_prefix[(u64)tile * 4 + 3] + sp.sum3; // runs begun before this thread's entries
+#pragma unroll
+    for (int k = 0; k < COLLECT_ITEMS; ++k)
+        if (tie[k] & TIE_LONG) {
+            ordinal += (tie[k] & TIE_HEAD) ? 1u : 0u;
+            const u32 x = a.sufs_out[base + k];
+            const u64 word = word_after(a, x);
+            a.run_keys[slot] = a.words2[slot] = word;
+            a.run_slots[slot] = slot;
+            a.members[slot] = x;
+            a.ordinals[slot] = ordinal - 1u;
+            a.places[slot] = (u32)(base + k);
+            ++slot;
+        }
+}
+
+__global__ __launch_bounds__(256) void gather_ordinals_kernel(const u32* __restrict__ ordinals, const u32* __restrict__ slots, u32 count, u64* __restrict__ keys)
+{
+    const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
+    if (i < count)
+        keys[i] = ordinals[slots[i]];
+}
+
+// The members of long runs, sorted by run and second word (run_slots), to their places.
+__global__ __launch_bounds__(256) void place_words_kernel(WordArgs a, u32 count)
+{
+    const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count)
+        return;
+    const u32 slot = a.run_slots[i], place = a.places[i], x = a.members[slot];
+    a.sufs_out[place] = x;
+    const u32 before = i > 0 ? a.run_slots[i - 1] : slot;
+    if (i > 0 && a.ordinals[before] == a.ordinals[slot]) { // (the first of a run ties with its left neighbour as before)
+        const u32 y = a.members[before], last = x > y ? x : y;
+        const u64 diff = a.words2[slot] ^ a.words2[before];
+        a.ties[place] = (u8)(TIE_LONG | levels_of(a, 0ull, diff, x, y));
+        if (diff == 0 && (u64)last + a.syms < a.n && (u64)last + 2u * a.syms >= a.n)
+            *a.at_end = 1u;
+    }
+}
+
+} // namespace csa

@@ -994,3 +994,51 @@ def test_lower_digits_are_sorted_in_buckets(n, kind):
         got, active, _ = emu_sort(lib, T, key_words)
         sa, counts = oracle_lib.prefix_doubling(T, key_words)
         assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+
+
+@pytest.mark.parametrize("key_words", [1, 2, 3, 4])
+@pytest.mark.parametrize("kind", ["words", "few", "copies", "run", "period", "zeros", "even", "seven_bits", "end"])
+def test_written_text_is_sorted_by_two_words(kind, key_words):
+    """Texts over 17 to 128 values, of 8192 symbols or more in this build: the first sort takes words of 9 to 12 symbols and reads the next word of those that tie. Lists
+    with few ties, that are settled on the first word, with many, with runs past the in-tile limit, ranked on the first word because of runs and periods, with
+    suffixes that run off the text inside either word, beside zeros that look like their padding. Suffix array and generation sizes are the oracle's."""
+    lib = load_emulation("libcascade_emu_buckets.so")
+    for n in (8192, 11001):
+        rng = np.random.default_rng(n)
+        T = texts.written_text(n, 12 if kind == "few" else 900, n)
+        if kind == "copies":
+            T[n // 2:n // 2 + n // 4] = T[:n // 4]
+            T[n - n // 9:] = T[:n // 9]
+        elif kind == "run":
+            T[n // 3:n // 3 + 400] = 65
+        elif kind == "period":
+            T[n // 3:n // 3 + n // 3] = np.resize(T[:5], n // 3)
+        elif kind in ("even", "seven_bits"):
+            T = rng.integers(1, 21 if kind == "even" else 100, n).astype(np.uint16)
+        elif kind == "zeros":
+            T = rng.integers(0, 30, n).astype(np.uint16)
+            for at in rng.permutation(n // 40 - 1)[:n // 60]:
+                T[40 * at:40 * at + int(rng.integers(3, 36))] = 0
+            T[-17:] = 0
+        elif kind == "end":
+            phrase = np.arange(97, 97 + 20)
+            for at in rng.permutation(n // 32 - 1)[:90]:
+                T[32 * at:32 * at + 20] = phrase
+            T[-18:] = phrase[:18]
+        got, active, _ = emu_sort(lib, T, key_words)
+        sa, counts = oracle_lib.prefix_doubling(T, key_words)
+        assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts, n
+
+
+@pytest.mark.parametrize("values", [17, 32, 33, 64, 65, 128])
+def test_streams_of_five_to_seven_bits(values):
+    """Alphabets at both ends of the widths of a symbol's code."""
+    lib = load_emulation("libcascade_emu_buckets.so")
+    rng = np.random.default_rng(values)
+    alphabet = np.concatenate([[0], np.sort(rng.permutation(255)[:values - 1] + 1)]).astype(np.uint16)
+    T = alphabet[rng.integers(0, values, 9001)]
+    T[1500:2000] = T[300:800]
+    got, active, _ = emu_sort(lib, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    assert emu_sort.key_symbols == 8 and emu_sort.first_sort_generations == 2

@@ -891,3 +891,19 @@ def test_lower_digits_are_sorted_in_buckets(torch_mod, n, letters):
             assert s.verify(d, out)
             seen.append(s.last_stats["active"])
     assert seen[0] == seen[1]
+
+
+@pytest.mark.parametrize("n,words,key_words", [(1 << 18, 900, 1), (300001, 60, 1), (300003, 900, 4), (1 << 20, 5000, 2), ((1 << 22) + 7, 20000, 1)])
+def test_written_text_is_sorted_by_two_words(torch_mod, n, words, key_words):
+    """Words of twelve letters, and the next twelve of the suffixes that tie: written text with copied passages, from the shortest that goes this way on, against the
+    oracle, generation sizes included."""
+    from cascade_amd import PartitionSorter
+    T = texts.written_text(n, words, n)
+    for k in range(1, 6):
+        T[k * n // 6 - 600:k * n // 6] = T[100 * k:100 * k + 600]
+    with PartitionSorter(n, key_words=key_words) as s:
+        print(f"  written text {n} {words} {key_words}", flush=True)
+        got = gpu_sa40(torch_mod, s, T)
+        stats = s.last_stats
+    sa, counts = oracle_lib.prefix_doubling(T, key_words)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts

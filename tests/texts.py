@@ -230,3 +230,12 @@ def text_of_an_undecided_group(copies):
     for _ in range(2):
         parts += [rng.integers(100, 60000, 20).astype(np.uint16), twice]
     return np.concatenate(parts + [rng.integers(100, 60000, 20).astype(np.uint16)])
+
+
+def written_text(n, words, seed, letters=26):
+    """n byte symbols of words of 1 to 9 lower-case letters, the first ones the most frequent, a space between words."""
+    rng = np.random.default_rng(seed)
+    vocabulary = [rng.integers(97, 97 + letters, int(rng.integers(1, 10))).tolist() + [32] for _ in range(words)]
+    ids = np.minimum(rng.zipf(1.3, n), words) - 1  # (a word is two symbols at least)
+    text = [symbol for i in ids[:n // 2 + 1] for symbol in vocabulary[i]]
+    return np.array(text[:n], dtype=np.uint16)
