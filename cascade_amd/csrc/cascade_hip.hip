@@ -1578,7 +1578,8 @@ struct Settle {
     u32* sa32;      // the sorted list, whose groups are put in order
     u32 ctx, wide_ell; // symbols the groups are tied on; of the caller's key
     u64 next;          // 0, or the doubling's first context past ctx, where it has none of ctx
-    bool words;        // the list is tied on words of written text
+    const u32* stream; // null, or the words of a written text that the list is tied on, and the bits of its symbols and words
+    u32 sym_bits, word_bits;
     bool settled;   // the list is in order, and the doubling would have gone through num generations more, of these sizes
     u32 num;
     u64 active[SETTLE_CONTEXTS], groups[SETTLE_CONTEXTS];
@@ -1615,7 +1616,10 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     a.gprim = ra.gprim_out;
     a.m = m;
     a.groups = groups;
-    a.most = st.words ? SETTLE_MAX_WORDS : SETTLE_MAX;
+    a.most = st.stream ? SETTLE_MAX_WORDS : SETTLE_MAX;
+    a.stream = st.stream;
+    a.sym_bits = st.sym_bits;
+    a.word_bits = st.word_bits;
     a.words[0] = (a.anchors + 63u) / 64u;
     a.words[1] = (a.words[0] + 63u) / 64u;
     a.words[2] = (a.words[1] + 63u) / 64u;
@@ -1654,7 +1658,7 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     hipLaunchKernelGGL(copy_links_top_kernel, dim3((a.words[1] + 255u) / 256u), dim3(256), 0, s, a);
     hipLaunchKernelGGL(copy_spread_kernel, dim3((u32)(((u64)a.anchors + 255) / 256)), dim3(256), 0, s, a);
     const dim3 settle_grid((u32)(((u64)m + SETTLE_TILE - 1) / SETTLE_TILE));
-    if (st.words)
+    if (st.stream)
         hipLaunchKernelGGL((settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX_WORDS>), settle_grid, dim3(SETTLE_BLOCK), 0, s, a);
     else
         hipLaunchKernelGGL((settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX>), settle_grid, dim3(SETTLE_BLOCK), 0, s, a);
@@ -2333,7 +2337,9 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         auto next = [&](u64 c) { return c + (c < wide_ell ? (c < wide_ell - c ? c : wide_ell - c) : c); };
         auto settle_at = [&](u64 context, u32 tied, u32 in_groups) -> int {
             settle.ctx = (u32)context;
-            settle.words = true;
+            settle.stream = ps.stream;
+            settle.sym_bits = ps.sym_bits;
+            settle.word_bits = ps.key_bits;
             settle.next = 4;
             while (settle.next <= context)
                 settle.next = next(settle.next);

@@ -25,6 +25,7 @@
 #pragma once
 
 #include "device_utils.hpp"
+#include "packed_text.hpp"
 
 namespace csa {
 
@@ -66,6 +67,8 @@ struct SettleArgs {
     const u32* gprim;
     u32 m, groups;
     u32 most;     // members of a group: SETTLE_MAX or SETTLE_MAX_WORDS
+    const u32* stream; // with SETTLE_MAX_WORDS: the text's words, and the bits of a symbol and of a word
+    u32 sym_bits, word_bits;
     u64* records; // [anchors + 1], NO_RECORD
     unsigned long long* links[3]; // bits of the anchors, of the words of links[0] that are all ones, of those of links[1]
     u32 words[3];
@@ -326,8 +329,9 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
     constexpr int TILE = BLOCK * SETTLE_ITEMS, SPAN = TILE + MAXG, ITEMS = (SPAN + BLOCK - 1) / BLOCK;
     constexpr u32 TALLIES = 2 * (SETTLE_CONTEXTS + 1), COPIES = 4;
     __shared__ u64 s_key[SPAN];
-    // Of groups that may be long, the four symbols after those in the key: members that are told from their root in the same way are told apart by these as a
-    // rule (one tile with a group of a thousand: 3.1 ms when all such pairs were compared by the text).
+    // Of groups that may be long, the word of nine to twelve symbols after those in the key: members that are told from their root in the same way are told apart
+    // by it as a rule. (10^8 letters, 1.8 ms of the kernel in one tile with a
+    // group of a thousand, when all such pairs were compared by the text or by four symbols more; 1.0 with the word.)
     constexpr bool MORE = MAXG > SETTLE_MAX;
     __shared__ u64 s_more[MORE ? SPAN : 1];
     __shared__ u32 s_suf[SPAN];
@@ -407,7 +411,7 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
             const u64 symbol = to[k] - from[k] > 2 && next < a.n ? (u64)a.text[next] + 1u : 0u; // (a pair has nobody else to be told from)
             key[k] = w.larger ? LARGER | ((FAR - w.length) << 17) | symbol : ((u64)w.length << 17) | symbol;
             if constexpr (MORE)
-                more[k] = symbol && next + 1 < a.n ? load_kgram(a.text, a.n, (u32)next + 1u, 0) : 0u;
+                more[k] = symbol && next + 1 < a.n ? packed_window(a.stream, (next + 1) * a.sym_bits, a.word_bits) : 0u;
         }
         s_key[k * BLOCK + t] = key[k];
         if constexpr (MORE)
@@ -423,8 +427,10 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
     // (more_left: steps that comparisons may take past their first two)
     auto further = [&](u32 y, u32 z, u64 w, u32& more_left) -> Agreement {
         const u32 r = y < z ? y : z, o = y < z ? z : y;
-        u32 steps_left = more_left + 2u;
-        const Agreement v = agreement(a, r, o, agreement_of(w) + 1u, steps_left);
+        u32 steps_left = more_left + 2u, tied = agreement_of(w) + 1u;
+        if constexpr (MORE) // (they share the word behind it, too, and where that is inside the text its symbols)
+            tied += (u64)o + tied + a.word_bits / a.sym_bits <= a.n ? a.word_bits / a.sym_bits : 0u;
+        const Agreement v = agreement(a, r, o, tied, steps_left);
         more_left = steps_left < more_left ? steps_left : more_left;
         return v;
     };
@@ -480,7 +486,7 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         u32 agree = of_v < of_w ? of_v : of_w;
         const u64 differ = MORE && v == w ? s_more[MORE ? right - 1 : 0] ^ s_more[MORE ? right : 0] : 0u;
         if (differ) {
-            agree = of_w + 1u + (u32)__builtin_clzll(differ) / 16u;
+            agree = of_w + 1u + ((u32)__builtin_clzll(differ) - (64u - a.word_bits)) / a.sym_bits;
         } else if (v == w) {
             u32 more_left = SETTLE_STEPS; // (enough: the two have been compared before)
             agree = further(y, z, w, more_left).length;
