@@ -117,10 +117,11 @@ __global__ __launch_bounds__(WINDOW_BLOCK) void word_digits_kernel(const u32* __
 
 // Texts that the second word does little for: padding, lines that come again and again, few words. Long runs of one first word are sorted again, to find them
 // long and of one second word as well. Looked for at 1024 places of the sorted list: more than 143 in runs of 256 or more, or more than 51 in
-// runs of 2048. (10^8 letters of written text have 10 and 2 % of their suffixes in such, 5 * 10^7 with a fifth in runs of spaces and a
-// period 28 and 22 %: those take 9.3 ms by the doubling and 10.4 when the second words are read first.) Such lists are ranked on the doubling's last
-// context inside the first word.
-constexpr u32 WORD_PLACES = 1024, WORD_LONG = 256, WORD_LONG_FEW = 143, WORD_LONGER = 2048, WORD_LONGER_FEW = 51;
+// runs of 2048; the runs of a written text grow with it, so from 2^26 symbols on in runs of n / 2^18, and eight times that. (10^8 letters of written text have 10
+// and 2 % of their suffixes in such, 5 * 10^7 with a fifth in runs of spaces and a period 28 and 22 %: those take 9.3 ms by the doubling and 10.4 when the
+// second words are read first. 2 * 10^8 letters: 31.9 ms by the doubling, where runs of 256 would send them, and 21.8; 3 * 10^8 49.1 and 42.2.) Such lists are
+// ranked on the doubling's last context inside the first word.
+constexpr u32 WORD_PLACES = 1024, WORD_LONG = 256, WORD_LONG_FEW = 143, WORD_LONG_SHIFT = 18, WORD_LONGER_FEW = 51;
 
 // (Launched before the list is counted, which is then left out: nothing would be done with the counts.)
 __global__ __launch_bounds__(WORD_PLACES) void choose_seconds_kernel(const u64* __restrict__ keys, u32 n, u32* skip)
@@ -130,7 +131,8 @@ __global__ __launch_bounds__(WORD_PLACES) void choose_seconds_kernel(const u64* 
     if (t < 2)
         s_in[t] = 0;
     __syncthreads();
-    const u64 in_long = __ballot(in_long_run(keys, n, WORD_LONG, t, WORD_PLACES)), in_longer = __ballot(in_long_run(keys, n, WORD_LONGER, t, WORD_PLACES));
+    const u32 is_long = n >> WORD_LONG_SHIFT > WORD_LONG ? n >> WORD_LONG_SHIFT : WORD_LONG, longer = 8 * is_long;
+    const u64 in_long = __ballot(in_long_run(keys, n, is_long, t, WORD_PLACES)), in_longer = __ballot(in_long_run(keys, n, longer, t, WORD_PLACES));
     if ((t & 63u) == 0) {
         atomicAdd(&s_in[0], (u32)__popcll(in_long));
         atomicAdd(&s_in[1], (u32)__popcll(in_longer));
