@@ -1578,8 +1578,9 @@ struct Settle {
     u32* sa32;      // the sorted list, whose groups are put in order
     u32 ctx, wide_ell; // symbols the groups are tied on; of the caller's key
     u64 next;          // 0, or the doubling's first context past ctx, where it has none of ctx
-    const u32* stream; // null, or the words of a written text that the list is tied on, and the bits of its symbols and words
+    const u32* stream; // null, or the codes of the text's symbols, as for the first sort, the bits of one, and of as many as 64 bits hold
     u32 sym_bits, word_bits;
+    bool words;        // the list is tied on words of written text
     bool settled;   // the list is in order, and the doubling would have gone through num generations more, of these sizes
     u32 num;
     u64 active[SETTLE_CONTEXTS], groups[SETTLE_CONTEXTS];
@@ -1616,7 +1617,7 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     a.gprim = ra.gprim_out;
     a.m = m;
     a.groups = groups;
-    a.most = st.stream ? SETTLE_MAX_WORDS : SETTLE_MAX;
+    a.most = st.words ? SETTLE_MAX_WORDS : SETTLE_MAX;
     a.stream = st.stream;
     a.sym_bits = st.sym_bits;
     a.word_bits = st.word_bits;
@@ -1654,14 +1655,15 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
         return rc;
     HIP_TRY(hipMemsetAsync(a.records, 0xFF, ((u64)a.anchors + 1) * sizeof(u64), s));
     hipLaunchKernelGGL(copy_roots_kernel, dim3((u32)(((u64)m + 255) / 256)), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(copy_links_kernel, dim3(a.words[1]), dim3(1024), 0, s, a);
+    auto* const links = st.stream ? copy_links_kernel<true> : copy_links_kernel<false>;
+    hipLaunchKernelGGL(links, dim3(a.words[1]), dim3(1024), 0, s, a);
     hipLaunchKernelGGL(copy_links_top_kernel, dim3((a.words[1] + 255u) / 256u), dim3(256), 0, s, a);
     hipLaunchKernelGGL(copy_spread_kernel, dim3((u32)(((u64)a.anchors + 255) / 256)), dim3(256), 0, s, a);
     const dim3 settle_grid((u32)(((u64)m + SETTLE_TILE - 1) / SETTLE_TILE));
-    if (st.stream)
-        hipLaunchKernelGGL((settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX_WORDS>), settle_grid, dim3(SETTLE_BLOCK), 0, s, a);
-    else
-        hipLaunchKernelGGL((settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX>), settle_grid, dim3(SETTLE_BLOCK), 0, s, a);
+    auto* const settle = st.words    ? settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX_WORDS, true>
+                         : st.stream ? settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX, true>
+                                     : settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX, false>;
+    hipLaunchKernelGGL(settle, settle_grid, dim3(SETTLE_BLOCK), 0, s, a);
     HIP_TRY(hipGetLastError());
     u32* const h_tallies = h->h_pinned + PINNED_HIST;
     add_table(seen, h_tallies, a.tallies, SETTLE_SLOTS * TALLIES * sizeof(u32));
@@ -2327,6 +2329,9 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     settle.sa32 = sa32;
     settle.ctx = ell;
     settle.wide_ell = (u32)wide_ell;
+    settle.stream = ps.stream;
+    settle.sym_bits = ps.sym_bits;
+    settle.word_bits = ps.stream ? 64u / ps.sym_bits * ps.sym_bits : 0u;
     WordList words;
     memset(&words, 0, sizeof(words));
     u32 by_words_settled = 0; // generations of the reference that such a sort has left nothing of, and one
@@ -2337,9 +2342,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         auto next = [&](u64 c) { return c + (c < wide_ell ? (c < wide_ell - c ? c : wide_ell - c) : c); };
         auto settle_at = [&](u64 context, u32 tied, u32 in_groups) -> int {
             settle.ctx = (u32)context;
-            settle.stream = ps.stream;
-            settle.sym_bits = ps.sym_bits;
-            settle.word_bits = ps.key_bits;
+            settle.words = true;
             settle.next = 4;
             while (settle.next <= context)
                 settle.next = next(settle.next);

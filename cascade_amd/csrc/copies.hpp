@@ -67,7 +67,7 @@ struct SettleArgs {
     const u32* gprim;
     u32 m, groups;
     u32 most;     // members of a group: SETTLE_MAX or SETTLE_MAX_WORDS
-    const u32* stream; // with SETTLE_MAX_WORDS: the text's words, and the bits of a symbol and of a word
+    const u32* stream; // null, or the codes of the symbols (packed_text.hpp), the bits of one, and of as many as 64 bits hold
     u32 sym_bits, word_bits;
     u64* records; // [anchors + 1], NO_RECORD
     unsigned long long* links[3]; // bits of the anchors, of the words of links[0] that are all ones, of those of links[1]
@@ -118,6 +118,40 @@ __device__ __forceinline__ bool differ_within(const u16* __restrict__ text, u32 
     return true;
 }
 
+// The same from the stream, where there is one: as many symbols at a time as 64 bits hold, 32 of four letters, and an eighth of the memory.
+__device__ __forceinline__ bool differ_within_stream(const SettleArgs& a, u32 r, u32 y, u32 from, u32 to, Agreement& out)
+{
+    const u32 syms = a.word_bits / a.sym_bits, room = a.n - y; // (y < n; zeros follow the text)
+    u64 off = from;
+    bool larger = false;
+    for (; off < to && off < room; off += syms) {
+        const u64 of_r = packed_window(a.stream, (r + off) * a.sym_bits, a.word_bits), of_y = packed_window(a.stream, (y + off) * a.sym_bits, a.word_bits);
+        if (of_r != of_y) {
+            off += ((u32)__builtin_clzll(of_r ^ of_y) - (64u - a.word_bits)) / a.sym_bits;
+            larger = of_y > of_r;
+            break;
+        }
+    }
+    if (off >= room) {
+        off = room;
+        larger = false;
+    }
+    if (off >= to)
+        return false;
+    out.length = (u32)off;
+    out.larger = larger;
+    out.found = true;
+    return true;
+}
+
+template <bool STREAM> __device__ __forceinline__ bool differ_within(const SettleArgs& a, u32 r, u32 y, u32 from, u32 to, Agreement& out)
+{
+    if constexpr (STREAM)
+        return differ_within_stream(a, r, y, from, to, out);
+    else
+        return differ_within(a.text, a.n, r, y, from, to, out);
+}
+
 // The first anchor at or after i that is not linked to the next (the last anchor never is).
 __device__ __forceinline__ u32 chain_end(const SettleArgs& a, u32 i)
 {
@@ -162,7 +196,15 @@ __device__ __forceinline__ u32 chain_end(const SettleArgs& a, u32 i)
 __device__ __forceinline__ u32 root_of(u64 record) { return (u32)(record >> 32) & 0x7FFFFFFFu; }
 __device__ __forceinline__ u32 length_of(u64 record) { return (u32)record >> 1; }
 
+// The last anchor up to which suffix y is known to agree with whoever shares its group (at y or after it: ctx >= gap).
+__device__ __forceinline__ u32 first_anchor(const SettleArgs& a, u32 y)
+{
+    const u64 reach = (u64)y + a.ctx;
+    return (u32)((reach < a.n ? reach : (u64)a.n) >> a.log2_gap);
+}
+
 // How far suffixes r < y agree, which are tied on their first `tied` >= ctx symbols; takes its steps from steps_left.
+template <bool STREAM>
 __device__ __forceinline__ Agreement agreement(const SettleArgs& a, u32 r, u32 y, u32 tied, u32& steps_left)
 {
     Agreement out = {tied, false, false};
@@ -211,7 +253,7 @@ __device__ __forceinline__ Agreement agreement(const SettleArgs& a, u32 r, u32 y
                 off = both > off ? both : off;
             }
         }
-        if (differ_within(a.text, a.n, r, y, (u32)off, (u32)off + gap, out))
+        if (differ_within<STREAM>(a, r, y, (u32)off, (u32)off + gap, out))
             return out;
         off += gap;
     }
@@ -247,6 +289,7 @@ __global__ __launch_bounds__(256) void copy_roots_kernel(SettleArgs a)
 }
 
 // links[0], links[1] and the ends. Bounded by reading the records once; the anchors that are not linked are few.
+template <bool STREAM>
 __global__ __launch_bounds__(1024) void copy_links_kernel(SettleArgs a)
 {
     __shared__ unsigned long long s_word[LINK_TILE / 64];
@@ -273,7 +316,7 @@ __global__ __launch_bounds__(1024) void copy_links_kernel(SettleArgs a)
             for (u32 skip = 2; skip <= SETTLE_ENDS; ++skip) {
                 const u32 to = skip << a.log2_gap;
                 if (from < to) {
-                    if (differ_within(a.text, a.n, root, y, from, to, out))
+                    if (differ_within<STREAM>(a, root, y, from, to, out))
                         break;
                     from = to;
                 }
@@ -323,7 +366,7 @@ __global__ __launch_bounds__(256) void copy_spread_kernel(SettleArgs a)
 // The members of every group in order, to their places in the suffix array, and the tallies. A tile settles the groups that start in it.
 // What bounds it is the random read of a member: its anchor's record. (1e9 Zipf tokens with 6 % of their documents copied, 55.7 M members
 // tied on 8 symbols: 1.5 ms here, 1.1 for the records, where the update of 1e9 ranks took 10.5 and ten generations 9.8.)
-template <int BLOCK, int MAXG>
+template <int BLOCK, int MAXG, bool STREAM>
 __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
 {
     constexpr int TILE = BLOCK * SETTLE_ITEMS, SPAN = TILE + MAXG, ITEMS = (SPAN + BLOCK - 1) / BLOCK;
@@ -333,9 +376,12 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
     // by it as a rule. (10^8 letters, 1.8 ms of the kernel in one tile with a
     // group of a thousand, when all such pairs were compared by the text or by four symbols more; 1.0 with the word.)
     constexpr bool MORE = MAXG > SETTLE_MAX;
+    static_assert(STREAM || !MORE, "the words are those of the stream");
     __shared__ u64 s_more[MORE ? SPAN : 1];
     __shared__ u32 s_suf[SPAN];
     __shared__ u32 s_tally[TALLIES * COPIES];
+    __shared__ u16 s_queue[SPAN];
+    __shared__ u32 s_queued;
     __shared__ u32 s_over;   // a tile before has given up
     __shared__ u32 s_lost[2]; // some member of the tile could not be compared with its root; two members with each other
     const u32 t = threadIdx.x;
@@ -343,13 +389,13 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         s_tally[i] = 0;
     if (t == 0) {
         s_over = *a.failed;
-        s_lost[0] = s_lost[1] = 0;
+        s_lost[0] = s_lost[1] = s_queued = 0;
     }
     const u64 t0 = (u64)blockIdx.x * TILE;
     u32 x[ITEMS], place[ITEMS];
     int from[ITEMS], to[ITEMS]; // the group, by places of the span; to = 0: nothing to do
     u32 prim[ITEMS];
-    u64 key[ITEMS], more[MORE ? ITEMS : 1] = {};
+    u64 key[ITEMS] = {}, more[MORE ? ITEMS : 1] = {};
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         const u32 j = k * BLOCK + t;
@@ -392,30 +438,54 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         return (w >> 48) == 0 ? v : (w >> 48) == 1 ? (u32)FAR : (u32)FAR - v;
     };
     volatile u32* const lost = s_lost;
+    auto put_key = [&](u32 j, u32 y, bool alone, const Agreement& w) { // (alone: one of a pair has nobody else to be told from)
+        const u64 next = (u64)y + w.length;
+        const u64 symbol = alone || next >= a.n ? 0u : (STREAM ? packed_window(a.stream, next * a.sym_bits, a.sym_bits) : (u64)a.text[next]) + 1u;
+        s_key[j] = w.larger ? LARGER | ((FAR - w.length) << 17) | symbol : ((u64)w.length << 17) | symbol;
+        if constexpr (MORE)
+            s_more[j] = symbol && next + 1 < a.n ? packed_window(a.stream, (next + 1) * a.sym_bits, a.word_bits) : 0u;
+    };
+    // Most members' first record tells. Those whose does not are queued, and take their steps side by side: a wave would wait for the one
+    // lane in each item that takes the most. (4e8 letters, 108 M members, every member at its item: 6.57 ms; queued
+    // 5.92; and what the records leave open read from the stream of codes, 100 MB that stay in the cache, instead of the text: 5.12.)
+    u32 root[ITEMS];
+    u64 first[ITEMS];
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
-        key[k] = ROOT;
-        if constexpr (MORE)
-            more[k] = 0;
-        if (to[k] == 0 || lost[0]) // (a tile that has lost a member writes nothing)
+        root[k] = x[k];
+        first[k] = NO_RECORD;
+        if (to[k] == 0)
             continue;
-        u32 root = x[k];
         for (int i = from[k]; i < to[k]; ++i)
-            root = s_suf[i] < root ? s_suf[i] : root;
-        if (root != x[k]) {
-            u32 steps_left = SETTLE_STEPS;
-            const Agreement w = agreement(a, root, x[k], a.ctx, steps_left);
-            if (!w.found)
-                lost[0] = 1u;
-            const u64 next = (u64)x[k] + w.length;
-            const u64 symbol = to[k] - from[k] > 2 && next < a.n ? (u64)a.text[next] + 1u : 0u; // (a pair has nobody else to be told from)
-            key[k] = w.larger ? LARGER | ((FAR - w.length) << 17) | symbol : ((u64)w.length << 17) | symbol;
+            root[k] = s_suf[i] < root[k] ? s_suf[i] : root[k];
+        if (root[k] != x[k])
+            first[k] = a.records[first_anchor(a, x[k])];
+    }
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        if (to[k] == 0)
+            continue;
+        const u32 j = k * BLOCK + t, shift = (first_anchor(a, x[k]) << a.log2_gap) - x[k];
+        if (root[k] == x[k]) {
+            s_key[j] = ROOT;
             if constexpr (MORE)
-                more[k] = symbol && next + 1 < a.n ? packed_window(a.stream, (next + 1) * a.sym_bits, a.word_bits) : 0u;
+                s_more[j] = 0;
+        } else if (first[k] != NO_RECORD && root_of(first[k]) == root[k] + shift && !(first[k] & OPEN)) {
+            put_key(j, x[k], to[k] - from[k] == 2, Agreement{shift + length_of(first[k]), (first[k] & 1u) != 0, true});
+        } else {
+            s_queue[atomicAdd(&s_queued, 1u)] = (u16)j;
+            s_key[j] = (u64)root[k] << 1 | (to[k] - from[k] == 2 ? 1u : 0u);
         }
-        s_key[k * BLOCK + t] = key[k];
-        if constexpr (MORE)
-            s_more[k * BLOCK + t] = more[k];
+    }
+    __syncthreads();
+    for (u32 q = t; q < s_queued && !lost[0]; q += BLOCK) { // (a tile that has lost a member writes nothing)
+        const u32 j = s_queue[q], y = s_suf[j];
+        u32 steps_left = SETTLE_STEPS;
+        const Agreement w = agreement<STREAM>(a, (u32)(s_key[j] >> 1), y, a.ctx, steps_left);
+        if (!w.found)
+            lost[0] = 1u;
+        else
+            put_key(j, y, (s_key[j] & 1u) != 0, w);
     }
     __syncthreads();
     if (s_lost[0]) {
@@ -423,6 +493,13 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
             *a.failed = 1u;
         return;
     }
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+        if (to[k] != 0) {
+            key[k] = s_key[k * BLOCK + t];
+            if constexpr (MORE)
+                more[k] = s_more[k * BLOCK + t];
+        }
     // does suffix y go before suffix z of the same key: their agreement from the symbol after the one that tells them from their root
     // (more_left: steps that comparisons may take past their first two)
     auto further = [&](u32 y, u32 z, u64 w, u32& more_left) -> Agreement {
@@ -430,7 +507,7 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         u32 steps_left = more_left + 2u, tied = agreement_of(w) + 1u;
         if constexpr (MORE) // (they share the word behind it, too, and where that is inside the text its symbols)
             tied += (u64)o + tied + a.word_bits / a.sym_bits <= a.n ? a.word_bits / a.sym_bits : 0u;
-        const Agreement v = agreement(a, r, o, tied, steps_left);
+        const Agreement v = agreement<STREAM>(a, r, o, tied, steps_left);
         more_left = steps_left < more_left ? steps_left : more_left;
         return v;
     };
