@@ -24,6 +24,7 @@ RADIX_PASS_BYTES_PER_PAIR = 2 * (8 + 5)
 # the same of a pass of the first sort over (32-bit code, index) pairs, which texts over large alphabets take: a 4-byte key
 CODED_PASS_BYTES_PER_PAIR = 2 * (4 + 5)
 CODED_PASSES = 4
+BUCKET_PASSES = 2  # of a long text's codes: the lower digits are sorted in LDS, bucket by bucket
 
 
 def algorithmic_bytes(n, active):
@@ -637,7 +638,8 @@ def main():
     # a first sort on packed symbols resolves 8 or more; one on K-gram keys, which none of these workloads takes, makes 8 passes, and so
     # does one on 64-bit packed keys (32 letters on narrow keys: four, as codes, unless long runs were sorted again)
     coded = st["passes"][0] != 8 if st["key_symbols"] == 4 else st["key_symbols"] == 32 and st["passes"][0] == 4
-    coded_pairs = CODED_PASSES * n * args.steps if coded else 0
+    coded_passes = CODED_PASSES if radix_pairs >= CODED_PASSES * n * args.steps else BUCKET_PASSES
+    coded_pairs = min(coded_passes * n * args.steps, radix_pairs) if coded else 0
     radix_bytes = RADIX_PASS_BYTES_PER_PAIR * (radix_pairs - coded_pairs) + CODED_PASS_BYTES_PER_PAIR * coded_pairs
     achieved = radix_bytes / (radix_ms * 1e-3) / 1e9 if radix_ms > 0 else 0.0
     pairs_per_launch = radix_pairs / radix_launches if radix_launches else 0
@@ -681,8 +683,8 @@ def main():
         result["job_alg_note"] = (f"the first sort (keys of {st['key_symbols']} packed symbols) stands for generations 0-"
                                   f"{st['first_sort_generations'] - 1} of the reference's list, whose bytes the yardstick still counts")
     elif coded_pairs:
-        result["job_alg_note"] = ("the yardstick counts generation 0 as eight passes over (64-bit key, index) pairs; the sort makes four over "
-                                  "(32-bit code, index) pairs")
+        result["job_alg_note"] = (f"the yardstick counts generation 0 as eight passes over (64-bit key, index) pairs; the sort makes {coded_passes} over "
+                                  "(32-bit code, index) pairs" + (", and the lower digits in LDS" if coded_passes == BUCKET_PASSES else ""))
     if moved_gen_dropped:
         result["generation_traffic_dropped"] = moved_gen_dropped
     if args.cpu_sample > 0:

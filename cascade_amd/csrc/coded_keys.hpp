@@ -8,7 +8,9 @@
 // intervals, so that the codes spread evenly over the 32 bits where the raw symbols of a token text crowd into few values.
 // Four passes over 8-byte (code, suffix) pairs put the suffixes into the order of their codes, where K-gram keys take
 // eight passes over 12-byte pairs: 66 instead of 185 bytes moved per suffix (2^28 Zipf tokens: generation 0's passes 11.5 ->
-// 4.1 ms).
+// 4.1 ms). From 2^24 suffixes on two passes over the upper digits are enough, and the lower ones are sorted bucket by bucket in LDS
+// (bucket_sort.hpp); codes of token texts then take 16 bits of what follows with them (EXT), which settles most of what shares a code
+// without a line of the text (1e9 tokens 45.5 -> 35.7 ms).
 //
 // A string whose interval of codes holds at least two 32-bit values takes the second of them, which no other string can
 // have: its suffixes carry a flag (OWN_CODE) through the sort and are known to be equal where their codes are.

@@ -51,7 +51,8 @@ typedef struct csa_stats {
     uint64_t groups[CSA_MAX_GENERATIONS]; /* unresolved groups entering generation g (0 for g = 0) */
     uint64_t big[CSA_MAX_GENERATIONS];    /* of active[g], members of groups too large for the in-tile sort */
     int32_t passes[CSA_MAX_GENERATIONS];  /* radix passes run in generation g (over the large groups for g > 0; for g = 0 four
-                                             on codes or up to eight on keys, and those over runs that had to be sorted again) */
+                                             on codes, the digits that are sorted in LDS bucket by bucket counted among them,
+                                             or up to eight on keys, and those over runs that had to be sorted again) */
     int32_t rank_update[CSA_MAX_GENERATIONS]; /* how generation g wrote its ranks: 0 scattered from the rank pass,
                                                  1 bucketed by two passes into LDS-sized windows (generation 0),
                                                  2 bucketed by one pass into cache-sized windows */
@@ -64,7 +65,7 @@ typedef struct csa_stats {
     float ms_total;                       /* first kernel to last kernel, on the stream */
     /* with CSA_FLAG_KERNEL_TIMING: the radix-pass kernel, summed over all its launches */
     uint64_t radix_launches;
-    uint64_t radix_pairs; /* (key, index) pairs moved, summed over launches */
+    uint64_t radix_pairs; /* (key, index) pairs moved, summed over launches (digits sorted in LDS: none) */
     double radix_ms;
     uint64_t presorted[CSA_MAX_GENERATIONS]; /* of big[g], members that skipped the radix sort: every large group of the
                                                 list was in order of rank[x + h] already (rising or falling along the
@@ -81,7 +82,9 @@ typedef struct csa_stats {
                                         which are settled at once without ranks (rank_update[0] is 0 then), and those after the
                                         first of a list of runs and periods, which is settled at once as well (big[] and presorted[]
                                         as the generations would have had them). Texts of up to 8192 symbols are ranked by counting:
-                                        no passes, all time in ms[0], and 4 here whatever the alphabet */
+                                        no passes, all time in ms[0], and 4 here whatever the alphabet. Written text (17 to 128 byte
+                                        values, 2^18 symbols or more) is sorted by words of 9 to 12 symbols, and the next word where
+                                        those tie, and reports the key_symbols and first_sort_generations of 8-bit codes */
     uint32_t first_sort_generations; /* generations of the reference that sort stands for: 1, or 1 + j when its keys held
                                         4 * key_words * 2^j symbols. Generations 1 .. j are then reported with the lists
                                         they would have had (active[], groups[]) and with no time or passes of their own */
