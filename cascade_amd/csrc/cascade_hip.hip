@@ -2136,9 +2136,6 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     TableGroup zeros = {};
     add_table(zeros, h->counts, nullptr, 13 * sizeof(u32));
     add_table(zeros, h->ghist, nullptr, (MAX_PASSES + 2) * RADIX_BINS * sizeof(u32));
-    u32* const windows = reinterpret_cast<u32*>(h->key[1]); // for written text; the first pass of the sort writes it, afterwards
-    if (n >= CSA_WORD_KEYS_MIN)
-        add_table(zeros, windows, nullptr, sizeof(u32) << WINDOW_BITS<7>);
     int rc = move_tables(zeros, s);
     if (rc)
         return rc;
@@ -2239,7 +2236,9 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         ps.sym_bits = word_bits;
         ps.key_bits = word_bits * word_syms;
         ps.words = ((u64)n * word_bits + 31) / 32 + 4;
-        hipLaunchKernelGGL(encode_words_kernel, dim3((u32)((ps.words + WORD_SPAN - 1) / WORD_SPAN)), dim3(WORD_BLOCK), 0, s, d_text, n, codes, h->rank, ps.words);
+        u32* const windows = reinterpret_cast<u32*>(K[1]); // (the first pass writes it, afterwards)
+        hipLaunchKernelGGL(encode_words_kernel, dim3((u32)((ps.words + WORD_SPAN - 1) / WORD_SPAN)), dim3(WORD_BLOCK), 0, s, d_text, n, codes, h->rank, ps.words,
+                           windows, 1u << (word_bits + 7));
         const u32 blocks = hist_blocks(WINDOW_BLOCK * 4, n);
         auto* const count = word_bits == 5 ? window_hist_kernel<5> : word_bits == 6 ? window_hist_kernel<6> : window_hist_kernel<7>;
         hipLaunchKernelGGL(count, dim3(blocks < WINDOW_HIST_BLOCKS ? blocks : WINDOW_HIST_BLOCKS), dim3(WINDOW_BLOCK), 0, s, (const u32*)h->rank, n, windows);

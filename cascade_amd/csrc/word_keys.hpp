@@ -30,13 +30,15 @@ struct WordLevels {
 constexpr int WORD_BLOCK = 256;
 constexpr u32 WORD_SPAN = 256;      // words of a workgroup's stretch
 
-// stream[wd], wd < words: bits 32 wd .. of the codes of all symbols, `bits` each, zero past the text.
-__global__ __launch_bounds__(WORD_BLOCK) void encode_words_kernel(const u16* __restrict__ text, u32 n, SymbolCodes codes, u32* __restrict__ stream, u64 words)
+// stream[wd], wd < words: bits 32 wd .. of the codes of all symbols, `bits` each, zero past the text. Sets the counts of windows to zero.
+__global__ __launch_bounds__(WORD_BLOCK) void encode_words_kernel(const u16* __restrict__ text, u32 n, SymbolCodes codes, u32* __restrict__ stream, u64 words, u32* __restrict__ windows, u32 bins)
 {
     constexpr u32 MAX_SYMS = WORD_SPAN * 32 / 5 + 8;
     __shared__ u64 s_text[(MAX_SYMS + 6) / 4 + 2];
     __shared__ SymbolCodes s_codes;
     const u32 t = threadIdx.x, b = codes.bits;
+    for (u64 i = (u64)blockIdx.x * WORD_BLOCK + t; i < bins; i += (u64)gridDim.x * WORD_BLOCK)
+        windows[i] = 0;
     for (u32 i = t; i < sizeof(SymbolCodes) / 4; i += WORD_BLOCK)
         reinterpret_cast<u32*>(&s_codes)[i] = reinterpret_cast<const u32*>(&codes)[i];
     const u64 w0 = (u64)blockIdx.x * WORD_SPAN, first = w0 * 32 / b;
