@@ -1659,11 +1659,11 @@ int settle_copies(Launch& L, Settle& st, const RerankArgs& ra, u32 m, u32 groups
     hipLaunchKernelGGL(links, dim3(a.words[1]), dim3(1024), 0, s, a);
     hipLaunchKernelGGL(copy_links_top_kernel, dim3((a.words[1] + 255u) / 256u), dim3(256), 0, s, a);
     hipLaunchKernelGGL(copy_spread_kernel, dim3((u32)(((u64)a.anchors + 255) / 256)), dim3(256), 0, s, a);
-    const dim3 settle_grid((u32)(((u64)m + SETTLE_TILE - 1) / SETTLE_TILE));
-    auto* const settle = st.words    ? settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX_WORDS, true>
-                         : st.stream ? settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX, true>
-                                     : settle_groups_kernel<SETTLE_BLOCK, SETTLE_MAX, false>;
-    hipLaunchKernelGGL(settle, settle_grid, dim3(SETTLE_BLOCK), 0, s, a);
+    auto* const settle = st.words    ? settle_groups_kernel<SETTLE_WORDS_BLOCK, SETTLE_WORDS_ITEMS, SETTLE_MAX_WORDS, true>
+                         : st.stream ? settle_groups_kernel<SETTLE_BLOCK, SETTLE_ITEMS, SETTLE_MAX, true>
+                                     : settle_groups_kernel<SETTLE_BLOCK, SETTLE_ITEMS, SETTLE_MAX, false>;
+    const u32 block = st.words ? SETTLE_WORDS_BLOCK : SETTLE_BLOCK, tile = block * (st.words ? SETTLE_WORDS_ITEMS : SETTLE_ITEMS);
+    hipLaunchKernelGGL(settle, dim3((u32)(((u64)m + tile - 1) / tile)), dim3(block), 0, s, a);
     HIP_TRY(hipGetLastError());
     u32* const h_tallies = h->h_pinned + PINNED_HIST;
     add_table(seen, h_tallies, a.tallies, SETTLE_SLOTS * TALLIES * sizeof(u32));

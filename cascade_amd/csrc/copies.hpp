@@ -29,9 +29,11 @@
 
 namespace csa {
 
-constexpr int SETTLE_BLOCK = 512;
-constexpr int SETTLE_ITEMS = 4;
-constexpr int SETTLE_TILE = SETTLE_BLOCK * SETTLE_ITEMS;
+// Small tiles, whose waves wait for few others at the barriers, as far as the SETTLE_MAX places behind a tile, which it reads as well, allow (ms of 108 M members of
+// 4e8 letters / of 2^28 tokens' copies: 512 x 4 members 5.12 / 0.42, 256 x 4 4.81 / 0.39, 256 x 3 4.56 / 0.35, 128 x 8 5.54 / 0.44). Groups of up to
+// SETTLE_MAX_WORDS take the largest block, which settles the longest of them (10^8 letters: 256 x 4 1.18, 512 x 4 0.95, 1024 x 2 0.67).
+constexpr int SETTLE_BLOCK = 256, SETTLE_ITEMS = 3;
+constexpr int SETTLE_WORDS_BLOCK = 1024, SETTLE_WORDS_ITEMS = 2;
 constexpr int SETTLE_MAX = 256; // longest group ...
 // ... and of lists that are tied on two words of written text, where one phrase may come a thousand times (5 * 10^7 symbols: 434 times on 24
 // letters, the next longest group has 55 members).
@@ -366,10 +368,10 @@ __global__ __launch_bounds__(256) void copy_spread_kernel(SettleArgs a)
 // The members of every group in order, to their places in the suffix array, and the tallies. A tile settles the groups that start in it.
 // What bounds it is the random read of a member: its anchor's record. (1e9 Zipf tokens with 6 % of their documents copied, 55.7 M members
 // tied on 8 symbols: 1.5 ms here, 1.1 for the records, where the update of 1e9 ranks took 10.5 and ten generations 9.8.)
-template <int BLOCK, int MAXG, bool STREAM>
+template <int BLOCK, int PER, int MAXG, bool STREAM>
 __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
 {
-    constexpr int TILE = BLOCK * SETTLE_ITEMS, SPAN = TILE + MAXG, ITEMS = (SPAN + BLOCK - 1) / BLOCK;
+    constexpr int TILE = BLOCK * PER, SPAN = TILE + MAXG, ITEMS = (SPAN + BLOCK - 1) / BLOCK;
     constexpr u32 TALLIES = 2 * (SETTLE_CONTEXTS + 1), COPIES = 4;
     __shared__ u64 s_key[SPAN];
     // Of groups that may be long, the word of nine to twelve symbols after those in the key: members that are told from their root in the same way are told apart
