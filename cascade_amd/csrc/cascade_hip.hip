@@ -1898,11 +1898,8 @@ int sort_by_words(Launch& L, u32 n, const TextSource& ps, u32 syms, u64* spare, 
     a.levels = list.levels;
     a.sufs_out = sufs_out;
     a.ties = ties;
-    a.at_end = h->counts + 4;
     a.any_long = h->counts + 5;
-    TableGroup cleared = {};
-    add_table(cleared, h->counts + 4, nullptr, 2 * sizeof(u32));
-    int rc = move_tables(cleared, s);
+    int rc = move_table(a.any_long, nullptr, sizeof(u32), s);
     if (rc)
         return rc;
     hipLaunchKernelGGL(resolve_words_kernel, dim3((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE)), dim3(RESOLVE_BLOCK), 0, s, a);
@@ -1994,11 +1991,8 @@ int sort_by_words(Launch& L, u32 n, const TextSource& ps, u32 syms, u64* spare, 
     a.run_slots = V[first ^ second];
     hipLaunchKernelGGL(place_words_kernel, member_grid, dim3(256), 0, s, a, list.members);
     HIP_TRY(hipGetLastError());
-    if ((rc = count_and_read()) != CSA_OK)
-        return rc;
-    if (h->h_pinned[4] == 0)
-        list.valid = list.levels.count;
-    return CSA_OK;
+    list.valid = list.levels.count;
+    return count_and_read();
 }
 
 // The contexts of a list that is resolved on two words of syms symbols: the doubling's from the caller's key on, the last of those before it that the first
@@ -2204,7 +2198,8 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     int folded = 0; // generations after the first that still belong to the reported generation 0
     for (u64 c = ell; c < wide_ell; c += (c < wide_ell - c ? c : wide_ell - c))
         ++folded;
-    const u32 tail = by_words ? (n < word_syms ? n : word_syms) : n < ell ? n : ell;
+    // suffixes that come first, shortest first: those that run off the text inside what the first sort resolves
+    const u32 front = by_words ? 2 * word_syms : ell, tail = n < front ? n : front;
     bool coded = !pp.enabled && !pp.byte_wide && !by_words;
     if (coded) {
         const bool probed = n >= PROBE_MIN, ahead = !probed || n < CODE_AHEAD_MAX;

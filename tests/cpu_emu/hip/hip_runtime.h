@@ -21,6 +21,7 @@
 #include <cstring>
 #include <functional>
 #include <memory>
+#include <string>
 #include <vector>
 
 #define __global__
@@ -231,7 +232,20 @@ inline void hipemu::launch(dim3 grid, dim3 blk, size_t shmem, const std::functio
 }
 
 #define hipLaunchKernelGGL(kernel, grid, blk, shmem, stream, ...) \
-    hipemu::launch((grid), (blk), (shmem), [&] { kernel(__VA_ARGS__); })
+    (hipemu::log_launch(#kernel), hipemu::launch((grid), (blk), (shmem), [&] { kernel(__VA_ARGS__); }))
+
+// The kernels that have been launched since hipemu_forget_launches(), as they are written at the launch, one a line: which way a
+// sort has taken, where its results do not tell.
+namespace hipemu {
+inline std::string& launch_log()
+{
+    static std::string s;
+    return s;
+}
+inline void log_launch(const char* kernel) { (launch_log() += kernel) += '\n'; }
+} // namespace hipemu
+extern "C" inline __attribute__((used)) const char* hipemu_launches() { return hipemu::launch_log().c_str(); }
+extern "C" inline __attribute__((used)) void hipemu_forget_launches() { hipemu::launch_log().clear(); }
 
 // ---- synchronisation and wave operations ----
 inline void __syncthreads() { hipemu::barrier(hipemu::run->arrived, hipemu::run->phase, (unsigned)hipemu::run->fibers.size()); }

@@ -47,6 +47,7 @@ def load_emulation(target):
     lib.csa_scratch_high_water.argtypes = [vp]
     lib.csa_last_step_result.argtypes = [vp, C.POINTER(_native.CsaStepResult)]
     lib.csa_set_tuning.argtypes = [vp, i32, u32]
+    lib.hipemu_launches.restype = C.c_char_p
     return lib
 
 
@@ -86,9 +87,11 @@ def emu_sort(lib, T, key_words, pack=True, expect_presorted=False, defer_min=Non
         assert lib.csa_set_tuning(h, _native.CSA_TUNE_DEFER_MIN, defer_min) == 0
     out = np.zeros(5 * n + 8, dtype=np.uint8)
     st = _native.CsaStats()
+    lib.hipemu_forget_launches()
     rc = lib.csa_sort_partition_u16_dev(h, T.ctypes.data, n, 0, out.ctypes.data, None, 0, C.byref(st))
     lib.csa_destroy(h)
     assert rc == 0, lib.csa_last_error()
+    emu_sort.launches = lib.hipemu_launches().decode().split("\n")  # as they are written in the sources
     emu_sort.rank_update = [int(st.rank_update[i]) for i in range(st.generations)]
     emu_sort.small_only = [int(st.small_only[i]) for i in range(st.generations)]
     emu_sort.dense = [int(st.dense[i]) for i in range(st.generations)]
@@ -1042,3 +1045,49 @@ def test_streams_of_five_to_seven_bits(values):
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
     assert emu_sort.key_symbols == 8 and emu_sort.first_sort_generations == 2
+
+
+@pytest.mark.parametrize("cut", [12, 17, 23, 24, 25])
+@pytest.mark.parametrize("zeros", [0, 1])
+def test_the_end_of_written_text_in_a_long_run(cut, zeros):
+    """The text ends inside the second word of a member of a long run, whose padded word others have (zeros are symbols here) or as which others go on: it is the first of
+    those, and the list is settled as any other is."""
+    lib = load_emulation("libcascade_emu_buckets.so")
+    n = 9001
+    rng = np.random.default_rng(cut)
+    T = rng.integers(97, 123, n).astype(np.uint16)
+    phrase = np.concatenate([np.arange(97, 97 + 16), np.full(10, 0 if zeros else 120)])
+    for at in rng.permutation(n // 40 - 2)[:90]:
+        T[40 * at:40 * at + 26] = phrase
+    T[n // 2:n // 2 + n // 4] = T[n // 9:n // 9 + n // 4]
+    T[-cut:] = phrase[:cut]
+    got, active, _ = emu_sort(lib, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    assert "place_words_kernel" in emu_sort.launches and not any("smallsort_kernel" in k for k in emu_sort.launches)
+
+
+def test_written_text_most_of_which_is_in_long_runs():
+    """Phrases that come a hundred times: more than a quarter of the suffixes are in runs that are too long for a tile, but not in such that the second words are
+    left out for, so those of short runs alone are resolved by them, and the doubling goes on from the first words."""
+    lib = load_emulation("libcascade_emu_buckets.so")
+    rng = np.random.default_rng(5)
+    phrases = rng.integers(97, 123, (6, 20)).astype(np.uint16)
+    T = np.concatenate([phrases[rng.permutation(np.repeat(np.arange(6), 90))].reshape(-1), rng.integers(97, 123, 3001).astype(np.uint16)])
+    got, active, _ = emu_sort(lib, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    assert "(collect_words_kernel<false>)" in emu_sort.launches or "collect_words_kernel<false>" in emu_sort.launches
+    assert "place_words_kernel" not in emu_sort.launches
+
+
+def test_written_text_without_long_runs():
+    """More suffixes tie on the first word than are settled on it, none in runs that are too long for a tile."""
+    lib = load_emulation("libcascade_emu_buckets.so")
+    rng = np.random.default_rng(6)
+    phrases = rng.integers(97, 123, (200, 20)).astype(np.uint16)
+    T = phrases[rng.permutation(np.repeat(np.arange(200), 5))[:500]].reshape(-1)
+    got, active, _ = emu_sort(lib, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    assert "resolve_words_kernel" in emu_sort.launches and not any("collect_words_kernel" in k for k in emu_sort.launches)
