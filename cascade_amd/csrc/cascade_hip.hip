@@ -1580,7 +1580,7 @@ struct Settle {
     u64 next;          // 0, or the doubling's first context past ctx, where it has none of ctx
     const u32* stream; // null, or the codes of the text's symbols, as for the first sort, the bits of one, and of as many as 64 bits hold
     u32 sym_bits, word_bits;
-    bool words;        // the list is tied on words of written text
+    bool words;        // written text: groups may be long
     bool settled;   // the list is in order, and the doubling would have gone through num generations more, of these sizes
     u32 num;
     u64 active[SETTLE_CONTEXTS], groups[SETTLE_CONTEXTS];
@@ -2334,15 +2334,18 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         const WordLevels& lv = words.levels;
         const u32 all = lv.count - 1;
         auto next = [&](u64 c) { return c + (c < wide_ell ? (c < wide_ell - c ? c : wide_ell - c) : c); };
-        auto settle_at = [&](u64 context, u32 tied, u32 in_groups) -> int {
+        auto settle_at = [&](u64 context, u32 tied, u32 in_groups, bool long_groups) -> int {
             settle.ctx = (u32)context;
-            settle.words = true;
+            settle.words = long_groups;
             settle.next = 4;
             while (settle.next <= context)
                 settle.next = next(settle.next);
             return settle_copies(L, settle, ra, tied, in_groups);
         };
-        // A list with few ties on the first word has them counted and settled as they are: nothing is read from the text.
+        // A list with few ties on the first word has them counted and settled as they are, and so has one whose ties are copies, two or three to a
+        // group: the second words would tell nothing of those apart. (Independent letters of 60 with a fifth of the text copied, 2.2 to a group, us with
+        // the second words read / settled on the first, in tiles for short groups / in those for long ones: 2^18 symbols 333 / 312 / 327, 10^7 1137 / 900 /
+        // 981, 5 * 10^7 4621 / 3585 / 3887. Written text from 2.67 to a group on, 2^18 letters: 327 / 530 / 373.)
         const RankTables r = rank_tables<RANK_TILE>(h, n);
         RerankArgs firsts = ra;
         firsts.ell = word_syms;
@@ -2381,11 +2384,12 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             words.groups[i] = (u32)hd;
         }
         firsts.skip = nullptr;
-        if (!skip && tied > 0 && tied < n / 8 && (u64)tied <= (u64)in_groups * SETTLE_AVG_LIMIT) {
+        const bool few_ties = tied < n / 8, copies = 2 * (u64)tied <= 5 * (u64)in_groups;
+        if (!skip && tied > 0 && (few_ties ? (u64)tied <= (u64)in_groups * SETTLE_AVG_LIMIT : copies)) {
             firsts.rank = nullptr;
             hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS, false>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, firsts);
             HIP_TRY(hipGetLastError());
-            if ((rc = settle_at(word_syms, tied, in_groups)) != CSA_OK)
+            if ((rc = settle_at(word_syms, tied, in_groups, few_ties)) != CSA_OK)
                 return rc;
         }
         const bool seconds = !skip && tied > 0 && !settle.settled;
@@ -2410,7 +2414,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                 active.rank = nullptr;
                 hipLaunchKernelGGL((compact_ties_kernel<RANK_TILE>), dim3((r.tiles + 3) / 4), dim3(256), 0, s, active, r.tiles);
                 HIP_TRY(hipGetLastError());
-                if ((rc = settle_at(lv.context[all], tied, in_groups)) != CSA_OK)
+                if ((rc = settle_at(lv.context[all], tied, in_groups, true)) != CSA_OK)
                     return rc;
             }
         }

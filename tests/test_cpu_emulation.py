@@ -1091,3 +1091,18 @@ def test_written_text_without_long_runs():
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
     assert "resolve_words_kernel" in emu_sort.launches and not any("collect_words_kernel" in k for k in emu_sort.launches)
+
+
+@pytest.mark.parametrize("values", [20, 60, 100])
+def test_copies_among_independent_letters_are_settled_on_the_first_word(values):
+    """A third of the suffixes tie, two or three to a group: nothing is read of their second words."""
+    lib = load_emulation("libcascade_emu_buckets.so")
+    rng = np.random.default_rng(values)
+    T = rng.integers(1, values, 9001).astype(np.uint16)
+    for k in range(6):
+        T[1400 * k + 700:1400 * k + 1000] = T[1400 * k:1400 * k + 300]
+    T[8600:8900] = T[700:1000]
+    got, active, _ = emu_sort(lib, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    assert 9001 // 8 < counts[-4] and "settle" in emu_sort.launches and "resolve_words_kernel" not in emu_sort.launches
