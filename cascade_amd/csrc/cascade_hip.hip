@@ -1763,9 +1763,10 @@ int settle_chains(Launch& L, Chains& ch, const u16* d_text, u32 n, u64 ctx, u64 
 // Generation 0: ranks the sorted list described by `ra`: counts per tile, scans the counts, reads the totals back, then
 // applies them and brings rank[] up to date, directly from the kernel or through the two-pass bucketed update.
 // coded: the list comes from sort_by_codes and carries its ties. settle: the ties of a list of short groups are settled at once if possible; the
-// ranks are not needed then, nor are they when nothing is tied.
+// ranks are not needed then, nor are they when nothing is tied. counted: the counts are in the tables, and *survivors, *groups and *rank_update are set.
 int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivors, u32* groups, int* rank_update,
-                u32* level_counts = nullptr, CodedList* coded = nullptr, int* passes = nullptr, Settle* settle = nullptr)
+                u32* level_counts = nullptr, CodedList* coded = nullptr, int* passes = nullptr, Settle* settle = nullptr,
+                bool counted = false)
 {
     csa_handle* h = L.h;
     hipStream_t s = L.stream;
@@ -1803,7 +1804,7 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
             add_table(beside, h_levels, ra.level_totals, LEVEL_SLOTS * 8 * sizeof(unsigned long long));
         return rank_totals(L, r, true, ra.m, ra.n, false, survivors, groups, rank_update, beside);
     };
-    int rc = count_and_read();
+    int rc = counted ? CSA_OK : count_and_read();
     if (rc)
         return rc;
     if (coded && !coded->by_levels) {
@@ -1865,10 +1866,17 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
 
 // Written text (word_keys.hpp): texts of at least this many symbols over 17 to 128 values (a symbol of eight bits gains nothing in the first word). Below,
 // its round trips and launches cost as much as they save: 40000 letters of written text take 361 us by the doubling and 364 this way, independent ones of an
-// alphabet of 20 217 and 238; 3 * 10^5 of written text 681 and 416. Texts whose runs of equal first words are long (choose_seconds_kernel) lose the launches that
-// tell: 10^6 symbols of log lines 1203 us and 1210, 3 * 10^7 with long runs of spaces 6.20 ms and 6.30.
+// alphabet of 20 217 and 238; 3 * 10^5 of written text 681 and 416. Texts that the second words are left out of (choose_seconds_kernel) are
+// counted once, on the context that the doubling goes on from, and take what they took on keys of eight symbols: 2^18 symbols of log lines 940 us and 934, 10^6 1206 and
+// 1193, 2 * 10^7 5.41 ms and 5.39, with runs of spaces 4.29 and 4.33.
 #ifndef CSA_WORD_KEYS_MIN
 #define CSA_WORD_KEYS_MIN (1u << 18)
+#endif
+// Texts with a run or a period that the settling would give up at: the second words are read from this many symbols on, and the doubling goes on from them. (us with
+// the second words left out / read: 10^6 letters of written text with a period of 11 over 1 % of them 1138 / 1175, 2 * 10^6 1212 / 1339, 4 * 10^6 1529 / 1537, 5.6 * 10^6
+// 1740 / 1721, 1.2 * 10^7 2748 / 2540; with 2 % in runs of spaces 1257 / 1303, 1396 / 1443, 1746 / 1736, 1863 / 1878, 2941 / 2827.)
+#ifndef CSA_WORD_ENDLESS_MIN
+#define CSA_WORD_ENDLESS_MIN (1u << 22)
 #endif
 static_assert(CSA_WORD_KEYS_MIN * sizeof(u64) >= sizeof(u32) << WINDOW_BITS<7>, "the windows are counted in a list of keys");
 
@@ -2328,6 +2336,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     settle.word_bits = ps.stream ? 64u / ps.sym_bits * ps.sym_bits : 0u;
     WordList words;
     memset(&words, 0, sizeof(words));
+    bool counted_firsts = false; // a list by words has been counted on the context it is ranked on
     u32 by_words_settled = 0; // generations of the reference that such a sort has left nothing of, and one
     if (by_words) {
         words.levels = word_levels(word_syms, word_bits, wide_ell);
@@ -2362,9 +2371,9 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         firsts.err = h->counts + 2;
         firsts.level_totals = reinterpret_cast<unsigned long long*>(h->ghist);
         unsigned long long* const h_levels = reinterpret_cast<unsigned long long*>(h->h_pinned + PINNED_HIST + 512);
-        HIP_TRY(hipMemsetAsync(firsts.level_totals, 0, LEVEL_SLOTS * 8 * sizeof(unsigned long long), s));
-        hipLaunchKernelGGL(choose_seconds_kernel, dim3(1), dim3(WORD_PLACES), 0, s, (const u64*)k_sorted, n, h->counts + 6);
-        firsts.skip = h->counts + 6;
+        hipLaunchKernelGGL(choose_seconds_kernel, dim3(ENDLESS_BLOCKS), dim3(WORD_PLACES), 0, s, (const u64*)k_sorted, (const u32*)sa32, n, word_syms,
+                           n < CSA_WORD_ENDLESS_MIN ? SECONDS_LEFT_OUT : SECONDS_ONLY, h->counts + 6, firsts.level_totals);
+        firsts.choice = h->counts + 6;
         hipLaunchKernelGGL((rerank_count_kernel<RANK_BLOCK, RANK_ITEMS>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, firsts);
         TableGroup beside = {};
         add_table(beside, h_levels, firsts.level_totals, LEVEL_SLOTS * 8 * sizeof(unsigned long long));
@@ -2372,7 +2381,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         int update = 0;
         if ((rc = rank_totals(L, r, true, n, n, false, &tied, &in_groups, &update, beside)) != CSA_OK)
             return rc;
-        const bool skip = h->h_pinned[6] != 0; // (nothing has been counted then)
+        const u32 choice = h->h_pinned[6];
         u32 known = lv.in_first; // levels whose lists are known
         for (u32 i = 0; i < known; ++i) {
             u64 sv = 0, hd = 0;
@@ -2383,16 +2392,15 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             words.survivors[i] = (u32)sv;
             words.groups[i] = (u32)hd;
         }
-        firsts.skip = nullptr;
         const bool few_ties = tied < n / 8, copies = 2 * (u64)tied <= 5 * (u64)in_groups;
-        if (!skip && tied > 0 && (few_ties ? (u64)tied <= (u64)in_groups * SETTLE_AVG_LIMIT : copies)) {
+        if (choice == SECONDS_AND_SETTLE && tied > 0 && (few_ties ? (u64)tied <= (u64)in_groups * SETTLE_AVG_LIMIT : copies)) {
             firsts.rank = nullptr;
             hipLaunchKernelGGL((rerank_kernel<RANK_BLOCK, RANK_ITEMS, false>), dim3(r.tiles), dim3(RANK_BLOCK), 0, s, firsts);
             HIP_TRY(hipGetLastError());
             if ((rc = settle_at(word_syms, tied, in_groups, few_ties)) != CSA_OK)
                 return rc;
         }
-        const bool seconds = !skip && tied > 0 && !settle.settled;
+        const bool seconds = choice == SECONDS_ONLY || (choice == SECONDS_AND_SETTLE && tied > 0 && !settle.settled);
         bool whole = false;
         if (seconds) {
             u8* const ties = reinterpret_cast<u8*>(K[cur ^ 1]);
@@ -2409,7 +2417,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             known = lv.count;
             tied = words.survivors[all];
             in_groups = words.groups[all];
-            if (whole && tied > 0 && (u64)tied <= (u64)in_groups * SETTLE_AVG_LIMIT) {
+            if (whole && choice == SECONDS_AND_SETTLE && tied > 0 && (u64)tied <= (u64)in_groups * SETTLE_AVG_LIMIT) {
                 RerankArgs active = ra;
                 active.rank = nullptr;
                 hipLaunchKernelGGL((compact_ties_kernel<RANK_TILE>), dim3((r.tiles + 3) / 4), dim3(256), 0, s, active, r.tiles);
@@ -2418,7 +2426,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                     return rc;
             }
         }
-        if (!skip && (settle.settled || (tied == 0 && (whole || known == lv.in_first)))) {
+        if (choice != SECONDS_LEFT_OUT && (settle.settled || (tied == 0 && (whole || known == lv.in_first)))) {
             // the lists of all generations are known: those of the contexts inside the words, and those that were settled
             u32 gens = 1;
             auto report = [&](u64 active, u64 groups_of) {
@@ -2455,21 +2463,20 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
                 list.told = list.by_levels = true;
                 ra.words = at;
                 coded = true;
-            } else {
+            } else { // (counted on that context)
                 ra.ell = ell;
                 ra.drop = lv.drop[at - 1];
-                ra.levels = ra.first_level = 0;
-                for (u32 i = 0; i + 1 < at; ++i) // (counted with it)
-                    if (lv.context[i] >= wide_ell) {
-                        ra.level_ell[ra.levels] = lv.context[i];
-                        ra.level_drop[ra.levels++] = lv.drop[i];
-                    }
+                m = tied;
+                groups = in_groups;
+                st->rank_update[0] = update;
+                counted_firsts = true;
             }
+            ra.levels = ra.first_level = 0;
             folded = 0;
             for (u64 f = ell; f < wide_ell; f = next(f))
                 ++folded;
-            pp.skipped = ra.levels;
-            for (u32 i = 0; i + 1 < at && seconds; ++i)
+            pp.skipped = 0;
+            for (u32 i = 0; i + 1 < at; ++i) // (counted with it)
                 if (lv.context[i] >= wide_ell) {
                     level_counts[2 * pp.skipped] = words.survivors[i];
                     level_counts[2 * pp.skipped + 1] = words.groups[i];
@@ -2478,9 +2485,9 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
             settle.settled = false;
         }
     }
-    if (by_words_settled == 0) // (a list by levels has had its shorter contexts counted)
-        rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], by_words && coded ? nullptr : level_counts, coded ? &list : nullptr, &passes,
-                         h->pack_symbols && h->settle && !by_words ? &settle : nullptr);
+    if (by_words_settled == 0) // (a list of words has had its shorter contexts counted)
+        rc = rerank_step(L, ra, defer_buffers(), &m, &groups, &st->rank_update[0], by_words ? nullptr : level_counts, coded ? &list : nullptr, &passes,
+                         h->pack_symbols && h->settle && !by_words ? &settle : nullptr, counted_firsts);
     range_gen0.close();
     if (rc)
         return rc;

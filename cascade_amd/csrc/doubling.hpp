@@ -63,6 +63,10 @@ __device__ __forceinline__ SlabPrefix slabs_before(const u32* __restrict__ slab_
 
 constexpr u32 MAX_LEVELS = 4, LEVEL_SLOTS = 64;
 
+// A list of first words (word_keys.hpp) is counted as such, or not at all (the second words are read first), or on the last of the levels (they are left out).
+// Of what several workgroups say the largest counts.
+enum : u32 { SECONDS_AND_SETTLE = 0, SECONDS_ONLY = 1, SECONDS_LEFT_OUT = 2 };
+
 struct RerankArgs {
     const u64* keys; // unused where the list carries its ties (TIED)
     const u32* sufs;
@@ -73,7 +77,7 @@ struct RerankArgs {
     u32 n;         // partition size
     u32 ell;       // symbols in the generation-0 key, or in its bits above the lowest `drop`, which the list is ranked on then
     u32 drop;
-    const u32* skip; // null, or where a word other than zero says that the list need not be counted
+    const u32* choice; // rerank_count_kernel: null, or where one of these stands
     // Packed keys of many symbols (packed_text.hpp): the counting pass also counts what the list would leave at shorter
     // contexts. Level i looks at the key bits above level_drop[i] and sets apart the suffixes that run off the text inside
     // level_ell[i] symbols; its survivors and groups are added to level_totals[slot * 8 + 2 i] and [.. + 1], slot = tile
@@ -148,11 +152,11 @@ __device__ __forceinline__ void load_with_neighbours(const u64* __restrict__ key
     }
 }
 
-// Whether sorted element c (key_c, suf_c) belongs to the run of element c - 1 (key_b, suf_b); both exist.
-__device__ __forceinline__ bool same_run(const RerankArgs& a, u64 key_b, u32 suf_b, u64 key_c, u32 suf_c)
+// Whether sorted element c (key_c, suf_c) belongs to the run of element c - 1 (key_b, suf_b) on the ell symbols above the lowest `drop` bits; both exist.
+__device__ __forceinline__ bool same_run(u32 n, u32 ell, u32 drop, u64 key_b, u32 suf_b, u64 key_c, u32 suf_c)
 {
     // a suffix that runs off the text inside its key ties with nobody (include/bit-layout.hpp:99-100)
-    return ((key_b ^ key_c) >> a.drop) == 0 && (u64)suf_b + a.ell < a.n && (u64)suf_c + a.ell < a.n;
+    return ((key_b ^ key_c) >> drop) == 0 && (u64)suf_b + ell < n && (u64)suf_c + ell < n;
 }
 
 // The counting pass of generation 0 on its own: the per-tile aggregates need no ordering inside the tile, so every
@@ -170,7 +174,9 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
     const u32 tile = blockIdx.x;
     const u64 base = (u64)tile * TILE + (u64)t * ITEMS;
     const u32 m = a.m;
-    if (a.skip && *a.skip) {
+    const u32 choice = a.choice ? *a.choice : SECONDS_AND_SETTLE;
+    const u32 ell = choice == SECONDS_LEFT_OUT ? a.level_ell[a.levels - 1] : a.ell, drop = choice == SECONDS_LEFT_OUT ? a.level_drop[a.levels - 1] : a.drop;
+    if (choice == SECONDS_ONLY) {
         if (t < 4)
             a.tile_agg[(u64)tile * 4 + t] = 0;
         if (t == 0)
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
 #pragma unroll
     for (int k = 0; k < ITEMS + 1; ++k) {
         const u64 c = base + k; // right element of the pair (c - 1, c)
-        const bool e = c >= 1 && c < m && same_run(a, key[k], suf[k], key[k + 1], suf[k + 1]);
+        const bool e = c >= 1 && c < m && same_run(a.n, ell, drop, key[k], suf[k], key[k + 1], suf[k + 1]);
         if (k >= 1 && c - 1 < m) { // element c - 1 = base + k - 1: prev_eq ties it to its left, e to its right
             const bool ka = !prev_eq;
             const bool single = ka && !e;
@@ -199,14 +205,14 @@ __global__ __launch_bounds__(BLOCK) void rerank_count_kernel(RerankArgs a)
     // the same counts at the shorter contexts of packed keys (one-word keys: nothing is read from the text)
     __shared__ u32 s_level[WAVES][MAX_LEVELS];
     for (u32 i = 0; i < a.levels; ++i) {
-        const u32 drop = a.level_drop[i];
+        const u32 ldrop = a.level_drop[i];
         const u64 lell = a.level_ell[i];
         u32 cs = 0, ch = 0;
         bool pe = false;
 #pragma unroll
         for (int k = 0; k < ITEMS + 1; ++k) {
             const u64 c = base + k;
-            const bool e = c >= 1 && c < m && ((key[k] ^ key[k + 1]) >> drop) == 0 && (u64)suf[k] + lell < a.n && (u64)suf[k + 1] + lell < a.n;
+            const bool e = c >= 1 && c < m && ((key[k] ^ key[k + 1]) >> ldrop) == 0 && (u64)suf[k] + lell < a.n && (u64)suf[k + 1] + lell < a.n;
             if (k >= 1 && c - 1 < m) {
                 const bool ka = !pe;
                 const bool single = ka && !e;
@@ -440,7 +446,7 @@ __global__ __launch_bounds__(BLOCK) void rerank_kernel(RerankArgs a)
 #pragma unroll
         for (int k = 0; k < ITEMS + 1; ++k) {
             const u64 c = base + k; // right element of the pair
-            eq[k] = c >= 1 && c < m && same_run(a, key[k], suf[k], key[k + 1], suf[k + 1]);
+            eq[k] = c >= 1 && c < m && same_run(a.n, a.ell, a.drop, key[k], suf[k], key[k + 1], suf[k + 1]);
         }
     }
 

@@ -10,6 +10,7 @@
 #pragma once
 
 #include "coded_keys.hpp"
+#include "copies.hpp"
 #include "device_utils.hpp"
 #include "doubling.hpp"
 #include "packed_text.hpp"
@@ -125,23 +126,49 @@ __global__ __launch_bounds__(WINDOW_BLOCK) void word_digits_kernel(const u32* __
 // ranked on the doubling's last context inside the first word.
 constexpr u32 WORD_PLACES = 1024, WORD_LONG = 256, WORD_LONG_FEW = 143, WORD_LONG_SHIFT = 18, WORD_LONGER_FEW = 51;
 
-// (Launched before the list is counted, which is then left out: nothing would be done with the counts.)
-__global__ __launch_bounds__(WORD_PLACES) void choose_seconds_kernel(const u64* __restrict__ keys, u32 n, u32* skip)
+// One long run or period is enough for the settling to give up, after it has looked at the period's groups (11 groups of 1818 members, all tied for thousands of
+// symbols: 0.4 ms): a region of more than ENDLESS_SYMBOLS symbols and ENDLESS_TIMES periods, or many short ones of one run that make a group of more than
+// SETTLE_MAX_WORDS members on both words. A place of the list is in a region if the places behind it with the same first word stand equally far apart in the text, all
+// the way. Looked for at 4096 places, by as many workgroups as take 1024 (one of 1024 threads took four times as long, 20 us). Where some are found nothing is settled,
+// and in texts of fewer than CSA_WORD_ENDLESS_MIN symbols the second words are left out as well.
+constexpr u32 ENDLESS_BLOCKS = 4, ENDLESS_SYMBOLS = 512, ENDLESS_TIMES = 32, PIECES_FEW = 1; // (of 1024 places)
+
+// Launched before the list is counted, which it says how (rerank_count_kernel). *choice is zero before; the totals of levels are set to zero.
+__global__ __launch_bounds__(WORD_PLACES) void choose_seconds_kernel(const u64* __restrict__ keys, const u32* __restrict__ sufs, u32 n, u32 syms, u32 if_endless, u32* choice, unsigned long long* level_totals)
 {
-    __shared__ u32 s_in[2];
-    const u32 t = threadIdx.x;
-    if (t < 2)
+    __shared__ u32 s_in[4];
+    const u32 t = threadIdx.x, places = gridDim.x * WORD_PLACES, place = t * gridDim.x + blockIdx.x;
+    if (t < 4)
         s_in[t] = 0;
+    if (place < LEVEL_SLOTS * 8)
+        level_totals[place] = 0;
     __syncthreads();
-    const u32 is_long = n >> WORD_LONG_SHIFT > WORD_LONG ? n >> WORD_LONG_SHIFT : WORD_LONG, longer = 8 * is_long;
-    const u64 in_long = __ballot(in_long_run(keys, n, is_long, t, WORD_PLACES)), in_longer = __ballot(in_long_run(keys, n, longer, t, WORD_PLACES));
-    if ((t & 63u) == 0) {
-        atomicAdd(&s_in[0], (u32)__popcll(in_long));
-        atomicAdd(&s_in[1], (u32)__popcll(in_longer));
+    const u32 is_long = n >> WORD_LONG_SHIFT > WORD_LONG ? n >> WORD_LONG_SHIFT : WORD_LONG;
+    const u32 e = (u32)((u64)n * place / places), next = e + 1 < n ? e + 1 : e;
+    const u64 key = keys[e];
+    const bool equal = keys[next] == key;
+    const u32 x = sufs[e], y = sufs[next];
+    u32 found[4];
+    found[0] = in_long_run(keys, n, is_long, place, places) ? 1u : 0u;
+    found[1] = in_long_run(keys, n, 8 * is_long, place, places) ? 1u : 0u;
+    const u32 gap = y > x ? y - x : 0u; // (members of a run come in text order, but for those that end the text)
+    auto goes_on = [&](u32 times) { return (u64)e + times < n && keys[e + times] == key && sufs[e + times] - x == times * gap; };
+    const bool near = equal && gap > 0;
+    found[2] = near && goes_on(gap * ENDLESS_TIMES < ENDLESS_SYMBOLS ? (ENDLESS_SYMBOLS + gap - 1) / gap : ENDLESS_TIMES) ? 1u : 0u;
+    // (gaps of up to a word: the second words are the same as well)
+    found[3] = near && gap <= syms && goes_on(2 * syms / gap) && in_long_run(keys, n, (u32)SETTLE_MAX_WORDS, place, places) ? 1u : 0u;
+#pragma unroll
+    for (u32 i = 0; i < 4; ++i) {
+        const u64 b = __ballot(found[i] != 0);
+        if ((t & 63u) == 0 && b)
+            atomicAdd(&s_in[i], (u32)__popcll(b));
     }
     __syncthreads();
-    if (t == 0)
-        *skip = s_in[0] > WORD_LONG_FEW || s_in[1] > WORD_LONGER_FEW ? 1u : 0u;
+    if (t == 0) {
+        const u32 mine = s_in[0] > WORD_LONG_FEW || s_in[1] > WORD_LONGER_FEW ? SECONDS_LEFT_OUT : s_in[2] > 0 || s_in[3] > PIECES_FEW ? if_endless : SECONDS_AND_SETTLE;
+        if (mine)
+            atomicMax(choice, mine);
+    }
 }
 
 constexpr int WORDS_MAX = RESOLVE_MAX;

@@ -372,6 +372,12 @@ inline unsigned long long atomicCAS(unsigned long long* p, unsigned long long ex
     __atomic_compare_exchange_n(p, &expected, desired, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);
     return expected; // the value found, as the device function returns it
 }
+inline unsigned atomicMax(unsigned* p, unsigned v)
+{
+    unsigned found = __atomic_load_n(p, __ATOMIC_SEQ_CST);
+    while (found < v && !__atomic_compare_exchange_n(p, &found, v, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST)) {}
+    return found;
+}
 inline unsigned atomicCAS(unsigned* p, unsigned expected, unsigned desired)
 {
     __atomic_compare_exchange_n(p, &expected, desired, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);

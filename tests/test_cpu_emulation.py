@@ -1106,3 +1106,32 @@ def test_copies_among_independent_letters_are_settled_on_the_first_word(values):
     sa, counts = oracle_lib.prefix_doubling(T, 1)
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
     assert 9001 // 8 < counts[-4] and "settle" in emu_sort.launches and "resolve_words_kernel" not in emu_sort.launches
+
+
+@pytest.mark.parametrize("n,kind", [(n, kind) for n in (9001, 11001) for kind in ("run", "period", "long_period", "short_run", "run_and_copies")] + [(60001, "pieces")])
+def test_long_runs_and_periods_of_written_text_are_not_settled(n, kind):
+    """One period of a few percent of the text, far from what the second words are left out for: the settling would give it up, and is not tried. Texts of 10000
+    symbols or more have their second words read all the same in this build. A run that the settling can end is none such."""
+    lib = load_emulation("libcascade_emu_buckets.so")
+    T = texts.written_text(n, 300, n)
+    rng = np.random.default_rng(n)
+    if kind.startswith("run"):
+        T[3000:3560] = 65
+    elif kind == "period":
+        T[3000:3800] = np.resize(T[:11], 800)
+    elif kind == "long_period":
+        T[3000:3000 + 90 * 25] = np.resize(rng.integers(97, 123, 25), 90 * 25)
+    elif kind == "short_run":
+        T[3000:3100] = 65
+    elif kind == "pieces":
+        for at in rng.permutation(n // 300)[:25]:
+            T[300 * at:300 * at + 110] = 65
+    if kind == "run_and_copies":
+        T[:3000] = rng.integers(97, 123, 3000)
+        T[4000:n - 1000] = rng.integers(97, 123, n - 5000)
+        T[5000:6500] = T[1200:2700]
+    got, active, _ = emu_sort(lib, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    assert ("settle" in emu_sort.launches) == (kind == "short_run")
+    assert ("resolve_words_kernel" in emu_sort.launches) == (kind == "short_run" or n > 10000)
