@@ -505,6 +505,7 @@ struct TextSource {
     const u32* stream; // SRC_PACKED
     u64 words;
     u32 sym_bits, key_bits;
+    bool scanned; // digit_base is filled as well
 };
 
 int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64* kout,
@@ -561,7 +562,8 @@ int radix_sort(Launch& L, int src, u32 text_n, u32 tail, u64* kin, u32* vin, u64
             hipLaunchKernelGGL(radix_hist_kernel, dim3(hist_blocks(256 * 16, n)), dim3(256), 0, s, ha);
         }
     }
-    hipLaunchKernelGGL(radix_scan_hist_kernel<RADIX_BINS>, dim3(1), dim3(RADIX_BINS), 0, s, h->ghist, h->digit_base, plan.num_passes);
+    if (!source || !source->scanned)
+        hipLaunchKernelGGL(radix_scan_hist_kernel<RADIX_BINS>, dim3(1), dim3(RADIX_BINS), 0, s, h->ghist, h->digit_base, plan.num_passes);
     HIP_TRY(hipGetLastError());
     // (the digits of K-gram keys are the two bytes of a symbol, four times: where both take several values no pass is skipped)
     const bool all_run = src == SRC_TEXT && !source->byte_wide;
@@ -2245,9 +2247,12 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         const u32 blocks = hist_blocks(WINDOW_BLOCK * 4, n);
         auto* const count = word_bits == 5 ? window_hist_kernel<5> : word_bits == 6 ? window_hist_kernel<6> : window_hist_kernel<7>;
         hipLaunchKernelGGL(count, dim3(blocks < WINDOW_HIST_BLOCKS ? blocks : WINDOW_HIST_BLOCKS), dim3(WINDOW_BLOCK), 0, s, (const u32*)h->rank, n, windows);
-        hipLaunchKernelGGL(word_digits_kernel, dim3((ps.key_bits + 7) / 8), dim3(WINDOW_BLOCK), 0, s, (const u32*)h->rank, (const u32*)windows, n, word_bits, ps.key_bits, h->ghist);
+        auto* const expand = word_bits == 5 ? word_digits_kernel<5> : word_bits == 6 ? word_digits_kernel<6> : word_digits_kernel<7>;
+        const PassPlan plan = make_plan(0, (int)ps.key_bits); // (digits of eight bits, and what is left)
+        hipLaunchKernelGGL(expand, dim3(plan.num_passes), dim3(WINDOW_BLOCK), 0, s, (const u32*)h->rank, (const u32*)windows, n, ps.key_bits, h->ghist, h->digit_base);
+        ps.scanned = true;
         HIP_TRY(hipGetLastError());
-        rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, make_plan(0, (int)ps.key_bits), &in_out, &p1, nullptr, 0, 0, &ps);
+        rc = radix_sort(L, SRC_PACKED, n, tail, K[0], V[0], K[1], V[1], n, plan, &in_out, &p1, nullptr, 0, 0, &ps);
     } else if (pp.enabled) {
         const PassPlan plan = make_plan(0, narrow ? 32 : (int)ps.key_bits);
         hipLaunchKernelGGL(packed_hist_expand_kernel, dim3(1), dim3(256), 0, s, ps.stream, n, ps.sym_bits, ell, plan.num_passes, bytehist,
