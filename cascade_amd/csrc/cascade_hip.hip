@@ -1871,8 +1871,14 @@ int rerank_step(Launch& L, RerankArgs& ra, const DeferBuffers& buf, u32* survivo
 // alphabet of 20 217 and 238; 3 * 10^5 of written text 681 and 416. Texts that the second words are left out of (choose_seconds_kernel) are
 // counted once, on the context that the doubling goes on from, and take what they took on keys of eight symbols: 2^18 symbols of log lines 940 us and 934, 10^6 1206 and
 // 1193, 2 * 10^7 5.41 ms and 5.39, with runs of spaces 4.29 and 4.33.
+// More than 64 values, which leave nine symbols to a word, from four times as many on (us on keys of eight symbols and by words: independent letters of 100 2^18 symbols 234 / 240,
+// 3.5 * 10^5 240 / 246, 2^19 257 / 259, 10^6 291 / 293, 4 * 10^6 453 / 413; of written text with capitals, digits and marks 507 / 518, 565 / 552, 581 / 582, 663 / 632,
+// 967 / 873; the same over 60 values 505 / 340, 569 / 358, 577 / 570, 659 / 623).
 #ifndef CSA_WORD_KEYS_MIN
 #define CSA_WORD_KEYS_MIN (1u << 18)
+#endif
+#ifndef CSA_WORD_KEYS_MIN_SEVEN_BITS
+#define CSA_WORD_KEYS_MIN_SEVEN_BITS (1u << 20)
 #endif
 // Texts with a run or a period that the settling would give up at: the second words are read from this many symbols on, and the doubling goes on from them. (us with
 // the second words left out / read: 10^6 letters of written text with a period of 11 over 1 % of them 1138 / 1175, 2 * 10^6 1212 / 1339, 4 * 10^6 1529 / 1537, 5.6 * 10^6
@@ -2179,7 +2185,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     }
     TextSource ps;
     memset(&ps, 0, sizeof(ps));
-    const bool by_words = pp.values > 16 && pp.values <= 128 && n >= CSA_WORD_KEYS_MIN && h->pack_symbols && h->settle && !h->expect_presorted;
+    const bool by_words = pp.values > 16 && pp.values <= 128 && n >= (pp.values > 64 ? CSA_WORD_KEYS_MIN_SEVEN_BITS : CSA_WORD_KEYS_MIN) && h->pack_symbols && h->settle && !h->expect_presorted;
     const u32 word_bits = by_words ? (u32)bit_length(pp.values - 1) : 0u, word_syms = by_words ? 64u / word_bits : 0u;
     const PackedPlan as_reported = pp; // what callers are told of the first sort of such texts
     if (by_words)

@@ -83,7 +83,7 @@ typedef struct csa_stats {
                                         first of a list of runs and periods, which is settled at once as well (big[] and presorted[]
                                         as the generations would have had them). Texts of up to 8192 symbols are ranked by counting:
                                         no passes, all time in ms[0], and 4 here whatever the alphabet. Written text (17 to 128 byte
-                                        values, 2^18 symbols or more) is sorted by words of 9 to 12 symbols, and the next word where
+                                        values, 2^18 symbols or more; over more than 64, 2^20) is sorted by words of 9 to 12 symbols, and the next word where
                                         those tie, and reports the key_symbols and first_sort_generations of 8-bit codes */
     uint32_t first_sort_generations; /* generations of the reference that sort stands for: 1, or 1 + j when its keys held
                                         4 * key_words * 2^j symbols. Generations 1 .. j are then reported with the lists
