@@ -41,7 +41,7 @@ struct BucketArgs {
     u32* starts;         // [buckets + 1]: where they start
     const u32* top_base; // of the last pass: where its digits start ...
     u32 top_shift;       // ... and the bit of the code that they start from
-    u32* over;           // zeroed: [0] suffixes in buckets of more than BUCKET_MAX, [1] such buckets
+    u32* over;           // zeroed: [0] suffixes in buckets of more than BUCKET_MAX, [1] such buckets, [2] suffixes in the largest
     u32* over_list;      // [n / BUCKET_MAX]: them, in any order
     u32* crowded;        // zeroed: buckets with a cell of more than CELL_MAX ...
     u32* crowded_list;   // ... [buckets]: them, in any order
@@ -59,6 +59,7 @@ struct BucketArgs {
     u64* over_keys;
     u32* over_sufs;
     u32* over_open; // EXT: where they start in the list of open runs
+    u32 over_slices; // workgroups a bucket
 };
 
 constexpr int STARTS_BLOCK = 256;
@@ -92,6 +93,7 @@ __global__ __launch_bounds__(STARTS_BLOCK) void bucket_starts_kernel(BucketArgs 
         if (size > BUCKET_MAX) {
             a.over_list[atomicAdd(&a.over[1], 1u)] = b;
             atomicAdd(&a.over[0], size);
+            atomicMax(&a.over[2], size);
         }
     }
 }
@@ -414,7 +416,12 @@ __global__ __launch_bounds__(BUCKET_BLOCK) void finish_crowded_kernel(BucketArgs
 // ---- buckets that do not fit ----
 
 constexpr int OVER_TILE = 1024;
-constexpr u32 OVER_SLICES = 16; // workgroups a bucket
+// A workgroup moves OVER_SLICE suffixes of a bucket; of many buckets, one of which is much larger than the others, more, so that there are no more than OVER_BLOCKS
+// workgroups or 16 a bucket. (10^8 letters with 6 % in a run of one letter and 3 % in one of another, 16 workgroups a bucket whatever its size: 675 us there and 804 back, 37 and 36 now.)
+#ifndef CSA_OVER_SLICE
+#define CSA_OVER_SLICE 4096
+#endif
+constexpr u32 OVER_SLICE = CSA_OVER_SLICE, OVER_BLOCKS = 1u << 15;
 
 __global__ __launch_bounds__(OVER_TILE) void over_before_kernel(BucketArgs a)
 {
@@ -439,13 +446,16 @@ __global__ __launch_bounds__(OVER_TILE) void over_before_kernel(BucketArgs a)
         *a.over_open = atomicAdd(a.open_count, a.over[0]);
 }
 
-// The suffixes of the buckets in over_list to their places in over_keys and over_sufs, or back from there (BACK), OVER_SLICES workgroups a bucket.
+// The suffixes of the buckets in over_list to their places in over_keys and over_sufs, or back from there (BACK), over_slices workgroups a bucket.
 // EXT: by the code and ext; on the way back the ties follow from those.
 template <bool BACK, bool EXT>
 __global__ __launch_bounds__(256) void over_move_kernel(BucketArgs a)
 {
     __shared__ u32 s_sum[256 / WAVE];
-    const u32 t = threadIdx.x, b = a.over_list[blockIdx.x / OVER_SLICES];
+    const u32 t = threadIdx.x, b = a.over_list[blockIdx.x / a.over_slices], start = a.starts[b], size = a.starts[b + 1] - start;
+    const u32 per = (size + a.over_slices - 1) / a.over_slices, first = blockIdx.x % a.over_slices * per, last = size - first < per ? size : first + per;
+    if (first >= size)
+        return;
     u32 earlier = 0;
     for (u32 i = t; i < b / OVER_TILE; i += 256)
         earlier += a.over_tiles[i];
@@ -456,8 +466,7 @@ __global__ __launch_bounds__(256) void over_move_kernel(BucketArgs a)
     u32 to = a.over_before[b];
     for (u32 ww = 0; ww < 256 / WAVE; ++ww)
         to += s_sum[ww];
-    const u32 start = a.starts[b], size = a.starts[b + 1] - start;
-    for (u32 i = blockIdx.x % OVER_SLICES * 256 + t; i < size; i += OVER_SLICES * 256) {
+    for (u32 i = first + t; i < last; i += 256) {
         if constexpr (!BACK) {
             a.over_keys[to + i] = EXT ? (u64)a.codes[start + i] << 16 | a.ext[start + i] : (u64)a.codes[start + i];
             a.over_sufs[to + i] = a.sufs[start + i];

@@ -1080,10 +1080,15 @@ void probe_buckets(ProbeArgs& a, const CodeDigits& digits, u32* room)
     a.full_from = full > 2 ? full : 2;
 }
 
-// Buckets that do not fit are sorted by radix passes after all: from a tenth of the suffixes on all passes are made at once.
-bool buckets_fit(const ProbeCounts& c, u32 n, const CodeDigits& digits)
+// Buckets that do not fit are sorted by radix passes after all: from a tenth of the suffixes on all passes are made at once, and from a fiftieth on in four-letter texts of
+// fewer than 2^25 symbols, which save the least. (Time with all passes / with buckets, by the share that the sample shows. Tokens, strings that come often: 10^8 symbols 0.06 4417 / 3575 us,
+// 0.12 5007 / 3667, 0.18 5665 / 4136; past a quarter all that do not fit are given up, 3 * 10^7 0.30 1738 / 2393. Tokens, a run and a period: 1.7 * 10^7 0.08 1908 / 1880, 0.12 1932 / 1952; 10^8 0.11
+// 7983 / 7280; 4 * 10^8 0.12 31.0 / 26.9 ms, 0.19 35.2 / 38.4. Letters, two runs: 1.7 * 10^7 0.04 2253 / 2289 us, 0.08 2344 / 2425; 3 * 10^7 0.04 3395 / 3397, 0.08 3580 / 3607, 0.12 3741 / 3789; 10^8 0.08
+// 9402 / 9204, 0.16 10989 / 11017; 4 * 10^8 0.10 35.6 / 34.5 ms. Texts all of whose buckets fit show up to 0.01 below 3.3 * 10^8 symbols, and 0.04 at 4.2 * 10^8.)
+bool buckets_fit(const ProbeCounts& c, u32 n, const CodeDigits& digits, bool packed)
 {
-    return (u64)c.packed * 10 * (bucket_skip(n, digits) + 1u) <= probed_suffixes(n);
+    const u32 one_in = packed && n < 1u << 25 ? 50 : 10;
+    return (u64)c.packed * one_in * (bucket_skip(n, digits) + 1u) <= probed_suffixes(n);
 }
 
 // What a sort by codes starts from: the shares of the symbols, and for texts of PROBE_MIN symbols or more what a sample of the suffixes
@@ -1186,7 +1191,7 @@ int narrow_keys_pay(Launch& L, const TextSource& ps, u32 n, bool* pay, CodeDigit
         return rc;
     HIP_TRY(hipStreamSynchronize(s));
     *pay = (u64)seen->crowded * 6 <= a.taken;
-    *digits = buckets_fit(*seen, n, in_buckets) ? in_buckets : ALL_DIGITS;
+    *digits = buckets_fit(*seen, n, in_buckets, true) ? in_buckets : ALL_DIGITS;
     return CSA_OK;
 }
 
@@ -1285,22 +1290,22 @@ int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* co
     a.over = h->counts + 8;
     a.over_list = h->gprim[1];
     a.tail = tail;
-    a.crowded = h->counts + 10;
+    a.crowded = h->counts + 11;
     a.crowded_list = h->gstart[0]; // (done with before over_before)
     if (ext) {
         a.ext = ext;
         a.ext_bits = digits.buckets_log2 < 16u ? digits.buckets_log2 : 16u;
         a.sufs_out = h->idx[1];
         a.ties = ties_of(h);
-        a.open_count = h->counts + 11;
+        a.open_count = h->counts + 12;
         a.open_sufs = open_sufs_of(h);
         a.open_places = open_places_of(h);
-        a.over_open = h->counts + 12;
+        a.over_open = h->counts + 13;
     }
     a.over_before = h->gstart[0];
     a.over_tiles = h->gstart[1];
     hipLaunchKernelGGL(bucket_starts_kernel, dim3(a.buckets / (STARTS_BLOCK - 1) + 1), dim3(STARTS_BLOCK), 0, s, a);
-    int rc = move_table(h->h_pinned + 8, a.over, 2 * sizeof(u32), s);
+    int rc = move_table(h->h_pinned + 8, a.over, 3 * sizeof(u32), s);
     if (rc)
         return rc;
     HIP_TRY(hipEventRecord(h->ev_gen[2], s)); // (recorded again when a generation ends)
@@ -1314,7 +1319,7 @@ int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* co
     }
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventSynchronize(h->ev_gen[2]));
-    const u32 over = h->h_pinned[8], over_buckets = h->h_pinned[9];
+    const u32 over = h->h_pinned[8], over_buckets = h->h_pinned[9], largest = h->h_pinned[10];
     *finished = over <= n / 4 && over <= h->cap / 2;
     if (over == 0 || !*finished)
         return CSA_OK;
@@ -1323,7 +1328,9 @@ int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* co
     a.over_keys = K[0];
     a.over_sufs = V[0];
     hipLaunchKernelGGL(over_before_kernel, dim3((a.buckets + OVER_TILE - 1) / OVER_TILE), dim3(OVER_TILE), 0, s, a);
-    const dim3 over_grid(over_buckets * OVER_SLICES);
+    const u32 wanted = (largest + OVER_SLICE - 1) / OVER_SLICE, most = OVER_BLOCKS / over_buckets;
+    a.over_slices = wanted < most ? wanted : most < 16u ? 16u : most;
+    const dim3 over_grid(over_buckets * a.over_slices);
     if (ext)
         hipLaunchKernelGGL((over_move_kernel<false, true>), over_grid, dim3(256), 0, s, a);
     else
@@ -1446,7 +1453,7 @@ int sort_by_codes(Launch& L, const u16* d_text, u32 n, u32 tail, u32 words, Code
     const dim3 resolve_grid((u32)(((u64)n + RESOLVE_TILE - 1) / RESOLVE_TILE));
     if (digits.buckets_log2 && !packed) { // the list stands in idx[1] already, but for its open runs
         r.codes = nullptr;
-        r.open_count = h->counts + 11;
+        r.open_count = h->counts + 12;
         r.sufs = open_sufs_of(h);
         r.places = open_places_of(h);
         hipLaunchKernelGGL((resolve_runs_kernel<RESOLVE_MAX, false, false, false, true>), dim3(resolve_grid.x < OPEN_BLOCKS ? resolve_grid.x : OPEN_BLOCKS),
@@ -2144,7 +2151,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
     // The byte histograms of the text come first: they tell whether the alphabet is small enough for keys of more than four
     // symbols. (The digit counts are zeroed with them.)
     TableGroup zeros = {};
-    add_table(zeros, h->counts, nullptr, 13 * sizeof(u32));
+    add_table(zeros, h->counts, nullptr, 14 * sizeof(u32));
     add_table(zeros, h->ghist, nullptr, (MAX_PASSES + 2) * RADIX_BINS * sizeof(u32));
     int rc = move_tables(zeros, s);
     if (rc)
@@ -2228,7 +2235,7 @@ int sort_partition(Launch& L, const u16* d_text, u64 n64, u64 index_base, u8* d_
         if (probed) {
             HIP_TRY(hipEventSynchronize(h->ev_gen[1]));
             coded = codes_pay(*seen, n);
-            if (coded && in_buckets && !ahead && buckets_fit(*seen, n, bucket_digits(n, false)))
+            if (coded && in_buckets && !ahead && buckets_fit(*seen, n, bucket_digits(n, false), false))
                 digits = bucket_digits(n, false);
         }
         if (coded && !ahead && (rc = code_suffixes(L, d_text, n, tail, counted = digits)) != CSA_OK)
