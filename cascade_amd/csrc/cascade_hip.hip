@@ -1048,8 +1048,10 @@ CodeDigits bucket_digits(u32 n, bool packed)
     u32 log2 = 1;
     while ((n >> log2) > BUCKET_AVERAGE)
         ++log2;
-    // (the digits of packed keys are counted by eight bits: up to nine tenths of BUCKET_MAX)
-    if (packed && log2 == CSA_TWO_PASS_LOG2 + 1 && (n >> CSA_TWO_PASS_LOG2) <= BUCKET_MAX / 10 * 9)
+    // The digits of packed keys are counted by eight bits, so there are no more buckets: as long as the average one is 2.5 standard deviations of its size below
+    // BUCKET_MAX (4.5 * 10^8 symbols). (Four letters, with copies / independent, ms with all passes and with buckets: 3.4 * 10^8 symbols 16.6, 14.9 / 10.4, 8.7; 4.4 * 10^8 21.2,
+    // 19.4 / 13.3, 11.2; 4.55 * 10^8 22.4, 20.5 / 14.0, 11.8; 4.62 * 10^8, where a tenth of the buckets does not fit, 22.7, 22.3 / 14.1, 13.1; 4.66 * 10^8 22.8, 28.5 / 14.3, 15.8.)
+    if (packed && log2 == CSA_TWO_PASS_LOG2 + 1 && (n >> CSA_TWO_PASS_LOG2) <= BUCKET_MAX / 100 * 97)
         log2 = CSA_TWO_PASS_LOG2;
     if (log2 <= CSA_TWO_PASS_LOG2)
         return CodeDigits{2, RADIX_BITS, {16, 24}, log2};
