@@ -2022,17 +2022,15 @@ int sort_by_words(Launch& L, u32 n, const TextSource& ps, u32 syms, u64* spare, 
 
 // The contexts of a list that is resolved on two words of syms symbols: the doubling's from the caller's key on, the last of those before it that the first
 // word holds, from which the doubling may go on, and the two words themselves.
-WordLevels word_levels(u32 syms, u32 bits, u64 wide_ell)
+// (Evaluated for all of them by the compiler, which does not let one past the last level be written.)
+constexpr WordLevels word_levels(u32 syms, u32 bits, u64 wide_ell)
 {
-    WordLevels l;
-    memset(&l, 0, sizeof(l));
-    auto next = [&](u64 c) { return c + (c < wide_ell ? (c < wide_ell - c ? c : wide_ell - c) : c); };
+    WordLevels l = {};
+    auto next = [=](u64 c) { return c + (c < wide_ell ? (c < wide_ell - c ? c : wide_ell - c) : c); };
     auto add = [&](u64 c) {
-        if (l.count < WORD_LEVELS) {
-            l.in_first += c <= syms ? 1u : 0u;
-            l.context[l.count] = (u32)c;
-            l.drop[l.count++] = (u32)(c <= syms ? syms - c : 2 * syms - c) * bits;
-        }
+        l.in_first += c <= syms ? 1u : 0u;
+        l.context[l.count] = (u32)c;
+        l.drop[l.count++] = (u32)(c <= syms ? syms - c : 2 * syms - c) * bits;
     };
     for (u64 c = 4; c <= 2 * syms; c = next(c))
         if (c >= wide_ell || (c <= syms && next(c) > syms))
@@ -2041,6 +2039,17 @@ WordLevels word_levels(u32 syms, u32 bits, u64 wide_ell)
         add(2 * syms);
     return l;
 }
+
+template <u32 BITS>
+constexpr bool word_levels_fit()
+{
+    constexpr WordLevels of[4] = {word_levels(64 / BITS, BITS, 4), word_levels(64 / BITS, BITS, 8), word_levels(64 / BITS, BITS, 12), word_levels(64 / BITS, BITS, 16)};
+    for (const WordLevels& l : of)
+        if (l.in_first == 0 || l.in_first > l.count)
+            return false;
+    return true;
+}
+static_assert(word_levels_fit<5>() && word_levels_fit<6>() && word_levels_fit<7>(), "some key width has no context of the doubling inside the first word");
 
 // Texts of this length on are looked at before their bytes are counted (text_byte_hist_kernel). us of that kernel without the look and with it, independent ids / 26
 // letters, which are counted all the same: 2^18 symbols 5.2, 4.1 / 5.1, 7.9; 2^20 7.3, 4.8 / 6.2, 9.4; 2^22 12.5, 5.0 / 10.5, 12.9; 2^24 23.0, 5.7 / 19.2, 23.3. From 2^22
