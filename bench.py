@@ -24,7 +24,6 @@ RADIX_PASS_BYTES_PER_PAIR = 2 * (8 + 5)
 # the same of a pass of the first sort over (32-bit code, index) pairs, which texts over large alphabets take: a 4-byte key
 CODED_PASS_BYTES_PER_PAIR = 2 * (4 + 5)
 CODED_PASSES = 4
-BUCKET_PASSES = 2  # of a long text's codes: the lower digits are sorted in LDS, bucket by bucket
 
 
 def algorithmic_bytes(n, active):
@@ -476,6 +475,19 @@ def untimed_as(st, g):
     return "covered_by_first_sort" if g < first else "settled_at_once"
 
 
+def passes_over_codes(st, launches, pairs):
+    """Of the radix passes of one sort (its statistics; its launches and the pairs they moved), those of the first sort over (32-bit code, index) pairs of the
+    whole list: 0 where it took 64-bit keys, so that all its passes are over the whole list and there are more than four. Otherwise four less the ones that
+    passes[0] counts and nobody launched, the digits sorted in LDS; what else passes[0] holds are runs and buckets that had to be sorted again, of a few suffixes each."""
+    n, gens = st["n"], range(1, st["generations"])
+    later = sum(st["passes"][g] * (n if st["dense"][g] else st["big"][g] - st["presorted"][g]) for g in gens)
+    if st["passes"][0] > CODED_PASSES and pairs - later > 0.9 * n * st["passes"][0]:
+        return 0
+    if st["key_symbols"] not in (4, 32):  # (8, 16 or 64 packed symbols: always 64-bit keys)
+        return 0
+    return CODED_PASSES - (sum(st["passes"][:st["generations"]]) - launches)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -635,11 +647,8 @@ def main():
 
     # dominant kernel: the one-sweep radix pass, timed per launch with HIP events on the sort's stream
     avg_launch_ms = radix_ms / radix_launches if radix_launches else 0.0
-    # a first sort on packed symbols resolves 8 or more; one on K-gram keys, which none of these workloads takes, makes 8 passes, and so
-    # does one on 64-bit packed keys (32 letters on narrow keys: four, as codes, unless long runs were sorted again)
-    coded = st["passes"][0] != 8 if st["key_symbols"] == 4 else st["key_symbols"] == 32 and st["passes"][0] == 4
-    coded_passes = CODED_PASSES if radix_pairs >= CODED_PASSES * n * args.steps else BUCKET_PASSES
-    coded_pairs = min(coded_passes * n * args.steps, radix_pairs) if coded else 0
+    coded_passes = passes_over_codes(st, radix_launches // args.steps, radix_pairs // args.steps)
+    coded_pairs = min(coded_passes * n * args.steps, radix_pairs)
     radix_bytes = RADIX_PASS_BYTES_PER_PAIR * (radix_pairs - coded_pairs) + CODED_PASS_BYTES_PER_PAIR * coded_pairs
     achieved = radix_bytes / (radix_ms * 1e-3) / 1e9 if radix_ms > 0 else 0.0
     pairs_per_launch = radix_pairs / radix_launches if radix_launches else 0
@@ -684,7 +693,7 @@ def main():
                                   f"{st['first_sort_generations'] - 1} of the reference's list, whose bytes the yardstick still counts")
     elif coded_pairs:
         result["job_alg_note"] = (f"the yardstick counts generation 0 as eight passes over (64-bit key, index) pairs; the sort makes {coded_passes} over "
-                                  "(32-bit code, index) pairs" + (", and the lower digits in LDS" if coded_passes == BUCKET_PASSES else ""))
+                                  "(32-bit code, index) pairs" + (", and the lower digits in LDS" if coded_passes < CODED_PASSES else ""))
     if moved_gen_dropped:
         result["generation_traffic_dropped"] = moved_gen_dropped
     if args.cpu_sample > 0:

@@ -60,3 +60,22 @@ def test_the_bench_line_tells_covered_generations_from_settled_ones():
     assert bench.untimed_as(dict(codes, key_words=4), 1) == "settled_at_once"  # (generation 0 of wide keys takes the eight symbols)
     packed = {"first_sort_generations": 4, "key_symbols": 32, "key_words": 1}
     assert [bench.untimed_as(packed, g) for g in (1, 3, 4)] == ["covered_by_first_sort", "covered_by_first_sort", "settled_at_once"]
+
+
+def test_bench_tells_passes_over_codes_from_those_over_wide_keys():
+    """From the statistics alone, whatever had to be sorted again besides: four passes in one of these cases are those over K-grams in another."""
+    sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    import bench
+    n = 1000
+
+    def stats(passes, key_symbols=4, big=(0, 0, 0), presorted=(0, 0, 0), dense=(0, 0, 0)):
+        return {"n": n, "generations": 3, "passes": [passes, 3, 0], "key_symbols": key_symbols, "big": list(big), "presorted": list(presorted), "dense": list(dense)}
+
+    assert bench.passes_over_codes(stats(4, big=(0, 50, 0)), 7, 4 * n + 150) == 4
+    assert bench.passes_over_codes(stats(8, big=(0, 50, 0)), 11, 8 * n + 150) == 0  # K-grams
+    assert bench.passes_over_codes(stats(8, big=(0, 50, 0)), 9, 2 * n + 4 * 90 + 150) == 2  # buckets, and what fits none in four passes more
+    assert bench.passes_over_codes(stats(8, big=(0, 50, 0)), 11, 4 * n + 4 * 90 + 150) == 4  # runs that were out of order
+    assert bench.passes_over_codes(stats(8, big=(0, n, 0), dense=(0, 1, 0)), 11, 4 * n + 4 * 90 + 3 * n) == 4
+    assert bench.passes_over_codes(stats(8, 32, big=(0, 50, 0)), 11, 8 * n + 150) == 0  # 32 letters in 64 bits
+    assert bench.passes_over_codes(stats(4, 32, big=(0, 50, 0)), 5, 2 * n + 150) == 2
+    assert bench.passes_over_codes(stats(8, 8, big=(0, 50, 0)), 11, 8 * n + 150) == 0
