@@ -1087,9 +1087,12 @@ void probe_buckets(ProbeArgs& a, const CodeDigits& digits, u32* room)
 // 0.12 5007 / 3667, 0.18 5665 / 4136; past a quarter all that do not fit are given up, 3 * 10^7 0.30 1738 / 2393. Tokens, a run and a period: 1.7 * 10^7 0.08 1908 / 1880, 0.12 1932 / 1952; 10^8 0.11
 // 7983 / 7280; 4 * 10^8 0.12 31.0 / 26.9 ms, 0.19 35.2 / 38.4. Letters, two runs: 1.7 * 10^7 0.04 2253 / 2289 us, 0.08 2344 / 2425; 3 * 10^7 0.04 3395 / 3397, 0.08 3580 / 3607, 0.12 3741 / 3789; 10^8 0.08
 // 9402 / 9204, 0.16 10989 / 11017; 4 * 10^8 0.10 35.6 / 34.5 ms. Texts all of whose buckets fit show up to 0.01 below 3.3 * 10^8 symbols, and 0.04 at 4.2 * 10^8.)
+#ifndef CSA_MANY_LETTERS
+#define CSA_MANY_LETTERS (1u << 25)
+#endif
 bool buckets_fit(const ProbeCounts& c, u32 n, const CodeDigits& digits, bool packed)
 {
-    const u32 one_in = packed && n < 1u << 25 ? 50 : 10;
+    const u32 one_in = packed && n < CSA_MANY_LETTERS ? 50 : 10;
     return (u64)c.packed * one_in * (bucket_skip(n, digits) + 1u) <= probed_suffixes(n);
 }
 

@@ -1137,3 +1137,28 @@ def test_long_runs_and_periods_of_written_text_are_not_settled(n, kind):
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
     assert ("settle" in emu_sort.launches) == (kind == "short_run")
     assert ("resolve_words_kernel" in emu_sort.launches) == (kind == "short_run" or n > 10000)
+
+
+@pytest.mark.parametrize("n,symbols", [(17003, 50000), (33001, 50000), (60001, 4), (90003, 4)])
+def test_buckets_all_over_the_range(n, symbols):
+    """More buckets than the upper digit has values, in several tiles: crowded ones, ones that do not fit, and such that just do, wherever their codes put them, of
+    tokens and of letters."""
+    lib = load_emulation("libcascade_emu_search.so")
+    T = texts.text_of_planted_strings(n, symbols, [25, 40, 200, 230, 260, 300, 90, 60, 280], n)
+    got, active, _ = emu_sort(lib, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts
+    ext = "true" if symbols > 4 else "false"
+    for kernel in ("finish_crowded_kernel<%s>" % ext, "(over_move_kernel<true, %s>)" % ext):
+        assert kernel in emu_sort.launches
+
+
+@pytest.mark.parametrize("values", [32, 33, 65])
+@pytest.mark.parametrize("kind", ["copies", "period", "zeros", "end"])
+def test_marked_text(values, kind):
+    """The texts that the GPU's tests of words take, in small."""
+    lib = load_emulation("libcascade_emu_buckets.so")
+    T = texts.marked_text(20001, values, kind, values)
+    got, active, _ = emu_sort(lib, T, 1)
+    sa, counts = oracle_lib.prefix_doubling(T, 1)
+    assert np.unique(T).size == values and np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and active == counts

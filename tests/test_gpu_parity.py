@@ -869,12 +869,14 @@ def test_lists_with_many_suffixes_in_long_runs(torch_mod, n, phrases, lo, hi):
 
 @pytest.mark.parametrize("n,letters", [((1 << 24) + 1, 50000), ((1 << 24) + 4099, 50000), (30000001, 4)])
 def test_lower_digits_are_sorted_in_buckets(torch_mod, n, letters):
-    """Texts of more than 2^24 symbols: two passes over the upper digits, then buckets in LDS, with strings that come 300 times (a crowded cell) and 20000
-    times (a bucket that does not fit) among independent ones, and four-letter texts with copies. The device verifier judges, and the generation
+    """Texts of more than 2^24 symbols: two passes over the upper digits, then buckets in LDS, with strings that come 300 times and 20000
+    times (buckets that do not fit, at the lower end of the range) among independent ones, and four-letter texts with copies. The device verifier judges, and the generation
     sizes are those of the sort with K-gram keys."""
     from cascade_amd import PartitionSorter, _native
     rng = np.random.default_rng(n)
     T = rng.integers(1, letters + 1, n).astype(np.uint16)
+    if letters == 4:
+        T -= 1  # (zero is a value whether it occurs or not: five values take four bits)
     if letters > 4:
         for string, times in enumerate([300, 20000, 7300, 256, 258]):
             at = 8 * rng.permutation(n // 8 - 1)[:times]
@@ -903,6 +905,60 @@ def test_written_text_is_sorted_by_two_words(torch_mod, n, words, key_words):
         T[k * n // 6 - 600:k * n // 6] = T[100 * k:100 * k + 600]
     with PartitionSorter(n, key_words=key_words) as s:
         print(f"  written text {n} {words} {key_words}", flush=True)
+        got = gpu_sa40(torch_mod, s, T)
+        stats = s.last_stats
+    sa, counts = oracle_lib.prefix_doubling(T, key_words)
+    assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
+
+
+@pytest.mark.parametrize("n,symbols", [((1 << 24) + 1, 50000), (30000001, 4)])
+def test_buckets_all_over_the_range(torch_mod, n, symbols):
+    """Strings that come 600 to 2500 times (cells of more than CELL_MAX in buckets that fit), some 7168 with the others of their bucket, and 20000 and 50000 times
+    (buckets that do not fit), their codes spread over the whole range."""
+    from cascade_amd import PartitionSorter, _native
+    T = texts.text_of_planted_strings(n, symbols, [600, 2500, 20000, 1000, 3000, 3071, 3072, 50000, 700, 3100, 20000, 2500, 30000], n)
+    d = to_dev(torch_mod, T)
+    seen = []
+    with PartitionSorter(n, key_words=1) as s:
+        for pack in (1, 0):
+            print(f"  buckets all over {n} {symbols} {pack}", flush=True)
+            s.set_tuning(_native.CSA_TUNE_PACK_SYMBOLS, pack)
+            out = s.sort(d)
+            assert s.verify(d, out)
+            seen.append(s.last_stats["active"])
+    assert seen[0] == seen[1]
+
+
+def test_nine_bit_digits(torch_mod):
+    """The shortest text whose buckets take two digits of nine bits, and one that takes two of eight, with copies and strings that come often."""
+    from cascade_amd import PartitionSorter
+    for n in (5001 << 16, (5001 << 16) - 1):
+        g = torch_mod.Generator(device="cuda").manual_seed(n)
+        d = torch_mod.randint(1, 30000, (n,), generator=g, device="cuda", dtype=torch_mod.int32).to(torch_mod.int16)
+        d[n // 2:n // 2 + 70000] = d[1000:71000].clone()
+        for i, times in enumerate([3000, 60000, 1000, 20000]):
+            at = 8 * torch_mod.randperm(n // 8 - 1, generator=g, device="cuda")[:times]
+            for k, symbol in enumerate([100 + 8000 * i, 7, 8, 9]):
+                d[at + k] = symbol
+        torch_mod.cuda.synchronize()
+        torch_mod.cuda.empty_cache()
+        with PartitionSorter(n, key_words=1) as s:
+            print(f"  nine-bit digits {n}", flush=True)
+            assert s.verify(d, s.sort(d))
+
+
+@pytest.mark.parametrize("n,values,kind,key_words", [(1 << 18, 32, "copies", 1), ((1 << 18) + 3, 33, "copies", 3), (1 << 20, 65, "copies", 1), ((1 << 20) - 1, 65, "copies", 1),
+                                                     (1 << 18, 32, "period", 1), (300007, 64, "period", 2), ((1 << 22) - 1, 33, "period", 1), ((1 << 22) + 1, 40, "period", 1),
+                                                     ((1 << 20) + 9, 128, "zeros", 1), (1 << 18, 33, "zeros", 3), (300001, 17, "zeros", 4),
+                                                     (1 << 18, 64, "end", 1), (1 << 20, 128, "end", 3), ((1 << 18) + 1, 32, "end", 1)])
+def test_words_of_symbols_of_five_to_seven_bits(torch_mod, n, values, kind, key_words):
+    """Alphabets at both ends of the widths of a symbol's code, from the shortest texts of each on: copies, which are settled on the first word; a period, for which
+    nothing is settled, with the second words read from 2^22 symbols on; zeros that look like padding; an end of the text inside a long run. Against the oracle, generation
+    sizes included."""
+    from cascade_amd import PartitionSorter
+    T = texts.marked_text(n, values, kind, n + values)
+    with PartitionSorter(n, key_words=key_words) as s:
+        print(f"  words {n} {values} {kind} {key_words}", flush=True)
         got = gpu_sa40(torch_mod, s, T)
         stats = s.last_stats
     sa, counts = oracle_lib.prefix_doubling(T, key_words)

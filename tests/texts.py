@@ -239,3 +239,46 @@ def written_text(n, words, seed, letters=26):
     ids = np.minimum(rng.zipf(1.3, n), words) - 1  # (a word is two symbols at least)
     text = [symbol for i in ids[:n // 2 + 1] for symbol in vocabulary[i]]
     return np.array(text[:n], dtype=np.uint16)
+
+
+def text_of_planted_strings(n, symbols, repeats, seed):
+    """n independent symbols, 1 to `symbols` (or 0 to 3, of two bits), among them strings that come repeats[i] times each, at multiples of 16, their first symbols spread over the whole alphabet: of
+    four symbols, or of 16 where the alphabet has four letters."""
+    rng = np.random.default_rng(seed)
+    T = rng.integers(1, symbols + 1, n).astype(np.uint16)
+    places = 16 * rng.permutation(n // 16 - 1)[:sum(repeats)]
+    for i, times in enumerate(repeats):
+        at, places = places[:times], places[times:]
+        if symbols > 4:
+            string = np.concatenate([[1 + (2 * i + 1) * (symbols - 1) // (2 * len(repeats))], rng.integers(1, symbols + 1, 3)])
+        else:
+            string = np.concatenate([[1 + i * 16 // len(repeats) // 4, 1 + i * 16 // len(repeats) % 4], rng.integers(1, symbols + 1, 14)])
+        T[at[:, None] + np.arange(string.size)] = string
+    return T if symbols > 4 else T - np.uint16(1)
+
+
+def marked_text(n, values, kind, seed):
+    """n symbols over `values` values, zero among them: independent ones with copies, or words with marks in between, and what `kind` says (a period over a
+    fiftieth of it, zeros here and there and at the end, a phrase that comes 700 times and ends the text inside)."""
+    rng = np.random.default_rng(seed)
+    if kind == "copies":
+        T = rng.integers(0, values, n).astype(np.uint16)
+        for k in range(10):
+            T[k * n // 10 + n // 20:k * n // 10 + n // 20 + n // 50] = T[k * n // 10:k * n // 10 + n // 50]
+    else:
+        T = np.maximum(written_text(n, 1500, seed, min(values - 1, 26)).astype(np.int64) - 96, 0)  # (the space is zero)
+        marks = rng.permutation(n // 20)[:n // 40] * 20
+        T[marks] = rng.integers(0, values, marks.size)
+    if kind == "period":
+        T[n // 3:n // 3 + n // 50] = np.resize(T[:11], n // 50)
+    elif kind == "zeros":
+        for at in rng.permutation(n // 40 - 1)[:n // 400]:
+            T[40 * at:40 * at + int(rng.integers(3, 36))] = 0
+        T[-30:] = 0
+    elif kind == "end":
+        phrase = rng.integers(1, values, 24)
+        for at in rng.permutation(n // 64 - 1)[:700]:
+            T[64 * at:64 * at + 24] = phrase
+        T[-16:] = phrase[:16]
+    T[:values] = np.arange(values)
+    return T.astype(np.uint16)
