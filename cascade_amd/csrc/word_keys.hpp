@@ -133,12 +133,16 @@ __global__ __launch_bounds__(WINDOW_BLOCK) void word_digits_kernel(const u32* __
 // ---- the second words ----
 
 // Texts that the second word does little for: padding, lines that come again and again, few words. Long runs of one first word are sorted again, to find them
-// long and of one second word as well. Looked for at 1024 places of the sorted list: more than 143 in runs of 256 or more, or more than 51 in
-// runs of 2048; the runs of a written text grow with it, so from 2^26 symbols on in runs of n / 2^18, and eight times that. (10^8 letters of written text have 10
-// and 2 % of their suffixes in such, 5 * 10^7 with a fifth in runs of spaces and a period 28 and 22 %: those take 9.3 ms by the doubling and 10.4 when the
-// second words are read first. 2 * 10^8 letters: 31.9 ms by the doubling, where runs of 256 would send them, and 21.8; 3 * 10^8 49.1 and 42.2.) Such lists are
-// ranked on the doubling's last context inside the first word.
-constexpr u32 WORD_PLACES = 1024, WORD_LONG = 256, WORD_LONG_FEW = 143, WORD_LONG_SHIFT = 18, WORD_LONGER_FEW = 51;
+// long and of one second word as well. Looked for at 1024 places of the sorted list, in runs of 256 or more; the runs of a written text grow with it, so from 2^26 symbols on in
+// runs of n / 2^18, and in more places, from 26 of them in texts of 2^18 symbols to 220, a quarter of the list less what such a sample is off by: from a quarter on the
+// second words are given up (sort_by_words). Such lists are ranked on the doubling's last context inside the first word. (Places, and us with the second words left out / read. Words of 400 to 32000,
+// Zipf(1.1), letters alike: 6 * 10^5 symbols 107, 772 / 872, 10^6 99, 818 / 910, 2 * 10^6 129, 919 / 1020, 10^7 233, 2381 / 2584; log lines 10^6 526, 1202 / 1360. Words of which the
+// frequent ones are short, with copies, of 28 values 10^6 symbols 1, 755 / 587, 10^7 13, 2025 / 1280; of 100 values 2 * 10^6 21, 709 / 682, 4 * 10^6 36, 923 / 871, 10^7 56, 1805 / 1418, 5 * 10^7 141, 6366 / 5293;
+// with runs of spaces 5 * 10^7 190, 9560 / 8609, 252, 10716 / 11515; with a period 238, 9895 / 9030, 1.5 * 10^8 248, 27.8 / 30.1 ms.)
+#ifndef CSA_WORD_LONG_FEW
+#define CSA_WORD_LONG_FEW 24
+#endif
+constexpr u32 WORD_PLACES = 1024, WORD_LONG = 256, WORD_LONG_SHIFT = 18, WORD_LONG_FEW = CSA_WORD_LONG_FEW, WORD_LONG_FEW_SHIFT = 17, WORD_LONG_MOST = 220;
 
 // One long run or period is enough for the settling to give up, after it has looked at the period's groups (11 groups of 1818 members, all tied for thousands of
 // symbols: 0.4 ms): a region of more than ENDLESS_SYMBOLS symbols and ENDLESS_TIMES periods, or many short ones of one run that make a group of more than
@@ -150,9 +154,9 @@ constexpr u32 ENDLESS_BLOCKS = 4, ENDLESS_SYMBOLS = 512, ENDLESS_TIMES = 32, PIE
 // Launched before the list is counted, which it says how (rerank_count_kernel). *choice is zero before; the totals of levels are set to zero.
 __global__ __launch_bounds__(WORD_PLACES) void choose_seconds_kernel(const u64* __restrict__ keys, const u32* __restrict__ sufs, u32 n, u32 syms, u32 if_endless, u32* choice, unsigned long long* level_totals)
 {
-    __shared__ u32 s_in[4];
+    __shared__ u32 s_in[3];
     const u32 t = threadIdx.x, places = gridDim.x * WORD_PLACES, place = t * gridDim.x + blockIdx.x;
-    if (t < 4)
+    if (t < 3)
         s_in[t] = 0;
     if (place < LEVEL_SLOTS * 8)
         level_totals[place] = 0;
@@ -162,24 +166,25 @@ __global__ __launch_bounds__(WORD_PLACES) void choose_seconds_kernel(const u64* 
     const u64 key = keys[e];
     const bool equal = keys[next] == key;
     const u32 x = sufs[e], y = sufs[next];
-    u32 found[4];
+    u32 found[3];
     found[0] = in_long_run(keys, n, is_long, place, places) ? 1u : 0u;
-    found[1] = in_long_run(keys, n, 8 * is_long, place, places) ? 1u : 0u;
     const u32 gap = y > x ? y - x : 0u; // (members of a run come in text order, but for those that end the text)
     auto goes_on = [&](u32 times) { return (u64)e + times < n && keys[e + times] == key && sufs[e + times] - x == times * gap; };
     const bool near = equal && gap > 0;
-    found[2] = near && goes_on(gap * ENDLESS_TIMES < ENDLESS_SYMBOLS ? (ENDLESS_SYMBOLS + gap - 1) / gap : ENDLESS_TIMES) ? 1u : 0u;
+    found[1] = near && goes_on(gap * ENDLESS_TIMES < ENDLESS_SYMBOLS ? (ENDLESS_SYMBOLS + gap - 1) / gap : ENDLESS_TIMES) ? 1u : 0u;
     // (gaps of up to a word: the second words are the same as well)
-    found[3] = near && gap <= syms && goes_on(2 * syms / gap) && in_long_run(keys, n, (u32)SETTLE_MAX_WORDS, place, places) ? 1u : 0u;
+    found[2] = near && gap <= syms && goes_on(2 * syms / gap) && in_long_run(keys, n, (u32)SETTLE_MAX_WORDS, place, places) ? 1u : 0u;
 #pragma unroll
-    for (u32 i = 0; i < 4; ++i) {
+    for (u32 i = 0; i < 3; ++i) {
         const u64 b = __ballot(found[i] != 0);
         if ((t & 63u) == 0 && b)
             atomicAdd(&s_in[i], (u32)__popcll(b));
     }
     __syncthreads();
     if (t == 0) {
-        const u32 mine = s_in[0] > WORD_LONG_FEW || s_in[1] > WORD_LONGER_FEW ? SECONDS_LEFT_OUT : s_in[2] > 0 || s_in[3] > PIECES_FEW ? if_endless : SECONDS_AND_SETTLE;
+        const u32 few = WORD_LONG_FEW + (n >> WORD_LONG_FEW_SHIFT);
+        const bool many = blockIdx.x == 0 && s_in[0] > (few < WORD_LONG_MOST ? few : WORD_LONG_MOST); // (one sample, not the largest of several)
+        const u32 mine = many ? SECONDS_LEFT_OUT : s_in[1] > 0 || s_in[2] > PIECES_FEW ? if_endless : SECONDS_AND_SETTLE;
         if (mine)
             atomicMax(choice, mine);
     }
