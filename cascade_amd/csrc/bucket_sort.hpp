@@ -419,8 +419,8 @@ __global__ __launch_bounds__(BUCKET_BLOCK) void finish_crowded_kernel(BucketArgs
 #define CSA_OVER_TILE 1024
 #endif
 constexpr int OVER_TILE = CSA_OVER_TILE;
-// A workgroup moves OVER_SLICE suffixes of a bucket; of many buckets, one of which is much larger than the others, more, so that there are no more than OVER_BLOCKS
-// workgroups or 16 a bucket. (10^8 letters with 6 % in a run of one letter and 3 % in one of another, 16 workgroups a bucket whatever its size: 675 us there and 804 back, 37 and 36 now.)
+// A workgroup moves OVER_SLICE suffixes of a large bucket, a sixteenth of a small one; of many buckets, one of which is much larger than the others, more, so that there are no
+// more than OVER_BLOCKS workgroups or 16 a bucket. (10^8 letters with 6 % in a run of one letter and 3 % in one of another, 16 workgroups a bucket whatever its size: 675 us there and 804 back, 37 and 36 now.)
 #ifndef CSA_OVER_SLICE
 #define CSA_OVER_SLICE 4096
 #endif

@@ -1334,7 +1334,8 @@ int finish_buckets(Launch& L, const CodeDigits& digits, u32 n, u32 tail, u32* co
     a.over_sufs = V[0];
     hipLaunchKernelGGL(over_before_kernel, dim3((a.buckets + OVER_TILE - 1) / OVER_TILE), dim3(OVER_TILE), 0, s, a);
     const u32 wanted = (largest + OVER_SLICE - 1) / OVER_SLICE, most = OVER_BLOCKS / over_buckets;
-    a.over_slices = wanted < most ? wanted : most < 16u ? 16u : most;
+    a.over_slices = wanted < most ? wanted : most;
+    a.over_slices = a.over_slices < 16u ? 16u : a.over_slices;
     const dim3 over_grid(over_buckets * a.over_slices);
     if (ext)
         hipLaunchKernelGGL((over_move_kernel<false, true>), over_grid, dim3(256), 0, s, a);
@@ -2055,10 +2056,10 @@ constexpr bool word_levels_fit()
 static_assert(word_levels_fit<5>() && word_levels_fit<6>() && word_levels_fit<7>(), "some key width has no context of the doubling inside the first word");
 
 // Texts of this length on are looked at before their bytes are counted (text_byte_hist_kernel). us of that kernel without the look and with it, independent ids / 26
-// letters, which are counted all the same: 2^18 symbols 5.2, 4.1 / 5.1, 7.9; 2^20 7.3, 4.8 / 6.2, 9.4; 2^22 12.5, 5.0 / 10.5, 12.9; 2^24 23.0, 5.7 / 19.2, 23.3. From 2^22
-// symbols on the look saves the one two to three times what it costs the other (of the sort 2 and 1 %).
+// letters, which are counted all the same: 2^18 symbols 5.2, 4.1 / 5.1, 7.9; 2^20 7.3, 4.8 / 6.2, 9.4; 2^22 12.5, 5.0 / 10.5, 12.9; 2^24 23.0, 5.7 / 19.2, 23.3. From 2^20
+// symbols on the look saves the one as much as it costs the other, and more and more in longer texts (2^22 2 % of the sort and 1 %).
 #ifndef CSA_BYTE_LOOK_MIN
-#define CSA_BYTE_LOOK_MIN (1u << 22)
+#define CSA_BYTE_LOOK_MIN (1u << 20)
 #endif
 constexpr u32 BYTE_LOOK_MIN = CSA_BYTE_LOOK_MIN;
 
