@@ -64,8 +64,8 @@ struct BucketArgs {
 
 constexpr int STARTS_BLOCK = 256;
 
-// Where the buckets start, by a search inside their top digit: a thread a bucket, and one more a workgroup for the end of its last. (Up to 21
-// dependent reads, 10 to 80 us.)
+// Where the buckets start, by a search inside their top digit: a thread a bucket, and one more a workgroup for the end of its last. (As many
+// dependent reads as the number of suffixes of the top digit has bits: 17 to 21 where the digits are alike, 30 at most. 10 to 90 us.)
 __global__ __launch_bounds__(STARTS_BLOCK) void bucket_starts_kernel(BucketArgs a)
 {
     __shared__ u32 s_start[STARTS_BLOCK];

@@ -537,6 +537,8 @@ __device__ __forceinline__ u64 second_word(const ResolveArgs& a, u32 x)
 // second word pays, since generation 1 would read as many lines. (ms by two words and by one, and the share of the places: 2^28 symbols
 // Zipf(1.4) 0.51 25.4, 30.3; 2^29 of runs and Zipf(1.3) 0.45 52.0, 59.8; 2^26 Zipf(1.5) 0.58 9.2, 8.6; 2^28 0.66 37.9, 34.4; 2^26 Zipf(2) 0.93 14.2, 13.9;
 // 5 * 10^6 of written text in 16-bit symbols 0.65 1.80, 1.63. Token texts have 0.04.)
+// Lists whose lower digits were sorted in buckets (open runs) always take two words: a text so heavy that one would do has buckets that do not fit and goes
+// through all passes. (3 * 10^7 symbols Zipf(1.4), open runs and two words 2.71 ms, all passes 3.05.)
 constexpr u32 HALF_LONG = RESOLVE_MAX / 2, SHORT_LIST_FEW = 12, LONG_LIST_PLACES = 1024, LONG_LIST_FEW = 543;
 
 // Lists of WORDS_AHEAD suffixes or more are looked at by a workgroup of its own: a launch costs 4 us, and the look of every tile 2 % of the sort of 2^28
