@@ -151,6 +151,12 @@ constexpr u32 WORD_PLACES = 1024, WORD_LONG = 256, WORD_LONG_SHIFT = 18, WORD_LO
 // and in texts of fewer than CSA_WORD_ENDLESS_MIN symbols the second words are left out as well.
 constexpr u32 ENDLESS_BLOCKS = 4, ENDLESS_SYMBOLS = 512, ENDLESS_TIMES = 32, PIECES_FEW = 1; // (of 1024 places)
 
+// Places further on in the list that a region of this period is followed to. (Gaps are as long as the text allows: 2^27 symbols and its copy, whose gap times 32 is zero
+// in 32 bits, took 194 ms without the settling, 24 with it.)
+constexpr u32 endless_places(u32 gap) { return (u64)gap * ENDLESS_TIMES < ENDLESS_SYMBOLS ? (ENDLESS_SYMBOLS + gap - 1) / gap : ENDLESS_TIMES; }
+static_assert(endless_places(1) == ENDLESS_SYMBOLS && endless_places(15) == 35 && endless_places(16) == ENDLESS_TIMES && endless_places(1u << 27) == ENDLESS_TIMES
+                  && endless_places(31u << 27) == ENDLESS_TIMES, "512 symbols of short periods, 32 of all others");
+
 // Launched before the list is counted, which it says how (rerank_count_kernel). *choice is zero before; the totals of levels are set to zero.
 __global__ __launch_bounds__(WORD_PLACES) void choose_seconds_kernel(const u64* __restrict__ keys, const u32* __restrict__ sufs, u32 n, u32 syms, u32 if_endless, u32* choice, unsigned long long* level_totals)
 {
@@ -169,9 +175,9 @@ __global__ __launch_bounds__(WORD_PLACES) void choose_seconds_kernel(const u64* 
     u32 found[3];
     found[0] = in_long_run(keys, n, is_long, place, places) ? 1u : 0u;
     const u32 gap = y > x ? y - x : 0u; // (members of a run come in text order, but for those that end the text)
-    auto goes_on = [&](u32 times) { return (u64)e + times < n && keys[e + times] == key && sufs[e + times] - x == times * gap; };
+    auto goes_on = [&](u32 times) { return (u64)e + times < n && keys[e + times] == key && sufs[e + times] - x == (u64)times * gap; };
     const bool near = equal && gap > 0;
-    found[1] = near && goes_on(gap * ENDLESS_TIMES < ENDLESS_SYMBOLS ? (ENDLESS_SYMBOLS + gap - 1) / gap : ENDLESS_TIMES) ? 1u : 0u;
+    found[1] = near && goes_on(endless_places(gap)) ? 1u : 0u;
     // (gaps of up to a word: the second words are the same as well)
     found[2] = near && gap <= syms && goes_on(2 * syms / gap) && in_long_run(keys, n, (u32)SETTLE_MAX_WORDS, place, places) ? 1u : 0u;
 #pragma unroll

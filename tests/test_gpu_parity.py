@@ -911,6 +911,23 @@ def test_written_text_is_sorted_by_two_words(torch_mod, n, words, key_words):
     assert np.array_equal(got, oracle_lib.u64_to_sa40(sa)) and stats["active"] == counts
 
 
+@pytest.mark.parametrize("length", [1 << 27, (1 << 27) + 20])
+def test_a_long_text_and_its_copy_are_settled_at_once(torch_mod, length):
+    """Letters, and all of them once more: pairs that stand a power of two symbols apart are no more a period than others, and the generations after the first sort's take no time."""
+    from cascade_amd import PartitionSorter
+    g = torch_mod.Generator(device="cuda").manual_seed(length)
+    half = torch_mod.randint(97, 123, (length,), generator=g, device="cuda", dtype=torch_mod.int32).to(torch_mod.int16)
+    d = torch_mod.cat([half, half])
+    torch_mod.cuda.synchronize()
+    torch_mod.cuda.empty_cache()
+    with PartitionSorter(2 * length, key_words=1) as s:
+        print(f"  twice {length}", flush=True)
+        out = s.sort(d)
+        stats = s.last_stats
+        assert s.verify(d, out)
+    assert stats["generations"] > 20 and sum(stats["ms"][stats["first_sort_generations"] + 1:]) == 0
+
+
 @pytest.mark.parametrize("n,symbols", [((1 << 24) + 1, 50000), (30000001, 4)])
 def test_buckets_all_over_the_range(torch_mod, n, symbols):
     """Strings that come 600 to 2500 times (cells of more than CELL_MAX in buckets that fit), some 7168 with the others of their bucket, and 20000 and 50000 times
