@@ -390,7 +390,11 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
     for (u32 i = t; i < TALLIES * COPIES; i += BLOCK)
         s_tally[i] = 0;
     if (t == 0) {
-        s_over = *a.failed;
+        // (An atomic load: a plain one of this address comes from the scalar cache, where a word that other tiles write stays as it was for the whole kernel. 3 * 10^7
+        // letters of passages and their copies, 27.3 -> 20.3 ms: every tile did all of its work. 4 * 10^8 letters that are settled: 17.5 -> 17.6.
+        // The load stays in front of the others: a build that looked at the flag just before the barrier put some 90 of 4 * 10^8 suffixes in wrong places in every sort,
+        // other ones each time, for no reason that was found in the source or in the assembly.)
+        s_over = dev_failed(a.failed) ? 1u : 0u;
         s_lost[0] = s_lost[1] = s_queued = 0;
     }
     const u64 t0 = (u64)blockIdx.x * TILE;
@@ -418,7 +422,7 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
         if (gs < t0 || gs >= t0 + TILE)
             continue; // another tile's
         if (gs > e || ge <= e || ge > a.m || ge - gs > (u32)MAXG) {
-            *a.failed = 1u;
+            __hip_atomic_store(a.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             continue;
         }
         from[k] = (int)(gs - t0);
@@ -492,7 +496,7 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
     __syncthreads();
     if (s_lost[0]) {
         if (t == 0)
-            *a.failed = 1u;
+            __hip_atomic_store(a.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
 #pragma unroll
@@ -545,7 +549,7 @@ __global__ __launch_bounds__(BLOCK) void settle_groups_kernel(SettleArgs a)
     __syncthreads();
     if (s_lost[1]) { // (the same for all threads: nobody sets it past the barrier)
         if (t == 0)
-            *a.failed = 1u;
+            __hip_atomic_store(a.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
 #pragma unroll

@@ -928,6 +928,56 @@ def test_a_long_text_and_its_copy_are_settled_at_once(torch_mod, length):
     assert stats["generations"] > 20 and sum(stats["ms"][stats["first_sort_generations"] + 1:]) == 0
 
 
+def test_settled_letters_are_the_same_every_time(torch_mod):
+    """4 * 10^8 letters of four, a fifth of them passages of 10000 that come two, three or four times, some with a letter changed: a hundred million members of groups are settled
+    in thousands of tiles at once. Every sort gives the same permutation, which the device verifier accepts."""
+    from cascade_amd import PartitionSorter
+    length, n = 10000, 400000000
+    g = torch_mod.Generator(device="cuda").manual_seed(11)
+    d = torch_mod.randint(0, 4, (n,), generator=g, device="cuda", dtype=torch_mod.int32).to(torch_mod.int16)
+    pairs = d.view(-1, 2, length)
+    count = pairs.shape[0] * 2 // 5
+    to = torch_mod.randperm(pairs.shape[0], generator=g, device="cuda")[:count]
+    pairs[to, 1] = pairs[torch_mod.randint(0, pairs.shape[0], (count,), generator=g, device="cuda"), 0]
+    at = torch_mod.randint(0, count * length, (count * length // 100,), generator=g, device="cuda")
+    at = to[at // length] * 2 * length + length + at % length
+    d[at] = (d[at] + 1) & 3
+    torch_mod.cuda.synchronize()
+    torch_mod.cuda.empty_cache()
+    with PartitionSorter(n, key_words=1) as s:
+        print(f"  settled letters {n}", flush=True)
+        first = s.sort(d)
+        assert s.verify(d, first) and sum(s.last_stats["ms"][s.last_stats["first_sort_generations"] + 1:]) == 0
+        for _ in range(10):
+            assert torch_mod.equal(s.sort(d), first)
+
+
+def test_a_settling_that_gives_up_ends_soon(torch_mod):
+    """Passages of 400 letters that come again, all over the text, and the whole text once more: telling their copies apart takes more steps than a comparison is given. Once one
+    tile has given up all others leave. What is left of an attempt are some four passes over the list, for each of two attempts, where the doubling without them makes
+    more than forty: less than a fifth of its time."""
+    from cascade_amd import PartitionSorter, _native
+    half, length = 15000000, 400
+    g = torch_mod.Generator(device="cuda").manual_seed(7)
+    text = torch_mod.randint(97, 123, (half,), generator=g, device="cuda", dtype=torch_mod.int32).to(torch_mod.int16)
+    pairs = text[:half // (2 * length) * 2 * length].view(-1, 2, length)
+    pairs[pairs.shape[0] // 2 + 1:, 0] = pairs[:pairs.shape[0] // 2 - 1, 0].clone()
+    d = torch_mod.cat([text, text])
+    least = []
+    with PartitionSorter(d.numel(), key_words=1) as s:
+        for settle in (1, 0):
+            s.set_tuning(_native.CSA_TUNE_SETTLE, settle)
+            times = []
+            for _ in range(4):
+                out = s.sort(d)
+                ms = s.last_stats["ms"]
+                times.append(sum(ms))
+            print(f"  given up {settle} {min(times):.2f} ms", flush=True)
+            assert s.verify(d, out) and sum(ms[3:]) > 0
+            least.append(min(times))
+    assert least[0] < 1.2 * least[1]
+
+
 @pytest.mark.parametrize("n,symbols", [((1 << 24) + 1, 50000), (30000001, 4)])
 def test_buckets_all_over_the_range(torch_mod, n, symbols):
     """Strings that come 600 to 2500 times (cells of more than CELL_MAX in buckets that fit), some 7168 with the others of their bucket, and 20000 and 50000 times
